@@ -1,9 +1,12 @@
 // 32-bit GEMM on the f32 MFMA (v_mfma_f32_16x16x4_f32: f32 products, f32 accumulation) for models
 // that run in 32-bit: Y = epi(X . W^T), both operands row-major with K contiguous.
 //
-// A 4-wave workgroup computes 64 x 64; each wave 32 x 32 = 2 x 2 MFMA tiles.  A lane's 16-byte load
-// holds 4 consecutive k of its row; the four MFMAs of a 16-deep step take element j of every lane
-// group, so A and B use the same k order and no LDS is needed.
+// A lane's 16-byte operand holds 4 consecutive k of its row; the four MFMAs of a 16-deep step take
+// element j of every lane group, so A and B use the same k order.  Two kernels (launch() chooses):
+//   * rows: a workgroup owns 16 or 32 columns and up to 64 rows, its waves split K and add up through
+//     LDS.  Few rows stream the weights, so what counts is bytes in flight on every CU: the k split
+//     gives a 1024-column projection 64 x 16 waves of them.
+//   * tiles: 64 x 64 outputs, operands by LDS-DMA, for products bound by the MFMA.
 #include "common.h"
 #include "stack_kernels.h"
 
@@ -13,63 +16,240 @@ namespace {
 
 VWA_DEVICE f32x4 mfma4(float a, float b, const f32x4& c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
+VWA_DEVICE f32x4 mfma4x4(const float4& a, const float4& b, f32x4 c) {
+  c = mfma4(a.x, b.x, c);
+  c = mfma4(a.y, b.y, c);
+  c = mfma4(a.z, b.z, c);
+  return mfma4(a.w, b.w, c);
+}
+
+// rows m .. m+3 of column n (EPI 2: v0 gate and v1 up of feature n)
 template <int EPI>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Params p) {
+VWA_DEVICE void store4(const GemmF32Params& p, int m, int n, const f32x4& v0, const f32x4& v1) {
+  if (n >= (EPI == 2 ? p.N >> 1 : p.N)) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (m + r >= p.M) return;
+    float v = v0[r];
+    if constexpr (EPI == 2) v = silu(v) * v1[r];
+    if constexpr (EPI == 1) v += p.R[(size_t)(m + r) * p.ldr + n];
+    if (EPI == 6 && n >= p.n_split) {
+      v = fmaxf(v, 0.f);
+      p.Y2[(size_t)(m + r) * p.ldy2 + n - p.n_split] = v * v;
+    } else {
+      p.Y[(size_t)(m + r) * p.ldy + n] = v;
+    }
+  }
+}
+
+// Bound by the weights' stream: 4 x 1024 x 4096 12.9 us (1.3 TB/s from 64 workgroups; 122 with one wave per 32 x 32
+// outputs), 4 x 8192 x 1024 9.5 us (3.5 TB/s; 38), 4 x 32768 x 1024 34 us (4.0 TB/s; 50).
+// 16 MT rows x 16 NT columns; the KS waves take a run of K's 16-deep steps each, U steps' loads in
+// flight while the U before are multiplied.
+template <int EPI, int MT, int NT, int KS, int U>
+__global__ __launch_bounds__(64 * KS) void rows_f32_kernel(GemmF32Params p) {
+  __shared__ f32x4 part[KS * MT * NT * 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int rl = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.y * 64 + (w & 1) * 32, n0 = blockIdx.x * 64 + (w >> 1) * 32;
-  if (m0 >= p.M || n0 >= p.N) return;
+  const int m0 = blockIdx.y * 16 * MT, n0 = blockIdx.x * 16 * NT;
   // rows past the end read the last row (their results are not stored)
-  const float* xa[2];
-  const float* wb[2];
+  const float* xa[MT];
+  const float* wb[NT];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    xa[i] = p.X + (size_t)min(m0 + 16 * i + rl, p.M - 1) * p.ldx + 4 * g;
-    wb[i] = p.W + (size_t)min(n0 + 16 * i + rl, p.N - 1) * p.K + 4 * g;
+  for (int i = 0; i < MT; ++i) xa[i] = p.X + (size_t)min(m0 + 16 * i + rl, p.M - 1) * p.ldx + 4 * g;
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wb[j] = p.W + (size_t)min(n0 + 16 * j + rl, p.N - 1) * p.K + 4 * g;
+  f32x4 acc[MT][NT] = {};
+  const int steps = p.K / 16, s0 = steps * w / KS, n = steps * (w + 1) / KS - s0, full = n / U;
+  float4 a0[U][MT], b0[U][NT], a1[U][MT], b1[U][NT];
+  auto load = [&](float4 (&a)[U][MT], float4 (&b)[U][NT], int s) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) b[u][j] = *reinterpret_cast<const float4*>(wb[j] + (size_t)(s + u) * 16);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[u][i] = *reinterpret_cast<const float4*>(xa[i] + (size_t)(s + u) * 16);
+    }
+  };
+  auto multiply = [&](const float4 (&a)[U][MT], const float4 (&b)[U][NT]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = mfma4x4(a[u][i], b[u][j], acc[i][j]);
+  };
+  if (full > 0) load(a0, b0, s0);
+  for (int t = 0; t < full; t += 2) {
+    if (t + 1 < full) load(a1, b1, s0 + (t + 1) * U);
+    multiply(a0, b0);
+    if (t + 1 >= full) break;
+    if (t + 2 < full) load(a0, b0, s0 + (t + 2) * U);
+    multiply(a1, b1);
   }
-  f32x4 acc[2][2] = {};
-#pragma unroll 2
-  for (int k = 0; k < p.K; k += 16) {
-    float4 a[2], b[2];
+  for (int s = s0 + full * U; s < s0 + n; ++s) {
+    float4 a[MT], b[NT];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      a[i] = *reinterpret_cast<const float4*>(xa[i] + k);
-      b[i] = *reinterpret_cast<const float4*>(wb[i] + k);
+    for (int j = 0; j < NT; ++j) b[j] = *reinterpret_cast<const float4*>(wb[j] + (size_t)s * 16);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a[i] = *reinterpret_cast<const float4*>(xa[i] + (size_t)s * 16);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = mfma4x4(a[i], b[j], acc[i][j]);
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) part[(w * MT * NT + i * NT + j) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  constexpr int NF = EPI == 2 ? MT * NT / 2 : MT * NT;  // (gate and up fragments finish together)
+  for (int it = threadIdx.x; it < NF * 64; it += 64 * KS) {
+    const int f = it >> 6, i = EPI == 2 ? f / (NT / 2) : f / NT, j = EPI == 2 ? 2 * (f % (NT / 2)) : f % NT;
+    f32x4 v0 = {}, v1 = {};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      v0 += part[(k * MT * NT + i * NT + j) * 64 + lane];
+      if constexpr (EPI == 2) v1 += part[(k * MT * NT + i * NT + j + 1) * 64 + lane];
+    }
+    store4<EPI>(p, m0 + 16 * i + 4 * g, EPI == 2 ? (n0 + 16 * j) / 2 + rl : n0 + 16 * j + rl, v0, v1);
+  }
+}
+
+// Bound by the f32 MFMA (157 TFLOP/s): 108 TFLOP/s at 777 x 32768 x 1024, 106 at 1024 x 2048 x 8192.
+// KW groups of 4 waves (2 x 2), 16 FM x 16 FN outputs a wave; group kw multiplies the 32-deep slices kw, kw + KW, ..
+// of K and the groups add up through LDS at the end (a second group gives every SIMD a wave to run while the other
+// one waits for its operands).  A slice in LDS: A [32 FM rows][8 chunks of 16 B], then B [32 FN rows] alike, chunk c
+// of row r at slot c ^ ((r >> 1) & 7) (a read's 16-lane groups hit distinct banks).  NS stages of KW slices, all but
+// the one being read in flight.
+template <int EPI, int FM, int FN, int KW, int NS>
+__global__ __launch_bounds__(256 * KW) void tiles_f32_kernel(GemmF32Params p) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  constexpr int BM = 32 * FM, BN = 32 * FN, SLICE = (BM + BN) * 128, STAGE = KW * SLICE;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6 & 3, kw = threadIdx.x >> 8;
+  const int rl = lane & 15, g = lane >> 4, wm = w & 1, wn = w >> 1;
+  const int mb = (p.M + BM - 1) / BM, tile = xcd_remap(blockIdx.x, gridDim.x);
+  const int m0 = tile % mb * BM, n0 = tile / mb * BN;  // (row blocks of a column block follow one another: W from L2)
+  // (rows past the end lie outside the resources: zeros)
+  const auto rsrc = [](const float* base, size_t n) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), (short)0, (int)(n * 4), 0x00020000);
+  };
+  const auto rx = rsrc(p.X + (size_t)m0 * p.ldx, (size_t)(min(BM, p.M - m0) - 1) * p.ldx + p.K);
+  const auto rw = rsrc(p.W + (size_t)n0 * p.K, (size_t)min(BN, p.N - n0) * p.K);
+  const int sr = lane >> 3;  // this lane's row of a wave instruction's 8
+  auto issue = [&](int s, char* buf) {
+    buf += kw * SLICE;
+    auto rows = [&](__amdgpu_buffer_rsrc_t r, int q, int ld, char* to) {
+      const int row = 8 * q + sr, k = (s * KW + kw) * 32 + 4 * ((lane & 7) ^ ((row >> 1) & 7));
+      const unsigned off = k < p.K ? ((unsigned)row * (unsigned)ld + (unsigned)k) * 4u : 0xFFFFFFF0u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(to + q * 1024), 16, off, 0, 0, 0);
+    };
+#pragma unroll
+    for (int it = 0; it < FM; ++it) rows(rx, it * 4 + w, p.ldx, buf);
+#pragma unroll
+    for (int it = 0; it < FN; ++it) rows(rw, it * 4 + w, p.K, buf + BM * 128);
+  };
+  f32x4 acc[FM][FN] = {};
+  const int n = (p.K + 32 * KW - 1) / (32 * KW);
+  // (stages past the last are issued too: k >= K reads nothing, and the wait stays one constant)
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) issue(s, lds + s * STAGE);
+  for (int s = 0, at = 0; s < n; ++s, at = at + 1 == NS ? 0 : at + 1) {
+    const char* buf = lds + at * STAGE + kw * SLICE;
+    // this stage landed everywhere, and every wave is done reading the one before, which the next issue overwrites
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * (FM + FN)) : "memory");
+    issue(s + NS - 1, lds + (at == 0 ? NS - 1 : at - 1) * STAGE);
+    float4 a[2][FM], b[2][FN];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int slot = ((4 * t + g) ^ (rl >> 1)) << 4;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) a[t][i] = *reinterpret_cast<const float4*>(buf + (wm * 16 * FM + 16 * i + rl) * 128 + slot);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) b[t][j] = *reinterpret_cast<const float4*>(buf + (BM + wn * 16 * FN + 16 * j + rl) * 128 + slot);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[i][j] = mfma4(a[i].x, b[j].x, acc[i][j]);
-        acc[i][j] = mfma4(a[i].y, b[j].y, acc[i][j]);
-        acc[i][j] = mfma4(a[i].z, b[j].z, acc[i][j]);
-        acc[i][j] = mfma4(a[i].w, b[j].w, acc[i][j]);
-      }
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = mfma4(reinterpret_cast<const float*>(&a[t][i])[e], reinterpret_cast<const float*>(&b[t][j])[e], acc[i][j]);
   }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (no DMA outlives its stage)
+  if constexpr (KW > 1) {
+    constexpr int GROUP = 4 * FM * FN * 64;
+    f32x4* part = reinterpret_cast<f32x4*>(lds);
+    static_assert((KW - 1) * GROUP * 16 <= NS * STAGE, "the other groups' sums fit the stages");
+    if (kw > 0) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + 16 * i + 4 * g + r;
-      if (m >= p.M) continue;
-      if constexpr (EPI == 2) {  // (the wave's two column tiles are gate and up of the same 16 features)
-        p.Y[(size_t)m * p.ldy + (n0 >> 1) + rl] = silu(acc[i][0][r]) * acc[i][1][r];
-        continue;
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = n0 + 16 * j + rl;
-        if (n >= p.N) continue;
-        float v = acc[i][j][r];
-        if constexpr (EPI == 1) v += p.R[(size_t)m * p.ldr + n];
-        if (EPI == 6 && n >= p.n_split) {
-          v = fmaxf(v, 0.f);
-          p.Y2[(size_t)m * p.ldy2 + n - p.n_split] = v * v;
-        } else {
-          p.Y[(size_t)m * p.ldy + n] = v;
-        }
-      }
+        for (int j = 0; j < FN; ++j) part[(kw - 1) * GROUP + ((w * FM + i) * FN + j) * 64 + lane] = acc[i][j];
     }
+    __syncthreads();
+    if (kw > 0) return;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int k = 0; k < KW - 1; ++k) acc[i][j] += part[k * GROUP + ((w * FM + i) * FN + j) * 64 + lane];
+  }
+  const int m = m0 + wm * 16 * FM + 4 * g, c = n0 + wn * 16 * FN;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; j += EPI == 2 ? 2 : 1)
+      store4<EPI>(p, m + 16 * i, EPI == 2 ? (c + 16 * j) / 2 + rl : c + 16 * j + rl, acc[i][j], acc[i][EPI == 2 ? j + 1 : j]);
+}
+
+template <int EPI, int MT, int NT, int KS, int U>
+void launch_rows(const GemmF32Params& p, hipStream_t st) {
+  const dim3 grid((p.N + 16 * NT - 1) / (16 * NT), (p.M + 16 * MT - 1) / (16 * MT));
+  hipLaunchKernelGGL((rows_f32_kernel<EPI, MT, NT, KS, U>), grid, dim3(64 * KS), 0, st, p);
+}
+
+template <int EPI, int KW>
+void launch_tiles(const GemmF32Params& p, hipStream_t st) {
+  constexpr int F = 2, NS = 2;
+  const int tiles = ((p.M + 32 * F - 1) / (32 * F)) * ((p.N + 32 * F - 1) / (32 * F));
+  hipLaunchKernelGGL((tiles_f32_kernel<EPI, F, F, KW, NS>), dim3(tiles), dim3(256 * KW), NS * KW * 64 * F * 128, st, p);
+}
+
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+template <int EPI>
+void launch(const GemmF32Params& p, hipStream_t st) {
+  const int64_t t64 = (int64_t)cdiv(p.M, 64) * cdiv(p.N, 64);
+  const bool fits = (int64_t)64 * p.ldx * 4 < 0x7FFFFFF0ll && (int64_t)64 * p.K * 4 < 0x7FFFFFF0ll;  // (32-bit offsets in a tile)
+  // Tiles from where about half the CUs get one (us, rows / tiles kernel): 64 x 8720 x 1024 (137 tiles) 37 / 27, 333 x 1024
+  // x 1024 (96) 24 / 23, 128 x 2048 x 2048 (64) 23 / 43.  Waves per tile so that a CU holds 16 of them (1 / 2 / 4 groups):
+  // 777 x 1024 x 6144 (208 tiles) 192 / 151 / 123, 1024 x 2048 x 8192 (512) 380 / 323 / 348, 777 x 32768 x 1024 (6656) 481 /
+  // 508 / 584; the kernel without LDS or k groups that this one replaced: 202 / 507 / 777.  (A 128 x 128 tile: 290 against
+  // 307 at 1024 x 8192 x 2048, but 545 against 481 at 777 x 32768 x 1024.)
+  if (p.M > 32 && t64 >= 120 && fits) {
+    if (t64 <= 256) return launch_tiles<EPI, 4>(p, st);
+    if (t64 <= 512) return launch_tiles<EPI, 2>(p, st);
+    return launch_tiles<EPI, 1>(p, st);
+  }
+  // two column tiles per workgroup where one would already give every CU four workgroups (and for gate / up pairs)
+  const bool two = EPI == 2 || cdiv(p.N, 16) * cdiv(p.M, 64) >= 1024;
+  if (p.M <= 16) {
+    if (two) return launch_rows<EPI, 1, 2, 8, 4>(p, st);
+    if constexpr (EPI != 2) {
+      if (cdiv(p.N, 16) <= 128 && p.K >= 2048) return launch_rows<EPI, 1, 1, 16, 4>(p, st);
+      return launch_rows<EPI, 1, 1, 8, 4>(p, st);
+    }
+  }
+  if (p.M <= 32) {
+    if (two) return launch_rows<EPI, 2, 2, 8, 2>(p, st);
+    if constexpr (EPI != 2) return launch_rows<EPI, 2, 1, 8, 4>(p, st);
+  }
+  if (two) return launch_rows<EPI, 4, 2, 8, 2>(p, st);
+  if constexpr (EPI != 2) return launch_rows<EPI, 4, 1, 8, 2>(p, st);
 }
 
 }  // namespace
@@ -80,12 +260,11 @@ extern "C" int vwa_gemm_f32(int epi, const GemmF32Params* p, hipStream_t st) {
   if (epi == 1 && !p->R) return -3;
   if (epi == 6 && (!p->Y2 || p->n_split < 0 || p->n_split > p->N)) return -4;
   if (epi == 2 && p->N % 32) return -5;
-  const dim3 grid((p->N + 63) / 64, (p->M + 63) / 64), block(256);
   switch (epi) {
-    case 0: hipLaunchKernelGGL((gemm_f32_kernel<0>), grid, block, 0, st, *p); break;
-    case 1: hipLaunchKernelGGL((gemm_f32_kernel<1>), grid, block, 0, st, *p); break;
-    case 2: hipLaunchKernelGGL((gemm_f32_kernel<2>), grid, block, 0, st, *p); break;
-    case 6: hipLaunchKernelGGL((gemm_f32_kernel<6>), grid, block, 0, st, *p); break;
+    case 0: launch<0>(*p, st); break;
+    case 1: launch<1>(*p, st); break;
+    case 2: launch<2>(*p, st); break;
+    case 6: launch<6>(*p, st); break;
     default: return -6;
   }
   return (int)hipGetLastError();

@@ -77,6 +77,33 @@ def test_linear_split_and_f32_residual(dtype, M, N, K, ns):
     assert torch.equal(rd[:, N:].cpu(), r[:, N:])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 16), (16, 1003, 2064), (17, 2080, 48), (32, 16384, 32), (64, 7713, 144),  # rows kernel
+                                   (33, 16400, 80), (65, 3904, 16),                # tiles: one / two row blocks, K short of a slice
+                                   (200, 4096, 208), (449, 2001, 4112), (641, 3296, 96)])   # 4, 2 and 1 groups of waves
+def test_gemm_f32_kernels(M, N, K):
+    """Every kernel of the dispatch at remainders of rows, columns and K, all epilogues, X rows apart.  Tolerance: each of K
+    additions rounds by 2^-24 of a partial sum, signs at random."""
+    x = torch.randn(M, K + 12, device=DEV)[:, :K]
+    w, r = torch.randn(N, K, device=DEV) * K ** -0.5, torch.randn(M, N, device=DEV)
+    y, tol = x.double() @ w.double().T, 2.0 ** -24 * max(4.0, K ** 0.5)
+    err = lambda got, want: float((got.double() - want).norm() / want.norm())  # noqa: E731
+    E = ops.ext()
+    out = torch.full((M, N + 4), 7.0, device=DEV)
+    E.gemm_f32(x, w, out[:, :N], 0, None)
+    assert err(out[:, :N], y) < tol and bool((out[:, N:] == 7).all())
+    E.gemm_f32(x, w, out[:, :N], 1, r)
+    assert err(out[:, :N] - r, y) < tol + 4e-7 and bool((out[:, N:] == 7).all())
+    a, b = torch.empty(M, N // 3, device=DEV), torch.empty(M, N - N // 3, device=DEV)
+    if N > 2:
+        E.gemm_f32(x, w, a, 6, None, b)
+        assert err(a, y[:, : N // 3]) < tol and err(b, y[:, N // 3 :].clamp_min(0) ** 2) < 3 * tol
+    if N % 32 == 0:
+        h = torch.empty(M, N // 2, device=DEV)
+        E.gemm_f32(x, w, h, 2, None)
+        q = y.view(M, N // 32, 2, 16)
+        assert err(h, (torch.nn.functional.silu(q[:, :, 0]) * q[:, :, 1]).reshape(M, N // 2)) < 4 * tol + 4e-7
+
+
 # ----------------------------------------------------------------------------- cache + rotation
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,G,dk,dv,rot", [(6, 2, 32, 48, 12), (4, 4, 64, 16, 64), (3, 1, 128, 112, 32)])
