@@ -317,3 +317,54 @@ def test_rms_statistics_handoff_paths_without_the_tiled_gemm():
     a = ops.linear_swiglu(out, gu, fuse_rms=True, eps=1e-5, ss_in=ss[0])
     b = ops.linear_swiglu(out, gu, fuse_rms=True, eps=1e-5)
     assert torch.equal(a, b)
+
+
+def test_no_collection_inside_a_capture(monkeypatch):
+    """A dropped object in a reference cycle (as an engine with its graphs is) is not collected while a graph is captured,
+    on whichever thread, and is afterwards."""
+    import contextlib
+    import gc
+    import threading
+    import weakref
+
+    from voice_enabled_browser_automation_amd.utils import capture
+
+    monkeypatch.setattr(capture.torch.cuda, "graph", lambda g, **kw: contextlib.nullcontext())
+
+    class Cycle:
+        def __init__(self):
+            self.me = self
+
+    was, old = gc.isenabled(), gc.get_threshold()
+    gc.enable()
+    try:
+        gc.set_threshold(10, 1, 1)
+        inner, outer = threading.Event(), threading.Event()
+
+        def other():
+            with capture.capture_graph(None):
+                inner.set()
+                outer.wait(10)
+
+        t = threading.Thread(target=other)
+        with capture.capture_graph(None):
+            gone = weakref.ref(Cycle())
+            t.start()
+            assert inner.wait(10)
+            keep = [[] for _ in range(2000)]
+            assert gone() is not None and not gc.isenabled()
+        keep += [[] for _ in range(2000)]
+        assert gone() is not None and not gc.isenabled()  # the other thread's capture goes on
+        outer.set()
+        t.join()
+        assert gc.isenabled()
+        keep += [[] for _ in range(2000)]
+        assert gone() is None
+        with pytest.raises(ValueError):
+            with capture.capture_graph(None):
+                raise ValueError
+        assert gc.isenabled()
+    finally:
+        gc.set_threshold(*old)
+        if not was:
+            gc.disable()

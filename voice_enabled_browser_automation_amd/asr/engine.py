@@ -17,6 +17,7 @@ import torch
 
 from .. import ops
 from ..models.whisper import WhisperModel
+from ..utils.capture import capture_graph
 
 BUCKETS = (1, 2, 4, 8, 16, 32, 64)
 
@@ -110,7 +111,7 @@ class WhisperRunner:
         g = torch.cuda.CUDAGraph()
         if self.pool is None:
             self.pool = torch.cuda.graph_pool_handle()
-        with torch.cuda.graph(g, pool=self.pool):
+        with capture_graph(g, pool=self.pool):
             out = self._fwd(M)
         self.graphs[M] = (g, out)
         return self.graphs[M]
@@ -238,7 +239,7 @@ class AsrEngine:
             g = torch.cuda.CUDAGraph()
             if r.pool is None:
                 r.pool = torch.cuda.graph_pool_handle()
-            with torch.cuda.graph(g, pool=r.pool):
+            with capture_graph(g, pool=r.pool):
                 for _ in range(steps):  # identical steps: each reads what the previous advanced
                     self._loop_step(slot, allow_eot)
             self.loop_graphs[key] = g

@@ -30,6 +30,7 @@ import torch
 
 from .. import ops
 from .kv_cache import BlockManager, PagedKVCache
+from ..utils.capture import capture_graph
 from ..utils.env import knob
 
 # Row buckets of the captured step graphs (VWA_ROW_BUCKETS overrides).  48 between the powers of
@@ -347,7 +348,7 @@ class LLMEngine:
         g = torch.cuda.CUDAGraph()
         if self.graph_pool is None:
             self.graph_pool = torch.cuda.graph_pool_handle()
-        with torch.cuda.graph(g, pool=self.graph_pool):
+        with capture_graph(g, pool=self.graph_pool):
             out = self._forward_rows(M, L, upload_meta=True)
         self.graphs[(M, L, self._gated)] = (g, out)
         return self.graphs[(M, L, self._gated)]
