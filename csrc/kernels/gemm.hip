@@ -12,16 +12,13 @@
 //     i.e. exactly the MFMA B fragments: the block is copied to LDS verbatim;
 //   * row-major [N, K] (Whisper weights, tests): each 16-byte piece is scattered into the same
 //     fragment-ordered LDS image while staging.
-// Because the B fragments use the k order 32 g + 8 s + e, the A fragment of lane (row r, g) in
-// sub-step s is X[r][128 kg + 32 g + 8 s .. + 8): 16-byte chunk 4 g + s of the row's k-group.
+// Which k of a k-group a stage takes, and in which order, follows from the X rows' cache lines (swzk below).
 //
-// Tiling (gfx950, wave64): workgroup = 4 waves (2 x 2) computing a 128 x 128 output tile, one
-// k-group (128 deep) per stage: A [128 rows][128 k] (32 KB, chunk-XOR swizzled: 16 lanes reading
-// one chunk column of 16 rows hit 16 distinct 16-B slots -> conflict-free ds_read_b128) and B
-// [8 tiles][4 s][64 lanes][8] (32 KB, fragment order -> every ds_read_b128 is 1 KB contiguous).
-// Each wave owns 64 x 64 = 4 x 4 MFMA tiles (mfma_f32_16x16x32_bf16, 64 MFMAs per stage).
-// Software pipeline: the next stage's global loads are issued into registers before this
-// stage's MFMAs, written to LDS after them (one LDS buffer, 64 KB -> 2 workgroups per CU).
+// Tiling (gfx950, wave64), 128 x 128: workgroup = 4 waves (2 x 2), half a k-group (64 deep) per stage: A [128 rows][64
+// k] (16 KB, chunk-XOR swizzled: conflict-free ds_read_b128) and B [8 tiles][2 MFMAs][64 lanes][8] (16 KB, fragment
+// order -> every ds_read_b128 is 1 KB contiguous).  Each wave owns 64 x 64 = 4 x 4 MFMA tiles
+// (mfma_f32_16x16x32_bf16, 32 MFMAs per stage).  Two stages in LDS (64 KB -> 2 workgroups per CU), filled by LDS-DMA one
+// stage ahead.  256 x 256 (CfgP8): below.
 // Grid: (row blocks x column blocks) remapped XCD-aware so the row blocks of one column block
 // (same weight tile) share an XCD's L2, x split-K slices when the tile count alone cannot
 // fill the 256 CUs (weight-streaming shapes: few rows) -- slices write f32 partials, a second
@@ -87,6 +84,17 @@ using CfgW8 = Cfg<64, 128, 1, 4>;
 // (the other column of the group) cannot collide.  (Plain c ^ h measured 33 % bank conflicts.)
 VWA_DEVICE int swz(int h) { return (0x64753120 >> (4 * h)) & 7; }
 
+// bf16 stages: half hs & 1 = h of a k-group is k 64 h .. 64 h + 64, a whole 128-byte line of every X row.  In the tiled
+// weight's order (lane group g of substep s: k 32 g + 8 s) that is the groups g = 2 h, 2 h + 1 of all four substeps: MFMA
+// sp of the half takes, in lane group g, substep 2 sp + (g >> 1) of group 2 h + (g & 1) -- k 64 h + 32 (g & 1) + 16 sp +
+// 8 (g >> 1), chunk 4 (g & 1) + 2 sp + (g >> 1) of the X row's line.  (Substeps 2 h, 2 h + 1 of all groups took 32 of every
+// 64 bytes of two lines per row, each line twice, 1.5 times the bytes through L1: 128^2 tile 12000 x 1280 x 1280 583 ->
+// 646 TFLOP/s, 1500 x 5120 x 1280 532 -> 594.)
+// A read's 16-lane groups now hold chunks c and c ^ 4 of complementary half rows {0,1,6,7}, {2,3,4,5}: swzk maps both
+// halves to 0..3.
+VWA_DEVICE int swzk(int h) { return (h & 1) | (h >> 2 << 1); }
+VWA_DEVICE int chunk_of(int g, int sp) { return 4 * (g & 1) + 2 * sp + (g >> 1); }
+
 // buffer resource over [base, base + bytes): loads past the end return zero (rows >= M, weight
 // tiles >= N), so the stage issue needs no bounds branches
 VWA_DEVICE __amdgpu_buffer_rsrc_t rsrc(const void* base, size_t bytes) {
@@ -99,13 +107,12 @@ VWA_DEVICE void dma16(__amdgpu_buffer_rsrc_t r, char* lds_wave_base, unsigned vo
                                            0);
 }
 
-// Stage hs of the block's tile (bf16: half k-group hs = 2 kg + h, k = 128 kg + 32 g + 16 h + 8 s'
-// + e, s' = 0, 1), LDS-DMA'd straight into buffer `buf` (no registers): 8 wave-instructions of
-// 1 KB per thread.  Each wave-instruction's LDS destination is lane-linear (base + 16 lane), so
-// the A swizzle is applied on the per-lane SOURCE address (and undone on the read):
-//   A image [BM rows][8 chunks of 16 B], chunk c = 2 g + s' at slot c ^ swz((row >> 1) & 7)
-//   B image [BN/16 tiles][2 s'][64 lanes][16 B]: the tiled weight's fragment blocks verbatim (a
-//     row-major weight gathers each lane's fragment from its row instead)
+// Stage hs of the block's tile (bf16: half h of k-group kg, hs = 2 kg + h, see swzk), LDS-DMA'd
+// straight into buffer `buf` (no registers): 8 wave-instructions of 1 KB per thread.  Each
+// wave-instruction's LDS destination is lane-linear (base + 16 lane), so the A swizzle is applied on
+// the per-lane SOURCE address (and undone on the read):
+//   A image [BM rows][8 chunks of 16 B], chunk c at slot c ^ swzk((row >> 1) & 7)
+//   B image [BN/16 tiles][2 sp][64 lanes][16 B]: the lane's fragment of MFMA sp
 // F8 (W8A8): one FULL k-group per stage (16 fp8 = 16 B per chunk): A chunk c = 2 g + s2 holds
 // X8[row][128 kg + 32 g + 16 s2 .. + 16), B the fp8 tiled block [s2][lane][16 B] of the tile
 // (ops.tile_weight_fp8) -- the same stage images as a bf16 half k-group.
@@ -125,13 +132,15 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
 #pragma unroll
   for (int it = 0; it < C::BM / 8 / C::NW; ++it) {
     const int q = it * C::NW + w;  // wave-instruction index: rows 8q .. 8q + 7
-    const int r = 8 * q + (lane >> 3), c = (lane & 7) ^ swz((r >> 1) & 7);
+    const int r = 8 * q + (lane >> 3), c = (lane & 7) ^ (F8 || W8 ? swz((r >> 1) & 7) : swzk((r >> 1) & 7));
     const int m = GRP ? rows[it] : bm + r;
     unsigned off;
     if constexpr (F8)
       off = (unsigned)((size_t)m * p.ldx + (size_t)kg * BKG + 32 * (c >> 1) + 16 * (c & 1));
-    else
+    else if constexpr (W8)  // (the fp8 tiled order: k 32 g + 16 ha + 8 sp)
       off = (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 32 * (c >> 1) + 16 * ha + 8 * (c & 1)) * 2);
+    else
+      off = (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 64 * ha + 8 * c) * 2);
     dma16(rx, buf + hh * C::A_BYTES + q * 1024, (GRP ? m >= 0 : m < p.M) ? off : 0xFFFFFFF0u);
   }
   }
@@ -156,10 +165,11 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
       off = T * 16 < p.N ? (unsigned)(((size_t)T * kgn + kg) * 2048 + sp * 1024 + lane * 16) : 0xFFFFFFF0u;
     } else if constexpr (WT) {
       const int T = (bn >> 4) + tile;
-      off = T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + (2 * h + sp) * 512 + lane * 8) * 2) : 0xFFFFFFF0u;
+      off = T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + (2 * sp + (lane >> 5)) * 512 + h * 256 + (lane & 31) * 8) * 2)
+                         : 0xFFFFFFF0u;
     } else {
       const int n = bn + tile * 16 + (lane & 15), g = lane >> 4;
-      off = n < p.N ? (unsigned)(((size_t)n * p.K + (size_t)kg * BKG + 32 * g + 16 * h + 8 * sp) * 2) : 0xFFFFFFF0u;
+      off = n < p.N ? (unsigned)(((size_t)n * p.K + (size_t)kg * BKG + 64 * h + 8 * chunk_of(g, sp)) * 2) : 0xFFFFFFF0u;
     }
     dma16(rw, buf + C::A_BYTES + q * 1024, off);
   }
@@ -231,7 +241,7 @@ VWA_DEVICE void compute_stage(const char* buf, f32x4 (&acc)[C::FM][C::FN], int w
 #pragma unroll
     for (int sp = 0; sp < 2; ++sp) {
       bf16x8 a[C::FM], b[C::FN];
-      const int ch = ((2 * g + sp) ^ swz(rl >> 1)) << 4;  // ((row >> 1) & 7) == rl >> 1 for every fragment row
+      const int ch = (chunk_of(g, sp) ^ swzk(rl >> 1)) << 4;  // ((row >> 1) & 7) == rl >> 1 for every fragment row
 #pragma unroll
       for (int i = 0; i < C::FM; ++i) a[i] = *reinterpret_cast<const bf16x8*>(la + i * 16 * 128 + ch);
 #pragma unroll
@@ -244,63 +254,46 @@ VWA_DEVICE void compute_stage(const char* buf, f32x4 (&acc)[C::FM][C::FN], int w
   }
 }
 
-// ---- 256 x 256 tile, 8 waves (2 x 4, each 128 x 64), 8-phase software pipeline (the guide's
-// "256^2 8-phase template": the 128^2 two-barrier loop above is capped near 900 TF/s because each
-// stage's DMA is drained by the barrier that publishes it).  A stage (one bf16 half k-group, 64
-// deep) is four half-tile images of 16 KB -- A-lo (rows 0-127), A-hi (rows 128-255), B-lo
-// (n-tiles 0-7), B-hi (8-15) -- in the same layouts as the 128^2 kernel.  Each stage runs 4
-// phases of 16 MFMAs per wave (one C quadrant: 4 row x 2 column fragments x 2 k-substeps):
-//   P0 reads A 0-3 + B 0-1, P1 B 2-3, P2 A 4-7, P3 B 0-1 (A stays in registers across P0/P1 and
-//   P2/P3), with the next stages' half-tiles DMA'd behind them: P0 A-hi + B-lo and P1 B-hi of
-//   stage s+1 (into the other buffer, free since the end of stage s-1), P3 A-lo of stage s+2
-//   (into this buffer: its A halves were last read in P2).  The only wait on the DMA is a counted
-//   vmcnt in P3 (A-lo of s+2 stays in flight).  The two wave groups (M halves) run one barrier
-//   apart, so one group's LDS reads overlap the other group's MFMAs; every phase retires its reads
-//   (lgkmcnt) before its first barrier, so a restage issued after that barrier by the other group
-//   cannot overwrite bytes still being read, and every staged byte is read after a barrier that
-//   follows every issuing wave's counted wait.
-constexpr int kP8Half = 16384;
+// ---- 256 x 256 tile, 8 waves (2 x 4, each 128 x 64).  A stage (one bf16 half k-group, 64 deep) is four half-tile
+// images of 16 KB -- A-lo (rows 0-63 and 128-191: the first half of either M half), A-hi (the other rows), B-lo (n-tiles
+// 0-7), B-hi (8-15) -- in the same layouts as the 128^2 kernel, and runs as two phases of 32 MFMAs per wave: A reads all
+// of the wave's B fragments and its four fragments of A-lo, B those of A-hi (the B fragments stay in registers).  A phase is operand reads and DMA issue; waits;
+// barrier; MFMAs; barrier -- and the two wave groups (M halves) run one barrier apart, so that one group's reads overlap
+// the other group's MFMAs.  What bounds it is the time a phase adds to its MFMAs (barriers, the tail of the LDS reads):
+// with four phases of 16 MFMAs and the DMA addresses computed per stage the matrix cores were busy 58 % of 4096 x 8192 x
+// 8192.
+//   DMA: the halves of a buffer are refilled as they fall free, two stages ahead: A-lo, B-lo and B-hi of stage s + 2 in
+//   phase B of stage s (all read in phase A), A-hi of stage s + 1 in phase A of stage s (read in phase B of s - 1); the
+//   two wave instructions of a half-tile need no vector address math (the stage is the scalar offset).  Each phase waits
+//   until 8 instructions are left, which covers what the next phase reads: both groups have passed that wait by the
+//   barrier after which the first of them reads it.  A group's reads are retired (lgkmcnt) before the barrier that lets
+//   the other one refill what they read.
+// Measured (TFLOP/s, four phases with 32-byte X pieces -> two phases -> whole lines): 4096 x 8192 x 8192 1194 -> 1297 ->
+// 1425, 2048 x 4096 x 22528 1106 -> 1226 -> 1329, 1011 x 28672 x 4096 SwiGLU 1020 -> 1217 -> 1244.
 using CfgP8 = Cfg<256, 256, 2, 4>;
 
-// half-tile `which` (0 A-lo, 1 A-hi, 2 B-lo, 3 B-hi) of stage hs into the stage image `st`:
-// 16 wave-instructions of 1 KB = 2 per wave (tiled bf16 weights only)
-// (rows: as issue_stage)
-template <bool GRP>
-VWA_DEVICE void p8_issue(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __amdgpu_buffer_rsrc_t rw, int bm, int bn,
-                         int hs, int which, char* st, const int (&rows)[4]) {
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int kg = hs >> 1, h = hs & 1;
-  const int kgn = p.K / BKG;
+// half-tile `which` (0 A-lo, 1 A-hi, 2 B-lo, 3 B-hi) into the stage image `st`: 16 wave-instructions of 1 KB, 2 per
+// wave, from the byte offsets voff (past the resource: zeros) + soff
+VWA_DEVICE void p8_issue(__amdgpu_buffer_rsrc_t r, const unsigned (&voff)[8], unsigned soff, int which, char* st) {
+  const int w = threadIdx.x >> 6;
 #pragma unroll
   for (int it = 0; it < 2; ++it) {
-    const int q = it * 8 + w;
-    if (which < 2) {
-      const int qa = 16 * which + q;  // rows 8 qa .. 8 qa + 7
-      const int r = 8 * qa + (lane >> 3), c = (lane & 7) ^ swz((r >> 1) & 7);
-      const int m = GRP ? rows[2 * which + it] : bm + r;
-      const unsigned off =
-          (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 32 * (c >> 1) + 16 * h + 8 * (c & 1)) * 2);
-      dma16(rx, st + qa * 1024, (GRP ? m >= 0 : m < p.M) ? off : 0xFFFFFFF0u);
-    } else {
-      const int tile = 8 * (which - 2) + (q >> 1), sp = q & 1;
-      const int T = (bn >> 4) + tile;
-      const unsigned off =
-          T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + (2 * h + sp) * 512 + lane * 8) * 2) : 0xFFFFFFF0u;
-      dma16(rw, st + CfgP8::A_BYTES + (2 * tile + sp) * 1024, off);
-    }
+    const int i = which < 2 ? 2 * it + which : 2 * which + it;
+    char* to = st + (which < 2 ? (8 * i + w) * 1024 : CfgP8::A_BYTES + (8 * (i - 4) + w) * 1024);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)to, 16, voff[i], soff, 0, 0);
   }
 }
 
-// one phase: 16 MFMAs acc[i0 .. i0+3][j0 .. j0+1] over both k-substeps of the stage
-template <int I0, int J0>
-VWA_DEVICE void p8_mfma(f32x4 (&acc)[8][4], const bf16x8 (&a)[4][2], const bf16x8 (&b)[2][2]) {
+// one phase: 32 MFMAs, acc[i0 .. i0+3][0 .. 3] over both k-substeps of the stage
+template <int I0>
+VWA_DEVICE void p8_mfma(f32x4 (&acc)[8][4], const bf16x8 (&a)[4][2], const bf16x8 (&b)[4][2]) {
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[I0 + i][J0 + j] = mfma16(a[i][sp], b[j][sp], acc[I0 + i][J0 + j]);
+      for (int j = 0; j < 4; ++j) acc[I0 + i][j] = mfma16(a[i][sp], b[j][sp], acc[I0 + i][j]);
   __builtin_amdgcn_s_setprio(0);
 }
 
@@ -579,20 +572,40 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
                 "8 LDS-DMA instructions per thread per stage (the counted vmcnt)");
   const int h0 = SPG * kg0, nh = SPG * (kg1 - kg0);
   // X extent: the last row starts at (M-1)*ldx and is K long (rows may overlap: conv views)
-  const __amdgpu_buffer_rsrc_t rx = rsrc(p.X, ((GRP ? x_rows - 1 : (size_t)(p.M - 1)) * p.ldx + p.K) * (F8 ? 1 : 2));
-  const __amdgpu_buffer_rsrc_t rw = rsrc(p.W, (size_t)p.N * p.K * (F8 || W8 ? 1 : 2));
+  const size_t x_bytes = ((GRP ? x_rows - 1 : (size_t)(p.M - 1)) * p.ldx + p.K) * (F8 ? 1 : 2);
+  const size_t w_bytes = (size_t)p.N * p.K * (F8 || W8 ? 1 : 2);
+  const __amdgpu_buffer_rsrc_t rx = rsrc(p.X, x_bytes), rw = rsrc(p.W, w_bytes);
   if constexpr (P8) {
-    static_assert(C::BM == 256 && C::BN == 256 && C::NW == 8 && WT && !F8, "8-phase pipeline: CfgP8, tiled bf16");
+    static_assert(C::BM == 256 && C::BN == 256 && C::NW == 8 && WT && !F8, "two-phase pipeline: CfgP8, tiled bf16");
     const int l = lane_id(), rl = l & 15, g = l >> 4;
     auto stage = [&](int s) { return lds + (s & 1) * C::STAGE; };
-    if (nh > 0) {
+    unsigned voff[8];  // this lane's pieces of the half-tiles (k-group 0)
 #pragma unroll
-      for (int hq = 0; hq < 4; ++hq) p8_issue<GRP>(p, rx, rw, bm, bn, h0, hq, stage(0), rows);
+    for (int it = 0; it < 4; ++it) {
+      const int q = it * 8 + w, r = 8 * q + (l >> 3), c = (l & 7) ^ swzk((r >> 1) & 7);  // A rows 8 q .. 8 q + 7
+      const int m = GRP ? rows[it] : bm + r;
+      voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)(((size_t)m * p.ldx + 8 * c) * 2) : 0xFFFFFFF0u;
+      const int T = (bn >> 4) + (q >> 1);                                                // B n-tile q / 2, MFMA q & 1
+      voff[4 + it] = T * 16 < p.N ? (unsigned)(((size_t)T * KG * 2048 + (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8) * 2) : 0xFFFFFFF0u;
     }
-    if (nh > 1) p8_issue<GRP>(p, rx, rw, bm, bn, h0 + 1, 0, stage(1), rows);
-    if (nh > 1) asm volatile("s_waitcnt vmcnt(2)\n\ts_barrier" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    bf16x8 a[4][2], b[2][2];
+    // (stages past the last are issued too, on empty resources: the waits stay one constant)
+    auto issue = [&](int s, int which) {
+      const int hs = h0 + s, kg = hs >> 1, h = hs & 1;
+      const bool in = s < nh;
+      if (which < 2)
+        p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, (kg * BKG + 64 * h) * 2, which, stage(s));
+      else
+        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (kg * 2048 + h * 256) * 2, which, stage(s));
+    };
+    issue(0, 0);
+    issue(0, 2);
+    issue(0, 3);
+    issue(0, 1);
+    issue(1, 0);
+    issue(1, 2);
+    issue(1, 3);
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");
+    bf16x8 a[4][2], b[4][2];
     if (wm == 1) asm volatile("s_barrier" ::: "memory");  // group 1 runs one barrier behind group 0
     for (int s = 0; s < nh; ++s) {
       const char* st = stage(s);
@@ -600,62 +613,34 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       const char* lb = st + C::A_BYTES + (wn * 4) * 2048 + l * 16;
       auto read_a = [&](int i0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
-          for (int sp = 0; sp < 2; ++sp)
-            a[i][sp] = *reinterpret_cast<const bf16x8*>(la + (i0 + i) * 16 * 128 + (((2 * g + sp) ^ swz(rl >> 1)) << 4));
+          for (int i = 0; i < 4; ++i)
+            a[i][sp] = *reinterpret_cast<const bf16x8*>(la + (i0 + i) * 16 * 128 + ((chunk_of(g, sp) ^ swzk(rl >> 1)) << 4));
       };
-      auto read_b = [&](int j0) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+      for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
-          for (int sp = 0; sp < 2; ++sp) b[j][sp] = *reinterpret_cast<const bf16x8*>(lb + (j0 + j) * 2048 + sp * 1024);
-      };
-      const bool n1 = s + 1 < nh, n2 = s + 2 < nh;
-      // phase = operand reads (+ DMA issue) ; lgkmcnt(0) ; barrier ; 16 MFMAs ; barrier.  The two
-      // wave groups (wm) run one barrier apart, so one group's reads overlap the other's MFMAs, and
-      // a buffer's reads are retired (lgkmcnt) before the barrier that lets the other group restage it
-      // P0
+        for (int j = 0; j < 4; ++j) b[j][sp] = *reinterpret_cast<const bf16x8*>(lb + j * 2048 + sp * 1024);
       read_a(0);
-      read_b(0);
-      if (n1) {
-        p8_issue<GRP>(p, rx, rw, bm, bn, h0 + s + 1, 1, stage(s + 1), rows);
-        p8_issue<GRP>(p, rx, rw, bm, bn, h0 + s + 1, 2, stage(s + 1), rows);
-      }
+      issue(s + 1, 1);
       __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      p8_mfma<0, 0>(acc, a, b);
+      asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      p8_mfma<0>(acc, a, b);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_barrier" ::: "memory");
-      // P1
-      read_b(2);
-      if (n1) p8_issue<GRP>(p, rx, rw, bm, bn, h0 + s + 1, 3, stage(s + 1), rows);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      p8_mfma<0, 2>(acc, a, b);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_barrier" ::: "memory");
-      // P2
       read_a(4);
+      issue(s + 2, 0);
+      issue(s + 2, 2);
+      issue(s + 2, 3);
       __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      p8_mfma<4, 2>(acc, a, b);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("s_barrier" ::: "memory");
-      // P3 (A-lo of this buffer was last read in P2: restage it with stage s + 2).  Stage s + 1 has
-      // landed for this wave (only A-lo of s + 2 may stay in flight) before this phase's first
-      // barrier; with the groups a barrier apart every wave has waited by the barrier that ends the
-      // phase, and the next stage is read only after it
-      read_b(0);
-      if (n2) p8_issue<GRP>(p, rx, rw, bm, bn, h0 + s + 2, 0, stage(s + 2), rows);
-      __builtin_amdgcn_sched_barrier(0);
-      if (n2) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      p8_mfma<4, 0>(acc, a, b);
+      asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      p8_mfma<4>(acc, a, b);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_barrier" ::: "memory");
     }
     if (wm == 0) asm volatile("s_barrier" ::: "memory");  // (group 1 started one barrier later)
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // (the epilogue reuses the LDS)
   } else {
   if (nh > 0) issue_stage<C, WT, F8, W8, GRP>(p, rx, rw, bm, bn, h0, lds, rows);
   if (nh > 1) issue_stage<C, WT, F8, W8, GRP>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
