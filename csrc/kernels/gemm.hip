@@ -576,7 +576,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   const size_t w_bytes = (size_t)p.N * p.K * (F8 || W8 ? 1 : 2);
   const __amdgpu_buffer_rsrc_t rx = rsrc(p.X, x_bytes), rw = rsrc(p.W, w_bytes);
   if constexpr (P8) {
-    static_assert(C::BM == 256 && C::BN == 256 && C::NW == 8 && WT && !F8, "two-phase pipeline: CfgP8, tiled bf16");
+    static_assert(C::BM == 256 && C::BN == 256 && C::NW == 8 && !F8, "two-phase pipeline: CfgP8, bf16");
     const int l = lane_id(), rl = l & 15, g = l >> 4;
     auto stage = [&](int s) { return lds + (s & 1) * C::STAGE; };
     unsigned voff[8];  // this lane's pieces of the half-tiles (k-group 0)
@@ -586,7 +586,9 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       const int m = GRP ? rows[it] : bm + r;
       voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)(((size_t)m * p.ldx + 8 * c) * 2) : 0xFFFFFFF0u;
       const int T = (bn >> 4) + (q >> 1);                                                // B n-tile q / 2, MFMA q & 1
-      voff[4 + it] = T * 16 < p.N ? (unsigned)(((size_t)T * KG * 2048 + (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8) * 2) : 0xFFFFFFF0u;
+      const size_t at = WT ? (size_t)T * KG * 2048 + (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8
+                           : (size_t)(T * 16 + rl) * p.K + 8 * chunk_of(g, q & 1);
+      voff[4 + it] = T * 16 < p.N ? (unsigned)(at * 2) : 0xFFFFFFF0u;
     }
     // (stages past the last are issued too, on empty resources: the waits stay one constant)
     auto issue = [&](int s, int which) {
@@ -595,7 +597,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       if (which < 2)
         p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, (kg * BKG + 64 * h) * 2, which, stage(s));
       else
-        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (kg * 2048 + h * 256) * 2, which, stage(s));
+        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (WT ? kg * 2048 + h * 256 : kg * BKG + 64 * h) * 2, which, stage(s));
     };
     issue(0, 0);
     issue(0, 2);
@@ -848,19 +850,57 @@ int launch_cfg(const GemmParams& p, hipStream_t st) {
   return 0;
 }
 
-int g_p8_mode = 2;  // 0: never, 1: every eligible shape, 2: the measured rule (p8_auto)
+int g_p8_mode = 2;       // 0: the 128^2 kernel only, 1: the 256^2 one for every shape it was made for, 2: plan()
+int g_split_fill_pct = 0;  // > 0: vwa_gemm_splits' fill, and no plan() for the 128^2 kernel's splits
 
-// Shapes the 8-phase 256^2 kernel takes: tiled bf16 weights, N % 256, one batch
-bool p8_eligible(const GemmParams& p) {
-  return p.w_tiled && !p.sw && p.N % 256 == 0 && p.nbatch <= 1 && p.M >= 256;
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// Tile and K slices of a bf16 product of >= 128 rows: the cheapest by an estimate in us, fitted to 180 shapes (130 .. 12000
+// rows, 384 .. 28672 columns, K 384 .. 14336; both tiles, 1 .. 16 slices): 9 % off (rms of the logarithm), and 1.4 % slower than the
+// best choice of each shape, where the rules before (256^2 from 256 tiles or from slices of >= 2048 k that fill the CUs;
+// slices in powers of two until 75 % of the CUs have a tile) were 12 %: 12000 x 1280 x 5120 (235 large tiles) 165 -> 115 us,
+// 768 x 4096 x 14336 155 -> 86, 512 x 28672 x 4096 132 -> 93, 1863 x 6144 x 4096 115 -> 83.
+//   a round of the CUs costs so much per k-group and so much to start and store; a part of a last round 70 % and its share;
+//   128^2 tiles run two to a CU, one alone is faster; the slices' f32 partials are written and read.
+struct Plan {
+  bool p8;
+  int splits;
+};
+Plan plan(const GemmParams& p) {
+  const int KG = p.K / BKG;
+  Plan best{false, 1};
+  float least = 0.f;
+  for (const int s0 : {1, 2, 3, 4, 6, 8, 12, 16}) {
+    if (s0 > 1 && (s0 > KG || !p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
+    const int kg = cdiv(KG, s0), s = cdiv(KG, kg);
+    const float sum = s > 1 ? 4.f + (float)s * p.M * p.N * 4.f / 3.55e6f : 0.f;
+    for (const bool p8 : {true, false}) {
+      const int b = p8 ? 256 : 128;
+      const int64_t t = (int64_t)cdiv(p.M, b) * cdiv(p.N, b) * s;
+      const bool alone = !p8 && t <= p.cus;
+      const float r = (float)t / (p8 || alone ? p.cus : 2 * p.cus), whole = floorf(r);
+      const float rounds = r <= 1.f ? 1.f : r > whole ? whole + 0.7f + 0.3f * (r - whole) : whole;
+      const float per = p8 ? 2.0f : alone ? 1.27f : r >= 1.f ? 1.84f : 1.27f + 0.57f * (2.f * r - 1.f);
+      const float us = rounds * (kg * per + (p8 ? 5.6f : 2.3f)) + sum;
+      if (least == 0.f || us < least) {
+        least = us;
+        best = {p8, s0};
+      }
+    }
+  }
+  return best;
 }
 
 template <int EPI>
 int launch_epi(const GemmParams& p, hipStream_t st, bool p8) {
   if (p8) {
-    const int tiles = ((p.M + 255) / 256) * (p.N / 256);
-    hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
-                       CfgP8::LDS, st, p);
+    const int tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
+    if (p.w_tiled)
+      hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
+                         CfgP8::LDS, st, p);
+    else
+      hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, false, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
+                         CfgP8::LDS, st, p);
   } else if (p.sw && !p.sx) {  // W8A16
     using C = CfgW8;
     const int tiles = ((p.M + C::BM - 1) / C::BM) * ((p.N + C::BN - 1) / C::BN);
@@ -891,8 +931,7 @@ int launch_grouped(const GemmParams& p, hipStream_t st) {
 // Split while the workgroups cover less than this % of the CUs (0: per-dtype default).  Measured
 // on the Llama-3-8B decode steps of 32 / 64 rows (tools/rows_sweep.py, profiles/r4_gemm_ab.md):
 // bf16 75 % (5.08 / 5.69 ms vs 5.21 / 6.08 at 100 %), fp8 100 % (4.42 / 5.03 vs 4.62 / 5.06 at 75 %).
-int g_split_fill_pct = 0;
-
+// (bf16 products of >= 128 rows: plan())
 extern "C" int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, int f8) {
   const int tiles = ((M + CfgS::BM - 1) / CfgS::BM) * ((N + CfgS::BN - 1) / CfgS::BN);
   const int KG = K / BKG;
@@ -922,20 +961,18 @@ extern "C" int vwa_gemm(int epi, const GemmParams* pp, hipStream_t st) {
                            (reinterpret_cast<uintptr_t>(p.Y2) & 15)))
     return -19;
   if (p.splits < 1) p.splits = 1;
-  // 8-phase 256^2 kernel (mode 2, measured rule, tools/bench_gemm.py): the prompt-sized shapes
-  // whose 256^2 tiles alone fill the CUs (>= 256 tiles, e.g. the 1011-row gate/up), or fill them
-  // with split-K slices of >= 2048 K each (the 1011-row down projection, K = 14336: 4 slices,
-  // 118.5 vs 140.4 us on the 128^2 kernel and 122.5 for hipBLASLt; shorter slices lose to the
-  // f32 partial traffic: o / QKV at K = 4096 58 / 92 vs 45 / 60 us).  Mode 1: every eligible shape.
   bool p8 = false;
-  if (g_p8_mode && p8_eligible(p)) {
-    const int tiles8 = ((p.M + 255) / 256) * (p.N / 256);
-    int s = 1;
-    const int KGs = p.K / BKG;
-    while (p.ws && tiles8 * s < p.cus && s * 2 <= KGs && (int64_t)(s * 2) * p.M * p.N <= p.ws_cap) s *= 2;
-    if (g_p8_mode == 1 || tiles8 >= 256 || (p.cus > 0 && tiles8 * s >= p.cus && p.K / s >= 2048)) {
+  if (!p.sw && p.nbatch <= 1 && p.cus > 0) {
+    if (g_p8_mode == 1 && p.w_tiled && p.N % 256 == 0 && p.M >= 256) {
+      const int tiles8 = cdiv(p.M, 256) * (p.N / 256);
       p8 = true;
-      p.splits = s;
+      p.splits = 1;
+      while (p.ws && tiles8 * p.splits < p.cus && p.splits * 2 <= p.K / BKG && (int64_t)p.splits * 2 * p.M * p.N <= p.ws_cap)
+        p.splits *= 2;
+    } else if (g_p8_mode == 2 && g_split_fill_pct == 0 && p.M >= 128) {
+      const Plan pl = plan(p);
+      p8 = pl.p8;
+      p.splits = pl.splits;
     }
   }
   const int KG = p.K / BKG;

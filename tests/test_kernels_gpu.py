@@ -681,6 +681,27 @@ def test_gemm_8phase_256_tile(M):
         E.gemm_set_p8(2)
 
 
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("M,N,K", [(128, 400, 4096), (130, 28688, 128), (300, 4096, 14336), (1011, 6144, 256), (1500, 3856, 1280),
+                                   (2049, 1296, 384), (6000, 2048, 1280)])
+def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
+    """What the plan of 128 and more rows picks -- either tile, both weight layouts, partial last blocks of rows and columns, one
+    stage pair to many, slices -- with f32 results: an operand read before it landed or after it was replaced shows, where bf16
+    rounding would cover it.  Tolerance: each of K additions rounds by 2^-24 of a partial sum, signs at random."""
+    x, w = torch.randn(M, K, device=DEV).to(BF), (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    wt = ops.TiledWeight(w) if tiled else w
+    exp = x.double() @ w.double().T
+    out = torch.empty(M, N, device=DEV)
+    for _ in range(3):
+        ops.gemm(x, wt, out.fill_(7.0))
+        assert float((out.double() - exp).norm() / exp.norm()) < 2.0 ** -24 * K ** 0.5
+    b = torch.randn(N, device=DEV).to(BF)
+    ops.gemm(x, wt, got := torch.empty(M, N, dtype=BF, device=DEV), epi="gelu", bias=b)
+    y = exp + b.double()
+    y = y * 0.5 * torch.erfc(-y / 2 ** 0.5)
+    assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
+
+
 def test_gemm_8phase_split_k_down_projection():
     """Measured routing (mode 2): the 1011-row Llama-3-8B down projection (K = 14336) runs the
     8-phase kernel in 4 split-K slices with the residual applied by the reduce kernel -- against
