@@ -84,6 +84,7 @@ class WhisperRunner:
         self.h_slots = self.h_in[4 * R :].view(torch.int64)
         self.h_i32[3].fill_(1)
         self.h_slots.fill_(-1)
+        self.np_i32, self.np_slots = self.h_i32.numpy(), self.h_slots.numpy()
         if use_graphs is None:
             use_graphs = ops.env_flag("VWA_HIPGRAPH")
         self.use_graphs = bool(use_graphs) and dev.type == "cuda"
@@ -120,20 +121,19 @@ class WhisperRunner:
         """rows: (session slot, token, position). Returns f32 logits [len(rows), vocab_padded]."""
         n = len(rows)
         M = next(bk for bk in BUCKETS if bk >= n)
+        # the rows' numbers first, while the previous step may still run
+        slot, tok, pos = np.asarray(rows, dtype=np.int64).reshape(n, 3).T
         if self._copy_done is not None:
             # the previous step's pinned -> device copy may still be queued behind its forward:
             # rewriting the pinned rows before it ran would feed that step the NEXT step's tokens /
             # positions / slots (back-to-back step() calls with no host sync in between; the
             # one-launch decoder leaves the host far ahead of the GPU)
             self._copy_done.synchronize()
-        hi = self.h_i32
-        for i, (slot, tok, pos) in enumerate(rows):
-            hi[0, i], hi[1, i], hi[2, i], hi[3, i] = tok, pos, slot, pos + 1
-            blk = 1 + slot * self.bps + pos // self.bs
-            self.h_slots[i] = blk * self.bs + pos % self.bs
-        for i in range(n, M):
-            hi[0, i], hi[1, i], hi[2, i], hi[3, i] = 0, 0, 0, 1
-            self.h_slots[i] = -1
+        hi = self.np_i32
+        hi[0, :n], hi[1, :n], hi[2, :n], hi[3, :n] = tok, pos, slot, pos + 1
+        self.np_slots[:n] = (1 + slot * self.bps + pos // self.bs) * self.bs + pos % self.bs
+        hi[:3, n:M], hi[3, n:M] = 0, 1
+        self.np_slots[n:M] = -1
         b = self.b
         b.step_in.copy_(self.h_in, non_blocking=True)
         if self.device.type == "cuda":

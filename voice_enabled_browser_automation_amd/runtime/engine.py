@@ -391,30 +391,19 @@ class LLMEngine:
         n = len(rows)
         M = bucket_for(n)
         b = self.bufs
-        if self._staging_inflight:
-            # back-to-back steps with no host sync in between (several admissions in one scheduler
-            # iteration, partial feeds, non-chained check=False steps): the previous step's copy of
-            # the staging rows may still be queued behind its forward
-            torch.cuda.current_stream().synchronize()
-            self._staging_inflight = False
         if getattr(self, "_chain_retry_at", None) is not None:
             self._maybe_rearm_chain()
-        if logits_for is None or len(logits_for) == n:
-            nl, L = n, M
-        else:
-            nl = len(logits_for)
-            L = min(bucket_for(nl), M)
-            if L < M:  # (L == M: no saving -- compute every row and index on the host side)
-                b.np_sel[:nl] = logits_for
-                b.np_sel[nl:L] = logits_for[-1]
+        # the rows' numbers first, while the previous step may still run; the pinned staging only once it is through
+        # (back-to-back steps with no host sync in between -- several admissions in one scheduler iteration, partial
+        # feeds, given tokens: its copy of the staging rows may still be queued behind its forward)
         pending: Dict[int, int] = {}
         bs = self.block_size
         toks, poss, sids, slots = [], [], [], []
-        rtab = b.np_row_table if b.rt_cols and M <= 4 else None
         for seq, tok in rows:
             sid = seq.sid
             pos = pending.get(sid, seq.n_computed)
             if pos // bs >= len(seq.blocks):
+                self._sync_staging()  # (the block table is staged as well)
                 self._ensure_blocks(seq, pos + 1)
             if pos >= len(seq.tokens):
                 seq.tokens.append(tok)
@@ -423,6 +412,17 @@ class LLMEngine:
             sids.append(sid)
             slots.append(seq.blocks[pos // bs] * bs + pos % bs)
             pending[sid] = pos + 1
+        shared = self._shared_prefix(rows, min(poss) + 1)
+        self._sync_staging()
+        if logits_for is None or len(logits_for) == n:
+            nl, L = n, M
+        else:
+            nl = len(logits_for)
+            L = min(bucket_for(nl), M)
+            if L < M:  # (L == M: no saving -- compute every row and index on the host side)
+                b.np_sel[:nl] = logits_for
+                b.np_sel[nl:L] = logits_for[-1]
+        rtab = b.np_row_table if b.rt_cols and M <= 4 else None
         if rtab is not None:  # after the loop: a later row of a sequence may have added its last block
             for i, (seq, _) in enumerate(rows):
                 rtab[i, : len(seq.blocks)] = seq.blocks
@@ -432,7 +432,7 @@ class LLMEngine:
         hi[2, :n] = sids
         hi[3, :n] = hi[1, :n] + 1
         b.np_slots[:n] = slots
-        b.np_shared[0] = self._shared_prefix(rows, min(poss) + 1)
+        b.np_shared[0] = shared
         b.np_shared[1] = n
         if M > n:  # padded rows: no KV write, 1-token context on scratch block 0
             hi[0:3, n:M] = 0
@@ -816,13 +816,16 @@ class LLMEngine:
             if self.bufs.table_dirty:
                 self.bufs.block_table.copy_(self.bufs.h_table)
                 self.bufs.table_dirty = False
-            dev = self.device
-            pos = torch.arange(start, start + n, dtype=torch.int32)
-            slots = torch.tensor([self.slot_of(seq, int(p)) for p in pos], dtype=torch.int64)
-            m = self.model
+            dev, m = self.device, self.model
+            pos = np.arange(start, start + n)
+            np_meta = np.stack([np.asarray(seq.tokens[start : start + n], dtype=np.int32), pos.astype(np.int32)])
+            meta = torch.from_numpy(np_meta)
+            slots = torch.from_numpy(np.asarray(seq.blocks, dtype=np.int64)[pos // self.block_size] * self.block_size
+                                     + pos % self.block_size)
+            if dev.type == "cuda":  # (pageable copies would wait for the stream)
+                meta, slots = (t.pin_memory().to(dev, non_blocking=True) for t in (meta, slots))
             scratch = SimpleNamespace(
-                tokens=torch.tensor(seq.tokens[start : start + n], dtype=torch.int32, device=dev),
-                positions=pos.to(dev), slots=slots.to(dev), block_table=self.bufs.block_table,
+                tokens=meta[0], positions=meta[1], slots=slots, block_table=self.bufs.block_table,
                 hidden=torch.empty(n, m.cfg.hidden, dtype=m.dtype, device=dev),
                 q=torch.empty(n, m.nq * m.hd, dtype=m.dtype, device=dev),
                 act=torch.empty(n, m.F, dtype=m.dtype, device=dev),
