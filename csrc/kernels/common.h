@@ -105,16 +105,29 @@ VWA_DEVICE bf16x8 as_bf16x8(const uint4& v) { return __builtin_bit_cast(bf16x8, 
 // need their global stores performed before the barrier wait for them explicitly.
 VWA_DEVICE void lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-VWA_DEVICE float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+// Reductions over the wave without LDS permutes (a __shfl_xor step is an LDS round trip; six of them were a third of a
+// one-row norm): halves by v_permlane32_swap / 16_swap, then rotations of the 16 lanes, which after the step before hold
+// every value twice, four, eight times.  Pairs and order are those of __shfl_xor over 32, 16, .. 1, and so are the bits.
+template <int N>
+VWA_DEVICE float row_ror(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, true));
 }
-
+template <class F>
+VWA_DEVICE float wave_reduce(float v, F f) {
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  v = f(v, row_ror<8>(v));
+  v = f(v, row_ror<4>(v));
+  v = f(v, row_ror<2>(v));
+  return f(v, row_ror<1>(v));
+}
+VWA_DEVICE float wave_sum(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
+}
 VWA_DEVICE float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 VWA_DEVICE int lane_id() { return threadIdx.x & 63; }

@@ -12,12 +12,32 @@ using namespace vwa;
 
 namespace {
 
-VWA_DEVICE float block_sum(float v, float* red) {
+// I: a number of its own for every sum of a kernel (so one barrier each).  lds_sync: stores in flight are not waited for.
+template <int I>
+VWA_DEVICE float block_sum(float v, float (*red)[4]) {
   v = wave_sum(v);
-  __syncthreads();  // (red may still be read from the previous sum)
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return (red[0] + red[1]) + (red[2] + red[3]);
+  if ((threadIdx.x & 63) == 0) red[I][threadIdx.x >> 6] = v;
+  lds_sync();
+  return (red[I][0] + red[I][1]) + (red[I][2] + red[I][3]);
+}
+
+// four weights from column c (0 past D)
+VWA_DEVICE void w4(const float* w, int c, int D, float (&v)[4]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = c + j < D ? w[min(c + j, D - 1)] : 0.f;
+}
+
+// this thread's weights of a row, STEPS x 4 as the row's columns
+template <int STEPS>
+VWA_DEVICE void row_weights(const float* w, int D, float (&o)[STEPS][4]) {
+  const int last = (D - 1) & ~3;
+  if (D % 4 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0) {
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) ld4(w + min((i * 256 + (int)threadIdx.x) * 4, last), o[i]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) w4(w, (i * 256 + (int)threadIdx.x) * 4, D, o[i]);
+  }
 }
 
 // one workgroup per row, the row held in registers: STEPS x 1024 columns, 4 per thread and step, all
@@ -27,10 +47,10 @@ template <class T, int STEPS>
 __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ x, int ldx,
                                                             const float* __restrict__ w, const float* __restrict__ b,
                                                             T* __restrict__ y, int ldy, int D, int Dpad, float eps) {
-  __shared__ float red[4];
+  __shared__ float red[2][4];
   const float* xr = x + (size_t)blockIdx.x * ldx;
   T* yr = y + (size_t)blockIdx.x * ldy;
-  float v[STEPS][4];
+  float v[STEPS][4], wv[STEPS][4], bv[STEPS][4];
   const int last = (D - 1) & ~3;
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
@@ -40,6 +60,8 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
     v[i][2] = f.z;
     v[i][3] = f.w;
   }
+  row_weights<STEPS>(w, D, wv);
+  row_weights<STEPS>(b ? b : w, D, bv);
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
@@ -50,7 +72,7 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
       s += v[i][j];
     }
   }
-  const float mu = block_sum(s, red) / (float)D;
+  const float mu = block_sum<0>(s, red) / (float)D;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
@@ -61,17 +83,14 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
       q += d * d;
     }
   }
-  const float rstd = 1.f / sqrtf(block_sum(q, red) / (float)D + eps);
+  const float rstd = 1.f / sqrtf(block_sum<1>(q, red) / (float)D + eps);
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
     const int c = (i * 256 + threadIdx.x) * 4;
     if (c >= D) continue;
     float o[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int cj = min(c + j, D - 1);
-      o[j] = c + j < D ? (v[i][j] - mu) * rstd * w[cj] + (b ? b[cj] : 0.f) : 0.f;
-    }
+    for (int j = 0; j < 4; ++j) o[j] = c + j < D ? (v[i][j] - mu) * rstd * wv[i][j] + (b ? bv[i][j] : 0.f) : 0.f;
     st4(yr + c, o);
   }
   for (int c = ((D + 3) & ~3) + threadIdx.x; c < Dpad; c += 256) stv(yr + c, 0.f);
@@ -88,14 +107,14 @@ void launch_ln(const float* x, int ldx, const float* w, const float* b, T* y, in
 }
 
 // mean and 1 / std of the row held as STEPS x 4 values per thread (columns past D are zero)
-template <int STEPS>
-VWA_DEVICE float2 row_stats(const float (&v)[STEPS][4], int D, float eps, float* red) {
+template <int I, int STEPS>
+VWA_DEVICE float2 row_stats(const float (&v)[STEPS][4], int D, float eps, float (*red)[4]) {
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < STEPS; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) s += v[i][j];
-  const float mu = block_sum(s, red) / (float)D;
+  const float mu = block_sum<I>(s, red) / (float)D;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < STEPS; ++i)
@@ -104,13 +123,7 @@ VWA_DEVICE float2 row_stats(const float (&v)[STEPS][4], int D, float eps, float*
       const float d = (i * 256 + (int)threadIdx.x) * 4 + j < D ? v[i][j] - mu : 0.f;
       q += d * d;
     }
-  return make_float2(mu, 1.f / sqrtf(block_sum(q, red) / (float)D + eps));
-}
-
-// four weights from column c (0 past D)
-VWA_DEVICE void w4(const float* w, int c, int D, float (&v)[4]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) v[j] = c + j < D ? w[min(c + j, D - 1)] : 0.f;
+  return make_float2(mu, 1.f / sqrtf(block_sum<I + 1>(q, red) / (float)D + eps));
 }
 
 // one workgroup per row: x += norm(sum of the branch rows) * w1; h = norm(x) * w2.  Loads of the branch,
@@ -119,7 +132,7 @@ template <class T, int STEPS>
 __global__ __launch_bounds__(256) void add_norm_kernel(float* __restrict__ x, int ldx, const T* __restrict__ br, int ldb,
                                                        int n_parts, const float* __restrict__ w1, const float* __restrict__ w2,
                                                        T* __restrict__ h, int ldh, int D, int Dpad, float eps) {
-  __shared__ float red[4];
+  __shared__ float red[4][4];
   float* xr = x + (size_t)blockIdx.x * ldx;
   const T* b = br + (size_t)blockIdx.x * n_parts * ldb;
   const int last = (D - 1) & ~3;
@@ -130,17 +143,8 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* __restrict__ x, in
     ld4(b + c, v[i]);
     ld4(xr + c, xs[i]);
   }
-  auto weights = [&](const float* w, float (&o)[STEPS][4]) {
-    if (D % 4 == 0) {
-#pragma unroll
-      for (int i = 0; i < STEPS; ++i) ld4(w + min((i * 256 + (int)threadIdx.x) * 4, last), o[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < STEPS; ++i) w4(w, (i * 256 + (int)threadIdx.x) * 4, D, o[i]);
-    }
-  };
-  weights(w1, wa);
-  weights(w2 ? w2 : w1, wb);
+  row_weights<STEPS>(w1, D, wa);
+  row_weights<STEPS>(w2 ? w2 : w1, D, wb);
   for (int k = 1; k < n_parts; k += 3) {
     float u[3][STEPS][4];
 #pragma unroll
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* __restrict__ x, in
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if ((i * 256 + (int)threadIdx.x) * 4 + j >= D) v[i][j] = xs[i][j] = 0.f;
-  const float2 sb = row_stats<STEPS>(v, D, eps, red);
+  const float2 sb = row_stats<0>(v, D, eps, red);
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
     const int c = (i * 256 + threadIdx.x) * 4;
@@ -170,7 +174,7 @@ __global__ __launch_bounds__(256) void add_norm_kernel(float* __restrict__ x, in
   }
   if (!w2) return;
   T* hr = h + (size_t)blockIdx.x * ldh;
-  const float2 sx = row_stats<STEPS>(xs, D, eps, red);
+  const float2 sx = row_stats<2>(xs, D, eps, red);
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
     const int c = (i * 256 + threadIdx.x) * 4;
