@@ -92,6 +92,9 @@ VWA_DEVICE int swz(int h) { return (0x64753120 >> (4 * h)) & 7; }
 // 646 TFLOP/s, 1500 x 5120 x 1280 532 -> 594.)
 // A read's 16-lane groups now hold chunks c and c ^ 4 of complementary half rows {0,1,6,7}, {2,3,4,5}: swzk maps both
 // halves to 0..3.
+// LINES false keeps the substeps' own order, for weights whose products choose experts further on (GemmParams::keep_order):
+// the same sums in another order move a product by its last bits, and a token whose scores nearly tie to another expert --
+// 1 in 300 decoded rows of a 16-expert model when its prompt alone was computed in the other order.
 VWA_DEVICE int swzk(int h) { return (h & 1) | (h >> 2 << 1); }
 VWA_DEVICE int chunk_of(int g, int sp) { return 4 * (g & 1) + 2 * sp + (g >> 1); }
 
@@ -121,7 +124,7 @@ VWA_DEVICE void dma16(__amdgpu_buffer_rsrc_t r, char* lds_wave_base, unsigned vo
 // holds the lane's k 32 g + 16 h .. + 16, both sub-steps of half h), converted to bf16 fragments on
 // the LDS read -- no quantised copy of X, half the weight bytes of bf16.
 // rows (grouped launches): X rows of this thread's pieces (< 0: none)
-template <class C, bool WT, bool F8, bool W8 = false, bool GRP = false>
+template <class C, bool WT, bool F8, bool W8 = false, bool GRP = false, bool LINES = true>
 VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __amdgpu_buffer_rsrc_t rw, int bm,
                             int bn, int hs, char* buf, const int (&rows)[C::BM / 8 / C::NW]) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -132,12 +135,12 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
 #pragma unroll
   for (int it = 0; it < C::BM / 8 / C::NW; ++it) {
     const int q = it * C::NW + w;  // wave-instruction index: rows 8q .. 8q + 7
-    const int r = 8 * q + (lane >> 3), c = (lane & 7) ^ (F8 || W8 ? swz((r >> 1) & 7) : swzk((r >> 1) & 7));
+    const int r = 8 * q + (lane >> 3), c = (lane & 7) ^ (LINES && !F8 && !W8 ? swzk((r >> 1) & 7) : swz((r >> 1) & 7));
     const int m = GRP ? rows[it] : bm + r;
     unsigned off;
     if constexpr (F8)
       off = (unsigned)((size_t)m * p.ldx + (size_t)kg * BKG + 32 * (c >> 1) + 16 * (c & 1));
-    else if constexpr (W8)  // (the fp8 tiled order: k 32 g + 16 ha + 8 sp)
+    else if constexpr (W8 || !LINES)  // (k 32 g + 16 ha + 8 sp)
       off = (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 32 * (c >> 1) + 16 * ha + 8 * (c & 1)) * 2);
     else
       off = (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 64 * ha + 8 * c) * 2);
@@ -165,17 +168,18 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
       off = T * 16 < p.N ? (unsigned)(((size_t)T * kgn + kg) * 2048 + sp * 1024 + lane * 16) : 0xFFFFFFF0u;
     } else if constexpr (WT) {
       const int T = (bn >> 4) + tile;
-      off = T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + (2 * sp + (lane >> 5)) * 512 + h * 256 + (lane & 31) * 8) * 2)
-                         : 0xFFFFFFF0u;
+      const int at = LINES ? (2 * sp + (lane >> 5)) * 512 + h * 256 + (lane & 31) * 8 : (2 * h + sp) * 512 + lane * 8;
+      off = T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + at) * 2) : 0xFFFFFFF0u;
     } else {
       const int n = bn + tile * 16 + (lane & 15), g = lane >> 4;
-      off = n < p.N ? (unsigned)(((size_t)n * p.K + (size_t)kg * BKG + 64 * h + 8 * chunk_of(g, sp)) * 2) : 0xFFFFFFF0u;
+      const int at = LINES ? 64 * h + 8 * chunk_of(g, sp) : 32 * g + 16 * h + 8 * sp;
+      off = n < p.N ? (unsigned)(((size_t)n * p.K + (size_t)kg * BKG + at) * 2) : 0xFFFFFFF0u;
     }
     dma16(rw, buf + C::A_BYTES + q * 1024, off);
   }
 }
 
-template <class C, bool F8, bool W8 = false>
+template <class C, bool F8, bool W8 = false, bool LINES = true>
 VWA_DEVICE void compute_stage(const char* buf, f32x4 (&acc)[C::FM][C::FN], int wm, int wn) {
   const int l = lane_id();
   const int rl = l & 15, g = l >> 4;
@@ -241,7 +245,8 @@ VWA_DEVICE void compute_stage(const char* buf, f32x4 (&acc)[C::FM][C::FN], int w
 #pragma unroll
     for (int sp = 0; sp < 2; ++sp) {
       bf16x8 a[C::FM], b[C::FN];
-      const int ch = (chunk_of(g, sp) ^ swzk(rl >> 1)) << 4;  // ((row >> 1) & 7) == rl >> 1 for every fragment row
+      // ((row >> 1) & 7) == rl >> 1 for every fragment row
+      const int ch = (LINES ? chunk_of(g, sp) ^ swzk(rl >> 1) : (2 * g + sp) ^ swz(rl >> 1)) << 4;
 #pragma unroll
       for (int i = 0; i < C::FM; ++i) a[i] = *reinterpret_cast<const bf16x8*>(la + i * 16 * 128 + ch);
 #pragma unroll
@@ -517,7 +522,7 @@ VWA_DEVICE float reduce_item(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, in
 // (round 4's 4-stage variant for one-row-block GEMMs measured slower in whole decode steps -- 128 KB
 // of LDS leaves one workgroup per CU, so split-K grids above 256 workgroups ran in two rounds:
 // fp8 32 rows 4.97 vs 4.36 ms, profiles/r4_gemm_ab.md -- and was removed in round 5)
-template <class C, int EPI, bool WT, bool F8 = false, bool P8 = false, bool W8 = false, bool GRP = false>
+template <class C, int EPI, bool WT, bool F8 = false, bool P8 = false, bool W8 = false, bool GRP = false, bool LINES = !GRP>
 __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int FM = C::FM, FN = C::FN;
@@ -582,12 +587,12 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     unsigned voff[8];  // this lane's pieces of the half-tiles (k-group 0)
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-      const int q = it * 8 + w, r = 8 * q + (l >> 3), c = (l & 7) ^ swzk((r >> 1) & 7);  // A rows 8 q .. 8 q + 7
+      const int q = it * 8 + w, r = 8 * q + (l >> 3), c = (l & 7) ^ (LINES ? swzk((r >> 1) & 7) : swz((r >> 1) & 7));  // A rows 8 q ..
       const int m = GRP ? rows[it] : bm + r;
-      voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)(((size_t)m * p.ldx + 8 * c) * 2) : 0xFFFFFFF0u;
+      voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)(((size_t)m * p.ldx + (LINES ? 8 * c : 32 * (c >> 1) + 8 * (c & 1))) * 2) : 0xFFFFFFF0u;
       const int T = (bn >> 4) + (q >> 1);                                                // B n-tile q / 2, MFMA q & 1
-      const size_t at = WT ? (size_t)T * KG * 2048 + (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8
-                           : (size_t)(T * 16 + rl) * p.K + 8 * chunk_of(g, q & 1);
+      const size_t at = WT ? (size_t)T * KG * 2048 + (LINES ? (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8 : (q & 1) * 512 + l * 8)
+                           : (size_t)(T * 16 + rl) * p.K + (LINES ? 8 * chunk_of(g, q & 1) : 32 * g + 8 * (q & 1));
       voff[4 + it] = T * 16 < p.N ? (unsigned)(at * 2) : 0xFFFFFFF0u;
     }
     // (stages past the last are issued too, on empty resources: the waits stay one constant)
@@ -595,9 +600,10 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       const int hs = h0 + s, kg = hs >> 1, h = hs & 1;
       const bool in = s < nh;
       if (which < 2)
-        p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, (kg * BKG + 64 * h) * 2, which, stage(s));
+        p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, (kg * BKG + (LINES ? 64 : 16) * h) * 2, which, stage(s));
       else
-        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (WT ? kg * 2048 + h * 256 : kg * BKG + 64 * h) * 2, which, stage(s));
+        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (WT ? kg * 2048 + (LINES ? 256 : 1024) * h : kg * BKG + (LINES ? 64 : 16) * h) * 2, which,
+                stage(s));
     };
     issue(0, 0);
     issue(0, 2);
@@ -618,7 +624,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
         for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            a[i][sp] = *reinterpret_cast<const bf16x8*>(la + (i0 + i) * 16 * 128 + ((chunk_of(g, sp) ^ swzk(rl >> 1)) << 4));
+            a[i][sp] = *reinterpret_cast<const bf16x8*>(la + (i0 + i) * 16 * 128 + ((LINES ? chunk_of(g, sp) ^ swzk(rl >> 1) : (2 * g + sp) ^ swz(rl >> 1)) << 4));
       };
 #pragma unroll
       for (int sp = 0; sp < 2; ++sp)
@@ -644,16 +650,16 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     if (wm == 0) asm volatile("s_barrier" ::: "memory");  // (group 1 started one barrier later)
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // (the epilogue reuses the LDS)
   } else {
-  if (nh > 0) issue_stage<C, WT, F8, W8, GRP>(p, rx, rw, bm, bn, h0, lds, rows);
-  if (nh > 1) issue_stage<C, WT, F8, W8, GRP>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
+  if (nh > 0) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0, lds, rows);
+  if (nh > 1) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
   for (int i = 0; i < nh; ++i) {
     if (i + 1 < nh)
       asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // this stage landed everywhere
     else
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    compute_stage<C, F8, W8>(lds + (i & 1) * STG, acc, wm, wn);
+    compute_stage<C, F8, W8, LINES>(lds + (i & 1) * STG, acc, wm, wn);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave done reading it
-    if (i + 2 < nh) issue_stage<C, WT, F8, W8, GRP>(p, rx, rw, bm, bn, h0 + i + 2, lds + (i & 1) * STG, rows);
+    if (i + 2 < nh) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + i + 2, lds + (i & 1) * STG, rows);
   }
   }
   const int l = lane_id();
@@ -862,6 +868,17 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // 768 x 4096 x 14336 155 -> 86, 512 x 28672 x 4096 132 -> 93, 1863 x 6144 x 4096 115 -> 83.
 //   a round of the CUs costs so much per k-group and so much to start and store; a part of a last round 70 % and its share;
 //   128^2 tiles run two to a CU, one alone is faster; the slices' f32 partials are written and read.
+float estimate(const GemmParams& p, bool p8, int s) {
+  const int kg = cdiv(p.K / BKG, s), b = p8 ? 256 : 128;
+  const int64_t t = (int64_t)cdiv(p.M, b) * cdiv(p.N, b) * s;
+  const bool alone = !p8 && t <= p.cus;
+  const float r = (float)t / (p8 || alone ? p.cus : 2 * p.cus), whole = floorf(r);
+  const float rounds = r <= 1.f ? 1.f : r > whole ? whole + 0.7f + 0.3f * (r - whole) : whole;
+  const float per = p8 ? 2.0f : alone ? 1.27f : r >= 1.f ? 1.84f : 1.27f + 0.57f * (2.f * r - 1.f);
+  const float sum = s > 1 ? 4.f + (float)s * p.M * p.N * 4.f / 3.55e6f : 0.f;
+  return rounds * (kg * per + (p8 ? 5.6f : 2.3f)) + sum;
+}
+
 struct Plan {
   bool p8;
   int splits;
@@ -872,16 +889,8 @@ Plan plan(const GemmParams& p) {
   float least = 0.f;
   for (const int s0 : {1, 2, 3, 4, 6, 8, 12, 16}) {
     if (s0 > 1 && (s0 > KG || !p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
-    const int kg = cdiv(KG, s0), s = cdiv(KG, kg);
-    const float sum = s > 1 ? 4.f + (float)s * p.M * p.N * 4.f / 3.55e6f : 0.f;
     for (const bool p8 : {true, false}) {
-      const int b = p8 ? 256 : 128;
-      const int64_t t = (int64_t)cdiv(p.M, b) * cdiv(p.N, b) * s;
-      const bool alone = !p8 && t <= p.cus;
-      const float r = (float)t / (p8 || alone ? p.cus : 2 * p.cus), whole = floorf(r);
-      const float rounds = r <= 1.f ? 1.f : r > whole ? whole + 0.7f + 0.3f * (r - whole) : whole;
-      const float per = p8 ? 2.0f : alone ? 1.27f : r >= 1.f ? 1.84f : 1.27f + 0.57f * (2.f * r - 1.f);
-      const float us = rounds * (kg * per + (p8 ? 5.6f : 2.3f)) + sum;
+      const float us = estimate(p, p8, cdiv(KG, cdiv(KG, s0)));
       if (least == 0.f || us < least) {
         least = us;
         best = {p8, s0};
@@ -891,9 +900,34 @@ Plan plan(const GemmParams& p) {
   return best;
 }
 
+// keep_order: the slices of few large tiles are part of the order (in powers of two until they cover the CUs, of >= 2048 k
+// each; p.splits holds those of the small tile); the tile is not
+Plan plan_kept(const GemmParams& p) {
+  Plan r{false, p.splits};
+  if (p.M >= 256 && p.N % 256 == 0) {
+    const int tiles8 = cdiv(p.M, 256) * (p.N / 256);
+    int s = 1;
+    while (p.ws && tiles8 * s < p.cus && s * 2 <= p.K / BKG && (int64_t)(s * 2) * p.M * p.N <= p.ws_cap) s *= 2;
+    if (tiles8 >= 256 || (tiles8 * s >= p.cus && p.K / s >= 2048)) r.splits = s;
+  }
+  r.p8 = p.M >= 128 && estimate(p, true, r.splits) < estimate(p, false, r.splits);
+  return r;
+}
+
 template <int EPI>
 int launch_epi(const GemmParams& p, hipStream_t st, bool p8) {
-  if (p8) {
+  constexpr bool kKeeps = EPI == EPI_STORE || EPI == EPI_SWIGLU;
+  if (kKeeps && p.keep_order) {
+    if constexpr (kKeeps) {
+      if (p8)
+        hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, false, true, false, false, false>),
+                           dim3(cdiv(p.M, 256) * cdiv(p.N, 256) * p.splits), dim3(CfgP8::THREADS), CfgP8::LDS, st, p);
+      else
+        hipLaunchKernelGGL((gemm_kernel<CfgS, EPI, true, false, false, false, false, false>),
+                           dim3(cdiv(p.M, CfgS::BM) * cdiv(p.N, CfgS::BN) * p.splits), dim3(CfgS::THREADS),
+                           2 * CfgS::STAGE > CfgS::LDS ? 2 * CfgS::STAGE : CfgS::LDS, st, p);
+    }
+  } else if (p8) {
     const int tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
     if (p.w_tiled)
       hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
@@ -962,7 +996,12 @@ extern "C" int vwa_gemm(int epi, const GemmParams* pp, hipStream_t st) {
     return -19;
   if (p.splits < 1) p.splits = 1;
   bool p8 = false;
-  if (!p.sw && p.nbatch <= 1 && p.cus > 0) {
+  p.keep_order = p.keep_order && p.w_tiled && !p.sw && p.nbatch <= 1 && p.cus > 0 && (epi == EPI_STORE || epi == EPI_SWIGLU);
+  if (p.keep_order) {
+    const Plan pl = plan_kept(p);
+    p8 = pl.p8;
+    p.splits = pl.splits;
+  } else if (!p.sw && p.nbatch <= 1 && p.cus > 0) {
     if (g_p8_mode == 1 && p.w_tiled && p.N % 256 == 0 && p.M >= 256) {
       const int tiles8 = cdiv(p.M, 256) * (p.N / 256);
       p8 = true;

@@ -702,6 +702,24 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
+def test_gemm_keeps_the_order_of_its_sums():
+    """A TiledWeight with keep_order: the same bits from either tile (4096 rows take the 256^2 one, 2048 the 128^2 one), with
+    and without the SwiGLU epilogue; other epilogues and f32 results are served as ever."""
+    N, K = 4096, 2048
+    x, w = torch.randn(4096, K, device=DEV).to(BF), (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    wt = ops.TiledWeight(w, keep_order=True)
+    for op in (lambda a: ops.linear(a, wt), lambda a: ops.linear_swiglu(a, wt)):
+        assert torch.equal(op(x)[:2048], op(x[:2048]))
+    exp = x[:300].double() @ w.double().T
+    out = torch.empty(300, N, device=DEV)
+    ops.linear(x[:300], wt, out=out, out_dtype=torch.float32)
+    assert float((out.double() - exp).norm() / exp.norm()) < 2.0 ** -24 * K ** 0.5
+    r = torch.randn(300, N, device=DEV)
+    ops.linear(x[:300], wt, out=out, residual=r)
+    assert float((out - r - exp).norm() / exp.norm()) < 2.0 ** -24 * K ** 0.5 + 4e-7
+    assert wt.to("cpu").keep_order and not ops.TiledWeight(w).keep_order
+
+
 def test_gemm_8phase_split_k_down_projection():
     """Measured routing (mode 2): the 1011-row Llama-3-8B down projection (K = 14336) runs the
     8-phase kernel in 4 split-K slices with the residual applied by the reduce kernel -- against

@@ -146,7 +146,8 @@ class RipupelModel:
         cfg, dev, dt, d = self.cfg, self.device, self.dtype, self.cfg.hidden
         gpu = dev.type == "cuda"
         tiled = gpu and dt == torch.bfloat16
-        place = (lambda t: ops.TiledWeight(t)) if tiled else (lambda t: t)
+        # (a routed model's products keep one order of their sums: a near tie of two experts falls the same way)
+        place = (lambda t, keep=True: ops.TiledWeight(t, keep_order=keep)) if tiled else (lambda t, keep=True: t)
         frag = ops.fragments if gpu else (lambda t: t)
 
         def get(name, shape, dtype):
@@ -198,7 +199,7 @@ class RipupelModel:
         self.final_w = vec("final.norm", d)
         head = zeros(self.v_pad, self.d_pad)
         head[: cfg.vocab_size, :d] = self.embed
-        self.lm_head = place(head)
+        self.lm_head = place(head, keep=False)
 
     def _build_rglru(self, c: RgLruConfig, D: RgLruDims, m: str, mat, vec, zeros, w_in, w_out, gpu: bool) -> RgLruWeights:
         d, W, nb, k, bs, dev = self.cfg.hidden, c.width, D.nb, D.block, D.bs, self.device
@@ -242,7 +243,7 @@ class RipupelModel:
             w_kv = zeros(_columns(H * (D.dim + vdk)), _up(D.rank, 128))
             w_kv[: H * D.dim, : D.rank].view(H, D.dim, D.rank).copy_(uk.transpose(1, 2))
             w_kv[H * D.dim : H * (D.dim + vdk), : D.rank].view(H, vdk, D.rank)[:, : D.vd] = uv
-            w_kv = ops.TiledWeight(w_kv)
+            w_kv = ops.TiledWeight(w_kv, keep_order=True)
         return LatentWeights(H=H, dim_p=D.dim, rot_p=D.rot, rank_p=D.rank, vd=D.vd, scale=c.scale, eps=self.cfg.norm_eps,
                              norm=vec(m + "dkv.norm", c.kv_rank) if D.own else None, sink=vec(m + "sink", H), uk=frag(uk),
                              uv=frag(uv), w_kv=w_kv)

@@ -271,12 +271,16 @@ class TiledWeight:
     streaming / chained kernels (1 KB contiguous load instructions) and the LDS-tiled GEMM for
     prefill and > 16-row steps (gemm.hip copies the 4 KB fragment blocks to LDS verbatim) -- so
     the model keeps one copy of each weight.  ``dense()`` rebuilds the row-major matrix for the
-    CPU reference and diagnostics."""
+    CPU reference and diagnostics.
 
-    __slots__ = ("t",)
+    ``keep_order``: its products in a many-row GEMM keep one order of their sums whatever kernel serves the shape best
+    (models whose products choose experts further on: gemm.hip)."""
 
-    def __init__(self, w: Optional[torch.Tensor] = None, t: Optional[torch.Tensor] = None):
+    __slots__ = ("t", "keep_order")
+
+    def __init__(self, w: Optional[torch.Tensor] = None, t: Optional[torch.Tensor] = None, keep_order: bool = False):
         self.t = tile_weight(w) if t is None else t
+        self.keep_order = keep_order
 
     def dense(self) -> torch.Tensor:
         return untile_weight(self.t)
@@ -304,7 +308,7 @@ class TiledWeight:
         return self.t.element_size()
 
     def to(self, device) -> "TiledWeight":
-        return TiledWeight(t=self.t.to(device))
+        return TiledWeight(t=self.t.to(device), keep_order=self.keep_order)
 
 
 def _stream_ok(x: torch.Tensor, w) -> bool:
@@ -474,7 +478,7 @@ def gemm(x: torch.Tensor, w, out: torch.Tensor, *, epi: str = "none", bias: Opti
     wt = w.t if tiled else w
     ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
     E.gemm(x, wt, bias, out, _GEMM_EPI[epi], rstd, residual, tiled, ws, ss_out, ss_zero,
-           ss_in if fuse_rms else None, eps)
+           ss_in if fuse_rms else None, eps, keep_order=tiled and w.keep_order)
     return out
 
 
