@@ -224,19 +224,32 @@ int64_t max_tiles(int64_t max_ctx, int64_t window, int64_t keep) {
 void talk_attention(Tensor q, Tensor k, Tensor v, Tensor table, Tensor positions, Tensor seq_ids, Tensor slots,
                     c10::optional<Tensor> row_list, int64_t n_rows, int64_t H, double scale, int64_t window, int64_t keep,
                     c10::optional<Tensor> talk, c10::optional<Tensor> gate, double out_scale, int64_t max_ctx, Tensor s,
-                    Tensor stat, Tensor part, Tensor counters, Tensor out) {
+                    Tensor stat, Tensor part, Tensor counters, Tensor out, c10::optional<Tensor> groups, int64_t nq) {
   c10::DeviceGuard g(q.device());
   const int64_t total = q.size(0);
-  TalkAttnParams p = attn_params(q, k, v, table, positions, seq_ids, slots, row_list.has_value() ? total : n_rows, H, scale,
-                                 window, keep, talk, gate, out_scale, out);
+  TORCH_CHECK(!(row_list.has_value() && groups.has_value()), "row_list or groups");
+  TalkAttnParams p = attn_params(q, k, v, table, positions, seq_ids, slots,
+                                 row_list.has_value() || groups.has_value() ? total : n_rows, H, scale, window, keep, talk, gate,
+                                 out_scale, out);
   TORCH_CHECK(max_ctx >= 1 && max_ctx <= table.size(1) * k.size(2), "max_ctx exceeds the block table");
   if (row_list.has_value()) p.row_list = i32p(*row_list, n_rows, "row_list");
+  const int64_t R = H / p.G;
+  if (groups.has_value()) {  // n_rows: groups of at most nq rows
+    TORCH_CHECK(groups->dim() == 2 && groups->size(1) == 2, "groups int32 [n, 2]");
+    TORCH_CHECK(nq >= 1 && nq * R <= 16, "groups: nq * H / G <= 16");
+    p.groups = i32p(*groups, n_rows * 2, "groups");
+  } else {
+    nq = 1;
+  }
+  p.nq = (int)nq;
   p.rows = (int)n_rows;
-  const int64_t nch = (max_tiles(max_ctx, window, keep) + 7) / 8, R = H / p.G;
+  const int64_t ct = talk_chunk_tiles((int)H, groups.has_value());
+  const int64_t nch = (max_tiles(max_ctx, window > 0 ? window + nq - 1 : 0, keep) + ct - 1) / ct;
   p.nch = (int)nch;
-  p.s = f32p(s, n_rows * H * nch * 128, "s");
-  p.stat = f32p(stat, n_rows * H * nch * 2, "stat");
-  p.part = f32p(part, n_rows * nch * H * p.dv, "part");
+  p.s = f32p(s, n_rows * nq * H * nch * ct * 16, "s");
+  p.nst = (int)(nch * ct / kTalkStat);
+  p.stat = f32p(stat, n_rows * nq * H * p.nst * 2, "stat");
+  p.part = f32p(part, n_rows * nq * nch * H * p.dv, "part");
   i32p(counters, n_rows * p.G * ((R + 15) / 16), "counters");
   p.counters = counters.data_ptr<int>();
   check_rc(vwa_talk_attention(&p, cur_stream(q)), "talk_attention");
@@ -354,7 +367,8 @@ void bind_stack(py::module_& m) {
   m.def("talk_attention", &talk_attention, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("table"), py::arg("positions"),
         py::arg("seq_ids"), py::arg("slots"), py::arg("row_list"), py::arg("n_rows"), py::arg("H"), py::arg("scale"),
         py::arg("window"), py::arg("keep"), py::arg("talk"), py::arg("gate"), py::arg("out_scale"), py::arg("max_ctx"),
-        py::arg("s"), py::arg("stat"), py::arg("part"), py::arg("counters"), py::arg("out"));
+        py::arg("s"), py::arg("stat"), py::arg("part"), py::arg("counters"), py::arg("out"), py::arg("groups") = py::none(),
+        py::arg("nq") = 1);
   m.def("talk_prefill", &talk_prefill, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("table"), py::arg("positions"),
         py::arg("seq_ids"), py::arg("slots"), py::arg("tiles"), py::arg("H"), py::arg("scale"), py::arg("window"),
         py::arg("keep"), py::arg("talk_frag"), py::arg("gate"), py::arg("out_scale"), py::arg("max_ctx"), py::arg("splits"),

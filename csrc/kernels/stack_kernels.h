@@ -34,22 +34,28 @@ struct QkvCacheParams {
 // Attention over the visible keys of each row (j <= i and (i - j < window or j < keep); window 0: all)
 // with the heads' softmax weights mixed across heads (talk [H][H]; null: not mixed), an optional
 // per-head output gate sigmoid(gate[row][h]) and a constant output scale.
-// Keys are walked in 16-key tiles (a tile never crosses a cache block), dealt to workgroups in chunks of at most 8.
+// Keys are walked in 16-key tiles (a tile never crosses a cache block), dealt to workgroups in chunks of at most
+// talk_chunk_tiles (16 while the weights of 256 keys and all heads fit LDS, else 8).
+constexpr int kTalkStat = 4;        // tiles of a workgroup that scores
+inline int talk_chunk_tiles(int H, bool groups) { return !groups && H <= 128 ? 16 : 8; }
 struct TalkAttnParams {
   const void* q; int ldq;           // [rows, H * dk]
   const void* k; const void* v; int64_t k_sb, k_sh, v_sb, v_sh;
   const int* block_table; int table_stride, block_size;
   const int* positions; const int* seq_ids; const int64_t* slots;
   const int* row_list;              // rows this launch serves (null: 0 .. rows - 1)
+  const int* groups;                // [rows][2]: first row and count (<= nq) of consecutive positions of a sequence, or null
+  int nq;                           // rows of a unit the scratch holds (1 without groups; nq * H / G <= 16)
   int rows, H, G, dk, dv, f32;
   float scale; int window, keep;
   const float* talk;
   const void* gate; int ldg;        // [.., H] pre-activations (T) or null
   float out_scale;
   int nch;                          // chunks per row the scratch holds
-  float* s;                         // [rows][H][nch * 128] scores
-  float* stat;                      // [rows][H][nch][2] (max, sum) per chunk
-  float* part;                      // [rows][nch][H][dv] partial outputs
+  int nst;                          // statistics per (row, head): nch * talk_chunk_tiles / kTalkStat
+  float* s;                         // [rows][nq][H][nch * 16 talk_chunk_tiles] scores, by visible tile
+  float* stat;                      // [rows][nq][H][nst][2] (max, sum) of kTalkStat tiles
+  float* part;                      // [rows][nq][nch][H][dv] partial outputs
   int* counters;                    // [rows * G * ceil(H / G / 16)] chunk tickets, zero between launches
   void* out; int ldo;               // [.., H * dv] T
 };

@@ -9,7 +9,7 @@
 // Keys are walked in 16-key tiles inside cache blocks.  The visible tiles of a row are those of the
 // kept first keys, then those of the window (vis_tiles); edges are masked per key.
 //
-//  1) rows form (decode; any T, any sizes): launch A -- a workgroup per (row, kv head, 8 tiles)
+//  1) rows form (decode; any T, any sizes): launch A -- a workgroup per (row or few rows of a run, kv head, chunk of tiles)
 //     computes S^T = K.Q^T on the MFMA (the kv head's query heads are the 16 columns), stores the
 //     scores and the chunk's (max, sum) per head; launch B -- same grid -- folds the chunk statistics
 //     of every head, mixes the chunk's weights into LDS in B-operand order and multiplies by V^T,
@@ -54,69 +54,99 @@ VWA_DEVICE f32x4 ld_sc1_x4(__amdgpu_buffer_rsrc_t r, int off) {
 }
 
 // ------------------------------------------------------------------------------------------ rows form
-constexpr int kChunkTiles = 8;             // most tiles of a workgroup's chunk
-constexpr int kChunk = kTile * kChunkTiles;
+// A workgroup takes a unit of rows and a kv head: one row (its query heads are columns of the MFMA; decoded tokens) or
+// GRP: up to p.nq = 16 / R consecutive rows of a sequence (columns: row, query head), so that a key is read and multiplied
+// once for all of them.  777 rows of a 32-bit prompt, 8 / 4 heads of 128: both launches 332 -> 86 us per layer.
+//
+// Few rows are bound by the dependent round trips through memory (about 0.8 us each), not by bytes: everything whose address
+// is known is requested first; scores are spread by a tile per wave (kTalkStat tiles a workgroup); and a mixing chunk holds CT
+// = 16 tiles, so that contexts of up to 256 keys take no partial sums, tickets and merging.  1 row of 225 keys, 16 / 4 heads
+// of 128: scores 5.4 -> 4.8, mixing 9.9 -> 8.4 us; 48 rows of 90 .. 250 keys, 8 / 4 heads: 7.4 -> 6.7, 10.5 -> 8.2.
+constexpr int kWaves = 8;                      // of the mixing
+// (CT, most tiles of a chunk: talk_chunk_tiles)
 
-// A row's visible tiles are dealt evenly to the fewest chunks; chunk c holds tiles c * per ..
 struct Chunks {
   int per, n;
 };
+// the visible tiles are dealt evenly to the fewest chunks; chunk c holds tiles c * per ..
+template <int CT>
 VWA_DEVICE Chunks chunks_of(int tiles) {
-  const int k = (tiles + kChunkTiles - 1) / kChunkTiles, per = (tiles + k - 1) / k;
+  const int k = (tiles + CT - 1) / CT, per = (tiles + k - 1) / k;
   return Chunks{per, (tiles + per - 1) / per};
 }
 
-template <class T>
+struct Unit {
+  int row, cnt;    // first row, rows
+  bool live;       // false: an inert row of a padded step
+  int pos, seq;
+  Vis v;
+};
+template <bool GRP>
+VWA_DEVICE Unit unit_of(const TalkAttnParams& p, int ri) {
+  Unit u;
+  u.row = GRP ? p.groups[2 * ri] : p.row_list ? p.row_list[ri] : ri;
+  u.cnt = GRP ? p.groups[2 * ri + 1] : 1;
+  const int64_t slot = p.slots[u.row];  // (requested together)
+  u.pos = p.positions[u.row];
+  u.seq = p.seq_ids[u.row];
+  u.live = GRP || slot >= 0;
+  u.v = vis_tiles(u.pos, u.pos + u.cnt - 1, p.window, p.keep);
+  return u;
+}
+
+template <class T, bool GRP>
 __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
   using M = MM<T>;
-  constexpr int NU = kChunkTiles / 4;                // tiles per wave
+  constexpr int NU = kTalkStat / 4;                  // tiles per wave
   __shared__ float sm[4][16][2];
   const int ri = blockIdx.x / p.G, c = blockIdx.x % p.G, chunk = blockIdx.y, r0 = blockIdx.z * 16;
-  const int row = p.row_list ? p.row_list[ri] : ri;
-  if (p.slots[row] < 0) return;
-  const int pos = p.positions[row], seq = p.seq_ids[row];
-  const Vis v = vis_tiles(pos, pos, p.window, p.keep);
-  const Chunks ck = chunks_of(v.n);
-  if (chunk >= ck.n) return;
+  const Unit un = unit_of<GRP>(p, ri);
+  if (!un.live) return;
+  const Vis v = un.v;
+  if (chunk * kTalkStat >= v.n) return;
   const int R = p.H / p.G, Rb = min(16, R - r0);
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, b = lane >> 4;
-  const T* q = reinterpret_cast<const T*>(p.q) + (size_t)row * p.ldq + (size_t)(c * R + r0 + min(rl, Rb - 1)) * p.dk + b * M::EPL;
+  const int qi = GRP ? rl / R : 0, r = GRP ? rl % R : rl;  // this column's row of the unit and query head
+  const bool col = qi < un.cnt && r < Rb;
+  const T* q = reinterpret_cast<const T*>(p.q) + (size_t)(un.row + min(qi, un.cnt - 1)) * p.ldq +
+               (size_t)(c * R + r0 + min(r, Rb - 1)) * p.dk + b * M::EPL;
   const int lb = __builtin_ctz(p.block_size);
   const T* kp[NU];
   int key0[NU];
   bool ok[NU];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int lt = w + 4 * u, t = chunk * ck.per + lt;
-    ok[u] = lt < ck.per && t < v.n;
+    const int t = chunk * kTalkStat + w + 4 * u;
+    ok[u] = t < v.n;
     key0[u] = tile_of(v, ok[u] ? t : v.n - 1) * kTile;
-    const int64_t blk = p.block_table[(int64_t)seq * p.table_stride + (key0[u] >> lb)];
+    const int64_t blk = p.block_table[(int64_t)un.seq * p.table_stride + (key0[u] >> lb)];
     kp[u] = reinterpret_cast<const T*>(p.k) + blk * p.k_sb + (int64_t)c * p.k_sh +
             (int64_t)((key0[u] & (p.block_size - 1)) + rl) * p.dk + b * M::EPL;
   }
   f32x4 acc[NU] = {};
-#pragma unroll 4
+#pragma unroll 8
   for (int k = 0; k < p.dk; k += M::KS) {
     const uint4 qf = *reinterpret_cast<const uint4*>(q + k);
 #pragma unroll
     for (int u = 0; u < NU; ++u) acc[u] = M::mma(*reinterpret_cast<const uint4*>(kp[u] + k), qf, acc[u]);
   }
-  // lane (column rl = head, keys 4b .. 4b+3 of both tiles): mask, store, chunk statistics
+  // lane (column rl, keys 4b .. 4b+3 of its tiles): mask, store, chunk statistics
   float mx = -INFINITY;
 #pragma unroll
   for (int u = 0; u < NU; ++u)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const bool vis = ok[u] && sees(pos, key0[u] + 4 * b + i, p.window, p.keep);
+      const bool vis = ok[u] && sees(un.pos + qi, key0[u] + 4 * b + i, p.window, p.keep);
       acc[u][i] = vis ? acc[u][i] * p.scale : -INFINITY;
       mx = fmaxf(mx, acc[u][i]);
     }
-  if (rl < Rb) {
+  const size_t srow = (size_t)ri * p.nq + qi;         // scratch row
+  if (col) {
 #pragma unroll
     for (int u = 0; u < NU; ++u)
       if (ok[u])
-        *reinterpret_cast<float4*>(p.s + ((size_t)ri * p.H + c * R + r0 + rl) * p.nch * kChunk +
-                                   chunk * kChunk + (w + 4 * u) * kTile + 4 * b) =
+        *reinterpret_cast<float4*>(p.s + (srow * p.H + c * R + r0 + r) * p.nst * (kTalkStat * kTile) +
+                                   (chunk * kTalkStat + w + 4 * u) * kTile + 4 * b) =
             make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
   }
   mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -132,17 +162,16 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
     sm[w][rl][0] = mx;
     sm[w][rl][1] = l;
   }
-  __syncthreads();
-  if ((int)threadIdx.x < Rb) {
-    const int r = threadIdx.x;
-    float m = -INFINITY, s = 0.f;
+  lds_sync();
+  if (threadIdx.x < 16 && col) {                       // (thread = column: its qi and r)
+    float m = -INFINITY, sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m = fmaxf(m, sm[i][r][0]);
+    for (int i = 0; i < 4; ++i) m = fmaxf(m, sm[i][rl][0]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) s += sm[i][r][1] > 0.f ? sm[i][r][1] * __expf(sm[i][r][0] - m) : 0.f;
-    float* st = p.stat + (((size_t)ri * p.H + c * R + r0 + r) * p.nch + chunk) * 2;
+    for (int i = 0; i < 4; ++i) sum += sm[i][rl][1] > 0.f ? sm[i][rl][1] * __expf(sm[i][rl][0] - m) : 0.f;
+    float* st = p.stat + ((srow * p.H + c * R + r0 + r) * p.nst + chunk) * 2;
     st[0] = m;
-    st[1] = s;
+    st[1] = sum;
   }
 }
 
@@ -152,47 +181,68 @@ VWA_DEVICE float head_gate(const TalkAttnParams& p, int row, int h) {
   return p.out_scale / (1.f + __expf(-ldv(reinterpret_cast<const T*>(p.gate) + (size_t)row * p.ldg + h)));
 }
 
-// LDS: statistics [H][2], weights [H][keys] f32, mixed weights [keys / KS][64][16 B]
-template <class T>
-size_t mix_lds(int H) { return (size_t)H * (2 + kChunk) * 4 + kChunk * 16 * sizeof(T); }
+// LDS: mixed weights [keys / KS][64][16 B], weights [rows of the unit x heads][keys] f32, statistics [rows x heads][2]
+template <class T, int CT>
+size_t mix_lds(int H, int nq) {
+  constexpr int CH = CT * kTile;
+  return (size_t)nq * H * (2 + CH) * 4 + CH * 16 * sizeof(T);
+}
 
-template <class T>
-__global__ __launch_bounds__(256) void talk_mix_kernel(TalkAttnParams p) {
+template <class T, int CT, bool GRP>
+__global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p) {
   using M = MM<T>;
-  constexpr int HP = 256 / kChunk;                   // heads side by side over the threads
-  static_assert(HP == 2);
+  constexpr int CH = CT * kTile, NT = 64 * kWaves;
+  constexpr int HP = NT / CH;                        // (row, head)s side by side over the threads
+  static_assert(CH % 64 == 0 && HP >= 1);
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int s_last;
   const int ri = blockIdx.x / p.G, c = blockIdx.x % p.G, chunk = blockIdx.y, r0 = blockIdx.z * 16;
-  const int row = p.row_list ? p.row_list[ri] : ri;
+  const Unit un = unit_of<GRP>(p, ri);
   const int R = p.H / p.G, Rb = min(16, R - r0), h0 = c * R + r0;
-  T* out = reinterpret_cast<T*>(p.out) + (size_t)row * p.ldo;
-  if (p.slots[row] < 0) {  // inert row of a padded step
+  T* out = reinterpret_cast<T*>(p.out) + (size_t)un.row * p.ldo;
+  if (!un.live) {
     if (chunk == 0)
-      for (int i = threadIdx.x; i < Rb * p.dv; i += 256) stv(out + (size_t)h0 * p.dv + i, 0.f);
+      for (int i = threadIdx.x; i < Rb * p.dv; i += NT) stv(out + (size_t)h0 * p.dv + i, 0.f);
     return;
   }
-  const int pos = p.positions[row], seq = p.seq_ids[row];
-  const Vis v = vis_tiles(pos, pos, p.window, p.keep);
-  const Chunks ck = chunks_of(v.n);
+  const Vis v = un.v;
+  const Chunks ck = chunks_of<CT>(v.n);
   if (chunk >= ck.n) return;
+  const int nstat = (v.n + kTalkStat - 1) / kTalkStat;                  // statistics of a (row, head)
   const int nact = ck.n, t0 = chunk * ck.per, nt = min(ck.per, v.n - t0), nkey = nt * kTile;
+  const int g0 = p.talk ? 0 : h0, hn = p.talk ? p.H : Rb;               // heads whose weights are needed
+  const int nw = un.cnt * hn, ncol = un.cnt * Rb;
   T* pf = reinterpret_cast<T*>(smem);                                   // mixed weights, B-operand order
-  float* wt = reinterpret_cast<float*>(smem + kChunk * 16 * sizeof(T));  // [H][keys]
-  float* hm = wt + p.H * kChunk;                                        // [H] max
-  float* hl = hm + p.H;                                                 // [H] 1 / sum
-  const int g0 = p.talk ? 0 : h0, g1 = p.talk ? p.H : h0 + Rb;          // heads whose weights are needed
+  float* wt = reinterpret_cast<float*>(smem + CH * 16 * sizeof(T));     // [row][head][keys]
+  float* hm = wt + nw * CH;                                             // [row][head] max
+  float* hl = hm + nw;                                                  // [row][head] 1 / sum
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, b = lane >> 4;
-  // ---- everything that is read is requested first: the scores of this thread's (key, heads), the first
-  // value tiles of this wave (16-column tiles w, w + 4, ...), the chunk statistics
-  constexpr int kPre = 16 / HP;
-  const int j = threadIdx.x & (kChunk - 1), hp = w >> 1;                // key, first head
-  const float* srow = p.s + (size_t)ri * p.H * p.nch * kChunk + chunk * kChunk + j;
+  // ---- everything that is read is requested first: the scores of this thread's (key; row, head)s, the first value tiles
+  // of this wave (16-column tiles w, w + 8, ...), the mixing rows of this wave's columns, the gates, the chunk statistics
+  constexpr int kPre = GRP ? 16 : 8;
+  const int j = threadIdx.x & (CH - 1), hp = w / (CH / 64);             // key, first (row, head)
+  const size_t srow = (size_t)ri * p.nq;
+  const int64_t sld = (int64_t)p.nst * (kTalkStat * kTile);
+  const float* sbase = p.s + (srow * p.H + g0) * sld + t0 * kTile + j;
+  auto head_of = [&](int i) { return GRP ? (i / hn) * p.H + i % hn : i; };  // (row, needed head) i from the unit's first
+  auto score = [&](int i) -> const float* { return sbase + (int64_t)head_of(i) * sld; };
   float sv[kPre];
 #pragma unroll
-  for (int k = 0; k < kPre; ++k) sv[k] = srow[(size_t)min(g0 + hp + HP * k, g1 - 1) * p.nch * kChunk];
+  for (int k = 0; k < kPre; ++k) sv[k] = j < nkey ? *score(min(hp + HP * k, nw - 1)) : 0.f;
+  constexpr int kCols = 16 / HP;                                        // columns of a wave
+  const bool in_lanes = p.talk && p.H <= 64;                            // lane g holds the weight of head g
+  float tk[kCols];
+  if (in_lanes) {
+#pragma unroll
+    for (int i = 0; i < kCols; ++i)
+      tk[i] = p.talk[(size_t)(h0 + (GRP ? min(hp + HP * i, ncol - 1) % Rb : min(hp + HP * i, Rb - 1))) * p.H + min(lane, p.H - 1)];
+  }
+  const int qi = GRP ? rl / R : 0, r = GRP ? rl % R : rl;               // this column's row and query head
+  const bool col = qi < un.cnt && r < Rb;
+  float gate = 0.f;
+  if (nact == 1 && col) gate = !GRP || p.slots[un.row + qi] >= 0 ? head_gate<T>(p, un.row + qi, h0 + r) : 0.f;
   constexpr int TPS = M::KS / kTile;                 // tiles per step (bf16 2, f32 1)
-  constexpr int NST = kChunkTiles / TPS;
+  constexpr int NST = CT / TPS;
   const int lb = __builtin_ctz(p.block_size);
   const T* vb[NST];
   bool vok[NST];
@@ -201,23 +251,22 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(TalkAttnParams p) {
     const int lt = s * TPS + (TPS == 2 ? b >> 1 : 0);
     vok[s] = lt < nt;
     const int key = tile_of(v, vok[s] ? t0 + lt : v.n - 1) * kTile;
-    const int64_t blk = p.block_table[(int64_t)seq * p.table_stride + (key >> lb)];
+    const int64_t blk = p.block_table[(int64_t)un.seq * p.table_stride + (key >> lb)];
     vb[s] = reinterpret_cast<const T*>(p.v) + blk * p.v_sb + (int64_t)c * p.v_sh + (int64_t)rl * p.block_size +
             (key & (p.block_size - 1)) + (TPS == 2 ? (b & 1) : b) * M::EPL;
   }
-  uint4 va[NST], vn[NST];
-  auto load_v = [&](uint4 (&x)[NST], int d) {
+  uint4 va[NST];
+  auto load_v = [&](int d) {
 #pragma unroll
     for (int s = 0; s < NST; ++s)
-      x[s] = vok[s] ? *reinterpret_cast<const uint4*>(vb[s] + (int64_t)min(d, p.dv - 16) * p.block_size) : make_uint4(0, 0, 0, 0);
+      va[s] = vok[s] ? *reinterpret_cast<const uint4*>(vb[s] + (int64_t)min(d, p.dv - 16) * p.block_size) : make_uint4(0, 0, 0, 0);
   };
-  load_v(va, w * 16);
-  load_v(vn, w * 16 + 64);
-  // ---- statistics of every needed head: 16 lanes per head
-  for (int h = g0 + (threadIdx.x >> 4); h < g1; h += 16) {
-    const float* st = p.stat + ((size_t)ri * p.H + h) * p.nch * 2;
+  load_v(w * 16);
+  // ---- statistics of every needed (row, head): 16 lanes each
+  for (int i = threadIdx.x >> 4; i < nw; i += NT / 16) {
+    const float* st = p.stat + (srow * p.H + g0 + head_of(i)) * p.nst * 2;
     float m = -INFINITY, s = 0.f;
-    for (int k = threadIdx.x & 15; k < nact; k += 16) {
+    for (int k = threadIdx.x & 15; k < nstat; k += 16) {
       const float2 ms = *reinterpret_cast<const float2*>(st + 2 * k);
       const float mn = fmaxf(m, ms.x);
       if (ms.y > 0.f) s = (s > 0.f ? s * __expf(m - mn) : 0.f) + ms.y * __expf(ms.x - mn);
@@ -230,54 +279,60 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(TalkAttnParams p) {
       m = mn;
     }
     if ((threadIdx.x & 15) == 0) {
-      hm[h] = m;
-      hl[h] = 1.f / s;
+      hm[i] = m;
+      hl[i] = 1.f / s;
     }
   }
-  __syncthreads();
+  lds_sync();
   // ---- normalised weights of the chunk's keys (0 past the last tile)
-  auto weight = [&](int h, float s) { wt[h * kChunk + j] = j < nkey && s != -INFINITY ? __expf(s - hm[h]) * hl[h] : 0.f; };
+  auto weight = [&](int i, float s) { wt[i * CH + j] = j < nkey && s != -INFINITY ? __expf(s - hm[i]) * hl[i] : 0.f; };
 #pragma unroll
   for (int k = 0; k < kPre; ++k)
-    if (g0 + hp + HP * k < g1) weight(g0 + hp + HP * k, sv[k]);
-  for (int h = g0 + hp + HP * kPre; h < g1; h += HP) weight(h, srow[(size_t)h * p.nch * kChunk]);
-  __syncthreads();
-  // ---- mixed weights of this kv head's query heads
+    if (hp + HP * k < nw) weight(hp + HP * k, sv[k]);
+#pragma unroll 4
+  for (int i = hp + HP * kPre; i < nw; i += HP) weight(i, *score(i));
+  lds_sync();
+  // ---- mixed weights of this kv head's columns (row, query head)
   {
     const int idx = ((j / M::KS) * 64 + 16 * ((j % M::KS) / M::EPL)) * M::EPL + j % M::EPL;
-    for (int r = hp; r < Rb; r += HP) {
+#pragma unroll
+    for (int i = 0; i < kCols; ++i) {
+      const int cc = hp + HP * i, cr = GRP ? cc % Rb : cc;
+      if (cc >= ncol) break;                         // (uniform per wave)
+      const float* wr = wt + (GRP ? cc / Rb : 0) * hn * CH + j;
       float x = 0.f;
-      if (p.talk) {
-        const float* tk = p.talk + (size_t)(h0 + r) * p.H;  // (uniform per wave: scalar loads)
+      if (in_lanes) {
 #pragma unroll 8
-        for (int g = 0; g < p.H; ++g) x += tk[g] * wt[g * kChunk + j];
+        for (int g = 0; g < p.H; ++g)
+          x += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tk[i]), g)) * wr[g * CH];
+      } else if (p.talk) {
+        const float* t = p.talk + (size_t)(h0 + cr) * p.H;
+#pragma unroll 8
+        for (int g = 0; g < p.H; ++g) x += t[g] * wr[g * CH];
       } else {
-        x = wt[(h0 + r) * kChunk + j];
+        x = wr[cr * CH];
       }
-      stv(pf + idx + r * M::EPL, x);
+      stv(pf + idx + cc * M::EPL, x);
     }
   }
-  __syncthreads();
+  lds_sync();
   // ---- O^T = V^T . P^T
   const int nz = gridDim.z;
-  float* prow = p.part + ((size_t)ri * p.nch) * p.H * p.dv;
-  const __amdgpu_buffer_rsrc_t rp = rsrc_f32(prow, (int64_t)p.nch * p.H * p.dv);
-  for (int d = w * 16; d < p.dv; d += 64) {
+  float* prow = p.part + srow * p.nch * p.H * p.dv;
+  const __amdgpu_buffer_rsrc_t rp = rsrc_f32(prow, (int64_t)p.nq * p.nch * p.H * p.dv);
+  for (int d = w * 16; d < p.dv; d += 16 * kWaves) {
     f32x4 acc = {};
 #pragma unroll
     for (int s = 0; s < NST; ++s)
       acc = M::mma(va[s], *reinterpret_cast<const uint4*>(pf + ((size_t)s * 64 + lane) * M::EPL), acc);
-#pragma unroll
-    for (int s = 0; s < NST; ++s) va[s] = vn[s];
-    if (d + 128 < p.dv) load_v(vn, d + 128);
-    if (rl >= Rb) continue;
-    const int h = h0 + rl;
+    if (d + 16 * kWaves < p.dv) load_v(d + 16 * kWaves);
+    if (!col) continue;
+    const int h = h0 + r;
     if (nact == 1) {
-      const float g = head_gate<T>(p, row, h);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) stv(out + (size_t)h * p.dv + d + 4 * b + i, acc[i] * g);
+      for (int i = 0; i < 4; ++i) stv(out + (size_t)qi * p.ldo + (size_t)h * p.dv + d + 4 * b + i, acc[i] * gate);
     } else {
-      st_sc1_x4(rp, (int)((((int64_t)chunk * p.H + h) * p.dv + d + 4 * b) * 4), acc);
+      st_sc1_x4(rp, (int)(((((int64_t)qi * p.nch + chunk) * p.H + h) * p.dv + d + 4 * b) * 4), acc);
     }
   }
   if (nact == 1) return;
@@ -294,18 +349,20 @@ __global__ __launch_bounds__(256) void talk_mix_kernel(TalkAttnParams p) {
   __syncthreads();
   if (!s_last) return;
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  for (int i = threadIdx.x * 2; i < Rb * p.dv; i += 512) {
-    const int64_t o = (int64_t)h0 * p.dv + i;
+  const int per_row = Rb * p.dv;
+  for (int i = threadIdx.x * 2; i < un.cnt * per_row; i += 2 * NT) {
+    const int k0 = i / per_row, e = i % per_row, row = un.row + k0;
+    const int64_t o = (int64_t)h0 * p.dv + e;
     float a0 = 0.f, a1 = 0.f;
 #pragma unroll 8
     for (int k = 0; k < nact; ++k) {
-      const float2 x = ld_sc1_f2(rp, (int64_t)k * p.H * p.dv + o);
+      const float2 x = ld_sc1_f2(rp, ((int64_t)k0 * p.nch + k) * p.H * p.dv + o);
       a0 += x.x;
       a1 += x.y;
     }
-    const float g = head_gate<T>(p, row, h0 + i / p.dv);
-    stv(out + o, a0 * g);
-    stv(out + o + 1, a1 * g);
+    const float g = !GRP || p.slots[row] >= 0 ? head_gate<T>(p, row, h0 + e / p.dv) : 0.f;
+    stv(out + (size_t)k0 * p.ldo + o, a0 * g);
+    stv(out + (size_t)k0 * p.ldo + o + 1, a1 * g);
   }
 }
 
@@ -794,13 +851,13 @@ int check_attn(const TalkAttnParams& p) {
   return 0;
 }
 
-template <class T>
+template <class T, int CT, bool GRP>
 int launch_rows(const TalkAttnParams& p, hipStream_t st) {
-  const size_t lds = mix_lds<T>(p.H);
+  const size_t lds = mix_lds<T, CT>(p.H, p.nq);
   if (lds > kMaxLds - 64) return -5;
-  const dim3 grid(p.rows * p.G, p.nch, (p.H / p.G + 15) / 16), block(256);
-  hipLaunchKernelGGL((talk_scores_kernel<T>), grid, block, 0, st, p);
-  hipLaunchKernelGGL((talk_mix_kernel<T>), grid, block, lds, st, p);
+  const int nz = (p.H / p.G + 15) / 16;
+  hipLaunchKernelGGL((talk_scores_kernel<T, GRP>), dim3(p.rows * p.G, p.nst, nz), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((talk_mix_kernel<T, CT, GRP>), dim3(p.rows * p.G, p.nch, nz), dim3(64 * kWaves), lds, st, p);
   return (int)hipGetLastError();
 }
 
@@ -809,9 +866,15 @@ int launch_rows(const TalkAttnParams& p, hipStream_t st) {
 extern "C" int vwa_talk_attention(const TalkAttnParams* p, hipStream_t st) {
   const int rc = check_attn(*p);
   if (rc) return rc;
-  if (p->nch < 1 || !p->s || !p->stat || !p->part || !p->counters) return -4;
-  if ((int64_t)p->nch * p->H * p->dv * 4 >= (1ll << 31)) return -5;
-  return p->f32 ? launch_rows<float>(*p, st) : launch_rows<u16>(*p, st);
+  if (p->nch < 1 || p->nst < 1 || !p->s || !p->stat || !p->part || !p->counters) return -4;
+  if (p->nq < 1 || (int64_t)p->nq * p->nch * p->H * p->dv * 4 >= (1ll << 31)) return -5;
+  if (p->groups) {
+    if (p->nq * (p->H / p->G) > 16) return -6;
+    return p->f32 ? launch_rows<float, 8, true>(*p, st) : launch_rows<u16, 8, true>(*p, st);
+  }
+  if (p->nq != 1) return -6;
+  if (talk_chunk_tiles(p->H, 0) == 16) return p->f32 ? launch_rows<float, 16, false>(*p, st) : launch_rows<u16, 16, false>(*p, st);
+  return p->f32 ? launch_rows<float, 8, false>(*p, st) : launch_rows<u16, 8, false>(*p, st);
 }
 
 extern "C" int64_t vwa_talk_prefill_part(int H, int G, int dk, int dv) {

@@ -47,8 +47,15 @@ def plan_runs(runs: Sequence[Tuple[int, int]], device, max_pos: int, scan_rows: 
         t = torch.tensor(x, dtype=torch.int32).view(-1, cols)
         return t.pin_memory().to(device, non_blocking=True) if torch.device(device).type == "cuda" else t
 
+    def groups(n: int):
+        """[first row, rows] of the runs cut into groups of at most n rows (made once for each n)."""
+        if n not in made:
+            made[n] = dev([[r0 + i, min(n, k - i)] for r0, k, *_ in runs for i in range(0, k, n)], 2)
+        return made[n]
+
+    made: dict = {}
     return SimpleNamespace(max_pos=max_pos, tiles=dev(tiles, 2) if tiles else None, chunks=dev(chunks, 4),
-                           singles=dev(singles, 1).view(-1) if singles else None)
+                           singles=dev(singles, 1).view(-1) if singles else None, groups=groups)
 
 
 def visible_tiles(max_ctx: int, window: int, keep: int) -> int:
@@ -57,9 +64,17 @@ def visible_tiles(max_ctx: int, window: int, keep: int) -> int:
     return min(tiles, -(-keep // 16) + (window + 14) // 16 + 1) if window > 0 else tiles
 
 
-def visible_chunks(max_ctx: int, window: int, keep: int) -> int:
-    """128-key chunks a row can see at most: sizes the rows-form scratch."""
-    return -(-visible_tiles(max_ctx, window, keep) // 8)
+def chunk_tiles(heads: int, groups: bool = False) -> int:
+    """Most tiles of a rows-form chunk (stack_kernels.h talk_chunk_tiles)."""
+    return 16 if heads <= 128 and not groups else 8
+
+
+def rows_scratch(units: int, nq: int, H: int, G: int, dv: int, max_ctx: int, window: int, keep: int, groups: bool = False):
+    """Numbers the rows form keeps of ``units`` units of at most nq rows: scores, statistics, partial outputs, tickets."""
+    ct = chunk_tiles(H, groups)
+    n = -(-visible_tiles(max_ctx, window + nq - 1 if window > 0 else 0, keep) // ct)
+    rows = units * nq
+    return rows * H * n * ct * 16, rows * H * n * ct // 4 * 2, rows * n * H * dv, units * G * -(-(H // G) // 16)
 
 
 class TalkScratch:
@@ -68,16 +83,11 @@ class TalkScratch:
 
     def __init__(self, layers: Sequence[Tuple[int, int, int, int, int]], max_ctx: int, device):
         """layers: (query heads, kv heads, dv, window, keep) of every layer."""
-        s = stat = part = cnt = 1
-        for H, G, dv, window, keep in layers:
-            n = visible_chunks(max_ctx, window, keep)
-            s, stat = max(s, H * n * 128), max(stat, H * n * 2)
-            part, cnt = max(part, n * H * dv), max(cnt, G * -(-(H // G) // 16))
+        sizes = [rows_scratch(ROW_SLICE, 1, H, G, dv, max_ctx, window, keep) for H, G, dv, window, keep in layers]
+        s, stat, part, cnt = (max(x) for x in zip(*sizes))
         f32 = dict(dtype=torch.float32, device=device)
-        self.s = torch.zeros(ROW_SLICE * s, **f32)
-        self.stat = torch.zeros(ROW_SLICE * stat, **f32)
-        self.part = torch.zeros(ROW_SLICE * part, **f32)
-        self.counters = torch.zeros(ROW_SLICE * cnt, dtype=torch.int32, device=device)
+        self.s, self.stat, self.part = (torch.zeros(n, **f32) for n in (s, stat, part))
+        self.counters = torch.zeros(cnt, dtype=torch.int32, device=device)
 
 
 # ----------------------------------------------------------------------------- ops
@@ -194,6 +204,20 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
             for i in range(0, n, ROW_SLICE):
                 lst = plan.singles[i : min(n, i + ROW_SLICE)]
                 rows_form(q, positions, seq_ids, slots, gate, out, lst, lst.shape[0])
+        return out
+    nq = min(16 // (n_q_heads // G), (140 << 10) // (520 * n_q_heads)) if n_q_heads // G <= 16 else 1
+    if plan is not None and nq > 1:  # a prompt: groups of consecutive rows, as many a launch as 64 MB of scores hold
+        from . import scratch as ws
+
+        groups = plan.groups(nq)
+        size = lambda n: rows_scratch(n, nq, n_q_heads, G, dv, max_ctx, window, keep, True)  # noqa: E731
+        step = max(1, min(groups.shape[0], (16 << 20) // size(1)[0]))
+        s, stat, part, cnt = size(step)
+        bufs = (ws(q.device, "talk_s", s), ws(q.device, "talk_stat", stat), ws(q.device, "talk_rows", part), _tickets(q.device, cnt))
+        for i in range(0, groups.shape[0], step):
+            lst = groups[i : i + step]
+            E.talk_attention(q, k_cache, v_cache, block_table, positions, seq_ids, slots, None, lst.shape[0], n_q_heads, scale,
+                             window, keep, talk, gate, out_scale, max_ctx, *bufs, out, groups=lst, nq=nq)
         return out
     for i in range(0, rows, ROW_SLICE):
         j = min(rows, i + ROW_SLICE)
