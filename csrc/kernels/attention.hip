@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_mq_kernel(DecodeAttnParams
   mq_body<D, G, kWaves, false>(p, lds, (int)gridDim.x, (int)blockIdx.x);
 }
 
-constexpr int kMqMaxGrid = 512;  // two 67 KB-LDS workgroups per CU: the whole grid is resident
+constexpr int kMqMaxGrid = 512;  // two workgroups per CU (D = 64: both resident)
 
 template <int D>
 int dispatch_mq(const DecodeAttnParams& p, hipStream_t st) {

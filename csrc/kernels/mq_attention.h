@@ -34,12 +34,12 @@ VWA_DEVICE float ld_sc1_f1(__amdgpu_buffer_rsrc_t r, int64_t idx) {
 // 3) multi-query MFMA decode attention (default; ops.set_attention_impl("split") selects 1)
 // ------------------------------------------------------------------------------------------
 // Work item = (row group, kv head, key chunk), one 4-wave workgroup each; the grid is capped at
-// 512 resident workgroups that walk the items.  A row group is a run of up to 16/G
+// 512 workgroups that walk the items.  A row group is a run of up to 16/G
 // consecutive rows of ONE sequence (the last sampled token plus its jump-forward rows, a
 // prompt-suffix chunk, Whisper's prompt rows), so its K/V bytes are read once for all of its
 // rows x GQA heads: the 16 MFMA query columns are (row, q-head) pairs.  The number of chunks
-// per (group, kv head) is chosen in-kernel from the step's actual group count so the items
-// fill the grid: a lone decode row spreads its context over up to 16 chunks, 32 concurrent
+// per (group, kv head) is chosen in-kernel from the step's actual group count and contexts so the
+// busiest CU ends first: a lone decode row spreads its context over many chunks, 32 concurrent
 // sessions get one chunk each (measured first version with a static rows x heads x 16 grid:
 // 64 rows of one sequence spent most of 89 us dispatching workgroups that exit at once).
 // Per 32-key step a wave computes
@@ -56,6 +56,7 @@ VWA_DEVICE float ld_sc1_f1(__amdgpu_buffer_rsrc_t r, int64_t idx) {
 // of them), and they merge in-launch through the sc1 hand-off + last-arriver ticket above.
 constexpr int kMqCols = 16;                 // query columns per workgroup (group rows x G)
 constexpr int kMqStep = 32;                 // keys per wave step
+constexpr int kMqCus = 256;                 // CUs of the chip
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
@@ -163,7 +164,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   int& s_last = *reinterpret_cast<int*>(lds + L::last);
 
   const int nkv = p.n_kv_heads, nq = p.n_q_heads;
-  const int lane = VWA_TX & 63, w = VWA_TX >> 6;
+  const int lane = VWA_TX & 63, w = FINE ? VWA_TX >> 6 : __builtin_amdgcn_readfirstlane(VWA_TX >> 6);
   const int n = lane & 15, g = lane >> 4;
 
   // ---- row groups of the whole step (<= 64 rows; every wave derives the same answer): runs of
@@ -253,12 +254,32 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   static_assert(!FINE || NW == 8, "the FINE merge pairs two threads per (column, slice): 512 threads");
   // cascade: n_pc prefix chunks + up to RG own-key chunks (one per sequence run of the group) per
   // group -- the partial slots 0 .. n_pc + RG - 1
-  // (standalone kernel: about one item per CU -- grid / 2 -- measured best over the chunk cap,
-  // tools/attn_probe.py --split-sweep, profiles/r4_attn_split_sweep.jsonl: e.g. 8 sessions 14.5 vs
-  // 21.2 us with a full-grid split, 16 grouped sessions 14.7 vs 23.2 us)
-  const int tgt = FINE ? grid : max(1, grid / 2);
-  const int n_pc = cascade ? max(1, min(p.n_splits - RG, tgt / max(1, n_groups * nkv) - RG)) : 0;
-  const int n_eff = cascade ? n_pc + RG : max(1, min(FINE ? min(p.n_splits, 16) : p.n_splits, tgt / max(1, n_groups * nkv)));
+  const int gh = max(1, n_groups * nkv);
+  int n_eff, n_pc = 0;
+  if constexpr (FINE) {
+    n_eff = max(1, min(min(p.n_splits, 16), grid / gh));
+  } else if (cascade) {
+    // one item per CU over prefix and own chunks, and prefix chunks for half of the CUs where the own
+    // chunks alone take them all (they are short): 32 sessions x 8 kv heads of D = 128 behind 1008
+    // shared keys (gh = 64) measured 24.4 / 18.7 / 21.1 us at 1 / 2 / 4 prefix chunks
+    n_pc = max(1, min(p.n_splits - RG, max(kMqCus / gh - RG, kMqCus / 2 / gh)));
+    n_eff = n_pc + RG;
+  } else {
+    // the count whose busiest CU ends first, counted in keys (lane c - 1: c chunks): its items' keys,
+    // what each chunk adds to the merge (0.3 - 0.5 us) and what every further item adds (~0.7 us; ~4 us
+    // where one workgroup's registers fill a CU, D = 128).  Measured (us at 1 / 2 / 3 / 4 / 6 chunks):
+    // 20 heads of D = 64 x 1500 keys, 1 row 16.1 / 12.6 / 11.3 / 9.9 / 10.4 and 8 rows 21.3 / 22.5 /
+    // 19.7; 8 kv heads of D = 128 x 1110 keys, 4 rows 19.0 / 15.5 / 12.9 / 12.9 / 11.8 and 16 rows
+    // 23.2 / 21.0 / 27.1
+    const int ctx_all = (int)wave_max((float)cl);
+    const int c = min(lane + 1, p.n_splits);
+    const int len = ((ctx_all + c - 1) / c + kChunk - 1) / kChunk * kChunk;
+    const int cnt = len > 0 ? (ctx_all + len - 1) / len : 1;
+    const int per_cu = (gh * cnt + kMqCus - 1) / kMqCus;
+    const int cost = per_cu * len + (cnt > 1 ? cnt * (D == 64 ? 70 : 30) : 0) + (per_cu - 1) * (D == 64 ? 100 : 350);
+    const float best = wave_max(-(float)cost);
+    n_eff = __builtin_ctzll(__ballot((float)cost == -best)) + 1;
+  }
   const int n_items = plan ? __builtin_amdgcn_readlane(ev, 0) : n_groups * nkv * n_eff;
   if (n_items_out) *n_items_out = n_items;
   if (n_final_out) *n_final_out = plan ? __builtin_amdgcn_readlane(ev, 1) : n_groups * nkv;
@@ -388,10 +409,36 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   const int kmax = kend - 1;  // keys past the chunk are clamped (finite data, masked scores)
   if (item == bid) stamp(20);
 
+  // ---- block ids (standalone kernel): lane j holds the cache offsets of the two 16-key halves of
+  //      the wave's step 64 i + j, one table round trip per 64 steps; a step reads its pair into
+  //      scalars.  Where a half lies in one block: halves start at multiples of 16 and the block size
+  //      is one, or the whole context is one block (the cross-attention's 1500 keys).  (A table load
+  //      per key instead is a dependent round trip in front of every step's K/V loads, and its wait
+  //      also waits for the step before's: nothing overlapped.  8 rows x 20 heads x 1500 keys of
+  //      D = 64: 28.9 -> 21.3 us; 1 row x 8 kv heads x 1110 keys of D = 128 in 4 chunks: 19.0 -> 12.6 us.)
+  const int bs = p.kv.block_size;
+  const bool halves = !FINE && (bs >= kend || (bs % 16 == 0 && kbeg % 16 == 0));
+  int64_t tabA = 0, tabB = 0;
+  auto load_tab = [&](int s0) {
+    const int ka = min(wb + (s0 + lane) * kMqStep, kmax), kb = min(ka + 16, kmax);
+    const int ia = ka / bs, ib = kb / bs;
+    gint* tab = (gint*)(p.kv.block_table + (int64_t)kv_seq * p.kv.table_stride);
+    const int ba = tab[ia], bb = tab[ib];
+    tabA = ba * p.kv.stride_block + (ka - ia * bs) * p.kv.stride_tok;
+    tabB = bb * p.kv.stride_block + (kb - ib * bs) * p.kv.stride_tok;
+  };
+  auto lane64 = [](int64_t v, int l) {
+    return (int64_t)(((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(v >> 32), l) << 32) |
+                     (unsigned)__builtin_amdgcn_readlane((int)v, l));
+  };
+  if constexpr (!FINE) {
+    if (halves && nsteps > 0) load_tab(0);
+  }
+
   // ---- Q^T fragments (B operand): Q[column n][dims 32ks + 8g ..], pre-scaled by scale*log2(e)
   bf16x8 qf[NKS];
-  auto make_qf = [&]() {
-    const float qs = p.scale * 1.4426950408889634f;
+  uint4 qraw[NKS];
+  auto load_q = [&]() {
     const int64_t qo = (int64_t)(r0 + min(rho, nr - 1)) * p.ldq + (kvh * G + n % G) * D + 8 * g;
     // FINE (the chained launch): Q is written by the QKV phase of the same launch when several
     // layers run in one launch (chain_kernel MULTI), possibly on another XCD whose L2 line this
@@ -400,24 +447,25 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
         const_cast<u16*>(p.q), (short)0, FINE ? (int)((int64_t)p.rows * p.ldq * 2) : 0, 0x00020000);
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {
-      float f[8];
       if constexpr (FINE) {
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r_q, (int)((qo + 32 * ks) * 2), 0, 16);
-        unpack8(make_uint4(v.x, v.y, v.z, v.w), f);
+        qraw[ks] = make_uint4(v.x, v.y, v.z, v.w);
       } else {
-        unpack8(ld128(p.q + qo + 32 * ks), f);
+        qraw[ks] = ld128(p.q + qo + 32 * ks);
       }
+    }
+  };
+  auto make_qf = [&]() {
+    const float qs = p.scale * 1.4426950408889634f;
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+      float f[8];
+      unpack8(qraw[ks], f);
 #pragma unroll
       for (int j = 0; j < 8; ++j) f[j] = rho < nr ? f[j] * qs : 0.f;
       qf[ks] = as_bf16x8(pack8(f));
     }
   };
-  if constexpr (DB) {
-    make_qf();
-    if (item == bid) stamp(10);  // q fragments in registers
-  }
-  // (measured: staging the wave's block-table entries in lanes and fetching them with __shfl,
-  // instead of the per-key table loads below, was 1.5-3 us SLOWER on every shape)
   const int2 rtr = r0 == 0 ? rt[0] : r0 == 1 ? rt[1] : r0 == 2 ? rt[2] : rt[3];  // the group's row table
 
   // K: A-operand row n of tile t is key kb + 8(n>>2) + 4t + (n&3) (so the S^T accumulator of lane
@@ -426,7 +474,8 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   // loads back to back -- no wait between them
   // (the two block-id sources in separate uniform branches, each finishing its offsets: a shared
   // helper left a vmcnt(0) at every join, which also waited for the Q loads in flight)
-  auto load_step = [&](int kb, uint4 (&kr)[2][NKS], uint4 (&vr)[NVL]) {
+  auto load_step = [&](int s, uint4 (&kr)[2][NKS], uint4 (&vr)[NVL]) {
+    const int kb = wb + s * kMqStep;
     int64_t ko[2], vo[NVL];
     auto offsets = [&](auto off) {
 #pragma unroll
@@ -445,6 +494,12 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       const int64_t hoff = (int64_t)kvh * p.kv.stride_head;
       const int st = (int)p.kv.stride_tok;
       offsets([&](int key) -> int64_t { return ((key & 16) ? bB : bA) + hoff + (key & 15) * st; });
+    } else if (halves) {
+      if (s > 0 && (s & 63) == 0) load_tab(s);
+      const int64_t hoff = (int64_t)kvh * p.kv.stride_head;
+      const int64_t oA = lane64(tabA, s & 63) + hoff, oB = lane64(tabB, s & 63) + hoff;
+      const int st = (int)p.kv.stride_tok;
+      offsets([&](int key) -> int64_t { return (((key - kb) & 16) ? oB : oA) + ((key - kb) & 15) * st; });
     } else {
       offsets([&](int key) -> int64_t { return kv_offset(p.kv, kv_seq, kvh, key); });
     }
@@ -513,13 +568,16 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   if constexpr (DB) {
     if (nsteps > 0) {
       uint4 kA[2][NKS], vA[NVL], kB[2][NKS], vB[NVL];
-      load_step(wb, kA, vA);
+      load_q();  // (in flight with the block ids; scaled behind the first two steps' loads)
+      load_step(0, kA, vA);
+      if (nsteps > 1) load_step(1, kB, vB);
+      make_qf();
       for (int s = 0; s < nsteps; s += 2) {
-        if (s + 1 < nsteps) load_step(wb + (s + 1) * kMqStep, kB, vB);
         compute_step(wb + s * kMqStep, kA, vA);
         if (s + 1 >= nsteps) break;
-        if (s + 2 < nsteps) load_step(wb + (s + 2) * kMqStep, kA, vA);
+        if (s + 2 < nsteps) load_step(s + 2, kA, vA);
         compute_step(wb + (s + 1) * kMqStep, kB, vB);
+        if (s + 3 < nsteps) load_step(s + 3, kB, vB);
       }
     }
   } else {  // single register set (the chained launch holds the next GEMM's weights meanwhile)
@@ -529,8 +587,9 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     for (int s = FINE ? w : 0; s < nsteps; s += FINE ? kWv : 1) {
       uint4 kA[2][NKS], vA[NVL];
       if (item == bid && s == w) stamp(13);  // (diagnostic: about to issue the first K/V step)
-      load_step(wb + s * kMqStep, kA, vA);
+      load_step(s, kA, vA);
       if (!have_q) {
+        load_q();
         make_qf();
         have_q = true;
       }

@@ -303,6 +303,34 @@ def test_decode_attention_cross_contiguous(attn_impl):
     close(out, exp, 2e-2)
 
 
+@pytest.mark.parametrize("hd,nq,nkv,bs,ctx,splits", [
+    (64, 2, 2, 16, [8730, 8193, 31, 1], 1),     # more than 64 steps a wave: the block ids load again
+    (128, 8, 2, 48, [257, 1000, 49, 16], None),  # blocks of three halves
+    (64, 4, 4, 24, [300, 24, 25, 7], None),      # halves across blocks: a table entry per key
+    (128, 4, 1, 8, [130, 513, 9, 128], None),
+    (64, 3, 3, 1009, [1009, 1008, 17, 992], None),  # one odd block for the whole context
+    (128, 8, 8, 16, [600] * 48, None),           # more items than workgroups
+])
+def test_decode_attention_block_sizes(hd, nq, nkv, bs, ctx, splits):
+    rows, per = len(ctx), -(-max(ctx) // bs)
+    seqs = min(rows, 4)
+    kc, vc = rnd(seqs * per, nkv, bs, hd), rnd(seqs * per, nkv, bs, hd)
+    table = torch.randperm(seqs * per, device=DEV)[:seqs * per].view(seqs, per).to(torch.int32)
+    seq_ids = torch.tensor([i % seqs for i in range(rows)], dtype=torch.int32, device=DEV)
+    ctx_lens = torch.tensor(ctx, dtype=torch.int32, device=DEV)
+    q = rnd(rows, nq * hd)
+    out = torch.empty_like(q)
+    cnt = torch.zeros(rows * nkv, dtype=torch.int32, device=DEV)
+    for _ in range(2):
+        ops.decode_attention(q, ops.KVLayout.paged(kc, vc, table), ctx_lens, seq_ids, n_q_heads=nq, n_kv_heads=nkv,
+                             head_dim=hd, scale=hd ** -0.5, max_ctx=per * bs, out=out, counters=cnt, n_splits=splits)
+    assert int(cnt.abs().sum()) == 0
+    exp = ref.decode_attention(q.cpu(), ops.KVLayout.paged(kc.cpu(), vc.cpu(), table.cpu()), ctx_lens.cpu(),
+                               seq_ids.cpu(), n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, scale=hd ** -0.5,
+                               out=torch.empty(rows, nq * hd, dtype=BF))
+    close(out, exp, 2e-2)  # q, the weights and the output are rounded to bf16 (2^-9 each; scores are ~N(0, 1))
+
+
 def test_flash_attention_causal_paged_prefix():
     hd, nq, nkv, bs = 128, 8, 2, 16
     blocks = 40
