@@ -68,7 +68,8 @@ struct Cfg {
   static constexpr int NCOL_MAX = BN / WN;
   static constexpr int EPI_LDS = NW * (FM * 16) * (NCOL_MAX * 2 + 16);
   static constexpr int LDS = 2 * STAGE > EPI_LDS ? 2 * STAGE : EPI_LDS;
-  static constexpr int W8LDS = 2 * W8STAGE > EPI_LDS ? 2 * W8STAGE : EPI_LDS;
+  static constexpr int W8NST = BM <= 32 ? 3 : 2;  // its stage buffers: what lets two workgroups share a CU
+  static constexpr int W8LDS = W8NST * W8STAGE > EPI_LDS ? W8NST * W8STAGE : EPI_LDS;
   static_assert((BM / 8) % NW == 0 && (BN / 8) % NW == 0, "whole LDS-DMA instructions per wave");
 };
 using CfgS = Cfg<128, 128, 2, 2>;
@@ -76,6 +77,10 @@ using CfgS = Cfg<128, 128, 2, 2>;
 // of fp8 weights each -- the W8A8 kernel's weight bytes per stage: a half-k-group bf16-style stage
 // carried 8 KB and measured 1.25x slower whole decode steps), 2 workgroups per CU
 using CfgW8 = Cfg<64, 128, 1, 4>;
+// ... of <= 32 rows: 24 KB stages, so three fit where two did and two are in flight behind the one being read (a slice of a
+// 32-row step is weights arriving and little else: with the sum of the slices, 4096 x 4096 14.6 -> 11.4 us, 4096 x 14336
+// 27.9 -> 24.7, 28672 x 4096 35.6 -> 33.1)
+using CfgW8s = Cfg<32, 128, 1, 4>;
 
 // A-image slot swizzle: chunk c of row r sits at slot c ^ F((r >> 1) & 7).  F makes every
 // ds_read_b128 lane group ({0-3,12-15,20-27}, {4-11,16-19,28-31}, ... : two k-chunk columns g,
@@ -341,7 +346,12 @@ VWA_DEVICE void store_out(const GemmParams& p, int m, int n, float v) {
 // EPI_QKV: output chunk n .. n+7 (o) of row m and its rotation partner n^8 (q) -> rotary (q / k
 // heads) -> q_out or the paged K / V caches, 16-byte stores.  Within a head (permuted rows) the
 // chunk at column 16 t + 8 hi holds dims hi * hd/2 + 8 t .. + 8, its partner the other half.
-VWA_DEVICE void qkv_store(const GemmParams& p, int m, int n, const float (&o)[8], const float (&q)[8]) {
+//   rope: the row's (cos, sin) of the chunk's 8 dims (use_rope); slot: the row's cache slot
+VWA_DEVICE const float4* rope_at(const GemmParams& p, int pos, int n) {
+  return reinterpret_cast<const float4*>(p.rope + ((size_t)pos * (p.head_dim >> 1) + 8 * ((n % p.head_dim) >> 4)) * 2);
+}
+VWA_DEVICE void qkv_store(const GemmParams& p, int m, int n, const float (&o)[8], const float (&q)[8],
+                          const float4 (&rope)[4], int64_t slot) {
   const int hd = p.head_dim, half = hd >> 1;
   const int head = n / hd, wc = n % hd;
   const int t = wc >> 4;
@@ -349,10 +359,9 @@ VWA_DEVICE void qkv_store(const GemmParams& p, int m, int n, const float (&o)[8]
   const bool is_v = head >= p.n_q_heads + p.n_kv_heads;
   float y[8];
   if (p.use_rope && !is_v) {
-    const float4* cs = reinterpret_cast<const float4*>(p.rope + ((size_t)p.positions[m] * half + 8 * t) * 2);
 #pragma unroll
     for (int e2 = 0; e2 < 4; ++e2) {
-      const float4 v = cs[e2];  // (cos, sin) of dims 2 e2, 2 e2 + 1
+      const float4 v = rope[e2];  // (cos, sin) of dims 2 e2, 2 e2 + 1
       const int e = 2 * e2;
       y[e] = hi ? o[e] * v.x + q[e] * v.y : o[e] * v.x - q[e] * v.y;
       y[e + 1] = hi ? o[e + 1] * v.z + q[e + 1] * v.w : o[e + 1] * v.z - q[e + 1] * v.w;
@@ -366,7 +375,6 @@ VWA_DEVICE void qkv_store(const GemmParams& p, int m, int n, const float (&o)[8]
     *reinterpret_cast<uint4*>(p.q_out + (size_t)m * p.ldq + head * hd + d) = pack8(y);
     return;
   }
-  const int64_t slot = p.slots[m];
   if (slot < 0) return;
   const int kvh = is_v ? head - p.n_q_heads - p.n_kv_heads : head - p.n_q_heads;
   const int64_t idx = (slot / p.block_size) * p.cache_sb + kvh * p.cache_sh + (slot % p.block_size) * p.cache_st;
@@ -433,29 +441,65 @@ VWA_DEVICE void sum_items(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, int m
   }
 }
 
+// what the epilogue of an item reads besides the slabs, requested in front of them: behind the sums each was one more
+// dependent round trip (two with the rotary row), and a reduction of few rows is nothing else (32 rows x 8 slices: 4096
+// columns 5.8 -> 5.1 us, 6144 with the rotation 7.3 -> 5.5)
+template <int EPI> struct ItemPre {
+  float scale, swa[8], swb[8], ba[8], bb[8];
+  uint4 r[2];      // residual: 8 bf16 (r[0]) or f32
+  float4 rope[4];
+  int64_t slot;
+};
+template <int EPI>
+VWA_DEVICE ItemPre<EPI> item_pre(const GemmParams& p, int m, int c) {
+  ItemPre<EPI> q;
+  const int n0 = item_src0<EPI>(c), n1 = item_src1<EPI>(c);
+  const int pos = EPI == EPI_QKV && p.use_rope ? p.positions[m] : 0;
+  q.slot = EPI == EPI_QKV ? p.slots[m] : 0;
+  const float sx = p.sx ? p.sx[m] : 1.f;
+  q.scale = row_scale(p, m) * sx;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    q.swa[e] = p.sw ? p.sw[n0 + e] : 1.f;
+    q.ba[e] = EPI == EPI_SWIGLU ? 0.f : bias_at(p, n0 + e);
+    if constexpr (kTwoSrc<EPI>) q.swb[e] = p.sw ? p.sw[n1 + e] : 1.f;
+    if constexpr (EPI == EPI_QKV) q.bb[e] = bias_at(p, n1 + e);
+  }
+  if (p.y_f32 == 2) {  // f32 residual stream: 16-byte accesses (rows are 32-byte aligned)
+    const uint4* r = reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(p.R) + (size_t)m * p.ldr + c);
+    q.r[0] = r[0];
+    q.r[1] = r[1];
+  } else if (kResid<EPI> && !p.y_f32) {
+    q.r[0] = *reinterpret_cast<const uint4*>(p.R + (size_t)m * p.ldr + c);
+  }
+  if (EPI == EPI_QKV && p.use_rope) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) q.rope[e] = rope_at(p, pos, c)[e];
+  }
+  return q;
+}
+
 // epilogue of one summed item + its stores
 // returns the sum of squares of the stored bf16 values (residual epilogue with ss_out; else 0)
 template <int EPI>
-VWA_DEVICE float finish_item(const GemmParams& p, int m, int c, const float (&a)[8], float (&b)[8]) {
-  const float rs = row_scale(p, m) * (p.sx ? p.sx[m] : 1.f);
-  const int n0 = item_src0<EPI>(c), n1 = item_src1<EPI>(c);
+VWA_DEVICE float finish_item(const GemmParams& p, const ItemPre<EPI>& q, int m, int c, const float (&a)[8], float (&b)[8]) {
+  const float rs = q.scale;
   float v[8];
   if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float gs = p.sw ? p.sw[n0 + e] : 1.f, us = p.sw ? p.sw[n1 + e] : 1.f;
-      v[e] = silu(a[e] * gs * rs) * (b[e] * us * rs);
+      v[e] = silu(a[e] * q.swa[e] * rs) * (b[e] * q.swb[e] * rs);
     }
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      v[e] = a[e] * rs * (p.sw ? p.sw[c + e] : 1.f) + bias_at(p, c + e);
+      v[e] = a[e] * rs * q.swa[e] + q.ba[e];
       if constexpr (kGelu<EPI>) v[e] = gelu_erf(v[e]);
     }
     if constexpr (EPI == EPI_QKV) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) b[e] = b[e] * rs * (p.sw ? p.sw[n1 + e] : 1.f) + bias_at(p, n1 + e);
-      qkv_store(p, m, c, v, b);
+      for (int e = 0; e < 8; ++e) b[e] = b[e] * rs * q.swb[e] + q.bb[e];
+      qkv_store(p, m, c, v, b, q.rope, q.slot);
       return 0.f;
     }
   }
@@ -467,10 +511,9 @@ VWA_DEVICE float finish_item(const GemmParams& p, int m, int c, const float (&a)
       return 0.f;
     }
   }
-  if (p.y_f32 == 2) {  // f32 residual stream: 16-byte accesses (rows are 32-byte aligned)
-    const float4* r = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p.R) + (size_t)m * p.ldr + c);
+  if (p.y_f32 == 2) {
     float4* y = reinterpret_cast<float4*>(reinterpret_cast<float*>(p.Y) + (size_t)m * p.ldy + c);
-    const float4 r0 = r[0], r1 = r[1];
+    const float4 r0 = __builtin_bit_cast(float4, q.r[0]), r1 = __builtin_bit_cast(float4, q.r[1]);
     y[0] = make_float4(v[0] + r0.x, v[1] + r0.y, v[2] + r0.z, v[3] + r0.w);
     y[1] = make_float4(v[4] + r1.x, v[5] + r1.y, v[6] + r1.z, v[7] + r1.w);
     return 0.f;
@@ -482,7 +525,7 @@ VWA_DEVICE float finish_item(const GemmParams& p, int m, int c, const float (&a)
   }
   if constexpr (kResid<EPI>) {
     float r[8];
-    unpack8(*reinterpret_cast<const uint4*>(p.R + (size_t)m * p.ldr + c), r);
+    unpack8(q.r[0], r);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] += r[e];
   }
@@ -510,13 +553,14 @@ VWA_DEVICE void ss_add(unsigned long long* ss_out, int m, float sq) {
   }
 }
 
-template <int EPI, int AUX>
+template <int EPI, int AUX, int ZB>
 VWA_DEVICE float reduce_item(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, int m, int c) {
   const int cc[1] = {c};
   const bool ok[1] = {true};
   float a[1][8], b[1][8];
-  sum_items<EPI, AUX, 1, 4>(p, rws, m, cc, ok, a, b);
-  return finish_item<EPI>(p, m, c, a[0], b[0]);
+  const ItemPre<EPI> q = item_pre<EPI>(p, m, c);
+  sum_items<EPI, AUX, 1, ZB>(p, rws, m, cc, ok, a, b);
+  return finish_item<EPI>(p, q, m, c, a[0], b[0]);
 }
 
 // (round 4's 4-stage variant for one-row-block GEMMs measured slower in whole decode steps -- 128 KB
@@ -573,8 +617,10 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   // barriers with counted vmcnt (a __syncthreads would drain the in-flight DMA)
   constexpr int SPG = F8 || W8 ? 1 : 2;  // stages per k-group
   constexpr int STG = W8 ? C::W8STAGE : C::STAGE;
-  static_assert(W8 ? 2 * (C::BM / 8 / C::NW) + C::BN / 8 / C::NW == 8 : C::BM / 8 / C::NW + C::BN / 8 / C::NW == 8,
-                "8 LDS-DMA instructions per thread per stage (the counted vmcnt)");
+  constexpr int NST = W8 ? C::W8NST : 2;  // stage buffers
+  constexpr int PER = (W8 ? 2 : 1) * (C::BM / 8 / C::NW) + C::BN / 8 / C::NW;  // LDS-DMA instructions of a stage and wave
+  static_assert(PER == (NST == 3 ? 6 : 8),
+                "LDS-DMA instructions per thread per stage (the counted vmcnt)");
   const int h0 = SPG * kg0, nh = SPG * (kg1 - kg0);
   // X extent: the last row starts at (M-1)*ldx and is K long (rows may overlap: conv views)
   const size_t x_bytes = ((GRP ? x_rows - 1 : (size_t)(p.M - 1)) * p.ldx + p.K) * (F8 ? 1 : 2);
@@ -652,14 +698,18 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   } else {
   if (nh > 0) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0, lds, rows);
   if (nh > 1) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
+  if (NST == 3 && nh > 2) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 2, lds + 2 * STG, rows);
   for (int i = 0; i < nh; ++i) {
-    if (i + 1 < nh)
-      asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // this stage landed everywhere
+    char* at = lds + (NST == 2 ? i & 1 : i % NST) * STG;
+    if (NST == 3 && i + 2 < nh)
+      asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");  // this stage landed everywhere
+    else if (i + 1 < nh)
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PER) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    compute_stage<C, F8, W8, LINES>(lds + (i & 1) * STG, acc, wm, wn);
+    compute_stage<C, F8, W8, LINES>(at, acc, wm, wn);
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave done reading it
-    if (i + 2 < nh) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + i + 2, lds + (i & 1) * STG, rows);
+    if (i + NST < nh) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + i + NST, at, rows);
   }
   }
   const int l = lane_id();
@@ -776,7 +826,13 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       float o[8], q[8];
       unpack8(v, o);
       unpack8(*reinterpret_cast<const uint4*>(wl + row * RS + (ch ^ 1) * 16), q);
-      qkv_store(p, m, n, o, q);
+      float4 rope[4];
+      if (p.use_rope) {
+        const int pos = p.positions[m];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rope[e] = rope_at(p, pos, n)[e];
+      }
+      qkv_store(p, m, n, o, q, rope, p.slots[m]);
       continue;
     }
     if constexpr (kResid<EPI>) {
@@ -811,15 +867,15 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   }
 }
 
-// sum of the split-K slabs + epilogue (two-launch split-K): one thread per (row, 8 output columns)
-template <int EPI>
+// sum of the split-K slabs + epilogue (two-launch split-K): one thread per (row, 8 output columns), ZB slices in flight
+template <int EPI, int ZB>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p) {
   const int cpr = (EPI == EPI_SWIGLU ? p.N / 2 : p.N) / 8;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const bool ok = id < (int64_t)p.M * cpr;
   const __amdgpu_buffer_rsrc_t rws = rsrc(p.ws, (size_t)p.splits * p.M * p.N * 4);
   float sq = 0.f;
-  if (ok) sq = reduce_item<EPI, 0>(p, rws, (int)(id / cpr), (int)(id % cpr) * 8);
+  if (ok) sq = reduce_item<EPI, 0, ZB>(p, rws, (int)(id / cpr), (int)(id % cpr) * 8);
   if (kResid<EPI> && p.ss_out) ss_add(p.ss_out, ok ? (int)(id / cpr) : -1, sq);
 }
 
@@ -936,16 +992,21 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8) {
       hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, false, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
                          CfgP8::LDS, st, p);
   } else if (p.sw && !p.sx) {  // W8A16
-    using C = CfgW8;
-    const int tiles = ((p.M + C::BM - 1) / C::BM) * ((p.N + C::BN - 1) / C::BN);
-    hipLaunchKernelGGL((gemm_kernel<C, EPI, true, false, false, true>), dim3(tiles * p.splits), dim3(C::THREADS),
-                       C::W8LDS, st, p);
+    const dim3 grid((unsigned)(cdiv(p.M, CfgW8::BM) * cdiv(p.N, CfgW8::BN) * p.splits)), block(CfgW8::THREADS);
+    if (p.M <= CfgW8s::BM)
+      hipLaunchKernelGGL((gemm_kernel<CfgW8s, EPI, true, false, false, true>), grid, block, CfgW8s::W8LDS, st, p);
+    else
+      hipLaunchKernelGGL((gemm_kernel<CfgW8, EPI, true, false, false, true>), grid, block, CfgW8::W8LDS, st, p);
   } else {
     launch_cfg<CfgS, EPI>(p, st);
   }
   if (p.splits > 1) {
     const int64_t n = (int64_t)p.M * (EPI == EPI_SWIGLU ? p.N / 2 : p.N) / 8;
-    hipLaunchKernelGGL((gemm_reduce_kernel<EPI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
+    // one wave per workgroup up to four per CU: a CU alone draws ~25 GB/s of slabs
+    const int t = n <= (int64_t)p.cus * 256 ? 64 : 256;
+    const dim3 grid((unsigned)((n + t - 1) / t));
+    if (p.splits > 4 && t == 64) hipLaunchKernelGGL((gemm_reduce_kernel<EPI, 8>), grid, dim3(t), 0, st, p);
+    else hipLaunchKernelGGL((gemm_reduce_kernel<EPI, 4>), grid, dim3(t), 0, st, p);
   }
   return (int)hipGetLastError();
 }
@@ -969,9 +1030,17 @@ int launch_grouped(const GemmParams& p, hipStream_t st) {
 extern "C" int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, int f8) {
   const int tiles = ((M + CfgS::BM - 1) / CfgS::BM) * ((N + CfgS::BN - 1) / CfgS::BN);
   const int KG = K / BKG;
+  int s = 1;
+  if (f8 == 2 && g_split_fill_pct <= 0) {
+    // W8A16, two workgroups to a CU: slices while they fit and keep 4 k-groups each, 2 below half a chip.  Measured, 32 rows
+    // (us at 4 / 8 / 16 slices): 4096 x 4096 13.9 / 11.4 / 11.4 (64 rows 17.3 / 14.3 / 16.6), 4096 x 14336 34.7 / 24.7 / 21.4,
+    // 6144 x 4096 16.2 / 16.4 / 16.8, 14336 x 4096 22.0 / 25.5 / -
+    const int t = cdiv(M, CfgW8::BM) * cdiv(N, CfgW8::BN);
+    while (t * s * 2 <= 2 * cus && KG / (2 * s) >= (t * s < cus / 2 ? 2 : 4) && (int64_t)(s * 2) * M * N <= ws_floats) s *= 2;
+    return s;
+  }
   const int pct = g_split_fill_pct > 0 ? g_split_fill_pct : f8 ? 100 : 75;
   const int fill = (int)((int64_t)cus * pct / 100);
-  int s = 1;
   while (tiles * s < fill && s * 2 <= KG && (int64_t)(s * 2) * M * N <= ws_floats) s *= 2;
   return s;
 }

@@ -894,6 +894,24 @@ def test_llama70b_tp8_per_rank_decode_shapes(M):
         close(a, b, 3e-2)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(208, 128), (128, 256), (144, 384), (4096, 1152), (512, 5120)])
+def test_gemm_fp8_weights_few_rows(M, N, K):
+    """Stages of one to a few k-groups, column remainders, slices of a few k-groups; f32 sums of exact products
+    (K roundings of at most 2^-24 of the sum of magnitudes); the product and its sum with the residual each rounded
+    to bf16 (2^-8; a product of one slice passes through bf16 before the residual is added)."""
+    w = ops.FP8Weight.quantize(rnd(N, K, scale=K ** -0.5), tiled=True)
+    x, r = rnd(M, K), rnd(M, N)
+    y = torch.empty(M, N, dtype=BF, device=DEV)
+    for _ in range(2):
+        ops.gemm_fp8(x, w, y, epi="resid", residual=r)
+    wd = w.rows().double() * w.scale.double().view(-1, 1)
+    prod = x.double() @ wd.T
+    exp = prod + r.double()
+    tol = (exp.abs() + prod.abs()) * 2 ** -8 * (1 + 2 ** -8) + (x.double().abs() @ wd.abs().T + r.double().abs()) * (K + 2) * 2 ** -24
+    assert bool(((y.double() - exp).abs() <= tol).all())
+
+
 def test_quant_fp8_rows_with_rstd():
     """The fp8 row quantiser's optional RMSNorm output (one row pass for the W8A8 GEMM's two row
     statistics) equals row_rstd, and the codes / scales are unchanged by it."""
