@@ -294,10 +294,20 @@ VWA_DEVICE void p8_issue(__amdgpu_buffer_rsrc_t r, const unsigned (&voff)[8], un
   }
 }
 
-// one phase: 32 MFMAs, acc[i0 .. i0+3][0 .. 3] over both k-substeps of the stage
-template <int I0>
+// one phase: 32 MFMAs, acc[i0 .. i0+3][0 .. 3] over both k-substeps of the stage (fp8: 16 of twice the depth)
+template <int I0, bool F8>
 VWA_DEVICE void p8_mfma(f32x4 (&acc)[8][4], const bf16x8 (&a)[4][2], const bf16x8 (&b)[4][2]) {
   __builtin_amdgcn_s_setprio(1);
+  if constexpr (F8) {
+    auto both = [](const bf16x8 (&v)[2]) {
+      typedef int i32x4 __attribute__((ext_vector_type(4)));
+      return __builtin_shufflevector(__builtin_bit_cast(i32x4, v[0]), __builtin_bit_cast(i32x4, v[1]), 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[I0 + i][j] = mfma16x128_fp8(both(a[i]), both(b[j]), acc[I0 + i][j]);
+  } else
 #pragma unroll
   for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
@@ -627,25 +637,30 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   const size_t w_bytes = (size_t)p.N * p.K * (F8 || W8 ? 1 : 2);
   const __amdgpu_buffer_rsrc_t rx = rsrc(p.X, x_bytes), rw = rsrc(p.W, w_bytes);
   if constexpr (P8) {
-    static_assert(C::BM == 256 && C::BN == 256 && C::NW == 8 && !F8, "two-phase pipeline: CfgP8, bf16");
+    static_assert(C::BM == 256 && C::BN == 256 && C::NW == 8, "two-phase pipeline: CfgP8");
+    constexpr bool PAIRS = F8 || !LINES;  // a lane group's two chunks side by side (k 32 g ..), not by whole cache lines
     const int l = lane_id(), rl = l & 15, g = l >> 4;
     auto stage = [&](int s) { return lds + (s & 1) * C::STAGE; };
     unsigned voff[8];  // this lane's pieces of the half-tiles (k-group 0)
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-      const int q = it * 8 + w, r = 8 * q + (l >> 3), c = (l & 7) ^ (LINES ? swzk((r >> 1) & 7) : swz((r >> 1) & 7));  // A rows 8 q ..
+      const int q = it * 8 + w, r = 8 * q + (l >> 3), c = (l & 7) ^ (PAIRS ? swz((r >> 1) & 7) : swzk((r >> 1) & 7));  // A rows 8 q ..
       const int m = GRP ? rows[it] : bm + r;
-      voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)(((size_t)m * p.ldx + (LINES ? 8 * c : 32 * (c >> 1) + 8 * (c & 1))) * 2) : 0xFFFFFFF0u;
+      const size_t xa = F8 ? (size_t)m * p.ldx + 16 * c : ((size_t)m * p.ldx + (LINES ? 8 * c : 32 * (c >> 1) + 8 * (c & 1))) * 2;
+      voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)xa : 0xFFFFFFF0u;
       const int T = (bn >> 4) + (q >> 1);                                                // B n-tile q / 2, MFMA q & 1
       const size_t at = WT ? (size_t)T * KG * 2048 + (LINES ? (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8 : (q & 1) * 512 + l * 8)
                            : (size_t)(T * 16 + rl) * p.K + (LINES ? 8 * chunk_of(g, q & 1) : 32 * g + 8 * (q & 1));
-      voff[4 + it] = T * 16 < p.N ? (unsigned)(at * 2) : 0xFFFFFFF0u;
+      voff[4 + it] = T * 16 < p.N ? (unsigned)(F8 ? (size_t)T * KG * 2048 + (q & 1) * 1024 + l * 16 : at * 2) : 0xFFFFFFF0u;
     }
     // (stages past the last are issued too, on empty resources: the waits stay one constant)
     auto issue = [&](int s, int which) {
       const int hs = h0 + s, kg = hs >> 1, h = hs & 1;
       const bool in = s < nh;
-      if (which < 2)
+      if (F8)
+        p8_issue(which < 2 ? rsrc(p.X, in ? x_bytes : 0) : rsrc(p.W, in ? w_bytes : 0), voff, hs * (which < 2 ? BKG : 2048), which,
+                 stage(s));
+      else if (which < 2)
         p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, (kg * BKG + (LINES ? 64 : 16) * h) * 2, which, stage(s));
       else
         p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (WT ? kg * 2048 + (LINES ? 256 : 1024) * h : kg * BKG + (LINES ? 64 : 16) * h) * 2, which,
@@ -670,7 +685,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
         for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            a[i][sp] = *reinterpret_cast<const bf16x8*>(la + (i0 + i) * 16 * 128 + ((LINES ? chunk_of(g, sp) ^ swzk(rl >> 1) : (2 * g + sp) ^ swz(rl >> 1)) << 4));
+            a[i][sp] = *reinterpret_cast<const bf16x8*>(la + (i0 + i) * 16 * 128 + ((PAIRS ? (2 * g + sp) ^ swz(rl >> 1) : chunk_of(g, sp) ^ swzk(rl >> 1)) << 4));
       };
 #pragma unroll
       for (int sp = 0; sp < 2; ++sp)
@@ -680,7 +695,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       issue(s + 1, 1);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      p8_mfma<0>(acc, a, b);
+      p8_mfma<0, F8>(acc, a, b);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_barrier" ::: "memory");
       read_a(4);
@@ -689,7 +704,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       issue(s + 2, 3);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      p8_mfma<4>(acc, a, b);
+      p8_mfma<4, F8>(acc, a, b);
       __builtin_amdgcn_sched_barrier(0);
       asm volatile("s_barrier" ::: "memory");
     }
@@ -924,15 +939,23 @@ int cdiv(int a, int b) { return (a + b - 1) / b; }
 // 768 x 4096 x 14336 155 -> 86, 512 x 28672 x 4096 132 -> 93, 1863 x 6144 x 4096 115 -> 83.
 //   a round of the CUs costs so much per k-group and so much to start and store; a part of a last round 70 % and its share;
 //   128^2 tiles run two to a CU, one alone is faster; the slices' f32 partials are written and read.
+// W8A8 (k-groups of half the stages): fitted to 690 timings of 60 shapes (80 .. 6000 rows, 1024 .. 28672 columns, K 1280 ..
+// 14336), 11 % off; it picks the tile alone: slices in another order move a few bf16 activations by a bit, and every moved one
+// can flip its fp8 code further on, so they stay those of vwa_gemm_splits.  2720 x 4096 x 14336 224 -> 125 us, 2720 x 28672 x
+// 4096 407 -> 294, 1863 x 6144 x 4096 75 -> 48; small ones keep the 128^2 tile (2720 x 2560 x 1280: 18.4, 24.7 on the large one).
 float estimate(const GemmParams& p, bool p8, int s) {
   const int kg = cdiv(p.K / BKG, s), b = p8 ? 256 : 128;
   const int64_t t = (int64_t)cdiv(p.M, b) * cdiv(p.N, b) * s;
   const bool alone = !p8 && t <= p.cus;
   const float r = (float)t / (p8 || alone ? p.cus : 2 * p.cus), whole = floorf(r);
   const float rounds = r <= 1.f ? 1.f : r > whole ? whole + 0.7f + 0.3f * (r - whole) : whole;
+  const float slabs = (float)s * p.M * p.N * 4.f;
+  if (p.sx) {
+    const float per = p8 ? 1.21f : alone ? 0.97f : r >= 1.f ? 1.17f : 0.97f + 0.2f * (2.f * r - 1.f);
+    return rounds * (kg * per + (p8 ? 6.8f : 3.3f)) + (s > 1 ? 5.3f + slabs / 3.27e6f : 0.f);
+  }
   const float per = p8 ? 2.0f : alone ? 1.27f : r >= 1.f ? 1.84f : 1.27f + 0.57f * (2.f * r - 1.f);
-  const float sum = s > 1 ? 4.f + (float)s * p.M * p.N * 4.f / 3.55e6f : 0.f;
-  return rounds * (kg * per + (p8 ? 5.6f : 2.3f)) + sum;
+  return rounds * (kg * per + (p8 ? 5.6f : 2.3f)) + (s > 1 ? 4.f + slabs / 3.55e6f : 0.f);
 }
 
 struct Plan {
@@ -985,7 +1008,10 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8) {
     }
   } else if (p8) {
     const int tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
-    if (p.w_tiled)
+    if (p.sx)
+      hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, true, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
+                         CfgP8::LDS, st, p);
+    else if (p.w_tiled)
       hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
                          CfgP8::LDS, st, p);
     else
@@ -1070,6 +1096,8 @@ extern "C" int vwa_gemm(int epi, const GemmParams* pp, hipStream_t st) {
     const Plan pl = plan_kept(p);
     p8 = pl.p8;
     p.splits = pl.splits;
+  } else if (p.sx && p.nbatch <= 1 && p.cus > 0) {
+    p8 = g_p8_mode == 1 ? p.M >= 256 : g_p8_mode == 2 && estimate(p, true, p.splits) < estimate(p, false, p.splits);
   } else if (!p.sw && p.nbatch <= 1 && p.cus > 0) {
     if (g_p8_mode == 1 && p.w_tiled && p.N % 256 == 0 && p.M >= 256) {
       const int tiles8 = cdiv(p.M, 256) * (p.N / 256);

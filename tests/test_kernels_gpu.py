@@ -912,6 +912,39 @@ def test_gemm_fp8_weights_few_rows(M, N, K):
     assert bool(((y.double() - exp).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("mode,M,N,K", [
+    (1, 256, 256, 128), (1, 257, 256, 256), (1, 300, 512, 384), (1, 511, 256, 1152),  # 1, 2, 3 and 9 k-groups, sliced
+    (2, 1400, 6160, 512), (2, 700, 4112, 8192),                                        # a last column tile of 16 columns
+])
+def test_gemm_fp8_large_tile_against_f64(mode, M, N, K):
+    """f32 sums of exact products in the matrix unit (K roundings or truncations of at most 2^-23 of the sum of
+    magnitudes), scaled (two roundings); the product and its sum with the residual each rounded to bf16 (2^-8)."""
+    E = ops.ext()
+    w = ops.FP8Weight.quantize(rnd(N, K, scale=K ** -0.5), tiled=True)
+    x, r = rnd(M, K), rnd(M, N)
+    x8, sx, _ = ops._fp8_input(x, False, 1e-5)
+    y, z = (torch.empty(M, N, dtype=BF, device=DEV) for _ in range(2))
+    gu = torch.empty(M, N // 2, dtype=BF, device=DEV)
+    E.gemm_set_p8(mode)
+    try:
+        for out in (y, z):
+            ops.gemm_fp8(x, w, out, epi="resid", residual=r)
+        if N % 32 == 0:
+            ops.gemm_fp8(x, w, gu, epi="swiglu")
+    finally:
+        E.gemm_set_p8(2)
+    assert torch.equal(y, z)
+    xd, wd = x8.double() * sx.double().view(-1, 1), w.rows().double() * w.scale.double().view(-1, 1)
+    prod = xd @ wd.T
+    exp = prod + r.double()
+    acc = (xd.abs() @ wd.abs().T + r.double().abs()) * (K + 4) * 2 ** -23
+    assert bool(((y.double() - exp).abs() <= (exp.abs() + prod.abs()) * 2 ** -8 * (1 + 2 ** -8) + acc).all())
+    if N % 32 == 0:
+        q = prod.view(M, N // 32, 2, 16)
+        e = (torch.nn.functional.silu(q[:, :, 0]) * q[:, :, 1]).reshape(M, N // 2)
+        close(gu, e, 2e-2)
+
+
 def test_quant_fp8_rows_with_rstd():
     """The fp8 row quantiser's optional RMSNorm output (one row pass for the W8A8 GEMM's two row
     statistics) equals row_rstd, and the codes / scales are unchanged by it."""
