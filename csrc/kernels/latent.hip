@@ -323,9 +323,14 @@ __global__ __launch_bounds__(256, 2) void latent_attn_kernel(LatentAttnParams p)
   attn_finish<NT>(p, x, m, l, acc);
 }
 
-// 32-bit: keys straight from the cache
-template <int NT>
-__global__ __launch_bounds__(256) void latent_attn_f32_kernel(LatentAttnParams p) {
+// 32-bit: keys straight from the cache, twice (a tile of 64 keys x 576 columns is 147 KB, LDS holds no second one).  A decode
+// step is a workgroup or two per row with one tile each, so the tile's chain of round trips is the kernel: the block ids of all
+// its keys at once, the keys kKeyPre steps ahead of the products, the value columns of 16 keys ahead of theirs, the first ones
+// in flight over the softmax.  4 rows x 8 heads x 140 keys, rank 512: 25.3 -> 13.9 us (144 + 128
+// MFMAs of a wave: 3.6); 64 rows x 1000 keys 161 -> 55.
+constexpr int kKeyPre = 12;
+template <int NT, bool EXACT>  // EXACT: rank_p = 64 NT, the columns at constant offsets of a key's first
+__global__ __launch_bounds__(256, EXACT && NT <= 8 ? 2 : 1) void latent_attn_f32_kernel(LatentAttnParams p) {
   using M = MM<float>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float s_max[2][4][16];
@@ -335,39 +340,80 @@ __global__ __launch_bounds__(256) void latent_attn_f32_kernel(LatentAttnParams p
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6), rl = lane & 15, g = lane >> 4;
   char* pf = smem;                                   // [4][64][16 B]
   char* qf = smem + 4096;                            // [steps][64][16 B]
-  for (int i = tid; i < steps * 64; i += 256) {
-    const int s = i >> 6, ln = i & 63;
-    const float* q = reinterpret_cast<const float*>(p.q) + (size_t)x.row * p.ldq + (size_t)(x.h0 + min(ln & 15, x.Hb - 1)) * dk;
-    *reinterpret_cast<uint4*>(qf + i * 16) = *reinterpret_cast<const uint4*>(q + s * M::KS + (ln >> 4) * M::EPL);
-  }
   const int lb = __builtin_ctz(p.block_size);
   const float* cache = reinterpret_cast<const float*>(p.cache);
   auto key_row = [&](int key) {                      // (keys past pos, in the last tile, repeat it)
     key = min(key, x.pos);
     return cache + (int64_t)x.table[key >> lb] * p.c_sb + (int64_t)(key & (p.block_size - 1)) * dk;
   };
+  constexpr int ST = kKeys / M::KS;
+  const int own = (p.rank_p / 16 - w + 3) / 4 - 1;  // this wave's last value tile
+  const float* ka = nullptr;
+  const float* va[ST][4];
+  auto rows_of = [&](int key0) {
+    ka = key_row(key0 + 16 * w + rl) + g * M::EPL;
+#pragma unroll
+    for (int st = 0; st < ST; ++st)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) va[st][j] = key_row(key0 + 16 * st + 4 * g + j) + 16 * min(w, p.rank_p / 16 - 1) + rl;
+  };
+  rows_of(x.t_beg * kKeys);
+  for (int i = tid; i < steps * 64; i += 256) {
+    const int s = i >> 6, ln = i & 63;
+    const float* q = reinterpret_cast<const float*>(p.q) + (size_t)x.row * p.ldq + (size_t)(x.h0 + min(ln & 15, x.Hb - 1)) * dk;
+    *reinterpret_cast<uint4*>(qf + i * 16) = *reinterpret_cast<const uint4*>(q + s * M::KS + (ln >> 4) * M::EPL);
+  }
   const float sl2 = p.scale * kLog2e;
   float m = -1e30f, l = 0.f;
   f32x4 acc[NT] = {};
   for (int t = x.t_beg; t < x.t_end; ++t) {
     const int key0 = t * kKeys;
-    lds_sync();
-    f32x4 s0 = {};
-    const float* ka = key_row(key0 + 16 * w + rl) + g * M::EPL;
-    for (int s = 0; s < steps; ++s)
-      s0 = M::mma(*reinterpret_cast<const uint4*>(ka + s * M::KS), *reinterpret_cast<const uint4*>(qf + (s * 64 + lane) * 16), s0);
-    attn_weights<float, NT>(s0, sl2, key0, x.pos, s_max[t & 1], pf, m, l, acc);
+    if (t > x.t_beg) rows_of(key0);
+    u32x4 kf[2][kKeyPre];
+    float vf[2][NT][4];
+    auto load_k = [&](int q, int s0) {
 #pragma unroll
-    for (int st = 0; st < kKeys / M::KS; ++st) {
-      const uint4 pb = *reinterpret_cast<const uint4*>(pf + (st * 64 + lane) * 16);
-      const int k = key0 + 16 * st + 4 * g;
-      const float *k0 = key_row(k) + rl, *k1 = key_row(k + 1) + rl, *k2 = key_row(k + 2) + rl, *k3 = key_row(k + 3) + rl;
+      for (int i = 0; i < kKeyPre; ++i)
+        kf[q][i] = *reinterpret_cast<const u32x4*>(ka + min(s0 + i, steps - 1) * M::KS);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_v = [&](int q, int st) {
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
-        const int d = (w + 4 * n) * 16;
-        if (d >= p.rank_p) continue;
-        acc[n] = M::mma(make_uint4(__float_as_uint(k0[d]), __float_as_uint(k1[d]), __float_as_uint(k2[d]), __float_as_uint(k3[d])), pb, acc[n]);
+        const int d = 64 * (EXACT ? n : min(n, max(own, 0)));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) vf[q][n][j] = va[st][j][d];
       }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    load_k(0, 0);
+    lds_sync();
+    f32x4 s0 = {};
+    auto products = [&](int q, int s1) {
+#pragma unroll
+      for (int i = 0; i < kKeyPre; ++i)
+        if (s1 + i < steps) s0 = M::mma(__builtin_bit_cast(uint4, kf[q][i]), *reinterpret_cast<const uint4*>(qf + ((s1 + i) * 64 + lane) * 16), s0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int s = 0; s < steps; s += 2 * kKeyPre) {
+      if (s + kKeyPre < steps) load_k(1, s + kKeyPre);
+      products(0, s);
+      if (s + 2 * kKeyPre < steps) load_k(0, s + 2 * kKeyPre);
+      if (s + kKeyPre < steps) products(1, s + kKeyPre);
+    }
+    load_v(0, 0);
+    attn_weights<float, NT>(s0, sl2, key0, x.pos, s_max[t & 1], pf, m, l, acc);
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+      if (st + 1 < ST) load_v((st + 1) & 1, st + 1);
+      const uint4 pb = *reinterpret_cast<const uint4*>(pf + (st * 64 + lane) * 16);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        if (!EXACT && n > own) continue;
+        const float* v = vf[st & 1][n];
+        acc[n] = M::mma(make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])), pb, acc[n]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   attn_finish<NT>(p, x, m, l, acc);
@@ -541,7 +587,9 @@ template <int NT>
 int launch_attn_f32(const LatentAttnParams& p, hipStream_t st) {
   const size_t lds = 4096 + (size_t)(p.rank_p + p.rot_p) * 64;
   if (lds > kMaxLds) return -10;
-  hipLaunchKernelGGL((latent_attn_f32_kernel<NT>), dim3(p.rows * ((p.H + 15) / 16), p.nch), dim3(256), lds, st, p);
+  const dim3 grid(p.rows * ((p.H + 15) / 16), p.nch), block(256);
+  if (p.rank_p == 64 * NT) hipLaunchKernelGGL((latent_attn_f32_kernel<NT, true>), grid, block, lds, st, p);
+  else hipLaunchKernelGGL((latent_attn_f32_kernel<NT, false>), grid, block, lds, st, p);
   return (int)hipGetLastError();
 }
 

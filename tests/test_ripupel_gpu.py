@@ -318,6 +318,13 @@ def test_latent_attention(dtype, case):
     assert got[5].abs().sum() == 0 and rel(got[:5, :, :vd], want[:5]) < tol
 
 
+@pytest.mark.parametrize("case", [(2, 32, 32, 32, 1024, 16, 90), (5, 32, 64, 32, 512, 32, 1100), (3, 24, 16, 32, 480, 16, 1030)], ids=str)
+def test_latent_attention_32_bit_tiles(case):
+    """Ranks of whole and partly idle waves, several rounds of 64 keys to a chunk.  Sums of n weights and rank products in
+    32 bits: 2^-24 times about sqrt(n + rank) of the outputs' norm, 2e-6, five times of it for the exponent of large scores."""
+    test_latent_attention(F32, case)
+
+
 @pytest.mark.parametrize("case", LATENT, ids=str)
 @pytest.mark.parametrize("cuts", [[(0, 1000)], [(7, 2), (30, 60), (3, 1), (-1, 1), (16, 49)], [(0, 33), (64, 64), (33, 31)], [(1, 40)]], ids=str)
 def test_latent_prefill(case, cuts, monkeypatch):
