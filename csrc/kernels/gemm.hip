@@ -12,7 +12,7 @@
 //     i.e. exactly the MFMA B fragments: the block is copied to LDS verbatim;
 //   * row-major [N, K] (Whisper weights, tests): each 16-byte piece is scattered into the same
 //     fragment-ordered LDS image while staging.
-// Which k of a k-group a stage takes, and in which order, follows from the X rows' cache lines (swzk below).
+// Which k of a k-group a stage takes, and in which order, follows from the X rows' cache lines (swzk, gemm_stage.h).
 //
 // Tiling (gfx950, wave64), 128 x 128: workgroup = 4 waves (2 x 2), half a k-group (64 deep) per stage: A [128 rows][64
 // k] (16 KB, chunk-XOR swizzled: conflict-free ds_read_b128) and B [8 tiles][2 MFMAs][64 lanes][8] (16 KB, fragment
@@ -39,6 +39,7 @@
 // conv over a zero-padded channels-last buffer is X row t = padded rows t*stride .. t*stride+2
 // (ldx = stride*Cin, K = 3*Cin) -- the A tiles are staged through the same LDS-DMA pipeline.
 #include "common.h"
+#include "gemm_stage.h"
 #include "vwa_kernels.h"
 
 using namespace vwa;
@@ -81,27 +82,6 @@ using CfgW8 = Cfg<64, 128, 1, 4>;
 // 32-row step is weights arriving and little else: with the sum of the slices, 4096 x 4096 14.6 -> 11.4 us, 4096 x 14336
 // 27.9 -> 24.7, 28672 x 4096 35.6 -> 33.1)
 using CfgW8s = Cfg<32, 128, 1, 4>;
-
-// A-image slot swizzle: chunk c of row r sits at slot c ^ F((r >> 1) & 7).  F makes every
-// ds_read_b128 lane group ({0-3,12-15,20-27}, {4-11,16-19,28-31}, ... : two k-chunk columns g,
-// 16 rows) hit 16 distinct (row parity, slot) bank groups: F maps the half-row indices
-// {0,1,6,7} to the even slots and {2,3,4,5} to the odd ones, so XOR-ing the chunk index with 2
-// (the other column of the group) cannot collide.  (Plain c ^ h measured 33 % bank conflicts.)
-VWA_DEVICE int swz(int h) { return (0x64753120 >> (4 * h)) & 7; }
-
-// bf16 stages: half hs & 1 = h of a k-group is k 64 h .. 64 h + 64, a whole 128-byte line of every X row.  In the tiled
-// weight's order (lane group g of substep s: k 32 g + 8 s) that is the groups g = 2 h, 2 h + 1 of all four substeps: MFMA
-// sp of the half takes, in lane group g, substep 2 sp + (g >> 1) of group 2 h + (g & 1) -- k 64 h + 32 (g & 1) + 16 sp +
-// 8 (g >> 1), chunk 4 (g & 1) + 2 sp + (g >> 1) of the X row's line.  (Substeps 2 h, 2 h + 1 of all groups took 32 of every
-// 64 bytes of two lines per row, each line twice, 1.5 times the bytes through L1: 128^2 tile 12000 x 1280 x 1280 583 ->
-// 646 TFLOP/s, 1500 x 5120 x 1280 532 -> 594.)
-// A read's 16-lane groups now hold chunks c and c ^ 4 of complementary half rows {0,1,6,7}, {2,3,4,5}: swzk maps both
-// halves to 0..3.
-// LINES false keeps the substeps' own order, for weights whose products choose experts further on (GemmParams::keep_order):
-// the same sums in another order move a product by its last bits, and a token whose scores nearly tie to another expert --
-// 1 in 300 decoded rows of a 16-expert model when its prompt alone was computed in the other order.
-VWA_DEVICE int swzk(int h) { return (h & 1) | (h >> 2 << 1); }
-VWA_DEVICE int chunk_of(int g, int sp) { return 4 * (g & 1) + 2 * sp + (g >> 1); }
 
 // buffer resource over [base, base + bytes): loads past the end return zero (rows >= M, weight
 // tiles >= N), so the stage issue needs no bounds branches
@@ -149,7 +129,7 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
       off = (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 32 * (c >> 1) + 16 * ha + 8 * (c & 1)) * 2);
     else
       off = (unsigned)(((size_t)m * p.ldx + (size_t)kg * BKG + 64 * ha + 8 * c) * 2);
-    dma16(rx, buf + hh * C::A_BYTES + q * 1024, (GRP ? m >= 0 : m < p.M) ? off : 0xFFFFFFF0u);
+    dma16(rx, buf + hh * C::A_BYTES + q * 1024, (GRP ? m >= 0 : m < p.M) ? off : kPastEnd);
   }
   }
   const int kgn = p.K / BKG;
@@ -158,7 +138,7 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
 #pragma unroll
     for (int it = 0; it < C::BN / 8 / C::NW; ++it) {
       const int q = it * C::NW + w, T = (bn >> 4) + (q >> 1);
-      const unsigned off = T * 16 < p.N ? (unsigned)(((size_t)T * kgn + kg) * 2048 + (q & 1) * 1024 + lane * 16) : 0xFFFFFFF0u;
+      const unsigned off = T * 16 < p.N ? (unsigned)(((size_t)T * kgn + kg) * 2048 + (q & 1) * 1024 + lane * 16) : kPastEnd;
       dma16(rw, buf + 2 * C::A_BYTES + q * 1024, off);
     }
     return;
@@ -170,15 +150,15 @@ VWA_DEVICE void issue_stage(const GemmParams& p, __amdgpu_buffer_rsrc_t rx, __am
     unsigned off;
     if constexpr (F8) {
       const int T = (bn >> 4) + tile;
-      off = T * 16 < p.N ? (unsigned)(((size_t)T * kgn + kg) * 2048 + sp * 1024 + lane * 16) : 0xFFFFFFF0u;
+      off = T * 16 < p.N ? (unsigned)(((size_t)T * kgn + kg) * 2048 + sp * 1024 + lane * 16) : kPastEnd;
     } else if constexpr (WT) {
       const int T = (bn >> 4) + tile;
       const int at = LINES ? (2 * sp + (lane >> 5)) * 512 + h * 256 + (lane & 31) * 8 : (2 * h + sp) * 512 + lane * 8;
-      off = T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + at) * 2) : 0xFFFFFFF0u;
+      off = T * 16 < p.N ? (unsigned)((((size_t)T * kgn + kg) * 2048 + at) * 2) : kPastEnd;
     } else {
       const int n = bn + tile * 16 + (lane & 15), g = lane >> 4;
       const int at = LINES ? 64 * h + 8 * chunk_of(g, sp) : 32 * g + 16 * h + 8 * sp;
-      off = n < p.N ? (unsigned)(((size_t)n * p.K + (size_t)kg * BKG + at) * 2) : 0xFFFFFFF0u;
+      off = n < p.N ? (unsigned)(((size_t)n * p.K + (size_t)kg * BKG + at) * 2) : kPastEnd;
     }
     dma16(rw, buf + C::A_BYTES + q * 1024, off);
   }
@@ -644,27 +624,18 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     unsigned voff[8];  // this lane's pieces of the half-tiles (k-group 0)
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
-      const int q = it * 8 + w, r = 8 * q + (l >> 3), c = (l & 7) ^ (PAIRS ? swz((r >> 1) & 7) : swzk((r >> 1) & 7));  // A rows 8 q ..
-      const int m = GRP ? rows[it] : bm + r;
-      const size_t xa = F8 ? (size_t)m * p.ldx + 16 * c : ((size_t)m * p.ldx + (LINES ? 8 * c : 32 * (c >> 1) + 8 * (c & 1))) * 2;
-      voff[it] = (GRP ? m >= 0 : m < p.M) ? (unsigned)xa : 0xFFFFFFF0u;
-      const int T = (bn >> 4) + (q >> 1);                                                // B n-tile q / 2, MFMA q & 1
-      const size_t at = WT ? (size_t)T * KG * 2048 + (LINES ? (2 * (q & 1) + (l >> 5)) * 512 + (l & 31) * 8 : (q & 1) * 512 + l * 8)
-                           : (size_t)(T * 16 + rl) * p.K + (LINES ? 8 * chunk_of(g, q & 1) : 32 * g + 8 * (q & 1));
-      voff[4 + it] = T * 16 < p.N ? (unsigned)(F8 ? (size_t)T * KG * 2048 + (q & 1) * 1024 + l * 16 : at * 2) : 0xFFFFFFF0u;
+      const int q = it * 8 + w, r = 8 * q + (l >> 3), m = GRP ? rows[it] : bm + r;  // A rows 8 q ..
+      voff[it] = (GRP ? m >= 0 : m < p.M) ? p8_x_piece<F8, LINES>(m, p.ldx, r, l) : kPastEnd;
+      const int T = (bn >> 4) + (q >> 1);  // B n-tile q / 2, MFMA q & 1
+      voff[4 + it] = T * 16 < p.N ? p8_w_piece<F8, WT, LINES>(T, q & 1, p.K, l) : kPastEnd;
     }
     // (stages past the last are issued too, on empty resources: the waits stay one constant)
     auto issue = [&](int s, int which) {
-      const int hs = h0 + s, kg = hs >> 1, h = hs & 1;
       const bool in = s < nh;
-      if (F8)
-        p8_issue(which < 2 ? rsrc(p.X, in ? x_bytes : 0) : rsrc(p.W, in ? w_bytes : 0), voff, hs * (which < 2 ? BKG : 2048), which,
-                 stage(s));
-      else if (which < 2)
-        p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, (kg * BKG + (LINES ? 64 : 16) * h) * 2, which, stage(s));
+      if (which < 2)
+        p8_issue(rsrc(p.X, in ? x_bytes : 0), voff, p8_x_step<F8, LINES>(h0 + s, in), which, stage(s));
       else
-        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, (WT ? kg * 2048 + (LINES ? 256 : 1024) * h : kg * BKG + (LINES ? 64 : 16) * h) * 2, which,
-                stage(s));
+        p8_issue(rsrc(p.W, in ? w_bytes : 0), voff, p8_w_step<F8, WT, LINES>(h0 + s, in), which, stage(s));
     };
     issue(0, 0);
     issue(0, 2);
