@@ -769,6 +769,89 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
       }
     return;
   }
+  // bf16 results that something is done to behind the product -- the residual added, heads rotated: through LDS in 32 bits,
+  // PI fragment rows at a time, and rounded once, as the slices' sum does (rounded in front of it too, a residual of the
+  // product's size: 2.15e-3 from float64 instead of 1.66e-3).  A pass's residual chunks are requested in front of its LDS round
+  // trip: 1500 x 1280 x 1280 19.7 -> 17.6 us, 12000 x 1280 x 1280 41.2 -> 39.0.  W8A8 products keep both roundings: their
+  // results choose fp8 codes further on, and stay as they were.
+  if constexpr (!F8 && (kResid<EPI> || EPI == EPI_QKV)) {
+    constexpr int CPR = FN * 2, RSF = FN * 64 + 16;  // 8-column chunks of a row; LDS row stride (bytes: 4 rows apart, 16 banks)
+    constexpr int LDSB = (W8 ? C::W8LDS : C::LDS) / C::NW / (16 * RSF);
+    constexpr int PI = LDSB >= FM ? FM : LDSB >= FM / 2 ? FM / 2 : FM / 4, ITS = PI * 16 * CPR / 64;
+    static_assert(PI >= 1 && PI <= LDSB && FM % PI == 0, "a pass fits the wave's share of the LDS");
+    char* wl = lds + w * (PI * 16 * RSF);
+#pragma unroll
+    for (int i0 = 0; i0 < FM; i0 += PI) {
+      const int mw = bm + (wm * FM + i0) * 16 + l / CPR, n = bn + wn * FN * 16 + l % CPR * 8;  // chunk of iteration 0
+      uint4 rv[ITS];
+      if constexpr (kResid<EPI>) {
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+          const int m = mw + it * (64 / CPR);
+          if (m < p.M && n < p.N) rv[it] = *reinterpret_cast<const uint4*>(p.R + (size_t)m * p.ldr + n);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < PI; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) {
+            float v = acc[i0 + i][j][r] * rsv[i0 + i][r] * cz[j] + bz[j];
+            if constexpr (kGelu<EPI>) v = gelu_erf(v);
+            *reinterpret_cast<float*>(wl + (i * 16 + 4 * (l >> 4) + r) * RSF + (j * 16 + (l & 15)) * 4) = v;
+          }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      float sqv[ITS];  // (ss_out: squares of each stored chunk)
+#pragma unroll
+      for (int it = 0; it < ITS; ++it) {
+        sqv[it] = 0.f;
+        const int m = mw + it * (64 / CPR);
+        if (m >= p.M || n >= p.N) continue;
+        const char* row = wl + (it * (64 / CPR) + l / CPR) * RSF;
+        auto chunk = [&](int ch, float (&f)[8]) {
+          const float4 a = *reinterpret_cast<const float4*>(row + ch * 32), b = *reinterpret_cast<const float4*>(row + ch * 32 + 16);
+          f[0] = a.x, f[1] = a.y, f[2] = a.z, f[3] = a.w, f[4] = b.x, f[5] = b.y, f[6] = b.z, f[7] = b.w;
+        };
+        float v[8], u[8];
+        chunk(l % CPR, v);
+        if constexpr (EPI == EPI_QKV) {
+          chunk(l % CPR ^ 1, u);
+          float4 rope[4];
+          if (p.use_rope) {
+            const int pos = p.positions[m];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) rope[e] = rope_at(p, pos, n)[e];
+          }
+          qkv_store(p, m, n, v, u, rope, p.slots[m]);
+        } else {
+          unpack8(rv[it], u);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] += u[e];
+          const uint4 o = pack8(v);
+          if (p.ss_out) {
+            unpack8(o, u);  // (the stored bf16 values)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sqv[it] += u[e] * u[e];
+          }
+          *reinterpret_cast<uint4*>(reinterpret_cast<u16*>(p.Y) + (size_t)m * p.ldy + n) = o;
+        }
+      }
+      if (kResid<EPI> && p.ss_out) {  // one atomic per (row, wave): the CPR lanes of a row reduce first
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+          const int m = mw + it * (64 / CPR);
+          float sq = sqv[it];
+#pragma unroll
+          for (int o = 1; o < CPR; o <<= 1) sq += __shfl_xor(sq, o, 64);
+          if (l % CPR == 0 && m < p.M && bn + wn * FN * 16 < p.N)
+            __hip_atomic_fetch_add(gp(p.ss_out + m), ss_fix(sq), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    return;
+  }
   // bf16 out: the wave's tile goes through LDS (padded rows: the four row groups of a store hit
   // different banks) and leaves as 16-byte row chunks -- coalesced stores, 16-byte residual reads
   constexpr int NCOL = EPI == EPI_SWIGLU ? FN * 8 : FN * 16;  // output columns of this wave

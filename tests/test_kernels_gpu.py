@@ -730,6 +730,80 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
+@pytest.mark.parametrize("kind", ["tiled", "rowmajor", "fp8"])
+@pytest.mark.parametrize("mode,M,N,K", [(2, 17, 400, 128), (2, 64, 384, 128), (2, 200, 400, 128), (1, 300, 512, 128), (2, 1500, 384, 384)])
+def test_gemm_residual_is_added_before_rounding(mode, M, N, K, kind):
+    """A product of one slice and its residual are rounded once, together: with a residual that takes away all but the last bits
+    of the product, a rounding of the product (2^-9 of it) in front of the sum would be larger than what is left.
+    Tolerance: that one rounding (2^-8) and K + 2 roundings of at most 2^-24 of the sum of magnitudes."""
+    E = ops.ext()
+    if kind == "fp8" and M > ops.FP8_A16_ROWS:
+        pytest.skip("8-bit activations")
+    x, w = rnd(M, K), rnd(N, K, scale=K ** -0.5)
+    ww = {"tiled": lambda: ops.TiledWeight(w), "rowmajor": lambda: w, "fp8": lambda: ops.FP8Weight.quantize(w, tiled=True)}[kind]()
+    wd = ww.rows().double() * ww.scale.double().view(-1, 1) if kind == "fp8" else w.double()
+    prod = x.double() @ wd.T
+    r = (-prod).to(BF)
+    y = r.clone()
+    E.gemm_set_p8(mode)
+    try:
+        (ops.gemm_fp8 if kind == "fp8" else ops.gemm)(x, ww, y, epi="resid", residual=y)
+    finally:
+        E.gemm_set_p8(2)
+    exp = prod + r.double()
+    tol = exp.abs() * 2 ** -8 + (x.double().abs() @ wd.abs().T + r.double().abs()) * (K + 2) * 2 ** -24
+    assert bool(((y.double() - exp).abs() <= tol).all())
+    assert bool((exp.abs() > 4 * tol).any())  # (rounded in front, the sum is 0 or the last bit of the product: off by as much as exp)
+
+
+@pytest.mark.parametrize("kind", ["tiled", "rowmajor", "fp8"])
+@pytest.mark.parametrize("mode,M", [(2, 17), (2, 64), (2, 200), (1, 300)])
+def test_gemm_qkv_is_rotated_before_rounding(mode, M, kind):
+    """Heads of a product of one slice are rotated in 32 bits and rounded once: where the two terms of a rotation cancel, a
+    rounding of each in front of it would be larger than the tolerance of one rounding of their difference."""
+    E = ops.ext()
+    if kind == "fp8" and M > ops.FP8_A16_ROWS:
+        pytest.skip("8-bit activations")
+    K, nq, nkv, hd, bs = 128, 3, 1, 64, 16
+    n = nq + 2 * nkv
+    if mode == 1:
+        nq, n = 6, 8  # (whole 256-column tiles)
+    x, w = rnd(M, K), rnd(n * hd, K, scale=K ** -0.5)
+    wp = ops.permute_qkv_rows(w, n, hd)
+    ww = {"tiled": lambda: ops.TiledWeight(wp), "rowmajor": lambda: wp, "fp8": lambda: ops.FP8Weight.quantize(wp, tiled=True)}[kind]()
+    wd = (ww.rows().double() * ww.scale.double().view(-1, 1)) if kind == "fp8" else wp.double()
+    at = ops.permute_qkv_rows(torch.arange(n * hd, device=DEV).view(-1, 1), n, hd).view(-1)
+    rope = ops.rope_table(1024, hd, 1e4, device=DEV)
+    pos = torch.randint(0, 1024, (M,), device=DEV, dtype=torch.int32)
+    slots = torch.randperm(M, device=DEV)
+    kc = torch.zeros(-(-M // bs), nkv, bs, hd, dtype=BF, device=DEV)
+    vc, q = torch.zeros_like(kc), torch.zeros(M, nq * hd, dtype=BF, device=DEV)
+    E.gemm_set_p8(mode)
+    try:
+        ops.qkv_rope_write(x, ww, None, fuse_rms=False, eps=1e-5, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, rope=rope,
+                           positions=pos, slots=slots, q_out=q, k_cache=kc, v_cache=vc)
+    finally:
+        E.gemm_set_p8(2)
+    y, mag = torch.zeros(M, n * hd, dtype=torch.float64, device=DEV), torch.zeros(M, n * hd, dtype=torch.float64, device=DEV)
+    y[:, at], mag[:, at] = x.double() @ wd.T, x.double().abs() @ wd.abs().T
+    cs = rope[pos.long()].double()[:, None]  # [M, 1, hd / 2, 2]
+
+    def rotated(v, s):
+        v = v.view(M, n, hd)
+        lo, hi = v[..., : hd // 2], v[..., hd // 2 :]
+        c, d = cs[..., 0], cs[..., 1]
+        if s:
+            return torch.cat([lo * c.abs() + hi * d.abs(), hi * c.abs() + lo * d.abs()], -1)
+        return torch.cat([lo * c - hi * d, hi * c + lo * d], -1)
+
+    exp, m = rotated(y, False), rotated(mag, True)
+    exp[:, nq + nkv :], m[:, nq + nkv :] = y.view(M, n, hd)[:, nq + nkv :], mag.view(M, n, hd)[:, nq + nkv :]
+    rows = lambda c: c.permute(0, 2, 1, 3).reshape(-1, nkv, hd)[slots]  # noqa: E731
+    got = torch.cat([q.view(M, nq, hd), rows(kc), rows(vc)], 1).double()
+    tol = exp.abs() * 2 ** -8 + m * (K + 4) * 2 ** -24
+    assert bool(((got - exp).abs() <= tol).all())
+
+
 def test_gemm_keeps_the_order_of_its_sums():
     """A TiledWeight with keep_order: the same bits from either tile (4096 rows take the 256^2 one, 2048 the 128^2 one), with
     and without the SwiGLU epilogue; other epilogues and f32 results are served as ever."""
