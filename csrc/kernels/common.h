@@ -171,26 +171,7 @@ VWA_DEVICE uint32_t cvt_pk_fp8(float a, float b) {
 
 VWA_DEVICE float silu(float x) { return x / (1.f + __expf(-x)); }
 
-// x Phi(x) by Phi(-|x|) = erfc(z) / 2 = t P(t) e^(-z^2), z = |x| / sqrt 2, t = 1 / (1 + 0.38 z); P is a minimax fit (relative
-// error 2e-8 for z <= 9.5).  One exponential and no branch, in a GEMM's epilogue
-// that nothing hides (12000 x 5120 x 1280: 204 -> 199 us with erff's instructions gone, 158 without the activation).  Against
-// float64 over [-12, 12] the largest error is 3.8e-7 (0.5 x (1 + erff): 4.5e-7), and it stays relative (1.4e-5) where
-// 1 + erff cancels.
-VWA_DEVICE float gelu_erf(float x) {
-  const float z = fabsf(x) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(0.38f, z, 1.f));
-  float q = 0.02943703904747963f;
-  q = fmaf(q, t, -0.13090457022190094f);
-  q = fmaf(q, t, 0.181418314576149f);
-  q = fmaf(q, t, -0.08011052012443542f);
-  q = fmaf(q, t, 0.11455845832824707f);
-  q = fmaf(q, t, 0.06953151524066925f);
-  q = fmaf(q, t, 0.10189659893512726f);
-  q = fmaf(q, t, 0.1069682389497757f);
-  q = fmaf(q, t, 0.10720493644475937f);
-  q *= t * __expf(-z * z);
-  return x * (x > 0.f ? 1.f - q : q);
-}
+VWA_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
 // Bijective XCD-aware remap of a 1-D block index (8 XCDs, each with a private L2):
 // consecutive logical tiles land on the same XCD so neighbouring tiles share L2 lines.

@@ -804,6 +804,23 @@ def test_gemm_qkv_is_rotated_before_rounding(mode, M, kind):
     assert bool(((got - exp).abs() <= tol).all())
 
 
+def test_gelu_is_as_close_as_its_plain_form():
+    """GELU of a product in 32 bits (weights the identity: the values are known exactly) against float64: on every interval no
+    further off than x / 2 (1 + erf(x / sqrt 2)) in 32 bits by plain torch (a tenth for another rounding of the same steps)."""
+    K = 128
+    x, b = ((torch.rand(s, device=DEV) - 0.5) * f for s, f in (((4096, K), 12.0), ((K,), 0.2)))
+    x, b = x.to(BF), b.to(BF)
+    got = torch.empty(4096, K, device=DEV)
+    ops.gemm(x, ops.TiledWeight(torch.eye(K, device=DEV).to(BF)), got, epi="gelu", bias=b)
+    v = x.float() + b.float()
+    plain = 0.5 * v * (1 + torch.erf(v * 0.5 ** 0.5))
+    exp = 0.5 * v.double() * torch.erfc(-v.double() * 0.5 ** 0.5)
+    for lo, hi in ((-6, -3), (-3, -1), (-1, 0), (0, 1), (1, 3), (3, 6)):
+        at = (v > lo) & (v < hi)
+        err = lambda y: float((y.double() - exp)[at].abs().max())  # noqa: E731
+        assert err(got) <= 1.1 * err(plain), (lo, hi, err(got), err(plain))
+
+
 def test_gemm_keeps_the_order_of_its_sums():
     """A TiledWeight with keep_order: the same bits from either tile (4096 rows take the 256^2 one, 2048 the 128^2 one), with
     and without the SwiGLU epilogue; other epilogues and f32 results are served as ever."""
