@@ -91,6 +91,7 @@ VWA_DEVICE Unit unit_of(const TalkAttnParams& p, int ri) {
   u.seq = p.seq_ids[u.row];
   u.live = GRP || slot >= 0;
   u.v = vis_tiles(u.pos, u.pos + u.cnt - 1, p.window, p.keep);
+  u.v.n = min(u.v.n, p.nst * kTalkStat);  // (a position past the context that the scratch is sized for stays inside of it)
   return u;
 }
 

@@ -262,6 +262,44 @@ def test_talk_attention_inert_row_in_a_group():
     assert got[6].abs().sum() == 0 and torch.equal(got[:6], want[:6]) and torch.equal(got[7:], want[7:])
 
 
+def test_prompts_of_rising_length_leave_no_memory_behind():
+    """Rows-form prompts of a 32-bit model: what their lengths size goes back with the step, it follows the prompt and not the
+    engine's longest context, and two streams have sets of their own."""
+    H, G, dk, dv, ctx = 8, 4, 32, 16, 1 << 16
+    k, v = (torch.randn(ctx // 16, G, *s, device=DEV) for s in ((16, dk), (dv, 16)))
+    table = torch.arange(ctx // 16, dtype=torch.int32, device=DEV)[None].contiguous()
+    T = torch.eye(H, device=DEV)
+    sc = ops.TalkScratch([(H, G, dv, 0, 0)], ctx, DEV)
+
+    def step(n):
+        pos = torch.arange(n, dtype=torch.int32, device=DEV)
+        plan = ops.plan_runs([(0, n)], DEV, n - 1)
+        q, out = torch.randn(n, H * dk, device=DEV), torch.empty(n, H * dv, device=DEV)
+        for _ in range(2):
+            ops.talk_attention(q, k, v, table, pos, torch.zeros_like(pos), pos.long(), n_q_heads=H, scale=0.3, window=0, keep=0,
+                               talk=T, talk_frag=None, gate=None, out_scale=1.0, max_ctx=ctx, scratch=sc, out=out, plan=plan)
+        return plan, out
+
+    step(40)
+    torch.cuda.synchronize()
+    base, retired = torch.cuda.memory_allocated(), sum(t.numel() for t in ops._SCRATCH_RETIRED)
+    for n in (50, 300, 500, 700, 900):
+        torch.cuda.reset_peak_memory_stats()
+        step(n)
+        # scores, statistics and partial sums of n rows in whole groups of 8 and whole chunks of 128 keys, beside the rows' own
+        per_row = H * -(-n // 128) * (128 + 4 + dv) * 4
+        assert torch.cuda.max_memory_allocated() - base < (n + 8) * per_row + n * (H * (dk + dv) * 4 + 64) + (1 << 20)
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() == base
+    assert sum(t.numel() for t in ops._SCRATCH_RETIRED) == retired
+    plan, _ = step(60)
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        other = ops.stack.plan_scratch(plan, DEV, 16, 16, 16, 16)
+    torch.cuda.synchronize()
+    assert len(plan.work) == 2 and all(a.data_ptr() != b.data_ptr() for a, b in zip(other, plan.work[torch.cuda.current_stream().cuda_stream]))
+
+
 def test_prefill_form_takes_the_usual_sizes():
     part = ops.ext().talk_prefill_part
     for H, G, dk, dv in [(4, 2, 64, 128), (16, 4, 128, 128), (32, 8, 128, 128), (6, 2, 96, 192), (8, 1, 256, 64), (12, 12, 64, 64)]:

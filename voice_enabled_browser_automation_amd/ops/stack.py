@@ -55,7 +55,19 @@ def plan_runs(runs: Sequence[Tuple[int, int]], device, max_pos: int, scan_rows: 
 
     made: dict = {}
     return SimpleNamespace(max_pos=max_pos, tiles=dev(tiles, 2) if tiles else None, chunks=dev(chunks, 4),
-                           singles=dev(singles, 1).view(-1) if singles else None, groups=groups)
+                           singles=dev(singles, 1).view(-1) if singles else None, groups=groups, work={})
+
+
+def plan_scratch(plan: SimpleNamespace, device, s: int, stat: int, part: int, cnt: int) -> Tuple[torch.Tensor, ...]:
+    """The rows form's buffers of a prompt, on the stream of the call: the step's layers share one set, which goes back to the
+    caching allocator with the step's plan (a prompt's size decides theirs, so nothing of it may stay behind)."""
+    key, want = torch.cuda.current_stream(device).cuda_stream, (s, stat, part, cnt)
+    have = plan.work.get(key)
+    if have is None or any(t.numel() < n for t, n in zip(have, want)):
+        have = tuple(torch.empty(n, dtype=torch.float32, device=device) for n in want[:3])
+        have += (torch.zeros(cnt, dtype=torch.int32, device=device),)  # (tickets: a launch leaves them zero)
+        plan.work[key] = have
+    return have
 
 
 def visible_tiles(max_ctx: int, window: int, keep: int) -> int:
@@ -206,18 +218,17 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
                 rows_form(q, positions, seq_ids, slots, gate, out, lst, lst.shape[0])
         return out
     nq = min(16 // (n_q_heads // G), (140 << 10) // (520 * n_q_heads)) if n_q_heads // G <= 16 else 1
-    if plan is not None and nq > 1:  # a prompt: groups of consecutive rows, as many a launch as 64 MB of scores hold
-        from . import scratch as ws
-
-        groups = plan.groups(nq)
-        size = lambda n: rows_scratch(n, nq, n_q_heads, G, dv, max_ctx, window, keep, True)  # noqa: E731
-        step = max(1, min(groups.shape[0], (16 << 20) // size(1)[0]))
-        s, stat, part, cnt = size(step)
-        bufs = (ws(q.device, "talk_s", s), ws(q.device, "talk_stat", stat), ws(q.device, "talk_rows", part), _tickets(q.device, cnt))
+    # a prompt: groups of consecutive rows, as many a launch as 128 MB of scores and partial sums hold.  (Not while capturing:
+    # the groups' table is an upload of its own.)
+    if plan is not None and nq > 1 and not torch.cuda.is_current_stream_capturing():
+        groups, ctx = plan.groups(nq), min(max_ctx, plan.max_pos + 1)
+        size = lambda n: rows_scratch(n, nq, n_q_heads, G, dv, ctx, window, keep, True)  # noqa: E731
+        step = max(1, min(groups.shape[0], (32 << 20) // sum(size(1)[:3])))
+        bufs = plan_scratch(plan, q.device, *size(step))
         for i in range(0, groups.shape[0], step):
             lst = groups[i : i + step]
             E.talk_attention(q, k_cache, v_cache, block_table, positions, seq_ids, slots, None, lst.shape[0], n_q_heads, scale,
-                             window, keep, talk, gate, out_scale, max_ctx, *bufs, out, groups=lst, nq=nq)
+                             window, keep, talk, gate, out_scale, ctx, *bufs, out, groups=lst, nq=nq)
         return out
     for i in range(0, rows, ROW_SLICE):
         j = min(rows, i + ROW_SLICE)
