@@ -240,8 +240,10 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
   }
   const int qi = GRP ? rl / R : 0, r = GRP ? rl % R : rl;               // this column's row and query head
   const bool col = qi < un.cnt && r < Rb;
+  // (an inert row of a group is zero whatever its query and its key hold)
+  const bool on = !GRP || (col && p.slots[un.row + qi] >= 0);
   float gate = 0.f;
-  if (nact == 1 && col) gate = !GRP || p.slots[un.row + qi] >= 0 ? head_gate<T>(p, un.row + qi, h0 + r) : 0.f;
+  if (nact == 1 && col && on) gate = head_gate<T>(p, un.row + qi, h0 + r);
   constexpr int TPS = M::KS / kTile;                 // tiles per step (bf16 2, f32 1)
   constexpr int NST = CT / TPS;
   const int lb = __builtin_ctz(p.block_size);
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
     const int h = h0 + r;
     if (nact == 1) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) stv(out + (size_t)qi * p.ldo + (size_t)h * p.dv + d + 4 * b + i, acc[i] * gate);
+      for (int i = 0; i < 4; ++i) stv(out + (size_t)qi * p.ldo + (size_t)h * p.dv + d + 4 * b + i, on ? acc[i] * gate : 0.f);
     } else {
       st_sc1_x4(rp, (int)(((((int64_t)qi * p.nch + chunk) * p.H + h) * p.dv + d + 4 * b) * 4), acc);
     }
@@ -361,7 +363,12 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
       a0 += x.x;
       a1 += x.y;
     }
-    const float g = !GRP || p.slots[row] >= 0 ? head_gate<T>(p, row, h0 + e / p.dv) : 0.f;
+    if (GRP && p.slots[row] < 0) {
+      stv(out + (size_t)k0 * p.ldo + o, 0.f);
+      stv(out + (size_t)k0 * p.ldo + o + 1, 0.f);
+      continue;
+    }
+    const float g = head_gate<T>(p, row, h0 + e / p.dv);
     stv(out + (size_t)k0 * p.ldo + o, a0 * g);
     stv(out + (size_t)k0 * p.ldo + o + 1, a1 * g);
   }

@@ -262,6 +262,31 @@ def test_talk_attention_inert_row_in_a_group():
     assert got[6].abs().sum() == 0 and torch.equal(got[:6], want[:6]) and torch.equal(got[7:], want[7:])
 
 
+@pytest.mark.parametrize("n", [21, 400])
+def test_inert_row_of_a_group_is_zero_whatever_it_holds(n):
+    """A row without a cache slot was never computed: its query may hold anything.  One chunk, and several."""
+    H, G, dk, dv = 4, 2, 32, 16
+    q, k, v = (rnd(n, x, d, seed=i, dtype=F32) for i, (x, d) in enumerate(((H, dk), (G, dk), (G, dv))))
+    blocks = -(-n // 16)
+    kc, vc = paged(k, v, list(range(blocks)), 16, F32)
+    table, pos = torch.arange(blocks, dtype=torch.int32, device=DEV)[None].contiguous(), torch.arange(n, dtype=torch.int32, device=DEV)
+    slots = pos.long()
+    inert = [6, n - 2]
+    slots[inert] = -1
+
+    def run(q):
+        out = torch.full((n, H * dv), float("nan"), device=DEV)
+        ops.talk_attention(q.reshape(n, -1).to(DEV), kc, vc, table, pos, torch.zeros_like(pos), slots, n_q_heads=H, scale=0.3,
+                           window=0, keep=0, talk=torch.eye(H, device=DEV), talk_frag=None, gate=None, out_scale=1.0, max_ctx=16 * blocks,
+                           scratch=ops.TalkScratch([(H, G, dv, 0, 0)], 16 * blocks, DEV), out=out, plan=ops.plan_runs([(0, n)], DEV, n - 1))
+        return out
+
+    want = run(q)
+    q[inert] = float("nan")
+    got = run(q)
+    assert got[inert].abs().sum() == 0 and torch.equal(got, want)
+
+
 def test_prompts_of_rising_length_leave_no_memory_behind():
     """Rows-form prompts of a 32-bit model: what their lengths size goes back with the step, it follows the prompt and not the
     engine's longest context, and two streams have sets of their own."""
