@@ -981,8 +981,8 @@ int launch_cfg(const GemmParams& p, hipStream_t st) {
   return 0;
 }
 
-int g_p8_mode = 2;       // 0: the 128^2 kernel only, 1: the 256^2 one for every shape it was made for, 2: plan()
-int g_split_fill_pct = 0;  // > 0: vwa_gemm_splits' fill, and no plan() for the 128^2 kernel's splits
+int g_p8_mode = 2;         // 0: the 128^2 kernel only, 1: the 256^2 one from 256 rows (bf16: of pre-tiled whole column tiles), 2: choose()
+int g_split_fill_pct = 0;  // > 0: vwa_gemm_splits' fill, and the rules by shape alone instead of plan()
 
 int cdiv(int a, int b) { return (a + b - 1) / b; }
 
@@ -1033,17 +1033,34 @@ Plan plan(const GemmParams& p) {
   return best;
 }
 
-// keep_order: the slices of few large tiles are part of the order (in powers of two until they cover the CUs, of >= 2048 k
-// each; p.splits holds those of the small tile); the tile is not
-Plan plan_kept(const GemmParams& p) {
-  Plan r{false, p.splits};
-  if (p.M >= 256 && p.N % 256 == 0) {
-    const int tiles8 = cdiv(p.M, 256) * (p.N / 256);
-    int s = 1;
-    while (p.ws && tiles8 * s < p.cus && s * 2 <= p.K / BKG && (int64_t)(s * 2) * p.M * p.N <= p.ws_cap) s *= 2;
-    if (tiles8 >= 256 || (tiles8 * s >= p.cus && p.K / s >= 2048)) r.splits = s;
+// Slices of whole large tiles by shape alone, in powers of two until they cover the CUs; *fill: the tiles alone, or slices of
+// >= 2048 k each, do
+int slices_256(const GemmParams& p, bool* fill) {
+  const int tiles = cdiv(p.M, 256) * (p.N / 256);
+  int s = 1;
+  while (p.ws && tiles * s < p.cus && s * 2 <= p.K / BKG && (int64_t)(s * 2) * p.M * p.N <= p.ws_cap) s *= 2;
+  *fill = tiles >= 256 || (tiles * s >= p.cus && p.K / s >= 2048);
+  return s;
+}
+
+bool keeps_order(int epi, const GemmParams& p) {
+  return p.keep_order && p.w_tiled && !p.sw && p.nbatch <= 1 && p.cus > 0 && (epi == EPI_STORE || epi == EPI_SWIGLU);
+}
+
+// Tile and slices of a launch (p.splits: those of vwa_gemm_splits)
+Plan choose(const GemmParams& p) {
+  Plan r{false, p.splits < 1 ? 1 : p.splits};
+  if (p.nbatch > 1 || p.cus <= 0 || (p.sw && !p.sx)) return r;
+  bool fill = false;
+  const int s = p.M >= 256 && p.N % 256 == 0 ? slices_256(p, &fill) : 0;
+  // (g_p8_mode picks the tile; the slices of W8A8 and kept-order products are part of the order of their sums)
+  if (p.keep_order || p.sx) {
+    if (p.keep_order && fill) r.splits = s;
+    r.p8 = g_p8_mode == 1 ? p.M >= 256 : g_p8_mode == 2 && (p.sx || p.M >= 128) && estimate(p, true, r.splits) < estimate(p, false, r.splits);
+    return r;
   }
-  r.p8 = p.M >= 128 && estimate(p, true, r.splits) < estimate(p, false, r.splits);
+  if (g_p8_mode == 2 && g_split_fill_pct == 0) return p.M >= 128 ? plan(p) : r;
+  if (p.w_tiled && s && (g_p8_mode == 1 || (g_p8_mode == 2 && fill))) r = Plan{true, s};
   return r;
 }
 
@@ -1129,6 +1146,15 @@ extern "C" void vwa_gemm_set_split_fill(int pct) { g_split_fill_pct = pct < 0 ? 
 
 extern "C" void vwa_gemm_set_p8(int mode) { g_p8_mode = mode; }
 
+extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int* large, int* splits) {
+  GemmParams p = *pp;
+  p.keep_order = keeps_order(epi, p);
+  const Plan pl = choose(p);
+  const int per = cdiv(p.K / BKG, pl.splits);
+  *large = pl.p8;
+  *splits = cdiv(p.K / BKG, per);
+}
+
 extern "C" int vwa_gemm(int epi, const GemmParams* pp, hipStream_t st) {
   GemmParams p = *pp;
   if (p.M < 1 || p.N < 16 || p.N % 16 || p.K < BKG || p.K % BKG) return -10;
@@ -1143,28 +1169,10 @@ extern "C" int vwa_gemm(int epi, const GemmParams* pp, hipStream_t st) {
   if (epi == EPI_SPLIT && (p.y_f32 || !p.Y2 || p.n_split % 16 || p.n_split < 0 || p.n_split > p.N || p.ldy2 % 8 ||
                            (reinterpret_cast<uintptr_t>(p.Y2) & 15)))
     return -19;
-  if (p.splits < 1) p.splits = 1;
-  bool p8 = false;
-  p.keep_order = p.keep_order && p.w_tiled && !p.sw && p.nbatch <= 1 && p.cus > 0 && (epi == EPI_STORE || epi == EPI_SWIGLU);
-  if (p.keep_order) {
-    const Plan pl = plan_kept(p);
-    p8 = pl.p8;
-    p.splits = pl.splits;
-  } else if (p.sx && p.nbatch <= 1 && p.cus > 0) {
-    p8 = g_p8_mode == 1 ? p.M >= 256 : g_p8_mode == 2 && estimate(p, true, p.splits) < estimate(p, false, p.splits);
-  } else if (!p.sw && p.nbatch <= 1 && p.cus > 0) {
-    if (g_p8_mode == 1 && p.w_tiled && p.N % 256 == 0 && p.M >= 256) {
-      const int tiles8 = cdiv(p.M, 256) * (p.N / 256);
-      p8 = true;
-      p.splits = 1;
-      while (p.ws && tiles8 * p.splits < p.cus && p.splits * 2 <= p.K / BKG && (int64_t)p.splits * 2 * p.M * p.N <= p.ws_cap)
-        p.splits *= 2;
-    } else if (g_p8_mode == 2 && g_split_fill_pct == 0 && p.M >= 128) {
-      const Plan pl = plan(p);
-      p8 = pl.p8;
-      p.splits = pl.splits;
-    }
-  }
+  p.keep_order = keeps_order(epi, p);
+  const Plan pl = choose(p);
+  const bool p8 = pl.p8;
+  p.splits = pl.splits;
   const int KG = p.K / BKG;
   p.kg_per_split = (KG + p.splits - 1) / p.splits;
   p.splits = (KG + p.kg_per_split - 1) / p.kg_per_split;  // no empty slice

@@ -1,0 +1,54 @@
+"""Which tile and how many K slices the GEMM takes (gemm.hip): a rule on sizes, types and the diagnostic switches, no launch."""
+import os
+
+import pytest
+
+from voice_enabled_browser_automation_amd.ops import build
+
+pytestmark = pytest.mark.skipif(not os.path.exists(build.KERNEL_SO), reason="the kernel library is not built")
+
+
+@pytest.fixture
+def E():
+    import torch  # noqa: F401  (the HIP runtime comes with it)
+
+    from voice_enabled_browser_automation_amd.ops import _vwa_kernels as E
+
+    yield E
+    E.gemm_set_p8(2)
+    E.gemm_set_split_fill(0)
+
+
+SIZES = [(1011, 6144, 4096), (4096, 4096, 2048), (2048, 4096, 2048), (1011, 4096, 14336), (3000, 28672, 4096), (300, 512, 512)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+def test_the_switch_for_the_large_tile_reaches_kept_order_products(E, M, N, K):
+    """0: never, 1: from 256 rows; the slices, and with them the order of the sums, are those of the estimate's choice."""
+    for kw in (dict(keep_order=True), dict(f8=1)):
+        splits = E.gemm_plan(0, M, N, K, **kw)[1]
+        E.gemm_set_p8(0)
+        assert E.gemm_plan(0, M, N, K, **kw) == (False, splits)
+        E.gemm_set_p8(1)
+        assert E.gemm_plan(0, M, N, K, **kw) == (True, splits)
+        E.gemm_set_p8(2)
+
+
+def test_the_estimate_takes_either_tile_for_kept_order(E):
+    """(what the tests of the kept order's bits rely on: the same slices, another tile)"""
+    assert E.gemm_plan(0, 4096, 4096, 2048, keep_order=True) == (True, 1)
+    assert E.gemm_plan(0, 2048, 4096, 2048, keep_order=True) == (False, 1)
+
+
+def test_a_split_fill_keeps_the_large_tile(E):
+    """The split-K fill target replaces the estimate by the rules on shape alone: large tiles that cover the CUs, or do so in
+    slices of 2048 and more, stay large."""
+    E.gemm_set_split_fill(75)
+    assert E.gemm_plan(0, 1011, 28672, 4096) == (True, 1)      # 448 large tiles
+    assert E.gemm_plan(1, 1011, 4096, 14336) == (True, 4)      # 64, in slices of 3584
+    assert E.gemm_plan(1, 1011, 4096, 4096)[0] is False        # slices of 1024
+    assert E.gemm_plan(0, 1011, 28672, 4096, w_tiled=False)[0] is False
+    E.gemm_set_p8(0)
+    assert E.gemm_plan(0, 1011, 28672, 4096)[0] is False
+    E.gemm_set_p8(1)
+    assert E.gemm_plan(0, 300, 512, 512)[0] is True and E.gemm_plan(0, 300, 528, 512)[0] is False

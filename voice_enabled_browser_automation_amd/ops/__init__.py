@@ -71,7 +71,7 @@ def ext():
         impl = knob("VWA_ATTN_IMPL")
         if impl:
             m.set_attention_impl(ATTENTION_IMPLS[impl])
-        p8 = knob("VWA_GEMM_P8")  # 0: 128x128 GEMM only, 1: 256x256 from 256 rows of whole column tiles
+        p8 = knob("VWA_GEMM_P8")  # 0: 128x128 GEMM only, 1: 256x256 from 256 rows (bf16: of pre-tiled whole column tiles)
         if p8 not in (None, ""):
             m.gemm_set_p8(int(p8))
         xsk = knob("VWA_SKINNY_X_SKEW")  # LDS-staged X rows: 64-B skew every 4 rows (1) / none (0)

@@ -142,7 +142,7 @@ class Settings(BaseModel):
     VWA_CHAIN_BAR_MODE: int = Field(2, description="chained launches' grid barrier: 2 two-level tickets + scalar polls (default), 4 no-return arrivals + polled sum of the 8 group counters")
     VWA_CHAIN_SCHED: Optional[str] = Field(None, description="DIAGNOSTIC: chained schedule override name=value,...")
     VWA_GEMM_QKV: bool = Field(True, description="> 16-row QKV: rotary + KV write in the tiled GEMM epilogue")
-    VWA_GEMM_P8: Optional[str] = Field(None, description="DIAGNOSTIC: 256x256 GEMM eligibility override (0: never, 1: wherever it fits, unset: by an estimate)")
+    VWA_GEMM_P8: Optional[str] = Field(None, description="DIAGNOSTIC: 256x256 GEMM tile (0: never, 1: from 256 rows, bf16 only for pre-tiled whole column tiles, unset: by an estimate)")
     VWA_GEMM_SPLIT_FILL: Optional[str] = Field(None, description="DIAGNOSTIC: split-K fill target (% of CUs)")
     VWA_SKINNY_X_SKEW: Optional[str] = Field(None, description="DIAGNOSTIC: LDS X-row skew of the streaming GEMM")
     VWA_ATTN_IMPL: Optional[str] = Field(None, description="DIAGNOSTIC: decode attention implementation")
