@@ -158,10 +158,10 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
 
 // ------------------------------------------------------------------------------------------ small tiles (16 NP pairs)
 // A workgroup per (tile, NU x 16 features | columns); its 4 waves split K, the sums meet in LDS.  Bound by the experts' weights
-// arriving: a wave has two to four k-groups, and the next is requested before this one's products (4 rows over 16 experts of
-// 1024 x 1024 in 32 bits: gate / up 25.2 -> 23.4 us, down 17.3 -> 13.2); two workgroups a CU bound the registers.
-template <class T, bool DOWN, int NP, int NU>
-__global__ __launch_bounds__(256, 2) void moe_small_kernel(MoeGemmParams p) {
+// arriving: SUB substeps of a wave's k-groups (of 4 each) are requested before the products of the SUB before; SUB 0: a k-group
+// is requested when the one before is done, which leaves registers for twice the workgroups (launch_small chooses).
+template <class T, bool DOWN, int NP, int NU, int SUB>
+__global__ __launch_bounds__(256, SUB ? 2 : 1) void moe_small_kernel(MoeGemmParams p) {
   using M = MM<T>;
   constexpr int NA = DOWN ? 1 : 2;                   // 16-row tiles of the matrix per unit
   __shared__ float red[4][NP][NU][NA][64][4];
@@ -181,38 +181,70 @@ __global__ __launch_bounds__(256, 2) void moe_small_kernel(MoeGemmParams p) {
   for (int u = 0; u < NU; ++u)
     wp[u] = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(p.w) + e * p.w_expert) + (size_t)min(unit0 + u, units - 1) * NA * KG * 256;
   f32x4 acc[NP][NU][NA] = {};
-  u32x4 f[2][NU][NA][4], a[2][NP][4];                // a wave's next k-group arrives under this one's products
-  auto load = [&](int b, int kg) {
+  if constexpr (SUB == 0) {
+    for (int kg = w; kg < KG; kg += 4) {
+      uint4 f[NU][NA][4], a[NP][4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+      for (int s = 0; s < 4; ++s) {
 #pragma unroll
-      for (int u = 0; u < NU; ++u)
+        for (int u = 0; u < NU; ++u)
 #pragma unroll
-        for (int j = 0; j < NA; ++j)
-          f[b][u][j][s] = *reinterpret_cast<const u32x4*>(wp[u] + ((size_t)j * KG + kg) * 256 + s * 64 + (unsigned)lane);
+          for (int j = 0; j < NA; ++j) f[u][j][s] = (wp[u] + ((size_t)j * KG + kg) * 256 + s * 64)[(unsigned)lane];
 #pragma unroll
-      for (int t = 0; t < NP; ++t) a[b][t][s] = *reinterpret_cast<const u32x4*>(x[t] + kg * 16 * M::EPL + s * M::EPL);
+        for (int t = 0; t < NP; ++t) a[t][s] = *reinterpret_cast<const uint4*>(x[t] + kg * 16 * M::EPL + s * M::EPL);
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int t = 0; t < NP; ++t)
+#pragma unroll
+          for (int u = 0; u < NU; ++u)
+#pragma unroll
+            for (int j = 0; j < NA; ++j) acc[t][u][j] = M::mma(a[t][s], f[u][j][s], acc[t][u][j]);
     }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto products = [&](int b) {
+  } else {
+    u32x4 f[2][NU][NA][SUB], a[2][NP][SUB];
+    auto load = [&](int b, int kg, int s0) {         // substeps s0 .. of a k-group
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int t = 0; t < NP; ++t)
+      for (int s = 0; s < SUB; ++s) {
 #pragma unroll
         for (int u = 0; u < NU; ++u)
 #pragma unroll
           for (int j = 0; j < NA; ++j)
-            acc[t][u][j] = M::mma(__builtin_bit_cast(uint4, a[b][t][s]), __builtin_bit_cast(uint4, f[b][u][j][s]), acc[t][u][j]);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  if (w < KG) load(0, w);
-  for (int kg = w; kg < KG; kg += 8) {
-    if (kg + 4 < KG) load(1, kg + 4);
-    products(0);
-    if (kg + 8 < KG) load(0, kg + 8);
-    if (kg + 4 < KG) products(1);
+            f[b][u][j][s] = *reinterpret_cast<const u32x4*>(wp[u] + ((size_t)j * KG + kg) * 256 + (s0 + s) * 64 + (unsigned)lane);
+#pragma unroll
+        for (int t = 0; t < NP; ++t) a[b][t][s] = *reinterpret_cast<const u32x4*>(x[t] + kg * 16 * M::EPL + (s0 + s) * M::EPL);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto products = [&](int b) {
+#pragma unroll
+      for (int s = 0; s < SUB; ++s)
+#pragma unroll
+        for (int t = 0; t < NP; ++t)
+#pragma unroll
+          for (int u = 0; u < NU; ++u)
+#pragma unroll
+            for (int j = 0; j < NA; ++j)
+              acc[t][u][j] = M::mma(__builtin_bit_cast(uint4, a[b][t][s]), __builtin_bit_cast(uint4, f[b][u][j][s]), acc[t][u][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (w < KG) load(0, w, 0);
+    if constexpr (SUB == 2) {
+      for (int kg = w; kg < KG; kg += 4) {
+        load(1, kg, 2);
+        products(0);
+        if (kg + 4 < KG) load(0, kg + 4, 0);
+        products(1);
+      }
+    } else {
+      for (int kg = w; kg < KG; kg += 8) {
+        if (kg + 4 < KG) load(1, kg + 4, 0);
+        products(0);
+        if (kg + 8 < KG) load(0, kg + 8, 0);
+        if (kg + 4 < KG) products(1);
+      }
+    }
   }
 #pragma unroll
   for (int t = 0; t < NP; ++t)
@@ -244,13 +276,26 @@ __global__ __launch_bounds__(256, 2) void moe_small_kernel(MoeGemmParams p) {
 }
 
 // (units: as many matrix tiles per row of x read, gate / up or down)
+// Two sets of whole k-groups, or, for 32-bit gate / up, of halves (120 registers or 72).  Against one set at a time, mean over 22
+// to 45 shapes (widths 512 .. 4096, 1 .. 64 rows): 16-pair tiles 0.86 gate / up and 0.87 down, in 32 bits 0.89 (halves; whole: 0.905, and
+// up to 1.08) and 0.86; 32-pair tiles 0.96 and 0.93, single shapes up to 1.03 (down, 3072 x 1024: 20.8 -> 21.4 us).  32-pair gate / up
+// of up to four k-groups to a wave keeps one set where two would run in a second round of the CUs (240 registers: two
+// workgroups a CU) and one does not (five): 48 rows of 2048 x 2048, 16 experts, 47.3 us (50.5 with two), 1024 x 2048 26.2 (27.5); but
+// 13.8 (12.4) of 1024 x 1024, one round, 49.1 (49.9) of 1024 x 4096, rounds either way, and 97.9 (91.6) of 4096 x 2048.
+constexpr int kCus = 256;
 template <class T, int NP>
 void launch_small(const MoeGemmParams& p, hipStream_t st) {
   constexpr int NG = NP, ND = NP == 1 ? 1 : 2 * NP;
   const int units = p.N / (p.down ? 16 : 32), nu = p.down ? ND : NG;
   const dim3 grid((units + nu - 1) / nu, p.max_tiles), block(256);
-  if (p.down) hipLaunchKernelGGL((moe_small_kernel<T, true, NP, ND>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((moe_small_kernel<T, false, NP, NG>), grid, block, 0, st, p);
+  const int64_t live = (int64_t)grid.x * (p.max_tiles - (int64_t)p.x_rows * p.top / p.tile);  // workgroups if no expert has a second tile
+  if (p.down) hipLaunchKernelGGL((moe_small_kernel<T, true, NP, ND, 4>), grid, block, 0, st, p);
+  else if constexpr (NP == 2) {
+    if (p.K <= 16 * 128 && live > 2 * kCus && live <= 5 * kCus) hipLaunchKernelGGL((moe_small_kernel<T, false, NP, NG, 0>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((moe_small_kernel<T, false, NP, NG, 4>), grid, block, 0, st, p);
+  } else {
+    hipLaunchKernelGGL((moe_small_kernel<T, false, NP, NG, sizeof(T) == 4 ? 2 : 4>), grid, block, 0, st, p);
+  }
 }
 
 }  // namespace

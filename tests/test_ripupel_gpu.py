@@ -413,6 +413,14 @@ def test_moe(dtype, E, top, ff, d, M, monkeypatch):
             assert int(bufs.ticket) == 0
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E,top,ff,d", [(12, 2, 1536, 130), (3, 2, 8320, 40), (16, 4, 1100, 520)])
+def test_moe_sets_in_flight(dtype, E, top, ff, d, monkeypatch):
+    """The forms of the small tiles' loop: gate / up with one set between two and five workgroups a CU (the first two), one to
+    five k-groups dealt to four waves, the last set's partner missing."""
+    test_moe(dtype, E, top, ff, d, 33, monkeypatch)
+
+
 # ----------------------------------------------------------------------------- the model through the engine
 CFGS = {
     "odd": O.model_config(76, 101, [
