@@ -77,6 +77,25 @@ def test_linear_split_and_f32_residual(dtype, M, N, K, ns):
     assert torch.equal(rd[:, N:].cpu(), r[:, N:])
 
 
+@pytest.mark.parametrize("N,K", [(1003, 2064), (2048, 6144), (1024, 1024), (3904, 16), (4096, 208), (130, 48), (16416, 80), (2080, 4112)])
+def test_gemm_f32_rows_do_not_depend_on_their_company(N, K):
+    """A row's results have the same bits alone, in a decoded step and in a prompt, whichever kernel and waves serve it (a
+    token's expert does not change with what it is batched with)."""
+    gen = torch.Generator(device=DEV).manual_seed(N)
+    x, w, r = torch.randn(1100, K, device=DEV, generator=gen), torch.randn(N, K, device=DEV, generator=gen), torch.randn(1100, N, device=DEV, generator=gen)
+    E = ops.ext()
+
+    def run(M, epi):
+        out, rest = torch.empty(M, {2: N // 2, 6: N // 3}.get(epi, N), device=DEV), torch.empty(M, N - N // 3, device=DEV) if epi == 6 else None
+        E.gemm_f32(x[:M], w, out, epi, r[:M] if epi == 1 else None, rest)
+        return out if rest is None else torch.cat([out, rest], 1)
+
+    for epi in (0, 1, 6) + ((2,) if N % 32 == 0 else ()):
+        want = run(1100, epi)
+        for M in (1, 4, 16, 17, 32, 33, 64, 65, 200, 449, 777):
+            assert torch.equal(run(M, epi), want[:M]), (epi, M)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 1, 16), (16, 1003, 2064), (17, 2080, 48), (32, 16384, 32), (64, 7713, 144),  # rows kernel
                                    (33, 16400, 80), (65, 3904, 16),                # tiles: one / two row blocks, K short of a slice
                                    (200, 4096, 208), (449, 2001, 4112), (641, 3296, 96)])   # 4, 2 and 1 groups of waves
