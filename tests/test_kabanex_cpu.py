@@ -343,3 +343,9 @@ def test_intent_engine_serves_a_kabanex_preset():
     brain = LLMIntentEngine(eng, load_tokenizer("llama3"), budget_chars=160)
     out = brain.parse({"text": "scroll down", "context": {}})
     assert safe_parse(ParseResponse, out).success
+
+
+def test_scratch_of_no_layers():
+    """A stack without attention layers still gets its (empty) rows-form scratch."""
+    sc = ops.TalkScratch([], 128, "cpu")
+    assert sc.s.numel() and sc.stat.numel() and sc.part.numel() and not sc.counters.any()

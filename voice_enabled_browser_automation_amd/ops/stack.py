@@ -95,7 +95,7 @@ class TalkScratch:
 
     def __init__(self, layers: Sequence[Tuple[int, int, int, int, int]], max_ctx: int, device):
         """layers: (query heads, kv heads, dv, window, keep) of every layer."""
-        sizes = [rows_scratch(ROW_SLICE, 1, H, G, dv, max_ctx, window, keep) for H, G, dv, window, keep in layers]
+        sizes = [rows_scratch(ROW_SLICE, 1, H, G, dv, max_ctx, window, keep) for H, G, dv, window, keep in layers] or [(1, 1, 1, 1)]
         s, stat, part, cnt = (max(x) for x in zip(*sizes))
         f32 = dict(dtype=torch.float32, device=device)
         self.s, self.stat, self.part = (torch.zeros(n, **f32) for n in (s, stat, part))
