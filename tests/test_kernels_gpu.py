@@ -309,7 +309,9 @@ def test_decode_attention_cross_contiguous(attn_impl):
     (64, 4, 4, 24, [300, 24, 25, 7], None),      # halves across blocks: a table entry per key
     (128, 4, 1, 8, [130, 513, 9, 128], None),
     (64, 3, 3, 1009, [1009, 1008, 17, 992], None),  # one odd block for the whole context
-    (128, 8, 8, 16, [600] * 48, None),           # more items than workgroups
+    (128, 8, 8, 16, [600] * 48, None),           # 384 items of one chunk each
+    (64, 20, 20, 16, [600, 97, 33, 350] * 12, None),  # 960 items on 512 workgroups: a second one with steps of its own
+    (128, 16, 16, 16, [129, 1000, 64, 31] * 12, 1),   # 768 items
 ])
 def test_decode_attention_block_sizes(hd, nq, nkv, bs, ctx, splits):
     rows, per = len(ctx), -(-max(ctx) // bs)
@@ -675,8 +677,8 @@ def test_tiled_mfma_gemm_epilogues(M, tiled):
 
 
 @pytest.mark.parametrize("M", [256, 300, 1011])
-def test_gemm_8phase_256_tile(M):
-    """The 256 x 256 8-phase pipelined GEMM (gemm.hip P8; forced on every eligible shape) on
+def test_gemm_256_tile(M):
+    """The 256 x 256 two-phase pipelined GEMM (gemm.hip P8; forced on every eligible shape) on
     pre-tiled weights: every epilogue, split-K (few tiles) and a partial last row block, against
     the f32 reference -- then back to the measured routing."""
     E = ops.ext()
@@ -839,9 +841,30 @@ def test_gemm_keeps_the_order_of_its_sums():
     assert wt.to("cpu").keep_order and not ops.TiledWeight(w).keep_order
 
 
-def test_gemm_8phase_split_k_down_projection():
+@pytest.mark.parametrize("M,N,K,splits", [(2048, 4096, 2048, 1), (1011, 4096, 14336, 4), (1500, 4112, 384, 1),  # whole, sliced, partial blocks
+                                          (300, 4112, 640, 2), (257, 1296, 1152, 5), (300, 2064, 1664, 4)])  # slices that do not divide K
+def test_gemm_kept_order_has_the_bits_of_either_tile(M, N, K, splits):
+    """Both tiles forced in turn: the same slices, the same bits, rows and columns past the last whole tile among them."""
+    E = ops.ext()
+    x, w = rnd(M, K), rnd(N, K, scale=K ** -0.5)
+    wt, got = ops.TiledWeight(w, keep_order=True), []
+    try:
+        for mode in (0, 1):
+            E.gemm_set_p8(mode)
+            assert E.gemm_plan(0, M, N, K, keep_order=True, ws_floats=ops.GEMM_WS_FLOATS) == (mode == 1, splits)
+            got.append([ops.gemm(x, wt, torch.full((M, N), 7.0, dtype=BF, device=DEV))])
+            if N % 32 == 0:
+                got[-1].append(ops.gemm(x, wt, torch.full((M, N // 2), 7.0, dtype=BF, device=DEV), epi="swiglu"))
+    finally:
+        E.gemm_set_p8(2)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    exp = x.double() @ w.double().T
+    assert float((got[0][0].double() - exp).norm() / exp.norm()) < 2.0 ** -8  # (one rounding to bf16)
+
+
+def test_gemm_large_tile_split_k_down_projection():
     """Measured routing (mode 2): the 1011-row Llama-3-8B down projection (K = 14336) runs the
-    8-phase kernel in 4 split-K slices with the residual applied by the reduce kernel -- against
+    256 x 256 kernel in 4 split-K slices with the residual applied by the reduce kernel -- against
     an f32 reference (GPU fp32 matmul of the same bf16 operands)."""
     M, N, K = 1011, 4096, 14336
     x = rnd(M, K)
@@ -989,8 +1012,7 @@ def test_llama70b_tp8_per_rank_decode_shapes(M):
 @pytest.mark.parametrize("N,K", [(208, 128), (128, 256), (144, 384), (4096, 1152), (512, 5120)])
 def test_gemm_fp8_weights_few_rows(M, N, K):
     """Stages of one to a few k-groups, column remainders, slices of a few k-groups; f32 sums of exact products
-    (K roundings of at most 2^-24 of the sum of magnitudes); the product and its sum with the residual each rounded
-    to bf16 (2^-8; a product of one slice passes through bf16 before the residual is added)."""
+    (K roundings of at most 2^-24 of the sum of magnitudes); the sum with the residual rounded to bf16 once (2^-8)."""
     w = ops.FP8Weight.quantize(rnd(N, K, scale=K ** -0.5), tiled=True)
     x, r = rnd(M, K), rnd(M, N)
     y = torch.empty(M, N, dtype=BF, device=DEV)
@@ -999,7 +1021,7 @@ def test_gemm_fp8_weights_few_rows(M, N, K):
     wd = w.rows().double() * w.scale.double().view(-1, 1)
     prod = x.double() @ wd.T
     exp = prod + r.double()
-    tol = (exp.abs() + prod.abs()) * 2 ** -8 * (1 + 2 ** -8) + (x.double().abs() @ wd.abs().T + r.double().abs()) * (K + 2) * 2 ** -24
+    tol = exp.abs() * 2 ** -8 + (x.double().abs() @ wd.abs().T + r.double().abs()) * (K + 2) * 2 ** -24
     assert bool(((y.double() - exp).abs() <= tol).all())
 
 
