@@ -54,11 +54,10 @@ constexpr int BKG = 128;
 constexpr int kGroup = 4;  // row blocks of a grouped launch that walk the columns together
 
 // Workgroup shapes: BM x BN output tile, WM x WN waves, each wave (BM/WM) x (BN/WN).
-//   Cfg<128, 128, 2, 2>: 4 waves of 64 x 64, 64 KB LDS -> 2 workgroups per CU -- the one in use.
-//   (Measured and dropped: Cfg<256, 256, 2, 4>, 8 waves of 128 x 64, which reads 25 % fewer
-//   fragment bytes from LDS per MFMA: 929 vs 915 TF/s on the 1011-row gate/up projection and
-//   2-3x SLOWER on 1011-row o / down -- 64 workgroups cannot fill 256 CUs;
-//   profiles/r3_gemm_bench.md.)
+//   CfgS, 128 x 128: 4 waves of 64 x 64, 64 KB LDS, two workgroups per CU: few or odd tiles
+//   CfgP8, 256 x 256: 8 waves of 128 x 64, 144 KB, one per CU: a quarter less read from LDS per MFMA where its tiles fill the
+//     CUs (1011 x 28672 x 4096 237 -> 179 us) or their slices do (choose())
+//   CfgW8, CfgW8s: fp8 weights of <= 64 and <= 32 rows
 template <int BM_, int BN_, int WM_, int WN_>
 struct Cfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM_ * WN_, THREADS = 64 * NW;
