@@ -732,15 +732,14 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
-@pytest.mark.parametrize("kind", ["tiled", "rowmajor", "fp8"])
-@pytest.mark.parametrize("mode,M,N,K", [(2, 17, 400, 128), (2, 64, 384, 128), (2, 200, 400, 128), (1, 300, 512, 128), (2, 1500, 384, 384)])
+@pytest.mark.parametrize("mode,M,N,K,kind", [(*c, k) for c in ((2, 17, 400, 128), (2, 64, 384, 128), (2, 200, 400, 128), (1, 300, 512, 128),
+                                                               (2, 1500, 384, 384))
+                                             for k in ("tiled", "rowmajor", "fp8") if k != "fp8" or c[1] <= 64])  # (more: 8-bit x)
 def test_gemm_residual_is_added_before_rounding(mode, M, N, K, kind):
     """A product of one slice and its residual are rounded once, together: with a residual that takes away all but the last bits
     of the product, a rounding of the product (2^-9 of it) in front of the sum would be larger than what is left.
     Tolerance: that one rounding (2^-8) and K + 2 roundings of at most 2^-24 of the sum of magnitudes."""
     E = ops.ext()
-    if kind == "fp8" and M > ops.FP8_A16_ROWS:
-        pytest.skip("8-bit activations")
     x, w = rnd(M, K), rnd(N, K, scale=K ** -0.5)
     ww = {"tiled": lambda: ops.TiledWeight(w), "rowmajor": lambda: w, "fp8": lambda: ops.FP8Weight.quantize(w, tiled=True)}[kind]()
     wd = ww.rows().double() * ww.scale.double().view(-1, 1) if kind == "fp8" else w.double()
@@ -758,14 +757,12 @@ def test_gemm_residual_is_added_before_rounding(mode, M, N, K, kind):
     assert bool((exp.abs() > 4 * tol).any())  # (rounded in front, the sum is 0 or the last bit of the product: off by as much as exp)
 
 
-@pytest.mark.parametrize("kind", ["tiled", "rowmajor", "fp8"])
-@pytest.mark.parametrize("mode,M", [(2, 17), (2, 64), (2, 200), (1, 300)])
+@pytest.mark.parametrize("mode,M,kind", [(*c, k) for c in ((2, 17), (2, 64), (2, 200), (1, 300))
+                                         for k in ("tiled", "rowmajor", "fp8") if k != "fp8" or c[1] <= 64])
 def test_gemm_qkv_is_rotated_before_rounding(mode, M, kind):
     """Heads of a product of one slice are rotated in 32 bits and rounded once: where the two terms of a rotation cancel, a
     rounding of each in front of it would be larger than the tolerance of one rounding of their difference."""
     E = ops.ext()
-    if kind == "fp8" and M > ops.FP8_A16_ROWS:
-        pytest.skip("8-bit activations")
     K, nq, nkv, hd, bs = 128, 3, 1, 64, 16
     n = nq + 2 * nkv
     if mode == 1:
