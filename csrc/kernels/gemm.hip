@@ -552,9 +552,9 @@ VWA_DEVICE float reduce_item(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, in
   return finish_item<EPI>(p, q, m, c, a[0], b[0]);
 }
 
-// (round 4's 4-stage variant for one-row-block GEMMs measured slower in whole decode steps -- 128 KB
+// (a 4-stage variant for one-row-block GEMMs measured slower in whole decode steps -- 128 KB
 // of LDS leaves one workgroup per CU, so split-K grids above 256 workgroups ran in two rounds:
-// fp8 32 rows 4.97 vs 4.36 ms, profiles/r4_gemm_ab.md -- and was removed in round 5)
+// fp8 32 rows 4.97 vs 4.36 ms, profiles/r4_gemm_ab.md -- and was removed)
 template <class C, int EPI, bool WT, bool F8 = false, bool P8 = false, bool W8 = false, bool GRP = false, bool LINES = !GRP>
 __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(GemmParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];

@@ -78,7 +78,7 @@ def main():
         err = (out.float() - ref).abs().max().item() / (ref.abs().max().item() + 1e-6)
         fl = 2.0 * M * N * K
         r = dict(shape=name, M=M, N=N, K=K, hipblaslt_us=round(t_ref, 1), gemm_us=round(t_own, 1),
-                 tile128_us=round(t_128, 1), tile256_8phase_us=None if t_p8 is None else round(t_p8, 1),
+                 tile128_us=round(t_128, 1), tile256_us=None if t_p8 is None else round(t_p8, 1),
                  speedup=round(t_ref / t_own, 3), gemm_tflops=round(fl / t_own / 1e6, 1),
                  gemm_weight_tbps=round(N * K * 2 / t_own / 1e6, 2), rel_err=round(err, 5))
         r["cold"] = bool(a.cold)

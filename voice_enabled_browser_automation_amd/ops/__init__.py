@@ -447,7 +447,7 @@ def scratch(device, name: str, numel: int, dtype=torch.float32) -> torch.Tensor:
 GEMM_WS_FLOATS = 32 << 20  # split-K workspace (128 MB per device: 4 f32 slices of a 1k x 4096 output)
 # (a one-launch split-K -- the last slice of each tile reducing -- measured no faster at 32 decode
 # rows: the write-through drain + ticket + L2-missing partial loads cost what the reduce launch
-# does, fp8 o / down 26.3 vs 20.2 + 5.2 us, profiles/r4_gemm_one_launch_ab.md; removed in round 5.
+# does, fp8 o / down 26.3 vs 20.2 + 5.2 us, profiles/r4_gemm_one_launch_ab.md; removed.
 # The reduce loading all 8 slabs of an 8-way split in ONE batch instead of two batches of 4 measured 0.3-1.6 % slower whole
 # steps at 32-64 rows in workgroups of four waves, profiles/r6_reduce_one_batch_rejected_*.jsonl; in workgroups of one wave,
 # which small sums now take, eight in flight are the faster: gemm.hip launch_epi)
@@ -494,8 +494,8 @@ def _fp8_staging(x: torch.Tensor, K: int):
 
 def _fp8_input(x: torch.Tensor, fuse_rms: bool, eps: float):
     """(x8 [M, K], sx, rstd or None): x quantised per row by one kernel that also yields the
-    RMSNorm 1/rms.  (Round 4's opt-in hand-off -- the previous GEMM's split-K reduce quantising its
-    output rows -- measured slower in whole fp8 steps, profiles/r4_gemm_ab.md; removed in round 5.)"""
+    RMSNorm 1/rms.  (An opt-in hand-off -- the previous GEMM's split-K reduce quantising its
+    output rows -- measured slower in whole fp8 steps, profiles/r4_gemm_ab.md; removed.)"""
     M, K = x.shape
     x8, sx, rs = _fp8_staging(x, K)
     ext().quant_fp8_rows(x, x8[: M * K].view(M, K), sx, rs if fuse_rms else None, eps)
@@ -551,9 +551,9 @@ def gemm_ok(x: torch.Tensor, w, out: Optional[torch.Tensor] = None, residual: Op
 # Rows handled by the MFMA streaming (skinny) kernels; above this the hand-written LDS-tiled MFMA
 # GEMM (gemm.hip) takes the step (continuous batching of many sessions, prefill).
 SKINNY_MAX_M = 16
-# (round 4 built a 17..64-row form of the streaming kernel -- X streamed with the weights, MT = 2 /
+# (a 17..64-row form of the streaming kernel was built -- X streamed with the weights, MT = 2 /
 # 4 row fragments -- and measured it slower than the tiled GEMM for whole decode steps, 32 rows
-# 6.89 vs 5.65 ms, 64 rows 11.0 vs 6.9 ms, profiles/r4_rows_sweep_*; removed in round 5.)
+# 6.89 vs 5.65 ms, 64 rows 11.0 vs 6.9 ms, profiles/r4_rows_sweep_*; removed.)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None, *, out: Optional[torch.Tensor] = None,
