@@ -5,14 +5,12 @@
 
 namespace vwa {
 
-#define VWA_HD __host__ __device__ inline
-
 // A-image slot swizzle: chunk c of row r sits at slot c ^ F((r >> 1) & 7).  F makes every
 // ds_read_b128 lane group ({0-3,12-15,20-27}, {4-11,16-19,28-31}, ... : two k-chunk columns g,
 // 16 rows) hit 16 distinct (row parity, slot) bank groups: F maps the half-row indices
 // {0,1,6,7} to the even slots and {2,3,4,5} to the odd ones, so XOR-ing the chunk index with 2
 // (the other column of the group) cannot collide.  (Plain c ^ h measured 33 % bank conflicts.)
-VWA_HD int swz(int h) { return (0x64753120 >> (4 * h)) & 7; }
+__host__ __device__ inline int swz(int h) { return (0x64753120 >> (4 * h)) & 7; }
 
 // bf16 stages: half hs & 1 = h of a k-group is k 64 h .. 64 h + 64, a whole 128-byte line of every X row.  In the tiled
 // weight's order (lane group g of substep s: k 32 g + 8 s) that is the groups g = 2 h, 2 h + 1 of all four substeps: MFMA
@@ -25,20 +23,20 @@ VWA_HD int swz(int h) { return (0x64753120 >> (4 * h)) & 7; }
 // LINES false keeps the substeps' own order, for weights whose products choose experts further on (GemmParams::keep_order):
 // the same sums in another order move a product by its last bits, and a token whose scores nearly tie to another expert --
 // 1 in 300 decoded rows of a 16-expert model when its prompt alone was computed in the other order.
-VWA_HD int swzk(int h) { return (h & 1) | (h >> 2 << 1); }
-VWA_HD int chunk_of(int g, int sp) { return 4 * (g & 1) + 2 * sp + (g >> 1); }
+__host__ __device__ inline int swzk(int h) { return (h & 1) | (h >> 2 << 1); }
+__host__ __device__ inline int chunk_of(int g, int sp) { return 4 * (g & 1) + 2 * sp + (g >> 1); }
 
 constexpr unsigned kPastEnd = 0xFFFFFFF0u;  // vector offset outside of every resource (they end below 2 GB): reads zeros
 
 // Byte offset, in k-group 0, of lane l's 16-byte piece of tile row r (row m of X, ldx elements apart)
 template <bool F8, bool LINES>
-VWA_HD unsigned p8_x_piece(int m, int ldx, int r, int l) {
+__host__ __device__ inline unsigned p8_x_piece(int m, int ldx, int r, int l) {
   const int h = (r >> 1) & 7, c = (l & 7) ^ (F8 || !LINES ? swz(h) : swzk(h));
   return (unsigned)(F8 ? (size_t)m * ldx + 16 * c : ((size_t)m * ldx + (LINES ? 8 * c : 32 * (c >> 1) + 8 * (c & 1))) * 2);
 }
 // ... of MFMA sp of the weight's 16-column tile T (WT: pre-tiled, else row-major [N, K])
 template <bool F8, bool WT, bool LINES>
-VWA_HD unsigned p8_w_piece(int T, int sp, int K, int l) {
+__host__ __device__ inline unsigned p8_w_piece(int T, int sp, int K, int l) {
   if (F8) return (unsigned)((size_t)T * (K / 128) * 2048 + sp * 1024 + l * 16);
   const int g = l >> 4;
   return (unsigned)(2 * (WT ? (size_t)T * (K / 128) * 2048 + (LINES ? (2 * sp + (l >> 5)) * 512 + (l & 31) * 8 : sp * 512 + l * 8)
@@ -49,11 +47,11 @@ VWA_HD unsigned p8_w_piece(int T, int sp, int K, int l) {
 // one wraps there, then does not matter, and neither for any other piece (a piece inside by its vector offset stays inside
 // with the scalar one added).
 template <bool F8, bool LINES>
-VWA_HD unsigned p8_x_step(int hs, bool in) {
+__host__ __device__ inline unsigned p8_x_step(int hs, bool in) {
   return !in ? 0 : F8 ? hs * 128 : 2 * ((hs >> 1) * 128 + (LINES ? 64 : 16) * (hs & 1));
 }
 template <bool F8, bool WT, bool LINES>
-VWA_HD unsigned p8_w_step(int hs, bool in) {
+__host__ __device__ inline unsigned p8_w_step(int hs, bool in) {
   return !in ? 0 : F8 ? hs * 2048 : WT ? 2 * ((hs >> 1) * 2048 + (LINES ? 256 : 1024) * (hs & 1)) : p8_x_step<false, LINES>(hs, true);
 }
 

@@ -552,7 +552,7 @@ def gemm_ok(x: torch.Tensor, w, out: Optional[torch.Tensor] = None, residual: Op
 # GEMM (gemm.hip) takes the step (continuous batching of many sessions, prefill).
 SKINNY_MAX_M = 16
 # (a 17..64-row form of the streaming kernel was built -- X streamed with the weights, MT = 2 /
-# 4 row fragments -- and measured it slower than the tiled GEMM for whole decode steps, 32 rows
+# 4 row fragments -- and measured slower than the tiled GEMM for whole decode steps, 32 rows
 # 6.89 vs 5.65 ms, 64 rows 11.0 vs 6.9 ms, profiles/r4_rows_sweep_*; removed.)
 
 
