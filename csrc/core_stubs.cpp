@@ -11,6 +11,8 @@ int vwa_skinny_gemm(int, const SkinnyParams*, hipStream_t) { return kNotBuilt; }
 int vwa_chain_prepare(ChainParams*, int) { return kNotBuilt; }
 int vwa_chain_launch(const ChainParams*, int, int, int, int, int, hipStream_t, int, int, int, int) { return kNotBuilt; }
 int vwa_wdec_launch(const WdecParams*, int, hipStream_t) { return kNotBuilt; }
+int vwa_wdec_narrow_launch(const WdecParams*, int, hipStream_t) { return kNotBuilt; }
+int64_t vwa_wdec_narrow_part(int) { return 0; }
 int vwa_decode_attention(const DecodeAttnParams*, hipStream_t) { return kNotBuilt; }
 void vwa_set_attention_impl(int) {}
 int vwa_flash_attention(const FlashAttnParams*, hipStream_t) { return kNotBuilt; }

@@ -253,6 +253,7 @@ struct WdecParams {
   const uint32_t* smp_mask; int* smp_tok; int* smp_step; float* smp_part; int* loop_out; int* loop_cnt;
   int loop_max, loop_base_block;
   int* adv_tokens; int* adv_positions; int* adv_ctx; int64_t* adv_slots;
+  float* part;                        // narrow models (whisper_dec_narrow.hip): partial rows, vwa_wdec_narrow_part(d) numbers
 };
 
 #ifdef __cplusplus
@@ -268,6 +269,9 @@ int vwa_chain_launch(const ChainParams* d_cp, int seq, int n_phases, int attn_g,
                      int xg2 = 0, int f8 = 0, int o2 = 0, int n_layers = 1);
 // -10: a shape / role table the kernel does not take (the caller keeps per-kernel launches)
 int vwa_wdec_launch(const WdecParams* p, int grid, hipStream_t st);
+// d <= 512: three hand-offs a layer (no roles, n_prod; cnt holds 2048 + grid words)
+int vwa_wdec_narrow_launch(const WdecParams* p, int grid, hipStream_t st);
+int64_t vwa_wdec_narrow_part(int d);
 int vwa_gemm(int epi, const GemmParams* p, hipStream_t st);
 // routed experts' products over 128-pair tiles (GemmParams::g_*): epi 2 SwiGLU, 0 store
 int vwa_gemm_grouped(int epi, const GemmParams* p, hipStream_t st);

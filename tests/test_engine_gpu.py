@@ -501,6 +501,44 @@ def test_whisper_persistent_decoder_matches_per_kernel_path(graphs, model, monke
         assert err < 0.02 * (1 + b.abs().max().item()), (i, err)
 
 
+@pytest.mark.parametrize("ns,T,steps", [(1, 1500, 448), (2, 101, 70), (3, 1536, 130), (4, 1499, 70)])
+def test_narrow_persistent_decoder_matches_per_kernel_path(ns, T, steps, monkeypatch):
+    """whisper_dec_narrow.hip at every width it takes (128 ns), contexts up to the longest and across the 16- and 64-key edges,
+    whole, ragged and short key chunks, against the per-kernel path on the same weights and caches."""
+    import dataclasses
+
+    from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner
+
+    cfg = dataclasses.replace(get_config("whisper-tiny"), d_model=128 * ns, n_heads=2 * ns, n_enc_layers=1, n_dec_layers=2,
+                              n_audio_ctx=T)
+    m = WhisperModel(cfg, device="cuda", seed=6)
+    torch.manual_seed(7)
+    enc = [torch.randn(1, T, cfg.d_model, device="cuda").to(torch.bfloat16) for _ in range(2)]
+    watch = {0, 1, 14, 15, 16, 17, 62, 63, 64, 65, 127, 128, steps - 1}
+    runners = []
+
+    def run(persist: bool):
+        monkeypatch.setenv("VWA_ASR_PERSIST", "1" if persist else "0")
+        r = WhisperRunner(m, max_sessions=2, use_graphs=True)
+        runners.append(r)
+        for s in (0, 1):
+            r.set_cross(s, enc[s])
+        out = []
+        for p in range(steps):
+            for s in ((0, 1) if p < 20 else (1,)):
+                lg = r.step([(s, (13 * p + 5 * s) % 1000, p)])
+                if p in watch:
+                    out.append(lg.float().cpu().clone())
+        return out
+
+    ref, got = run(False), run(True)
+    assert not m.chain_error()
+    assert next(iter(m._wdec.values()))["part"] is not None  # (the narrow kernel ran)
+    for i, (a, b) in enumerate(zip(got, ref)):
+        err = (a - b).abs().max().item()
+        assert err < 0.02 * (1 + b.abs().max().item()), (i, err)
+
+
 @pytest.mark.parametrize("model", ["whisper-large-v3", "whisper-tiny"])
 def test_whisper_persistent_device_loop_is_one_launch_and_matches(model, monkeypatch):
     """The device-resident greedy loop (asr/engine.py) with the persistent decoder: each step is ONE

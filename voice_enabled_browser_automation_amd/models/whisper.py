@@ -489,7 +489,7 @@ class WhisperModel:
                       (tail[0], len(E), tail[1]) if tail[0].numel() else None)
         return cache[key]
 
-    # ---- persistent decoder (csrc/kernels/whisper_dec.hip wdec_kernel): a one-row step of the
+    # ---- persistent decoder (csrc/kernels/whisper_dec.hip wdec_kernel; d <= 512: whisper_dec_narrow.hip): a one-row step of the
     # Whisper model (tiny .. large: d a multiple of 128 up to 1536, ffn 4 d, head_dim 64) as ONE launch
     # over every decoder layer; each workgroup's weight tiles stay in its registers a layer ahead.
     def _wdec_ok(self, M: int) -> bool:
@@ -513,8 +513,15 @@ class WhisperModel:
         # cross-attention key chunks per head: 4 (8 measured: the cross level 0.3 us shorter, the
         # merge in the cross out-projection's staging 3.2 us longer, profiles/r6_wdec_nch_ab.jsonl)
         nch = 4
+        T = bufs.cross[0][0].shape[1]
+        # narrow models (d <= 512): three hand-offs a layer (whisper_dec_narrow.hip), one workgroup per head, per (head, key
+        # chunk) and per 64 hidden units, the LM head on the others
+        part = E.wdec_narrow_part(cfg.d_model)
+        narrow = part > 0 and grid >= 9 * self.H + 16 and 3 * -(-T // 4) < T <= 4 * 384
+        roles, n_prod = None, []
         try:
-            roles, n_prod = wdec_roles(grid, cfg.d_model, self.H, cfg.ffn, nch)
+            if not narrow:
+                roles, n_prod = wdec_roles(grid, cfg.d_model, self.H, cfg.ffn, nch)
         except ValueError:  # (a partitioned device with too few CUs for the tiles: per-kernel launches)
             self._wdec_disabled = True
             return None
@@ -531,16 +538,17 @@ class WhisperModel:
         flat = []
         for li, L in enumerate(self.dec):
             (wq, bq, cq), (wx, bx, cx), (w1, b1, c1) = L.f_qkv, L.f_xq, L.f_fc1
-            wxo, bxo = self._wdec_xq_o(L)
+            wxo, bxo = (None, None) if narrow else self._wdec_xq_o(L)
             flat += [wt(wq), bq, cq, wt(L.o), L.o_b, None, wt(wx), bx, cx, wt(L.xo), L.xo_b, None,
-                     wt(w1), b1, c1, wt(L.fc2), L.fc2_b, None, wt(wxo), bxo, None,
+                     wt(w1), b1, c1, wt(L.fc2), L.fc2_b, None, None if narrow else wt(wxo), bxo, None,
                      bufs.k_cache[li], bufs.v_cache[li], bufs.cross[li][0], bufs.cross[li][1]]
-        layers = E.wdec_layers(flat, len(self.dec), bufs.hidden)
-        cnt = E.alloc_uncached_i32(4096, bufs.hidden)  # level counters [8][8] x 128 B + error word
+        layers = E.wdec_layers(flat, len(self.dec), bufs.hidden, narrow)
+        # level counters [8][8] x 128 B, error word; narrow: each workgroup's launches behind them
+        cnt = E.alloc_uncached_i32(4096 + (2 * grid if narrow else 0), bufs.hidden)
         xpart = torch.zeros(self.H * nch * 68 + 3 * cfg.d_model, dtype=torch.float32, device=self.device)
-        T = bufs.cross[0][0].shape[1]
         w_lm = wt(self.f_lm[0])
-        st = dict(layers=layers, roles=torch.from_numpy(roles).to(self.device), n_prod=n_prod, cnt=cnt, xpart=xpart,
+        st = dict(layers=layers, roles=None if narrow else torch.from_numpy(roles).to(self.device), n_prod=n_prod, cnt=cnt,
+                  xpart=xpart, part=torch.zeros(part, dtype=torch.float32, device=self.device) if narrow else None,
                   keep=keep, lm_w=w_lm,
                   ints=[len(self.dec), cfg.d_model, self.H, cfg.ffn, T, bufs.k_cache.shape[3],
                         bufs.block_table.shape[1], nch, -(-T // nch), bufs.cross[0][0].shape[0], grid])
@@ -588,7 +596,7 @@ class WhisperModel:
                            [bufs.hidden, bufs.h, bufs.q, bufs.att, bufs.f, st["xpart"], bufs.seq_ids, bufs.ctx_lens,
                             bufs.slots, bufs.block_table, bufs.cross_table, st["cnt"]],
                            st["ints"], self.cfg.ln_eps, self.hd ** -0.5, st["n_prod"], st.get("ts"),
-                           int(st.get("opt", ops.env_int("VWA_WDEC_OPT"))), lm, emb, smp, base_block)
+                           int(st.get("opt", ops.env_int("VWA_WDEC_OPT"))), lm, emb, smp, base_block, st["part"])
         return bufs.logits[:1]
 
     def wdec_loop_step(self, bufs, mask: torch.Tensor, tok: torch.Tensor, step: torch.Tensor, out: torch.Tensor,
