@@ -50,7 +50,17 @@ void gemm_f32(Tensor x, Tensor w, Tensor y, int64_t epi, c10::optional<Tensor> r
   check_rc(vwa_gemm_f32((int)epi, &p, cur_stream(x)), "gemm_f32");
 }
 
-void layernorm_f32(Tensor x, Tensor w, c10::optional<Tensor> b, Tensor y, double eps) {
+// f32 partial rows [parts][rows][N] of a projection
+const float* slabs(const Tensor& t, int64_t rows, int64_t q, const char* name) {
+  check_t(t, true, name);
+  TORCH_CHECK(t.dim() == 3 && t.is_contiguous() && t.size(0) >= 1 && t.size(1) == rows && t.size(2) >= q && t.size(2) % 4 == 0, name,
+              " must be contiguous [parts, ", rows, ", >= ", q, " (a multiple of 4)]");
+  check_aligned(t, name);
+  return t.data_ptr<float>();
+}
+
+// parts (optional): x += their sum first
+void layernorm_f32(Tensor x, Tensor w, c10::optional<Tensor> b, Tensor y, double eps, c10::optional<Tensor> parts) {
   c10::DeviceGuard g(x.device());
   check_t(x, true, "x");
   const bool f32 = t_is_f32(y, "y");
@@ -60,7 +70,10 @@ void layernorm_f32(Tensor x, Tensor w, c10::optional<Tensor> b, Tensor y, double
   check_rows(y, rows, D, "y");
   check_aligned(x, "x");
   check_aligned(y, "y");
-  check_rc(vwa_layernorm_f32(x.data_ptr<float>(), (int)x.stride(0), w.data_ptr<float>(),
+  const float* br = parts.has_value() ? slabs(*parts, rows, (D + 3) / 4 * 4, "parts") : nullptr;
+  TORCH_CHECK(!br || x.size(0) == rows, "parts: x and y of the same rows");
+  check_rc(vwa_layernorm_f32(x.data_ptr<float>(), (int)x.stride(0), br, br ? (int)parts->size(2) : 0, br ? (int)parts->size(0) : 0,
+                             w.data_ptr<float>(),
                              b.has_value() ? f32p(*b, D, "b") : nullptr, y.data_ptr(),
                              (int)y.stride(0), (int)rows, (int)D, (int)y.size(1), (float)eps, f32, cur_stream(x)),
            "layernorm_f32");
@@ -356,7 +369,8 @@ void qkv_mingru(Tensor x, int64_t H, int64_t G, int64_t dk, int64_t dv, int64_t 
 void bind_stack(py::module_& m) {
   m.def("gemm_f32", &gemm_f32, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("epi"), py::arg("residual") = py::none(),
         py::arg("y2") = py::none());
-  m.def("layernorm_f32", &layernorm_f32);
+  m.def("layernorm_f32", &layernorm_f32, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("b"), pybind11::arg("y"), pybind11::arg("eps"),
+        pybind11::arg("parts") = pybind11::none());
   m.def("add_norm", &add_norm);
   m.def("embedding_f32", &embedding_f32);
   m.def("qkv_cache", &qkv_cache);

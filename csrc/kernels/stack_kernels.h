@@ -98,8 +98,8 @@ extern "C" {
 #endif
 int vwa_gemm_f32(int epi, const GemmF32Params* p, hipStream_t st);
 // y (T) [rows, ldy] = layer norm of x f32 rows over D columns (b null: no bias); columns D .. Dpad-1 of y are zeroed
-int vwa_layernorm_f32(const float* x, int ldx, const float* w, const float* b, void* y, int ldy, int rows, int D, int Dpad,
-                      float eps, int f32, hipStream_t st);
+int vwa_layernorm_f32(float* x, int ldx, const float* br, int ldb, int parts, const float* w, const float* b, void* y, int ldy,
+                      int rows, int D, int Dpad, float eps, int f32, hipStream_t st);
 // out f32 [rows, ldo] = table (T) rows * scale; ids outside the table give zeros; columns D .. Dpad-1 are zeroed
 int vwa_embedding_f32(const int* ids, const void* table, int ld, float* out, int ldo, int rows, int D, int Dpad, int vocab,
                       float scale, int f32, hipStream_t st);

@@ -40,15 +40,38 @@ VWA_DEVICE void row_weights(const float* w, int D, float (&o)[STEPS][4]) {
   }
 }
 
+// sum of n rows `slab` elements apart at this thread's columns, in their order, four rows' loads in flight
+template <int STEPS>
+VWA_DEVICE void sum_parts(const float* b, int64_t slab, int n, int last, float (&v)[STEPS][4]) {
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) ld4(b + min((i * 256 + (int)threadIdx.x) * 4, last), v[i]);
+  for (int k = 1; k < n; k += 3) {
+    float u[3][STEPS][4];
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+#pragma unroll
+      for (int i = 0; i < STEPS; ++i)
+        ld4(b + min(k + e, n - 1) * slab + min((i * 256 + (int)threadIdx.x) * 4, last), u[e][i]);
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+#pragma unroll
+      for (int i = 0; i < STEPS; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[i][j] += k + e < n ? u[e][i][j] : 0.f;
+  }
+}
+
 // one workgroup per row, the row held in registers: STEPS x 1024 columns, 4 per thread and step, all
 // loads in flight at once (columns past the row repeat its last quad and count as zero)
 constexpr int kLnSteps = 8;
-template <class T, int STEPS>
-__global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restrict__ x, int ldx,
-                                                            const float* __restrict__ w, const float* __restrict__ b,
-                                                            T* __restrict__ y, int ldy, int D, int Dpad, float eps) {
+// PARTS: x += the sum of `parts` rows (a projection's K slices, slab elements apart) first, in their order
+template <class T, int STEPS, bool PARTS>
+__global__ __launch_bounds__(256) void layernorm_f32_kernel(float* __restrict__ x, int ldx, const float* __restrict__ br, int ldb,
+                                                            int64_t slab, int parts, const float* __restrict__ w,
+                                                            const float* __restrict__ b, T* __restrict__ y, int ldy, int D,
+                                                            int Dpad, float eps) {
   __shared__ float red[2][4];
-  const float* xr = x + (size_t)blockIdx.x * ldx;
+  float* xr = x + (size_t)blockIdx.x * ldx;
   T* yr = y + (size_t)blockIdx.x * ldy;
   float v[STEPS][4], wv[STEPS][4], bv[STEPS][4];
   const int last = (D - 1) & ~3;
@@ -62,6 +85,17 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
   }
   row_weights<STEPS>(w, D, wv);
   row_weights<STEPS>(b ? b : w, D, bv);
+  if constexpr (PARTS) {
+    float u[STEPS][4];
+    sum_parts<STEPS>(br + (size_t)blockIdx.x * ldb, slab, parts, last, u);
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const int c = (i * 256 + (int)threadIdx.x) * 4;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[i][j] += u[i][j];
+      if (c < D) st4(xr + c, v[i]);
+    }
+  }
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < STEPS; ++i) {
@@ -96,14 +130,21 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(const float* __restr
   for (int c = ((D + 3) & ~3) + threadIdx.x; c < Dpad; c += 256) stv(yr + c, 0.f);
 }
 
+template <class T, int STEPS>
+void launch_ln_steps(float* x, int ldx, const float* br, int ldb, int64_t slab, int parts, const float* w, const float* b, T* y,
+                     int ldy, int rows, int D, int Dpad, float eps, hipStream_t st) {
+  if (br)
+    hipLaunchKernelGGL((layernorm_f32_kernel<T, STEPS, true>), dim3(rows), dim3(256), 0, st, x, ldx, br, ldb, slab, parts, w, b, y, ldy, D, Dpad, eps);
+  else
+    hipLaunchKernelGGL((layernorm_f32_kernel<T, STEPS, false>), dim3(rows), dim3(256), 0, st, x, ldx, br, ldb, slab, parts, w, b, y, ldy, D, Dpad, eps);
+}
 template <class T>
-void launch_ln(const float* x, int ldx, const float* w, const float* b, T* y, int ldy, int rows, int D, int Dpad, float eps,
-               hipStream_t st) {
-  const dim3 grid(rows), block(256);
-  if (D <= 1024) hipLaunchKernelGGL((layernorm_f32_kernel<T, 1>), grid, block, 0, st, x, ldx, w, b, y, ldy, D, Dpad, eps);
-  else if (D <= 2048) hipLaunchKernelGGL((layernorm_f32_kernel<T, 2>), grid, block, 0, st, x, ldx, w, b, y, ldy, D, Dpad, eps);
-  else if (D <= 4096) hipLaunchKernelGGL((layernorm_f32_kernel<T, 4>), grid, block, 0, st, x, ldx, w, b, y, ldy, D, Dpad, eps);
-  else hipLaunchKernelGGL((layernorm_f32_kernel<T, 8>), grid, block, 0, st, x, ldx, w, b, y, ldy, D, Dpad, eps);
+void launch_ln(float* x, int ldx, const float* br, int ldb, int64_t slab, int parts, const float* w, const float* b, T* y, int ldy,
+               int rows, int D, int Dpad, float eps, hipStream_t st) {
+  if (D <= 1024) launch_ln_steps<T, 1>(x, ldx, br, ldb, slab, parts, w, b, y, ldy, rows, D, Dpad, eps, st);
+  else if (D <= 2048) launch_ln_steps<T, 2>(x, ldx, br, ldb, slab, parts, w, b, y, ldy, rows, D, Dpad, eps, st);
+  else if (D <= 4096) launch_ln_steps<T, 4>(x, ldx, br, ldb, slab, parts, w, b, y, ldy, rows, D, Dpad, eps, st);
+  else launch_ln_steps<T, 8>(x, ldx, br, ldb, slab, parts, w, b, y, ldy, rows, D, Dpad, eps, st);
 }
 
 // mean and 1 / std of the row held as STEPS x 4 values per thread (columns past D are zero)
@@ -278,13 +319,15 @@ __global__ __launch_bounds__(256) void qkv_mingru_kernel(QkvCacheParams p, MinGr
 
 }  // namespace
 
-extern "C" int vwa_layernorm_f32(const float* x, int ldx, const float* w, const float* b, void* y, int ldy, int rows,
-                                 int D, int Dpad, float eps, int f32, hipStream_t st) {
-  if (rows < 1 || D < 1 || D > kLnSteps * 1024 || Dpad < D || ldx % 4 || ldy % 4 || ldx < ((D + 3) & ~3) || ldy < Dpad ||
-      Dpad % 4)
-    return -1;
-  if (f32) launch_ln(x, ldx, w, b, reinterpret_cast<float*>(y), ldy, rows, D, Dpad, eps, st);
-  else launch_ln(x, ldx, w, b, reinterpret_cast<u16*>(y), ldy, rows, D, Dpad, eps, st);
+// br (optional): f32 rows [parts][rows][ldb] added to x first (x is written then)
+extern "C" int vwa_layernorm_f32(float* x, int ldx, const float* br, int ldb, int parts, const float* w, const float* b, void* y,
+                                 int ldy, int rows, int D, int Dpad, float eps, int f32, hipStream_t st) {
+  const int q = (D + 3) & ~3;
+  if (rows < 1 || D < 1 || D > kLnSteps * 1024 || Dpad < D || ldx % 4 || ldy % 4 || ldx < q || ldy < Dpad || Dpad % 4) return -1;
+  if (br && (ldb % 4 || ldb < q || parts < 1)) return -2;
+  const int64_t slab = (int64_t)rows * ldb;
+  if (f32) launch_ln(x, ldx, br, ldb, slab, parts, w, b, reinterpret_cast<float*>(y), ldy, rows, D, Dpad, eps, st);
+  else launch_ln(x, ldx, br, ldb, slab, parts, w, b, reinterpret_cast<u16*>(y), ldy, rows, D, Dpad, eps, st);
   return (int)hipGetLastError();
 }
 

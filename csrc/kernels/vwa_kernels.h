@@ -260,6 +260,7 @@ struct WdecParams {
 extern "C" {
 #endif
 int vwa_skinny_gemm(int epi, const SkinnyParams* p, hipStream_t st);
+int vwa_gemm_parts(const GemmParams* p, int* parts, hipStream_t st);
 int vwa_skinny_stream(int epi, const SkinnyParams* p, int grid_cap, int ks, hipStream_t st);
 void vwa_skinny_set_x_skew(int skew);  // LDS-staged X rows: 64-B skew every 4 rows (default) or none (0)
 int vwa_chain_prepare(ChainParams* cp, int grid);

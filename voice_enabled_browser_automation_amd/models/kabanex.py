@@ -218,17 +218,22 @@ class KabanexModel:
         rows = dict(positions=bufs.positions[:M], seq_ids=bufs.seq_ids[:M], slots=bufs.slots[:M])
         ops.embedding_f32(bufs.tokens[:M], self.embed, out=x)
         h = bufs.normed[:M]
+        self._norm(0, x, h)
         for li in range(self.cfg.n_layers):
             self._layer(li, bufs, M, kv, x, h, rows, plan)
         if n_sel is not None:
             x = torch.index_select(x, 0, bufs.sel[:n_sel], out=bufs.hidden_sel[:n_sel])
         return self.lm_logits(bufs, x) if head else x
 
+    def _norm(self, li: int, x, h, parts=None) -> None:
+        L = self.layers[li]
+        ops.layernorm_f32(x, L.norm_w, L.norm_b, eps=self.cfg.norm_eps, out=h, parts=parts)
+
     def _layer(self, li: int, bufs, M: int, kv, x, h, rows, plan) -> None:
+        """One layer of normed rows h; leaves the next layer's in h."""
         C, D, L = self.cfg.layers[li], self.dims[li], self.layers[li]
         a = C.left
         _, _, g0, z0, x0, r0 = D.at
-        ops.layernorm_f32(x, L.norm_w, L.norm_b, eps=self.cfg.norm_eps, out=h)
         y = bufs.mix[: M * D.n_mix].view(M, D.n_mix)
         cat = bufs.cat[D][:M]
         r_at, f_at = D.heads_out, D.heads_out + D.w
@@ -242,8 +247,13 @@ class KabanexModel:
                            keep=a.keep_first, talk=L.talk, talk_frag=L.talk_frag, gate=y[:, g0 : g0 + D.gate],
                            out_scale=C.left_scale, max_ctx=bufs.max_ctx, scratch=bufs.talk, out=cat[:, : D.heads_out],
                            plan=plan, **rows)
-        xo = x[:, : self.n_out]
-        ops.linear(cat, L.w_out, out=xo, residual=xo)
+        last = li + 1 == self.cfg.n_layers
+        parts = None if last else ops.linear_parts(cat, L.w_out)  # (few rows: K slices, which the norm adds to x)
+        if parts is None:
+            xo = x[:, : self.n_out]
+            ops.linear(cat, L.w_out, out=xo, residual=xo)
+        if not last:
+            self._norm(li + 1, x, h, parts)
 
     def lm_logits(self, bufs, hs: torch.Tensor, col_mask: Optional[torch.Tensor] = None, mask_rows: int = 1,
                   gather: bool = True) -> torch.Tensor:

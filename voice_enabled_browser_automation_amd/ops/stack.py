@@ -103,12 +103,33 @@ class TalkScratch:
 
 
 # ----------------------------------------------------------------------------- ops
-def layernorm_f32(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], *, eps: float, out: torch.Tensor) -> torch.Tensor:
-    """out = (x - mean) / sqrt(var + eps) * w (+ b) of f32 rows; out may be wider than w (zero columns)."""
+def layernorm_f32(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], *, eps: float, out: torch.Tensor,
+                  parts: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out = (x - mean) / sqrt(var + eps) * w (+ b) of f32 rows; out may be wider than w (zero columns).
+    parts: linear_parts' rows, added to x first."""
     if not x.is_cuda:
         return ref.layernorm_f32(x, w, b, eps=eps, out=out)
-    _ext().layernorm_f32(x, w, b, out, eps)
+    _ext().layernorm_f32(x, w, b, out, eps, parts)
     return out
+
+
+# Rows whose projections leave their K slices to the norm behind them: those of the tiled GEMM that take more slices than tiles
+# fill the chip.  (A decoded row's streaming kernel cut in two by K, so that 2048 columns have a workgroup on every CU: 2048 x 12288
+# 15.6 -> 14.3 us alone, whole steps 25.2 -> 25.4 ms -- it is bound by its start and the chip's rate, not by a CU's -- so not.)
+PARTS_ROWS = 64
+
+
+def linear_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
+    """x @ w^T as f32 partial rows [parts, rows, N] for layernorm_f32, or None: this call has none (more or fewer rows, other
+    weights; the caller takes linear).  They lie in the GEMMs' workspace: the norm is the next launch on the stream."""
+    from . import GEMM_WS_FLOATS, SKINNY_MAX_M, TiledWeight, gemm_ok, scratch
+
+    if not x.is_cuda or not SKINNY_MAX_M < x.shape[0] <= PARTS_ROWS or not isinstance(w, TiledWeight) or not gemm_ok(x, w):
+        return None
+    ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
+    M, N = x.shape[0], w.shape[0]
+    n = _ext().linear_parts(x, w.t, ws)
+    return ws[: n * M * N].view(n, M, N)
 
 
 def add_norm(x: torch.Tensor, branch: torch.Tensor, w1: torch.Tensor, w2: Optional[torch.Tensor], *, eps: float,
