@@ -57,7 +57,7 @@ constexpr int kGroup = 4;  // row blocks of a grouped launch that walk the colum
 //   CfgS, 128 x 128: 4 waves of 64 x 64, 64 KB LDS, two workgroups per CU: few or odd tiles
 //   CfgP8, 256 x 256: 8 waves of 128 x 64, 144 KB, one per CU: a quarter less read from LDS per MFMA where its tiles fill the
 //     CUs (1011 x 28672 x 4096 237 -> 179 us) or their slices do (choose())
-//   CfgW8, CfgW8s: fp8 weights of <= 64 and <= 32 rows
+//   CfgF, CfgFs: <= 64 and <= 32 rows, bf16 or fp8 weights
 template <int BM_, int BN_, int WM_, int WN_>
 struct Cfg {
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM_ * WN_, THREADS = 64 * NW;
@@ -67,20 +67,23 @@ struct Cfg {
   static constexpr int W8STAGE = 2 * BM * 128 + BN * 128;
   static constexpr int NCOL_MAX = BN / WN;
   static constexpr int EPI_LDS = NW * (FM * 16) * (NCOL_MAX * 2 + 16);
-  static constexpr int LDS = 2 * STAGE > EPI_LDS ? 2 * STAGE : EPI_LDS;
-  static constexpr int W8NST = BM <= 32 ? 3 : 2;  // its stage buffers: what lets two workgroups share a CU
+  static constexpr int NST = BM <= 32 ? 4 : BM <= 64 ? 3 : 2;   // stage buffers: few rows take what lets two workgroups share a CU
+  static constexpr int LDS = NST * STAGE > EPI_LDS ? NST * STAGE : EPI_LDS;
+  static constexpr int W8NST = BM <= 32 ? 3 : 2;
   static constexpr int W8LDS = W8NST * W8STAGE > EPI_LDS ? W8NST * W8STAGE : EPI_LDS;
   static_assert((BM / 8) % NW == 0 && (BN / 8) % NW == 0, "whole LDS-DMA instructions per wave");
 };
 using CfgS = Cfg<128, 128, 2, 2>;
-// W8A16 decode tile (<= 64 rows: one row block): 64 x 128, 4 waves of 64 x 32, 32 KB stages (16 KB
-// of fp8 weights each -- the W8A8 kernel's weight bytes per stage: a half-k-group bf16-style stage
-// carried 8 KB and measured 1.25x slower whole decode steps), 2 workgroups per CU
-using CfgW8 = Cfg<64, 128, 1, 4>;
-// ... of <= 32 rows: 24 KB stages, so three fit where two did and two are in flight behind the one being read (a slice of a
-// 32-row step is weights arriving and little else: with the sum of the slices, 4096 x 4096 14.6 -> 11.4 us, 4096 x 14336
-// 27.9 -> 24.7, 28672 x 4096 35.6 -> 33.1)
-using CfgW8s = Cfg<32, 128, 1, 4>;
+// Few rows (<= 64: one row block): 64 x 128, 4 waves of 64 x 32, 2 workgroups per CU.  Such a product is weights arriving and
+// little else, so what counts is how many of their bytes are on the way.
+// bf16: three 24 KB stages where the 128-row tile had two of 32 KB, half of them rows that are not there (and one stage in flight
+// behind the one being read): BFMEASURE
+// W8A16: 32 KB stages (16 KB of fp8 weights each -- the W8A8 kernel's weight bytes per stage: a half-k-group bf16-style stage
+// carried 8 KB and measured 1.25x slower whole decode steps)
+using CfgF = Cfg<64, 128, 1, 4>;
+// ... of <= 32 rows: bf16 four stages of 20 KB; fp8 24 KB stages, so three fit where two did and two are in flight behind the one
+// being read (with the sum of the slices, 4096 x 4096 14.6 -> 11.4 us, 4096 x 14336 27.9 -> 24.7, 28672 x 4096 35.6 -> 33.1)
+using CfgFs = Cfg<32, 128, 1, 4>;
 
 // buffer resource over [base, base + bytes): loads past the end return zero (rows >= M, weight
 // tiles >= N), so the stage issue needs no bounds branches
@@ -103,7 +106,7 @@ VWA_DEVICE void dma16(__amdgpu_buffer_rsrc_t r, char* lds_wave_base, unsigned vo
 // F8 (W8A8): one FULL k-group per stage (16 fp8 = 16 B per chunk): A chunk c = 2 g + s2 holds
 // X8[row][128 kg + 32 g + 16 s2 .. + 16), B the fp8 tiled block [s2][lane][16 B] of the tile
 // (ops.tile_weight_fp8) -- the same stage images as a bf16 half k-group.
-// W8 (W8A16, CfgW8): one FULL k-group per stage -- X as the two bf16 half-k-group A images (each as
+// W8 (W8A16): one FULL k-group per stage -- X as the two bf16 half-k-group A images (each as
 // above) and B the fp8 tiled k-group of every tile verbatim ([tile][s2][lane][16 B]: block s2 = h
 // holds the lane's k 32 g + 16 h .. + 16, both sub-steps of half h), converted to bf16 fragments on
 // the LDS read -- no quantised copy of X, half the weight bytes of bf16.
@@ -435,7 +438,7 @@ VWA_DEVICE void sum_items(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, int m
 // columns 5.8 -> 5.1 us, 6144 with the rotation 7.3 -> 5.5)
 template <int EPI> struct ItemPre {
   float scale, swa[8], swb[8], ba[8], bb[8];
-  uint4 r[2];      // residual: 8 bf16 (r[0]) or f32
+  u32x4 r0, r1;    // residual: 8 bf16 (r0) or f32 (vectors: as structs they went through 272 bytes of scratch a lane)
   float4 rope[4];
   int64_t slot;
 };
@@ -454,12 +457,13 @@ VWA_DEVICE ItemPre<EPI> item_pre(const GemmParams& p, int m, int c) {
     if constexpr (kTwoSrc<EPI>) q.swb[e] = p.sw ? p.sw[n1 + e] : 1.f;
     if constexpr (EPI == EPI_QKV) q.bb[e] = bias_at(p, n1 + e);
   }
+  q.r0 = q.r1 = u32x4{0, 0, 0, 0};
   if (p.y_f32 == 2) {  // f32 residual stream: 16-byte accesses (rows are 32-byte aligned)
-    const uint4* r = reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(p.R) + (size_t)m * p.ldr + c);
-    q.r[0] = r[0];
-    q.r[1] = r[1];
+    const u32x4* r = reinterpret_cast<const u32x4*>(reinterpret_cast<const float*>(p.R) + (size_t)m * p.ldr + c);
+    q.r0 = r[0];
+    q.r1 = r[1];
   } else if (kResid<EPI> && !p.y_f32) {
-    q.r[0] = *reinterpret_cast<const uint4*>(p.R + (size_t)m * p.ldr + c);
+    q.r0 = *reinterpret_cast<const u32x4*>(p.R + (size_t)m * p.ldr + c);
   }
   if (EPI == EPI_QKV && p.use_rope) {
 #pragma unroll
@@ -502,7 +506,7 @@ VWA_DEVICE float finish_item(const GemmParams& p, const ItemPre<EPI>& q, int m, 
   }
   if (p.y_f32 == 2) {
     float4* y = reinterpret_cast<float4*>(reinterpret_cast<float*>(p.Y) + (size_t)m * p.ldy + c);
-    const float4 r0 = __builtin_bit_cast(float4, q.r[0]), r1 = __builtin_bit_cast(float4, q.r[1]);
+    const float4 r0 = __builtin_bit_cast(float4, q.r0), r1 = __builtin_bit_cast(float4, q.r1);
     y[0] = make_float4(v[0] + r0.x, v[1] + r0.y, v[2] + r0.z, v[3] + r0.w);
     y[1] = make_float4(v[4] + r1.x, v[5] + r1.y, v[6] + r1.z, v[7] + r1.w);
     return 0.f;
@@ -514,7 +518,7 @@ VWA_DEVICE float finish_item(const GemmParams& p, const ItemPre<EPI>& q, int m, 
   }
   if constexpr (kResid<EPI>) {
     float r[8];
-    unpack8(q.r[0], r);
+    unpack8(__builtin_bit_cast(uint4, q.r0), r);
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] += r[e];
   }
@@ -606,10 +610,9 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   // barriers with counted vmcnt (a __syncthreads would drain the in-flight DMA)
   constexpr int SPG = F8 || W8 ? 1 : 2;  // stages per k-group
   constexpr int STG = W8 ? C::W8STAGE : C::STAGE;
-  constexpr int NST = W8 ? C::W8NST : 2;  // stage buffers
+  constexpr int NST = W8 ? C::W8NST : C::NST;  // stage buffers
   constexpr int PER = (W8 ? 2 : 1) * (C::BM / 8 / C::NW) + C::BN / 8 / C::NW;  // LDS-DMA instructions of a stage and wave
-  static_assert(PER == (NST == 3 ? 6 : 8),
-                "LDS-DMA instructions per thread per stage (the counted vmcnt)");
+  static_assert(PER * (NST - 1) < 64, "LDS-DMA instructions of the stages in flight (the counted vmcnt)");
   const int h0 = SPG * kg0, nh = SPG * (kg1 - kg0);
   // X extent: the last row starts at (M-1)*ldx and is K long (rows may overlap: conv views)
   const size_t x_bytes = ((GRP ? x_rows - 1 : (size_t)(p.M - 1)) * p.ldx + p.K) * (F8 ? 1 : 2);
@@ -683,11 +686,16 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   } else {
   if (nh > 0) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0, lds, rows);
   if (nh > 1) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
-  if (NST == 3 && nh > 2) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 2, lds + 2 * STG, rows);
+  if (NST > 2 && nh > 2) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 2, lds + 2 * STG, rows);
+  if (NST > 3 && nh > 3) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 3, lds + 3 * STG, rows);
+  static_assert(NST <= 4, "stages issued ahead");
   for (int i = 0; i < nh; ++i) {
-    char* at = lds + (NST == 2 ? i & 1 : i % NST) * STG;
-    if (NST == 3 && i + 2 < nh)
-      asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");  // this stage landed everywhere
+    char* at = lds + (NST == 2 || NST == 4 ? i & (NST - 1) : i % NST) * STG;
+    // this stage landed everywhere (the ones behind it stay in flight)
+    if (NST > 3 && i + 3 < nh)
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * PER) : "memory");
+    else if (NST > 2 && i + 2 < nh)
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * PER) : "memory");
     else if (i + 1 < nh)
       asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PER) : "memory");
     else
@@ -964,26 +972,29 @@ __global__ __launch_bounds__(256) void row_rstd_kernel(const u16* __restrict__ x
   if (lane_id() == 0) rstd[row] = rsqrtf(ss / (float)K + eps);
 }
 
+int cdiv(int a, int b) { return (a + b - 1) / b; }
+
+// bf16 weights on tile C
 template <class C, int EPI>
 int launch_cfg(const GemmParams& p, hipStream_t st) {
   const int tiles = ((p.M + C::BM - 1) / C::BM) * ((p.N + C::BN - 1) / C::BN);
   const dim3 grid(tiles * p.splits * (p.nbatch > 1 ? p.nbatch : 1));
-  const int lds = 2 * C::STAGE > C::LDS ? 2 * C::STAGE : C::LDS;  // two stage buffers
-  if (p.sw && p.sx)
-    hipLaunchKernelGGL((gemm_kernel<C, EPI, true, true>), grid, dim3(C::THREADS), lds, st, p);
-  else if (p.sw)  // W8A16: bf16 X, fp8 tiled weights, on its own tile (launch_epi)
-    return -17;
-  else if (p.w_tiled)
-    hipLaunchKernelGGL((gemm_kernel<C, EPI, true, false>), grid, dim3(C::THREADS), lds, st, p);
+  if (p.w_tiled)
+    hipLaunchKernelGGL((gemm_kernel<C, EPI, true, false>), grid, dim3(C::THREADS), C::LDS, st, p);
   else
-    hipLaunchKernelGGL((gemm_kernel<C, EPI, false, false>), grid, dim3(C::THREADS), lds, st, p);
+    hipLaunchKernelGGL((gemm_kernel<C, EPI, false, false>), grid, dim3(C::THREADS), C::LDS, st, p);
   return 0;
+}
+
+// a product that keeps its order of sums, on any tile
+template <class C, int EPI, bool P8>
+void launch_kept(const GemmParams& p, hipStream_t st) {
+  hipLaunchKernelGGL((gemm_kernel<C, EPI, true, false, P8, false, false, false>), dim3(cdiv(p.M, C::BM) * cdiv(p.N, C::BN) * p.splits),
+                     dim3(C::THREADS), C::LDS, st, p);
 }
 
 int g_p8_mode = 2;         // 0: the 128^2 kernel only, 1: the 256^2 one from 256 rows (bf16: of pre-tiled whole column tiles), 2: choose()
 int g_split_fill_pct = 0;  // > 0: vwa_gemm_splits' fill, and the rules by shape alone instead of plan()
-
-int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // Tile and K slices of a bf16 product of >= 128 rows: the cheapest by an estimate in us, fitted to 180 shapes (130 .. 12000
 // rows, 384 .. 28672 columns, K 384 .. 14336; both tiles, 1 .. 16 slices): 9 % off (rms of the logarithm), and 1.4 % slower than the
@@ -1069,13 +1080,10 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
   constexpr bool kKeeps = EPI == EPI_STORE || EPI == EPI_SWIGLU;
   if (kKeeps && p.keep_order) {
     if constexpr (kKeeps) {
-      if (p8)
-        hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, true, false, true, false, false, false>),
-                           dim3(cdiv(p.M, 256) * cdiv(p.N, 256) * p.splits), dim3(CfgP8::THREADS), CfgP8::LDS, st, p);
-      else
-        hipLaunchKernelGGL((gemm_kernel<CfgS, EPI, true, false, false, false, false, false>),
-                           dim3(cdiv(p.M, CfgS::BM) * cdiv(p.N, CfgS::BN) * p.splits), dim3(CfgS::THREADS),
-                           2 * CfgS::STAGE > CfgS::LDS ? 2 * CfgS::STAGE : CfgS::LDS, st, p);
+      if (p8) launch_kept<CfgP8, EPI, true>(p, st);
+      else if (p.M <= CfgFs::BM) launch_kept<CfgFs, EPI, false>(p, st);
+      else if (p.M <= CfgF::BM) launch_kept<CfgF, EPI, false>(p, st);
+      else launch_kept<CfgS, EPI, false>(p, st);
     }
   } else if (p8) {
     const int tiles = ((p.M + 255) / 256) * ((p.N + 255) / 256);
@@ -1089,11 +1097,18 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
       hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, false, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
                          CfgP8::LDS, st, p);
   } else if (p.sw && !p.sx) {  // W8A16
-    const dim3 grid((unsigned)(cdiv(p.M, CfgW8::BM) * cdiv(p.N, CfgW8::BN) * p.splits)), block(CfgW8::THREADS);
-    if (p.M <= CfgW8s::BM)
-      hipLaunchKernelGGL((gemm_kernel<CfgW8s, EPI, true, false, false, true>), grid, block, CfgW8s::W8LDS, st, p);
+    const dim3 grid((unsigned)(cdiv(p.M, CfgF::BM) * cdiv(p.N, CfgF::BN) * p.splits)), block(CfgF::THREADS);
+    if (p.M <= CfgFs::BM)
+      hipLaunchKernelGGL((gemm_kernel<CfgFs, EPI, true, false, false, true>), grid, block, CfgFs::W8LDS, st, p);
     else
-      hipLaunchKernelGGL((gemm_kernel<CfgW8, EPI, true, false, false, true>), grid, block, CfgW8::W8LDS, st, p);
+      hipLaunchKernelGGL((gemm_kernel<CfgF, EPI, true, false, false, true>), grid, block, CfgF::W8LDS, st, p);
+  } else if (p.sw) {  // W8A8
+    hipLaunchKernelGGL((gemm_kernel<CfgS, EPI, true, true>), dim3(cdiv(p.M, CfgS::BM) * cdiv(p.N, CfgS::BN) * p.splits),
+                       dim3(CfgS::THREADS), CfgS::LDS, st, p);
+  } else if (p.M <= CfgFs::BM) {  // (the slices are those of the 128-row tile, and so are the bits)
+    launch_cfg<CfgFs, EPI>(p, st);
+  } else if (p.M <= CfgF::BM) {
+    launch_cfg<CfgF, EPI>(p, st);
   } else {
     launch_cfg<CfgS, EPI>(p, st);
   }
@@ -1111,8 +1126,7 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
 template <class C, int EPI, bool P8>
 int launch_grouped(const GemmParams& p, hipStream_t st) {
   const dim3 grid(p.g_max * ((p.N + C::BN - 1) / C::BN)), block(C::THREADS);
-  const int lds = 2 * C::STAGE > C::LDS ? 2 * C::STAGE : C::LDS;
-  hipLaunchKernelGGL((gemm_kernel<C, EPI, true, false, P8, false, true>), grid, block, lds, st, p);
+  hipLaunchKernelGGL((gemm_kernel<C, EPI, true, false, P8, false, true>), grid, block, C::LDS, st, p);
   return (int)hipGetLastError();
 }
 
@@ -1132,7 +1146,7 @@ extern "C" int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, 
     // W8A16, two workgroups to a CU: slices while they fit and keep 4 k-groups each, 2 below half a chip.  Measured, 32 rows
     // (us at 4 / 8 / 16 slices): 4096 x 4096 13.9 / 11.4 / 11.4 (64 rows 17.3 / 14.3 / 16.6), 4096 x 14336 34.7 / 24.7 / 21.4,
     // 6144 x 4096 16.2 / 16.4 / 16.8, 14336 x 4096 22.0 / 25.5 / -
-    const int t = cdiv(M, CfgW8::BM) * cdiv(N, CfgW8::BN);
+    const int t = cdiv(M, CfgF::BM) * cdiv(N, CfgF::BN);
     while (t * s * 2 <= 2 * cus && KG / (2 * s) >= (t * s < cus / 2 ? 2 : 4) && (int64_t)(s * 2) * M * N <= ws_floats) s *= 2;
     return s;
   }
