@@ -1043,6 +1043,30 @@ Plan plan(const GemmParams& p) {
   return best;
 }
 
+// K slices of a bf16 product of <= 64 rows (tiles of 32 or 64 rows x 128 columns): the cheapest by an estimate in us, fitted to 270
+// timings (24, 48 and 64 rows, 22 weights of 1024 .. 32768 columns and K 1024 .. 14336, 1 .. 32 slices), 7 % off (rms of the
+// logarithm).  Its choices are 0.8 % slower than the best of each shape; powers of two until three quarters of the CUs have a
+// tile, the rule before, 6.0 %, and 20 - 48 % where one slice fills half the chip (48 rows: 9472 x 1024 15.0 us in four slices,
+// 11.0 whole; 17664 x 2048 25.9 -> 20.4; 2048 x 2048 12.1 in sixteen, 10.6 in eight).
+//   a workgroup's k-groups one after another, against all of the weight at the chip's rate (the larger counts, both where they are
+//   close); a sum of slices is a launch and its f32 partials
+int few_slices(const GemmParams& p) {
+  const int KG = p.K / BKG;
+  int best = 1;
+  float least = 0.f;
+  for (int s0 = 1; s0 <= 32 && s0 <= KG; s0 *= 2) {
+    if (s0 > 1 && (!p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
+    const int per = cdiv(KG, s0), s = cdiv(KG, per);
+    const float alone = (0.52f + 0.0063f * p.M) * per, chip = (float)p.N * p.K * (2.f / 6.1e6f) * (256.f / p.cus);
+    const float us = cbrtf(alone * alone * alone + chip * chip * chip) + (s > 1 ? 3.2f + (float)s * p.M * p.N * (4 * 0.44e-6f) : 0.f);
+    if (s0 == 1 || us < least) {
+      least = us;
+      best = s0;
+    }
+  }
+  return best;
+}
+
 // Slices of whole large tiles by shape alone, in powers of two until they cover the CUs; *fill: the tiles alone, or slices of
 // >= 2048 k each, do
 int slices_256(const GemmParams& p, bool* fill) {
@@ -1069,7 +1093,10 @@ Plan choose(const GemmParams& p) {
     r.p8 = g_p8_mode == 1 ? p.M >= 256 : g_p8_mode == 2 && (p.sx || p.M >= 128) && estimate(p, true, r.splits) < estimate(p, false, r.splits);
     return r;
   }
-  if (g_p8_mode == 2 && g_split_fill_pct == 0) return p.M >= 128 ? plan(p) : r;
+  if (g_p8_mode == 2 && g_split_fill_pct == 0) {
+    if (p.M <= CfgF::BM) r.splits = few_slices(p);
+    return p.M >= 128 ? plan(p) : r;
+  }
   if (p.w_tiled && s && (g_p8_mode == 1 || (g_p8_mode == 2 && fill))) r = Plan{true, s};
   return r;
 }

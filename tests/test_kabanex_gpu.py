@@ -648,7 +648,7 @@ def test_norm_adds_a_projections_slices(M, N, K, D):
     want = x[:, :D].double() + a.double() @ w[:D].double().T
     nw, nb = rnd(D), rnd(D)
     parts = ops.linear_parts(a, ops.TiledWeight(w))
-    assert parts.shape[1:] == (M, N) and (parts.shape[0] > 1) == (K > 128)
+    assert parts.shape == (ops.ext().gemm_plan(0, M, N, K)[1], M, N) and (parts.shape[0] > 1) == (K >= 2048)
     out = torch.full((M, ld), 7.0, device="cuda", dtype=torch.bfloat16)
     ops.layernorm_f32(x, nw, nb, eps=1e-5, out=out, parts=parts)
     # (f32 sums of K bf16 products: about sqrt(K) roundings of 2^-24)

@@ -1243,18 +1243,22 @@ def test_flash_attention_is_bitwise_reproducible(hd, causal, qmul):
 @pytest.mark.parametrize("M", [17, 31, 32, 33, 48, 63, 64])
 def test_gemm_few_row_tiles_give_the_bits_of_the_128_row_tile(M, K):
     """17 .. 64 rows on the 32- and 64-row tiles (three and four stage buffers; products of fewer stages than buffers) against the
-    same rows of a 128-row-tile call: the slices depend on the weight alone, and a tile of rows does not change a row's sums."""
+    same rows of a 128-row-tile call in the same slices: a tile of rows does not change a row's sums."""
     torch.manual_seed(M * K)
     N = 272
     x = torch.randn(65, K, device="cuda").to(torch.bfloat16)
     w = (torch.randn(N, K, device="cuda") * K ** -0.5).to(torch.bfloat16)
     r = torch.randn(65, N, device="cuda").to(torch.bfloat16)
-    for tw in (ops.TiledWeight(w), ops.TiledWeight(w, keep_order=True), w):
-        for epi, res in (("none", None), ("resid", r), ("gelu", None)):
-            outs = [torch.empty(m, N, dtype=torch.bfloat16, device="cuda") for m in (M, 65)]
-            for m, o in zip((M, 65), outs):
-                ops.gemm(x[:m], tw, o, epi=epi, residual=None if res is None else res[:m])
-            assert torch.equal(outs[0], outs[1][:M]), (epi, type(tw))
+    ops.ext().gemm_set_split_fill(75)  # (both by one rule for the slices)
+    try:
+        for tw in (ops.TiledWeight(w), ops.TiledWeight(w, keep_order=True), w):
+            for epi, res in (("none", None), ("resid", r), ("gelu", None)):
+                outs = [torch.empty(m, N, dtype=torch.bfloat16, device="cuda") for m in (M, 65)]
+                for m, o in zip((M, 65), outs):
+                    ops.gemm(x[:m], tw, o, epi=epi, residual=None if res is None else res[:m])
+                assert torch.equal(outs[0], outs[1][:M]), (epi, type(tw))
+    finally:
+        ops.ext().gemm_set_split_fill(0)
     want = x[:M].double() @ w.double().T
     got = ops.gemm(x[:M], ops.TiledWeight(w), torch.empty(M, N, dtype=torch.bfloat16, device="cuda"))
     assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
