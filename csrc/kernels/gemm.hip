@@ -1173,7 +1173,9 @@ extern "C" int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, 
     // W8A16, two workgroups to a CU: slices while they fit and keep 4 k-groups each, 2 below half a chip.  Measured, 32 rows
     // (us at 4 / 8 / 16 slices): 4096 x 4096 13.9 / 11.4 / 11.4 (64 rows 17.3 / 14.3 / 16.6), 4096 x 14336 34.7 / 24.7 / 21.4,
     // 6144 x 4096 16.2 / 16.4 / 16.8, 14336 x 4096 22.0 / 25.5 / -
+    // None of 8 k-groups and a quarter of the chip's tiles: 8192 x 1024 9.3 us in two, 8.1 whole, 32768 x 1024 16.6 and 12.0
     const int t = cdiv(M, CfgF::BM) * cdiv(N, CfgF::BN);
+    if (KG <= 8 && t >= cus / 4) return 1;
     while (t * s * 2 <= 2 * cus && KG / (2 * s) >= (t * s < cus / 2 ? 2 : 4) && (int64_t)(s * 2) * M * N <= ws_floats) s *= 2;
     return s;
   }

@@ -1262,3 +1262,58 @@ def test_gemm_few_row_tiles_give_the_bits_of_the_128_row_tile(M, K):
     want = x[:M].double() @ w.double().T
     got = ops.gemm(x[:M], ops.TiledWeight(w), torch.empty(M, N, dtype=torch.bfloat16, device="cuda"))
     assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
+
+
+def test_rows_take_tiles_line():
+    """(no launch) a large weight at any row count, smaller ones from 4 and 8 rows on, never one that keeps an order."""
+    w = lambda n, k, keep=False: ops.TiledWeight(t=torch.empty(n, k, dtype=torch.bfloat16, device="meta"), keep_order=keep)  # noqa: E731
+    assert [ops.rows_take_tiles(m, w(17664, 2048)) for m in (1, 3, 4, 16)] == [True] * 4
+    assert [ops.rows_take_tiles(m, w(2048, 12288)) for m in (1, 3, 4, 7, 8)] == [False, False, True, True, True]
+    assert [ops.rows_take_tiles(m, w(2048, 4096)) for m in (1, 4, 7, 8, 16)] == [False, False, False, True, True]
+    assert [ops.rows_take_tiles(m, w(9472, 1024)) for m in (1, 16)] == [True, True] and not ops.rows_take_tiles(16, w(8192, 512))
+    assert not ops.rows_take_tiles(16, w(32768, 4096, True)) and not ops.rows_take_tiles(16, torch.empty(32768, 4096, device="meta"))
+
+
+@pytest.mark.parametrize("M", [1, 2, 5, 8, 15, 16])
+@pytest.mark.parametrize("N,K", [(8208, 896), (12288, 1024), (1104, 6144), (4096, 4096)])
+def test_few_rows_on_either_kernel(M, N, K, monkeypatch):
+    """Every form of a projection that rows_take_tiles sends to the tiled GEMM, against the streaming kernel and float64: bias,
+    GELU, bf16 and f32 residuals, f32 results, split columns, rows wider than K."""
+    torch.manual_seed(M + N)
+    xw = torch.randn(M, K + 64, device="cuda").bfloat16()
+    x = xw[:, :K]
+    tw = ops.TiledWeight((torch.randn(N, K, device="cuda") * K ** -0.5).bfloat16())
+    b = torch.randn(N, device="cuda").bfloat16()
+    r16, r32 = torch.randn(M, N, device="cuda").bfloat16(), torch.randn(M, N, device="cuda")
+    prod = x.double() @ tw.dense().double().T
+    n1 = N // 32 * 16
+    bf = lambda n=N: torch.full((M, n), 9.0, device="cuda", dtype=torch.bfloat16)  # noqa: E731
+    f32 = lambda: torch.full((M, N), 9.0, device="cuda")  # noqa: E731
+
+    def forms():
+        yield ops.linear(x, tw, out=bf()), prod
+        yield ops.linear(x, tw, b, out=bf()), prod + b.double()
+        yield ops.linear(x, tw, b, out=bf(), act="gelu"), torch.nn.functional.gelu(prod + b.double())
+        yield ops.linear(x, tw, b, out=bf(), residual=r16), prod + b.double() + r16.double()
+        yield ops.linear(x, tw, out=f32(), out_dtype=torch.float32), prod
+        y = r32.clone()
+        yield ops.linear(x, tw, out=y, residual=y), prod + r32.double()
+        y, y2 = bf(n1), bf(N - n1)
+        ops.linear_split(x, tw, y, y2)
+        yield torch.cat([y, y2], 1), torch.cat([prod[:, :n1], prod[:, n1:].clamp_min(0) ** 2], 1)
+        if N % 32 == 0:
+            gu = prod.view(M, N // 32, 2, 16)
+            yield (ops.linear_swiglu(x, tw, out=bf(N // 2)),
+                   (torch.nn.functional.silu(gu[:, :, 0]) * gu[:, :, 1]).reshape(M, N // 2))
+
+    outs = []
+    for tiles in (True, False):
+        monkeypatch.setattr(ops, "rows_take_tiles", lambda m, w, t=tiles: t)
+        outs.append([])
+        for got, want in forms():
+            # f32 sums, then one rounding to bf16 (a relu's square: its own rounding, twice the relative error of the sum)
+            tol = 1e-5 if got.dtype == torch.float32 else 2.0 ** -8
+            assert (got.double() - want).norm() / want.norm() < tol
+            outs[-1].append(got)
+    for a, c in zip(*outs):
+        assert (a.double() - c.double()).norm() / c.double().norm() < (1e-5 if a.dtype == torch.float32 else 2.0 ** -7)

@@ -204,10 +204,11 @@ class LlamaModel:
     # ------------------------------------------------------------------ forward
     def _rms_stats(self, M: int):
         """The two RMS-statistics buffers of the per-kernel many-row path (None when the projections
-        run elsewhere: <= 16 rows -- the streaming kernels fuse the RMSNorm themselves -- CPU, or TP,
+        run elsewhere: few rows of the streaming kernels, which fuse the RMSNorm themselves, CPU, or TP,
         whose row-parallel outputs are partial sums until the all-reduce)."""
-        if M <= ops.SKINNY_MAX_M or self.device.type != "cuda" or self.tp.size > 1 or \
-                not ops.env_flag("VWA_RMS_HANDOFF"):
+        L = self.layers[0]
+        few = M <= ops.SKINNY_MAX_M and not all(ops.rows_take_tiles(M, w) for w in (L.qkv, L.o, L.gu, L.down))
+        if few or self.device.type != "cuda" or self.tp.size > 1 or not ops.env_flag("VWA_RMS_HANDOFF"):
             return None
         if getattr(self, "_ss", None) is None:
             # (int64: u64 fixed-point sums, ops.SS_SCALE -- integer atomics keep them reproducible)

@@ -316,6 +316,21 @@ def _stream_ok(x: torch.Tensor, w) -> bool:
     return x.shape[0] <= SKINNY_MAX_M and x.shape[1] % 128 == 0 and w.shape[0] % 16 == 0
 
 
+def rows_take_tiles(M: int, w) -> bool:
+    """Up to SKINNY_MAX_M rows of a pre-tiled weight are the tiled GEMM's (gemm.hip, its 32-row tile) where it is the faster one:
+    a large weight, a smaller one the more rows there are.  The streaming kernel finishes 16 columns at a time (a large weight is
+    many rounds of them, the last one rarely full), and every row costs it reads of X beside the weights; the tiled one has four
+    stages of 128 columns in flight, and a sum of slices where its tiles leave the chip idle.  us, streaming / tiled, 1 and 16 rows:
+    32768 x 1024 21.3 / 14.6 and 23.8 / 14.4, 17664 x 2048 19.7 / 17.4 and 22.7 / 18.3, 2048 x 12288 15.4 / 16.2 and 23.2 / 15.4,
+    4096 x 4096 11.2 / 12.2 and 15.8 / 12.3, 2048 x 2048 6.1 / 7.6 and 8.0 / 8.3.  Over 37 weights and 1, 2, 4, 8, 16 rows this
+    line is 0.7 % slower than the better of both (the streaming kernel alone 8.9 %), and nowhere more than 7 % slower than it.
+    Weights that keep one order of their sums stay with the one kernel."""
+    if not isinstance(w, TiledWeight) or w.keep_order:
+        return False
+    N, K = w.shape
+    return (K <= 1024 and N > 8192) or 2 * N * K >= (70e6 if M < 4 else 25e6 if M < 8 else 12e6)
+
+
 def plain(w):
     """The row-major tensor of a weight (TiledWeight -> dense(); anything else unchanged)."""
     return w.dense() if isinstance(w, TiledWeight) else w
@@ -622,7 +637,11 @@ def _linear_impl(x, w, bias, out, residual, act, fuse_rms, eps, out_dtype, ln_c,
     if out is None:
         out = torch.empty((M, w.shape[0]), dtype=dt, device=x.device)
     if isinstance(w, TiledWeight):
-        if _gpu(x) and _stream_ok(x, w) and (ln_c is None or _ln_fold_fits(x, w)):
+        tiles = gemm_ok(x, w, out, residual) and (act == "none" or residual is None) and \
+            (out.dtype == torch.bfloat16 or _f32_resid(out, residual) or (residual is None and act == "none"))
+        # (a norm or a mask of the streaming kernel's own keeps the call there)
+        few = tiles and not mk and ln_c is None and not (fuse_rms and ss["ss_in"] is None) and rows_take_tiles(M, w)
+        if _gpu(x) and _stream_ok(x, w) and not few and (ln_c is None or _ln_fold_fits(x, w)):
             epi = {"none": 0, "gelu": 3}[act]
             if residual is not None:
                 assert act == "none"
@@ -632,8 +651,7 @@ def _linear_impl(x, w, bias, out, residual, act, fuse_rms, eps, out_dtype, ln_c,
             return out
         if ln_c is not None:
             return linear(_layernorm_plain(x, eps), w, bias, out=out, residual=residual, act=act, out_dtype=out_dtype)
-        if _gpu(x) and gemm_ok(x, w, out, residual) and (act == "none" or residual is None) and \
-                (out.dtype == torch.bfloat16 or _f32_resid(out, residual) or (residual is None and act == "none")):
+        if tiles:
             e = "resid" if residual is not None else ("gelu" if act == "gelu" else "none")
             return gemm(x, w, out, epi=e, bias=bias, residual=residual, fuse_rms=fuse_rms, eps=eps, **ssk())
         w = w.dense()
@@ -699,7 +717,8 @@ def linear_swiglu(x: torch.Tensor, w_gu: torch.Tensor, *, fuse_rms: bool = False
         ext().gemm_f32(x, w_gu, out, 2)
         return out
     if isinstance(w_gu, TiledWeight):
-        if _gpu(x) and _stream_ok(x, w_gu):
+        few = (not fuse_rms or ss_in is not None) and gemm_ok(x, w_gu, out) and rows_take_tiles(M, w_gu)
+        if _gpu(x) and _stream_ok(x, w_gu) and not few:
             ext().skinny_gemm_swiglu(x, w_gu.t, None, out, fuse_rms, eps, None, True)
             return out
         if _gpu(x) and gemm_ok(x, w_gu, out):
@@ -766,7 +785,9 @@ def qkv_rope_write(x: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Te
     ln_c: folded LayerNorm on x (see linear).  ss_in: handed-off sums of squares (see ops.gemm)."""
     M = x.shape[0]
     if isinstance(w_qkv, TiledWeight):
-        if _gpu(x) and _stream_ok(x, w_qkv) and (ln_c is None or _ln_fold_fits(x, w_qkv)):
+        few = (ln_c is None and (not fuse_rms or ss_in is not None) and GEMM_QKV_FUSED and gemm_ok(x, w_qkv)
+               and rows_take_tiles(M, w_qkv))
+        if _gpu(x) and _stream_ok(x, w_qkv) and not few and (ln_c is None or _ln_fold_fits(x, w_qkv)):
             ext().skinny_gemm_qkv(x, w_qkv.t, bias, fuse_rms and ln_c is None, eps, n_q_heads, n_kv_heads, head_dim,
                                   rope is not None, positions, slots, rope, q_out, k_cache, v_cache, None, ln_c, True)
             return q_out[:M]

@@ -122,9 +122,10 @@ PARTS_ROWS = 64
 def linear_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
     """x @ w^T as f32 partial rows [parts, rows, N] for layernorm_f32, or None: this call has none (more or fewer rows, other
     weights; the caller takes linear).  They lie in the GEMMs' workspace: the norm is the next launch on the stream."""
-    from . import GEMM_WS_FLOATS, SKINNY_MAX_M, TiledWeight, gemm_ok, scratch
+    from . import GEMM_WS_FLOATS, SKINNY_MAX_M, TiledWeight, gemm_ok, rows_take_tiles, scratch
 
-    if not x.is_cuda or not SKINNY_MAX_M < x.shape[0] <= PARTS_ROWS or not isinstance(w, TiledWeight) or not gemm_ok(x, w):
+    if not x.is_cuda or x.shape[0] > PARTS_ROWS or not isinstance(w, TiledWeight) or not gemm_ok(x, w) or (
+            x.shape[0] <= SKINNY_MAX_M and not rows_take_tiles(x.shape[0], w)):
         return None
     ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
     M, N = x.shape[0], w.shape[0]
@@ -152,7 +153,7 @@ def embedding_f32(ids: torch.Tensor, table: torch.Tensor, *, out: torch.Tensor, 
 def linear_split(x: torch.Tensor, w, out: torch.Tensor, out2: Optional[torch.Tensor]) -> torch.Tensor:
     """One projection of a normed row for a layer's mixers and its feed-forward: the first out.shape[1]
     columns of x @ w^T to ``out``, relu(.)^2 of the others to ``out2`` (None: there are none)."""
-    from . import SKINNY_MAX_M, TiledWeight, GEMM_WS_FLOATS, linear, scratch
+    from . import SKINNY_MAX_M, TiledWeight, GEMM_WS_FLOATS, gemm_ok, linear, rows_take_tiles, scratch
 
     if out2 is None:
         return linear(x, w, out=out)
@@ -163,7 +164,8 @@ def linear_split(x: torch.Tensor, w, out: torch.Tensor, out2: Optional[torch.Ten
         return out
     tiled = isinstance(w, TiledWeight)
     wt = w.t if tiled else w
-    if x.shape[0] <= SKINNY_MAX_M and tiled:
+    few = tiled and gemm_ok(x, w, out) and gemm_ok(x, w, out2) and rows_take_tiles(x.shape[0], w)
+    if x.shape[0] <= SKINNY_MAX_M and tiled and not few:
         _ext().skinny_gemm(x, wt, None, out, 5, False, 0.0, None, None, None, True, y2=out2)
     else:
         _ext().gemm(x, wt, None, out, 6, None, None, tiled, scratch(x.device, "gemm_ws", GEMM_WS_FLOATS), y2=out2)
