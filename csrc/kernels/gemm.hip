@@ -1050,7 +1050,8 @@ Plan plan(const GemmParams& p) {
 // 11.0 whole; 17664 x 2048 25.9 -> 20.4; 2048 x 2048 12.1 in sixteen, 10.6 in eight).
 //   a workgroup's k-groups one after another, against all of the weight at the chip's rate (the larger counts, both where they are
 //   close); a sum of slices is a launch and its f32 partials
-int few_slices(const GemmParams& p) {
+// parts: no launch adds the slices up, but the workgroup of a row's norm reads its row of each (at about 40 GB/s)
+int few_slices(const GemmParams& p, bool parts) {
   const int KG = p.K / BKG;
   int best = 1;
   float least = 0.f;
@@ -1058,7 +1059,8 @@ int few_slices(const GemmParams& p) {
     if (s0 > 1 && (!p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
     const int per = cdiv(KG, s0), s = cdiv(KG, per);
     const float alone = (0.52f + 0.0063f * p.M) * per, chip = (float)p.N * p.K * (2.f / 6.1e6f) * (256.f / p.cus);
-    const float us = cbrtf(alone * alone * alone + chip * chip * chip) + (s > 1 ? 3.2f + (float)s * p.M * p.N * (4 * 0.44e-6f) : 0.f);
+    const float sum = parts ? (float)s * p.N * (4 / 4.e4f) : s > 1 ? 3.2f + (float)s * p.M * p.N * (4 * 0.44e-6f) : 0.f;
+    const float us = cbrtf(alone * alone * alone + chip * chip * chip) + sum;
     if (s0 == 1 || us < least) {
       least = us;
       best = s0;
@@ -1082,7 +1084,7 @@ bool keeps_order(int epi, const GemmParams& p) {
 }
 
 // Tile and slices of a launch (p.splits: those of vwa_gemm_splits)
-Plan choose(const GemmParams& p) {
+Plan choose(const GemmParams& p, bool parts = false) {
   Plan r{false, p.splits < 1 ? 1 : p.splits};
   if (p.nbatch > 1 || p.cus <= 0 || (p.sw && !p.sx)) return r;
   bool fill = false;
@@ -1094,7 +1096,7 @@ Plan choose(const GemmParams& p) {
     return r;
   }
   if (g_p8_mode == 2 && g_split_fill_pct == 0) {
-    if (p.M <= CfgF::BM) r.splits = few_slices(p);
+    if (p.M <= CfgF::BM) r.splits = few_slices(p, parts);
     return p.M >= 128 ? plan(p) : r;
   }
   if (p.w_tiled && s && (g_p8_mode == 1 || (g_p8_mode == 2 && fill))) r = Plan{true, s};
@@ -1199,7 +1201,7 @@ extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int* large, int* sp
 }
 
 namespace {
-int checks_and_plan(int epi, GemmParams& p, bool* p8) {
+int checks_and_plan(int epi, GemmParams& p, bool* p8, bool parts = false) {
   if (p.M < 1 || p.N < 16 || p.N % 16 || p.K < BKG || p.K % BKG) return -10;
   if (p.ldx % (p.sx ? 16 : 8) || (reinterpret_cast<uintptr_t>(p.X) & 15) || (reinterpret_cast<uintptr_t>(p.W) & 15))
     return -11;
@@ -1213,7 +1215,7 @@ int checks_and_plan(int epi, GemmParams& p, bool* p8) {
                            (reinterpret_cast<uintptr_t>(p.Y2) & 15)))
     return -19;
   p.keep_order = keeps_order(epi, p);
-  const Plan pl = choose(p);
+  const Plan pl = choose(p, parts);
   *p8 = pl.p8;
   p.splits = pl.splits;
   const int KG = p.K / BKG;
@@ -1235,7 +1237,7 @@ extern "C" int vwa_gemm_parts(const GemmParams* pp, int* parts, hipStream_t st) 
   p.ldy = p.N;
   p.y_f32 = 1;
   if (!p.ws || p.bias || p.rstd || p.ss_in || p.sx || p.nbatch > 1 || (int64_t)p.M * p.N > p.ws_cap) return -10;
-  const int r = checks_and_plan(EPI_STORE, p, &p8);
+  const int r = checks_and_plan(EPI_STORE, p, &p8, true);
   if (r) return r;
   *parts = p.splits;
   return launch_epi<EPI_STORE>(p, st, p8, false);

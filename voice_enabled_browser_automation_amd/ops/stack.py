@@ -113,22 +113,24 @@ def layernorm_f32(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], *
     return out
 
 
-# Rows whose projections leave their K slices to the norm behind them: those of the tiled GEMM that take more slices than tiles
-# fill the chip.  (A decoded row's streaming kernel cut in two by K, so that 2048 columns have a workgroup on every CU: 2048 x 12288
-# 15.6 -> 14.3 us alone, whole steps 25.2 -> 25.4 ms -- it is bound by its start and the chip's rate, not by a CU's -- so not.)
+# Rows whose projections leave their K slices to the norm behind them.  Without a launch for their sum the tiled GEMM is ahead of the
+# streaming kernel from the first row on (us with the norm, 1 / 16 rows: 1024 x 6144 12.3 -> 9.5 / 16.0 -> 10.0, 2048 x 2048 8.7 -> 8.5 /
+# 10.8 -> 8.8, 2048 x 12288 18.9 -> 17.5 / 25.6 -> 17.2) but for few rows of wide outputs, whose columns fill the chip by themselves
+# (4096 x 8192: 20.3 / 22.2 at one row, 21.7 / 21.4 at four).
+# (The streaming kernel cut in two by K for the same norm: 2048 x 12288 15.6 -> 14.3 us alone, whole steps 25.2 -> 25.4 ms.)
 PARTS_ROWS = 64
 
 
 def linear_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
-    """x @ w^T as f32 partial rows [parts, rows, N] for layernorm_f32, or None: this call has none (more or fewer rows, other
-    weights; the caller takes linear).  They lie in the GEMMs' workspace: the norm is the next launch on the stream."""
-    from . import GEMM_WS_FLOATS, SKINNY_MAX_M, TiledWeight, gemm_ok, rows_take_tiles, scratch
+    """x @ w^T as f32 partial rows [parts, rows, N] for layernorm_f32, or None: this call has none (more rows, other weights;
+    the caller takes linear).  They lie in the GEMMs' workspace: the norm is the next launch on the stream."""
+    from . import GEMM_WS_FLOATS, TiledWeight, gemm_ok, rows_take_tiles, scratch
 
-    if not x.is_cuda or x.shape[0] > PARTS_ROWS or not isinstance(w, TiledWeight) or not gemm_ok(x, w) or (
-            x.shape[0] <= SKINNY_MAX_M and not rows_take_tiles(x.shape[0], w)):
+    M, N = x.shape[0], w.shape[0]
+    if not x.is_cuda or M > PARTS_ROWS or not isinstance(w, TiledWeight) or w.keep_order or not gemm_ok(x, w) or (
+            M < 4 and N >= 4096 and not rows_take_tiles(M, w)):
         return None
     ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
-    M, N = x.shape[0], w.shape[0]
     n = _ext().linear_parts(x, w.t, ws)
     return ws[: n * M * N].view(n, M, N)
 
