@@ -1060,16 +1060,23 @@ Plan plan(const GemmParams& p) {
 // 11.0 whole; 17664 x 2048 25.9 -> 20.4; 2048 x 2048 12.1 in sixteen, 10.6 in eight).
 //   a workgroup's k-groups one after another, against all of the weight at the chip's rate (the larger counts, both where they are
 //   close); a sum of slices is a launch and its f32 partials
+// fp8 weights (W8A16): the same of 520 timings (20, 32, 48 and 64 rows, 21 weights of 1024 .. 32768 columns and K 1024 .. 14336,
+// 1 .. 32 slices), 5 % off; its choices are 0.6 % slower than the best of each shape, slices until twice the CUs have a tile, the rule
+// before, 10 % and up to 50 % (32 rows: 28672 x 4096 30.0 us in two slices, 23.1 whole; 6144 x 4096 14.3 -> 12.9).
 // parts: no launch adds the slices up, but the workgroup of a row's norm reads its row of each (at about 40 GB/s)
 int few_slices(const GemmParams& p, bool parts) {
-  const int KG = p.K / BKG;
+  const int KG = p.K / BKG, blocks = cdiv(p.M, CfgF::BM);
+  const bool w8 = p.sw != nullptr;
+  const float per_kg = w8 ? (p.M <= CfgFs::BM ? 0.42f : 0.68f) + 0.00065f * (blocks > 1 ? CfgF::BM : p.M) : 0.52f + 0.0063f * p.M;
+  const float chip = (float)p.N * p.K * blocks * (w8 ? 1.f / 6.2e6f : 2.f / 6.1e6f) * (256.f / p.cus);
+  const float launch = w8 ? 2.6f : 3.2f, slab = (float)p.M * p.N * (4 * (w8 ? 0.53e-6f : 0.44e-6f));
   int best = 1;
   float least = 0.f;
   for (int s0 = 1; s0 <= 32 && s0 <= KG; s0 *= 2) {
     if (s0 > 1 && (!p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
     const int per = cdiv(KG, s0), s = cdiv(KG, per);
-    const float alone = (0.52f + 0.0063f * p.M) * per, chip = (float)p.N * p.K * (2.f / 6.1e6f) * (256.f / p.cus);
-    const float sum = parts ? (float)s * p.N * (4 / 4.e4f) : s > 1 ? 3.2f + (float)s * p.M * p.N * (4 * 0.44e-6f) : 0.f;
+    const float alone = per_kg * per;
+    const float sum = parts ? (float)s * p.N * (4 / 4.e4f) : s > 1 ? launch + s * slab : 0.f;
     const float us = cbrtf(alone * alone * alone + chip * chip * chip) + sum;
     if (s0 == 1 || us < least) {
       least = us;
@@ -1096,7 +1103,11 @@ bool keeps_order(int epi, const GemmParams& p) {
 // Tile and slices of a launch (p.splits: those of vwa_gemm_splits)
 Plan choose(const GemmParams& p, bool parts = false) {
   Plan r{false, p.splits < 1 ? 1 : p.splits};
-  if (p.nbatch > 1 || p.cus <= 0 || (p.sw && !p.sx)) return r;
+  if (p.nbatch > 1 || p.cus <= 0) return r;
+  if (p.sw && !p.sx) {
+    if (g_split_fill_pct == 0) r.splits = few_slices(p, false);
+    return r;
+  }
   bool fill = false;
   const int s = p.M >= 256 && p.N % 256 == 0 ? slices_256(p, &fill) : 0;
   // (g_p8_mode picks the tile; the slices of W8A8 and kept-order products are part of the order of their sums)
@@ -1176,21 +1187,11 @@ int launch_grouped(const GemmParams& p, hipStream_t st) {
 // Split while the workgroups cover less than this % of the CUs (0: per-dtype default).  Measured
 // on the Llama-3-8B decode steps of 32 / 64 rows (tools/rows_sweep.py, profiles/r4_gemm_ab.md):
 // bf16 75 % (5.08 / 5.69 ms vs 5.21 / 6.08 at 100 %), fp8 100 % (4.42 / 5.03 vs 4.62 / 5.06 at 75 %).
-// (bf16 products of >= 128 rows: plan())
+// (bf16 products of >= 128 rows: plan(); of <= 64 rows and W8A16: few_slices())
 extern "C" int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, int f8) {
   const int tiles = ((M + CfgS::BM - 1) / CfgS::BM) * ((N + CfgS::BN - 1) / CfgS::BN);
   const int KG = K / BKG;
   int s = 1;
-  if (f8 == 2 && g_split_fill_pct <= 0) {
-    // W8A16, two workgroups to a CU: slices while they fit and keep 4 k-groups each, 2 below half a chip.  Measured, 32 rows
-    // (us at 4 / 8 / 16 slices): 4096 x 4096 13.9 / 11.4 / 11.4 (64 rows 17.3 / 14.3 / 16.6), 4096 x 14336 34.7 / 24.7 / 21.4,
-    // 6144 x 4096 16.2 / 16.4 / 16.8, 14336 x 4096 22.0 / 25.5 / -
-    // None of 8 k-groups and a quarter of the chip's tiles: 8192 x 1024 9.3 us in two, 8.1 whole, 32768 x 1024 16.6 and 12.0
-    const int t = cdiv(M, CfgF::BM) * cdiv(N, CfgF::BN);
-    if (KG <= 8 && t >= cus / 4) return 1;
-    while (t * s * 2 <= 2 * cus && KG / (2 * s) >= (t * s < cus / 2 ? 2 : 4) && (int64_t)(s * 2) * M * N <= ws_floats) s *= 2;
-    return s;
-  }
   const int pct = g_split_fill_pct > 0 ? g_split_fill_pct : f8 ? 100 : 75;
   const int fill = (int)((int64_t)cus * pct / 100);
   while (tiles * s < fill && s * 2 <= KG && (int64_t)(s * 2) * M * N <= ws_floats) s *= 2;

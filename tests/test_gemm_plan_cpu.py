@@ -52,3 +52,16 @@ def test_a_split_fill_keeps_the_large_tile(E):
     assert E.gemm_plan(0, 1011, 28672, 4096)[0] is False
     E.gemm_set_p8(1)
     assert E.gemm_plan(0, 300, 512, 512)[0] is True and E.gemm_plan(0, 300, 528, 512)[0] is False
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64, 65, 200])
+def test_slices_of_fp8_weights_fit_the_k_groups_and_the_workspace(E, M):
+    """W8A16: the slices come from an estimate; whatever the sizes they leave none empty and fit the workspace."""
+    for N, K in ((16, 128), (4096, 4096), (28672, 4096), (4096, 14336), (2064, 1408), (32768, 1024)):
+        for ws in (0, M * N, 3 * M * N, 1 << 25):
+            large, s = E.gemm_plan(1, M, N, K, f8=2, ws_floats=ws)
+            kg = K // 128
+            assert not large and 1 <= s <= kg and -(-kg // -(-kg // s)) == s
+            assert s == 1 or s * M * N <= ws
+    if M <= 64:  # (one slice covers the chip; four and eight are the measured best)
+        assert [E.gemm_plan(1, M, N, K, f8=2)[1] for N, K in ((28672, 4096), (6144, 4096), (4096, 14336))] == [1, 4, 8]
