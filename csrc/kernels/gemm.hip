@@ -82,8 +82,12 @@ using CfgS = Cfg<128, 128, 2, 2>;
 // carried 8 KB and measured 1.25x slower whole decode steps)
 using CfgF = Cfg<64, 128, 1, 4>;
 // ... of <= 32 rows: bf16 four stages of 20 KB; fp8 24 KB stages, so three fit where two did and two are in flight behind the one
-// being read (with the sum of the slices, 4096 x 4096 14.6 -> 11.4 us, 4096 x 14336 27.9 -> 24.7, 28672 x 4096 35.6 -> 33.1)
+// being read (32 rows: 28672 x 4096 23.3 us, 4096 x 4096 10.1 and 4096 x 14336 17.6 in eight slices with their sum; six stages here and
+// four of 64 rows, one workgroup to a CU: 24.3, 10.7, 19.1, and 3 - 15 % slower over 21 weights)
 using CfgFs = Cfg<32, 128, 1, 4>;
+// ... of few columns as well, in one slice: 64 columns to a tile, so that twice the CUs draw weights (narrow())
+using CfgN = Cfg<64, 64, 1, 4>;
+using CfgNs = Cfg<32, 64, 1, 4>;
 
 // buffer resource over [base, base + bytes): loads past the end return zero (rows >= M, weight
 // tiles >= N), so the stage issue needs no bounds branches
@@ -1124,6 +1128,15 @@ Plan choose(const GemmParams& p, bool parts = false) {
   return r;
 }
 
+// Tiles of 64 columns: a product of <= 64 rows in one slice whose 128-column tiles leave half of the CUs without one: twice as many
+// draw weights, each k-group is over sooner, and a row's sums are the same.  us on 128 / 64 columns, 1, 32 and 48 rows: 9472 x 1024
+// 9.1 / 7.4, 9.5 / 7.5, 11.2 / 9.3, 16384 x 2048 18.7 / 16.0, 19.0 / 15.4, 20.4 / 16.6, 3072 x 512 5.7 / 4.7, 5.8 / 4.8, 7.0 / 5.9;
+// 1.12 - 1.36 times faster on all 17 weights of 1536 .. 16384 columns and K 384 .. 2048, row-major ones 1.18 - 1.59.
+template <int EPI> constexpr bool kNarrow = EPI == EPI_STORE || EPI == EPI_SPLIT;
+bool narrow(const GemmParams& p) {
+  return g_p8_mode == 2 && p.M <= CfgN::BM && p.splits == 1 && p.nbatch <= 1 && 2 * cdiv(p.N, 128) <= p.cus;
+}
+
 // sum false: the slices' partial rows stay in the workspace
 template <int EPI>
 int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
@@ -1155,7 +1168,12 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
   } else if (p.sw) {  // W8A8
     hipLaunchKernelGGL((gemm_kernel<CfgS, EPI, true, true>), dim3(cdiv(p.M, CfgS::BM) * cdiv(p.N, CfgS::BN) * p.splits),
                        dim3(CfgS::THREADS), CfgS::LDS, st, p);
-  } else if (p.M <= CfgFs::BM) {  // (the slices are those of the 128-row tile, and so are the bits)
+  } else if (kNarrow<EPI> && narrow(p)) {
+    if constexpr (kNarrow<EPI>) {
+      if (p.M <= CfgNs::BM) launch_cfg<CfgNs, EPI>(p, st);
+      else launch_cfg<CfgN, EPI>(p, st);
+    }
+  } else if (p.M <= CfgFs::BM) {  // (a row's sums are those of the 128-row tile, and so are the bits)
     launch_cfg<CfgFs, EPI>(p, st);
   } else if (p.M <= CfgF::BM) {
     launch_cfg<CfgF, EPI>(p, st);

@@ -285,8 +285,9 @@ void launch(const GemmF32Params& p, hipStream_t st) {
   const bool fits = (int64_t)64 * p.ldx * 4 < 0x7FFFFFF0ll && (int64_t)64 * p.K * 4 < 0x7FFFFFF0ll;  // (32-bit offsets in a tile)
   // Tiles from where about half the CUs get one (us, rows / tiles kernel): 64 x 8720 x 1024 (137 tiles) 37 / 27, 333 x 1024
   // x 1024 (96) 24 / 23, 128 x 2048 x 2048 (64) 23 / 43.  Waves per tile so that a CU holds 16 of them (1 / 2 / 4 groups):
-  // 777 x 1024 x 6144 (208 tiles) 192 / 149 / 126, 1024 x 2048 x 8192 (512) 389 / 332 / 361, 777 x 32768 x 1024 (6656) 478 /
-  // 512 / 586; the kernel without LDS or k groups that this one replaced: 202 / 507 / 777.  (A 128 x 128 tile: 290 against
+  // 777 x 1024 x 6144 (208 tiles) 133 / 112 / 105, 1024 x 2048 x 8192 (512) 279 / 267 / 276, 777 x 32768 x 1024 (6656) 431 /
+  // 457 / 513; the kernel without LDS or k groups that this one replaced: 202 / 507 / 777.  (Three stages of one k group: 441 and,
+  // 480 x 8192 x 1024, 83 against 74.)  (A 128 x 128 tile: 290 against
   // 307 at 1024 x 8192 x 2048, but 545 against 481 at 777 x 32768 x 1024.)
   if (p.M > 32 && t64 >= 120 && fits) {
     if (t64 <= 256) return launch_tiles<EPI, 4>(p, st);

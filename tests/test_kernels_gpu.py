@@ -1264,6 +1264,31 @@ def test_gemm_few_row_tiles_give_the_bits_of_the_128_row_tile(M, K):
     assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
 
 
+@pytest.mark.parametrize("M", [1, 16, 32, 33, 64])
+@pytest.mark.parametrize("N,n_split,K", [(16, 0, 128), (48, 16, 256), (64, 64, 384), (80, 48, 640), (144, 128, 128), (16384, 8208, 1024)])
+def test_gemm_tiles_of_64_columns(M, N, n_split, K):
+    """<= 64 rows in one slice: column remainders, a split inside a tile, stages of fewer k-groups than buffers, bf16 and f32 results,
+    against f64 (K roundings of at most 2^-24 of the sum of magnitudes; bf16 results rounded once, 2^-8, relu(.)^2 after its square)."""
+    assert ops.ext().gemm_plan(0, M, N, K)[1] == 1
+    x, w = rnd(M, K), rnd(N, K, scale=K ** -0.5)
+    exact = x.double() @ w.double().T
+    err = (x.double().abs() @ w.double().abs().T) * (K + 2) * 2 ** -24
+    for tw in (ops.TiledWeight(w), w):
+        got = ops.gemm(x, tw, torch.full((M, N), 7.0, dtype=BF, device=DEV))
+        assert bool(((got.double() - exact).abs() <= exact.abs() * 2 ** -8 + err).all())
+        got = ops.gemm(x, tw, torch.full((M, N), 7.0, dtype=torch.float32, device=DEV))
+        assert bool(((got.double() - exact).abs() <= err).all())
+    if not 0 < n_split < N or not ops.rows_take_tiles(M, ops.TiledWeight(w)) and M <= ops.SKINNY_MAX_M:
+        return  # (one matrix alone, or rows of the streaming kernel)
+    from voice_enabled_browser_automation_amd.ops import stack
+
+    a, b = torch.empty(M, n_split, dtype=BF, device=DEV), torch.empty(M, N - n_split, dtype=BF, device=DEV)
+    stack.linear_split(x, ops.TiledWeight(w), a, b)
+    assert bool(((a.double() - exact[:, :n_split]).abs() <= exact[:, :n_split].abs() * 2 ** -8 + err[:, :n_split]).all())
+    r, e = exact[:, n_split:].clamp_min(0), err[:, n_split:]
+    assert bool(((b.double() - r * r).abs() <= r * r * 2 ** -7 + 2 * r * e + e * e).all())
+
+
 def test_rows_take_tiles_line():
     """(no launch) a large weight at any row count, smaller ones from 4 and 8 rows on, never one that keeps an order."""
     w = lambda n, k, keep=False: ops.TiledWeight(t=torch.empty(n, k, dtype=torch.bfloat16, device="meta"), keep_order=keep)  # noqa: E731
