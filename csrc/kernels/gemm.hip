@@ -85,7 +85,7 @@ using CfgF = Cfg<64, 128, 1, 4>;
 // being read (32 rows: 28672 x 4096 23.3 us, 4096 x 4096 10.1 and 4096 x 14336 17.6 in eight slices with their sum; six stages here and
 // four of 64 rows, one workgroup to a CU: 24.3, 10.7, 19.1, and 3 - 15 % slower over 21 weights)
 using CfgFs = Cfg<32, 128, 1, 4>;
-// ... of few columns as well, in one slice: 64 columns to a tile, so that twice the CUs draw weights (narrow())
+// ... of few columns as well: 64 columns to a tile, so that twice the CUs draw weights (narrow())
 using CfgN = Cfg<64, 64, 1, 4>;
 using CfgNs = Cfg<32, 64, 1, 4>;
 
@@ -1128,13 +1128,14 @@ Plan choose(const GemmParams& p, bool parts = false) {
   return r;
 }
 
-// Tiles of 64 columns: a product of <= 64 rows in one slice whose 128-column tiles leave half of the CUs without one: twice as many
+// Tiles of 64 columns: a product of <= 64 rows whose 128-column tiles and slices leave half of the CUs without one: twice as many
 // draw weights, each k-group is over sooner, and a row's sums are the same.  us on 128 / 64 columns, 1, 32 and 48 rows: 9472 x 1024
 // 9.1 / 7.4, 9.5 / 7.5, 11.2 / 9.3, 16384 x 2048 18.7 / 16.0, 19.0 / 15.4, 20.4 / 16.6, 3072 x 512 5.7 / 4.7, 5.8 / 4.8, 7.0 / 5.9;
-// 1.12 - 1.36 times faster on all 17 weights of 1536 .. 16384 columns and K 384 .. 2048, row-major ones 1.18 - 1.59.
-template <int EPI> constexpr bool kNarrow = EPI == EPI_STORE || EPI == EPI_SPLIT;
+// 1.12 - 1.36 times faster on all 17 weights of 1536 .. 16384 columns and K 384 .. 2048, row-major ones 1.18 - 1.59.  In slices, with
+// their sum, 16 and 48 rows: 1024 x 4096 8.8 / 8.4, 10.5 / 9.5, 1280 x 1280 7.3 / 6.7, 8.6 / 7.5; 1.03 - 1.17 times on 7 weights.
+template <int EPI> constexpr bool kNarrow = EPI != EPI_SWIGLU && EPI != EPI_GELU_RESID;
 bool narrow(const GemmParams& p) {
-  return g_p8_mode == 2 && p.M <= CfgN::BM && p.splits == 1 && p.nbatch <= 1 && 2 * cdiv(p.N, 128) <= p.cus;
+  return g_p8_mode == 2 && p.M <= CfgN::BM && p.nbatch <= 1 && 2 * cdiv(p.N, 128) * p.splits <= p.cus;
 }
 
 // sum false: the slices' partial rows stay in the workspace
