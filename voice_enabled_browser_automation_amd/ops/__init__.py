@@ -320,7 +320,8 @@ def rows_take_tiles(M: int, w) -> bool:
     """Up to SKINNY_MAX_M rows of a pre-tiled weight are the tiled GEMM's (gemm.hip, its 32-row tile) where it is the faster one:
     a large weight, a smaller one the more rows there are.  The streaming kernel finishes 16 columns at a time (a large weight is
     many rounds of them, the last one rarely full), and every row costs it reads of X beside the weights; the tiled one has four
-    stages of 128 columns in flight, and a sum of slices where its tiles leave the chip idle.  us, streaming / tiled, 1 and 16 rows:
+    stages of 128 columns in flight, and a sum of slices where its tiles leave the chip idle.  us, streaming / tiled
+    (in tiles of 128 columns; those of 64 are up to 1.2 times faster), 1 and 16 rows:
     32768 x 1024 21.3 / 14.6 and 23.8 / 14.4, 17664 x 2048 19.7 / 17.4 and 22.7 / 18.3, 2048 x 12288 15.4 / 16.2 and 23.2 / 15.4,
     4096 x 4096 11.2 / 12.2 and 15.8 / 12.3, 2048 x 2048 6.1 / 7.6 and 8.0 / 8.3.  Over 37 weights and 1, 2, 4, 8, 16 rows this
     line is 0.7 % slower than the better of both (the streaming kernel alone 8.9 %), and nowhere more than 7 % slower than it.
