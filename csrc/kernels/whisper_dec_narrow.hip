@@ -14,8 +14,8 @@
 // d / 4 x 4 B partial rows of 6 (tiny) to 32 (base) producers are 9 - 64 KB a consumer: at d = 768 they would be 147 KB and
 // cost what the hand-offs saved, so wider models keep whisper_dec.hip.
 // Every role keeps its weights of the next layer in registers (<= 32 x 16 B a lane), refilled right after use.
-// Same rounding as whisper_dec.hip (activations bf16, sums f32) but for two places: the cross query is one product of the
-// normed row, and a quarter's attention output is rounded before its weight is known instead of behind the merge.
+// Same rounding as whisper_dec.hip (activations bf16, sums f32) but for two places, both finer: the cross query is one product
+// of the normed row, and the cross-attention's output is not rounded at all (nd_attend: PIECES).
 // Measured, whisper-tiny, 30 keys of context: 137 -> 62 us a token (A 5.0, B 4.4, C 3.4 us a layer, of which the hand-off --
 // arrival to release -- is 0.5 each and a consumer's partial rows 1.0 - 1.4; 8.7 us until the first layer's weights and keys are
 // there, 192 KB a head; the LM head 4 behind the last layer).
@@ -29,7 +29,7 @@ constexpr int kChunks = 4;              // key chunks of a head (WdecParams::nch
 constexpr int kGenWord = 2048;          // (WdecParams::cnt u64 index: launches each workgroup completed)
 constexpr int kLmTiles = 20;            // vocabulary tiles a workgroup has in flight
 constexpr int L_PS = 1024;              // f32 [NG][D] partial sums of a row, <= 8 KB (behind the row, in front of L_RED)
-constexpr int L_AV = L_VA + 512;        // bf16 [64] slice of an activation that meets the next projection
+constexpr int L_AV = L_VA + 512;        // bf16 [3][64] slice of an activation that meets the next projection: its pieces
 constexpr int L_SK = 20480, L_SV = L_SK + 65536;  // self-attention: keys and values [512][64] bf16
 static_assert(L_SV + 65536 <= kLds, "LDS");
 
@@ -223,21 +223,23 @@ VWA_DEVICE void nd_load_k64(const u16* W, int KG, int unit, uint4 (&wr)[R]) {
       wr[O + 2 * t + j] = make_uint4(v.x, v.y, v.z, v.w);
     }
 }
-// ... times the 64 values in LDS -> a partial row
-template <int NS, int O, int R>
+// ... times the 64 values in LDS, each the sum of its PIECES, -> a partial row
+template <int NS, int O, int PIECES = 1, int R>
 VWA_DEVICE void nd_k64(const char* lds, const uint4 (&wr)[R], float* out) {
   const int tx = VWA_TX, lane = tx & 63, g = lane >> 4, w = uni(tx >> 6);
   const u16* av = reinterpret_cast<const u16*>(lds + L_AV);
-  uint4 a[2];
+  uint4 a[PIECES][2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    a[j] = *reinterpret_cast<const uint4*>(av + 32 * (g & 1) + 8 * (2 * j + (g >> 1)));
-  }
+  for (int e = 0; e < PIECES; ++e)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) a[e][j] = *reinterpret_cast<const uint4*>(av + 64 * e + 32 * (g & 1) + 8 * (2 * j + (g >> 1)));
 #pragma unroll
   for (int t = 0; t < NS; ++t) {
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc = mfma16(as_bf16x8(a[j]), as_bf16x8(wr[O + 2 * t + j]), acc);
+    for (int e = PIECES - 1; e >= 0; --e)  // (the small ones first)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc = mfma16(as_bf16x8(a[e][j]), as_bf16x8(wr[O + 2 * t + j]), acc);
     if (lane < 16) stf_sc1(out + (w + 8 * t) * 16 + lane, acc[0]);
   }
 }
@@ -257,13 +259,18 @@ VWA_DEVICE float nd_cols64(char* lds, const uint4 (&wr)[R]) {
 VWA_DEVICE float nd_bias(const u16* b, int n) { return b ? bf2f(gld(b + n)) : 0.f; }
 
 // Attention of the query in LDS (L_QF, bf16) over nk <= 512 keys in LDS, K rows at kl (16-byte piece c of key t at c ^ (t & 7)),
-// V rows at vl; the normalized output goes to L_AV as bf16.  Thread 0 gets (max, sum) of the scores' softmax.
+// V rows at vl; the normalized output goes to L_AV as bf16, or whole: PIECES 3 are its 24 bits in three bf16 numbers, so that what
+// is not finished yet -- a quarter of a head's keys -- stays f32 through the matrix units too (three products where one bf16
+// number a value takes one: no difference in a token's time.  Logits of whisper-tiny against 64 bits, mean of 8 utterances:
+// whisper_dec.hip 5.67e-3, quarters rounded to one bf16 5.61e-3, this 5.56e-3).
+// Thread 0 gets (max, sum) of the scores' softmax.
 // A wave takes tiles of 16 keys on its own -- max, weights, sum and output -- and one round puts the eight together:
 //   scores: K as the MFMA's B operand, 16 keys to a tile, the wave's four tiles then one key a lane (products and sums as exact
 //   as a chain of f32 FMAs: q and K are bf16);
 //   values: 8 keys to a wave instruction, 16 bytes a lane, weights in f32; the lanes' sums halve what they hold at each step
 // What bounds it is the instructions of a wave, two waves to a SIMD.  375 keys: a key per thread, 2 bytes of V a lane and three
 // rounds of the workgroup 3.4 us, scores in every lane (four exponentials a tile) and full sums 2.0, this form 1.4.
+template <int PIECES>
 VWA_DEVICE float2 nd_attend(const WdecParams& p, int nk, const u16* kl, const u16* vl, char* lds) {
   static_assert(kT / 16 / 8 == 4, "a wave's tiles, one to a lane group");
   const int tx = VWA_TX, lane = tx & 63, nl = lane & 15, g = lane >> 4, w = uni(tx >> 6);
@@ -340,7 +347,13 @@ VWA_DEVICE float2 nd_attend(const WdecParams& p, int nk, const u16* kl, const u1
       ml.y += e * lw[k];
       s += e * ow[k * 64 + tx];
     }
-    reinterpret_cast<u16*>(lds + L_AV)[tx] = f2bf(s / ml.y);
+    float left = s / ml.y;
+#pragma unroll
+    for (int e = 0; e < PIECES; ++e) {
+      const u16 b = f2bf(left);
+      reinterpret_cast<u16*>(lds + L_AV)[64 * e + tx] = b;
+      left = (b & 0x7F80) == 0x7F80 ? 0.f : left - bf2f(b);  // (infinities stay what they are)
+    }
   }
   lds_sync();
   return ml;
@@ -431,7 +444,7 @@ VWA_DEVICE void nd_self(const WdecParams& p, int h, unsigned long long gen, char
       if (j >= 4 && new_at >= 0) *gp((j < 8 ? kc : vc) + new_at + dd) = o;
     }
     lds_sync();
-    nd_attend(p, ctx, kl, vl, lds);
+    nd_attend<1>(p, ctx, kl, vl, lds);
     nd_k64<NS, 6 * NS>(lds, wr, p.part + N::PA + h * N::D);
     wd_arrive(p, PH_A);
     if (li + 1 < NL) {
@@ -471,8 +484,8 @@ VWA_DEVICE void nd_cross(const WdecParams& p, int item, unsigned long long gen, 
     if (tx < 64) reinterpret_cast<u16*>(lds + L_QF)[tx] = f2bf((v - st.x * ec) * st.y + eb);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of the K / V chunk
     lds_sync();
-    const float2 ml = nd_attend(p, nk, reinterpret_cast<const u16*>(lds + L_KV), reinterpret_cast<const u16*>(lds + L_KV + L_KVV), lds);
-    nd_k64<NS, 2 * NS>(lds, wr, p.part + N::PB + item * N::D);
+    const float2 ml = nd_attend<3>(p, nk, reinterpret_cast<const u16*>(lds + L_KV), reinterpret_cast<const u16*>(lds + L_KV + L_KVV), lds);
+    nd_k64<NS, 2 * NS, 3>(lds, wr, p.part + N::PB + item * N::D);
     if (tx == 0) {
       stf_sc1(p.part + N::ML + 2 * item, ml.x);
       stf_sc1(p.part + N::ML + 2 * item + 1, ml.y);

@@ -539,6 +539,35 @@ def test_narrow_persistent_decoder_matches_per_kernel_path(ns, T, steps, monkeyp
         assert err < 0.02 * (1 + b.abs().max().item()), (i, err)
 
 
+@pytest.mark.parametrize("ns,T", [(1, 1500), (3, 1500), (4, 1499)])
+def test_narrow_persistent_decoder_keeps_the_quarters_of_the_keys_in_f32(ns, T, monkeypatch):
+    """Equal scores over values of +-3000 whose quarters nearly cancel: what is left (about 15) is a product of the f32 sums, so it
+    shows any rounding of a quarter's output (to bf16: by 8 each).  Against the per-kernel path, which adds f32 partials."""
+    import dataclasses
+
+    from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner
+
+    cfg = dataclasses.replace(get_config("whisper-tiny"), d_model=128 * ns, n_heads=2 * ns, n_enc_layers=1, n_dec_layers=2,
+                              n_audio_ctx=T)
+    m = WhisperModel(cfg, device="cuda", seed=6)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    quarter = -(-T // 4)
+    sign = torch.where(torch.arange(T, device="cuda") // quarter % 2 == 0, 1.0, -1.0)
+    values = [(sign[:, None, None] * (2048 + 16 * torch.randint(0, 127, (T, 2 * ns, 64), device="cuda", generator=gen))).bfloat16()
+              for _ in range(2)]
+    out = []
+    for persist in (False, True):
+        monkeypatch.setenv("VWA_ASR_PERSIST", "1" if persist else "0")
+        r = WhisperRunner(m, max_sessions=1, use_graphs=False)
+        for li in range(2):
+            r.b.cross[li][0].zero_()
+            r.b.cross[li][1][0].copy_(values[li])
+        out.append([r.step([(0, 13 * p, p)]).float().cpu().clone() for p in range(3)])
+    assert not m.chain_error() and next(iter(m._wdec.values()))["part"] is not None
+    for a, b in zip(*out):
+        assert (a - b).abs().max() < 0.02 * (1 + a.abs().max())
+
+
 @pytest.mark.parametrize("model", ["whisper-large-v3", "whisper-tiny"])
 def test_whisper_persistent_device_loop_is_one_launch_and_matches(model, monkeypatch):
     """The device-resident greedy loop (asr/engine.py) with the persistent decoder: each step is ONE
