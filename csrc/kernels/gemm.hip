@@ -1045,7 +1045,7 @@ Plan plan(const GemmParams& p) {
   Plan best{false, 1};
   float least = 0.f;
   for (const int s0 : {1, 2, 3, 4, 6, 8, 12, 16}) {
-    if (s0 > 1 && (s0 > KG || !p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
+    if (s0 > 1 && (s0 > KG || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
     for (const bool p8 : {true, false}) {
       const float us = estimate(p, p8, cdiv(KG, cdiv(KG, s0)));
       if (least == 0.f || us < least) {
@@ -1077,7 +1077,7 @@ int few_slices(const GemmParams& p, bool parts) {
   int best = 1;
   float least = 0.f;
   for (int s0 = 1; s0 <= 32 && s0 <= KG; s0 *= 2) {
-    if (s0 > 1 && (!p.ws || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
+    if (s0 > 1 && (int64_t)s0 * p.M * p.N > p.ws_cap) break;
     const int per = cdiv(KG, s0), s = cdiv(KG, per);
     const float alone = per_kg * per;
     const float sum = parts ? (float)s * p.N * (4 / 4.e4f) : s > 1 ? launch + s * slab : 0.f;
@@ -1095,7 +1095,7 @@ int few_slices(const GemmParams& p, bool parts) {
 int slices_256(const GemmParams& p, bool* fill) {
   const int tiles = cdiv(p.M, 256) * (p.N / 256);
   int s = 1;
-  while (p.ws && tiles * s < p.cus && s * 2 <= p.K / BKG && (int64_t)(s * 2) * p.M * p.N <= p.ws_cap) s *= 2;
+  while (tiles * s < p.cus && s * 2 <= p.K / BKG && (int64_t)(s * 2) * p.M * p.N <= p.ws_cap) s *= 2;
   *fill = tiles >= 256 || (tiles * s >= p.cus && p.K / s >= 2048);
   return s;
 }
@@ -1104,7 +1104,7 @@ bool keeps_order(int epi, const GemmParams& p) {
   return p.keep_order && p.w_tiled && !p.sw && p.nbatch <= 1 && p.cus > 0 && (epi == EPI_STORE || epi == EPI_SWIGLU);
 }
 
-// Tile and slices of a launch (p.splits: those of vwa_gemm_splits)
+// Tile and slices of a launch (p.splits: those of vwa_gemm_splits; p.ws_cap: the f32 numbers that slices may take)
 Plan choose(const GemmParams& p, bool parts = false) {
   Plan r{false, p.splits < 1 ? 1 : p.splits};
   if (p.nbatch > 1 || p.cus <= 0) return r;

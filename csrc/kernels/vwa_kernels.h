@@ -169,7 +169,7 @@ struct GemmParams {
   // X rows may overlap (ldx < K: the Whisper conv stem as an implicit GEMM, row t = the 3 input
   // rows t*stride-1 .. t*stride+1 of a zero-padded channels-last buffer)
   int nbatch; int64_t bsx, bsy, bsr;
-  int cus; int64_t ws_cap;  // CU count and workspace floats (split-K choice of the 256^2 kernel)
+  int cus; int64_t ws_cap;  // CU count and the f32 numbers slices may take (the choice of tile and slices; ws holds what it says)
   // epilogue 5 (QKV): rotary embedding + paged-KV write of a QKV projection with permuted head rows
   // (ops.permute_qkv_rows: each 16-column tile holds the rotation pairs (c, c + 8)) -- q heads go
   // to q_out in natural dim order, k / v heads to the caches at slots[m] (< 0: not written);

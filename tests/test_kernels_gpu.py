@@ -1342,3 +1342,63 @@ def test_few_rows_on_either_kernel(M, N, K, monkeypatch):
             outs[-1].append(got)
     for a, c in zip(*outs):
         assert (a.double() - c.double()).norm() / c.double().norm() < (1e-5 if a.dtype == torch.float32 else 2.0 ** -7)
+
+
+def _sliced_products():
+    """(name, call): one product of every binding that cuts K into slices, at few rows."""
+    torch.manual_seed(3)
+    x = rnd(12, 4096)
+    tw = ops.TiledWeight(rnd(1024, 4096, scale=1 / 64))
+    w8 = ops.FP8Weight.quantize(rnd(1024, 4096, scale=1 / 64))
+    x24 = rnd(24, 4096)
+    bs, D = 16, 128
+    kc, vc = (torch.zeros(4, 2, bs, D, dtype=BF, device=DEV) for _ in range(2))
+    pos = torch.arange(12, dtype=torch.int32, device=DEV)
+    slots = pos.long() + bs
+    rope = ops.rope_table(64, D, 10000.0, device=DEV)
+
+    def qkv():
+        q = torch.empty(12, 4 * D, dtype=BF, device=DEV)
+        ops._gemm_qkv(x, tw, None, False, 1e-5, 4, 2, D, rope, pos, slots, q, kc, vc)
+        return torch.cat([q, kc[1, :, :12].transpose(0, 1).reshape(12, -1), vc[1, :, :12].transpose(0, 1).reshape(12, -1)], 1)
+
+    def split():
+        a, b = torch.empty(12, 512, dtype=BF, device=DEV), torch.empty(12, 512, dtype=BF, device=DEV)
+        ops.ext().gemm(x, tw.t, None, a, 6, None, None, True, ops.GEMM_WS_FLOATS, y2=b)
+        return torch.cat([a, b], 1)
+
+    return [("store", lambda: ops.gemm(x, tw, torch.empty(12, 1024, dtype=BF, device=DEV))), ("qkv", qkv), ("split", split),
+            ("fp8 weights", lambda: ops.gemm_fp8(x24, w8, torch.empty(24, 1024, dtype=BF, device=DEV)))]
+
+
+def test_products_on_two_streams_keep_their_slices_apart():
+    """Products in K slices, eager and out of replayed graphs, on two streams at once: each has the bits it has alone.  (One slice
+    buffer a device was shared by all of them.)"""
+    assert ops.ext().gemm_plan(0, 12, 1024, 4096)[1] > 1 and ops.ext().gemm_plan(0, 24, 1024, 4096, f8=2)[1] > 1
+    calls = _sliced_products()
+    alone = [f().clone() for _, f in calls]
+    streams = [torch.cuda.Stream() for _ in calls]
+    graphs = []
+    for _, f in calls:
+        f()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            outs = [f() for _ in range(8)]
+        graphs.append((g, outs))
+    for _ in range(5):
+        for s, (g, _) in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                g.replay()
+        torch.cuda.synchronize()
+        for (name, _), (_, outs), want in zip(calls, graphs, alone):
+            assert all(torch.equal(o, want) for o in outs), name
+        eager = []
+        for _ in range(4):
+            for s, (_, f) in zip(streams, calls):
+                with torch.cuda.stream(s):
+                    eager.append(f())
+        torch.cuda.synchronize()
+        for i, o in enumerate(eager):
+            assert torch.equal(o, alone[i % len(calls)]), calls[i % len(calls)][0]
+    assert not any(name == "gemm_ws" for _, name, _ in ops._SCRATCH)

@@ -460,7 +460,9 @@ def scratch(device, name: str, numel: int, dtype=torch.float32) -> torch.Tensor:
     return t[:numel]
 
 
-GEMM_WS_FLOATS = 32 << 20  # split-K workspace (128 MB per device: 4 f32 slices of a 1k x 4096 output)
+# Most f32 numbers the K slices of one product take (128 MB: 8 slices of a 1k x 4096 output).  Each call has its own from the
+# caching allocator (csrc/bindings.cpp slices()): one buffer a device was shared by the steps of engines on different streams.
+GEMM_WS_FLOATS = 32 << 20
 # (a one-launch split-K -- the last slice of each tile reducing -- measured no faster at 32 decode
 # rows: the write-through drain + ticket + L2-missing partial loads cost what the reduce launch
 # does, fp8 o / down 26.3 vs 20.2 + 5.2 us, profiles/r4_gemm_one_launch_ab.md; removed.
@@ -492,8 +494,7 @@ def gemm(x: torch.Tensor, w, out: torch.Tensor, *, epi: str = "none", bias: Opti
     rstd = _rstd(x, eps) if fuse_rms and ss_in is None else None
     tiled = isinstance(w, TiledWeight)
     wt = w.t if tiled else w
-    ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
-    E.gemm(x, wt, bias, out, _GEMM_EPI[epi], rstd, residual, tiled, ws, ss_out, ss_zero,
+    E.gemm(x, wt, bias, out, _GEMM_EPI[epi], rstd, residual, tiled, GEMM_WS_FLOATS, ss_out, ss_zero,
            ss_in if fuse_rms else None, eps, keep_order=tiled and w.keep_order)
     return out
 
@@ -533,14 +534,13 @@ def gemm_fp8(x: torch.Tensor, w: "FP8Weight", out: torch.Tensor, *, epi: str = "
     also yields the RMSNorm 1/rms), the fp8 MFMA runs on the tiled fp8 weight.  The scales (and the
     RMSNorm 1/rms of the unquantised x) apply in the epilogue."""
     E = ext()
-    ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
     if x.shape[0] <= FP8_A16_ROWS:
         E.gemm_fp8(x, None, w.w8, w.scale, bias, out, _GEMM_EPI[epi],
-                   _rstd(x, eps) if fuse_rms and ss_in is None else None, residual, ws, ss_out, ss_zero,
+                   _rstd(x, eps) if fuse_rms and ss_in is None else None, residual, GEMM_WS_FLOATS, ss_out, ss_zero,
                    ss_in if fuse_rms else None, eps)
         return out
     x8, sx, rstd = _fp8_input(x, fuse_rms, eps)  # (the quantiser yields the 1/rms: ss_in unused)
-    E.gemm_fp8(x8, sx, w.w8, w.scale, bias, out, _GEMM_EPI[epi], rstd, residual, ws, ss_out, ss_zero)
+    E.gemm_fp8(x8, sx, w.w8, w.scale, bias, out, _GEMM_EPI[epi], rstd, residual, GEMM_WS_FLOATS, ss_out, ss_zero)
     return out
 
 
@@ -760,21 +760,20 @@ def _gemm_qkv(x, w, bias, fuse_rms, eps, n_q_heads, n_kv_heads, head_dim, rope, 
               v_cache, ss_in=None) -> None:
     E = ext()
     M, K = x.shape
-    ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
     common = (n_q_heads, n_kv_heads, head_dim, rope is not None, positions, slots, rope, q_out, k_cache, v_cache)
     if isinstance(w, FP8Weight):
         if M <= FP8_A16_ROWS:  # W8A16 (see gemm_fp8)
             hand = fuse_rms and ss_in is not None
-            E.gemm_qkv(x, None, w.w8, w.scale, bias, _rstd(x, eps) if fuse_rms and not hand else None, True, ws,
+            E.gemm_qkv(x, None, w.w8, w.scale, bias, _rstd(x, eps) if fuse_rms and not hand else None, True, GEMM_WS_FLOATS,
                        *common, ss_in if hand else None, eps)
             return
         x8, sx, rstd = _fp8_input(x, fuse_rms, eps)
-        E.gemm_qkv(x8, sx, w.w8, w.scale, bias, rstd, True, ws, *common)
+        E.gemm_qkv(x8, sx, w.w8, w.scale, bias, rstd, True, GEMM_WS_FLOATS, *common)
         return
     hand = fuse_rms and ss_in is not None
     rstd = _rstd(x, eps) if fuse_rms and not hand else None
     tiled = isinstance(w, TiledWeight)
-    E.gemm_qkv(x, None, w.t if tiled else w, None, bias, rstd, tiled, ws, *common, ss_in if hand else None, eps)
+    E.gemm_qkv(x, None, w.t if tiled else w, None, bias, rstd, tiled, GEMM_WS_FLOATS, *common, ss_in if hand else None, eps)
 
 
 def qkv_rope_write(x: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Tensor], *, fuse_rms: bool, eps: float,

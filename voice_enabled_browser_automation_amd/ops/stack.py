@@ -155,7 +155,7 @@ def embedding_f32(ids: torch.Tensor, table: torch.Tensor, *, out: torch.Tensor, 
 def linear_split(x: torch.Tensor, w, out: torch.Tensor, out2: Optional[torch.Tensor]) -> torch.Tensor:
     """One projection of a normed row for a layer's mixers and its feed-forward: the first out.shape[1]
     columns of x @ w^T to ``out``, relu(.)^2 of the others to ``out2`` (None: there are none)."""
-    from . import SKINNY_MAX_M, TiledWeight, GEMM_WS_FLOATS, gemm_ok, linear, rows_take_tiles, scratch
+    from . import SKINNY_MAX_M, TiledWeight, GEMM_WS_FLOATS, gemm_ok, linear, rows_take_tiles
 
     if out2 is None:
         return linear(x, w, out=out)
@@ -170,7 +170,7 @@ def linear_split(x: torch.Tensor, w, out: torch.Tensor, out2: Optional[torch.Ten
     if x.shape[0] <= SKINNY_MAX_M and tiled and not few:
         _ext().skinny_gemm(x, wt, None, out, 5, False, 0.0, None, None, None, True, y2=out2)
     else:
-        _ext().gemm(x, wt, None, out, 6, None, None, tiled, scratch(x.device, "gemm_ws", GEMM_WS_FLOATS), y2=out2)
+        _ext().gemm(x, wt, None, out, 6, None, None, tiled, GEMM_WS_FLOATS, y2=out2)
     return out
 
 
