@@ -1221,10 +1221,10 @@ extern "C" void vwa_gemm_set_split_fill(int pct) { g_split_fill_pct = pct < 0 ? 
 
 extern "C" void vwa_gemm_set_p8(int mode) { g_p8_mode = mode; }
 
-extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int* large, int* splits) {
+extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int parts, int* large, int* splits) {
   GemmParams p = *pp;
   p.keep_order = keeps_order(epi, p);
-  const Plan pl = choose(p);
+  const Plan pl = choose(p, parts);
   const int per = cdiv(p.K / BKG, pl.splits);
   *large = pl.p8;
   *splits = cdiv(p.K / BKG, per);
@@ -1257,20 +1257,20 @@ int checks_and_plan(int epi, GemmParams& p, bool* p8, bool parts = false) {
 }
 }  // namespace
 
-// Products whose consumer adds the slices up itself, in their order: f32 partial rows [n][M][N] in p.ws, n to *parts (1: the
-// product).  Few rows take many slices (48 x 1024 x 6144: 24 when this was timed), whose sum is a launch of its own and nothing but
+// Products whose consumer adds the slices up itself, in their order: f32 partial rows [parts][M][N] in p.ws, as many as
+// vwa_gemm_plan says (1: the product).  Few rows take many slices (48 x 1024 x 6144: 24 when this was timed), whose sum is a launch of its own and nothing but
 // round trips; the norm that reads its result reads the slices instead: sum 5.1 + norm 3.6 -> 5.8 us, whole steps of 48 rows 2.7 %
 // less.
-extern "C" int vwa_gemm_parts(const GemmParams* pp, int* parts, hipStream_t st) {
+extern "C" int vwa_gemm_parts(const GemmParams* pp, int parts, hipStream_t st) {
   GemmParams p = *pp;
   bool p8 = false;
   p.Y = p.ws;
   p.ldy = p.N;
   p.y_f32 = 1;
-  if (!p.ws || p.bias || p.rstd || p.ss_in || p.sx || p.nbatch > 1 || (int64_t)p.M * p.N > p.ws_cap) return -10;
+  if (!p.ws || p.bias || p.rstd || p.ss_in || p.sx || p.nbatch > 1) return -10;
   const int r = checks_and_plan(EPI_STORE, p, &p8, true);
   if (r) return r;
-  *parts = p.splits;
+  if (p.splits != parts) return -20;  // (ws holds another number of rows)
   return launch_epi<EPI_STORE>(p, st, p8, false);
 }
 

@@ -260,7 +260,7 @@ struct WdecParams {
 extern "C" {
 #endif
 int vwa_skinny_gemm(int epi, const SkinnyParams* p, hipStream_t st);
-int vwa_gemm_parts(const GemmParams* p, int* parts, hipStream_t st);
+int vwa_gemm_parts(const GemmParams* p, int parts, hipStream_t st);
 int vwa_skinny_stream(int epi, const SkinnyParams* p, int grid_cap, int ks, hipStream_t st);
 void vwa_skinny_set_x_skew(int skew);  // LDS-staged X rows: 64-B skew every 4 rows (default) or none (0)
 int vwa_chain_prepare(ChainParams* cp, int grid);
@@ -279,7 +279,8 @@ int vwa_gemm_grouped(int epi, const GemmParams* p, hipStream_t st);
 int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, int f8);
 void vwa_gemm_set_split_fill(int pct);  // split-K while tiles x splits < pct % of the CUs (0: bf16 75, fp8 100)
 void vwa_gemm_set_p8(int mode);  // 0: 128^2 kernel only, 1: 256^2 from 256 rows (bf16: of pre-tiled whole column tiles), 2: by an estimate
-void vwa_gemm_plan(int epi, const GemmParams* p, int* large, int* splits);  // the tile (256^2 or not) and slices that vwa_gemm would take
+// the tile (256^2 or not) and slices that vwa_gemm (parts: vwa_gemm_parts) would take
+void vwa_gemm_plan(int epi, const GemmParams* p, int parts, int* large, int* splits);
 int vwa_row_rstd(const uint16_t* x, int ldx, int M, int K, float eps, float* rstd, hipStream_t st);
 int vwa_rmsnorm(const uint16_t* x, const uint16_t* residual, uint16_t* residual_out, const uint16_t* w,
                 uint16_t* y, int rows, int D, int ldx, float eps, hipStream_t st);

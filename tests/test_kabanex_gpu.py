@@ -656,3 +656,29 @@ def test_norm_adds_a_projections_slices(M, N, K, D):
     n = torch.nn.functional.layer_norm(want, (D,), nw.double(), nb.double(), 1e-5)
     assert rel(out[:, :D], n.cpu()) < 4e-3 and not out[:, D:].any()
     assert (ops.linear_parts(a[:1], ops.TiledWeight(w)) is None) == (N >= 4096)
+
+
+def test_a_projections_slices_are_the_callers():
+    """What linear_parts returned stands, whatever is launched before the norm that reads it: another projection's slices, a sum
+    of slices, both captured behind it."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()  # noqa: E731
+    w, v = ops.TiledWeight(rnd(1024, 4096)), ops.TiledWeight(rnd(1024, 4096))
+    a, b = rnd(20, 4096), rnd(20, 4096)
+    assert ops.ext().gemm_plan(0, 20, 1024, 4096)[1] > 1
+    first = ops.linear_parts(a, w)
+    want = first.clone()
+
+    def others():
+        return ops.linear_parts(b, v), ops.gemm(b, v, torch.empty(20, 1024, device="cuda", dtype=torch.bfloat16))
+
+    second = others()[0]
+    assert torch.equal(first, want) and not torch.equal(second, want)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        kept = ops.linear_parts(a, w)
+        others()
+    for _ in range(3):
+        g.replay()
+        others()
+        assert torch.equal(kept, want)

@@ -123,16 +123,14 @@ PARTS_ROWS = 64
 
 def linear_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
     """x @ w^T as f32 partial rows [parts, rows, N] for layernorm_f32, or None: this call has none (more rows, other weights;
-    the caller takes linear).  They lie in the GEMMs' workspace: the norm is the next launch on the stream."""
-    from . import GEMM_WS_FLOATS, TiledWeight, gemm_ok, rows_take_tiles, scratch
+    the caller takes linear)."""
+    from . import GEMM_WS_FLOATS, TiledWeight, gemm_ok, rows_take_tiles
 
     M, N = x.shape[0], w.shape[0]
     if not x.is_cuda or M > PARTS_ROWS or not isinstance(w, TiledWeight) or w.keep_order or not gemm_ok(x, w) or (
             M < 4 and N >= 4096 and not rows_take_tiles(M, w)):
         return None
-    ws = scratch(x.device, "gemm_ws", GEMM_WS_FLOATS)
-    n = _ext().linear_parts(x, w.t, ws)
-    return ws[: n * M * N].view(n, M, N)
+    return _ext().linear_parts(x, w.t, GEMM_WS_FLOATS)
 
 
 def add_norm(x: torch.Tensor, branch: torch.Tensor, w1: torch.Tensor, w2: Optional[torch.Tensor], *, eps: float,
