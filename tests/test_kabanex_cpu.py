@@ -349,3 +349,17 @@ def test_scratch_of_no_layers():
     """A stack without attention layers still gets its (empty) rows-form scratch."""
     sc = ops.TalkScratch([], 128, "cpu")
     assert sc.s.numel() and sc.stat.numel() and sc.part.numel() and not sc.counters.any()
+
+
+def test_norm_adds_a_projections_slices_on_the_cpu():
+    """layernorm_f32(parts): the partial rows' sum reaches the residual rows and the norm (columns past the norm's stay)."""
+    gen = torch.Generator().manual_seed(3)
+    x, parts = torch.randn(5, 64, generator=gen), torch.randn(3, 5, 48, generator=gen)
+    w, b = torch.randn(42, generator=gen), torch.randn(42, generator=gen)
+    want = x.clone()
+    want[:, :42] += parts.double().sum(0)[:, :42]
+    out = torch.full((5, 64), 7.0)
+    ops.layernorm_f32(x, w, b, eps=1e-5, out=out, parts=parts)
+    assert torch.allclose(x, want, rtol=0, atol=1e-6)  # (three f32 additions of numbers below 8)
+    n = torch.nn.functional.layer_norm(want[:, :42].double(), (42,), w.double(), b.double(), 1e-5)
+    assert torch.allclose(out[:, :42].double(), n, rtol=1e-5, atol=1e-5) and not out[:, 42:].any()

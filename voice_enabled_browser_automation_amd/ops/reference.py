@@ -110,8 +110,10 @@ def layernorm(x, w, b, *, eps=1e-5, residual=None, residual_out=None, out):
 
 
 # ----------------------------------------------------------------------------- layer stacks (ops/stack.py)
-def layernorm_f32(x, w, b, *, eps, out):
+def layernorm_f32(x, w, b, *, eps, out, parts=None):
     D = w.shape[0]
+    if parts is not None:
+        x[:, :D] += parts[:, :, :D].sum(0)
     y = F.layer_norm(x[:, :D].float(), (D,), w.float(), None if b is None else b.float(), eps)
     out.zero_()
     out[:, :D] = y.to(out.dtype)

@@ -108,7 +108,7 @@ def layernorm_f32(x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor], *
     """out = (x - mean) / sqrt(var + eps) * w (+ b) of f32 rows; out may be wider than w (zero columns).
     parts: linear_parts' rows, added to x first."""
     if not x.is_cuda:
-        return ref.layernorm_f32(x, w, b, eps=eps, out=out)
+        return ref.layernorm_f32(x, w, b, eps=eps, out=out, parts=parts)
     _ext().layernorm_f32(x, w, b, out, eps, parts)
     return out
 
