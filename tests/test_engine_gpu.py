@@ -903,3 +903,17 @@ def test_intent_parses_and_transcripts_are_reproducible():
     assert all(torch.equal(enc[0], e) for e in enc[1:])
     toks = [asr.decode_many([audio], exact_tokens=24)[0] for _ in range(2)]
     assert toks[0] == toks[1]
+
+
+@pytest.mark.parametrize("M", [4, 16, 17])
+def test_every_forward_has_its_own_row_statistics(M):
+    """The sums of squares that the GEMMs of a forward hand on (5 .. 16 rows of large weights among them) are no other forward's:
+    engines of one model may step on two streams."""
+    from types import SimpleNamespace
+
+    w = lambda n, k: ops.TiledWeight(t=torch.empty(n, k, dtype=torch.bfloat16, device="meta"))  # noqa: E731
+    model = SimpleNamespace(layers=[SimpleNamespace(qkv=w(6144, 4096), o=w(4096, 4096), gu=w(28672, 4096), down=w(4096, 14336))],
+                            device=torch.device("cuda"), tp=SimpleNamespace(size=1))
+    one, two = LlamaModel._rms_stats(model, M), LlamaModel._rms_stats(model, M)
+    assert len({t.data_ptr() for t in one + two}) == 4 and not any(t.any() for t in one + two)
+    assert all(t.numel() == M and t.is_contiguous() for t in one + two)

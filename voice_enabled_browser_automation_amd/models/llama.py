@@ -208,17 +208,12 @@ class LlamaModel:
         whose row-parallel outputs are partial sums until the all-reduce)."""
         L = self.layers[0]
         few = M <= ops.SKINNY_MAX_M and not all(ops.rows_take_tiles(M, w) for w in (L.qkv, L.o, L.gu, L.down))
-        if few or self.device.type != "cuda" or self.tp.size > 1 or not ops.env_flag("VWA_RMS_HANDOFF"):
+        if few or M > 4096 or self.device.type != "cuda" or self.tp.size > 1 or not ops.env_flag("VWA_RMS_HANDOFF"):
             return None
-        if getattr(self, "_ss", None) is None:
-            # (int64: u64 fixed-point sums, ops.SS_SCALE -- integer atomics keep them reproducible)
-            self._ss = torch.zeros(2, 4096, dtype=torch.int64, device=self.device)
-        if M > self._ss.shape[1]:
-            return None
-        # (the residual GEMMs keep ss[0] zero between forwards; cleared here too, so an interrupted
-        # forward cannot leave partial sums behind)
-        self._ss[0].zero_()
-        return self._ss[0], self._ss[1]
+        # (int64: u64 fixed-point sums, ops.SS_SCALE -- integer atomics keep them reproducible.  The forward's own: two engines of
+        # one model may step on two streams)
+        ss = torch.zeros(2, M, dtype=torch.int64, device=self.device)
+        return ss[0], ss[1]
 
     def _row_parallel(self, x: torch.Tensor, w: torch.Tensor, h: torch.Tensor, ss=None):
         """h <- h + x @ w^T summed over TP ranks (one all-reduce, residual folded into rank 0).
@@ -410,7 +405,7 @@ class LlamaModel:
             pf_sid = torch.full((M,), prefill_seq, **i32)
             pf_slices = [(i, min(M, i + 64)) for i in range(0, M, 64)]
             pf_out = torch.empty((M, self.nq * self.hd), dtype=self.dtype, device=self.device)
-        # > 16 rows on one rank (the tiled GEMMs): each residual GEMM hands the sums of squares of the
+        # rows of the tiled GEMMs on one rank: each residual GEMM hands the sums of squares of the
         # rows it writes to the next RMSNorm (ss[0]: after o_proj -> gate/up, ss[1]: after down ->
         # next QKV) and zeroes the other buffer, so no row_rstd launch (GemmParams::ss_*)
         ss = self._rms_stats(M) if not chain else None
