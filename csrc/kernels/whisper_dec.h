@@ -118,6 +118,14 @@ VWA_DEVICE void wd_arrive(const WdecParams& p, int lvl) {
     __hip_atomic_fetch_add(gp(lvl_cnt(p, lvl) + 16 * (blockIdx.x & 7)), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// diagnostic stamp k of (layer, level) (tools/wdec_probe.py): 0 entry, 1 released, 2 row staged
+// (attention levels of whisper_dec.hip: softmax done), 3 completed
+VWA_DEVICE void wd_stamp(const WdecParams& p, int li, int lvl, int k) {
+  if (p.ts && VWA_TX == 0)
+    *gp(p.ts + ((size_t)blockIdx.x * p.n_layers * kWdLevels + (size_t)li * kWdLevels + lvl) * 4 + k) =
+        __builtin_amdgcn_s_memrealtime();
+}
+
 // cross-attention K / V chunk of layer li (this workgroup's item) -> LDS by LDS-DMA (no registers;
 // completes on vmcnt: the level waits for it)
 VWA_DEVICE void wd_kv_prefetch(const WdecParams& p, int li, int item, char* lds) {

@@ -84,14 +84,6 @@ VWA_DEVICE void wd_wait_head(const WdecParams& p, int h, unsigned long long targ
   lds_sync();
 }
 
-// diagnostic stamp k of (layer, level) (tools/wdec_probe.py): 0 entry, 1 released, 2 row staged
-// (attention levels: softmax done), 3 completed
-VWA_DEVICE void wd_stamp(const WdecParams& p, int li, int lvl, int k) {
-  if (p.ts && VWA_TX == 0)
-    *gp(p.ts + ((size_t)blockIdx.x * p.n_layers * kWdLevels + (size_t)li * kWdLevels + lvl) * 4 + k) =
-        __builtin_amdgcn_s_memrealtime();
-}
-
 VWA_DEVICE int n_cols(const WdecParams& p, int gm) {
   return gm == G_QKV ? 3 * p.d : gm == G_FC1 ? p.ffn : p.d;
 }

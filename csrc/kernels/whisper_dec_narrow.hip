@@ -46,6 +46,12 @@ struct Nd {
 
 VWA_DEVICE float bits_f(unsigned v) { return __uint_as_float(v); }
 
+// (a kernel of its own stamps: 48 tests for null were 0.6 us of a token's 62)
+template <bool TS>
+VWA_DEVICE void nd_stamp(const WdecParams& p, int li, int phase, int k) {
+  if constexpr (TS) wd_stamp(p, li, phase, k);
+}
+
 // the finished row (4 columns o of thread tx < C4) -> LDS, and to `keep`; returns (mean, 1 / std) to every thread
 template <int NS>
 VWA_DEVICE float2 nd_row(const WdecParams& p, const float (&o)[4], char* lds, u16* keep) {
@@ -261,7 +267,7 @@ VWA_DEVICE float nd_bias(const u16* b, int n) { return b ? bf2f(gld(b + n)) : 0.
 // Attention of the query in LDS (L_QF, bf16) over nk <= 512 keys in LDS, K rows at kl (16-byte piece c of key t at c ^ (t & 7)),
 // V rows at vl; the normalized output goes to L_AV as bf16, or whole: PIECES 3 are its 24 bits in three bf16 numbers, so that what
 // is not finished yet -- a quarter of a head's keys -- stays f32 through the matrix units too (three products where one bf16
-// number a value takes one: no difference in a token's time.  Logits of whisper-tiny against 64 bits, mean of 8 utterances:
+// number a value takes one: 0.8 us of a token's 62.  Logits of whisper-tiny against 64 bits, mean of 8 utterances:
 // whisper_dec.hip 5.67e-3, quarters rounded to one bf16 5.61e-3, this 5.56e-3).
 // Thread 0 gets (max, sum) of the scores' softmax.
 // A wave takes tiles of 16 keys on its own -- max, weights, sum and output -- and one round puts the eight together:
@@ -360,7 +366,7 @@ VWA_DEVICE float2 nd_attend(const WdecParams& p, int nk, const u16* kl, const u1
 }
 
 // A: self-attention of head h and its part of the out-projection
-template <int NS>
+template <int NS, bool TS>
 VWA_DEVICE void nd_self(const WdecParams& p, int h, unsigned long long gen, char* lds) {
   using N = Nd<NS>;
   constexpr int NW = 8 * NS;
@@ -406,12 +412,16 @@ VWA_DEVICE void nd_self(const WdecParams& p, int h, unsigned long long gen, char
     const u32x2 bb = nd_bias4<NS>(li ? p.layers[li - 1].g[G_FC2].bias : nullptr);
     float2 st;
     u16* keep = h == 0 ? row : nullptr;
+    nd_stamp<TS>(p, li, PH_A, 0);
     if (li == 0) {
+      nd_stamp<TS>(p, li, PH_A, 1);
       st = nd_row<NS>(p, x, lds, keep);
     } else {
       wd_wait(p, PH_C, (gen * NL + li) * N::NI);
+      nd_stamp<TS>(p, li, PH_A, 1);
       st = nd_stage<NS, N::NI, false>(p, p.part + N::PC, row + 2 * N::D, bb, lds, keep);
     }
+    nd_stamp<TS>(p, li, PH_A, 2);
     // q, k, v of the head: 12 tiles over 8 waves -- one and a half a wave, three chains of half a tile
     float* red = reinterpret_cast<float*>(lds + L_RED);
     {
@@ -447,6 +457,7 @@ VWA_DEVICE void nd_self(const WdecParams& p, int h, unsigned long long gen, char
     nd_attend<1>(p, ctx, kl, vl, lds);
     nd_k64<NS, 6 * NS>(lds, wr, p.part + N::PA + h * N::D);
     wd_arrive(p, PH_A);
+    nd_stamp<TS>(p, li, PH_A, 3);
     if (li + 1 < NL) {
       load_qkv(li + 1);
       load_o(li + 1);
@@ -455,7 +466,7 @@ VWA_DEVICE void nd_self(const WdecParams& p, int h, unsigned long long gen, char
 }
 
 // B: cross-attention of (head, key chunk) and its part of the out-projection
-template <int NS>
+template <int NS, bool TS>
 VWA_DEVICE void nd_cross(const WdecParams& p, int item, unsigned long long gen, char* lds) {
   using N = Nd<NS>;
   constexpr int NW = 4 * NS;
@@ -478,8 +489,11 @@ VWA_DEVICE void nd_cross(const WdecParams& p, int item, unsigned long long gen, 
       ec = gld(L.g[G_XQ].ln_c + 64 * h + tx);
     }
     const u32x2 bb = nd_bias4<NS>(L.g[G_O].bias);
+    nd_stamp<TS>(p, li, PH_B, 0);
     wd_wait(p, PH_A, (gen * NL + li + 1) * N::H);
+    nd_stamp<TS>(p, li, PH_B, 1);
     const float2 st = nd_stage<NS, N::H, false>(p, p.part + N::PA, row, bb, lds, item == 0 ? row + N::D : nullptr);
+    nd_stamp<TS>(p, li, PH_B, 2);
     const float v = nd_cols64<NS, 0>(lds, wr);
     if (tx < 64) reinterpret_cast<u16*>(lds + L_QF)[tx] = f2bf((v - st.x * ec) * st.y + eb);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's share of the K / V chunk
@@ -491,12 +505,13 @@ VWA_DEVICE void nd_cross(const WdecParams& p, int item, unsigned long long gen, 
       stf_sc1(p.part + N::ML + 2 * item + 1, ml.y);
     }
     wd_arrive(p, PH_B);
+    nd_stamp<TS>(p, li, PH_B, 3);
     if (li + 1 < NL) load(li + 1);
   }
 }
 
 // C: 64 hidden units of the feed-forward
-template <int NS>
+template <int NS, bool TS>
 VWA_DEVICE void nd_ff(const WdecParams& p, int unit, unsigned long long gen, char* lds) {
   using N = Nd<NS>;
   constexpr int NW = 4 * NS;
@@ -518,13 +533,17 @@ VWA_DEVICE void nd_ff(const WdecParams& p, int unit, unsigned long long gen, cha
       ec = gld(L.g[G_FC1].ln_c + 64 * unit + tx);
     }
     const u32x2 bb = nd_bias4<NS>(L.g[G_XO].bias);
+    nd_stamp<TS>(p, li, PH_C, 0);
     wd_wait(p, PH_B, (gen * NL + li + 1) * N::NI);
+    nd_stamp<TS>(p, li, PH_C, 1);
     const float2 st = nd_stage<NS, N::NI, true>(p, p.part + N::PB, row + N::D, bb, lds, unit == 0 ? row + 2 * N::D : nullptr);
+    nd_stamp<TS>(p, li, PH_C, 2);
     const float v = nd_cols64<NS, 0>(lds, wr);
     if (tx < 64) reinterpret_cast<u16*>(lds + L_AV)[tx] = f2bf(gelu_erf((v - st.x * ec) * st.y + eb));
     lds_sync();
     nd_k64<NS, 2 * NS>(lds, wr, p.part + N::PC + unit * N::D);
     wd_arrive(p, PH_C);
+    nd_stamp<TS>(p, li, PH_C, 3);
     if (li + 1 < NL) load(li + 1);
   }
 }
@@ -662,7 +681,7 @@ VWA_DEVICE void nd_head(const WdecParams& p, int m, int n, unsigned long long ge
   if (p.smp_mask) nd_sample_part(p, m, lds, bv, bi);
 }
 
-template <int NS>
+template <int NS, bool TS>
 __global__ __launch_bounds__(kT) void wdec_narrow_kernel(WdecParams p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   using N = Nd<NS>;
@@ -673,9 +692,9 @@ __global__ __launch_bounds__(kT) void wdec_narrow_kernel(WdecParams p) {
                                  ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(g0 >> 32)) << 32);
   // (the sampler's arrivals need every level, and so this read)
   const unsigned long long smp = p.smp_mask && b == 0 && VWA_TX < 64 ? cnt_sum8(p.cnt + kSmpCnt) : 0;
-  if (b < N::H) nd_self<NS>(p, b, gen, lds);
-  else if (b < N::H + N::NI) nd_cross<NS>(p, b - N::H, gen, lds);
-  else if (b < N::ROLES) nd_ff<NS>(p, b - N::H - N::NI, gen, lds);
+  if (b < N::H) nd_self<NS, TS>(p, b, gen, lds);
+  else if (b < N::H + N::NI) nd_cross<NS, TS>(p, b - N::H, gen, lds);
+  else if (b < N::ROLES) nd_ff<NS, TS>(p, b - N::H - N::NI, gen, lds);
   else if (p.lm_W) nd_head<NS>(p, b - N::ROLES, n, gen, lds);
   if (p.smp_mask && b == 0) nd_sample_merge(p, n, smp);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -685,7 +704,8 @@ __global__ __launch_bounds__(kT) void wdec_narrow_kernel(WdecParams p) {
 template <int NS>
 int nd_launch(const WdecParams& p, int grid, hipStream_t st) {
   if (grid < Nd<NS>::ROLES + 16) return -10;
-  hipLaunchKernelGGL(wdec_narrow_kernel<NS>, dim3(grid), dim3(kT), kLds, st, p);
+  if (p.ts) hipLaunchKernelGGL((wdec_narrow_kernel<NS, true>), dim3(grid), dim3(kT), kLds, st, p);
+  else hipLaunchKernelGGL((wdec_narrow_kernel<NS, false>), dim3(grid), dim3(kT), kLds, st, p);
   return (int)hipGetLastError();
 }
 

@@ -917,3 +917,39 @@ def test_every_forward_has_its_own_row_statistics(M):
     one, two = LlamaModel._rms_stats(model, M), LlamaModel._rms_stats(model, M)
     assert len({t.data_ptr() for t in one + two}) == 4 and not any(t.any() for t in one + two)
     assert all(t.numel() == M and t.is_contiguous() for t in one + two)
+
+
+@pytest.mark.parametrize("opt", [0, 1])
+def test_narrow_persistent_decoder_stamps_its_levels(opt, monkeypatch):
+    """The diagnostic stamps come in order from every workgroup of a level, and a schedule option runs the kernel that has it
+    (whisper_dec.hip), with the same logits."""
+    import dataclasses
+
+    from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner
+    from voice_enabled_browser_automation_amd.models.whisper import WDEC_LEVELS, WDEC_NARROW_LEVELS
+
+    cfg = dataclasses.replace(get_config("whisper-tiny"), n_enc_layers=1, n_dec_layers=3)
+    m = WhisperModel(cfg, device="cuda", seed=6)
+    enc = torch.randn(1, cfg.n_audio_ctx, cfg.d_model, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)).bfloat16()
+    out = []
+    for persist in ("0", "1"):
+        monkeypatch.setenv("VWA_ASR_PERSIST", persist)
+        monkeypatch.setenv("VWA_WDEC_OPT", str(opt) if persist == "1" else "0")
+        r = WhisperRunner(m, max_sessions=1, use_graphs=False)
+        r.set_cross(0, enc)
+        r.step([(0, 5, 0)])
+        if persist == "1":
+            st = next(iter(m._wdec.values()))
+            assert (st["part"] is None) == bool(opt)
+            ts = st["ts"] = torch.zeros(st["ints"][10] * 3 * 8 * 4, dtype=torch.int64, device="cuda")
+        out.append(r.step([(0, 7, 1)]).float().clone())
+    torch.cuda.synchronize()
+    assert not m.chain_error() and (out[0] - out[1]).abs().max() < 0.02 * (1 + out[0].abs().max())
+    ts = ts.view(-1, 3, 8, 4).cpu()
+    H = cfg.n_heads
+    of = (ts[..., 3] > 0).sum(0)  # workgroups that finished [layer][level]
+    assert (of[:, : len(WDEC_LEVELS if opt else WDEC_NARROW_LEVELS)] > 0).all()
+    if not opt:
+        assert of[:, :3].tolist() == [[H, 4 * H, 4 * H]] * 3 and not ts[:, :, 3:].any()
+        done = ts[ts[..., 3] > 0]
+        assert (done[:, 1:] >= done[:, :-1]).all()

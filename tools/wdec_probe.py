@@ -1,5 +1,5 @@
-"""Per-level timing of the persistent Whisper decoder (csrc/kernels/whisper_dec.hip) from its
-s_memrealtime stamps (WdecParams::ts, 100 MHz): for every level of every layer, across the
+"""Per-level timing of the persistent Whisper decoder (csrc/kernels/whisper_dec.hip; models of d <= 512, and no --opt or
+--role-opts: whisper_dec_narrow.hip, whose levels are self, cross and ff) from its s_memrealtime stamps (WdecParams::ts, 100 MHz): for every level of every layer, across the
 workgroups that run it --
 
   hand-off   the level's first release (stamp 1) minus the previous level's LAST completion (stamp 3)
@@ -27,7 +27,7 @@ sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from voice_enabled_browser_automation_amd import ops  # noqa: E402
 from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner  # noqa: E402
 from voice_enabled_browser_automation_amd.models.config import get_config  # noqa: E402
-from voice_enabled_browser_automation_amd.models.whisper import WDEC_LEVELS, WhisperModel  # noqa: E402
+from voice_enabled_browser_automation_amd.models.whisper import WDEC_LEVELS, WDEC_NARROW_LEVELS, WhisperModel  # noqa: E402
 
 
 def main():
@@ -41,6 +41,7 @@ def main():
     a = ap.parse_args()
     ops.ext()
     os.environ["VWA_ASR_PERSIST"] = "1"
+    os.environ["VWA_WDEC_OPT"] = str(a.opt)
     from voice_enabled_browser_automation_amd.models import whisper as W
     for kv in filter(None, a.role_opts.split(",")):
         k, v = kv.split("=")
@@ -56,7 +57,7 @@ def main():
     r.step([(0, 5, 0)])
     st = next(iter(m._wdec.values()))
     grid, L = st["ints"][10], a.layers
-    st["opt"] = a.opt
+    levels = WDEC_NARROW_LEVELS if st["part"] is not None else WDEC_LEVELS
     # timing without stamps first (graph replays of one position: the launch's work is the same)
     for _ in range(3):
         r.step([(0, 7, 1)])
@@ -77,13 +78,13 @@ def main():
         torch.cuda.synchronize()
         rows.append(ts.view(grid, L, 8, 4).cpu())
     err = m.chain_error()
-    res = {lv: dict(handoff=[], stage=[], body=[], span=[]) for lv in WDEC_LEVELS}
-    late = {lv: {} for lv in WDEC_LEVELS}  # workgroup -> completion minus the level's median, per layer
+    res = {lv: dict(handoff=[], stage=[], body=[], span=[]) for lv in levels}
+    late = {lv: {} for lv in levels}  # workgroup -> completion minus the level's median, per layer
     for t in rows:
         t = t.double() / 100.0  # 100 MHz -> us
         done_prev = None
         for li in range(L):
-            for lvl, name in enumerate(WDEC_LEVELS):
+            for lvl, name in enumerate(levels):
                 s = t[:, li, lvl]
                 act = s[:, 3] > 0
                 if not act.any():
@@ -110,8 +111,8 @@ def main():
                per_layer_us=round(step_us / L, 2), error=bool(err))
     for name, d in res.items():
         out[name] = {k: round(statistics.median(v), 2) for k, v in d.items() if v}
-    out["layer_span_us"] = round(sum(out[n].get("span", 0) for n in WDEC_LEVELS if n != "xq_x"), 2)
-    for name in WDEC_LEVELS:  # the workgroups that finish a level latest (median lateness, us)
+    out["layer_span_us"] = round(sum(out[n].get("span", 0) for n in levels if n != "xq_x"), 2)
+    for name in levels:  # the workgroups that finish a level latest (median lateness, us)
         lw = sorted(((statistics.median(v), wg) for wg, v in late[name].items()), reverse=True)[:4]
         out[name]["late"] = [[wg, round(v, 2)] for v, wg in lw]
     print(json.dumps(out), flush=True)

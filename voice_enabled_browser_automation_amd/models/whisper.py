@@ -28,6 +28,7 @@ from .llama import move_model  # noqa: F401  (re-export)
 
 
 WDEC_LEVELS = ("qkv", "xq_x", "self_attn", "o_xq", "cross_attn", "xo", "fc1", "fc2")
+WDEC_NARROW_LEVELS = ("self", "cross", "ff")  # (whisper_dec_narrow.hip)
 # gemm ids of the persistent decoder (whisper_dec.hip G_*; WdecLayer::g order) and their levels
 WDEC_GEMMS = ("qkv", "o", "xq", "xo", "fc1", "fc2", "xq_o")
 WDEC_GEMM_LEVEL = (0, 3, 1, 5, 6, 7, 3)
@@ -515,9 +516,9 @@ class WhisperModel:
         nch = 4
         T = bufs.cross[0][0].shape[1]
         # narrow models (d <= 512): three hand-offs a layer (whisper_dec_narrow.hip), one workgroup per head, per (head, key
-        # chunk) and per 64 hidden units, the LM head on the others
-        part = E.wdec_narrow_part(cfg.d_model)
-        narrow = part > 0 and grid >= 9 * self.H + 16 and 3 * -(-T // 4) < T <= 4 * 384
+        # chunk) and per 64 hidden units, the LM head on the others.  A schedule or role option asks for whisper_dec.hip.
+        part, opt = E.wdec_narrow_part(cfg.d_model), ops.env_int("VWA_WDEC_OPT")
+        narrow = part > 0 and grid >= 9 * self.H + 16 and 3 * -(-T // 4) < T <= 4 * 384 and not opt and not WDEC_ROLE_OPTS
         roles, n_prod = None, []
         try:
             if not narrow:
@@ -552,6 +553,8 @@ class WhisperModel:
                   keep=keep, lm_w=w_lm,
                   ints=[len(self.dec), cfg.d_model, self.H, cfg.ffn, T, bufs.k_cache.shape[3],
                         bufs.block_table.shape[1], nch, -(-T // nch), bufs.cross[0][0].shape[0], grid])
+        if narrow:
+            st["opt"] = 0
         self._wdec[bufs] = st
         return st
 
