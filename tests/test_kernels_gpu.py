@@ -1290,12 +1290,12 @@ def test_gemm_tiles_of_64_columns(M, N, n_split, K):
 
 
 def test_rows_take_tiles_line():
-    """(no launch) a large weight at any row count, smaller ones from 4 and 8 rows on, never one that keeps an order."""
+    """(no launch) a large weight whatever the rows, never one that keeps an order: up to 16 rows the weight alone decides."""
     w = lambda n, k, keep=False: ops.TiledWeight(t=torch.empty(n, k, dtype=torch.bfloat16, device="meta"), keep_order=keep)  # noqa: E731
     assert [ops.rows_take_tiles(m, w(17664, 2048)) for m in (1, 3, 4, 16)] == [True] * 4
-    assert [ops.rows_take_tiles(m, w(2048, 12288)) for m in (1, 3, 4, 7, 8)] == [False, False, True, True, True]
-    assert [ops.rows_take_tiles(m, w(2048, 4096)) for m in (1, 4, 7, 8, 16)] == [False, False, False, True, True]
-    assert [ops.rows_take_tiles(m, w(9472, 1024)) for m in (1, 16)] == [True, True] and not ops.rows_take_tiles(16, w(8192, 512))
+    for n, k, tiles in ((17664, 2048, True), (2048, 12288, True), (2048, 4096, True), (9472, 1024, True), (3072, 2048, False),
+                        (3840, 1280, False), (8192, 512, False)):
+        assert {ops.rows_take_tiles(m, w(n, k)) for m in range(1, 17)} == {tiles}, (n, k)
     assert not ops.rows_take_tiles(16, w(32768, 4096, True)) and not ops.rows_take_tiles(16, torch.empty(32768, 4096, device="meta"))
 
 
@@ -1430,3 +1430,30 @@ def test_a_rows_sums_do_not_depend_on_the_rows_beside_it(N, K):
     for M in (1, 4, 8, 16, 17, 31, 32, 33, 48, 63):
         for i, (a, b) in enumerate(zip(forms(M), whole)):
             assert torch.equal(a, b[:M]), (M, i)
+
+
+@pytest.mark.parametrize("N,K", [(2048, 4096), (8208, 896), (4096, 4096), (3072, 2048), (1024, 1024)])
+def test_up_to_16_rows_take_one_kernel(N, K):
+    """A pre-tiled weight's products of 1 .. 16 rows: the bits of a row are those it has in a call of 16, on whichever kernel the
+    weight's products run."""
+    x, r, b = rnd(16, K), rnd(16, N), rnd(N)
+    x32 = torch.randn(16, N, device=DEV)
+    tw = ops.TiledWeight(rnd(N, K, scale=K ** -0.5))
+
+    def forms(M):
+        yield ops.linear(x[:M], tw, b)
+        yield ops.linear(x[:M], tw, b, act="gelu")
+        yield ops.linear(x[:M], tw, b, residual=r[:M])
+        yield ops.linear(x[:M], tw, out_dtype=torch.float32)
+        y = x32[:M].clone()
+        yield ops.linear(x[:M], tw, out=y, residual=y)
+        y, y2 = torch.empty(M, 512, dtype=BF, device=DEV), torch.empty(M, N - 512, dtype=BF, device=DEV)
+        ops.linear_split(x[:M], tw, y, y2)
+        yield torch.cat([y, y2], 1)
+        if N % 32 == 0:
+            yield ops.linear_swiglu(x[:M], tw)
+
+    whole = list(forms(16))
+    for M in (1, 2, 3, 4, 5, 7, 8, 12, 15):
+        for i, (got, want) in enumerate(zip(forms(M), whole)):
+            assert torch.equal(got, want[:M]), (M, i)

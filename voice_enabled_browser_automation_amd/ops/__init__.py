@@ -317,19 +317,19 @@ def _stream_ok(x: torch.Tensor, w) -> bool:
 
 
 def rows_take_tiles(M: int, w) -> bool:
-    """Up to SKINNY_MAX_M rows of a pre-tiled weight are the tiled GEMM's (gemm.hip, its 32-row tile) where it is the faster one:
-    a large weight, a smaller one the more rows there are.  The streaming kernel finishes 16 columns at a time (a large weight is
-    many rounds of them, the last one rarely full), and every row costs it reads of X beside the weights; the tiled one has four
-    stages of 128 columns in flight, and a sum of slices where its tiles leave the chip idle.  us, streaming / tiled
-    (in tiles of 128 columns; those of 64 are up to 1.2 times faster), 1 and 16 rows:
-    32768 x 1024 21.3 / 14.6 and 23.8 / 14.4, 17664 x 2048 19.7 / 17.4 and 22.7 / 18.3, 2048 x 12288 15.4 / 16.2 and 23.2 / 15.4,
-    4096 x 4096 11.2 / 12.2 and 15.8 / 12.3, 2048 x 2048 6.1 / 7.6 and 8.0 / 8.3.  Over 37 weights and 1, 2, 4, 8, 16 rows this
-    line is 0.7 % slower than the better of both (the streaming kernel alone 8.9 %), and nowhere more than 7 % slower than it.
-    Weights that keep one order of their sums stay with the one kernel."""
-    if not isinstance(w, TiledWeight) or w.keep_order:
+    """Whether M rows of a pre-tiled weight are the tiled GEMM's (gemm.hip): more than SKINNY_MAX_M, or of a large weight.  The
+    streaming kernel finishes 16 columns at a time (a large weight is many rounds of them, the last one rarely full), and every row
+    costs it reads of X beside the weights; the tiled one has four stages of 64 or 128 columns in flight, and a sum of slices where
+    its tiles leave the chip idle.  The weight alone decides, so that a row's sums are the same whatever rows come with it.  us, streaming /
+    tiled, 1 and 16 rows: 32768 x 1024 21.6 / 14.7 and 23.9 / 14.3, 17664 x 2048 19.9 / 19.1 and 23.0 / 18.4, 2048 x 12288
+    16.4 / 15.0 and 23.1 / 15.2, 4096 x 4096 11.1 / 11.6 and 15.3 / 12.4, 6144 x 4096 15.1 / 14.7 and 19.0 / 15.0; below the line
+    3072 x 2048 7.4 / 8.7 and 9.3 / 9.0, 3840 x 1280 6.5 / 8.1 and 8.4 / 8.5.  Over the 35 weights of 38 that this line gives
+    the tiles, at 1, 2, 3, 4, 6, 8, 12 and 16 rows they take 0.46 - 1.04 of the streaming kernel's time (0.80 in the mean), but for
+    one row of 4096 x 8192 (1.07).  Weights that keep one order of their sums stay with the one kernel."""
+    if not isinstance(w, TiledWeight):
         return False
     N, K = w.shape
-    return (K <= 1024 and N > 8192) or 2 * N * K >= (70e6 if M < 4 else 25e6 if M < 8 else 12e6)
+    return M > SKINNY_MAX_M or not w.keep_order and ((K <= 1024 and N > 8192) or 2 * N * K >= 13e6)
 
 
 def plain(w):
