@@ -1136,8 +1136,8 @@ Plan choose(const GemmParams& p, bool parts = false) {
 // 9.1 / 7.4, 9.5 / 7.5, 11.2 / 9.3, 16384 x 2048 18.7 / 16.0, 19.0 / 15.4, 20.4 / 16.6, 3072 x 512 5.7 / 4.7, 5.8 / 4.8, 7.0 / 5.9;
 // 1.12 - 1.36 times faster on all 17 weights of 1536 .. 16384 columns and K 384 .. 2048, row-major ones 1.18 - 1.59.  In slices, with
 // their sum, 16 and 48 rows: 1024 x 4096 8.8 / 8.4, 10.5 / 9.5, 1280 x 1280 7.3 / 6.7, 8.6 / 7.5; 1.03 - 1.17 times on 7 weights.
-template <int EPI> constexpr bool kNarrow = EPI != EPI_SWIGLU && EPI != EPI_GELU_RESID;
-bool narrow(const GemmParams& p) {
+constexpr bool takes_narrow(int epi) { return epi != EPI_SWIGLU && epi != EPI_GELU_RESID; }
+bool narrow(const GemmParams& p) {  // (bf16 weights that keep no order)
   return g_p8_mode == 2 && p.M <= CfgN::BM && p.nbatch <= 1 && 2 * cdiv(p.N, 128) * p.splits <= p.cus;
 }
 
@@ -1172,8 +1172,8 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
   } else if (p.sw) {  // W8A8
     hipLaunchKernelGGL((gemm_kernel<CfgS, EPI, true, true>), dim3(cdiv(p.M, CfgS::BM) * cdiv(p.N, CfgS::BN) * p.splits),
                        dim3(CfgS::THREADS), CfgS::LDS, st, p);
-  } else if (kNarrow<EPI> && narrow(p)) {
-    if constexpr (kNarrow<EPI>) {
+  } else if (takes_narrow(EPI) && narrow(p)) {
+    if constexpr (takes_narrow(EPI)) {
       if (p.M <= CfgNs::BM) launch_cfg<CfgNs, EPI>(p, st);
       else launch_cfg<CfgN, EPI>(p, st);
     }
@@ -1224,13 +1224,13 @@ extern "C" void vwa_gemm_set_split_fill(int pct) { g_split_fill_pct = pct < 0 ? 
 
 extern "C" void vwa_gemm_set_p8(int mode) { g_p8_mode = mode; }
 
-extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int parts, int* large, int* splits) {
+extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int parts, int* columns, int* splits) {
   GemmParams p = *pp;
   p.keep_order = keeps_order(epi, p);
   const Plan pl = choose(p, parts);
   const int per = cdiv(p.K / BKG, pl.splits);
-  *large = pl.p8;
-  *splits = cdiv(p.K / BKG, per);
+  p.splits = *splits = cdiv(p.K / BKG, per);
+  *columns = pl.p8 ? CfgP8::BN : !p.keep_order && !p.sw && takes_narrow(epi) && narrow(p) ? CfgN::BN : CfgS::BN;
 }
 
 namespace {

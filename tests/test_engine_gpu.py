@@ -953,3 +953,43 @@ def test_narrow_persistent_decoder_stamps_its_levels(opt, monkeypatch):
         assert of[:, :3].tolist() == [[H, 4 * H, 4 * H]] * 3 and not ts[:, :, 3:].any()
         done = ts[ts[..., 3] > 0]
         assert (done[:, 1:] >= done[:, :-1]).all()
+
+
+@pytest.mark.parametrize("ns,vocab", [(1, 80021), (3, 70003)])
+def test_narrow_persistent_decoder_over_a_large_vocabulary(ns, vocab, monkeypatch):
+    """More vocabulary tiles than the LM head's workgroups have in flight at once (20 each): the logits of both rounds against the
+    per-kernel path, and the greedy sample over a mask of the second round's columns, of the first's and of both."""
+    import dataclasses
+
+    from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner
+
+    cfg = dataclasses.replace(get_config("whisper-tiny"), d_model=128 * ns, n_heads=2 * ns, n_enc_layers=1, n_dec_layers=2, vocab_size=vocab)
+    m = WhisperModel(cfg, device="cuda", seed=6)
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    enc = torch.randn(1, cfg.n_audio_ctx, cfg.d_model, device="cuda", generator=gen).bfloat16()
+    out = []
+    for persist in ("0", "1"):
+        monkeypatch.setenv("VWA_ASR_PERSIST", persist)
+        r = WhisperRunner(m, max_sessions=1, use_graphs=False)
+        r.set_cross(0, enc)
+        out.append(torch.cat([r.step([(0, 11 * p, p)]).float().clone() for p in range(2)]))
+    st = next(iter(m._wdec.values()))
+    V, first = out[0].shape[1], 20 * 16 * (st["ints"][10] - 18 * ns)
+    assert st["part"] is not None and first + 16 < vocab
+    for part in (slice(0, first), slice(first, V)):
+        assert (out[0][:, part] - out[1][:, part]).abs().max() < 0.02 * (1 + out[0].abs().max())
+    b, i32 = r.b, dict(dtype=torch.int32, device="cuda")
+    state = [t.clone() for t in (b.tokens, b.positions, b.ctx_lens, b.slots)]
+    for lo, hi in ((first, vocab), (0, first), (0, vocab)):
+        bits = torch.zeros(-(-V // 32) * 32, dtype=torch.bool)
+        bits[lo:hi] = torch.rand(hi - lo, generator=torch.Generator().manual_seed(lo)) < 0.3
+        words = (bits.view(-1, 32).long() << torch.arange(32)).sum(1)
+        mask = torch.where(words >= 1 << 31, words - (1 << 32), words).to(**i32)
+        for t, s in zip((b.tokens, b.positions, b.ctx_lens, b.slots), state):
+            t.copy_(s)
+        tok, step, seen, n = (torch.zeros(k, **i32) for k in (1, 1, 4, 1))
+        assert m.wdec_loop_step(b, mask, tok, step, seen, n, 1)
+        logits = b.logits[0, :V].float().masked_fill(~bits[:V].cuda(), -math.inf)
+        assert torch.equal(b.logits[:1, :V].float(), out[1][1:])
+        assert tok.item() == logits.argmax().item() == seen[0].item() and n.item() == 1
+    assert not m.chain_error()

@@ -1242,8 +1242,8 @@ def test_flash_attention_is_bitwise_reproducible(hd, causal, qmul):
 @pytest.mark.parametrize("K", [128, 256, 384, 1152])
 @pytest.mark.parametrize("M", [17, 31, 32, 33, 48, 63, 64])
 def test_gemm_few_row_tiles_give_the_bits_of_the_128_row_tile(M, K):
-    """17 .. 64 rows on the 32- and 64-row tiles (three and four stage buffers; products of fewer stages than buffers) against the
-    same rows of a 128-row-tile call in the same slices: a tile of rows does not change a row's sums."""
+    """17 .. 64 rows on the 32- and 64-row tiles of 64 and of 128 columns (three and four stage buffers; products of fewer stages
+    than buffers) against the same rows of a 128-row-tile call in the same slices: a tile of rows does not change a row's sums."""
     torch.manual_seed(M * K)
     N = 272
     x = torch.randn(65, K, device="cuda").to(torch.bfloat16)
@@ -1251,14 +1251,18 @@ def test_gemm_few_row_tiles_give_the_bits_of_the_128_row_tile(M, K):
     r = torch.randn(65, N, device="cuda").to(torch.bfloat16)
     ops.ext().gemm_set_split_fill(75)  # (both by one rule for the slices)
     try:
-        for tw in (ops.TiledWeight(w), ops.TiledWeight(w, keep_order=True), w):
-            for epi, res in (("none", None), ("resid", r), ("gelu", None)):
-                outs = [torch.empty(m, N, dtype=torch.bfloat16, device="cuda") for m in (M, 65)]
-                for m, o in zip((M, 65), outs):
-                    ops.gemm(x[:m], tw, o, epi=epi, residual=None if res is None else res[:m])
-                assert torch.equal(outs[0], outs[1][:M]), (epi, type(tw))
+        for columns, mode in ((64, 2), (128, 0)):
+            ops.ext().gemm_set_p8(mode)
+            assert ops.ext().gemm_tile(0, M, N, K)[0] == columns and ops.ext().gemm_tile(0, 65, N, K)[0] == 128
+            for tw in (ops.TiledWeight(w), ops.TiledWeight(w, keep_order=True), w):
+                for epi, res in (("none", None), ("resid", r), ("gelu", None)):
+                    outs = [torch.empty(m, N, dtype=torch.bfloat16, device="cuda") for m in (M, 65)]
+                    for m, o in zip((M, 65), outs):
+                        ops.gemm(x[:m], tw, o, epi=epi, residual=None if res is None else res[:m])
+                    assert torch.equal(outs[0], outs[1][:M]), (epi, type(tw), columns)
     finally:
         ops.ext().gemm_set_split_fill(0)
+        ops.ext().gemm_set_p8(2)
     want = x[:M].double() @ w.double().T
     got = ops.gemm(x[:M], ops.TiledWeight(w), torch.empty(M, N, dtype=torch.bfloat16, device="cuda"))
     assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
@@ -1457,3 +1461,123 @@ def test_up_to_16_rows_take_one_kernel(N, K):
     for M in (1, 2, 3, 4, 5, 7, 8, 12, 15):
         for i, (got, want) in enumerate(zip(forms(M), whole)):
             assert torch.equal(got, want[:M]), (M, i)
+
+
+def _few_row_forms(x, tw, r, r32, bias, n_split):
+    """(name, result, f64 of it, roundings of the result behind its sum) of every epilogue that the few-row tiles have."""
+    M, N = x.shape[0], tw.shape[0]
+    bf = lambda n=N: torch.full((M, n), 9.0, device=DEV, dtype=BF)  # noqa: E731
+    prod = x.double() @ ops.plain(tw).double().T
+    yield "store", ops.gemm(x, tw, bf()), prod, 1
+    yield "bias", ops.gemm(x, tw, bf(), bias=bias), prod + bias.double(), 1
+    yield "f32", ops.gemm(x, tw, torch.full((M, N), 9.0, device=DEV)), prod, 0
+    yield "residual", ops.gemm(x, tw, bf(), epi="resid", residual=r), prod + r.double(), 1
+    y = r32.clone()
+    yield "f32 residual", ops.gemm(x, tw, y, epi="resid", residual=y), prod + r32.double(), 0
+    yield "gelu", ops.gemm(x, tw, bf(), epi="gelu", bias=bias), torch.nn.functional.gelu(prod + bias.double()), 1
+    a, b = bf(n_split), bf(N - n_split)
+    ops.ext().gemm(x, tw.t, None, a, 6, None, None, True, ops.GEMM_WS_FLOATS, y2=b)
+    yield "split", torch.cat([a, b], 1), torch.cat([prod[:, :n_split], prod[:, n_split:].clamp_min(0) ** 2], 1), 1
+    if N % 32 == 0:
+        gu = prod.view(M, N // 32, 2, 16)
+        yield "swiglu", ops.gemm(x, tw, bf(N // 2), epi="swiglu"), (torch.nn.functional.silu(gu[:, :, 0]) * gu[:, :, 1]).reshape(M, -1), 1
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K,columns,slices", [(17664, 256, 128, 1), (16400, 640, 128, 1), (17664, 2048, 128, 1),   # whole, last column tiles of 16
+                                                (1024, 4096, 64, 16), (1104, 2048, 64, 8), (6144, 4096, 128, 4)])     # in slices
+def test_few_row_tiles_and_their_epilogues(M, N, K, columns, slices):
+    """The 32- and 64-row tiles of 128 columns in one slice, those of 64 and of 128 in slices: every epilogue against float64.  f32
+    sums of K products: within 1e-5 (2-norm); bf16 results round once, 2^-9 at most (relu(.)^2 and a SwiGLU's product double a
+    sum's relative error, which stays far below)."""
+    assert ops.ext().gemm_tile(0, M, N, K) == (columns, slices)
+    x, tw = rnd(M, K), ops.TiledWeight(rnd(N, K, scale=K ** -0.5))
+    for name, got, want, roundings in _few_row_forms(x, tw, rnd(M, N), torch.randn(M, N, device=DEV), rnd(N), 528):
+        err = (got.double() - want).norm() / want.norm()
+        assert err < (2.0 ** -8 if roundings else 1e-5), (name, float(err))
+
+
+@pytest.mark.parametrize("M", [1, 5, 16, 32, 33, 64])
+@pytest.mark.parametrize("K,columns,slices", [(4096, 128, 8), (1024, 64, 4)])
+def test_few_row_tiles_rotate_and_write_the_cache(M, K, columns, slices):
+    """QKV on the few-row tiles (rotation, paged K / V rows, an inert row) against the 128-row tile, and the norm handed on as
+    sums of squares against float64."""
+    nq, nkv, hd = 16, 8, 128
+    H = nq + 2 * nkv
+    N = H * hd
+    assert ops.ext().gemm_tile(5, M, N, K) == (columns, slices)
+    x = rnd(65, K)
+    wd = rnd(N, K, scale=K ** -0.5)
+    tw = ops.TiledWeight(ops.permute_qkv_rows(wd, H, hd))
+    rope = ops.rope_table(512, hd, 1e4, device=DEV)
+    pos = torch.arange(65, dtype=torch.int32, device=DEV) * 3
+    slots = torch.randperm(128, generator=torch.Generator().manual_seed(M))[:65].to(DEV)
+    slots[M // 2] = -1
+    ss = ops.ss_fixed(x.float().pow(2).sum(-1))
+
+    def run(m, hand):
+        kc, vc = (torch.zeros(8, nkv, 16, hd, dtype=BF, device=DEV) for _ in range(2))
+        q = torch.full((m, nq * hd), 9.0, dtype=BF, device=DEV)
+        ops._gemm_qkv(x[:m], tw, None, hand, 1e-5, nq, nkv, hd, rope, pos, slots, q, kc, vc, ss_in=ss if hand else None)
+        return q, kc, vc
+
+    ops.ext().gemm_set_split_fill(75)  # (one rule for the slices: the bits of the 128-row tile)
+    try:
+        few, many = run(M, False), run(65, False)
+    finally:
+        ops.ext().gemm_set_split_fill(0)
+    assert torch.equal(few[0], many[0][:M])
+    live = slots[:M][slots[:M] >= 0]
+    for a, b in zip(few[1:], many[1:]):
+        rows = lambda c: c.transpose(1, 2).reshape(128, -1)  # noqa: E731
+        assert torch.equal(rows(a)[live], rows(b)[live])
+        rest = torch.ones(128, dtype=torch.bool, device=DEV)
+        rest[live] = False
+        assert not rows(a)[rest].any()
+    q, kc, vc = run(M, True)
+    n = x[:M].double() * torch.rsqrt(x[:M].double().pow(2).mean(-1, keepdim=True) + 1e-5)
+    y = (n @ wd.double().T).view(M, H, hd)
+    ang = rope[pos[:M].long()].double()
+    co, si = ang[:, None, :, 0], ang[:, None, :, 1]
+    u, v = y[..., : hd // 2], y[..., hd // 2 :]
+    rot = torch.cat([u * co - v * si, v * co + u * si], -1)
+    # (2-norm: one rounding to bf16, and the f32 scale of a row)
+    assert (q.double().view(M, nq, hd) - rot[:, :nq]).norm() / rot[:, :nq].norm() < 2.0 ** -8
+    keep = slots[:M] >= 0
+    if keep.any():
+        k, w = (c.transpose(1, 2).reshape(128, nkv, hd)[live].double() for c in (kc, vc))
+        assert (k - rot[keep, nq : nq + nkv]).norm() / rot[keep, nq : nq + nkv].norm() < 2.0 ** -8
+        assert (w - y[keep, nq + nkv :]).norm() / y[keep, nq + nkv :].norm() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("M", [1, 4, 8, 16])
+def test_rms_statistics_of_few_rows(M):
+    """The hand-off of the row statistics at the rows that the streaming kernel's own norm served: residual product -> sums of squares
+    -> SwiGLU and QKV products, against float64."""
+    d, F, nq, nkv, hd = 4096, 2048, 8, 4, 128
+    H = nq + 2 * nkv
+    wo, wg, wu, wq = rnd(d, d, scale=d ** -0.5), rnd(F, d, scale=0.02), rnd(F, d, scale=0.02), rnd(H * hd, d, scale=d ** -0.5)
+    to, tgu, tq = ops.TiledWeight(wo), ops.TiledWeight(ops.interleave_gate_up(wg, wu)), ops.TiledWeight(ops.permute_qkv_rows(wq, H, hd))
+    assert all(ops.rows_take_tiles(M, w) for w in (to, tgu, tq))
+    x, h0 = rnd(M, d), rnd(M, d)
+    ss = torch.full((2, M), 7, dtype=torch.int64, device=DEV)
+    ss[0].zero_()
+    h = h0.clone()
+    ops.linear(x, to, out=h, residual=h, ss_out=ss[0], ss_zero=ss[1])
+    want = x.double() @ wo.double().T + h0.double()
+    assert (h.double() - want).norm() / want.norm() < 2.0 ** -8 and not ss[1].any()
+    sq = h.double().pow(2).sum(-1)
+    assert bool(((ops.ss_float(ss[0]) - sq).abs() <= sq * 1e-5).all())  # (f32 sums of d squares)
+    n = h.double() * torch.rsqrt(h.double().pow(2).mean(-1, keepdim=True) + 1e-5)
+    g, u = n @ wg.double().T, n @ wu.double().T
+    want = torch.nn.functional.silu(g) * u
+    got = ops.linear_swiglu(h, tgu, fuse_rms=True, eps=1e-5, ss_in=ss[0])
+    assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
+    kc, vc = (torch.zeros(2, nkv, 16, hd, dtype=BF, device=DEV) for _ in range(2))
+    q = ops.qkv_rope_write(h, tq, None, fuse_rms=True, eps=1e-5, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, rope=None,
+                           positions=torch.zeros(M, dtype=torch.int32, device=DEV), slots=torch.arange(M, device=DEV),
+                           q_out=torch.empty(M, nq * hd, dtype=BF, device=DEV), k_cache=kc, v_cache=vc, ss_in=ss[0])
+    y = (n @ wq.double().T).view(M, H, hd)
+    for got, want in ((q.view(M, nq, hd), y[:, :nq]), (kc[0, :, :M].transpose(0, 1), y[:, nq : nq + nkv]),
+                      (vc[0, :, :M].transpose(0, 1), y[:, nq + nkv :])):
+        assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
