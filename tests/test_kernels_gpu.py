@@ -1581,3 +1581,45 @@ def test_rms_statistics_of_few_rows(M):
     for got, want in ((q.view(M, nq, hd), y[:, :nq]), (kc[0, :, :M].transpose(0, 1), y[:, nq : nq + nkv]),
                       (vc[0, :, :M].transpose(0, 1), y[:, nq + nkv :])):
         assert (got.double() - want).norm() / want.norm() < 2.0 ** -8
+
+
+@pytest.mark.parametrize("M", [1, 16, 24])
+def test_qkv_on_the_tiles_refuses_what_the_streaming_kernel_refuses(M):
+    """Operands that do not fit are errors of the host on either kernel: they would be addresses out of range."""
+    nq, nkv, hd, K = 8, 4, 128, 4096
+    tw = ops.TiledWeight(rnd((nq + 2 * nkv) * hd, K, scale=K ** -0.5))
+    assert ops.rows_take_tiles(M, tw)
+    cache = lambda g=nkv, d=hd: torch.zeros(4, g, 16, d, dtype=BF, device=DEV)  # noqa: E731
+    good = dict(rope=ops.rope_table(64, hd, 1e4, device=DEV), positions=torch.arange(M, dtype=torch.int32, device=DEV),
+                slots=torch.arange(M, device=DEV), q_out=torch.empty(M, nq * hd, dtype=BF, device=DEV), k_cache=cache(), v_cache=cache())
+
+    def call(**bad):
+        return ops.qkv_rope_write(rnd(M, K), tw, None, fuse_rms=False, eps=1e-5, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd,
+                                  **{**good, **bad})
+
+    call()
+    for bad in (dict(positions=good["positions"].cpu()), dict(slots=good["slots"].cpu()), dict(positions=good["positions"][: M - 1]),
+                dict(k_cache=cache(2), v_cache=cache(2)), dict(k_cache=cache(d=64), v_cache=cache(d=64)),
+                dict(rope=ops.rope_table(64, 64, 1e4, device=DEV)), dict(q_out=good["q_out"].half()),
+                dict(q_out=torch.empty(M, 4 * hd, dtype=BF, device=DEV))):
+        with pytest.raises(RuntimeError):
+            call(**bad)
+
+
+def test_qkv_of_few_rows_into_rows_that_are_not_16_byte_aligned():
+    """Query rows and caches of any stride, as the streaming kernel takes them, whatever the weight's size."""
+    M, nq, nkv, hd, K = 5, 8, 4, 128, 4096
+    x, tw = rnd(M, K), ops.TiledWeight(rnd((nq + 2 * nkv) * hd, K, scale=K ** -0.5))
+    assert ops.rows_take_tiles(M, tw)
+    pos, slots = torch.arange(M, dtype=torch.int32, device=DEV), torch.arange(M, device=DEV)
+    rope = ops.rope_table(64, hd, 1e4, device=DEV)
+    outs = []
+    for pad_q, pad_c in ((0, 0), (4, 0), (0, 4), (0, 1)):
+        q = torch.zeros(M, nq * hd + pad_q, dtype=BF, device=DEV)[:, : nq * hd]
+        kc, vc = (torch.zeros(2, nkv, 16, hd + pad_c, dtype=BF, device=DEV)[..., :hd] for _ in range(2))
+        ops.qkv_rope_write(x, tw, None, fuse_rms=False, eps=1e-5, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, rope=rope, positions=pos,
+                           slots=slots, q_out=q, k_cache=kc, v_cache=vc)
+        outs.append((q, kc, vc))
+    for o in outs[1:]:
+        for a, b in zip(o, outs[0]):
+            assert (a.double() - b.double()).norm() / b.double().norm() < 2.0 ** -7  # (two roundings to bf16 of sums in two orders)

@@ -503,6 +503,11 @@ def _rows16(t: Optional[torch.Tensor]) -> bool:
     return t is None or (t.stride(-1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
 
 
+def _cache_rows16(k: torch.Tensor, v: torch.Tensor) -> bool:
+    """K / V caches whose token rows the tiled GEMM's epilogue can write (16-byte rows, one set of strides)."""
+    return k.stride() == v.stride() and all(s % 8 == 0 for s in k.stride()[:3]) and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0
+
+
 def _fp8_staging(x: torch.Tensor, K: int):
     M = x.shape[0]
     x8 = scratch(x.device, "gemm_x8", M * K, torch.uint8).view(torch.float8_e4m3fn)
@@ -785,8 +790,8 @@ def qkv_rope_write(x: torch.Tensor, w_qkv: torch.Tensor, bias: Optional[torch.Te
     ln_c: folded LayerNorm on x (see linear).  ss_in: handed-off sums of squares (see ops.gemm)."""
     M = x.shape[0]
     if isinstance(w_qkv, TiledWeight):
-        few = (ln_c is None and (not fuse_rms or ss_in is not None) and GEMM_QKV_FUSED and gemm_ok(x, w_qkv)
-               and rows_take_tiles(M, w_qkv))
+        few = (ln_c is None and (not fuse_rms or ss_in is not None) and GEMM_QKV_FUSED and gemm_ok(x, w_qkv, q_out)
+               and _cache_rows16(k_cache, v_cache) and rows_take_tiles(M, w_qkv))
         if _gpu(x) and _stream_ok(x, w_qkv) and not few and (ln_c is None or _ln_fold_fits(x, w_qkv)):
             ext().skinny_gemm_qkv(x, w_qkv.t, bias, fuse_rms and ln_c is None, eps, n_q_heads, n_kv_heads, head_dim,
                                   rope is not None, positions, slots, rope, q_out, k_cache, v_cache, None, ln_c, True)
