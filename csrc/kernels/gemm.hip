@@ -1238,6 +1238,8 @@ int checks_and_plan(int epi, GemmParams& p, bool* p8, bool parts = false) {
   if (p.M < 1 || p.N < 16 || p.N % 16 || p.K < BKG || p.K % BKG) return -10;
   if (p.ldx % (p.sx ? 16 : 8) || (reinterpret_cast<uintptr_t>(p.X) & 15) || (reinterpret_cast<uintptr_t>(p.W) & 15))
     return -11;
+  constexpr int64_t kMost = 0x7FFFFFF0ll;  // (32-bit offsets, and loads past a resource's end are zeros)
+  if ((int64_t)p.N * p.K * (p.sw ? 1 : 2) >= kMost || ((int64_t)(p.M - 1) * p.ldx + p.K) * (p.sx ? 1 : 2) >= kMost) return -21;
   if ((p.sw && !p.w_tiled) || (p.sx && !p.sw)) return -14;  // fp8: the tiled layout; X codes need fp8 weights
   if (epi == EPI_SWIGLU && (p.N % 32 || p.y_f32)) return -12;
   if (epi == EPI_QKV && (p.y_f32 || p.head_dim % 16 || p.N != (p.n_q_heads + 2 * p.n_kv_heads) * p.head_dim ||

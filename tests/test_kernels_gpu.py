@@ -1623,3 +1623,24 @@ def test_qkv_of_few_rows_into_rows_that_are_not_16_byte_aligned():
     for o in outs[1:]:
         for a, b in zip(o, outs[0]):
             assert (a.double() - b.double()).norm() / b.double().norm() < 2.0 ** -7  # (two roundings to bf16 of sums in two orders)
+
+
+def test_weights_past_32_bit_offsets_never_reach_the_tiles(monkeypatch):
+    """2 GiB and more of a weight: <= 16 rows of the pre-tiled copy are refused, as the streaming kernel refuses them, more rows take
+    the library's product.  (On the tiles the columns past the limit were zeros.)"""
+    N, K = 131088, 8192
+    assert N * K * 2 >= ops.GEMM_MAX_BYTES
+    w = torch.empty(N, K, dtype=BF, device=DEV).normal_(0.0, K ** -0.5, generator=torch.Generator(device=DEV).manual_seed(1))
+    tw = ops.TiledWeight(w)
+    for M in (1, 16):
+        with pytest.raises(RuntimeError):
+            ops.linear(rnd(M, K), tw)
+    x = rnd(24, K)
+    out = torch.empty(24, N, dtype=BF, device=DEV)
+    for call in (lambda: ops.gemm(x, tw, out), lambda: ops.ext().linear_parts(x, tw.t, 0)):
+        with pytest.raises(RuntimeError):
+            call()
+    monkeypatch.setenv("VWA_STRICT_NATIVE", "0")
+    monkeypatch.setattr(ops, "vendor_fallbacks", {})
+    close(ops.linear(x, tw)[:, -64:], (x.double() @ w[-64:].double().T).float(), 1e-2, 1e-2)
+    assert len(ops.vendor_fallbacks) == 1

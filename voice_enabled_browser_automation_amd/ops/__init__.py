@@ -554,18 +554,25 @@ def _f32_resid(out: torch.Tensor, residual: Optional[torch.Tensor]) -> bool:
     return residual is not None and residual.dtype == torch.float32 and out.dtype == torch.float32
 
 
+GEMM_MAX_BYTES = 0x7FFFFFF0  # of a product's weight and of its rows (gemm.hip addresses both by 32-bit offsets)
+
+
+def _in_reach(x: torch.Tensor, n: int, k: int, w_bytes: int) -> bool:
+    return n * k * w_bytes < GEMM_MAX_BYTES and ((x.shape[0] - 1) * x.stride(0) + k) * 2 < GEMM_MAX_BYTES
+
+
 def gemm_fp8_ok(x: torch.Tensor, w, out: Optional[torch.Tensor] = None, residual: Optional[torch.Tensor] = None) -> bool:
     return (isinstance(w, FP8Weight) and w.tiled and _gpu(x) and x.dtype == torch.bfloat16 and w.shape[0] % 16 == 0
-            and w.shape[1] % 128 == 0 and _rows16(x) and _rows16(out) and _rows16(residual))
+            and w.shape[1] % 128 == 0 and _rows16(x) and _rows16(out) and _rows16(residual) and _in_reach(x, *w.shape, 1))
 
 
 def gemm_ok(x: torch.Tensor, w, out: Optional[torch.Tensor] = None, residual: Optional[torch.Tensor] = None) -> bool:
-    """Shapes the tiled GEMM takes (bf16 weights, N % 16, K % 128, 16-byte aligned rows)."""
+    """Shapes the tiled GEMM takes (bf16 weights, N % 16, K % 128, 16-byte aligned rows, less than 2 GiB of either operand)."""
     if isinstance(w, FP8Weight) or not _gpu(x) or x.dtype != torch.bfloat16:
         return False
     wt = w.t if isinstance(w, TiledWeight) else w
     return (wt.dtype == torch.bfloat16 and wt.shape[0] % 16 == 0 and wt.shape[1] % 128 == 0 and _rows16(x)
-            and _rows16(out) and _rows16(residual))
+            and _rows16(out) and _rows16(residual) and _in_reach(x, *wt.shape, 2))
 
 
 # ----------------------------------------------------------------------------- GEMM family
