@@ -149,6 +149,9 @@ class StepBuffers:
         self.np_row_table = self.h_row_table.numpy()
         self.h_i32[3].fill_(1)  # the same inert rows as the device copy (captured graphs upload it)
         self.h_slots.fill_(-1)
+        # the block table as the host has it (np_table; sequences come, grow and go at any time) and its pinned staging copy,
+        # which is written only when no copy of it can be queued
+        self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
         self.h_table = torch.zeros(max_seqs, max_blocks_per_seq, dtype=torch.int32, pin_memory=pin)
         self.table_dirty = True
         # numpy views of the pinned staging buffers: the per-step row metadata is written with a
@@ -156,15 +159,22 @@ class StepBuffers:
         self.np_i32 = self.h_i32.numpy()
         self.np_slots = self.h_slots.numpy()
         self.np_sel = self.h_sel.numpy()
-        self.np_table = self.h_table.numpy()
 
     def upload(self, n_rows: int, meta: bool = True) -> None:
         """H2D copy of the step metadata (skipped when the replayed graph contains it) and of the
-        block table when it changed."""
+        block table when it changed.  The staging copies are free (LLMEngine._sync_staging)."""
         if meta:
             self.meta.copy_(self.h_meta, non_blocking=True)
         if self.table_dirty:
+            self.h_table.numpy()[:] = self.np_table
             self.block_table.copy_(self.h_table, non_blocking=True)
+            self.table_dirty = False
+
+    def upload_table(self) -> None:
+        """H2D copy of the block table when it changed, out of pinned rows of its own: the staging copy may be queued."""
+        if self.table_dirty:
+            t = torch.from_numpy(self.np_table)
+            self.block_table.copy_(t.pin_memory() if self.block_table.is_cuda else t, non_blocking=True)
             self.table_dirty = False
 
 
@@ -403,7 +413,6 @@ class LLMEngine:
             sid = seq.sid
             pos = pending.get(sid, seq.n_computed)
             if pos // bs >= len(seq.blocks):
-                self._sync_staging()  # (the block table is staged as well)
                 self._ensure_blocks(seq, pos + 1)
             if pos >= len(seq.tokens):
                 seq.tokens.append(tok)
@@ -721,10 +730,7 @@ class LLMEngine:
         np_meta[2] = np.repeat([seq.sid for seq, _ in parts], [k for _, k in parts])
         np_meta[3] = np_meta[1] + 1
         runs = self._runs(parts, poss)
-        if self.bufs.table_dirty:
-            self.bufs.block_table.copy_(self.bufs.h_table, non_blocking=self.device.type == "cuda")
-            self.bufs.table_dirty = False
-            self._staging_inflight = self.device.type == "cuda"  # (the copy reads the pinned table)
+        self.bufs.upload_table()
         dev, m = self.device, self.model
         meta, slot_t = torch.from_numpy(np_meta), torch.from_numpy(np.concatenate(slots))
         if dev.type == "cuda":
@@ -813,9 +819,7 @@ class LLMEngine:
                 logits = self.model.lm_logits(self.bufs, hs)
                 continue
             self._ensure_blocks(seq, start + n)
-            if self.bufs.table_dirty:
-                self.bufs.block_table.copy_(self.bufs.h_table)
-                self.bufs.table_dirty = False
+            self.bufs.upload_table()
             dev, m = self.device, self.model
             pos = np.arange(start, start + n)
             np_meta = np.stack([np.asarray(seq.tokens[start : start + n], dtype=np.int32), pos.astype(np.int32)])
