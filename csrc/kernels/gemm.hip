@@ -1057,30 +1057,31 @@ Plan plan(const GemmParams& p) {
   return best;
 }
 
-// K slices of a bf16 product of <= 64 rows and of fp8 weights (W8A16): by the weight alone, so that a row's sums are added up in
-// one order whatever rows come with it (W8A16 of more than 64 rows: by the blocks of 64 too).  The cheapest by an estimate in us,
-// fitted to 270 timings (24, 48 and 64 rows, 22 weights of 1024 .. 32768 columns and K 1024 .. 14336, 1 .. 32 slices) and for fp8
-// weights to 520, priced at one number of rows each.  Over 28 weights in the tiles taken now, 1, 16, 32, 48, 64 rows, slower than the
-// best choice of each by
-//   bf16, priced at 48 rows     2.3, 3.8, 6.5, 3.8, 5.5 %      at the rows of the call  6.4, 4.8, 7.2, 3.8, 5.8 %
-//   the same for the norm, at 1 0.9, 1.1, 1.5, 0.2, 0.1 %                               1.0, 2.8, 4.6, 4.0, 5.0 %
-//   fp8 weights, at 24          0.7 (17 rows), 1.0, 1.0, 0.6 %                          0.8, 0.5, 0.5, 1.2 %
-// Powers of two until the CUs have a tile are 6 % (bf16) and 10 % (fp8) off and up to 50 % where one slice fills half the chip (48
-// rows: 17664 x 2048 26.3 us in two slices, 20.3 whole; fp8, 32 rows: 28672 x 4096 30.0 in two, 23.1 whole).
+// K slices of a bf16 product of <= 64 rows and of fp8 weights (W8A16): the cheapest by an estimate in us, fitted to 270 timings
+// (24, 48 and 64 rows, 22 weights of 1024 .. 32768 columns and K 1024 .. 14336, 1 .. 32 slices) and for fp8 weights to 520.
 //   a workgroup's k-groups one after another, against all of the weight at the chip's rate (the larger counts, both where they are
 //   close); a sum of slices is a launch and its f32 partials
+// bf16: priced at one number of rows, so that the weight alone decides and a row's sums are added up in one order whatever rows
+// come with it.  Over 28 weights in the tiles taken now, 1, 16, 32, 48, 64 rows, slower than the best choice of each by
+//   priced at 48 rows           2.3, 3.8, 6.5, 3.8, 5.5 %      at the rows of the call  6.4, 4.8, 7.2, 3.8, 5.8 %
+//   the same for the norm, at 1 0.9, 1.1, 1.5, 0.2, 0.1 %                               1.0, 2.8, 4.6, 4.0, 5.0 %
+// fp8 weights at the rows of the call (0.8, 0.5, 0.5, 1.2 % at 17, 32, 48, 64 rows; priced at 24 rows they would be 0.7, 1.0, 1.0,
+// 0.6 %, but rows summed in another order flip fp8 codes in the products of <= 16 rows behind them: logits of a 48-row prompt on
+// 1024-wide layers move by 0.03, with the same 0.028 from 64 bits).
+// Powers of two until the CUs have a tile are 6 % (bf16) and 10 % (fp8) off and up to 50 % where one slice fills half the chip (48
+// rows: 17664 x 2048 26.3 us in two slices, 20.3 whole; fp8, 32 rows: 28672 x 4096 30.0 in two, 23.1 whole).
 // parts: no launch adds the slices up, but the workgroup of a row's norm reads its row of each (at about 40 GB/s)
 int few_slices(const GemmParams& p, bool parts) {
   const int KG = p.K / BKG, blocks = cdiv(p.M, CfgF::BM);
   const bool w8 = p.sw != nullptr;
-  const int M = blocks > 1 ? p.M : parts ? 1 : w8 ? 24 : 48;
+  const int M = w8 ? p.M : parts ? 1 : 48, most = w8 ? p.M : CfgF::BM;
   const float per_kg = w8 ? (M <= CfgFs::BM ? 0.42f : 0.68f) + 0.00065f * (blocks > 1 ? CfgF::BM : M) : 0.52f + 0.0063f * M;
   const float chip = (float)p.N * p.K * blocks * (w8 ? 1.f / 6.2e6f : 2.f / 6.1e6f) * (256.f / p.cus);
   const float launch = w8 ? 2.6f : 3.2f, slab = (float)M * p.N * (4 * (w8 ? 0.53e-6f : 0.44e-6f));
   int best = 1;
   float least = 0.f;
   for (int s0 = 1; s0 <= 32 && s0 <= KG; s0 *= 2) {
-    if (s0 > 1 && (int64_t)s0 * (blocks > 1 ? p.M : CfgF::BM) * p.N > p.ws_cap) break;
+    if (s0 > 1 && (int64_t)s0 * most * p.N > p.ws_cap) break;
     const int per = cdiv(KG, s0), s = cdiv(KG, per);
     const float alone = per_kg * per;
     const float sum = parts ? (float)s * p.N * (4 / 4.e4f) : s > 1 ? launch + s * slab : 0.f;
