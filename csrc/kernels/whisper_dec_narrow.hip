@@ -229,24 +229,24 @@ VWA_DEVICE void nd_load_k64(const u16* W, int KG, int unit, uint4 (&wr)[R]) {
       wr[O + 2 * t + j] = make_uint4(v.x, v.y, v.z, v.w);
     }
 }
-// ... times the 64 values in LDS, each the sum of its PIECES, -> a partial row
+// ... times the 64 values in LDS, each the sum of its PIECES, -> a partial row (piece i is row i of A: one product for all)
 template <int NS, int O, int PIECES = 1, int R>
 VWA_DEVICE void nd_k64(const char* lds, const uint4 (&wr)[R], float* out) {
+  static_assert(PIECES <= 4, "rows of a lane");
   const int tx = VWA_TX, lane = tx & 63, g = lane >> 4, w = uni(tx >> 6);
-  const u16* av = reinterpret_cast<const u16*>(lds + L_AV);
-  uint4 a[PIECES][2];
+  const u16* av = reinterpret_cast<const u16*>(lds + L_AV) + 64 * min(lane & 15, PIECES - 1);
+  uint4 a[2];
 #pragma unroll
-  for (int e = 0; e < PIECES; ++e)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) a[e][j] = *reinterpret_cast<const uint4*>(av + 64 * e + 32 * (g & 1) + 8 * (2 * j + (g >> 1)));
+  for (int j = 0; j < 2; ++j) a[j] = *reinterpret_cast<const uint4*>(av + 32 * (g & 1) + 8 * (2 * j + (g >> 1)));
 #pragma unroll
   for (int t = 0; t < NS; ++t) {
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int e = PIECES - 1; e >= 0; --e)  // (the small ones first)
+    for (int j = 0; j < 2; ++j) acc = mfma16(as_bf16x8(a[j]), as_bf16x8(wr[O + 2 * t + j]), acc);
+    float v = acc[PIECES - 1];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc = mfma16(as_bf16x8(a[e][j]), as_bf16x8(wr[O + 2 * t + j]), acc);
-    if (lane < 16) stf_sc1(out + (w + 8 * t) * 16 + lane, acc[0]);
+    for (int e = PIECES - 2; e >= 0; --e) v += acc[e];  // (the small ones first)
+    if (lane < 16) stf_sc1(out + (w + 8 * t) * 16 + lane, v);
   }
 }
 
