@@ -1,7 +1,7 @@
-// LDS-tiled MFMA GEMM for the row counts the skinny decode kernels do not take (K12, M > 16):
-// the prompt suffix prefill of the intent LLM (apps/brain/src/server.ts:98-105: ~1.1k-token
-// prompt, the un-cached suffix), continuous-batching steps of 17..64 rows, and the Whisper
-// encoder (1500 rows per utterance).  Replaces hipBLASLt for every projection of both models.
+// LDS-tiled MFMA GEMM for what the skinny decode kernels do not take (K12): the prompt suffix prefill of the intent
+// LLM (apps/brain/src/server.ts:98-105: ~1.1k-token prompt, the un-cached suffix), continuous-batching steps of
+// 17..64 rows, the Whisper encoder (1500 rows per utterance), and fewer rows of large pre-tiled bf16 weights
+// (ops.rows_take_tiles).  Replaces hipBLASLt for every projection of both models.
 //
 //   Y[M, N] = epi( rstd[m] * (X[M, K] . W[N, K]^T) )       X bf16 row-major, f32 accumulate
 //
@@ -620,7 +620,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // pipeline: two LDS buffers, the next stage's DMA in flight during this one's MFMAs; raw
+  // pipeline: NST LDS buffers, the next NST - 1 stages' DMA in flight during this one's MFMAs; raw
   // barriers with counted vmcnt (a __syncthreads would drain the in-flight DMA)
   constexpr int SPG = F8 || W8 ? 1 : 2;  // stages per k-group
   constexpr int STG = W8 ? C::W8STAGE : C::STAGE;
@@ -1164,7 +1164,7 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
     else
       hipLaunchKernelGGL((gemm_kernel<CfgP8, EPI, false, false, true>), dim3(tiles * p.splits), dim3(CfgP8::THREADS),
                          CfgP8::LDS, st, p);
-  } else if (p.sw && !p.sx) {  // W8A16
+  } else if (p.sw && !p.sx) {  // W8A16 (tiles of 128 columns alone: of 64 they have not been built or timed)
     const dim3 grid((unsigned)(cdiv(p.M, CfgF::BM) * cdiv(p.N, CfgF::BN) * p.splits)), block(CfgF::THREADS);
     if (p.M <= CfgFs::BM)
       hipLaunchKernelGGL((gemm_kernel<CfgFs, EPI, true, false, false, true>), grid, block, CfgFs::W8LDS, st, p);

@@ -150,7 +150,7 @@ struct alignas(64) ChainParams {
   ChainTP tp;
 };
 
-// LDS-tiled MFMA GEMM (gemm.hip) for M > 16 rows: Y = epi(rstd[m] * X . W^T (+bias) ...)
+// LDS-tiled MFMA GEMM (gemm.hip): Y = epi(rstd[m] * X . W^T (+bias) ...)
 struct GemmParams {
   const uint16_t* X; int ldx;       // [M, K] bf16 row-major
   const uint16_t* W; int w_tiled;   // [N, K] bf16: pre-tiled (ops.tile_weight) or row-major
@@ -178,7 +178,7 @@ struct GemmParams {
   const int* positions; const int64_t* slots; const float* rope;
   uint16_t* q_out; int ldq; uint16_t* k_cache; uint16_t* v_cache; int block_size;
   int64_t cache_sb, cache_sh, cache_st;
-  // RMS statistics hand-off (decode steps of > 16 rows, one rank): ss_out -- the residual epilogue
+  // RMS statistics hand-off (decode steps on the tiled GEMMs, one rank): ss_out -- the residual epilogue
   // adds the squares of its bf16 output rows into ss_out[m] (the next RMSNorm's statistics);
   // ss_zero[0, ss_zero_n) is zeroed by workgroup 0 (the other buffer, already consumed); ss_in --
   // the per-row scale is rsqrt(ss_in[m] / K + ss_eps) instead of rstd[m] (no row_rstd launch).

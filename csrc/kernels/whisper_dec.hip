@@ -1,10 +1,11 @@
 // Persistent Whisper decoder step (any Whisper width: d a multiple of 128 up to 1536, ffn = 4 d,
-// head_dim 64 -- tiny 384 .. large 1280), one row: ONE launch for the whole token step -- the
+// head_dim 64; d <= 512 -- tiny, base -- take whisper_dec_narrow.hip unless a schedule or role option asks for
+// this kernel), one row: ONE launch for the whole token step -- the
 // embedding (layer 0 builds it from the tables), every decoder layer, the LM head (a last level
 // streaming the vocabulary tiles through the slots) and, in the device loop, the greedy masked
 // argmax + the loop advance (workgroup 0 merges the workgroups' partials).
 //
-// Why (VERDICT r5 #3, DESIGN.md round 5): the per-kernel decoder runs eight dependent launches per
+// Why: the per-kernel decoder runs eight dependent launches per
 // layer, each ~5-9 us of fixed latency (dispatch, X staging, the first weight bytes, reduce,
 // epilogue) for 0.3-13 MB of weights -- 2.3 ms per token for ~1.6 GB, 7x off the HBM roofline.
 // Here a workgroup's share of the NEXT use of each of its weight tiles is already in its registers
@@ -43,7 +44,7 @@
 // Weight slots: 5 slots x 5 loads of 1 KB per wave (100 VGPRs).  A 16-column tile of a K = 1280
 // projection is 40 load-slices (k-group, 32-k slice) of the pre-tiled layout; wave w takes slices
 // w, w + 8, ... -- 5 per wave = one slot (narrower models: K / 32 < 40 slices, the rest of the slot
-// reads nothing).  An fc2 tile (K = 4 d) is ceil(d / 320) slots: 4 for large, 2 for tiny.
+// reads nothing).  An fc2 tile (K = 4 d) is ceil(d / 320) slots: 4 for large, 3 for small.
 // The role table (models/whisper.py wdec_roles) gives each workgroup its slots (level, tile, part,
 // refill level), its self-attention head and its cross-attention item.
 #include "whisper_dec.h"

@@ -1,7 +1,7 @@
 // Persistent Whisper decoder step of narrow models (d = 128 .. 512, whisper-tiny and -base; ffn = 4 d, head_dim 64), one
 // row: the whole token step in ONE launch like whisper_dec.hip, with THREE hand-offs between workgroups a layer instead of
-// seven.  What bounds a narrow step is the hand-offs (a level of whisper_dec.hip costs 4.1 us here whatever it computes: arrival,
-// poll, the row's round trip, store drain; 33 of them are the 137 us of a whisper-tiny token, whose 68 MB take 11 us), so a
+// seven.  What bounds a narrow step is the number of dependent levels (one of whisper_dec.hip costs 4.1 us here whatever it computes:
+// arrival, poll, the row's round trip, store drain; 33 of them are the 137 us of a whisper-tiny token, whose 68 MB take 11 us), so a
 // workgroup that holds a slice of an activation multiplies it by its columns of the NEXT projection as well and hands on partial
 // rows, which every consumer adds up in one order:
 //   A  self     one workgroup per head: the layer's input row (sum of C's partials), LN1, the head's q / k / v columns,
@@ -16,9 +16,10 @@
 // Every role keeps its weights of the next layer in registers (<= 32 x 16 B a lane), refilled right after use.
 // Same rounding as whisper_dec.hip (activations bf16, sums f32) but for two places, both finer: the cross query is one product
 // of the normed row, and the cross-attention's output is not rounded at all (nd_attend: PIECES).
-// Measured, whisper-tiny, 30 keys of context: 137 -> 62 us a token (A 5.0, B 4.4, C 3.4 us a layer, of which the hand-off --
-// arrival to release -- is 0.5 each and a consumer's partial rows 1.0 - 1.4; 8.7 us until the first layer's weights and keys are
-// there, 192 KB a head; the LM head 4 behind the last layer).
+// Measured, whisper-tiny, 30 keys of context: 137 -> 62 us a token: 8.7 until the first layer's weights and keys are there (192 KB a
+// head), A 4.6, B 4.5, C 3.6 a layer (tools/wdec_probe.py; the first layer's A 1.7 less: it waits for no rows), 4 for the LM head
+// behind the last.  Of a phase the hand-off -- arrival to release -- is 0.5, a consumer's partial rows 1.0 - 1.4; the rest, 1.1 in C
+// and 2.6 in A and B, are the phase's own products, attention and stores.
 #include "whisper_dec.h"
 
 namespace {
@@ -266,9 +267,9 @@ VWA_DEVICE float nd_bias(const u16* b, int n) { return b ? bf2f(gld(b + n)) : 0.
 
 // Attention of the query in LDS (L_QF, bf16) over nk <= 512 keys in LDS, K rows at kl (16-byte piece c of key t at c ^ (t & 7)),
 // V rows at vl; the normalized output goes to L_AV as bf16, or whole: PIECES 3 are its 24 bits in three bf16 numbers, so that what
-// is not finished yet -- a quarter of a head's keys -- stays f32 through the matrix units too (three products where one bf16
-// number a value takes one: 0.8 us of a token's 62.  Logits of whisper-tiny against 64 bits, mean of 8 utterances:
-// whisper_dec.hip 5.67e-3, quarters rounded to one bf16 5.61e-3, this 5.56e-3).
+// is not finished yet -- a quarter of a head's keys -- stays f32 through the matrix units too.  Logits of whisper-tiny against 64
+// bits, mean of 8 utterances: whisper_dec.hip 5.67e-3, quarters rounded to one bf16 5.61e-3, this 5.55e-3 (and 0.3 us of a token's
+// 62; 0.8 where each piece had a product of its own).
 // Thread 0 gets (max, sum) of the scores' softmax.
 // A wave takes tiles of 16 keys on its own -- max, weights, sum and output -- and one round puts the eight together:
 //   scores: K as the MFMA's B operand, 16 keys to a tile, the wave's four tiles then one key a lane (products and sums as exact

@@ -344,8 +344,8 @@ class LlamaModel:
         when some layer cannot take it (per-layer chained / per-kernel launches then).  The
         descriptors are the per-layer ones (_chain_desc) concatenated into one device array; layer
         0's writes the attention step plan that layers 1.. of the same launch read, so a plan can
-        never be stale (ADVICE r5: a per-layer launch whose layer 0 dropped its attention phase would
-        have left layers 1.. reading an older step's entry)."""
+        never be stale (a per-layer launch whose layer 0 dropped its attention phase would
+        leave layers 1.. reading an older step's entry)."""
         n = len(self.layers)
         if n < 3 or not ops.env_flag("VWA_CHAIN_MULTI") or self.tp.size > 1 and not ops.env_flag("VWA_CHAIN_TP"):
             return None

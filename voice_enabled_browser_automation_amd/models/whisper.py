@@ -491,7 +491,7 @@ class WhisperModel:
         return cache[key]
 
     # ---- persistent decoder (csrc/kernels/whisper_dec.hip wdec_kernel; d <= 512: whisper_dec_narrow.hip): a one-row step of the
-    # Whisper model (tiny .. large: d a multiple of 128 up to 1536, ffn 4 d, head_dim 64) as ONE launch
+    # Whisper model (d a multiple of 128 up to 1536, ffn 4 d, head_dim 64) as ONE launch
     # over every decoder layer; each workgroup's weight tiles stay in its registers a layer ahead.
     def _wdec_ok(self, M: int) -> bool:
         cfg = self.cfg

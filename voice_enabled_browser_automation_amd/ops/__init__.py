@@ -269,7 +269,7 @@ class TiledWeight:
     """A bf16 projection weight stored ONLY in the pre-tiled layout ``t`` = tile_weight(w) (same
     [N, K] shape, MFMA B-fragment element order).  Every GPU consumer reads it directly: the decode
     streaming / chained kernels (1 KB contiguous load instructions) and the LDS-tiled GEMM for
-    prefill and > 16-row steps (gemm.hip copies the 4 KB fragment blocks to LDS verbatim) -- so
+    prefill, > 16-row steps and large weights (gemm.hip copies the 4 KB fragment blocks to LDS verbatim) -- so
     the model keeps one copy of each weight.  ``dense()`` rebuilds the row-major matrix for the
     CPU reference and diagnostics.
 
@@ -485,8 +485,8 @@ def gemm(x: torch.Tensor, w, out: torch.Tensor, *, epi: str = "none", bias: Opti
          residual: Optional[torch.Tensor] = None, fuse_rms: bool = False, eps: float = 1e-5,
          ss_out: Optional[torch.Tensor] = None, ss_zero: Optional[torch.Tensor] = None,
          ss_in: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """The hand-written LDS-tiled MFMA GEMM (csrc/kernels/gemm.hip) for M > 16 rows:
-    out = epi(rms(x) @ w^T + bias); w a TiledWeight (its single pre-tiled copy) or a row-major bf16
+    """The hand-written LDS-tiled MFMA GEMM (csrc/kernels/gemm.hip), for more than SKINNY_MAX_M rows and fewer of large weights
+    (rows_take_tiles): out = epi(rms(x) @ w^T + bias); w a TiledWeight (its single pre-tiled copy) or a row-major bf16
     [N, K] tensor.  fuse_rms: the per-row 1/rms of x scales the product (gamma folded into w) --
     from ``ss_in`` (the rows' sums of squares, handed off by the GEMM that wrote x) when given, else
     one row_rstd launch.  ss_out / ss_zero (residual epilogue): see GemmParams::ss_*."""
@@ -576,8 +576,8 @@ def gemm_ok(x: torch.Tensor, w, out: Optional[torch.Tensor] = None, residual: Op
 
 
 # ----------------------------------------------------------------------------- GEMM family
-# Rows handled by the MFMA streaming (skinny) kernels; above this the hand-written LDS-tiled MFMA
-# GEMM (gemm.hip) takes the step (continuous batching of many sessions, prefill).
+# Rows handled by the MFMA streaming (skinny) kernels; above this, and for large pre-tiled weights (rows_take_tiles), the
+# hand-written LDS-tiled MFMA GEMM (gemm.hip) takes the step (continuous batching of many sessions, prefill).
 SKINNY_MAX_M = 16
 # (a 17..64-row form of the streaming kernel was built -- X streamed with the weights, MT = 2 /
 # 4 row fragments -- and measured slower than the tiled GEMM for whole decode steps, 32 rows
@@ -592,9 +592,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None
            ss_in: Optional[torch.Tensor] = None) -> torch.Tensor:
     """y = act(rms(x) @ w^T + bias) [+ residual].
 
-    GPU: decode rows (<= SKINNY_MAX_M) -> the MFMA streaming GEMM with fused epilogue; more rows
-    -> the LDS-tiled MFMA GEMM (gemm.hip) with the same epilogues.  torch.matmul + the HIP
+    GPU: decode rows (<= SKINNY_MAX_M) -> the MFMA streaming GEMM with fused epilogue; more rows, and any number of a large
+    pre-tiled weight (rows_take_tiles) -> the LDS-tiled MFMA GEMM (gemm.hip) with the same epilogues.  torch.matmul + the HIP
     epilogue kernels only for shapes neither kernel takes.
+    A row's bits do not depend on the other rows of a call among the row counts that one kernel and one set of slices serve:
+    1 .. 64 rows of a bf16 weight that takes the tiles; 1 .. 16 of another one; then 17 .. 64, 65 .. 127 and more rows apart.
+    (fp8 weights' products are cut by the rows too.)  A call with col_mask, fuse_rms without ss_in or
+    ln_c runs on the streaming kernel, whose sums have another order than the tiles'.
     ln_c (from fold_layernorm): x goes through a LayerNorm whose affine is folded into (w, bias);
     decode rows compute its mean/rstd inside the streaming GEMM, other shapes normalise first.
     col_mask (int32 token bitmask rows, the sampler's grammar mask; plain store epilogue): the
@@ -762,7 +766,7 @@ def linear_swiglu(x: torch.Tensor, w_gu: torch.Tensor, *, fuse_rms: bool = False
     return out
 
 
-# > 16-row QKV projections with the rotary + paged-KV write in the tiled GEMM's epilogue (gemm.hip
+# QKV projections on the tiled GEMM with the rotary + paged-KV write in its epilogue (gemm.hip
 # EPI_QKV; with split-K: in the slab reduction) -- no qkv scratch round trip, no rope_kv_write
 # launch.  VWA_GEMM_QKV=0: GEMM -> qkv scratch -> rope_kv_write
 GEMM_QKV_FUSED = knob("VWA_GEMM_QKV")

@@ -59,7 +59,7 @@ def plan_memory(cfg, tp: int = 1, *, wdtype: str = "bf16", kv_gb: Optional[float
     """Bytes per rank.  ``kv_gb`` None: all remaining HBM after the rest (minus the reserve)
     becomes KV; otherwise that many GB (capped at what remains).  ``shared_gb``: HBM left to a
     co-located service (the voice worker's ASR on a shared single GPU).  The workspace counts the
-    GEMM split-K workspace (ops.GEMM_WS_FLOATS), the batched-prefill scratch rows and, under TP,
+    most that a GEMM's K slices take (ops.GEMM_WS_FLOATS; each call's own, the allocator keeps the block), the batched-prefill scratch rows and, under TP,
     the one-shot all-reduce staging + all-gather + chained-layer regions (allreduce.hip)."""
     if gemm_ws_floats is None:
         from .. import ops
