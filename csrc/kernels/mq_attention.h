@@ -256,6 +256,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   // group -- the partial slots 0 .. n_pc + RG - 1
   const int gh = max(1, n_groups * nkv);
   int n_eff, n_pc = 0;
+  bool wave_runs = false;  // cascade: the own keys of all of a group's runs are one chunk, a wave to a run
   if constexpr (FINE) {
     n_eff = max(1, min(min(p.n_splits, 16), grid / gh));
   } else if (cascade) {
@@ -264,6 +265,28 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     // shared keys (gh = 64) measured 24.4 / 18.7 / 21.1 us at 1 / 2 / 4 prefix chunks
     n_pc = max(1, min(p.n_splits - RG, max(kMqCus / gh - RG, kMqCus / 2 / gh)));
     n_eff = n_pc + RG;
+    if constexpr (RG <= NW) {
+      // ... or the own keys of all of a group's runs in one chunk, a wave to a run: many sessions' own chunks do not fit the CUs
+      // once, but a run's keys lie behind one wave then.  The cheaper form by the other branch's count over the groups of real
+      // rows (the padded ones' items are short); lane c - 1: c prefix chunks.
+      // Measured (us; 8 kv heads of D = 128, 992 shared keys): 32 sessions of ~110 own keys 18.2 -> 15.0 (384 items were two rounds of
+      // the CUs, 256 are one, and the merge reads four partials instead of six), 48 of ~110 25.1 -> 20.0, 64 of ~100 27.1 -> 20.6,
+      // 24 of ~150 19.7 -> 16.1; 32 of ~400 (kept as they were) 28.2 / 27.4.
+      const int gr = (n_real + RG - 1) / RG * nkv;
+      const int own = (int)wave_max(lane < n_real ? (float)max(cl - P, 0) : 0.f);
+      auto keys = [&](int pre, int n_own, int own_len) {
+        const int len = (int)ceilf((float)P * __builtin_amdgcn_rcpf((float)pre * kChunk)) * kChunk;
+        const int per_cu = (gr * (pre + n_own) + kMqCus - 1) / kMqCus;
+        return (float)(per_cu * max(len, own_len) + (pre + n_own) * 30 + (per_cu - 1) * (D == 64 ? 100 : 350));
+      };
+      const float cost = keys(min(lane + 1, p.n_splits - 1), 1, (own + kMqStep - 1) / kMqStep * kMqStep * NW);
+      const float best = -wave_max(-cost);
+      wave_runs = best < keys(n_pc, RG, (own + kChunk - 1) / kChunk * kChunk);
+      if (wave_runs) {
+        n_pc = min(__builtin_ctzll(__ballot(cost == best)) + 1, p.n_splits - 1);
+        n_eff = n_pc + 1;
+      }
+    }
   } else {
     // the count whose busiest CU ends first, counted in keys (lane c - 1: c chunks): its items' keys,
     // what each chunk adds to the merge (0.3 - 0.5 us) and what every further item adds (~0.7 us; ~4 us
@@ -312,6 +335,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   for (int item = bid; item < n_items; item += grid) {
   if (item == bid) stamp(18);
   int kvh, r0, nr, CL, kbeg, kend, nact, slot, kv_seq, ctx_n;
+  bool own_run = false;  // [kbeg, kend) are this wave's alone
   const int rho = n / G;  // group row of this lane's query column
   if (plan) {  // (one item per workgroup)
     if (__builtin_amdgcn_readlane(ev, 2) != 1) continue;  // empty chunk
@@ -341,9 +365,9 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   if (item == bid) stamp(9);  // step rows / contexts known
   const int c_src = __shfl(cl, min(r0 + lane, 63), 64);
   const int c_own = lane < nr ? c_src : 0;
-  int ctxmax = c_own;
+  int ctxmax = 0;  // (scalars: lane shuffles here and below were 0.3 us of every workgroup's start)
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) ctxmax = max(ctxmax, __shfl_xor(ctxmax, o, 64));
+  for (int r = 0; r < RG; ++r) ctxmax = r < nr ? max(ctxmax, __builtin_amdgcn_readlane(cl, min(r0 + r, 63))) : ctxmax;
   if (item == bid) stamp(19);
   ctx_n = __shfl(c_own, rho, 64);  // its context (0 for padded columns)
 
@@ -353,27 +377,32 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   if (cascade && r0 < n_real) {
     // prefix chunks (slots 0 .. npa-1) over [0, P) for every row of the group; then one chunk per
     // sequence run j of the group with keys past P: [P, max ctx of the run), the other runs'
-    // columns masked (slot npa + its rank among such runs)
+    // columns masked (slot npa + its rank among such runs).  wave_runs: one chunk for all of them, wave w on run w (slot npa)
     const unsigned long long gm = (nr >= 64 ? ~0ull : ((1ull << nr) - 1ull)) << r0;
     const unsigned long long subs = (seq_starts & gm) | (1ull << r0);
-    const int run_of = __builtin_popcountll(subs & ((2ull << min(r0 + lane, 63)) - 1ull)) - 1;  // lane < nr
     const int nruns = __builtin_popcountll(subs);
     int own_mask = 0, my_max = 0;  // runs with own keys; this item's run's max context
-    const int j = chunk - n_pc;
-    for (int rr = 0; rr < nruns; ++rr) {
-      int cm = (lane < nr && run_of == rr) ? c_src : 0;
+    const int j = wave_runs ? w : chunk - n_pc;
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) cm = max(cm, __shfl_xor(cm, o, 64));
-      if (cm > P) own_mask |= 1 << rr;
-      if (rr == j) my_max = cm;
+    for (int r = 0; r < RG; ++r) {
+      const int row = min(r0 + r, 63), c = r < nr ? __builtin_amdgcn_readlane(cl, row) : 0;
+      const int run = __builtin_popcountll(subs & ((2ull << row) - 1ull)) - 1;
+      if (c > P) own_mask |= 1 << run;
+      if (run == j) my_max = max(my_max, c);
     }
     CL = ((P + n_pc - 1) / n_pc + kChunk - 1) / kChunk * kChunk;
     const int npa = (P + CL - 1) / CL;
-    nact = npa + __builtin_popcount(own_mask);
+    nact = npa + (wave_runs ? own_mask != 0 : __builtin_popcount(own_mask));
     if (chunk < n_pc) {
       kbeg = chunk * CL;
       if (kbeg >= P) continue;
       kend = min(P, kbeg + CL);
+    } else if (wave_runs && !((own_mask >> j) & 1)) {
+      if (!own_mask) continue;
+      kbeg = kend = P;  // (no keys for this wave: it only takes part in the merge)
+      own_run = true;
+      slot = npa;
+      ctx_n = 0;
     } else {
       if (j >= nruns || !((own_mask >> j) & 1)) continue;
       unsigned long long sb = subs;
@@ -384,7 +413,8 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       kbeg = P;
       kend = my_max;
       CL = (kend - kbeg + kChunk - 1) / kChunk * kChunk;
-      slot = npa + __builtin_popcount(own_mask & ((1 << j) - 1));
+      own_run = wave_runs;
+      slot = npa + (wave_runs ? 0 : __builtin_popcount(own_mask & ((1 << j) - 1)));
       kv_seq = __shfl(sl, a, 64);
       if (rho < a - r0 || rho >= b - r0) ctx_n = 0;  // other runs' columns: no keys in this chunk
     }
@@ -403,8 +433,8 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   }  // (metadata path)
   // non-FINE: wave w takes the contiguous CL / NW keys from wb; FINE: the chunk's 32-key steps
   // round-robin over the waves (step s of the chunk -> wave s % NW)
-  const int wb = FINE ? kbeg : kbeg + w * (CL / kWv);
-  const int we = FINE ? kend : min(kend, wb + CL / kWv);
+  const int wb = FINE || own_run ? kbeg : kbeg + w * (CL / kWv);
+  const int we = FINE || own_run ? kend : min(kend, wb + CL / kWv);
   const int nsteps = we > wb ? (we - wb + kMqStep - 1) / kMqStep : 0;
   const int kmax = kend - 1;  // keys past the chunk are clamped (finite data, masked scores)
   if (item == bid) stamp(20);

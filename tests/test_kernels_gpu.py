@@ -1169,6 +1169,41 @@ def test_decode_attention_shared_prefix(hd, nq, nkv, n_sess, P):
 
 
 
+@pytest.mark.parametrize("hd,nq,nkv", [(128, 32, 8), (128, 16, 2), (64, 32, 8)])
+@pytest.mark.parametrize("n_sess,P,own", [(32, 1024, 90), (30, 992, 1), (17, 96, 33), (64, 640, 100), (23, 1024, 0)])
+def test_decode_attention_wave_runs(hd, nq, nkv, n_sess, P, own):
+    """Many sessions behind one prefix, whose own keys are one chunk per row group, a wave to a session: own keys of every session,
+    of some, of none; runs of two and three rows across group borders; padded rows."""
+    bs, per = 16, 80
+    seqs, ctx = [], []
+    for s in range(n_sess):
+        o = 0 if own and s % 4 == 1 else own + (5 * s) % 31 if own else 0
+        for i in range(1 + (s % 7 == 3) + (s % 7 == 5) * 2):
+            if len(seqs) < 62:
+                seqs.append(s)
+                ctx.append(P + o + i if o else P)
+    n_real = len(seqs)
+    seqs, ctx = seqs + [0, 0], ctx + [1, 1]
+    blocks = 8 + n_sess * per
+    kc, vc = rnd(blocks, nkv, bs, hd), rnd(blocks, nkv, bs, hd)
+    table = (torch.randperm(blocks - 8, device=DEV)[: n_sess * per] + 8).to(torch.int32).view(n_sess, per).contiguous()
+    table[:, : P // bs] = table[0, : P // bs]
+    seq_ids, ctx_lens, shared = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in (seqs, ctx, [P, n_real]))
+    q = rnd(len(seqs), nq * hd)
+    cnt = torch.zeros(len(seqs) * nkv, dtype=torch.int32, device=DEV)
+    outs = []
+    for sh in (shared, None):
+        outs.append(torch.full_like(q, float("nan")))
+        ops.decode_attention(q, ops.KVLayout.paged(kc, vc, table), ctx_lens, seq_ids, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd,
+                             scale=hd ** -0.5, max_ctx=per * bs, out=outs[-1], counters=cnt, shared=sh)
+    torch.cuda.synchronize()
+    assert int(cnt.abs().sum()) == 0
+    exp = ref.decode_attention(q.cpu(), ops.KVLayout.paged(kc.cpu(), vc.cpu(), table.cpu()), ctx_lens.cpu(), seq_ids.cpu(), n_q_heads=nq,
+                               n_kv_heads=nkv, head_dim=hd, scale=hd ** -0.5, out=torch.empty(len(seqs), nq * hd, dtype=BF))
+    close(outs[0], exp, 2e-2)
+    close(outs[1], exp, 2e-2)
+
+
 @pytest.mark.parametrize("M", [17, 40, 85, 600])
 @pytest.mark.parametrize("wdt", ["bf16", "fp8"])
 def test_rms_statistics_handoff(M, wdt):
