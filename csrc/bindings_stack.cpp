@@ -234,6 +234,22 @@ int64_t max_tiles(int64_t max_ctx, int64_t window, int64_t keep) {
   return std::min(all, (keep + 15) / 16 + (window + 14) / 16 + 1);
 }
 
+// sizes and scratch of the rows form
+void rows_scratch(TalkAttnParams& p, int64_t n_rows, int64_t nq, int64_t max_ctx, const Tensor& s, const Tensor& stat, const Tensor& part,
+                  Tensor& counters) {
+  p.nq = (int)nq;
+  p.rows = (int)n_rows;
+  const int64_t R = p.H / p.G, ct = talk_chunk_tiles(p.H, p.groups != nullptr);
+  const int64_t nch = (max_tiles(max_ctx, p.window > 0 ? p.window + nq - 1 : 0, p.keep) + ct - 1) / ct;
+  p.nch = (int)nch;
+  p.s = f32p(s, n_rows * nq * p.H * nch * ct * 16, "s");
+  p.nst = (int)(nch * ct / kTalkStat);
+  p.stat = f32p(stat, n_rows * nq * p.H * p.nst * 2, "stat");
+  p.part = f32p(part, n_rows * nq * nch * p.H * p.dv, "part");
+  i32p(counters, n_rows * p.G * ((R + 15) / 16), "counters");
+  p.counters = counters.data_ptr<int>();
+}
+
 void talk_attention(Tensor q, Tensor k, Tensor v, Tensor table, Tensor positions, Tensor seq_ids, Tensor slots,
                     c10::optional<Tensor> row_list, int64_t n_rows, int64_t H, double scale, int64_t window, int64_t keep,
                     c10::optional<Tensor> talk, c10::optional<Tensor> gate, double out_scale, int64_t max_ctx, Tensor s,
@@ -254,17 +270,7 @@ void talk_attention(Tensor q, Tensor k, Tensor v, Tensor table, Tensor positions
   } else {
     nq = 1;
   }
-  p.nq = (int)nq;
-  p.rows = (int)n_rows;
-  const int64_t ct = talk_chunk_tiles((int)H, groups.has_value());
-  const int64_t nch = (max_tiles(max_ctx, window > 0 ? window + nq - 1 : 0, keep) + ct - 1) / ct;
-  p.nch = (int)nch;
-  p.s = f32p(s, n_rows * nq * H * nch * ct * 16, "s");
-  p.nst = (int)(nch * ct / kTalkStat);
-  p.stat = f32p(stat, n_rows * nq * H * p.nst * 2, "stat");
-  p.part = f32p(part, n_rows * nq * nch * H * p.dv, "part");
-  i32p(counters, n_rows * p.G * ((R + 15) / 16), "counters");
-  p.counters = counters.data_ptr<int>();
+  rows_scratch(p, n_rows, nq, max_ctx, s, stat, part, counters);
   check_rc(vwa_talk_attention(&p, cur_stream(q)), "talk_attention");
 }
 
@@ -364,6 +370,22 @@ void qkv_mingru(Tensor x, int64_t H, int64_t G, int64_t dk, int64_t dv, int64_t 
   check_rc(vwa_qkv_mingru(&p, &m, cur_stream(x)), "qkv_mingru");
 }
 
+// a decode step's rows: qkv_mingru and the rows-form attention over them (arguments of both)
+void talk_step(Tensor x, int64_t H, int64_t rot_dims, Tensor rope, Tensor positions, Tensor seq_ids, Tensor slots, Tensor q_out, Tensor k,
+               Tensor v, Tensor z, Tensor u, Tensor gt, c10::optional<Tensor> zb, c10::optional<Tensor> xb, Tensor state, double rec_scale,
+               Tensor rec_out, Tensor table, double scale, int64_t window, int64_t keep, c10::optional<Tensor> talk,
+               c10::optional<Tensor> gate, double out_scale, int64_t max_ctx, Tensor s, Tensor stat, Tensor part, Tensor counters,
+               Tensor out) {
+  c10::DeviceGuard g(x.device());
+  TORCH_CHECK(k.dim() == 4 && v.dim() == 4, "caches must be 4-D");
+  const QkvCacheParams qc = qkv_params(x, H, k.size(1), k.size(3), v.size(2), rot_dims, rope, positions, slots, q_out, k, v);
+  const MinGruParams m = mingru_params(z, u, gt, zb, xb, seq_ids, positions, slots, state, rec_scale, rec_out);
+  TalkAttnParams p = attn_params(q_out, k, v, table, positions, seq_ids, slots, qc.rows, H, scale, window, keep, talk, gate, out_scale, out);
+  TORCH_CHECK(max_ctx >= 1 && max_ctx <= table.size(1) * k.size(2), "max_ctx exceeds the block table");
+  rows_scratch(p, qc.rows, 1, max_ctx, s, stat, part, counters);
+  check_rc(vwa_talk_step(&p, &qc, &m, cur_stream(x)), "talk_step");
+}
+
 }  // namespace
 
 void bind_stack(py::module_& m) {
@@ -375,6 +397,7 @@ void bind_stack(py::module_& m) {
   m.def("embedding_f32", &embedding_f32);
   m.def("qkv_cache", &qkv_cache);
   m.def("qkv_mingru", &qkv_mingru);
+  m.def("talk_step", &talk_step);
   m.def("talk_prefill_part", [](int64_t H, int64_t G, int64_t dk, int64_t dv) {
     return vwa_talk_prefill_part((int)H, (int)G, (int)dk, (int)dv);
   });

@@ -6,6 +6,7 @@
 //  qkv_cache     : partial rotation of q / k heads + paged cache write (V transposed inside a block)
 //  qkv_mingru    : qkv_cache and the recurrence's rows form of a decode step in one launch
 #include "mixer_kernels.h"
+#include "qkv_rows.h"
 #include "recurrence.h"
 
 using namespace vwa;
@@ -248,60 +249,6 @@ __global__ __launch_bounds__(256) void embedding_f32_kernel(const int* __restric
   const int c = blockIdx.y * 256 + threadIdx.x;
   if (c < Dpad)
     out[(size_t)row * ldo + c] = ok && c < D ? ldv(table + (size_t)id * ld + c) * scale : 0.f;
-}
-
-// Part of one row.  VEC consecutive dimensions per thread (8 when the half rotation is a
-// multiple of 8, else 1): a rotated chunk reads its partner chunk rot_dims / 2 away.
-template <class T, int VEC>
-VWA_DEVICE void qkv_cache_row(const QkvCacheParams& p, int row, int part, int parts) {
-  const T* x = reinterpret_cast<const T*>(p.x) + (size_t)row * p.ldx;
-  const int64_t slot = p.slots[row];
-  const int pos = min(max(p.positions[row], 0), p.max_pos - 1);
-  const int64_t blk = slot >= 0 ? slot / p.block_size : 0;
-  const int off = slot >= 0 ? (int)(slot % p.block_size) : 0;
-  const int half = p.rot_dims >> 1;
-  const float* cs = p.rope + (size_t)pos * p.rot_dims;
-  const int cph = p.dk / VEC, nqk = (p.H + p.G) * cph;
-  T* kc = reinterpret_cast<T*>(p.k) + blk * p.k_sb + (int64_t)off * p.dk;
-  for (int u = part * 256 + threadIdx.x; u < nqk; u += parts * 256) {
-    const int head = u / cph, e = (u % cph) * VEC;
-    const T* xh = x + head * p.dk;
-    float o[VEC];
-    if (e < p.rot_dims) {
-      const bool hi = e >= half;
-      const int i0 = hi ? e - half : e, pe = hi ? e - half : e + half;
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        const float a = ldv(xh + e + j), b = ldv(xh + pe + j);
-        const float c = cs[2 * (i0 + j)], s = cs[2 * (i0 + j) + 1];
-        o[j] = hi ? a * c + b * s : a * c - b * s;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) o[j] = ldv(xh + e + j);
-    }
-    T* dst;
-    if (head < p.H) {
-      dst = reinterpret_cast<T*>(p.q_out) + (size_t)row * p.ldq + head * p.dk + e;
-    } else {
-      if (slot < 0) continue;
-      dst = kc + (int64_t)(head - p.H) * p.k_sh + e;
-    }
-    if constexpr (VEC == 8) {
-      const float lo[4] = {o[0], o[1], o[2], o[3]}, hi4[4] = {o[4], o[5], o[6], o[7]};
-      st4(dst, lo);
-      st4(dst + 4, hi4);
-    } else {
-      stv(dst, o[0]);
-    }
-  }
-  if (slot < 0) return;
-  const T* xv = x + (p.H + p.G) * p.dk;
-  T* vc = reinterpret_cast<T*>(p.v) + blk * p.v_sb + off;
-  for (int u = part * 256 + threadIdx.x; u < p.G * p.dv; u += parts * 256) {
-    const int g = u / p.dv, d = u % p.dv;
-    vc[(int64_t)g * p.v_sh + (int64_t)d * p.block_size] = xv[u];
-  }
 }
 
 template <class T, int VEC>

@@ -20,6 +20,8 @@
 //     the weights passing between the waves through LDS in B-operand order.
 #include "common.h"
 #include "mq_attention.h"
+#include "qkv_rows.h"
+#include "recurrence.h"
 #include "stack_kernels.h"
 #include "stack_types.h"
 
@@ -95,6 +97,61 @@ VWA_DEVICE Unit unit_of(const TalkAttnParams& p, int ri) {
   return u;
 }
 
+// Steps of the head dimension whose operands are requested together: 128 dimensions.  (A loop over them unrolled eight times ran
+// the four of bf16 one after another, in its remainder.)
+template <class T>
+constexpr int kScoreStep = 128 / MM<T>::KS;
+
+// A workgroup's scores of its wave's tiles, masked, and their statistics over the workgroup
+template <bool GRP, int NU>
+VWA_DEVICE void store_scores(const TalkAttnParams& p, const Unit& un, int ri, int qi, int h, bool col, int chunk, const int (&key0)[NU],
+                             const bool (&ok)[NU], f32x4 (&acc)[NU], float (&sm)[4][16][2]) {
+  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, b = lane >> 4;
+  // lane (column rl, keys 4b .. 4b+3 of its tiles): mask, store, chunk statistics
+  float mx = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const bool vis = ok[u] && sees(un.pos + qi, key0[u] + 4 * b + i, p.window, p.keep);
+      acc[u][i] = vis ? acc[u][i] * p.scale : -INFINITY;
+      mx = fmaxf(mx, acc[u][i]);
+    }
+  const size_t srow = (size_t)ri * p.nq + qi;         // scratch row
+  if (col) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+      if (ok[u])
+        *reinterpret_cast<float4*>(p.s + (srow * p.H + h) * p.nst * (kTalkStat * kTile) +
+                                   (chunk * kTalkStat + w + 4 * u) * kTile + 4 * b) =
+            make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
+  }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  float l = 0.f;
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) l += acc[u][i] == -INFINITY ? 0.f : __expf(acc[u][i] - mx);
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (b == 0) {
+    sm[w][rl][0] = mx;
+    sm[w][rl][1] = l;
+  }
+  lds_sync();
+  if (threadIdx.x < 16 && col) {                       // (thread = column: its qi and r)
+    float m = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m = fmaxf(m, sm[i][rl][0]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum += sm[i][rl][1] > 0.f ? sm[i][rl][1] * __expf(sm[i][rl][0] - m) : 0.f;
+    float* st = p.stat + ((srow * p.H + h) * p.nst + chunk) * 2;
+    st[0] = m;
+    st[1] = sum;
+  }
+}
+
 template <class T, bool GRP>
 __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
   using M = MM<T>;
@@ -125,54 +182,131 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
             (int64_t)((key0[u] & (p.block_size - 1)) + rl) * p.dk + b * M::EPL;
   }
   f32x4 acc[NU] = {};
-#pragma unroll 8
-  for (int k = 0; k < p.dk; k += M::KS) {
-    const uint4 qf = *reinterpret_cast<const uint4*>(q + k);
+  constexpr int NB = kScoreStep<T>;
+  for (int k0 = 0; k0 < p.dk; k0 += NB * M::KS) {
+    uint4 qf[NB], kf[NU][NB];
 #pragma unroll
-    for (int u = 0; u < NU; ++u) acc[u] = M::mma(*reinterpret_cast<const uint4*>(kp[u] + k), qf, acc[u]);
-  }
-  // lane (column rl, keys 4b .. 4b+3 of its tiles): mask, store, chunk statistics
-  float mx = -INFINITY;
+    for (int s = 0; s < NB; ++s) {
+      const int k = min(k0 + s * M::KS, p.dk - M::KS);
+      qf[s] = *reinterpret_cast<const uint4*>(q + k);
 #pragma unroll
-  for (int u = 0; u < NU; ++u)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const bool vis = ok[u] && sees(un.pos + qi, key0[u] + 4 * b + i, p.window, p.keep);
-      acc[u][i] = vis ? acc[u][i] * p.scale : -INFINITY;
-      mx = fmaxf(mx, acc[u][i]);
+      for (int u = 0; u < NU; ++u) kf[u][s] = *reinterpret_cast<const uint4*>(kp[u] + k);
     }
-  const size_t srow = (size_t)ri * p.nq + qi;         // scratch row
-  if (col) {
 #pragma unroll
-    for (int u = 0; u < NU; ++u)
-      if (ok[u])
-        *reinterpret_cast<float4*>(p.s + (srow * p.H + c * R + r0 + r) * p.nst * (kTalkStat * kTile) +
-                                   (chunk * kTalkStat + w + 4 * u) * kTile + 4 * b) =
-            make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
+    for (int s = 0; s < NB; ++s)
+      if (k0 + s * M::KS < p.dk) {
+#pragma unroll
+        for (int u = 0; u < NU; ++u) acc[u] = M::mma(kf[u][s], qf[s], acc[u]);
+      }
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  float l = 0.f;
-#pragma unroll
-  for (int u = 0; u < NU; ++u)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) l += acc[u][i] == -INFINITY ? 0.f : __expf(acc[u][i] - mx);
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
-  if (b == 0) {
-    sm[w][rl][0] = mx;
-    sm[w][rl][1] = l;
+  store_scores<GRP, NU>(p, un, ri, qi, c * R + r0 + r, col, chunk, key0, ok, acc, sm);
+}
+
+// ---- a decode step's scores behind nothing but its projections
+// What qkv_mingru does ahead of the scores (heads turned, keys and values into the cache, the recurrence) in the scores' launch: a
+// launch of round trips less per layer.  The scoring workgroups turn their query themselves, and of the keys that belong to this
+// step's rows of their sequence -- those other workgroups of the launch are writing to the cache -- they turn the projections; every
+// other key comes from the cache.  The first workgroups write the cache and run the recurrence.
+// us, both launches -> this one: 1 row of 225 keys, 16 / 4 heads of 128 and 2048 channels 9.4 -> 5.9; 48 rows of 90 .. 250 keys, 8 / 4
+// heads and 1024 channels 10.9 -> 8.6.  The row's query and own key are turned once a workgroup, through LDS: every wave for itself
+// took 6.6 and 10.7 (94 registers, and the table's row four times).  Bound by its round trips: ids and positions, table, keys.
+constexpr int kStepParts = 2;                        // workgroups of a row's keys and values
+// Scoring workgroups of a launch at most: as many as are resident at once beside the others.  Each row's walk its chunks; one a
+// chunk of the longest context would be mostly workgroups without keys (48 rows of 2048: 3840, 11.1 -> 10.7 us).
+constexpr int kStepWgs = 768;
+
+template <class T>
+__global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, QkvCacheParams qc, MinGruParams g, int per_row) {
+  using M = MM<T>;
+  static_assert(kTalkStat == 4, "a tile per wave");
+  constexpr int NB = kScoreStep<T>;
+  __shared__ float sm[4][16][2];
+  __shared__ uint4 qs[NB][64], ks[NB][4];            // the query's fragments; those of the row's own key
+  const int parts = kStepParts + (g.width + 255) / 256, n_parts = parts * p.rows;
+  if ((int)blockIdx.x < n_parts) {
+    const int row = blockIdx.x / parts, part = blockIdx.x % parts;
+    if (part < kStepParts) qkv_cache_row<T, 8>(qc, row, part, kStepParts, p.H);
+    else mingru_row<T>(g, row, (part - kStepParts) * 256 + threadIdx.x);
+    return;
   }
-  lds_sync();
-  if (threadIdx.x < 16 && col) {                       // (thread = column: its qi and r)
-    float m = -INFINITY, sum = 0.f;
+  const int R = p.H / p.G, nz = (R + 15) / 16, bid = blockIdx.x - n_parts;
+  const int rg = bid % (p.rows * p.G), cz = bid / (p.rows * p.G);
+  const int ri = rg / p.G, c = rg % p.G, r0 = cz % nz * 16;
+  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, b = lane >> 4;
+  // the step's rows, one a lane: this row's place, and the first row of its run (rows of one sequence, at consecutive positions)
+  const int lr = min(lane, p.rows - 1);
+  const int64_t slot_l = p.slots[lr];
+  const int pos_l = p.positions[lr], seq_l = p.seq_ids[lr];
+  const int before = __shfl_up(seq_l, 1, 64), inert = __shfl_up((int)(slot_l < 0), 1, 64);
+  const unsigned long long heads = __ballot(lane == 0 || before != seq_l || inert);
+  if (!((__ballot(slot_l >= 0) >> ri) & 1)) return;
+  const int head = 63 - __builtin_clzll(heads & ((2ull << ri) - 1ull));
+  Unit un;
+  un.row = ri;
+  un.cnt = 1;
+  un.live = true;
+  un.pos = __builtin_amdgcn_readlane(pos_l, ri);
+  un.seq = __builtin_amdgcn_readlane(seq_l, ri);
+  un.v = vis_tiles(un.pos, un.pos, p.window, p.keep);
+  un.v.n = min(un.v.n, p.nst * kTalkStat);
+  const Vis v = un.v;
+  const int fresh = __builtin_amdgcn_readlane(pos_l, head);  // keys fresh .. un.pos are rows head .. ri
+  const int Rb = min(16, R - r0);
+  const T* x = reinterpret_cast<const T*>(qc.x);
+  const T* xq = x + (size_t)ri * qc.ldx + (size_t)(c * R + r0 + min(rl, Rb - 1)) * p.dk;
+  const T* xk = x + (size_t)ri * qc.ldx + (size_t)(p.H + c) * p.dk;
+  auto table_row = [&](int pos) { return qc.rope + (size_t)min(max(pos, 0), qc.max_pos - 1) * qc.rot_dims; };
+  const float* cq = table_row(un.pos);
+  const int lb = __builtin_ctz(p.block_size);
+  const int e0 = b * M::EPL;
+  bool have_q = false;
+  for (int chunk = cz / nz; chunk * kTalkStat < v.n; chunk += per_row) {
+    const int t = chunk * kTalkStat + w;
+    const bool ok[1] = {t < v.n};
+    const int key0[1] = {tile_of(v, ok[0] ? t : v.n - 1) * kTile}, key = key0[0] + rl;
+    const int64_t blk = p.block_table[(int64_t)un.seq * p.table_stride + (key0[0] >> lb)];
+    f32x4 acc[1] = {};
+    for (int k0 = 0; k0 < p.dk; k0 += NB * M::KS) {
+      const bool new_q = !have_q || p.dk > NB * M::KS;
+      if (have_q && new_q) lds_sync();                   // (the fragments before are read)
+      if (new_q) {
+#pragma unroll 1
+        for (int s = w; s < NB && k0 + s * M::KS < p.dk; s += 4) {
+          const uint4 fq = turned_frag(xq, k0 + s * M::KS + e0, qc.rot_dims, cq);
+          const uint4 fk = turned_frag(xk, k0 + s * M::KS + e0, qc.rot_dims, cq);
+          qs[s][lane] = fq;
+          ks[s][b] = fk;                                 // (the same of 16 lanes)
+        }
+      }
+      const T* kp = reinterpret_cast<const T*>(p.k) + blk * p.k_sb + (int64_t)c * p.k_sh +
+                    (int64_t)((key0[0] & (p.block_size - 1)) + rl) * p.dk + e0;
+      auto product = [&](const uint4& cached, int s) {
+        const uint4 own = ks[s][b];
+        acc[0] = M::mma(key == un.pos ? own : cached, qs[s][lane], acc[0]);
+      };
+      if (key0[0] + kTile <= fresh || fresh == un.pos) {
+        uint4 kf[NB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) m = fmaxf(m, sm[i][rl][0]);
+        for (int s = 0; s < NB; ++s) kf[s] = *reinterpret_cast<const uint4*>(kp + min(k0 + s * M::KS, p.dk - M::KS));
+        if (new_q) lds_sync();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sum += sm[i][rl][1] > 0.f ? sm[i][rl][1] * __expf(sm[i][rl][0] - m) : 0.f;
-    float* st = p.stat + ((srow * p.H + c * R + r0 + r) * p.nst + chunk) * 2;
-    st[0] = m;
-    st[1] = sum;
+        for (int s = 0; s < NB; ++s)
+          if (k0 + s * M::KS < p.dk) product(kf[s], s);
+      } else {                                           // keys of the run's rows in front of this one
+        const bool mine = key >= fresh && key < un.pos;  // (keys past the row's are masked)
+        const T* xr = x + (size_t)(mine ? head + key - fresh : ri) * qc.ldx + (size_t)(p.H + c) * p.dk;
+        const float* ck = table_row(mine ? key : un.pos);
+        if (new_q) lds_sync();
+#pragma unroll 1
+        for (int s = 0; s < NB && k0 + s * M::KS < p.dk; ++s) {
+          const uint4 old = *reinterpret_cast<const uint4*>(kp + k0 + s * M::KS), now = turned_frag(xr, k0 + s * M::KS + e0, qc.rot_dims, ck);
+          product(mine ? now : old, s);
+        }
+      }
+      have_q = true;
+    }
+    store_scores<false, 1>(p, un, ri, 0, c * R + r0 + rl, rl < Rb, chunk, key0, ok, acc, sm);
+    if ((chunk + per_row) * kTalkStat < v.n) lds_sync();  // (the statistics' LDS is written again)
   }
 }
 
@@ -860,11 +994,15 @@ int check_attn(const TalkAttnParams& p) {
 }
 
 template <class T, int CT, bool GRP>
-int launch_rows(const TalkAttnParams& p, hipStream_t st) {
+int launch_rows(const TalkAttnParams& p, hipStream_t st, const QkvCacheParams* qc = nullptr, const MinGruParams* g = nullptr) {
   const size_t lds = mix_lds<T, CT>(p.H, p.nq);
   if (lds > kMaxLds - 64) return -5;
   const int nz = (p.H / p.G + 15) / 16;
-  hipLaunchKernelGGL((talk_scores_kernel<T, GRP>), dim3(p.rows * p.G, p.nst, nz), dim3(256), 0, st, p);
+  if (qc) {
+    const int n = p.rows * p.G * nz, per_row = p.nst < kStepWgs / n ? p.nst : kStepWgs / n > 1 ? kStepWgs / n : 1;
+    hipLaunchKernelGGL((talk_step_kernel<T>), dim3(p.rows * (kStepParts + (g->width + 255) / 256) + n * per_row), dim3(256), 0, st, p, *qc, *g, per_row);
+  } else
+    hipLaunchKernelGGL((talk_scores_kernel<T, GRP>), dim3(p.rows * p.G, p.nst, nz), dim3(256), 0, st, p);
   hipLaunchKernelGGL((talk_mix_kernel<T, CT, GRP>), dim3(p.rows * p.G, p.nch, nz), dim3(64 * kWaves), lds, st, p);
   return (int)hipGetLastError();
 }
@@ -883,6 +1021,20 @@ extern "C" int vwa_talk_attention(const TalkAttnParams* p, hipStream_t st) {
   if (p->nq != 1) return -6;
   if (talk_chunk_tiles(p->H, 0) == 16) return p->f32 ? launch_rows<float, 16, false>(*p, st) : launch_rows<u16, 16, false>(*p, st);
   return p->f32 ? launch_rows<float, 8, false>(*p, st) : launch_rows<u16, 8, false>(*p, st);
+}
+
+extern "C" int vwa_talk_step(const TalkAttnParams* p, const QkvCacheParams* qc, const MinGruParams* g, hipStream_t st) {
+  const int rc = check_attn(*p);
+  if (rc) return rc;
+  if (p->nch < 1 || p->nst < 1 || !p->s || !p->stat || !p->part || !p->counters) return -4;
+  if (p->nq != 1 || p->groups || p->row_list || (int64_t)p->nch * p->H * p->dv * 4 >= (1ll << 31)) return -5;
+  if (p->rows > 64 || qc->rows != p->rows || g->rows != p->rows || g->width < 1 || qc->f32 != p->f32 || g->f32 != p->f32) return -6;
+  if (qc->H != p->H || qc->G != p->G || qc->dk != p->dk || qc->dv != p->dv || qc->k != p->k || qc->v != p->v ||
+      qc->block_size != p->block_size) return -7;
+  if (qc->rot_dims < 16 || qc->rot_dims > qc->dk || qc->rot_dims % 16 || qc->max_pos < 1 || qc->ldx % 8 ||
+      ((reinterpret_cast<uintptr_t>(qc->rope) | reinterpret_cast<uintptr_t>(qc->x)) & 15)) return -8;
+  if (talk_chunk_tiles(p->H, 0) == 16) return p->f32 ? launch_rows<float, 16, false>(*p, st, qc, g) : launch_rows<u16, 16, false>(*p, st, qc, g);
+  return p->f32 ? launch_rows<float, 8, false>(*p, st, qc, g) : launch_rows<u16, 8, false>(*p, st, qc, g);
 }
 
 extern "C" int64_t vwa_talk_prefill_part(int H, int G, int dk, int dv) {

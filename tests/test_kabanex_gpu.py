@@ -397,6 +397,65 @@ def test_mingru(dtype, W):
         assert rel(st, end) < 1e-5 and out[:, W:].abs().sum() == 0
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("H,G,dk,dv,rot,window,keep,bs", [
+    (8, 4, 128, 128, 64, 1024, 4, 16),
+    (6, 2, 32, 48, 16, 33, 3, 16),        # half of a fragment step rotates
+    (20, 1, 64, 16, 64, 0, 0, 32),        # two column groups; every dimension rotates
+    (4, 4, 96, 32, 32, 1, 17, 16),        # a window of one behind kept keys
+])
+def test_talk_mingru_step(dtype, H, G, dk, dv, rot, window, keep, bs):
+    """A decode step's two launches against the ops they stand for, over one set of caches: single rows, runs that start at 0, end
+    at, start at and cross tile borders, a run of two chunks of tiles, inert rows between and behind them.  The cache's places of
+    the step's own keys and of keys past them hold NaN before the step: the scores may take nothing from there."""
+    W, n_seq, per = 40, 7, 24
+    runs = [(3, 0, 1), (0, 31, 1), (5, 0, 18), (1, 90, 16), (2, 47, 2), (6, 200, 1), (4, 16, 5)]  # sequence, first position, rows
+    ids, pos = [], []
+    for s, p0, n in runs:
+        ids += [s] * n
+        pos += range(p0, p0 + n)
+    rows = len(ids) + 2
+    live = torch.tensor([True] * 20 + [False] + [True] * (len(ids) - 20) + [False])
+    ids, pos = ids[:20] + [5] + ids[20:] + [0], pos[:20] + [0] + pos[20:] + [0]
+    table = torch.randperm(n_seq * per, generator=torch.Generator().manual_seed(2)).int().view(n_seq, per)
+    posT, idT = torch.tensor(pos), torch.tensor(ids)
+    slots = torch.where(live, table[idT, posT // bs].long() * bs + posT % bs, -1)
+    kc, vc = rnd(n_seq * per, G, bs, dk, seed=1, dtype=dtype), rnd(n_seq * per, G, dv, bs, seed=2, dtype=dtype)
+    for s, p0, n in runs:
+        for p in range(p0, min(per * bs, p0 + n + 40)):
+            kc[table[s, p // bs], :, p % bs] = float("nan")
+    A = H * dk + G * (dk + dv)
+    y = rnd(rows, -(-(A + 3 * W + H) // 8) * 8, seed=3, dtype=dtype).to(DEV)
+    at = (A, A + W, A + 2 * W)
+    T, zb, xb, st = (rnd(*n, seed=i).to(DEV) for i, n in enumerate(((H, H), (W,), (W,), (n_seq, W))))
+    rope = ops.rope_table(512, rot, 10000.0, device=DEV)
+    sc = ops.TalkScratch([(H, G, dv, window, keep)], per * bs, DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    meta = dict(positions=i32(pos), seq_ids=i32(ids), slots=slots.to(DEV))
+    head = dict(n_q_heads=H, rot_dims=rot, rope=rope)
+    att = dict(scale=0.4, window=window, keep=keep, talk=T, talk_frag=None, gate=y[:, A + 3 * W : A + 3 * W + H], out_scale=0.8,
+               max_ctx=per * bs, scratch=sc)
+
+    def run(fused):
+        c = dict(k_cache=kc.clone().to(DEV), v_cache=vc.clone().to(DEV), state=st.clone())
+        q, rec = torch.zeros(rows, H * dk, dtype=dtype, device=DEV), torch.zeros(rows, W, dtype=dtype, device=DEV)
+        out = torch.full((rows, H * dv), float("nan"), dtype=dtype, device=DEV)
+        if fused:
+            ops.talk_mingru_step(y, at, zb, xb, table.to(DEV), **head, q_out=q, rec_scale=0.7, rec_out=rec, out=out, **c, **meta, **att)
+        else:
+            ops.qkv_cache_mingru(y, at, zb, xb, **head, q_out=q, out_scale=0.7, out=rec, **c, **meta)
+            ops.talk_attention(q, c["k_cache"], c["v_cache"], table.to(DEV), n_q_heads=H, out=out, **meta, **att)
+        torch.cuda.synchronize()
+        return out, rec, c["state"], c["k_cache"], c["v_cache"]
+
+    want, got = run(False), run(True)
+    for a, b in zip(got[1:], want[1:]):
+        assert torch.equal(torch.nan_to_num(a.float(), 1e9), torch.nan_to_num(b.float(), 1e9))
+    # (the turned heads may differ by a contraction: the bounds of the attention's own test)
+    assert rel(got[0], want[0].cpu()) < (5e-6 if dtype == F32 else 1.5e-2)
+    assert got[0][~live].abs().sum() == 0 and sc.counters.abs().sum() == 0
+
+
 # ----------------------------------------------------------------------------- the model through the engine
 CFGS = {
     "odd": O.model_config(72, 101, [

@@ -239,14 +239,12 @@ class KabanexModel:
         r_at, f_at = D.heads_out, D.heads_out + D.w
         ops.linear_split(h, L.w_in, y, cat[:, f_at : f_at + D.f] if D.f else None)
         W = C.right.width
-        q = ops.qkv_cache_mingru(y, (z0, x0, r0), L.zb, L.xb, n_q_heads=D.H, rot_dims=a.rot_dims,
-                                 rope=self.ropes[(a.rot_base, a.rot_dims)], q_out=bufs.q[: M * D.H * D.dk].view(M, D.H * D.dk),
-                                 k_cache=kv.k[li], v_cache=kv.v[li], state=kv.state[li], out_scale=C.right_scale,
-                                 out=cat[:, r_at : r_at + W], plan=plan, **rows)
-        ops.talk_attention(q, kv.k[li], kv.v[li], bufs.block_table, n_q_heads=D.H, scale=a.scale, window=a.window,
-                           keep=a.keep_first, talk=L.talk, talk_frag=L.talk_frag, gate=y[:, g0 : g0 + D.gate],
-                           out_scale=C.left_scale, max_ctx=bufs.max_ctx, scratch=bufs.talk, out=cat[:, : D.heads_out],
-                           plan=plan, **rows)
+        ops.talk_mingru_step(y, (z0, x0, r0), L.zb, L.xb, bufs.block_table, n_q_heads=D.H, rot_dims=a.rot_dims,
+                             rope=self.ropes[(a.rot_base, a.rot_dims)], q_out=bufs.q[: M * D.H * D.dk].view(M, D.H * D.dk),
+                             k_cache=kv.k[li], v_cache=kv.v[li], state=kv.state[li], rec_scale=C.right_scale,
+                             rec_out=cat[:, r_at : r_at + W], scale=a.scale, window=a.window, keep=a.keep_first, talk=L.talk,
+                             talk_frag=L.talk_frag, gate=y[:, g0 : g0 + D.gate], out_scale=C.left_scale, max_ctx=bufs.max_ctx,
+                             scratch=bufs.talk, out=cat[:, : D.heads_out], plan=plan, **rows)
         last = li + 1 == self.cfg.n_layers
         parts = None if last else ops.linear_parts(cat, L.w_out)  # (few rows: K slices, which the norm adds to x)
         if parts is None:

@@ -259,6 +259,29 @@ def talk_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     return out
 
 
+def talk_mingru_step(y: torch.Tensor, at: Tuple[int, int, int], zb: torch.Tensor, xb: torch.Tensor, block_table: torch.Tensor, *,
+                     n_q_heads: int, rot_dims: int, rope: torch.Tensor, positions: torch.Tensor, seq_ids: torch.Tensor,
+                     slots: torch.Tensor, q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, state: torch.Tensor,
+                     rec_scale: float, rec_out: torch.Tensor, scale: float, window: int, keep: int, talk: Optional[torch.Tensor],
+                     talk_frag: Optional[torch.Tensor], gate: Optional[torch.Tensor], out_scale: float, max_ctx: int,
+                     scratch: Optional[TalkScratch], out: torch.Tensor, plan: Optional[SimpleNamespace] = None) -> torch.Tensor:
+    """qkv_cache_mingru of a layer's projected rows and talk_attention over them.  A decode step on the GPU whose rows' heads
+    rotate by 16-byte pieces takes the attention's two launches for all of it (q_out is not written then)."""
+    W = state.shape[1]
+    if y.is_cuda and plan is None and y.shape[0] <= ROW_SLICE and rot_dims >= 16 and rot_dims % 16 == 0 and y.stride(0) % 8 == 0:
+        z, x, g = (y[:, a : a + W] for a in at)
+        _ext().talk_step(y, n_q_heads, rot_dims, rope, positions, seq_ids, slots, q_out, k_cache, v_cache, z, x, g, zb, xb, state,
+                         rec_scale, rec_out, block_table, scale, window, keep, talk, gate, out_scale, max_ctx, scratch.s,
+                         scratch.stat, scratch.part, scratch.counters, out)
+        return out
+    q = qkv_cache_mingru(y, at, zb, xb, n_q_heads=n_q_heads, rot_dims=rot_dims, rope=rope, positions=positions, seq_ids=seq_ids,
+                         slots=slots, q_out=q_out, k_cache=k_cache, v_cache=v_cache, state=state, out_scale=rec_scale, out=rec_out,
+                         plan=plan)
+    return talk_attention(q, k_cache, v_cache, block_table, positions, seq_ids, slots, n_q_heads=n_q_heads, scale=scale,
+                          window=window, keep=keep, talk=talk, talk_frag=talk_frag, gate=gate, out_scale=out_scale,
+                          max_ctx=max_ctx, scratch=scratch, out=out, plan=plan)
+
+
 def prefill_splits(n_tiles: int, max_pos: int, window: int, keep: int, cus: int) -> int:
     """Workgroups per 16-query tile over its keys: enough to give every CU one, and no more than leaves
     each a round of its waves (128 keys)."""
