@@ -16,7 +16,7 @@ const void* frag(const Tensor& w, bool f32, int64_t n, const char* name) {
 // y | x projections [rows, 2 width]; conv [taps, width]; state [slots, taps * width]; chunks / scratch: scan form
 void rglru(Tensor yx, Tensor yb, Tensor xb, Tensor cw, Tensor cb, Tensor gw, Tensor rb, Tensor ib, Tensor decay, int64_t nb,
            Tensor seq_ids, Tensor positions, Tensor slots, Tensor state, Tensor out, OptTensor chunks, OptTensor scratch,
-           OptTensor u) {
+           OptTensor u, OptTensor tickets) {
   c10::DeviceGuard g(yx.device());
   const bool f32 = t_is_f32(yx, "yx");
   const int64_t rows = out.size(0), W = decay.numel();
@@ -58,6 +58,10 @@ void rglru(Tensor yx, Tensor yb, Tensor xb, Tensor cw, Tensor cb, Tensor gw, Ten
   p.ldo = (int)out.stride(0);
   if (!chunks.has_value()) {
     TORCH_CHECK(rows <= 64, "rows form: at most 64 rows");
+    if (tickets.has_value()) {
+      i32p(*tickets, nb * ((rows + 15) / 16), "tickets");
+      p.tickets = tickets->data_ptr<int>();
+    }
     check_rc(vwa_rglru_rows(&p, cur_stream(yx)), "rglru_rows");
     return;
   }
@@ -399,7 +403,7 @@ void moe_gemm(Tensor x, Tensor w, int64_t rows, int64_t top, bool down, Tensor w
 void bind_mixers(py::module_& m) {
   m.def("rglru", &rglru, py::arg("yx"), py::arg("yb"), py::arg("xb"), py::arg("cw"), py::arg("cb"), py::arg("gw"), py::arg("rb"),
         py::arg("ib"), py::arg("decay"), py::arg("nb"), py::arg("seq_ids"), py::arg("positions"), py::arg("slots"), py::arg("state"),
-        py::arg("out"), py::arg("chunks") = py::none(), py::arg("scratch") = py::none(), py::arg("u") = py::none());
+        py::arg("out"), py::arg("chunks") = py::none(), py::arg("scratch") = py::none(), py::arg("u") = py::none(), py::arg("tickets") = py::none());
   m.def("head_linear", &head_linear, py::arg("x"), py::arg("xs"), py::arg("w"), py::arg("nb"), py::arg("N"), py::arg("K"), py::arg("y"),
         py::arg("ys"), py::arg("row_list") = py::none());
   m.def("latent_rows", &latent_rows);

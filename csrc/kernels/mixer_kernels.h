@@ -25,6 +25,7 @@ struct RgLruParams {
   const int* seq_ids; const int* positions; const int64_t* slots;  // slot < 0: inert row (output zero, no state)
   float* state; int64_t state_ld;   // [state slots][taps * width]: S, then the last taps - 1 inputs (oldest first)
   void* out; int ldo;
+  int* tickets;                     // rows form: [nb * ceil(rows / 16)], zero between launches (null: a workgroup per block)
   // scan form: chunks [n_chunks][4] = first row, rows (<= 64), index in its run, chunks of the run;
   // cA / cB / cS [n_chunks][width] f32 scratch, u [rows][width] T scratch
   const int* chunks; int n_chunks;

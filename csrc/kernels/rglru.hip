@@ -6,8 +6,8 @@
 // over the 16-row tiles.  A row that starts a run of its sequence folds the state it starts from into b and
 // takes a = 0, so one scan serves any mix of runs.
 //
-//  * rows form (decode steps, <= 64 rows): a workgroup per block and 16 rows, for the runs that start there; runs
-//    are found from the sequence ids.  It is the only reader and writer of its runs' state in the block.
+//  * rows form (decode steps, <= 64 rows): workgroups per block and 16 rows, for the runs that start there; runs are found
+//    from the sequence ids.  They are the only readers and writers of their runs' state in the block.
 //  * scan form (prompt-sized runs): workgroups per (chunk of a run, block, 128 channels).  Launch 1 forms u and
 //    reduces every chunk to S_end = A S_start + B; launch 2 folds the chunks in front of its own, scans again
 //    and writes the outputs; the run's last chunk writes the state.
@@ -216,8 +216,14 @@ VWA_DEVICE void save_inputs4(const RgLruParams& p, int r, int n, bool fresh, flo
 }
 
 // ------------------------------------------------------------------------------------------ rows form
-// Workgroup (block, tile): the runs whose first row lies in rows 16 tile .. 16 tile + 15, 16 rows at a time to
-// their ends (other runs' rows count as inert).
+// Workgroup (block, tile, part): the runs whose first row lies in rows 16 tile .. 16 tile + 15, 16 rows at a time to
+// their ends (other runs' rows count as inert); kRowTiles of the block's 16-channel tiles.  Every part forms the whole block's u,
+// so the inputs it is formed from are replaced by the last part that has read them (RgLruParams::tickets).
+// What bounds it is one CU drawing a block's gates (256 and 512 KB of 256 channels) behind a chain of round trips, on 4 - 16 CUs.
+// us with parts of all 16, 8, 4, 2 tiles, gates in L2: 32 bits, 4 rows x 4 blocks 16.1, 12.0, 10.6, 10.6; bf16, 16 rows x 8 11.2, 10.6,
+// 10.7, 11.0.  (The save by the waves without a tile, beside the products: 0.3 - 1 slower.)
+constexpr int kRowTiles = 4;
+
 template <class T>
 __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
   constexpr int PRE = 8;
@@ -225,9 +231,11 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
   // of a row: its sequence; its run's first row (-1: inert); its run's rows (at the run's last row, else 0); whether
   // tokens precede it / its run
   __shared__ int s_seq[64], s_first[64], s_len[64], s_old[64], s_run_old[64];
+  __shared__ int s_last;
   const int blk = blockIdx.x, lo = blockIdx.y * 16, bs = p.bs, c0 = blk * bs;
   const int tid0 = threadIdx.x, nthr = blockDim.x, w = __builtin_amdgcn_readfirstlane(tid0 >> 6);
   const int stride = u_stride<T>(bs), steps = bs / MM<T>::KS, tiles = bs / 16, waves = nthr >> 6;
+  const int tper = (tiles + gridDim.z - 1) / gridDim.z, ct0 = blockIdx.z * tper, ct1 = min(tiles, ct0 + tper);  // this workgroup's
   T* out = reinterpret_cast<T*>(p.out);
   const T* gw0 = reinterpret_cast<const T*>(p.gw) + (size_t)blk * tiles * 32 * bs;
   if (tid0 < 64) {                                   // (one wave: runs from the rows' ids)
@@ -252,11 +260,12 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
   for (int r0 = lo; r0 < p.rows; r0 += 16) {
     if (r0 > lo && !owned(r0)) break;                // (a run that goes past the tile owns the next row)
     const int n = min(16, p.rows - r0);
+    const bool ends = r0 + 16 >= p.rows || !owned(r0 + 16);
 #pragma unroll 1
-    for (int t0 = 0; t0 < tiles; t0 += waves) {
+    for (int t0 = ct0; t0 < ct1; t0 += waves) {
       // (mostly the only pass: addresses are formed where they are used, not kept across passes)
       const int tid = opaque(tid0), lane = tid & 63, rl = lane & 15, g = lane >> 4;
-      const int ct = min(t0 + w, tiles - 1), ch = c0 + ct * 16 + rl;
+      const int ct = min(t0 + w, ct1 - 1), ch = c0 + ct * 16 + rl;
       // ---- requested ahead of the convolution
       const T* gw = gw0 + (size_t)ct * 32 * bs;
       GateFrags<PRE> f;
@@ -270,7 +279,7 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
         yv[i] = reinterpret_cast<const T*>(p.yx)[(size_t)r * p.ld + ch];
         s_in[i] = state_of(r)[ch];
       }
-      if (t0 == 0) {
+      if (t0 == ct0) {
 #pragma unroll 1
         for (int x = tid; x < 16 * quads; x += nthr) {
           const int i = x / quads, c = (x % quads) * 4, r = r0 + i;
@@ -282,7 +291,12 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
       __builtin_amdgcn_sched_barrier(0);             // (the convolution's registers are free from here)
       f.load(gw, steps, 0, PRE / 2, PRE);
       __syncthreads();                               // (every read of the old inputs is done as well)
-      if (t0 + w >= tiles) continue;
+      if (gridDim.z > 1 && ends && t0 == ct0 && tid0 == 0) {
+        int* at = p.tickets + blockIdx.y * gridDim.x + blk;
+        s_last = __hip_atomic_fetch_add(at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.z - 1;
+        if (s_last) __hip_atomic_store(at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (t0 + w >= ct1) continue;
       f32x4 ar[1], ai[1];
       gate_products<T, 1, PRE>(us, stride, gw, steps, f, ar, ai);
       float a[4], b[4], s[4], A, B;
@@ -309,12 +323,15 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
         }
       }
     }
+    __syncthreads();                                 // u is overwritten; saved states are read by the next rows
+    if (!ends) continue;
+    if (gridDim.z > 1 && !s_last) return;            // (the last one of the block's workgroups to read the old inputs replaces them)
 #pragma unroll 1
-    for (int x = opaque(tid0); x < n * quads; x += nthr) {
-      const int r = r0 + x / quads, len = s_len[r];
+    for (int x = opaque(tid0); x < (r0 + n - lo) * quads; x += nthr) {
+      const int r = lo + x / quads, len = s_len[r];
       if (len > 0 && owned(r)) save_inputs4<T>(p, r, len, !s_run_old[r], state_of(r), c0 + (x % quads) * 4);
     }
-    __syncthreads();                                 // u is overwritten; saved states are read by the next rows
+    return;
   }
 }
 
@@ -470,7 +487,8 @@ size_t u_bytes(int rows, int bs) { return (size_t)rows * (bs * sizeof(T) + kPad)
 template <class T>
 int launch_rows(const RgLruParams& p, hipStream_t st) {
   if (u_bytes<T>(16, p.bs) > kMaxLds) return -10;
-  const dim3 grid(p.nb, (p.rows + 15) / 16), block(64 * (p.bs / 16 < 16 ? p.bs / 16 : 16));
+  const int tiles = p.bs / 16, per = p.tickets ? kRowTiles : tiles;
+  const dim3 grid(p.nb, (p.rows + 15) / 16, (tiles + per - 1) / per), block(64 * (tiles < 16 ? tiles : 16));
   hipLaunchKernelGGL((rglru_rows_kernel<T>), grid, block, u_bytes<T>(16, p.bs), st, p);
   return (int)hipGetLastError();
 }

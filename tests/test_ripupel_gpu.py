@@ -108,7 +108,8 @@ RGLRU = [(60, 3, 4), (40, 1, 1), (256, 2, 3), (96, 3, 2), (512, 2, 4), (640, 2, 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("W,nb,taps", RGLRU)
 @pytest.mark.parametrize("lens", [((2, 0, 1), (0, 5, 33), (3, 0, 64), (1, 100, 2), (4, 1, 95)), ((1, 0, 300), (0, 7, 257), (4, 2, 1)),
-                                  ((3, 9, 1), (1, 0, 1), (0, 1, 1), (4, 40, 1)), ((2, 0, 2), (1, 3, 30), (0, 0, 17))], ids=["mix", "long", "one", "short"])
+                                  ((3, 9, 1), (1, 0, 1), (0, 1, 1), (4, 40, 1)), ((2, 0, 2), (1, 3, 30), (0, 0, 17)),
+                                  ((0, 4, 14), (3, 0, 20), (1, 7, 1), (4, 2, 29))], ids=["mix", "long", "one", "short", "past"])
 def test_rglru(dtype, W, nb, taps, lens):
     """Rows form (where the rows fit) and scan form over several runs: fresh ones, continuing ones (also with
     fewer tokens behind them than the convolution has taps), slow and fast channels."""
@@ -137,15 +138,18 @@ def test_rglru(dtype, W, nb, taps, lens):
     yx = torch.cat([chan(y.float()), chan(x.float())], 1).to(dtype).to(DEV)
     ids, pos = torch.tensor(ids, dtype=torch.int32, device=DEV), torch.tensor(pos, dtype=torch.int32, device=DEV)
     real = chan(torch.ones(W)).bool()
-    for plan in ([None] if tot <= 64 else []) + [ops.plan_runs(runs, DEV, 400, scan_rows=mixers.SCAN_ROWS)]:
+    tickets = torch.zeros(p.nb * 4, dtype=torch.int32, device=DEV)
+    forms = [(None, None), (None, tickets)] if tot <= 64 else []  # (tickets: a block's channels over several workgroups)
+    for plan, t in forms + [(ops.plan_runs(runs, DEV, 400, scan_rows=mixers.SCAN_ROWS), None)]:
         st = chan(st0).reshape(5, -1).contiguous().to(DEV)
         out = torch.zeros(tot, Wp + 8, dtype=dtype, device=DEV)
-        ops.rglru(yx, p, seq_ids=ids, positions=pos, slots=pos.long(), state=st, out=out[:, :Wp], plan=plan)
+        ops.rglru(yx, p, seq_ids=ids, positions=pos, slots=pos.long(), state=st, out=out[:, :Wp], plan=plan, tickets=t)
         # (bf16: u is rounded where the kernel rounds it; a near-tie of that rounding moves u by a unit)
         tol = 2e-5 if dtype == F32 else 1.2e-2
         assert rel(out[:, :Wp].cpu()[:, real], want) < tol
         assert rel(st.cpu().view(5, taps, Wp)[..., real], end) < tol
         assert out[:, Wp:].abs().sum() == 0 and out[:, :Wp].cpu()[:, ~real].abs().sum() == 0
+        assert tickets.abs().sum() == 0
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -305,7 +305,9 @@ class RipupelModel:
         b.update(hidden_sel=torch.zeros(rows, self.d_pad, dtype=torch.float32, device=dev),
                  head_in=torch.zeros(rows, self.d_pad, dtype=self.dtype, device=dev),
                  logits_local=torch.zeros(rows, self.v_pad, dtype=torch.float32, device=dev),
-                 latent=LatentScratch(lat, max_ctx, dev) if lat else None)
+                 latent=LatentScratch(lat, max_ctx, dev) if lat else None,
+                 rglru_tickets=torch.zeros(max([1] + [D.nb * -(-rows // 16) for D in self.dims if isinstance(D, RgLruDims)]),
+                                           dtype=torch.int32, device=dev))
         return b
 
     def plan_rows(self, runs: Sequence[Tuple[int, int, int, int]], max_pos: int) -> SimpleNamespace:
@@ -333,7 +335,8 @@ class RipupelModel:
         ops.linear(h, L.w_in, out=y)
         cat, br = bufs.cat[D.cols][:M], bufs.branch
         if isinstance(D, RgLruDims):
-            ops.rglru(y, L.mixer, state=kv.state[li], out=cat[:, : D.cols], plan=plan, **rows)
+            ops.rglru(y, L.mixer, state=kv.state[li], out=cat[:, : D.cols], plan=plan,
+                      tickets=getattr(bufs, "rglru_tickets", None), **rows)
         else:
             self._attend(li, y, cat[:, : D.cols], bufs, M, kv, rows, plan)
         ops.linear(cat, L.w_out, out=br[:M])

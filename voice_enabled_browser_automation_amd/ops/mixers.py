@@ -69,15 +69,17 @@ def gate_fragments(gates: torch.Tensor) -> torch.Tensor:
 
 
 def rglru(yx: torch.Tensor, w: RgLruWeights, *, seq_ids: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor,
-          state: torch.Tensor, out: torch.Tensor, plan: Optional[SimpleNamespace] = None) -> torch.Tensor:
+          state: torch.Tensor, out: torch.Tensor, plan: Optional[SimpleNamespace] = None,
+          tickets: Optional[torch.Tensor] = None) -> torch.Tensor:
     """yx rows [y | x] (raw projections): u = causal conv of x + its bias, r / i from u block by block,
     S <- a S + sqrt(1 - a^2) i u with log a = decay r, out = S gelu_tanh(y + bias).  The state row of a
-    sequence is its id, read and written once per run (position 0 starts from zeros)."""
+    sequence is its id, read and written once per run (position 0 starts from zeros).  tickets: int32 zeros of the
+    caller's, nb for every 16 rows of a decode step, left zero: a block's channels are split over workgroups."""
     if not yx.is_cuda:
         return ref.rglru(yx, w, seq_ids=seq_ids, positions=positions, slots=slots, state=state, out=out)
     args = (yx, w.yb, w.xb, w.conv, w.conv_b, w.gates, w.rb, w.ib, w.decay, w.nb, seq_ids, positions, slots, state, out)
     if plan is None:
-        _ext().rglru(*args)
+        _ext().rglru(*args, tickets=tickets)
     else:
         from . import scratch
 
