@@ -1030,3 +1030,38 @@ def test_a_sequence_freed_behind_its_last_step_keeps_its_pages_there(rows):
     assert torch.equal(run(False), want)
     for _ in range(2):
         assert torch.equal(run(True), want)
+
+
+@pytest.mark.parametrize("rows", [1, 7])
+def test_steps_queued_behind_a_busy_device_read_their_own_rows(rows):
+    """More steps than there are staging rows, queued while the device is busy with something else: every step's logits are those
+    of steps that were waited for.  Pages and their table entries come on the way; one row's steps run the chained launch."""
+    from voice_enabled_browser_automation_amd.runtime.engine import STAGING
+
+    model = LlamaModel(CFG, device="cuda", seed=4)
+    eng = LLMEngine(model, max_seqs=rows, max_model_len=256, kv_blocks=16 * rows + 1)
+    n = 2 * STAGING + 5
+    toks = np.random.default_rng(3).integers(0, CFG.vocab_size, (n + 1, rows, 20)).tolist()
+
+    def run(wait):
+        seqs = [eng.new_sequence([], use_prefix_cache=False) for _ in range(rows)]
+        eng.step_batch([(s, t) for s, t in zip(seqs, toks[n])])
+        torch.cuda.synchronize()
+        if not wait:
+            torch.cuda._sleep(200_000_000)  # (some 100 ms)
+        out = []
+        for k in range(n):
+            lg = eng.run_rows([(s, t[0]) for s, t in zip(seqs, toks[k])], logits_for=[rows - 1], check=wait)
+            out.append(lg.clone())
+            if wait:
+                torch.cuda.synchronize()
+        out = torch.cat(out)
+        for s in seqs:
+            eng.free_sequence(s, publish=False)
+        torch.cuda.synchronize()
+        return out
+
+    want = run(True)
+    assert want.shape[0] == n and (want[1:] != want[:-1]).any(1).all()
+    for _ in range(2):
+        assert torch.equal(run(False), want)

@@ -131,51 +131,71 @@ class StepBuffers:
         self.attn_cnt = torch.zeros(max_rows * model.nkv, dtype=torch.int32, device=device)  # chunk tickets
 
     def _host_staging(self, R: int, max_seqs: int, max_blocks_per_seq: int, T: int, C: int, device) -> None:
-        pin = torch.device(device).type == "cuda"
+        self._cuda = torch.device(device).type == "cuda"
+        self.head_idx = torch.zeros(R, dtype=torch.int64, device=device)
+        self.row_table = self.meta_all[T:].view(R, C)
+        # the block table as the host has it (np_table; sequences come, grow and go at any time)
+        self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
+        self.table_dirty = True
+        self._ring = [StepStaging(R, T, C, self._cuda) for _ in range(STAGING if self._cuda else 1)]
+        self._ring_at = -1
+        self._ring_done = [torch.cuda.Event(), torch.cuda.Event()] if self._cuda else []  # behind the last use of either half
+        self._ring_used = False
+
+    def staging(self) -> "StepStaging":
+        """The next step's pinned rows.  Steps are queued without a wait for the one before; rows are written again only when the
+        step that had them is through: an event behind every half of the ring tells."""
+        if not self._cuda:
+            return self._ring[0]
+        self._ring_at = (self._ring_at + 1) % STAGING
+        half, first = divmod(self._ring_at, STAGING // 2)
+        if first == 0:
+            self._ring_done[1 - half].record()  # (behind every step queued so far)
+            if self._ring_used:
+                self._ring_done[half].synchronize()
+            self._ring_used = half == 1 or self._ring_used
+        return self._ring[self._ring_at]
+
+    def upload(self, st: "StepStaging", n_rows: int) -> None:
+        """H2D copy of a step's metadata (with the rows' block tables where the chained launch reads them) and of the block
+        table when it changed."""
+        n = self.meta_all.numel() - self.row_table.numel() + n_rows * self.row_table.shape[1] if self.rt_cols and n_rows <= 4 \
+            else self.meta.numel()
+        self.meta_all[:n].copy_(st.h_meta_all[:n], non_blocking=True)
+        self.upload_table()
+
+    def upload_table(self) -> None:
+        """H2D copy of the block table when it changed, out of pinned rows of its own: copies before it may be queued."""
+        if self.table_dirty:
+            t = torch.from_numpy(self.np_table)
+            self.block_table.copy_(t.pin_memory() if self.block_table.is_cuda else t, non_blocking=True)
+            self.table_dirty = False
+
+
+# Staging rows of a step in turn (a multiple of 2): a queued step holds its own until it is through
+STAGING = 16
+
+
+class StepStaging:
+    """Pinned host rows of one step: [tokens | positions | seq_ids | ctx_lens | slots | sel | shared | row tables] as on the device,
+    and numpy views of them -- the per-step row metadata is written with a handful of slice assignments instead of ~5 torch
+    element writes per row."""
+
+    def __init__(self, R: int, T: int, C: int, pin: bool):
         self.h_meta_all = torch.zeros(T + R * C, dtype=torch.int32, pin_memory=pin)
-        self.h_meta = self.h_meta_all[: 7 * R + 2]
-        self.h_i32 = self.h_meta[: 4 * R].view(4, R)
-        self.h_slots = self.h_meta[4 * R : 6 * R].view(torch.int64)
-        self.h_sel = self.h_meta[6 * R : 7 * R]
-        self.np_shared = self.h_meta[7 * R : 7 * R + 2].numpy()
+        meta = self.h_meta_all[: 7 * R + 2]
+        self.np_i32 = meta[: 4 * R].view(4, R).numpy()
+        self.np_slots = meta[4 * R : 6 * R].view(torch.int64).numpy()
+        self.np_sel = meta[6 * R : 7 * R].numpy()
+        self.np_shared = meta[7 * R : 7 * R + 2].numpy()
+        self.np_row_table = self.h_meta_all[T:].view(R, C).numpy()
         # rows whose hidden state feeds the LM head when the step computed every row (L == M):
         # gathered on the device through a pinned staging copy (a torch.tensor(list, device=...)
         # here was a pageable, host-blocking copy that waited for the whole step -- measured: 9 of
         # 172 iterations at 32 sessions stalled ~4.6 ms each)
         self.h_head_idx = torch.zeros(R, dtype=torch.int64, pin_memory=pin)
-        self.head_idx = torch.zeros(R, dtype=torch.int64, device=device)
-        self.row_table = self.meta_all[T:].view(R, C)
-        self.h_row_table = self.h_meta_all[T:].view(R, C)
-        self.np_row_table = self.h_row_table.numpy()
-        self.h_i32[3].fill_(1)  # the same inert rows as the device copy (captured graphs upload it)
-        self.h_slots.fill_(-1)
-        # the block table as the host has it (np_table; sequences come, grow and go at any time) and its pinned staging copy,
-        # which is written only when no copy of it can be queued
-        self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
-        self.h_table = torch.zeros(max_seqs, max_blocks_per_seq, dtype=torch.int32, pin_memory=pin)
-        self.table_dirty = True
-        # numpy views of the pinned staging buffers: the per-step row metadata is written with a
-        # handful of slice assignments instead of ~5 torch element writes per row
-        self.np_i32 = self.h_i32.numpy()
-        self.np_slots = self.h_slots.numpy()
-        self.np_sel = self.h_sel.numpy()
-
-    def upload(self, n_rows: int, meta: bool = True) -> None:
-        """H2D copy of the step metadata (skipped when the replayed graph contains it) and of the
-        block table when it changed.  The staging copies are free (LLMEngine._sync_staging)."""
-        if meta:
-            self.meta.copy_(self.h_meta, non_blocking=True)
-        if self.table_dirty:
-            self.h_table.numpy()[:] = self.np_table
-            self.block_table.copy_(self.h_table, non_blocking=True)
-            self.table_dirty = False
-
-    def upload_table(self) -> None:
-        """H2D copy of the block table when it changed, out of pinned rows of its own: the staging copy may be queued."""
-        if self.table_dirty:
-            t = torch.from_numpy(self.np_table)
-            self.block_table.copy_(t.pin_memory() if self.block_table.is_cuda else t, non_blocking=True)
-            self.table_dirty = False
+        self.np_i32[3].fill(1)  # inert rows, as the device's before the first step
+        self.np_slots.fill(-1)
 
 
 class LLMEngine:
@@ -251,10 +271,7 @@ class LLMEngine:
         self.graph_pool = None
         self.stats = dict(steps=0, rows=0, prefill_tokens=0, cached_tokens=0, graph_replays=0)
         self._last_step = None  # (rows, logits_for, n_computed before) of a chained step, for recover_step
-        # True from a step's launch until the host knows the stream has passed it: the pinned
-        # staging rows (h_meta, h_row_table) are read by that step's H2D copy -- inside the
-        # replayed graph -- so the next step may only rewrite them once it has executed
-        self._staging_inflight = False
+        self._step_err = None  # (pinned copy of a chained step's error word, event behind the copy)
         self._head_rows: Optional[torch.Tensor] = None  # the last step's hidden rows for head_logits()
         self._shared_cache: Dict[tuple, int] = {}  # sequences of a step -> shared prefix blocks
 
@@ -328,14 +345,7 @@ class LLMEngine:
         return seq.blocks[pos // self.block_size] * self.block_size + pos % self.block_size
 
     # ------------------------------------------------------------------ forward
-    def _forward_rows(self, M: int, L: int, upload_meta: bool = False) -> torch.Tensor:
-        if upload_meta:
-            # inside a captured graph: the pinned -> device metadata copy is the graph's first node,
-            # so a replay is one host call instead of a copy + a replay
-            b = self.bufs
-            n = (b.meta_all.numel() - b.row_table.numel() + M * b.row_table.shape[1]) if b.rt_cols and M <= 4 \
-                else b.meta.numel()
-            b.meta_all[:n].copy_(b.h_meta_all[:n], non_blocking=True)
+    def _forward_rows(self, M: int, L: int) -> torch.Tensor:
         return self.model.forward(self.bufs, M, self.kv, n_sel=None if L == M else L, head=False)
 
     def _capture(self, M: int, L: int):
@@ -344,22 +354,20 @@ class LLMEngine:
         if self.stateful:
             # the warm-up forwards below must not advance a recurrent state: they run this step's rows as
             # inert ones (no slot), the replay after the capture runs them for real
-            torch.cuda.current_stream().synchronize()
-            slots = b.np_slots[:M].copy()
-            b.np_slots[:M] = -1
+            slots = b.slots[:M].clone()
+            b.slots[:M] = -1
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
             for _ in range(2):
-                self._forward_rows(M, L, upload_meta=True)
+                self._forward_rows(M, L)
         torch.cuda.current_stream().wait_stream(s)
         if slots is not None:
-            s.synchronize()  # (the warm-ups have read the staging rows)
-            b.np_slots[:M] = slots
+            b.slots[:M] = slots
         g = torch.cuda.CUDAGraph()
         if self.graph_pool is None:
             self.graph_pool = torch.cuda.graph_pool_handle()
         with capture_graph(g, pool=self.graph_pool):
-            out = self._forward_rows(M, L, upload_meta=True)
+            out = self._forward_rows(M, L)
         self.graphs[(M, L, self._gated)] = (g, out)
         return self.graphs[(M, L, self._gated)]
 
@@ -403,9 +411,7 @@ class LLMEngine:
         b = self.bufs
         if getattr(self, "_chain_retry_at", None) is not None:
             self._maybe_rearm_chain()
-        # the rows' numbers first, while the previous step may still run; the pinned staging only once it is through
-        # (back-to-back steps with no host sync in between -- several admissions in one scheduler iteration, partial
-        # feeds, given tokens: its copy of the staging rows may still be queued behind its forward)
+        # (the previous step may still run: its rows are staged elsewhere)
         pending: Dict[int, int] = {}
         bs = self.block_size
         toks, poss, sids, slots = [], [], [], []
@@ -422,34 +428,32 @@ class LLMEngine:
             slots.append(seq.blocks[pos // bs] * bs + pos % bs)
             pending[sid] = pos + 1
         shared = self._shared_prefix(rows, min(poss) + 1)
-        self._sync_staging()
+        st = b.staging()
         if logits_for is None or len(logits_for) == n:
             nl, L = n, M
         else:
             nl = len(logits_for)
             L = min(bucket_for(nl), M)
             if L < M:  # (L == M: no saving -- compute every row and index on the host side)
-                b.np_sel[:nl] = logits_for
-                b.np_sel[nl:L] = logits_for[-1]
-        rtab = b.np_row_table if b.rt_cols and M <= 4 else None
+                st.np_sel[:nl] = logits_for
+                st.np_sel[nl:L] = logits_for[-1]
+        rtab = st.np_row_table if b.rt_cols and M <= 4 else None
         if rtab is not None:  # after the loop: a later row of a sequence may have added its last block
             for i, (seq, _) in enumerate(rows):
                 rtab[i, : len(seq.blocks)] = seq.blocks
-        hi = b.np_i32
+        hi = st.np_i32
         hi[0, :n] = toks
         hi[1, :n] = poss
         hi[2, :n] = sids
         hi[3, :n] = hi[1, :n] + 1
-        b.np_slots[:n] = slots
-        b.np_shared[0] = shared
-        b.np_shared[1] = n
+        st.np_slots[:n] = slots
+        st.np_shared[0] = shared
+        st.np_shared[1] = n
         if M > n:  # padded rows: no KV write, 1-token context on scratch block 0
             hi[0:3, n:M] = 0
             hi[3, n:M] = 1
-            b.np_slots[n:M] = -1
-        b.upload(M, meta=not self.use_graphs)  # the step graphs copy the metadata themselves
-        if rtab is not None and not self.use_graphs:
-            b.row_table[:M].copy_(b.h_row_table[:M], non_blocking=True)
+            st.np_slots[n:M] = -1
+        b.upload(st, M)
         if self.chain_gate is not None:
             self._gated = bool(self.chain_gate())
             self.model._chain_gated = self._gated
@@ -465,34 +469,47 @@ class LLMEngine:
             self.stats["graph_replays"] += 1
         else:
             hs = self._forward_rows(M, L)
-        self._staging_inflight = self.device.type == "cuda"
         for sid, ln in pending.items():
             self.seqs[sid].n_computed = ln
         self.stats["steps"] += 1
         self.stats["rows"] += n
         if self.stats["steps"] % 64 == 0:
             self._check_chain()
-        if check and chained and self.device.type == "cuda":
-            torch.cuda.current_stream().synchronize()
-            self._staging_inflight = False
-            if self.model.chain_error():
-                self._head_rows = None
-                return self.recover_step()
         if L == M and nl != n:
-            b.h_head_idx[:nl] = torch.as_tensor(logits_for, dtype=torch.int64)
+            st.h_head_idx[:nl] = torch.as_tensor(logits_for, dtype=torch.int64)
             idx = b.head_idx[:nl]
-            idx.copy_(b.h_head_idx[:nl], non_blocking=hs.device.type == "cuda")
+            idx.copy_(st.h_head_idx[:nl], non_blocking=hs.device.type == "cuda")
             self._head_rows = hs.index_select(0, idx)
         else:
             self._head_rows = hs[:nl]
-        if defer_head:
+        check = check and chained and self.device.type == "cuda"
+        done = self._chain_word() if check else None
+        logits = None if defer_head else self.head_logits()  # (queued while the host waits for the layers: a failed step's are dropped)
+        if check and self._chain_failed(done):
+            self._head_rows = None
+            return self.recover_step()
+        return logits
+
+    def _chain_word(self) -> Optional["torch.cuda.Event"]:
+        """Queues the copy of the chained launch's error word to the host behind the step's layers -> the event behind it."""
+        word = self.model.chain_error_word()
+        if word is None:
             return None
-        return self.head_logits()
+        if self._step_err is None:
+            self._step_err = (torch.zeros(1, dtype=torch.int64, pin_memory=True), torch.cuda.Event())
+        self._step_err[0].copy_(word, non_blocking=True)
+        self._step_err[1].record()
+        return self._step_err[1]
+
+    def _chain_failed(self, done: Optional["torch.cuda.Event"]) -> bool:
+        if done is None:
+            return False
+        done.synchronize()
+        return bool(self._step_err[0].item() != 0)
 
     def host_synced(self) -> None:
-        """The caller has observed the stream past the last step (e.g. read its sampled tokens):
-        the next run_rows may rewrite the pinned staging rows without a synchronize."""
-        self._staging_inflight = False
+        """The caller has observed the stream past the last step (e.g. read its sampled tokens).  (Steps need no such word any more:
+        each has staging rows of its own.)"""
 
     def head_logits(self, col_mask: Optional[torch.Tensor] = None, mask_rows: int = 1,
                     gather: bool = True) -> torch.Tensor:
@@ -645,7 +662,6 @@ class LLMEngine:
             self.run_rows(rows, logits_for=[len(rows) - 1], check=True, defer_head=True)
             self._head_rows = None
             return
-        self._sync_staging()
         for cut in self._cut(parts, chunk):
             self._ragged_forward(cut)
 
@@ -674,7 +690,6 @@ class LLMEngine:
             self.run_rows(rows, logits_for=[n - 1], defer_head=True)
             self._head_rows = None
             return None
-        self._sync_staging()
         hidden, at = [], 0
         for cut in self._cut(parts, chunk):
             m = sum(k for _, k in cut)
@@ -702,11 +717,6 @@ class LLMEngine:
                 room -= take
                 k -= take
         return out
-
-    def _sync_staging(self) -> None:
-        if self._staging_inflight and self.device.type == "cuda":
-            torch.cuda.current_stream().synchronize()
-            self._staging_inflight = False
 
     def _ragged_forward(self, parts: List[Tuple[Sequence_, int]], want: Sequence[int] = ()) -> Optional[torch.Tensor]:
         """One eager forward of ragged rows (more than the step buffers hold): the next tokens of each
@@ -814,7 +824,6 @@ class LLMEngine:
                 logits = self.run_rows([(seq, t) for t in toks], logits_for=[n - 1])
                 continue
             if hasattr(self.model, "row_buffers"):
-                self._sync_staging()
                 hs = self._ragged_forward([(seq, n)], [n - 1])
                 logits = self.model.lm_logits(self.bufs, hs)
                 continue
