@@ -1036,11 +1036,9 @@ def test_a_sequence_freed_behind_its_last_step_keeps_its_pages_there(rows):
 def test_steps_queued_behind_a_busy_device_read_their_own_rows(rows):
     """More steps than there are staging rows, queued while the device is busy with something else: every step's logits are those
     of steps that were waited for.  Pages and their table entries come on the way; one row's steps run the chained launch."""
-    from voice_enabled_browser_automation_amd.runtime.engine import STAGING
-
     model = LlamaModel(CFG, device="cuda", seed=4)
     eng = LLMEngine(model, max_seqs=rows, max_model_len=256, kv_blocks=16 * rows + 1)
-    n = 2 * STAGING + 5
+    n = 2 * len(eng.bufs.staging) + 5
     toks = np.random.default_rng(3).integers(0, CFG.vocab_size, (n + 1, rows, 20)).tolist()
 
     def run(wait):
@@ -1065,3 +1063,34 @@ def test_steps_queued_behind_a_busy_device_read_their_own_rows(rows):
     assert want.shape[0] == n and (want[1:] != want[:-1]).any(1).all()
     for _ in range(2):
         assert torch.equal(run(False), want)
+
+
+@pytest.mark.parametrize("d", [128, 192])
+def test_speech_steps_queued_behind_a_busy_device(d):
+    """More decoder steps than there are staging rows behind a busy device, launched alone (widths of 128) or as graphs: the logits
+    of steps that were waited for."""
+    import dataclasses
+
+    from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner
+
+    cfg = dataclasses.replace(get_config("whisper-tiny"), d_model=d, n_heads=d // 64, n_enc_layers=1, n_dec_layers=2, vocab_size=4096)
+    m = WhisperModel(cfg, device="cuda", seed=6)
+    r = WhisperRunner(m, max_sessions=1)
+    r.set_cross(0, torch.randn(1, cfg.n_audio_ctx, d, device="cuda").bfloat16())
+    assert m.one_launch(r.b, 1) == (d == 128)
+    n = 2 * len(r.staging) + 5
+
+    def run(wait):
+        torch.cuda.synchronize()
+        if not wait:
+            torch.cuda._sleep(200_000_000)  # (some 100 ms)
+        out = []
+        for p in range(n):
+            out.append(r.step([(0, (37 * p + 5) % 4096, p)]).clone())
+            if wait:
+                torch.cuda.synchronize()
+        return torch.cat(out)
+
+    want = run(True)
+    assert (want[1:] != want[:-1]).any(1).all() and not m.chain_error()
+    assert torch.equal(run(False), want)

@@ -18,6 +18,7 @@ import torch
 from .. import ops
 from ..models.whisper import WhisperModel
 from ..utils.capture import capture_graph
+from ..utils.staging import StagingRing
 
 BUCKETS = (1, 2, 4, 8, 16, 32, 64)
 
@@ -78,19 +79,18 @@ class WhisperRunner:
         b.cross_table = torch.arange(max_sessions, dtype=torch.int32, device=dev)[:, None].contiguous()
         b.cross_lens = torch.full((R,), cfg.n_audio_ctx, dtype=torch.int32, device=dev)
         self.b = b
-        pin = dev.type == "cuda"
-        self.h_in = torch.zeros(6 * R, dtype=torch.int32, pin_memory=pin)
-        self.h_i32 = self.h_in[: 4 * R].view(4, R)
-        self.h_slots = self.h_in[4 * R :].view(torch.int64)
-        self.h_i32[3].fill_(1)
-        self.h_slots.fill_(-1)
-        self.np_i32, self.np_slots = self.h_i32.numpy(), self.h_slots.numpy()
+        cuda = dev.type == "cuda"
+
+        def rows():
+            h = torch.zeros(6 * R, dtype=torch.int32, pin_memory=cuda)
+            return SimpleNamespace(h_in=h, np_i32=h[: 4 * R].view(4, R).numpy(), np_slots=h[4 * R :].view(torch.int64).numpy())
+
+        self.staging = StagingRing(rows, cuda)
         if use_graphs is None:
             use_graphs = ops.env_flag("VWA_HIPGRAPH")
         self.use_graphs = bool(use_graphs) and dev.type == "cuda"
         self.graphs: Dict[int, Tuple[torch.cuda.CUDAGraph, torch.Tensor]] = {}
         self.pool = None
-        self._copy_done: Optional["torch.cuda.Event"] = None  # the last step's staging copy (step())
 
     def set_cross(self, slot: int, enc_states: torch.Tensor) -> None:
         """Compute this session's cross-attention K/V from encoder states [1, T, d]."""
@@ -121,26 +121,17 @@ class WhisperRunner:
         """rows: (session slot, token, position). Returns f32 logits [len(rows), vocab_padded]."""
         n = len(rows)
         M = next(bk for bk in BUCKETS if bk >= n)
-        # the rows' numbers first, while the previous step may still run
         slot, tok, pos = np.asarray(rows, dtype=np.int64).reshape(n, 3).T
-        if self._copy_done is not None:
-            # the previous step's pinned -> device copy may still be queued behind its forward:
-            # rewriting the pinned rows before it ran would feed that step the NEXT step's tokens /
-            # positions / slots (back-to-back step() calls with no host sync in between; the
-            # one-launch decoder leaves the host far ahead of the GPU)
-            self._copy_done.synchronize()
-        hi = self.np_i32
+        st = self.staging.next()  # (the previous step may still run, or be queued: its rows are its own)
+        hi, slots = st.np_i32, st.np_slots
         hi[0, :n], hi[1, :n], hi[2, :n], hi[3, :n] = tok, pos, slot, pos + 1
-        self.np_slots[:n] = (1 + slot * self.bps + pos // self.bs) * self.bs + pos % self.bs
+        slots[:n] = (1 + slot * self.bps + pos // self.bs) * self.bs + pos % self.bs
         hi[:3, n:M], hi[3, n:M] = 0, 1
-        self.np_slots[n:M] = -1
+        slots[n:M] = -1
         b = self.b
-        b.step_in.copy_(self.h_in, non_blocking=True)
-        if self.device.type == "cuda":
-            if self._copy_done is None:
-                self._copy_done = torch.cuda.Event()
-            self._copy_done.record()
-        if self.use_graphs:
+        b.step_in.copy_(st.h_in, non_blocking=True)
+        # (a graph of one launch starts and ends later than the launch itself: 80 -> 69 us a token of whisper-tiny's sizes)
+        if self.use_graphs and not self.model.one_launch(b, M):
             g, out = self.graphs.get(M) or self._capture(M)
             g.replay()
         else:

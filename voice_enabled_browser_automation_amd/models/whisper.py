@@ -583,6 +583,10 @@ class WhisperModel:
         every KV position of a session."""
         return self.pos_emb.shape[0] >= bufs.block_table.shape[1] * bufs.k_cache.shape[3]
 
+    def one_launch(self, bufs, M: int) -> bool:
+        """Whether a step of M rows is a single launch (embedding, layers, LM head)."""
+        return self._wdec_ok(M) and self._wdec_emb_ok(bufs) and self._wdec_state(bufs) is not None
+
     def _wdec_step(self, bufs, smp: Optional[list] = None, base_block: int = 0) -> torch.Tensor:
         """Every decoder layer of a one-row step and the LM head (folded final LayerNorm) in ONE
         launch -- with the embedding of bufs.tokens[0] / bufs.positions[0] built by layer 0

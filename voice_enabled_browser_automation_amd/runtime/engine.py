@@ -32,6 +32,7 @@ from .. import ops
 from .kv_cache import BlockManager, PagedKVCache
 from ..utils.capture import capture_graph
 from ..utils.env import knob
+from ..utils.staging import StagingRing
 
 # Row buckets of the captured step graphs (VWA_ROW_BUCKETS overrides).  48 between the powers of
 # two: a 44-row step of 32 concurrent sessions (+ jump-forward rows) pays for 48 rows, not 64 --
@@ -131,30 +132,13 @@ class StepBuffers:
         self.attn_cnt = torch.zeros(max_rows * model.nkv, dtype=torch.int32, device=device)  # chunk tickets
 
     def _host_staging(self, R: int, max_seqs: int, max_blocks_per_seq: int, T: int, C: int, device) -> None:
-        self._cuda = torch.device(device).type == "cuda"
+        cuda = torch.device(device).type == "cuda"
         self.head_idx = torch.zeros(R, dtype=torch.int64, device=device)
         self.row_table = self.meta_all[T:].view(R, C)
         # the block table as the host has it (np_table; sequences come, grow and go at any time)
         self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
         self.table_dirty = True
-        self._ring = [StepStaging(R, T, C, self._cuda) for _ in range(STAGING if self._cuda else 1)]
-        self._ring_at = -1
-        self._ring_done = [torch.cuda.Event(), torch.cuda.Event()] if self._cuda else []  # behind the last use of either half
-        self._ring_used = False
-
-    def staging(self) -> "StepStaging":
-        """The next step's pinned rows.  Steps are queued without a wait for the one before; rows are written again only when the
-        step that had them is through: an event behind every half of the ring tells."""
-        if not self._cuda:
-            return self._ring[0]
-        self._ring_at = (self._ring_at + 1) % STAGING
-        half, first = divmod(self._ring_at, STAGING // 2)
-        if first == 0:
-            self._ring_done[1 - half].record()  # (behind every step queued so far)
-            if self._ring_used:
-                self._ring_done[half].synchronize()
-            self._ring_used = half == 1 or self._ring_used
-        return self._ring[self._ring_at]
+        self.staging = StagingRing(lambda: StepStaging(R, T, C, cuda), cuda)
 
     def upload(self, st: "StepStaging", n_rows: int) -> None:
         """H2D copy of a step's metadata (with the rows' block tables where the chained launch reads them) and of the block
@@ -170,10 +154,6 @@ class StepBuffers:
             t = torch.from_numpy(self.np_table)
             self.block_table.copy_(t.pin_memory() if self.block_table.is_cuda else t, non_blocking=True)
             self.table_dirty = False
-
-
-# Staging rows of a step in turn (a multiple of 2): a queued step holds its own until it is through
-STAGING = 16
 
 
 class StepStaging:
@@ -428,7 +408,7 @@ class LLMEngine:
             slots.append(seq.blocks[pos // bs] * bs + pos % bs)
             pending[sid] = pos + 1
         shared = self._shared_prefix(rows, min(poss) + 1)
-        st = b.staging()
+        st = b.staging.next()
         if logits_for is None or len(logits_for) == n:
             nl, L = n, M
         else:

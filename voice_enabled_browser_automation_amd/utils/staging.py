@@ -1,0 +1,34 @@
+"""Pinned host rows for steps that are queued without a wait for the one before."""
+from __future__ import annotations
+
+from typing import Callable, Generic, List, TypeVar
+
+import torch
+
+T = TypeVar("T")
+
+
+class StagingRing(Generic[T]):
+    """``n`` sets of rows (made by ``make``) in turn, one a step: a queued step's copies read its own set, and a set is written again
+    only when the step that had it is through, which an event behind every half of the ring tells.  (An event a step costs the
+    stream a few us.)  One stream at a time, as the device buffers that the rows go to.  Without a GPU one set is enough."""
+
+    def __init__(self, make: Callable[[], T], cuda: bool, n: int = 16):
+        self.sets: List[T] = [make() for _ in range(n if cuda else 1)]
+        self._done = [torch.cuda.Event(), torch.cuda.Event()] if cuda else []  # behind the last use of either half
+        self._at, self._used = -1, False
+
+    def __len__(self) -> int:
+        return len(self.sets)
+
+    def next(self) -> T:
+        if not self._done:
+            return self.sets[0]
+        self._at = (self._at + 1) % len(self.sets)
+        half, first = divmod(self._at, len(self.sets) // 2)
+        if first == 0:
+            self._done[1 - half].record()  # (behind every step queued so far)
+            if self._used:
+                self._done[half].synchronize()
+            self._used = self._used or half == 1
+        return self.sets[self._at]
