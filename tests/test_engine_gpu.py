@@ -1065,19 +1065,20 @@ def test_steps_queued_behind_a_busy_device_read_their_own_rows(rows):
         assert torch.equal(run(False), want)
 
 
-@pytest.mark.parametrize("d", [128, 192])
-def test_speech_steps_queued_behind_a_busy_device(d):
-    """More decoder steps than there are staging rows behind a busy device, launched alone (widths of 128) or as graphs: the logits
-    of steps that were waited for."""
+@pytest.mark.parametrize("persist", ["1", "0"])
+def test_speech_steps_queued_behind_a_busy_device(monkeypatch, persist):
+    """More decoder steps than there are staging rows behind a busy device, each a launch or a graph: the logits of steps that were
+    waited for."""
     import dataclasses
 
     from voice_enabled_browser_automation_amd.asr.engine import WhisperRunner
 
-    cfg = dataclasses.replace(get_config("whisper-tiny"), d_model=d, n_heads=d // 64, n_enc_layers=1, n_dec_layers=2, vocab_size=4096)
+    monkeypatch.setenv("VWA_ASR_PERSIST", persist)
+    cfg = dataclasses.replace(get_config("whisper-tiny"), d_model=128, n_heads=2, n_enc_layers=1, n_dec_layers=2, vocab_size=4096)
     m = WhisperModel(cfg, device="cuda", seed=6)
     r = WhisperRunner(m, max_sessions=1)
-    r.set_cross(0, torch.randn(1, cfg.n_audio_ctx, d, device="cuda").bfloat16())
-    assert m.one_launch(r.b, 1) == (d == 128)
+    r.set_cross(0, torch.randn(1, cfg.n_audio_ctx, 128, device="cuda").bfloat16())
+    assert m.one_launch(r.b, 1) == (persist == "1")
     n = 2 * len(r.staging) + 5
 
     def run(wait):
