@@ -32,4 +32,14 @@ void check_contig_rows(const Tensor& t, const char* name) {
 }
 void check_rc(int rc, const char* what) { TORCH_CHECK(rc == 0, what, " launch failed with code ", rc); }
 
+int device_cus(const Tensor& t) {
+  static int cached[64] = {0};
+  const int d = t.device().index();
+  if (d >= 0 && d < 64 && cached[d]) return cached[d];
+  int cus = 0;
+  TORCH_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, d) == hipSuccess, "CU count");
+  if (d >= 0 && d < 64) cached[d] = cus;
+  return cus;
+}
+
 }  // namespace

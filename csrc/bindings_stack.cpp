@@ -50,6 +50,38 @@ void gemm_f32(Tensor x, Tensor w, Tensor y, int64_t epi, c10::optional<Tensor> r
   check_rc(vwa_gemm_f32((int)epi, &p, cur_stream(x)), "gemm_f32");
 }
 
+// x @ w^T as the four quarters of its sums, y [4][rows][N] (any strides of its first two): for a norm that adds them up in order.
+// False: this product has none (nothing is written).
+bool gemm_f32_quarters(Tensor x, Tensor w, c10::optional<Tensor> y) {
+  c10::DeviceGuard g(x.device());
+  check_t(x, true, "x");
+  check_t(w, true, "w");
+  TORCH_CHECK(w.dim() == 2 && w.is_contiguous(), "w must be contiguous [N, K]");
+  const int64_t M = x.size(0), N = w.size(0), K = w.size(1);
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && x.size(1) == K, "x must be [M, K]");
+  TORCH_CHECK(K % 16 == 0 && x.stride(0) % 4 == 0, "gemm_f32: K % 16 == 0, 16-byte aligned rows");
+  check_aligned(x, "x");
+  check_aligned(w, "w");
+  GemmF32Params p{};
+  p.X = x.data_ptr<float>();
+  p.ldx = (int)x.stride(0);
+  p.W = w.data_ptr<float>();
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = (int)K;
+  if (y.has_value()) {
+    check_t(*y, true, "y");
+    TORCH_CHECK(y->dim() == 3 && y->size(0) == 4 && y->size(1) == M && y->size(2) == N && y->stride(2) == 1, "y [4, M, N]");
+    p.Y = y->data_ptr<float>();
+    p.ldy = (int)y->stride(1);
+    p.part = y->stride(0);
+  }
+  const int rc = vwa_gemm_f32_quarters(&p, device_cus(x), y.has_value(), cur_stream(x));
+  if (rc == -7) return false;
+  check_rc(rc, "gemm_f32_quarters");
+  return true;
+}
+
 // f32 partial rows [parts][rows][N] of a projection
 const float* slabs(const Tensor& t, int64_t rows, int64_t q, const char* name) {
   check_t(t, true, name);
@@ -391,6 +423,7 @@ void talk_step(Tensor x, int64_t H, int64_t rot_dims, Tensor rope, Tensor positi
 void bind_stack(py::module_& m) {
   m.def("gemm_f32", &gemm_f32, py::arg("x"), py::arg("w"), py::arg("y"), py::arg("epi"), py::arg("residual") = py::none(),
         py::arg("y2") = py::none());
+  m.def("gemm_f32_quarters", &gemm_f32_quarters, py::arg("x"), py::arg("w"), py::arg("y") = py::none());
   m.def("layernorm_f32", &layernorm_f32, pybind11::arg("x"), pybind11::arg("w"), pybind11::arg("b"), pybind11::arg("y"), pybind11::arg("eps"),
         pybind11::arg("parts") = pybind11::none());
   m.def("add_norm", &add_norm);

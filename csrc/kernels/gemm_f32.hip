@@ -50,9 +50,13 @@ VWA_DEVICE void store4(const GemmF32Params& p, int m, int n, const f32x4& v0, co
 // outputs), 4 x 8192 x 1024 9.6 us (3.5 TB/s; 38), 4 x 32768 x 1024 30 us (4.5 TB/s; 50).
 // 16 MT rows x 16 NT columns; the NW waves take one or two of K's KS runs each, U 16-deep steps' loads in
 // flight while the U before are multiplied.
-template <int EPI, int MT, int NT, int KS, int U, int NW>
+// QR: one quarter of the runs to a workgroup (blockIdx.z), its sum to rows of its own p.part further on: the norm behind the
+// product adds the quarters in the order in which they are added up here.  Four times the workgroups for products of few columns: 4 x 1024 x
+// 4096 13.5 -> 6.6 us, 4 x 1024 x 1024 5.5 -> 4.8.
+template <int EPI, int MT, int NT, int KS, int U, int NW, bool QR = false>
 __global__ __launch_bounds__(64 * NW) void rows_f32_kernel(GemmF32Params p) {
-  __shared__ f32x4 part[KS * MT * NT * 64];
+  static_assert(!QR || (EPI == 0 && KS == 4 * NW), "a quarter's runs, a wave each");
+  __shared__ f32x4 part[(QR ? NW : KS) * MT * NT * 64];
   const int lane = threadIdx.x & 63, w = NW == 16 || MT > 1 ? threadIdx.x >> 6 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rl = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.y * 16 * MT, n0 = blockIdx.x * 16 * NT;
@@ -86,8 +90,8 @@ __global__ __launch_bounds__(64 * NW) void rows_f32_kernel(GemmF32Params p) {
         for (int j = 0; j < NT; ++j) acc[i][j] = mfma4x4(a[u][i], b[u][j], acc[i][j]);
   };
 #pragma unroll
-  for (int h = 0; h < KS / NW; ++h) {
-    const int run = w * (KS / NW) + h, s0 = slices * run / KS * 2, n = min(slices * (run + 1) / KS * 2, steps) - s0, full = n / U;
+  for (int h = 0; h < (QR ? 1 : KS / NW); ++h) {
+    const int slot = QR ? w : w * (KS / NW) + h, run = QR ? blockIdx.z * NW + w : slot, s0 = slices * run / KS * 2, n = min(slices * (run + 1) / KS * 2, steps) - s0, full = n / U;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -114,15 +118,16 @@ __global__ __launch_bounds__(64 * NW) void rows_f32_kernel(GemmF32Params p) {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int j = 0; j < NT; ++j) part[(run * MT * NT + i * NT + j) * 64 + lane] = acc[i][j];
+      for (int j = 0; j < NT; ++j) part[(slot * MT * NT + i * NT + j) * 64 + lane] = acc[i][j];
   }
   __syncthreads();
+  if constexpr (QR) p.Y += blockIdx.z * p.part;
   constexpr int NF = EPI == 2 ? MT * NT / 2 : MT * NT;  // (gate and up fragments finish together)
   for (int it = threadIdx.x; it < NF * 64; it += 64 * NW) {
     const int f = it >> 6, i = EPI == 2 ? f / (NT / 2) : f / NT, j = EPI == 2 ? 2 * (f % (NT / 2)) : f % NT;
     f32x4 v0 = {}, v1 = {};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < (QR ? 1 : 4); ++q) {
       f32x4 z0 = {}, z1 = {};
 #pragma unroll
       for (int k = q * (KS / 4); k < (q + 1) * (KS / 4); ++k) {
@@ -318,9 +323,27 @@ void launch(const GemmF32Params& p, hipStream_t st) {
 
 }  // namespace
 
-extern "C" int vwa_gemm_f32(int epi, const GemmF32Params* p, hipStream_t st) {
+namespace {
+int check_f32(const GemmF32Params* p) {
   if (p->M < 1 || p->N < 1 || p->K < 16 || p->K % 16 || p->ldx % 4) return -1;
   if ((reinterpret_cast<uintptr_t>(p->X) & 15) || (reinterpret_cast<uintptr_t>(p->W) & 15)) return -2;
+  return 0;
+}
+}  // namespace
+
+// A product's four quarters (p->part floats apart), or -7: whole, it leaves no CU without columns, or its rows are too many
+extern "C" int vwa_gemm_f32_quarters(const GemmF32Params* p, int cus, int launch, hipStream_t st) {
+  if (const int rc = check_f32(p)) return rc;
+  if (p->M > 16 || 2 * cdiv(p->N, 16) > cus) return -7;
+  if (!launch) return 0;
+  const dim3 grid(cdiv(p->N, 16), 1, 4);
+  if (runs_log2<0>(*p) == 4) hipLaunchKernelGGL((rows_f32_kernel<0, 1, 1, 16, 8, 4, true>), grid, dim3(256), 0, st, *p);
+  else hipLaunchKernelGGL((rows_f32_kernel<0, 1, 1, 8, 8, 2, true>), grid, dim3(128), 0, st, *p);
+  return (int)hipGetLastError();
+}
+
+extern "C" int vwa_gemm_f32(int epi, const GemmF32Params* p, hipStream_t st) {
+  if (const int rc = check_f32(p)) return rc;
   if (epi == 1 && !p->R) return -3;
   if (epi == 6 && (!p->Y2 || p->n_split < 0 || p->n_split > p->N)) return -4;
   if (epi == 2 && p->N % 32) return -5;

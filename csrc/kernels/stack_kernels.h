@@ -14,6 +14,7 @@ struct GemmF32Params {
   float* Y; int ldy;
   const float* R; int ldr;
   int n_split; float* Y2; int ldy2;
+  int64_t part;                     // quarters: floats from one's rows to the next one's
 };
 
 // Rotation of the first rot_dims dimensions of every q / k head (pairs (i, i + rot_dims / 2), table
@@ -97,6 +98,7 @@ struct MinGruParams {
 extern "C" {
 #endif
 int vwa_gemm_f32(int epi, const GemmF32Params* p, hipStream_t st);
+int vwa_gemm_f32_quarters(const GemmF32Params* p, int cus, int launch, hipStream_t st);
 // y (T) [rows, ldy] = layer norm of x f32 rows over D columns (b null: no bias); columns D .. Dpad-1 of y are zeroed
 int vwa_layernorm_f32(float* x, int ldx, const float* br, int ldb, int parts, const float* w, const float* b, void* y, int ldy,
                       int rows, int D, int Dpad, float eps, int f32, hipStream_t st);

@@ -170,6 +170,37 @@ def test_rglru_inert_rows(dtype):
     assert out[[2, 4, 5]].abs().sum() == 0
 
 
+# ----------------------------------------------------------------------------- 32-bit products in quarters
+@pytest.mark.parametrize("M", [1, 3, 16, 17])
+@pytest.mark.parametrize("N,K", [(16, 16), (72, 48), (1024, 1024), (1000, 4096), (2048, 2000), (2048, 4112), (4096, 1024)])
+def test_quarters_of_a_product(M, N, K):
+    """A 32-bit product that leaves its quarters to the norm behind it against the whole one: the same bits, whatever norm adds
+    them (rows of one row side by side, or rows apart)."""
+    x, w = rnd(M, K, seed=1).to(DEV), rnd(N, K, seed=2, std=K ** -0.5).to(DEV)
+    w1, b1, w2 = (rnd(N, seed=s).to(DEV) for s in (3, 4, 5))
+    res = rnd(M, N, seed=6).to(DEV)
+    few = M <= 16 and N <= 2048
+    rows, whole = torch.full((4 * M, N), float("nan"), device=DEV), torch.zeros(M, N, device=DEV)
+    n = ops.linear_rows(x, w, rows)
+    ops.linear(x, w, out=whole)
+    assert n == (4 if few else 1)
+    outs = []
+    for br, k in ((rows[: n * M], n), (whole, 1)):
+        r, h = res.clone(), torch.zeros(M, N, device=DEV)
+        ops.add_norm(r, br, w1, w2, eps=1e-5, out=h, n_parts=k)
+        outs.append((r, h))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    parts = ops.linear_parts(x, w)
+    assert (parts is not None) == few
+    if few and N % 4 == 0:
+        a, ha, hb = res.clone(), torch.zeros(M, N, device=DEV), torch.zeros(M, N, device=DEV)
+        ops.layernorm_f32(a, w1, b1, eps=1e-5, out=ha, parts=parts)
+        b = torch.empty_like(res)
+        ops.linear(x, w, out=b, residual=res)
+        ops.layernorm_f32(b, w1, b1, eps=1e-5, out=hb)
+        assert torch.equal(a, b) and torch.equal(ha, hb)
+
+
 # ----------------------------------------------------------------------------- latent attention
 LATENT = [  # H, dim, rot, vd, rank, block size, n
     (3, 20, 6, 24, 40, 16, 150),

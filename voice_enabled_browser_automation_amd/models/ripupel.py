@@ -287,7 +287,7 @@ class RipupelModel:
         # once, never written (so each distinct layout has rows of its own)
         cols = {D.cols for D in self.dims}
         moes = [(L.mlp.experts, L.mlp.top, F) for L, F in zip(self.cfg.layers, self.ffs) if isinstance(L.mlp, MoEConfig)]
-        parts = max([1] + [t for _, t, _ in moes])
+        parts = max([4 if dt == torch.float32 else 1] + [t for _, t, _ in moes])  # (32-bit products leave quarters, ops.linear_rows)
         lat = [D.H * D.dk for D in self.dims if isinstance(D, LatentDims)]
         dense = [F for L, F in zip(self.cfg.layers, self.ffs) if isinstance(L.mlp, DenseFFConfig)]
         return dict(hidden=e(rows, self.d_pad, t=torch.float32), normed=e(rows, self.d_pad),
@@ -339,20 +339,19 @@ class RipupelModel:
                       tickets=getattr(bufs, "rglru_tickets", None), **rows)
         else:
             self._attend(li, y, cat[:, : D.cols], bufs, M, kv, rows, plan)
-        ops.linear(cat, L.w_out, out=br[:M])
+        parts = ops.linear_rows(cat, L.w_out, br)
         after = self.layers[li + 1].norm1 if li + 1 < self.cfg.n_layers else None
         if C.mlp is None:
-            ops.add_norm(x, br[:M], L.norm1b, after, eps=eps, out=h)
+            ops.add_norm(x, br[: M * parts], L.norm1b, after, eps=eps, out=h, n_parts=parts)
             return
-        ops.add_norm(x, br[:M], L.norm1b, L.norm2, eps=eps, out=h)
-        parts = 1
+        ops.add_norm(x, br[: M * parts], L.norm1b, L.norm2, eps=eps, out=h, n_parts=parts)
         if L.moe is not None:
             parts = L.moe.top
             ops.moe(h, L.moe, slots=rows["slots"], bufs=bufs.moe, out=br[: M * parts])
         else:
             act = bufs.act[: M * self.ffs[li]].view(M, self.ffs[li])
             ops.linear_swiglu(h, L.gate_up, out=act)
-            ops.linear(act, L.down, out=br[:M])
+            parts = ops.linear_rows(act, L.down, br)
         ops.add_norm(x, br[: M * parts], L.norm2b, after, eps=eps, out=h, n_parts=parts)
 
     def _attend(self, li: int, y, out, bufs, M: int, kv, rows, plan) -> None:

@@ -127,10 +127,28 @@ def linear_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
     from . import GEMM_WS_FLOATS, TiledWeight, gemm_ok, rows_take_tiles
 
     M, N = x.shape[0], w.shape[0]
+    if x.is_cuda and x.dtype == torch.float32 and _ext().gemm_f32_quarters(x, w):
+        out = torch.empty(4, M, N, dtype=torch.float32, device=x.device)
+        _ext().gemm_f32_quarters(x, w, out)
+        return out
     if not x.is_cuda or M > PARTS_ROWS or not isinstance(w, TiledWeight) or w.keep_order or not gemm_ok(x, w) or (
             M < 4 and N >= 4096 and not rows_take_tiles(M, w)):
         return None
     return _ext().linear_parts(x, w.t, GEMM_WS_FLOATS)
+
+
+def linear_rows(x: torch.Tensor, w, rows: torch.Tensor) -> int:
+    """x @ w^T to the first rows of ``rows`` for add_norm, as many for a row of x as this returns: one, or (few rows of 32-bit
+    weights) the four quarters of its sums, which add_norm adds in the order of a whole product's."""
+    from . import linear
+
+    M, N = x.shape[0], w.shape[0]
+    if x.is_cuda and x.dtype == torch.float32 and rows.shape[0] >= 4 * M and rows.is_contiguous() and rows.shape[1] == N:
+        if _ext().gemm_f32_quarters(x, w):
+            _ext().gemm_f32_quarters(x, w, rows[: 4 * M].view(M, 4, N).transpose(0, 1))
+            return 4
+    linear(x, w, out=rows[:M])
+    return 1
 
 
 def add_norm(x: torch.Tensor, branch: torch.Tensor, w1: torch.Tensor, w2: Optional[torch.Tensor], *, eps: float,
