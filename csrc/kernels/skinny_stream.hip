@@ -218,14 +218,25 @@ __global__ __launch_bounds__(KS * 64) void skinny_stream_kernel(SkinnyParams p, 
 
 int g_x_skew = 32;  // LDS X row skew (elements per 4 rows; 0: none -- A/B knob, vwa_skinny_set_x_skew)
 
+// Persistent workgroups of a launch: grid_cap (one a CU) times what a CU holds.  Of four waves (K < 2048; 148 - 189 registers) that
+// is three, two of the QKV epilogue, where the X rows leave LDS for them: more weight bytes are on the way, and tiles past one a CU
+// are not drawn one after the other.  us at one / two / three a CU, 8 rows: 5120 x 1280 10.7 / 9.9 / 9.9, 51872 x 1280 43.0 / 36.0 /
+// 33.0, 32768 x 1024 27.5 / 21.9 / 21.0, 6144 x 1536 11.7 / 10.7 / 10.7; fp8 weights 32768 x 1024 17.5 / 15.8 / 14.8, 8192 x 1024 7.9 / 7.7
+// / 7.6; up to 256 tiles the same launch.
+template <int EPI, int KS>
+int grid_of(int ntiles, int grid_cap, size_t lds) {
+  int per = KS == 4 ? EPI == EPI_QKV ? 2 : 3 : 1;
+  while (per > 1 && per * lds > 160 * 1024) --per;
+  return ntiles < grid_cap * per ? ntiles : grid_cap * per;
+}
+
 template <int EPI, int NT, int KS, bool XG, int MT = 1>
 int launch_v(const SkinnyParams& p, hipStream_t st, int grid_cap, size_t lds, int xstride) {
   constexpr int U = MT > 1 ? 1 : XG ? 2 : 4 / NT;
   const int G = p.K / 128;
   const int per_wave = (G + KS - 1) / KS;
   const int nb = (per_wave + U - 1) / U;
-  const int ntiles = p.N / (16 * NT);
-  const int grid = ntiles < grid_cap ? ntiles : grid_cap;
+  const int grid = grid_of<EPI, KS>(p.N / (16 * NT), grid_cap, lds);
   hipLaunchKernelGGL((skinny_stream_kernel<EPI, NT, KS, XG, MT>), dim3(grid), dim3(KS * 64), lds, st, p, nb, xstride,
                      XG ? 0 : g_x_skew);
   return 0;
@@ -245,7 +256,7 @@ int launch(const SkinnyParams& p0, hipStream_t st, int grid_cap) {
   // projection's 14336-wide rows at more than ~5 rows) streamed from L2 with the weights (XG)
   const bool lds_x = xbytes + red <= 160 * 1024;
   if (p.col_mask) {  // the masked tile list: NT 1, EPI store, LDS-staged X, <= 64 tiles per workgroup
-    const int ntiles = p.N / (16 * NT), grid = ntiles < grid_cap ? ntiles : grid_cap;
+    const int ntiles = p.N / (16 * NT), grid = grid_of<EPI, KS>(ntiles, grid_cap, xbytes + red);
     if (EPI != EPI_STORE || NT != 1 || !lds_x || (ntiles + grid - 1) / grid > 64 || p.col_mask_rows < 1)
       p.col_mask = nullptr;
   }
@@ -406,8 +417,7 @@ int launch_fp8(const SkinnyParams& p, hipStream_t st, int grid_cap) {
   const size_t xbytes = ((size_t)p.M * xstride + 15) & ~(size_t)15;
   const size_t lds = xbytes + (size_t)(KS * NT * 4 * 64 + 32) * sizeof(float);
   if (lds > 160 * 1024) return -10;
-  const int ntiles = p.N / (16 * NT);
-  const int grid = ntiles < grid_cap ? ntiles : grid_cap;
+  const int grid = grid_of<EPI, KS>(p.N / (16 * NT), grid_cap, lds);
   hipLaunchKernelGGL((skinny_fp8_kernel<EPI, NT, KS>), dim3(grid), dim3(KS * 64), lds, st, p, nb, xstride);
   return 0;
 }
