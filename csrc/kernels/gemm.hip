@@ -1040,7 +1040,7 @@ struct Plan {
   bool p8;
   int splits;
 };
-Plan plan(const GemmParams& p) {
+Plan plan(const GemmParams& p, float* took = nullptr) {
   const int KG = p.K / BKG;
   Plan best{false, 1};
   float least = 0.f;
@@ -1054,7 +1054,26 @@ Plan plan(const GemmParams& p) {
       }
     }
   }
+  if (took) *took = least;
   return best;
+}
+
+// Columns of a product that fill whole rounds of the CUs with large tiles, where it is cheaper by the estimate to give the rest a
+// launch of its own, with tiles and slices of its own (0: not).  The tiles past the last whole round cost nearly a round of their
+// own, however few: 2048 x 32896 x 4096 is four rounds and eight tiles, 482 -> 438 us in two launches (398 of them the whole rounds').
+// 1024 x 17664 x 2048 86 -> 76 us, 1300 x 22528 x 4096 238 -> 206, 1900 x 26624 x 4096 341 -> 333.
+int whole_rounds(const GemmParams& p) {
+  if (p.M < 128 || p.keep_order || p.sw || p.nbatch > 1 || p.cus <= 0 || g_p8_mode != 2 || g_split_fill_pct != 0) return 0;
+  const int mb = cdiv(p.M, 256), nb = cdiv(p.N, 256), tiles = mb * nb;
+  const int cols = mb <= p.cus ? (int)((int64_t)(tiles / p.cus) * p.cus / mb) : 0;  // column tiles of the whole rounds
+  if (cols < 1 || cols * 256 >= p.N) return 0;
+  float whole, rest;
+  plan(p, &whole);
+  GemmParams a = p, b = p;
+  a.N = cols * 256;
+  b.N = p.N - a.N;
+  plan(b, &rest);
+  return estimate(a, true, 1) + rest + 3.f < 0.97f * whole ? a.N : 0;
 }
 
 // K slices of a bf16 product of <= 64 rows and of fp8 weights (W8A16): the cheapest by an estimate in us, fitted to 270 timings
@@ -1294,6 +1313,34 @@ extern "C" int vwa_gemm(int epi, const GemmParams* pp, hipStream_t st) {
     case EPI_SPLIT: return launch_epi<EPI_SPLIT>(p, st, p8);
     default: return -3;
   }
+}
+
+// The first n columns of a product whose columns two launches share (vwa_gemm_cut), and the others
+extern "C" void vwa_gemm_part(int epi, const GemmParams* pp, int n, int second, GemmParams* part) {
+  GemmParams p = *pp;
+  if (!second) {
+    p.N = n;
+    p.n_split = p.n_split < n ? p.n_split : n;
+  } else {
+    const int out = epi == EPI_SWIGLU ? n / 2 : n;
+    p.N -= n;
+    p.W += (size_t)n * p.K;
+    if (p.bias) p.bias += n;
+    if (p.R) p.R += p.y_f32 == 2 ? 2 * out : out;
+    if (epi == EPI_SPLIT) {
+      if (n > p.n_split) p.Y2 += n - p.n_split;
+      p.n_split = p.n_split > n ? p.n_split - n : 0;
+    }
+    p.Y = reinterpret_cast<char*>(p.Y) + (size_t)out * (p.y_f32 ? 4 : 2);
+    p.ss_zero = nullptr;
+  }
+  *part = p;
+}
+
+extern "C" int vwa_gemm_cut(int epi, const GemmParams* pp) {
+  GemmParams p = *pp;
+  p.keep_order = keeps_order(epi, p);
+  return epi == EPI_STORE || epi == EPI_RESID || epi == EPI_SWIGLU || epi == EPI_GELU || epi == EPI_SPLIT ? whole_rounds(p) : 0;
 }
 
 extern "C" int vwa_gemm_grouped(int epi, const GemmParams* pp, hipStream_t st) {

@@ -77,3 +77,23 @@ def test_slices_of_few_rows_are_those_of_the_weight(E, kw):
             assert len(s) == 1, (N, K, s)
             seen |= s
     assert {1, 4, 8, 16} <= seen
+
+
+def test_columns_of_two_launches_are_whole_rounds(E):
+    """The first launch's columns: large tiles that fill the CUs a whole number of times, never all of them; products that keep an
+    order, few rows and switched-off tiles have one launch."""
+    seen = 0
+    for M in (128, 600, 1011, 1900, 2048, 4096, 12000):
+        for N in (4096, 8208, 9472, 17664, 22528, 28672, 32896):
+            for K in (128, 1024, 4096):
+                cut = E.gemm_cut(0, M, N, K)
+                assert 0 <= cut < N and cut % 256 == 0
+                if cut:
+                    seen += 1
+                    rows = -(-M // 256)
+                    tiles = rows * cut // 256
+                    assert tiles // 256 * 256 <= tiles and -(-tiles // 256) * 256 - tiles < rows  # (no column tile more fits its rounds)
+                assert E.gemm_cut(0, M, N, K, keep_order=True) == 0 and E.gemm_cut(5, M, N, K) == 0
+    assert seen > 5 and E.gemm_cut(0, 64, 32896, 4096) == 0 and E.gemm_cut(6, 2048, 32896, 4096) == 32768
+    E.gemm_set_p8(0)
+    assert E.gemm_cut(0, 2048, 32896, 4096) == 0

@@ -732,6 +732,46 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("M,N,K,n_split", [(2048, 8256, 1024, 8192), (2000, 8208, 1408, 4096), (1900, 8448, 1408, 8400)])
+def test_gemm_of_two_launches(M, N, K, n_split, tiled):
+    """A product whose last columns have a launch of their own against a single launch, over the epilogues: the first columns to the
+    bit, the others to one rounding of the result and K additions (2^-24 of a partial sum each, twice: either launch's own order).
+    The split falls on the cut, in front of it and behind it."""
+    E = ops.ext()
+    cut = E.gemm_cut(0, M, N, K)
+    assert cut == 8192
+    x, w, b = rnd(M, K), rnd(N, K, scale=K ** -0.5), rnd(N)
+    ww, wt = (ops.TiledWeight(w).t, True) if tiled else (w, False)
+    rstd = torch.rand(M, device=DEV) + 0.5
+    res, resf = rnd(M, N), torch.randn(M, N, device=DEV)
+    near = lambda a, e, sure, f32=False: float(((a.double() - e.double()).abs() - (0 if f32 else 2.0 ** -7 * e.double().abs())).max()) < sure
+
+    def both(epi, make, of, **kw):
+        got = []
+        for ws in (ops.GEMM_WS_FLOATS, 0):
+            y = make()
+            args = {k: v() if callable(v) else v for k, v in kw.items()}
+            E.gemm(x, ww, args.pop("bias", None), y, epi, rstd, w_tiled=wt, ws_floats=ws, **args)
+            got.append((y, args))
+        (a, ka), (e, ke) = got
+        assert torch.equal(a[:, :of], e[:, :of]) and near(a, e, 1e-3 if epi != 2 else 5e-3, a.dtype == torch.float32)
+        return ka, ke
+
+    bf = lambda n=N: (lambda: torch.full((M, n), 7.0, dtype=BF, device=DEV))
+    both(0, bf(), cut, bias=b)
+    both(0, lambda: torch.full((M, N), 7.0, device=DEV), cut)
+    both(1, bf(), cut, bias=b, residual=res)
+    both(1, lambda: torch.full((M, N), 7.0, device=DEV), cut, residual=resf)
+    both(2, bf(N // 2), cut // 2) if N % 32 == 0 else None
+    both(3, bf(), cut, bias=b)
+    ka, ke = both(6, bf(n_split), min(cut, n_split), y2=bf(N - n_split))
+    assert near(ka["y2"], ke["y2"], 1e-2) and torch.equal(ka["y2"][:, : max(0, cut - n_split)], ke["y2"][:, : max(0, cut - n_split)])
+    ss = lambda v: (lambda: torch.full((M,), v, dtype=torch.int64, device=DEV))
+    ka, ke = both(1, bf(), cut, residual=res, ss_out=ss(5), ss_zero=ss(3))
+    assert ka["ss_zero"].abs().sum() == 0 and near(ka["ss_out"], ke["ss_out"], 0)
+
+
 @pytest.mark.parametrize("mode,M,N,K,kind", [(*c, k) for c in ((2, 17, 400, 128), (2, 64, 384, 128), (2, 200, 400, 128), (1, 300, 512, 128),
                                                                (2, 1500, 384, 384))
                                              for k in ("tiled", "rowmajor", "fp8") if k != "fp8" or c[1] <= 64])  # (more: 8-bit x)
