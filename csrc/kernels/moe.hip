@@ -18,7 +18,14 @@ namespace {
 constexpr size_t kMaxLds = 160 * 1024 - 8192;
 constexpr int kRouteWaves = 8, kRouteThreads = kRouteWaves * 64, kMaxExperts = 256;
 
+// Experts whose places among a row's choices are counted: a lane each of the 32 that a row has.  The launch is bound by its serial
+// chain (loads, sums, choices, groups), and the choices one after another are top x 5 dependent exchanges of it.  us, chosen in turn ->
+// counted, top 4: bf16, K 2048, 16 rows of 16 experts 8.1 -> 6.5; K 1024, 48 rows 9.2 -> 7.5; 24 experts 10.5 -> 9.2; f32, K 1024,
+// 4 rows 7.5 -> 6.0.  Of more experts than lanes a lane would count several, and a maximum after another stays.
+constexpr int kRankExperts = 32;
+
 // pairs -> tiles of one expert each (the whole workgroup); id_of(pair): its expert
+// (One wave that counts expert after expert from ballots, without LDS and barriers: 0.25 us an expert.)
 template <class F>
 VWA_DEVICE void group_pairs(const MoeRouteParams& p, F&& id_of) {
   __shared__ int cnt[kMaxExperts], first[kMaxExperts], s_total;
@@ -109,6 +116,24 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
   int* lds_ids = reinterpret_cast<int*>(red);        // (a launch of one workgroup groups from here)
   __syncthreads();
   const int r = tid >> 5, q = tid & 31, row = r0 + r;  // 32 lanes per row: the choices stay inside a wave
+  if (p.E <= kRankExperts) {
+    // an expert's place is the number of experts ahead of it (a larger score; of equal ones the lower number): all choices at once
+    // where one maximum after another is a chain of lane exchanges.  (Not a number: behind every other.)
+    auto known = [](float v) { return v == v ? v : -2.5f; };
+    const float* s = sc + r * (Ep + 1);
+    const float v = known(s[min(q, p.E - 1)]);
+    int place = q < p.E ? 0 : p.E;
+#pragma unroll 4
+    for (int o = 0; o < p.E; ++o) {
+      const float u = known(s[o]);
+      place += u > v || (u == v && o < q) ? 1 : 0;
+    }
+    if (place < p.top && r < nr) {
+      p.wts[row * p.top + place] = live ? v : 0.f;
+      lds_ids[r * p.top + place] = live ? q : -1;
+      __hip_atomic_store(p.ids + row * p.top + place, live ? q : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  } else
   for (int k = 0; k < p.top; ++k) {
     float best = -3.f;
     int at = 0;

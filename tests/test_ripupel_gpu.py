@@ -449,6 +449,35 @@ def test_moe(dtype, E, top, ff, d, M, monkeypatch):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [1, 16, 17])
+@pytest.mark.parametrize("E,top", [(1, 1), (2, 2), (16, 4), (31, 31), (32, 1), (32, 32), (33, 33), (40, 3)])
+def test_route_of_equal_scores(dtype, rows, E, top):
+    """Both ways to choose (E up to 32 and above): the best first, of equal scores the lower number, inert rows none, every
+    pair in a tile of its expert.  Whole numbers of few bits add up exactly in any order, so that equal scores are equal."""
+    K, tile = 128, 16
+    h = torch.randint(-1, 2, (rows, K), generator=torch.Generator().manual_seed(1)).to(dtype)
+    router = torch.zeros(up(E, 16), K, dtype=dtype)
+    router[:E, : max(1, E // 4)] = torch.randint(-2, 3, (E, max(1, E // 4)), generator=torch.Generator().manual_seed(2)).to(dtype) / 4
+    s = O.sigmoid(h.double() @ router[:E].double().T)
+    val, idx = s.sort(dim=1, descending=True, stable=True)
+    slots = torch.zeros(rows, dtype=torch.int64)
+    if rows > 2:
+        slots[rows // 2] = -1
+    live = slots >= 0
+    bufs = ops.moe_buffers(rows, [(E, top, 128)], dtype, DEV)
+    n = mixers.moe_tiles(rows * top, E, tile)
+    tiles, order = bufs.tiles[: 1 + 3 * n], bufs.order[: n * tile]
+    for _ in range(2):
+        ops.ext().moe_route(h.to(DEV), ops.fragments(router.to(DEV)), E, top, slots.to(DEV), bufs.wts, bufs.ids, tile, tiles, order, bufs.ticket)
+        ids, wts = bufs.ids.cpu().view(rows, top), bufs.wts.cpu().view(rows, top)
+        assert torch.equal(ids[live].long(), idx[live][:, :top]) and (ids[~live] == -1).all() and (wts[~live] == 0).all()
+        assert rel(wts[live], val[live][:, :top]) < 1e-6  # (a sigmoid in f32: a few units in the last place)
+        t = tiles.cpu()
+        pairs = {int(p): int(e) for e, at, m in t[1: 1 + 3 * int(t[0])].view(-1, 3).tolist() for p in order.cpu()[at: at + m]}
+        assert pairs == {i: int(e) for i, e in enumerate(ids.flatten()) if e >= 0}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,top,ff,d", [(12, 2, 1536, 130), (3, 2, 8320, 40), (16, 4, 1100, 520)])
 def test_moe_sets_in_flight(dtype, E, top, ff, d, monkeypatch):
     """The forms of the small tiles' loop: gate / up with one set between two and five workgroups a CU (the first two), one to
