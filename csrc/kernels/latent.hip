@@ -180,8 +180,7 @@ VWA_DEVICE void attn_weights(const f32x4& sc_raw, float sl2, int key0, int pos, 
     sc[i] = key0 + 16 * w + 4 * g + i <= pos ? sc_raw[i] * sl2 : -1e30f;
     mx = fmaxf(mx, sc[i]);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = groups_max(mx);
   if (g == 0) s_max[w][rl] = mx;
   lds_sync();
   float mn = m;
@@ -207,8 +206,7 @@ template <int NT>
 VWA_DEVICE void attn_finish(const LatentAttnParams& p, const Item& x, float m, float l, const f32x4 (&acc)[NT]) {
   __shared__ float s_sum[4][16];
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, g = lane >> 4, tid = threadIdx.x;
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = groups_sum(l);
   if (g == 0) s_sum[w][rl] = l;
   lds_sync();
   if (tid < x.Hb) {                                  // (every wave holds the same maximum; tid = head here)
@@ -454,8 +452,7 @@ __global__ __launch_bounds__(kOutThreads) void latent_out_kernel(LatentOutParams
         const float2 v = st[(size_t)k * p.H];
         if (v.y > 0.f) mx = fmaxf(mx, v.x);
       }
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 32));
+      mx = half_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
       float sum = 0.f;
       for (int k = k0; k < p.nch; k += 32) {
         const float2 v = st[(size_t)k * p.H];
@@ -463,8 +460,7 @@ __global__ __launch_bounds__(kOutThreads) void latent_out_kernel(LatentOutParams
         fac[r * p.nch + k] = e;
         sum += v.y * e;
       }
-#pragma unroll
-      for (int o = 16; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 32);
+      sum = half_reduce(sum, [](float a, float b) { return a + b; });
       const float inv = 1.f / (sum + __builtin_amdgcn_exp2f(sink - mx));
       for (int k = k0; k < p.nch; k += 32) fac[r * p.nch + k] *= inv;
     }

@@ -571,8 +571,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
         pv[4 * t + i] = v;
         mx = fmaxf(mx, v);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = groups_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float alpha = (m_run == -INFINITY) ? 0.f : exp2f(m_run - m_new);
     float ps = 0.f;
@@ -633,8 +632,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   }
 
   // ---- per-wave (m, l, O) -> LDS; O^T accumulator of lane (n, g): dims 16dt + 4g + i
-  float l_tot = l_run + __shfl_xor(l_run, 16, 64);
-  l_tot += __shfl_xor(l_tot, 32, 64);
+  const float l_tot = groups_sum(l_run);
   if (g == 0) {
     mlw[(w * kMqCols + n) * 2 + 0] = m_run;
     mlw[(w * kMqCols + n) * 2 + 1] = l_tot;

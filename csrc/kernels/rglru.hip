@@ -108,10 +108,12 @@ VWA_DEVICE float scan_tile(const float (&a)[4], const float (&bb)[4], float carr
     pb[i] = a[i] * pb[i - 1] + bb[i];
   }
   // the lane groups in front: (ea, eb)
-  float ea = 1.f, eb = 0.f, ta = 1.f, tb = 0.f;
+  float ea = 1.f, eb = 0.f, ta = 1.f, tb = 0.f, ga[4], gb[4];
+  group_values(pa[3], ga);
+  group_values(pb[3], gb);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const float ka = __shfl(pa[3], (lane & 15) + 16 * k, 64), kb = __shfl(pb[3], (lane & 15) + 16 * k, 64);
+    const float ka = ga[k], kb = gb[k];
     tb = ka * tb + kb;
     ta = ka * ta;
     if (k + 1 == g) {

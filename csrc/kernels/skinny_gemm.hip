@@ -173,13 +173,11 @@ __global__ __launch_bounds__(KS * 64) void skinny_gemm_kernel(SkinnyParams p) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       float v = ssq[mt];
-      v += __shfl_xor(v, 16, 64);
-      v += __shfl_xor(v, 32, 64);
+      v = groups_sum(v);
       if (lane < 16) red_ssq[w * MT * 16 + mt * 16 + lane] = v;
       if (ln) {
         float t = ssum[mt];
-        t += __shfl_xor(t, 16, 64);
-        t += __shfl_xor(t, 32, 64);
+        t = groups_sum(t);
         if (lane < 16) red_sum[w * MT * 16 + mt * 16 + lane] = t;
       }
     }

@@ -126,15 +126,13 @@ VWA_DEVICE void store_scores(const TalkAttnParams& p, const Unit& un, int ri, in
                                    (chunk * kTalkStat + w + 4 * u) * kTile + 4 * b) =
             make_float4(acc[u][0], acc[u][1], acc[u][2], acc[u][3]);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  mx = groups_max(mx);
   float l = 0.f;
 #pragma unroll
   for (int u = 0; u < NU; ++u)
 #pragma unroll
     for (int i = 0; i < 4; ++i) l += acc[u][i] == -INFINITY ? 0.f : __expf(acc[u][i] - mx);
-  l += __shfl_xor(l, 16, 64);
-  l += __shfl_xor(l, 32, 64);
+  l = groups_sum(l);
   if (b == 0) {
     sm[w][rl][0] = mx;
     sm[w][rl][1] = l;
@@ -409,12 +407,15 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
       if (ms.y > 0.f) s = (s > 0.f ? s * __expf(m - mn) : 0.f) + ms.y * __expf(ms.x - mn);
       m = mn;
     }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) {
-      const float mo = __shfl_xor(m, o, 64), so = __shfl_xor(s, o, 64), mn = fmaxf(m, mo);
+    auto merge = [&](float mo, float so) {
+      const float mn = fmaxf(m, mo);
       s = (s > 0.f ? s * __expf(m - mn) : 0.f) + (so > 0.f ? so * __expf(mo - mn) : 0.f);
       m = mn;
-    }
+    };
+    merge(row_ror<8>(m), row_ror<8>(s));
+    merge(row_ror<4>(m), row_ror<4>(s));
+    merge(row_ror<2>(m), row_ror<2>(s));
+    merge(row_ror<1>(m), row_ror<1>(s));
     if ((threadIdx.x & 15) == 0) {
       hm[i] = m;
       hl[i] = 1.f / s;

@@ -127,11 +127,11 @@ VWA_DEVICE float2 nd_stage(const WdecParams& p, const float* part, const u16* ba
     if (tx < 64) {
       const float l = bits_f(ml.y);
       float m = bits_f(ml.x);
-      m = fmaxf(m, __shfl_xor(m, 1, 64));
-      m = fmaxf(m, __shfl_xor(m, 2, 64));
+      m = fmaxf(m, quad_xor<1>(m));
+      m = fmaxf(m, quad_xor<2>(m));
       const float e = __expf(bits_f(ml.x) - m) * l;
-      float den = e + __shfl_xor(e, 1, 64);
-      den += __shfl_xor(den, 2, 64);
+      float den = e + quad_xor<1>(e);
+      den += quad_xor<2>(den);
       if (tx < NP) cw[tx] = e / den;
     }
     lds_sync();
