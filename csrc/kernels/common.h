@@ -211,7 +211,28 @@ VWA_DEVICE uint32_t cvt_pk_fp8(float a, float b) {
 
 VWA_DEVICE float silu(float x) { return x / (1.f + __expf(-x)); }
 
-VWA_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
+// x Phi(x) = max(x, 0) - t Q(t), t = |x|, Q(t) = exp(-t^2 / 2) P(t) the normal tail.  P = exp(t^2 / 2) Q falls from 1/2 as 1 / t:
+// a polynomial in m = t / (t + 4.5), P(0) = 1/2 exactly, fitted here (least maximal relative error, 7e-9 up to t = 5; less is asked
+// of tails that vanish beside any result).  No branch and 16 vector instructions of which 2 are transcendental, where erff has two
+// branches of some 20 each, gone through element by element: an epilogue's waves do nothing else meanwhile.  us of a product with it,
+// 0.5 x (1 + erff(x / sqrt 2)) -> here (without: in brackets): 12000 x 5120 x 1280 197 -> 164 (145), 1500 x 5120 x 1280 32.5 -> 27.6
+// (25.1), 1500 x 2048 x 512 17.3 -> 12.3 (9.9), 8 x 5120 x 1280 9.0 -> 8.4 (7.8).
+// Error against 64 bits, |x| < 14: at most 4.5e-7 -> 2.4e-7, mean 1.5e-8 -> 1.1e-8; and relative, in [-4, -2), where 1 + erf
+// cancels, 4.7e-4 -> 1.5e-6.  NaN and -infinity give NaN, infinity itself, either way.
+VWA_DEVICE float gelu_erf(float x) {
+  const float t = fminf(fabsf(x), 14.5f), m = t * __builtin_amdgcn_rcpf(t + 4.5f);
+  float p = -0.10658054f;
+  p = fmaf(p, m, 0.38831303f);
+  p = fmaf(p, m, -0.33956796f);
+  p = fmaf(p, m, -0.78959513f);
+  p = fmaf(p, m, 2.66286087f);
+  p = fmaf(p, m, -3.78760266f);
+  p = fmaf(p, m, 3.26723218f);
+  p = fmaf(p, m, -1.79523969f);
+  p = fmaf(p, m, 0.5f);
+  const float e = __builtin_amdgcn_exp2f(t * t * -0.72134752f);
+  return fmaf(-(t * e), p, fmaf(0.5f, x, 0.5f * fabsf(x)));
+}
 
 // Bijective XCD-aware remap of a 1-D block index (8 XCDs, each with a private L2):
 // consecutive logical tiles land on the same XCD so neighbouring tiles share L2 lines.
