@@ -58,9 +58,10 @@ constexpr int kGroup = 4;  // row blocks of a grouped launch that walk the colum
 //   CfgP8, 256 x 256: 8 waves of 128 x 64, 144 KB, one per CU: a quarter less read from LDS per MFMA where its tiles fill the
 //     CUs (1011 x 28672 x 4096 237 -> 179 us) or their slices do (choose())
 //   CfgF, CfgFs: <= 64 and <= 32 rows, bf16 or fp8 weights
-template <int BM_, int BN_, int WM_, int WN_>
+// GROUPS: groups of WM x WN waves that take the stages of K in turn; their sums are added in LDS
+template <int BM_, int BN_, int WM_, int WN_, int GROUPS_ = 1>
 struct Cfg {
-  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, NW = WM_ * WN_, THREADS = 64 * NW;
+  static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, GROUPS = GROUPS_, NW = WM_ * WN_, THREADS = 64 * NW * GROUPS;
   static constexpr int FM = BM / WM / 16, FN = BN / WN / 16;  // MFMA fragments per wave
   static constexpr int A_BYTES = BM * 128, STAGE = BM * 128 + BN * 128;
   // W8A16 stage: a full k-group -- two bf16 A half images + the fp8 B block of every tile
@@ -68,12 +69,15 @@ struct Cfg {
   static constexpr int NCOL_MAX = BN / WN;
   static constexpr int EPI_LDS = NW * (FM * 16) * (NCOL_MAX * 2 + 16);
   static constexpr int NST = BM <= 32 ? 4 : BM <= 64 ? 3 : 2;   // stage buffers: few rows take what lets two workgroups share a CU
-  static constexpr int LDS = NST * STAGE > EPI_LDS ? NST * STAGE : EPI_LDS;
+  static constexpr int LDS = GROUPS * NST * STAGE > EPI_LDS ? GROUPS * NST * STAGE : EPI_LDS;
   static constexpr int W8NST = BM <= 32 ? 3 : 2;
   static constexpr int W8LDS = W8NST * W8STAGE > EPI_LDS ? W8NST * W8STAGE : EPI_LDS;
   static_assert((BM / 8) % NW == 0 && (BN / 8) % NW == 0, "whole LDS-DMA instructions per wave");
 };
 using CfgS = Cfg<128, 128, 2, 2>;
+// The same with two groups of four waves that take the stages in turn, one workgroup per CU: below.
+using CfgK = Cfg<128, 128, 2, 2, 2>;
+using CfgKw = Cfg<128, 192, 2, 2, 2>;
 // Few rows (<= 64: one row block): 64 x 128, 4 waves of 64 x 32, 2 workgroups per CU.  Such a product is weights arriving and
 // little else, so what counts is how many of their bytes are on the way.
 // bf16: three 24 KB stages where the 128-row tile had two of 32 KB, half of them rows that are not there (and one stage in flight
@@ -96,8 +100,8 @@ VWA_DEVICE __amdgpu_buffer_rsrc_t rsrc(const void* base, size_t bytes) {
                                            (int)(bytes < 0x7FFFFFF0ull ? bytes : 0x7FFFFFF0ull), 0x00020000);
 }
 
-VWA_DEVICE void dma16(__amdgpu_buffer_rsrc_t r, char* lds_wave_base, unsigned voff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_wave_base, 16, voff, 0, 0,
+VWA_DEVICE void dma16(__amdgpu_buffer_rsrc_t r, char* lds_wave_base, unsigned voff, unsigned soff = 0) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds_wave_base, 16, voff, soff, 0,
                                            0);
 }
 
@@ -278,6 +282,15 @@ VWA_DEVICE void compute_stage(const char* buf, f32x4 (&acc)[C::FM][C::FN], int w
 // 1425, 2048 x 4096 x 22528 1106 -> 1226 -> 1329, 1011 x 28672 x 4096 SwiGLU 1020 -> 1217 -> 1244.
 using CfgP8 = Cfg<256, 256, 2, 4>;
 
+// ---- 128 x 128 | 192 tile, two groups of 4 waves (each 64 x 64 | 96): products whose tiles are one to a CU at most.  Four waves
+// alone in a CU read a stage, multiply it and wait for the next by turns (1.27 us per k-group where two workgroups to a CU take 0.92
+// each; three and four stages ahead, or eight waves on the same stage, are 0 - 5 % faster).  Here group g takes the stages
+// g, g + 2, .. and runs one barrier behind the other: one reads while the other multiplies, and the sums meet in LDS at the end.
+//   A group's turn: operand reads; barrier; the next but one stage's DMA into what was read, MFMAs, wait for the next stage; barrier.
+//   (A ring of five stages, DMA between the MFMAs: the same.  Both groups at once, with one barrier per two stages: 52 us of
+//   the 41 below.  A CU draws 57 bytes a ns then, 64 on the 256^2 tile and 70 at most: the wide tile needs a sixth less of it.)
+// us, alone or two to a CU -> two groups: 1011 x 4096 x 4096 48.1 -> 40.9, 2048 x 2048 x 2048 28.2 -> 23.8, 700 x 1280 x 1280 (in
+// slices before) 20.6 -> 15.2; 192 columns: 1011 x 6144 x 4096 62.8 -> 54.0, 130 x 12288 x 2048 29.4 -> 24.0.
 // half-tile `which` (0 A-lo, 1 A-hi, 2 B-lo, 3 B-hi) into the stage image `st`: 16 wave-instructions of 1 KB, 2 per
 // wave, from the byte offsets voff (past the resource: zeros) + soff
 VWA_DEVICE void p8_issue(__amdgpu_buffer_rsrc_t r, const unsigned (&voff)[8], unsigned soff, int which, char* st) {
@@ -614,7 +627,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   }
   const int KG = p.K / BKG;
   const int kg0 = split * p.kg_per_split, kg1 = min(KG, kg0 + p.kg_per_split);
-  const int w = threadIdx.x >> 6, wm = w / C::WN, wn = w % C::WN;
+  const int w = C::GROUPS > 1 ? (threadIdx.x >> 6) % C::NW : threadIdx.x >> 6, wm = w / C::WN, wn = w % C::WN;
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -697,6 +710,82 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     }
     if (wm == 0) asm volatile("s_barrier" ::: "memory");  // (group 1 started one barrier later)
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // (the epilogue reuses the LDS)
+  } else if constexpr (C::GROUPS == 2) {
+    static_assert(C::NST == 2 && !F8 && !W8 && !GRP && LINES, "two K groups: bf16 products that keep no order");
+    const int l = lane_id(), rl = l & 15, g = l >> 4, grp = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * C::NW)), n = nh / 2;
+    constexpr int PA = C::BM / 8 / C::NW, PB = C::BN / 8 / C::NW;
+    char* const mine = lds + grp * 2 * C::STAGE;
+    unsigned xoff[PA], woff[PB];  // this lane's pieces of a stage (k-group 0)
+#pragma unroll
+    for (int it = 0; it < PA; ++it) {
+      const int r = 8 * (it * C::NW + w) + (l >> 3), m = bm + r;
+      xoff[it] = m < p.M ? p8_x_piece<F8, LINES>(m, p.ldx, r, l) : kPastEnd;
+    }
+#pragma unroll
+    for (int it = 0; it < PB; ++it) {
+      const int q = it * C::NW + w, T = (bn >> 4) + (q >> 1);
+      woff[it] = T * 16 < p.N ? p8_w_piece<F8, WT, LINES>(T, q & 1, p.K, l) : kPastEnd;
+    }
+    // this group's stage i (past the last: on empty resources, so that the waits stay one constant)
+    auto issue = [&](int i) {
+      const bool in = i < n;
+      const int s = h0 + 2 * i + grp;
+      char* to = mine + (i & 1) * C::STAGE + w * 1024;
+      const __amdgpu_buffer_rsrc_t ra = rsrc(p.X, in ? x_bytes : 0), rb = rsrc(p.W, in ? w_bytes : 0);
+      const unsigned sa = p8_x_step<F8, LINES>(s, in), sb = p8_w_step<F8, WT, LINES>(s, in);
+#pragma unroll
+      for (int it = 0; it < PA; ++it) dma16(ra, to + it * C::NW * 1024, xoff[it], sa);
+#pragma unroll
+      for (int it = 0; it < PB; ++it) dma16(rb, to + C::A_BYTES + it * C::NW * 1024, woff[it], sb);
+    };
+    issue(0);
+    issue(1);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PER) : "memory");
+    if (grp == 1) asm volatile("s_barrier" ::: "memory");
+    for (int i = 0; i < n; ++i) {
+      const char* st = mine + (i & 1) * C::STAGE;
+      const char* la = st + (wm * FM * 16 + rl) * 128;
+      const char* lb = st + C::A_BYTES + (wn * FN) * 2048 + l * 16;
+      bf16x8 a[FM][2], b[FN][2];
+#pragma unroll
+      for (int sp = 0; sp < 2; ++sp) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) b[j][sp] = *reinterpret_cast<const bf16x8*>(lb + j * 2048 + sp * 1024);
+#pragma unroll
+        for (int j = 0; j < FM; ++j) a[j][sp] = *reinterpret_cast<const bf16x8*>(la + j * 16 * 128 + ((chunk_of(g, sp) ^ swzk(rl >> 1)) << 4));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (read by all of the group: free)
+      issue(i + 2);
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int sp = 0; sp < 2; ++sp)
+#pragma unroll
+        for (int ii = 0; ii < FM; ++ii)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[ii][j] = mfma16(a[ii][sp], b[j][sp], acc[ii][j]);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PER) : "memory");  // (the next stage has landed)
+    }
+    if (grp == 0) asm volatile("s_barrier" ::: "memory");  // (group 1 started one barrier later)
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    f32x4* ex = reinterpret_cast<f32x4*>(lds) + w * FM * FN * 64 + l;
+    if (grp == 1) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) ex[(i * FN + j) * 64] = acc[i][j];
+    }
+    __syncthreads();
+    if (grp == 0) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] += ex[(i * FN + j) * 64];
+    }
+    __syncthreads();  // (the epilogue writes LDS again)
+    if (grp == 1) return;
   } else {
   if (nh > 0) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0, lds, rows);
   if (nh > 1) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
@@ -803,12 +892,14 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     char* wl = lds + w * (PI * 16 * RSF);
 #pragma unroll
     for (int i0 = 0; i0 < FM; i0 += PI) {
-      const int mw = bm + (wm * FM + i0) * 16 + l / CPR, n = bn + wn * FN * 16 + l % CPR * 8;  // chunk of iteration 0
+      const int mw = bm + (wm * FM + i0) * 16, nw = bn + wn * FN * 16;
+      auto row_of = [&](int it) { return (it * 64 + l) / CPR; };
+      auto chunk_at = [&](int it) { return (it * 64 + l) % CPR; };
       uint4 rv[ITS];
       if constexpr (kResid<EPI>) {
 #pragma unroll
         for (int it = 0; it < ITS; ++it) {
-          const int m = mw + it * (64 / CPR);
+          const int m = mw + row_of(it), n = nw + chunk_at(it) * 8;
           if (m < p.M && n < p.N) rv[it] = *reinterpret_cast<const uint4*>(p.R + (size_t)m * p.ldr + n);
         }
       }
@@ -827,17 +918,17 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
 #pragma unroll
       for (int it = 0; it < ITS; ++it) {
         sqv[it] = 0.f;
-        const int m = mw + it * (64 / CPR);
+        const int m = mw + row_of(it), n = nw + chunk_at(it) * 8;
         if (m >= p.M || n >= p.N) continue;
-        const char* row = wl + (it * (64 / CPR) + l / CPR) * RSF;
+        const char* row = wl + row_of(it) * RSF;
         auto chunk = [&](int ch, float (&f)[8]) {
           const float4 a = *reinterpret_cast<const float4*>(row + ch * 32), b = *reinterpret_cast<const float4*>(row + ch * 32 + 16);
           f[0] = a.x, f[1] = a.y, f[2] = a.z, f[3] = a.w, f[4] = b.x, f[5] = b.y, f[6] = b.z, f[7] = b.w;
         };
         float v[8], u[8];
-        chunk(l % CPR, v);
+        chunk(chunk_at(it), v);
         if constexpr (EPI == EPI_QKV) {
-          chunk(l % CPR ^ 1, u);
+          chunk(chunk_at(it) ^ 1, u);
           float4 rope[4];
           if (p.use_rope) {
             const int pos = p.positions[m];
@@ -858,10 +949,11 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
           *reinterpret_cast<uint4*>(reinterpret_cast<u16*>(p.Y) + (size_t)m * p.ldy + n) = o;
         }
       }
+      static_assert(!kResid<EPI> || 64 % CPR == 0, "a row's lanes side by side");
       if (kResid<EPI> && p.ss_out) {  // one atomic per (row, wave): the CPR lanes of a row reduce first
 #pragma unroll
         for (int it = 0; it < ITS; ++it) {
-          const int m = mw + it * (64 / CPR);
+          const int m = mw + row_of(it);
           float sq = sqv[it];
 #pragma unroll
           for (int o = 1; o < CPR; o <<= 1) sq += __shfl_xor(sq, o, 64);
@@ -1010,18 +1102,28 @@ void launch_kept(const GemmParams& p, hipStream_t st) {
 int g_p8_mode = 2;         // 0: the 128^2 kernel only, 1: the 256^2 one from 256 rows (bf16: of pre-tiled whole column tiles), 2: choose()
 int g_split_fill_pct = 0;  // > 0: vwa_gemm_splits' fill, and the rules by shape alone instead of plan()
 
+// Whether a product may take the two-group tile of n columns: pre-tiled bf16 weights whose sums keep no order (the two groups' are
+// added last).  The wide one has 12 chunks to a row, which the residual's epilogue does not deal out.
+constexpr bool takes_wide(int epi) { return epi != EPI_RESID && epi != EPI_GELU_RESID; }
+bool takes_groups(const GemmParams& p, int epi, int n) {
+  return g_p8_mode == 2 && p.w_tiled && !p.sw && !p.keep_order && p.nbatch <= 1 && p.cus > 0 && p.M > CfgF::BM && (n == CfgK::BN || takes_wide(epi));
+}
+
 // Tile and K slices of a bf16 product of >= 128 rows: the cheapest by an estimate in us, fitted to 180 shapes (130 .. 12000
 // rows, 384 .. 28672 columns, K 384 .. 14336; both tiles, 1 .. 16 slices): 9 % off (rms of the logarithm), and 1.4 % slower than the
 // best choice of each shape, where the rules before (256^2 from 256 tiles or from slices of >= 2048 k that fill the CUs;
 // slices in powers of two until 75 % of the CUs have a tile) were 12 %: 12000 x 1280 x 5120 (235 large tiles) 165 -> 115 us,
 // 768 x 4096 x 14336 155 -> 86, 512 x 28672 x 4096 132 -> 93, 1863 x 6144 x 4096 115 -> 83.
 //   a round of the CUs costs so much per k-group and so much to start and store; a part of a last round 70 % and its share;
-//   128^2 tiles run two to a CU, one alone is faster; the slices' f32 partials are written and read.
+//   128^2 tiles run two to a CU, one alone is faster, two groups on one (CfgK, CfgKw: fitted to 16 shapes against it) faster still
+//   wherever every tile has a CU; beyond that tiles by twos are (1024 x 8192 x 2048, 512 tiles: 41 us, 48 of two groups);
+//   the slices' f32 partials are written and read.
 // W8A8 (k-groups of half the stages): fitted to 690 timings of 60 shapes (80 .. 6000 rows, 1024 .. 28672 columns, K 1280 ..
 // 14336), 11 % off; it picks the tile alone: slices in another order move a few bf16 activations by a bit, and every moved one
 // can flip its fp8 code further on, so they stay those of vwa_gemm_splits.  2720 x 4096 x 14336 224 -> 125 us, 2720 x 28672 x
 // 4096 407 -> 294, 1863 x 6144 x 4096 75 -> 48; small ones keep the 128^2 tile (2720 x 2560 x 1280: 18.4, 24.7 on the large one).
-float estimate(const GemmParams& p, bool p8, int s) {
+// tile: columns of the small tile taken (CfgK: with a minus)
+float estimate(const GemmParams& p, bool p8, int s, int epi, int* tile = nullptr) {
   const int kg = cdiv(p.K / BKG, s), b = p8 ? 256 : 128;
   const int64_t t = (int64_t)cdiv(p.M, b) * cdiv(p.N, b) * s;
   const bool alone = !p8 && t <= p.cus;
@@ -1033,21 +1135,34 @@ float estimate(const GemmParams& p, bool p8, int s) {
     return rounds * (kg * per + (p8 ? 6.8f : 3.3f)) + (s > 1 ? 5.3f + slabs / 3.27e6f : 0.f);
   }
   const float per = p8 ? 2.0f : alone ? 1.27f : r >= 1.f ? 1.84f : 1.27f + 0.57f * (2.f * r - 1.f);
-  return rounds * (kg * per + (p8 ? 5.6f : 2.3f)) + (s > 1 ? 4.f + slabs / 3.55e6f : 0.f);
+  const float sum = s > 1 ? 4.f + slabs / 3.55e6f : 0.f;
+  float us = rounds * (kg * per + (p8 ? 5.6f : 2.3f));
+  if (!p8) {
+    if (tile) *tile = CfgS::BN;
+    for (const int n : {CfgK::BN, CfgKw::BN}) {
+      if (!takes_groups(p, epi, n) || (int64_t)cdiv(p.M, CfgK::BM) * cdiv(p.N, n) * s > p.cus) continue;
+      const float g = n == CfgK::BN ? kg * 0.99f + 3.6f : kg * 1.18f + 5.f;
+      if (g < us) {
+        us = g;
+        if (tile) *tile = n == CfgK::BN ? -CfgK::BN : CfgKw::BN;
+      }
+    }
+  }
+  return us + sum;
 }
 
 struct Plan {
   bool p8;
   int splits;
 };
-Plan plan(const GemmParams& p, float* took = nullptr) {
+Plan plan(const GemmParams& p, int epi, float* took = nullptr) {
   const int KG = p.K / BKG;
   Plan best{false, 1};
   float least = 0.f;
   for (const int s0 : {1, 2, 3, 4, 6, 8, 12, 16}) {
     if (s0 > 1 && (s0 > KG || (int64_t)s0 * p.M * p.N > p.ws_cap)) break;
     for (const bool p8 : {true, false}) {
-      const float us = estimate(p, p8, cdiv(KG, cdiv(KG, s0)));
+      const float us = estimate(p, p8, cdiv(KG, cdiv(KG, s0)), epi);
       if (least == 0.f || us < least) {
         least = us;
         best = {p8, s0};
@@ -1062,18 +1177,18 @@ Plan plan(const GemmParams& p, float* took = nullptr) {
 // launch of its own, with tiles and slices of its own (0: not).  The tiles past the last whole round cost nearly a round of their
 // own, however few: 2048 x 32896 x 4096 is four rounds and eight tiles, 482 -> 438 us in two launches (398 of them the whole rounds').
 // 1024 x 17664 x 2048 86 -> 76 us, 1300 x 22528 x 4096 238 -> 206, 1900 x 26624 x 4096 341 -> 333.
-int whole_rounds(const GemmParams& p) {
+int whole_rounds(const GemmParams& p, int epi) {
   if (p.M < 128 || p.keep_order || p.sw || p.nbatch > 1 || p.cus <= 0 || g_p8_mode != 2 || g_split_fill_pct != 0) return 0;
   const int mb = cdiv(p.M, 256), nb = cdiv(p.N, 256), tiles = mb * nb;
   const int cols = mb <= p.cus ? (int)((int64_t)(tiles / p.cus) * p.cus / mb) : 0;  // column tiles of the whole rounds
   if (cols < 1 || cols * 256 >= p.N) return 0;
   float whole, rest;
-  plan(p, &whole);
+  plan(p, epi, &whole);
   GemmParams a = p, b = p;
   a.N = cols * 256;
   b.N = p.N - a.N;
-  plan(b, &rest);
-  return estimate(a, true, 1) + rest + 3.f < 0.97f * whole ? a.N : 0;
+  plan(b, epi, &rest);
+  return estimate(a, true, 1, epi) + rest + 3.f < 0.97f * whole ? a.N : 0;
 }
 
 // K slices of a bf16 product of <= 64 rows and of fp8 weights (W8A16): the cheapest by an estimate in us, fitted to 270 timings
@@ -1128,7 +1243,7 @@ bool keeps_order(int epi, const GemmParams& p) {
 }
 
 // Tile and slices of a launch (p.splits: those of vwa_gemm_splits; p.ws_cap: the f32 numbers that slices may take)
-Plan choose(const GemmParams& p, bool parts = false) {
+Plan choose(const GemmParams& p, int epi, bool parts = false) {
   Plan r{false, p.splits < 1 ? 1 : p.splits};
   if (p.nbatch > 1 || p.cus <= 0) return r;
   if (p.sw && !p.sx) {
@@ -1140,12 +1255,12 @@ Plan choose(const GemmParams& p, bool parts = false) {
   // (g_p8_mode picks the tile; the slices of W8A8 and kept-order products are part of the order of their sums)
   if (p.keep_order || p.sx) {
     if (p.keep_order && fill) r.splits = s;
-    r.p8 = g_p8_mode == 1 ? p.M >= 256 : g_p8_mode == 2 && (p.sx || p.M >= 128) && estimate(p, true, r.splits) < estimate(p, false, r.splits);
+    r.p8 = g_p8_mode == 1 ? p.M >= 256 : g_p8_mode == 2 && (p.sx || p.M >= 128) && estimate(p, true, r.splits, epi) < estimate(p, false, r.splits, epi);
     return r;
   }
   if (g_p8_mode == 2 && g_split_fill_pct == 0) {
     if (p.M <= CfgF::BM) r.splits = few_slices(p, parts);
-    return p.M >= 128 ? plan(p) : r;
+    return p.M >= 128 ? plan(p, epi) : r;
   }
   if (p.w_tiled && s && (g_p8_mode == 1 || (g_p8_mode == 2 && fill))) r = Plan{true, s};
   return r;
@@ -1159,6 +1274,18 @@ Plan choose(const GemmParams& p, bool parts = false) {
 constexpr bool takes_narrow(int epi) { return epi != EPI_SWIGLU && epi != EPI_GELU_RESID; }
 bool narrow(const GemmParams& p) {  // (bf16 weights that keep no order)
   return g_p8_mode == 2 && p.M <= CfgN::BM && p.nbatch <= 1 && 2 * cdiv(p.N, 128) * p.splits <= p.cus;
+}
+
+// Columns of the tile of 128 rows that a product of > 64 takes (CfgK: with a minus)
+int small_tile(const GemmParams& p, int epi) {
+  int tile = CfgS::BN;
+  if (takes_groups(p, epi, CfgK::BN)) estimate(p, false, p.splits, epi, &tile);
+  return tile;
+}
+
+template <class C, int EPI>
+void launch_groups(const GemmParams& p, hipStream_t st) {
+  hipLaunchKernelGGL((gemm_kernel<C, EPI, true>), dim3(cdiv(p.M, C::BM) * cdiv(p.N, C::BN) * p.splits), dim3(C::THREADS), C::LDS, st, p);
 }
 
 // sum false: the slices' partial rows stay in the workspace
@@ -1202,7 +1329,14 @@ int launch_epi(const GemmParams& p, hipStream_t st, bool p8, bool sum = true) {
   } else if (p.M <= CfgF::BM) {
     launch_cfg<CfgF, EPI>(p, st);
   } else {
-    launch_cfg<CfgS, EPI>(p, st);
+    const int tile = small_tile(p, EPI);
+    if (tile == -CfgK::BN) {
+      launch_groups<CfgK, EPI>(p, st);
+    } else if (tile == CfgKw::BN) {
+      if constexpr (takes_wide(EPI)) launch_groups<CfgKw, EPI>(p, st);
+    } else {
+      launch_cfg<CfgS, EPI>(p, st);
+    }
   }
   if (sum && p.splits > 1) {
     const int64_t n = (int64_t)p.M * (EPI == EPI_SWIGLU ? p.N / 2 : p.N) / 8;
@@ -1247,10 +1381,10 @@ extern "C" void vwa_gemm_set_p8(int mode) { g_p8_mode = mode; }
 extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int parts, int* columns, int* splits) {
   GemmParams p = *pp;
   p.keep_order = keeps_order(epi, p);
-  const Plan pl = choose(p, parts);
+  const Plan pl = choose(p, epi, parts);
   const int per = cdiv(p.K / BKG, pl.splits);
   p.splits = *splits = cdiv(p.K / BKG, per);
-  *columns = pl.p8 ? CfgP8::BN : !p.keep_order && !p.sw && takes_narrow(epi) && narrow(p) ? CfgN::BN : CfgS::BN;
+  *columns = pl.p8 ? CfgP8::BN : !p.keep_order && !p.sw && takes_narrow(epi) && narrow(p) ? CfgN::BN : small_tile(p, epi) == CfgKw::BN ? CfgKw::BN : CfgS::BN;
 }
 
 namespace {
@@ -1270,7 +1404,7 @@ int checks_and_plan(int epi, GemmParams& p, bool* p8, bool parts = false) {
                            (reinterpret_cast<uintptr_t>(p.Y2) & 15)))
     return -19;
   p.keep_order = keeps_order(epi, p);
-  const Plan pl = choose(p, parts);
+  const Plan pl = choose(p, epi, parts);
   *p8 = pl.p8;
   p.splits = pl.splits;
   const int KG = p.K / BKG;
@@ -1340,7 +1474,7 @@ extern "C" void vwa_gemm_part(int epi, const GemmParams* pp, int n, int second, 
 extern "C" int vwa_gemm_cut(int epi, const GemmParams* pp) {
   GemmParams p = *pp;
   p.keep_order = keeps_order(epi, p);
-  return epi == EPI_STORE || epi == EPI_RESID || epi == EPI_SWIGLU || epi == EPI_GELU || epi == EPI_SPLIT ? whole_rounds(p) : 0;
+  return epi == EPI_STORE || epi == EPI_RESID || epi == EPI_SWIGLU || epi == EPI_GELU || epi == EPI_SPLIT ? whole_rounds(p, epi) : 0;
 }
 
 extern "C" int vwa_gemm_grouped(int epi, const GemmParams* pp, hipStream_t st) {

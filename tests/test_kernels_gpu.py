@@ -748,6 +748,31 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
+@pytest.mark.parametrize("M,N,K,columns", [(85, 28672, 4096, 128), (1011, 4096, 640, 128), (1010, 1040, 2048, 128), (700, 2048, 4096, 128),
+                                           (130, 24496, 2048, 192), (1011, 6144, 4096, 192), (513, 4096, 4096, 192), (300, 12208, 4224, 192)])
+def test_gemm_of_two_wave_groups(M, N, K, columns):
+    """Two groups of waves that take the stages of K in turn, over the epilogues: odd numbers of k-groups, slices, rows
+    and columns past the last whole tile.  f32 results: K additions, each rounded by 2^-24 of a partial sum, signs at random, and in
+    bf16 half a unit in the last place, of the result and (residuals) of nothing else."""
+    E = ops.ext()
+    assert E.gemm_tile(0, M, N, K)[0] == columns
+    x, w = torch.randn(M, K, device=DEV).to(BF), (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
+    wt, b, res = ops.TiledWeight(w), rnd(N), rnd(M, N)
+    exp = x.double() @ w.double().T
+    out = torch.empty(M, N, device=DEV)
+    for _ in range(3):
+        ops.gemm(x, wt, out.fill_(7.0))
+        assert float((out.double() - exp).norm() / exp.norm()) < 2.0 ** -24 * K ** 0.5
+    near = lambda got, y: float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
+    y = exp + b.double()
+    assert near(ops.linear(x, wt, b), y)
+    assert near(ops.linear(x, wt, b, act="gelu"), y / 2 * torch.erfc(-y / 2 ** 0.5))
+    assert near(ops.linear(x, wt, b, residual=res), y + res.double())
+    g, u = exp.view(M, N // 32, 2, 16).unbind(2) if N % 32 == 0 else (None, None)
+    if g is not None:
+        assert near(ops.linear_swiglu(x, wt), (g * torch.sigmoid(g) * u).reshape(M, N // 2))
+
+
 @pytest.mark.parametrize("tiled", [True, False])
 @pytest.mark.parametrize("M,N,K,n_split", [(2048, 8256, 1024, 8192), (2000, 8208, 1408, 4096), (1900, 8448, 1408, 8400)])
 def test_gemm_of_two_launches(M, N, K, n_split, tiled):
@@ -1169,6 +1194,31 @@ def test_gemm_qkv_epilogue_fused(M, kind, monkeypatch):
                            rope=rope.cpu(), positions=pos.cpu(), slots=slots.cpu(), q_out=q, k_cache=kc, v_cache=vc)
         for a, b in zip(fused, (q, kc, vc)):
             close(a, b, 3e-2, 3e-2)
+
+
+@pytest.mark.parametrize("hd,nq,nkv", [(128, 32, 8), (64, 64, 16)])
+def test_qkv_epilogue_of_two_wave_groups(hd, nq, nkv, monkeypatch):
+    """Heads rotated and written in the epilogue of the 192-column tile, heads across its edges, against product and rotation apart:
+    values of a normed row are of order one, 6 at most, rounded once (2^-9 of them) here and twice there, the first time both of a
+    rotated pair: 2^-9 6 (2 + sqrt 2) = 4e-2."""
+    M, K, n = 1011, 4096, (nq + 2 * nkv) * hd
+    assert ops.ext().gemm_tile(5, M, n, K)[0] == 192
+    w = ops.TiledWeight(ops.permute_qkv_rows(rnd(n, K, scale=K ** -0.5), nq + 2 * nkv, hd))
+    x, rope = rnd(M, K), ops.rope_table(2048, hd, 5e5, device=DEV)
+    pos = torch.arange(100, 100 + M, dtype=torch.int32, device=DEV)
+    slots = torch.randperm(64 * 16, device=DEV)[:M].to(torch.int64)
+    slots[M // 2] = -1
+    got = []
+    for fused in (True, False):
+        monkeypatch.setattr(ops, "GEMM_QKV_FUSED", fused)
+        kc, vc = (torch.full((64, nkv, 16, hd), 7.0, dtype=BF, device=DEV) for _ in range(2))
+        q = torch.zeros(M, nq * hd, dtype=BF, device=DEV)
+        ops.qkv_rope_write(x, w, None, fuse_rms=True, eps=1e-5, n_q_heads=nq, n_kv_heads=nkv, head_dim=hd, rope=rope,
+                           positions=pos, slots=slots, q_out=q, k_cache=kc, v_cache=vc)
+        got.append((q, kc, vc))
+    for a, b in zip(*got):
+        assert float((a.float() - b.float()).abs().max()) < 4e-2
+    assert int((got[0][2] == 7.0).all(-1).sum()) == (64 * 16 - M + 1) * nkv  # (slots of no row)
 
 
 @pytest.mark.parametrize("hd,nq,nkv", [(128, 32, 8), (128, 8, 1), (64, 8, 4)])
