@@ -81,9 +81,10 @@ class WhisperRunner:
         self.b = b
         cuda = dev.type == "cuda"
 
-        def rows():
-            h = torch.zeros(6 * R, dtype=torch.int32, pin_memory=cuda)
-            return SimpleNamespace(h_in=h, np_i32=h[: 4 * R].view(4, R).numpy(), np_slots=h[4 * R :].view(torch.int64).numpy())
+        def rows(n):
+            h = torch.zeros(n, 6 * R, dtype=torch.int32, pin_memory=cuda)
+            return [SimpleNamespace(h_in=t, np_i32=r[: 4 * R].reshape(4, R), np_slots=r[4 * R :].view(np.int64))
+                    for t, r in zip(h.unbind(), h.numpy())]
 
         self.staging = StagingRing(rows, cuda)
         if use_graphs is None:

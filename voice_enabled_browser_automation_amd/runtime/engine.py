@@ -138,7 +138,7 @@ class StepBuffers:
         # the block table as the host has it (np_table; sequences come, grow and go at any time)
         self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
         self.table_dirty = True
-        self.staging = StagingRing(lambda: StepStaging(R, T, C, cuda), cuda)
+        self.staging = StagingRing(lambda n: StepStaging.sets(n, R, T, C, cuda), cuda)
 
     def upload(self, st: "StepStaging", n_rows: int) -> None:
         """H2D copy of a step's metadata (with the rows' block tables where the chained launch reads them) and of the block
@@ -161,21 +161,27 @@ class StepStaging:
     and numpy views of them -- the per-step row metadata is written with a handful of slice assignments instead of ~5 torch
     element writes per row."""
 
-    def __init__(self, R: int, T: int, C: int, pin: bool):
-        self.h_meta_all = torch.zeros(T + R * C, dtype=torch.int32, pin_memory=pin)
-        meta = self.h_meta_all[: 7 * R + 2]
-        self.np_i32 = meta[: 4 * R].view(4, R).numpy()
-        self.np_slots = meta[4 * R : 6 * R].view(torch.int64).numpy()
-        self.np_sel = meta[6 * R : 7 * R].numpy()
-        self.np_shared = meta[7 * R : 7 * R + 2].numpy()
-        self.np_row_table = self.h_meta_all[T:].view(R, C).numpy()
+    @classmethod
+    def sets(cls, n: int, R: int, T: int, C: int, pin: bool) -> List["StepStaging"]:
+        meta = torch.zeros(n, -(-(T + R * C) // 4) * 4, dtype=torch.int32, pin_memory=pin)
+        head = torch.zeros(n, R, dtype=torch.int64, pin_memory=pin)
+        rows = meta.numpy()
+        rows[:, 3 * R : 4 * R] = 1  # inert rows, as the device's before the first step
+        rows[:, 4 * R : 6 * R] = -1
+        return [cls(m, r, h, R, T, C) for m, r, h in zip(meta.unbind(), rows, head.unbind())]
+
+    def __init__(self, meta_all: torch.Tensor, rows: np.ndarray, head_idx: torch.Tensor, R: int, T: int, C: int):
+        self.h_meta_all = meta_all
+        self.np_i32 = rows[: 4 * R].reshape(4, R)
+        self.np_slots = rows[4 * R : 6 * R].view(np.int64)
+        self.np_sel = rows[6 * R : 7 * R]
+        self.np_shared = rows[7 * R : 7 * R + 2]
+        self.np_row_table = rows[T : T + R * C].reshape(R, C)
         # rows whose hidden state feeds the LM head when the step computed every row (L == M):
         # gathered on the device through a pinned staging copy (a torch.tensor(list, device=...)
         # here was a pageable, host-blocking copy that waited for the whole step -- measured: 9 of
         # 172 iterations at 32 sessions stalled ~4.6 ms each)
-        self.h_head_idx = torch.zeros(R, dtype=torch.int64, pin_memory=pin)
-        self.np_i32[3].fill(1)  # inert rows, as the device's before the first step
-        self.np_slots.fill(-1)
+        self.h_head_idx = head_idx
 
 
 class LLMEngine:

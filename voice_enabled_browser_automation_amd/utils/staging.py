@@ -9,12 +9,12 @@ T = TypeVar("T")
 
 
 class StagingRing(Generic[T]):
-    """``n`` sets of rows (made by ``make``) in turn, one a step: a queued step's copies read its own set, and a set is written again
+    """``n`` sets of rows (``make(n)``: together, since an allocation of pinned memory costs a few us) in turn, one a step: a queued step's copies read its own set, and a set is written again
     only when the step that had it is through, which an event behind every half of the ring tells.  (An event a step costs the
     stream a few us.)  One stream at a time, as the device buffers that the rows go to.  Without a GPU one set is enough."""
 
-    def __init__(self, make: Callable[[], T], cuda: bool, n: int = 16):
-        self.sets: List[T] = [make() for _ in range(n if cuda else 1)]
+    def __init__(self, make: Callable[[int], List[T]], cuda: bool, n: int = 16):
+        self.sets: List[T] = make(n if cuda else 1)
         self._done = [torch.cuda.Event(), torch.cuda.Event()] if cuda else []  # behind the last use of either half
         self._at, self._used = -1, False
 
