@@ -291,6 +291,9 @@ using CfgP8 = Cfg<256, 256, 2, 4>;
 //   the 41 below.  A CU draws 57 bytes a ns then, 64 on the 256^2 tile and 70 at most: the wide tile needs a sixth less of it.)
 // us, alone or two to a CU -> two groups: 1011 x 4096 x 4096 48.1 -> 40.9, 2048 x 2048 x 2048 28.2 -> 23.8, 700 x 1280 x 1280 (in
 // slices before) 20.6 -> 15.2; 192 columns: 1011 x 6144 x 4096 62.8 -> 54.0, 130 x 12288 x 2048 29.4 -> 24.0.
+// Residuals and heads are stored by both groups, in turn, with a row's position and slot requested in front of the LDS round trip and
+// its rotation behind the sums: a product into rotated heads and cache, 1011 x 6144 x 4096, 69.5 -> 63.7 us, 600 rows 50.2 -> 47.0.
+// (Plain results: no difference.)
 // half-tile `which` (0 A-lo, 1 A-hi, 2 B-lo, 3 B-hi) into the stage image `st`: 16 wave-instructions of 1 KB, 2 per
 // wave, from the byte offsets voff (past the resource: zeros) + soff
 VWA_DEVICE void p8_issue(__amdgpu_buffer_rsrc_t r, const unsigned (&voff)[8], unsigned soff, int which, char* st) {
@@ -628,6 +631,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   const int KG = p.K / BKG;
   const int kg0 = split * p.kg_per_split, kg1 = min(KG, kg0 + p.kg_per_split);
   const int w = C::GROUPS > 1 ? (threadIdx.x >> 6) % C::NW : threadIdx.x >> 6, wm = w / C::WN, wn = w % C::WN;
+  const int grp = C::GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * C::NW)) : 0;
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -712,7 +716,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");  // (the epilogue reuses the LDS)
   } else if constexpr (C::GROUPS == 2) {
     static_assert(C::NST == 2 && !F8 && !W8 && !GRP && LINES, "two K groups: bf16 products that keep no order");
-    const int l = lane_id(), rl = l & 15, g = l >> 4, grp = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * C::NW)), n = nh / 2;
+    const int l = lane_id(), rl = l & 15, g = l >> 4, n = nh / 2;
     constexpr int PA = C::BM / 8 / C::NW, PB = C::BN / 8 / C::NW;
     char* const mine = lds + grp * 2 * C::STAGE;
     unsigned xoff[PA], woff[PB];  // this lane's pieces of a stage (k-group 0)
@@ -785,7 +789,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
         for (int j = 0; j < FN; ++j) acc[i][j] += ex[(i * FN + j) * 64];
     }
     __syncthreads();  // (the epilogue writes LDS again)
-    if (grp == 1) return;
+    if (grp == 1 && (!(kResid<EPI> || EPI == EPI_QKV) || p.splits > 1 || p.y_f32)) return;  // (these store by both groups)
   } else {
   if (nh > 0) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0, lds, rows);
   if (nh > 1) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
@@ -887,14 +891,14 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   if constexpr (!F8 && (kResid<EPI> || EPI == EPI_QKV)) {
     constexpr int CPR = FN * 2, RSF = FN * 64 + 16;  // 8-column chunks of a row; LDS row stride (bytes: 4 rows apart, 16 banks)
     constexpr int LDSB = (W8 ? C::W8LDS : C::LDS) / C::NW / (16 * RSF);
-    constexpr int PI = LDSB >= FM ? FM : LDSB >= FM / 2 ? FM / 2 : FM / 4, ITS = PI * 16 * CPR / 64;
-    static_assert(PI >= 1 && PI <= LDSB && FM % PI == 0, "a pass fits the wave's share of the LDS");
+    constexpr int PI = LDSB >= FM ? FM : LDSB >= FM / 2 ? FM / 2 : FM / 4, ITS = PI * 16 * CPR / 64 / C::GROUPS;
+    static_assert(PI >= 1 && PI <= LDSB && FM % PI == 0 && (C::GROUPS == 1 || PI == FM), "a pass fits the wave's share of the LDS");
     char* wl = lds + w * (PI * 16 * RSF);
 #pragma unroll
     for (int i0 = 0; i0 < FM; i0 += PI) {
       const int mw = bm + (wm * FM + i0) * 16, nw = bn + wn * FN * 16;
-      auto row_of = [&](int it) { return (it * 64 + l) / CPR; };
-      auto chunk_at = [&](int it) { return (it * 64 + l) % CPR; };
+      auto row_of = [&](int it) { return ((it * C::GROUPS + grp) * 64 + l) / CPR; };  // (two groups: in turn)
+      auto chunk_at = [&](int it) { return ((it * C::GROUPS + grp) * 64 + l) % CPR; };
       uint4 rv[ITS];
       if constexpr (kResid<EPI>) {
 #pragma unroll
@@ -903,6 +907,17 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
           if (m < p.M && n < p.N) rv[it] = *reinterpret_cast<const uint4*>(p.R + (size_t)m * p.ldr + n);
         }
       }
+      int posv[ITS];
+      int64_t slotv[ITS];
+      if constexpr (EPI == EPI_QKV) {
+#pragma unroll
+        for (int it = 0; it < ITS; ++it) {
+          const int m = min(mw + row_of(it), p.M - 1);
+          posv[it] = p.use_rope ? p.positions[m] : 0;
+          slotv[it] = p.slots[m];
+        }
+      }
+      if (grp == 0)
 #pragma unroll
       for (int i = 0; i < PI; ++i)
 #pragma unroll
@@ -913,7 +928,18 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
             if constexpr (kGelu<EPI>) v = gelu_erf(v);
             *reinterpret_cast<float*>(wl + (i * 16 + 4 * (l >> 4) + r) * RSF + (j * 16 + (l & 15)) * 4) = v;
           }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      constexpr bool AHEAD = EPI == EPI_QKV && ITS <= 6;  // (the sums' registers are free now)
+      float4 turn[AHEAD ? ITS : 1][4];
+      if constexpr (AHEAD) {
+        if (p.use_rope) {
+#pragma unroll
+          for (int it = 0; it < ITS; ++it)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) turn[it][e] = rope_at(p, posv[it], min(nw + chunk_at(it) * 8, p.N - 8))[e];
+        }
+      }
+      if constexpr (C::GROUPS > 1) __syncthreads();
+      else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       float sqv[ITS];  // (ss_out: squares of each stored chunk)
 #pragma unroll
       for (int it = 0; it < ITS; ++it) {
@@ -929,13 +955,16 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
         chunk(chunk_at(it), v);
         if constexpr (EPI == EPI_QKV) {
           chunk(chunk_at(it) ^ 1, u);
-          float4 rope[4];
-          if (p.use_rope) {
-            const int pos = p.positions[m];
+          if constexpr (AHEAD) {
+            qkv_store(p, m, n, v, u, turn[it], slotv[it]);
+          } else {
+            float4 rope[4];
+            if (p.use_rope) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) rope[e] = rope_at(p, pos, n)[e];
+              for (int e = 0; e < 4; ++e) rope[e] = rope_at(p, posv[it], n)[e];
+            }
+            qkv_store(p, m, n, v, u, rope, slotv[it]);
           }
-          qkv_store(p, m, n, v, u, rope, p.slots[m]);
         } else {
           unpack8(rv[it], u);
 #pragma unroll
