@@ -211,16 +211,18 @@ VWA_DEVICE uint32_t cvt_pk_fp8(float a, float b) {
 
 VWA_DEVICE float silu(float x) { return x / (1.f + __expf(-x)); }
 
-// x Phi(x) = max(x, 0) - t Q(t), t = |x|, Q(t) = exp(-t^2 / 2) P(t) the normal tail.  P = exp(t^2 / 2) Q falls from 1/2 as 1 / t:
-// a polynomial in m = t / (t + 4.5), P(0) = 1/2 exactly, fitted here (least maximal relative error, 7e-9 up to t = 5; less is asked
-// of tails that vanish beside any result).  No branch and 16 vector instructions of which 2 are transcendental, where erff has two
-// branches of some 20 each, gone through element by element: an epilogue's waves do nothing else meanwhile.  us of a product with it,
-// 0.5 x (1 + erff(x / sqrt 2)) -> here (without: in brackets): 12000 x 5120 x 1280 197 -> 164 (145), 1500 x 5120 x 1280 32.5 -> 27.6
-// (25.1), 1500 x 2048 x 512 17.3 -> 12.3 (9.9), 8 x 5120 x 1280 9.0 -> 8.4 (7.8).
-// Error against 64 bits, |x| < 14: at most 4.5e-7 -> 2.4e-7, mean 1.5e-8 -> 1.1e-8; and relative, in [-4, -2), where 1 + erf
-// cancels, 4.7e-4 -> 1.5e-6.  NaN and -infinity give NaN, infinity itself, either way.
+// x Phi(x).  From |x| = t = 1 on max(x, 0) - t Q(t), Q(t) = exp(-t^2 / 2) P(t) the normal tail: P = exp(t^2 / 2) Q falls from 1/2 as
+// 1 / t, a polynomial in m = t / (t + 4.5) fitted here (least maximal relative error, 7e-9 up to t = 5; less is asked of tails that
+// vanish beside any result).  Below x / 2 + x^2 R(x^2), where nothing cancels (fitted likewise, 1e-11).  Both are computed, without a
+// branch: some 25 vector instructions of which 2 are transcendental, where erff has two branches of some 20 each, gone through element
+// by element while an epilogue's waves do nothing else.  us of a product with it, 0.5 x (1 + erff(x / sqrt 2)) -> here (without: in
+// brackets): 12000 x 5120 x 1280 201 -> 180 (147), 1500 x 5120 x 1280 33.2 -> 29.4 (25.6), 8 x 5120 x 1280 8.7 -> 8.2 (8.1).
+// Error against 64 bits, at most (mean), erff -> here: [-4, -2) 6.0e-8 (2.3e-8) -> 2.5e-8 (2.3e-9), [-1, 0) 4.1e-8
+// (6.2e-9) -> 3.9e-8 (5.2e-9), [0, 1) 9.1e-8 (1.2e-8) -> 6.1e-8 (8.8e-9), [2, 6) 4.5e-7 (9.9e-8) -> 2.4e-7 (8.1e-8); nor is any other
+// part of [-14, 14) less exact.  The tail alone, at all |x|, would be: 166 us, but 4.8e-8 in [-1, -1/2).
+// NaN and -infinity give NaN, infinity itself, either way.
 VWA_DEVICE float gelu_erf(float x) {
-  const float t = fminf(fabsf(x), 14.5f), m = t * __builtin_amdgcn_rcpf(t + 4.5f);
+  const float t = fminf(fabsf(x), 14.5f), s = t * t, h = 0.5f * x, m = t * __builtin_amdgcn_rcpf(t + 4.5f);
   float p = -0.10658054f;
   p = fmaf(p, m, 0.38831303f);
   p = fmaf(p, m, -0.33956796f);
@@ -230,8 +232,15 @@ VWA_DEVICE float gelu_erf(float x) {
   p = fmaf(p, m, 3.26723218f);
   p = fmaf(p, m, -1.79523969f);
   p = fmaf(p, m, 0.5f);
-  const float e = __builtin_amdgcn_exp2f(t * t * -0.72134752f);
-  return fmaf(-(t * e), p, fmaf(0.5f, x, 0.5f * fabsf(x)));
+  const float e = __builtin_amdgcn_exp2f(s * -0.72134752f), tail = fmaf(-(t * e), p, h + fabsf(h));
+  float r = 5.36846771e-7f;
+  r = fmaf(r, s, -9.27314159e-6f);
+  r = fmaf(r, s, 1.15319323e-4f);
+  r = fmaf(r, s, -1.18728797e-3f);
+  r = fmaf(r, s, 9.97355022e-3f);
+  r = fmaf(r, s, -6.64903820e-2f);
+  r = fmaf(r, s, 0.398942292f);
+  return t < 1.f ? fmaf(s, r, h) : tail;
 }
 
 // Bijective XCD-aware remap of a 1-D block index (8 XCDs, each with a private L2):

@@ -5,13 +5,14 @@ feed-forward, all reading one LayerNorm of an f32 residual stream.
 
 Engine contract as models/llama.py (ragged rows with their own position, slot and block-table row;
 optional logit-row selection), plus a recurrent state row per sequence (``stateful``) next to the
-paged K / V (``cache_layers``).  MI355X layout of a layer -- six launches at decode:
+paged K / V (``cache_layers``).  MI355X layout of a layer -- five launches at decode:
 
     layernorm_f32 -> ONE input projection [q | k | v | gate | z | x | g || up] whose epilogue squares the
-    feed-forward part straight into the output projection's input -> rotation + cache write and the
-    minGRU (right_scale in its epilogue, into that same input) -> attention (two launches: scores, then
-    mixing and values; gate and left_scale in the epilogue, into that same input) -> ONE output projection over [heads | recurrence | feed-forward] with the f32 residual
-    in its epilogue
+    feed-forward part straight into the output projection's input -> rotation + cache write, the minGRU
+    (right_scale in its epilogue, into that same input) and the attention's scores in one launch (prompts:
+    two) -> mixing and values (gate and left_scale in the epilogue, into that same input) -> ONE output
+    projection over [heads | recurrence | feed-forward], whose K slices the next layer's norm adds to the
+    f32 residual (many rows: in its epilogue)
 
 Sizes are arbitrary: projection sections are padded to the MFMA tiles with zero weight rows / columns
 (head sizes: q / k to 32, v to 16), so every kernel runs whole tiles and the padding contributes zeros.
