@@ -1132,10 +1132,11 @@ int g_p8_mode = 2;         // 0: the 128^2 kernel only, 1: the 256^2 one from 25
 int g_split_fill_pct = 0;  // > 0: vwa_gemm_splits' fill, and the rules by shape alone instead of plan()
 
 // Whether a product may take the two-group tile of n columns: pre-tiled bf16 weights whose sums keep no order (the two groups' are
-// added last).  The wide one has 12 chunks to a row, which the residual's epilogue does not deal out.
+// added last).  65 .. 127 rows, whose slices are by shape alone, keep the other tile and their bits: of 10 weights at 85 rows one
+// gained (28672 x 4096 62.9 -> 58.7 us) and one lost (6144 x 4096 24.3 -> 24.8).  The wide one has 12 chunks to a row, which the residual's epilogue does not deal out.
 constexpr bool takes_wide(int epi) { return epi != EPI_RESID && epi != EPI_GELU_RESID; }
 bool takes_groups(const GemmParams& p, int epi, int n) {
-  return g_p8_mode == 2 && p.w_tiled && !p.sw && !p.keep_order && p.nbatch <= 1 && p.cus > 0 && p.M > CfgF::BM && (n == CfgK::BN || takes_wide(epi));
+  return g_p8_mode == 2 && p.w_tiled && !p.sw && !p.keep_order && p.nbatch <= 1 && p.cus > 0 && p.M >= 128 && (n == CfgK::BN || takes_wide(epi));
 }
 
 // Tile and K slices of a bf16 product of >= 128 rows: the cheapest by an estimate in us, fitted to 180 shapes (130 .. 12000
@@ -1305,7 +1306,7 @@ bool narrow(const GemmParams& p) {  // (bf16 weights that keep no order)
   return g_p8_mode == 2 && p.M <= CfgN::BM && p.nbatch <= 1 && 2 * cdiv(p.N, 128) * p.splits <= p.cus;
 }
 
-// Columns of the tile of 128 rows that a product of > 64 takes (CfgK: with a minus)
+// Columns of the tile of 128 rows that a product of more than 64 takes (CfgK: with a minus)
 int small_tile(const GemmParams& p, int epi) {
   int tile = CfgS::BN;
   if (takes_groups(p, epi, CfgK::BN)) estimate(p, false, p.splits, epi, &tile);
