@@ -1203,11 +1203,18 @@ Plan plan(const GemmParams& p, int epi, float* took = nullptr) {
   return best;
 }
 
+// Whether the kernels' 32-bit offsets reach all of a product's weight and rows (loads past a resource's end are zeros)
+bool reachable(const GemmParams& p) {
+  constexpr int64_t kMost = 0x7FFFFFF0ll;
+  return (int64_t)p.N * p.K * (p.sw ? 1 : 2) < kMost && ((int64_t)(p.M - 1) * p.ldx + p.K) * (p.sx ? 1 : 2) < kMost;
+}
+
 // Columns of a product that fill whole rounds of the CUs with large tiles, where it is cheaper by the estimate to give the rest a
 // launch of its own, with tiles and slices of its own (0: not).  The tiles past the last whole round cost nearly a round of their
 // own, however few: 2048 x 32896 x 4096 is four rounds and eight tiles, 482 -> 438 us in two launches (398 of them the whole rounds').
 // 1024 x 17664 x 2048 86 -> 76 us, 1300 x 22528 x 4096 238 -> 206, 1900 x 26624 x 4096 341 -> 333.
 int whole_rounds(const GemmParams& p, int epi) {
+  if (!reachable(p)) return 0;  // (one launch, which refuses it whole)
   if (p.M < 128 || p.keep_order || p.sw || p.nbatch > 1 || p.cus <= 0 || g_p8_mode != 2 || g_split_fill_pct != 0) return 0;
   const int mb = cdiv(p.M, 256), nb = cdiv(p.N, 256), tiles = mb * nb;
   const int cols = mb <= p.cus ? (int)((int64_t)(tiles / p.cus) * p.cus / mb) : 0;  // column tiles of the whole rounds
@@ -1422,8 +1429,7 @@ int checks_and_plan(int epi, GemmParams& p, bool* p8, bool parts = false) {
   if (p.M < 1 || p.N < 16 || p.N % 16 || p.K < BKG || p.K % BKG) return -10;
   if (p.ldx % (p.sx ? 16 : 8) || (reinterpret_cast<uintptr_t>(p.X) & 15) || (reinterpret_cast<uintptr_t>(p.W) & 15))
     return -11;
-  constexpr int64_t kMost = 0x7FFFFFF0ll;  // (32-bit offsets, and loads past a resource's end are zeros)
-  if ((int64_t)p.N * p.K * (p.sw ? 1 : 2) >= kMost || ((int64_t)(p.M - 1) * p.ldx + p.K) * (p.sx ? 1 : 2) >= kMost) return -21;
+  if (!reachable(p)) return -21;
   if ((p.sw && !p.w_tiled) || (p.sx && !p.sw)) return -14;  // fp8: the tiled layout; X codes need fp8 weights
   if (epi == EPI_SWIGLU && (p.N % 32 || p.y_f32)) return -12;
   if (epi == EPI_QKV && (p.y_f32 || p.head_dim % 16 || p.N != (p.n_q_heads + 2 * p.n_kv_heads) * p.head_dim ||

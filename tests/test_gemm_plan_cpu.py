@@ -97,3 +97,12 @@ def test_columns_of_two_launches_are_whole_rounds(E):
     assert seen > 5 and E.gemm_cut(0, 64, 32896, 4096) == 0 and E.gemm_cut(6, 2048, 32896, 4096) == 32768
     E.gemm_set_p8(0)
     assert E.gemm_cut(0, 2048, 32896, 4096) == 0
+
+
+def test_a_product_past_the_offsets_has_one_launch(E):
+    """A weight that 32-bit offsets do not reach is refused as a whole, wherever its columns would have been cut: the columns of the
+    whole rounds alone (32768 x 32640, bf16) are within reach."""
+    reach = 0x7FFFFFF0
+    assert 32768 * 32640 * 2 < 32896 * 32640 * 2 < reach <= 32912 * 32640 * 2
+    assert E.gemm_cut(0, 2048, 32896, 32640) == 32768
+    assert E.gemm_cut(0, 2048, 32912, 32640) == 0
