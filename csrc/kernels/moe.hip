@@ -23,6 +23,9 @@ constexpr int kRouteWaves = 8, kRouteThreads = kRouteWaves * 64, kMaxExperts = 2
 // counted, top 4: bf16, K 2048, 16 rows of 16 experts 8.1 -> 6.5; K 1024, 48 rows 9.2 -> 7.5; 24 experts 10.5 -> 9.2; f32, K 1024,
 // 4 rows 7.5 -> 6.0.  Of more experts than lanes a lane would count several, and a maximum after another stays.
 constexpr int kRankExperts = 32;
+// A score as it is ranked: one that is not a number is ahead of every other (they are <= 1) and its weight shows it, as torch.topk has it
+constexpr float kNoNumber = 2.f;
+VWA_DEVICE float rank_of(float score) { return score == score ? score : kNoNumber; }
 
 // pairs -> tiles of one expert each (the whole workgroup); id_of(pair): its expert
 // (One wave that counts expert after expert from ballots, without LDS and barriers: 0.25 us an expert.)
@@ -118,18 +121,17 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
   const int r = tid >> 5, q = tid & 31, row = r0 + r;  // 32 lanes per row: the choices stay inside a wave
   if (p.E <= kRankExperts) {
     // an expert's place is the number of experts ahead of it (a larger score; of equal ones the lower number): all choices at once
-    // where one maximum after another is a chain of lane exchanges.  (Not a number: behind every other.)
-    auto known = [](float v) { return v == v ? v : -2.5f; };
+    // where one maximum after another is a chain of lane exchanges.
     const float* s = sc + r * (Ep + 1);
-    const float v = known(s[min(q, p.E - 1)]);
+    const float mine = s[min(q, p.E - 1)], v = rank_of(mine);
     int place = q < p.E ? 0 : p.E;
 #pragma unroll 4
     for (int o = 0; o < p.E; ++o) {
-      const float u = known(s[o]);
+      const float u = rank_of(s[o]);
       place += u > v || (u == v && o < q) ? 1 : 0;
     }
     if (place < p.top && r < nr) {
-      p.wts[row * p.top + place] = live ? v : 0.f;
+      p.wts[row * p.top + place] = live ? mine : 0.f;
       lds_ids[r * p.top + place] = live ? q : -1;
       __hip_atomic_store(p.ids + row * p.top + place, live ? q : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -138,7 +140,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     float best = -3.f;
     int at = 0;
     for (int e = q; e < p.E; e += 32) {
-      const float v = sc[r * (Ep + 1) + e];
+      const float v = rank_of(sc[r * (Ep + 1) + e]);
       if (v > best) {
         best = v;
         at = e;
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     }
     if (q == 0 && r < nr) {
       sc[r * (Ep + 1) + at] = -1.f;                  // (taken; scores are positive)
-      p.wts[row * p.top + k] = live ? best : 0.f;
+      p.wts[row * p.top + k] = live ? (best == kNoNumber ? __builtin_nanf("") : best) : 0.f;
       lds_ids[r * p.top + k] = live ? at : -1;
       __hip_atomic_store(p.ids + row * p.top + k, live ? at : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }

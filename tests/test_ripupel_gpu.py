@@ -478,6 +478,31 @@ def test_route_of_equal_scores(dtype, rows, E, top):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("E,top", [(5, 2), (32, 4), (33, 4)])
+def test_route_of_scores_that_are_no_number(dtype, E, top):
+    """Both ways to choose: a score that is not a number is taken first, its weight shows it, and the row's other choices are its best
+    numbers; a row without numbers takes the first experts.  (As the CPU path's torch.topk.)"""
+    K, tile, rows, bad = 128, 16, 6, E - 2
+    g = torch.Generator().manual_seed(3)
+    h, router = torch.randn(rows, K, generator=g).to(dtype), torch.zeros(up(E, 16), K, dtype=dtype)
+    router[:E] = (torch.randn(E, K, generator=g) / 8).to(dtype)
+    router[bad, 7] = float("nan")                    # one expert's score in every row ...
+    h[2, 5] = float("nan")                           # ... and every score of a row
+    s = O.sigmoid(h.double() @ router[:E].double().T)
+    assert s.isnan().sum() == rows - 1 + E
+    want = torch.where(s.isnan(), 2.0, s).sort(dim=1, descending=True, stable=True)[1][:, :top]
+    assert (want[:, 0] == torch.where(torch.arange(rows) == 2, 0, bad)).all()
+    bufs = ops.moe_buffers(rows, [(E, top, 128)], dtype, DEV)
+    n = mixers.moe_tiles(rows * top, E, tile)
+    ops.ext().moe_route(h.to(DEV), ops.fragments(router.to(DEV)), E, top, torch.zeros(rows, dtype=torch.int64, device=DEV), bufs.wts,
+                        bufs.ids, tile, bufs.tiles[: 1 + 3 * n], bufs.order[: n * tile], bufs.ticket)
+    ids, wts = bufs.ids.cpu().view(rows, top).long(), bufs.wts.cpu().view(rows, top)
+    assert torch.equal(ids, want)
+    val = s.gather(1, want)
+    assert torch.equal(wts.isnan(), val.isnan()) and rel(wts[~val.isnan()], val[~val.isnan()]) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("E,top,ff,d", [(12, 2, 1536, 130), (3, 2, 8320, 40), (16, 4, 1100, 520)])
 def test_moe_sets_in_flight(dtype, E, top, ff, d, monkeypatch):
     """The forms of the small tiles' loop: gate / up with one set between two and five workgroups a CU (the first two), one to
