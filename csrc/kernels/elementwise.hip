@@ -8,6 +8,7 @@
 //  swiglu       : h = silu(g)*u on the interleaved gate/up layout                   (K11)
 //  bias_act     : y = act(x + b) [+ residual]  (act: 0 none, 1 gelu)
 //  embedding    : vocab-parallel row gather (+ learned positions)                   (K14)
+//  stage_rows   : the next of a ring of pinned host rows -> the step's device rows
 #include "common.h"
 #include "vwa_kernels.h"
 
@@ -355,3 +356,26 @@ extern "C" int vwa_decode_advance(int* tokens, int* positions, int* ctx_lens, in
   return (int)hipGetLastError();
 }
 
+// ---- a step's rows out of a ring of pinned host rows, the next one at every launch: a captured step graph draws its own rows although
+// steps are queued behind one another, and a step is one launch of the host's.  A copy in front of the graph cost every step whose
+// token is read back 3 - 4 us, since the host is waited for there: 349 -> 345, 444 -> 441, 778 -> 774 us a step of 4, 1 and 32 rows.
+// One workgroup, bound by one trip over the bus behind the cursor's.
+namespace {
+__global__ __launch_bounds__(512) void stage_rows_kernel(const unsigned long long* ring, int pitch, int sets, int* cursor,
+                                                         unsigned long long* dst, int n) {
+  const int at = *cursor;
+  const unsigned long long* src = ring + (size_t)at * pitch;
+  // (system scope: the host wrote these rows since they were last read)
+  for (int i = threadIdx.x; i < n; i += 512) dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __syncthreads();
+  if (threadIdx.x == 0) *cursor = at + 1 < sets ? at + 1 : 0;
+}
+}  // namespace
+
+extern "C" int vwa_stage_rows(const int* ring, int pitch, int sets, int* cursor, int* dst, int n, hipStream_t st) {
+  if (n < 1 || n > pitch || (n | pitch) % 2 || sets < 1 ||
+      ((reinterpret_cast<uintptr_t>(ring) | reinterpret_cast<uintptr_t>(dst)) & 7)) return -1;
+  hipLaunchKernelGGL(stage_rows_kernel, dim3(1), dim3(512), 0, st, reinterpret_cast<const unsigned long long*>(ring), pitch / 2, sets,
+                     cursor, reinterpret_cast<unsigned long long*>(dst), n / 2);
+  return (int)hipGetLastError();
+}

@@ -301,6 +301,8 @@ void vwa_set_attention_impl(int impl);  // 1: multi-query MFMA kernel (default),
 int vwa_flash_attention(const FlashAttnParams* p, hipStream_t st);
 int vwa_embedding(const int* ids, const uint16_t* table, const uint16_t* pos_table, const int* positions,
                   uint16_t* out, int rows, int D, int vocab_start, int vocab_end, hipStream_t st);
+// the first n of the cursor's row of ring [sets][pitch] (pinned host memory) -> dst; the cursor moves on
+int vwa_stage_rows(const int* ring, int pitch, int sets, int* cursor, int* dst, int n, hipStream_t st);
 int vwa_sample(const float* logits, int ld, int rows, int V, const uint32_t* mask, int mask_words,
                const float* temperature, const uint64_t* seed, const int* step, int* out_tokens,
                float* part_val, int* part_idx, int n_chunks, const int64_t* fail_word, hipStream_t st);

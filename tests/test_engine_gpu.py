@@ -1,6 +1,7 @@
 """Whole-model numerics on the GPU: the native-kernel engine (hipGraph-replayed ragged decode,
 prefill path, streaming GEMMs, fused attention) against the CPU reference engine with the SAME
 weights, for Llama (GQA + RoPE) and Whisper (encoder + decoder with cross-attention)."""
+import gc
 import math
 
 import numpy as np
@@ -1063,6 +1064,77 @@ def test_steps_queued_behind_a_busy_device_read_their_own_rows(rows):
     assert want.shape[0] == n and (want[1:] != want[:-1]).any(1).all()
     for _ in range(2):
         assert torch.equal(run(False), want)
+
+
+@pytest.mark.parametrize("rows", [1, 7])
+def test_a_step_is_its_graph(rows, monkeypatch):
+    """A captured step draws its own rows: a step whose pages are there queues no copy beside its replay.  A step that is given up
+    before its launch leaves the next one its rows, and graphs captured on the way (warm-up forwards) neither move the ring nor write
+    pages: all logits are those of steps without graphs."""
+    model = LlamaModel(CFG, device="cuda", seed=4)
+    n = 21
+    toks = np.random.default_rng(5).integers(0, CFG.vocab_size, (n + 1, rows, 3)).tolist()
+
+    def run(graphs):
+        eng = LLMEngine(model, max_seqs=8, max_model_len=256, use_graphs=graphs)
+        assert n > len(eng.bufs.staging)
+        seqs = [eng.new_sequence([], use_prefix_cache=False) for _ in range(rows)]
+        eng.step_batch([(s, t) for s, t in zip(seqs, toks[n])])
+        for s in seqs:
+            eng._ensure_blocks(s, 64)
+        out = []
+        for k in range(n):
+            step = [(s, t[0]) for s, t in zip(seqs, toks[k])]
+            if k == 9:
+                def lost():
+                    raise RuntimeError("given up")
+
+                for s in seqs:  # (its tokens are kept: the step is tried again)
+                    assert s.n_computed == len(s.tokens)
+                eng.chain_gate = lost
+                with pytest.raises(RuntimeError, match="given up"):
+                    eng.run_rows(step, logits_for=[rows - 1], check=False)
+                eng.chain_gate = None
+            if k == 14 and graphs:
+                eng.capture_all(buckets=(2, 16), logit_buckets=(2,))
+            copies = []
+            if graphs and k > 2:
+                with monkeypatch.context() as m:
+                    m.setattr(torch.Tensor, "copy_", lambda *a, **kw: copies.append(a))
+                    eng.run_rows(step, logits_for=list(range(rows)), check=False, defer_head=True)
+            else:
+                eng.run_rows(step, logits_for=list(range(rows)), check=False, defer_head=True)
+            assert not copies
+            out.append(eng.head_logits().clone())
+        return torch.stack(out)
+
+    want, got = run(False), run(True)
+    assert [k for k in range(n) if not torch.equal(got[k], want[k])] == []
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+def test_queued_steps_keep_their_rows_without_their_engine(graphs):
+    """An engine dropped while its last steps are queued: the next engine's pinned rows are others."""
+    model = LlamaModel(CFG, device="cuda", seed=4)
+
+    def run(busy):
+        eng = LLMEngine(model, max_seqs=2, max_model_len=256, kv_blocks=40, use_graphs=graphs)
+        seq = eng.new_sequence([5, 6, 7], use_prefix_cache=False)
+        eng.step_batch([(seq, [5, 6, 7])])
+        eng.run_rows([(seq, 8)], check=False)
+        torch.cuda.synchronize()
+        if busy:
+            torch.cuda._sleep(100_000_000)  # (some 50 ms)
+        return [eng.run_rows([(seq, t)], check=False).clone() for t in (9, 10, 11)]
+
+    want = run(False)
+    torch.cuda.synchronize()
+    got = run(True)
+    gc.collect()
+    others = [LLMEngine(model, max_seqs=2, max_model_len=256, kv_blocks=40, use_graphs=graphs) for _ in range(2)]
+    for e in others:  # (rows of other numbers, where they are the same memory)
+        e.bufs._ring.fill_(1)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 @pytest.mark.parametrize("persist", ["1", "0"])

@@ -107,8 +107,7 @@ class StepBuffers:
         self.slots = self.meta[4 * R : 6 * R].view(torch.int64)
         self.sel = self.meta[6 * R : 7 * R]
         self.shared = self.meta[7 * R : 7 * R + 2]
-        self.ctx_lens.fill_(1)
-        self.slots.fill_(-1)
+        self.inert()
         self.block_table = torch.zeros(max_seqs, max_blocks_per_seq, **i32)
         if hasattr(model, "step_buffers"):  # models with activations of their own
             for name, t in model.step_buffers(max_rows, max_ctx).items():
@@ -131,22 +130,38 @@ class StepBuffers:
         self.part_ml = torch.zeros(max_rows * ns * model.nq * 2, dtype=torch.float32, device=device)
         self.attn_cnt = torch.zeros(max_rows * model.nkv, dtype=torch.int32, device=device)  # chunk tickets
 
+    def inert(self) -> None:
+        """Rows without a slot, a token of context each, nothing shared, the first row selected."""
+        self.meta_all.zero_()
+        self.ctx_lens.fill_(1)
+        self.slots.fill_(-1)
+
     def _host_staging(self, R: int, max_seqs: int, max_blocks_per_seq: int, T: int, C: int, device) -> None:
         cuda = torch.device(device).type == "cuda"
         self.head_idx = torch.zeros(R, dtype=torch.int64, device=device)
-        self.row_table = self.meta_all[T:].view(R, C)
+        self.row_at, self.row_table = T, self.meta_all[T:].view(R, C)
         # the block table as the host has it (np_table; sequences come, grow and go at any time)
         self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
         self.table_dirty = True
         self.staging = StagingRing(lambda n: StepStaging.sets(n, R, T, C, cuda), cuda)
+        self._ring = self.staging.sets[0].ring
+        self._cursor = torch.zeros(1, dtype=torch.int32, device=device)  # the device's place in the ring
 
-    def upload(self, st: "StepStaging", n_rows: int) -> None:
-        """H2D copy of a step's metadata (with the rows' block tables where the chained launch reads them) and of the block
-        table when it changed."""
-        n = self.meta_all.numel() - self.row_table.numel() + n_rows * self.row_table.shape[1] if self.rt_cols and n_rows <= 4 \
-            else self.meta.numel()
-        self.meta_all[:n].copy_(st.h_meta_all[:n], non_blocking=True)
-        self.upload_table()
+    def stage(self, n_rows: int) -> None:
+        """The ring's next set -- the step's metadata, and the rows' block tables where the chained launch reads them -- to the
+        device's rows.  On the GPU a kernel that finds the set by a cursor of its own, so that a captured step holds it; whoever
+        launches it (or replays it) calls staged()."""
+        n = self.row_at + n_rows * self.row_table.shape[1] if self.rt_cols and n_rows <= 4 else -(-self.meta.numel() // 2) * 2
+        if self.meta_all.is_cuda:
+            ops.ext().stage_rows(self._ring, self._cursor, self.meta_all, n)
+        else:
+            self.meta_all[:n].copy_(self._ring[0, :n])
+
+    def staged(self) -> None:
+        """The step that reads the ring's next set is queued (its kernel knows the rows by their address alone)."""
+        self.staging.take()
+        if self.meta_all.is_cuda:
+            ops.ext().host_rows_used(self._ring, self.meta_all)
 
     def upload_table(self) -> None:
         """H2D copy of the block table when it changed, out of pinned rows of its own: copies before it may be queued."""
@@ -163,20 +178,20 @@ class StepStaging:
 
     @classmethod
     def sets(cls, n: int, R: int, T: int, C: int, pin: bool) -> List["StepStaging"]:
-        meta = torch.zeros(n, -(-(T + R * C) // 4) * 4, dtype=torch.int32, pin_memory=pin)
+        ring = torch.zeros(n, T + R * C, dtype=torch.int32, pin_memory=pin)
         head = torch.zeros(n, R, dtype=torch.int64, pin_memory=pin)
-        rows = meta.numpy()
+        rows = ring.numpy()
         rows[:, 3 * R : 4 * R] = 1  # inert rows, as the device's before the first step
         rows[:, 4 * R : 6 * R] = -1
-        return [cls(m, r, h, R, T, C) for m, r, h in zip(meta.unbind(), rows, head.unbind())]
+        return [cls(ring, r, h, R, T, C) for r, h in zip(rows, head.unbind())]
 
-    def __init__(self, meta_all: torch.Tensor, rows: np.ndarray, head_idx: torch.Tensor, R: int, T: int, C: int):
-        self.h_meta_all = meta_all
+    def __init__(self, ring: torch.Tensor, rows: np.ndarray, head_idx: torch.Tensor, R: int, T: int, C: int):
+        self.ring = ring  # (every set's)
         self.np_i32 = rows[: 4 * R].reshape(4, R)
         self.np_slots = rows[4 * R : 6 * R].view(np.int64)
         self.np_sel = rows[6 * R : 7 * R]
         self.np_shared = rows[7 * R : 7 * R + 2]
-        self.np_row_table = rows[T : T + R * C].reshape(R, C)
+        self.np_row_table = rows[T:].reshape(-1, C)
         # rows whose hidden state feeds the LM head when the step computed every row (L == M):
         # gathered on the device through a pinned staging copy (a torch.tensor(list, device=...)
         # here was a pageable, host-blocking copy that waited for the whole step -- measured: 9 of
@@ -336,23 +351,17 @@ class LLMEngine:
 
     def _capture(self, M: int, L: int):
         s = torch.cuda.Stream()
-        b, slots = self.bufs, None
-        if self.stateful:
-            # the warm-up forwards below must not advance a recurrent state: they run this step's rows as
-            # inert ones (no slot), the replay after the capture runs them for real
-            slots = b.slots[:M].clone()
-            b.slots[:M] = -1
+        self.bufs.inert()  # the warm-up forwards write no page and advance no recurrent state; the graph draws its step's own rows
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
             for _ in range(2):
                 self._forward_rows(M, L)
         torch.cuda.current_stream().wait_stream(s)
-        if slots is not None:
-            b.slots[:M] = slots
         g = torch.cuda.CUDAGraph()
         if self.graph_pool is None:
             self.graph_pool = torch.cuda.graph_pool_handle()
         with capture_graph(g, pool=self.graph_pool):
+            self.bufs.stage(M)
             out = self._forward_rows(M, L)
         self.graphs[(M, L, self._gated)] = (g, out)
         return self.graphs[(M, L, self._gated)]
@@ -414,7 +423,7 @@ class LLMEngine:
             slots.append(seq.blocks[pos // bs] * bs + pos % bs)
             pending[sid] = pos + 1
         shared = self._shared_prefix(rows, min(poss) + 1)
-        st = b.staging.next()
+        st = b.staging.peek()
         if logits_for is None or len(logits_for) == n:
             nl, L = n, M
         else:
@@ -439,7 +448,7 @@ class LLMEngine:
             hi[0:3, n:M] = 0
             hi[3, n:M] = 1
             st.np_slots[n:M] = -1
-        b.upload(st, M)
+        b.upload_table()
         if self.chain_gate is not None:
             self._gated = bool(self.chain_gate())
             self.model._chain_gated = self._gated
@@ -452,8 +461,11 @@ class LLMEngine:
         if self.use_graphs:
             g, hs = self.graphs.get((M, L, self._gated)) or self._capture(M, L)
             g.replay()
+            b.staged()
             self.stats["graph_replays"] += 1
         else:
+            b.stage(M)
+            b.staged()
             hs = self._forward_rows(M, L)
         for sid, ln in pending.items():
             self.seqs[sid].n_computed = ln
