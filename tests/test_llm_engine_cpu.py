@@ -368,3 +368,14 @@ def test_no_collection_inside_a_capture(monkeypatch):
         gc.set_threshold(*old)
         if not was:
             gc.disable()
+
+
+def test_staging_rows_are_small_and_made_when_used():
+    """Pinned rows hold the block tables of as many rows as a chained step has, not of every row, and a set's views are made at its
+    first step: both are paid for by whoever builds an engine."""
+    eng = LLMEngine(LlamaModel(SMALL, device="cpu", seed=0), max_seqs=2, max_model_len=256)
+    b = eng.bufs
+    assert b.rt_cols == 16 and b._ring.shape == (1, b.row_at + 4 * 16) and b.staging.sets == [None]
+    seq = eng.new_sequence([1, 2, 3], use_prefix_cache=False)
+    eng.run_rows([(seq, t) for t in (1, 2, 3)], logits_for=[2])
+    assert b.staging.sets[0].np_row_table.shape == (4, 16)

@@ -83,8 +83,8 @@ class WhisperRunner:
 
         def rows(n):
             h = torch.zeros(n, 6 * R, dtype=torch.int32, pin_memory=cuda)
-            return [SimpleNamespace(h_in=t, np_i32=r[: 4 * R].reshape(4, R), np_slots=r[4 * R :].view(np.int64))
-                    for t, r in zip(h.unbind(), h.numpy())]
+            r = h.numpy()
+            return lambda i: SimpleNamespace(h_in=h[i], np_i32=r[i, : 4 * R].reshape(4, R), np_slots=r[i, 4 * R :].view(np.int64))
 
         self.staging = StagingRing(rows, cuda)
         if use_graphs is None:

@@ -41,6 +41,7 @@ from ..utils.staging import StagingRing
 # 4.61 ms bf16, profiles/r4_rows_buckets_8_16.jsonl).  (24 measured the same as 32: the one
 # 128-row GEMM tile and the attention floor dominate there.)
 BUCKETS = tuple(int(b) for b in knob("VWA_ROW_BUCKETS").split(","))
+TABLE_ROWS = 4  # rows of a step whose block tables go with them: as many as the chained launch takes
 
 
 class TPGroupFailure(RuntimeError):
@@ -98,7 +99,8 @@ class StepBuffers:
         self.rt_cols = max_blocks_per_seq if max_blocks_per_seq <= 128 and max_blocks_per_seq % 2 == 0 else 0
         C = max(2, self.rt_cols)
         T = (7 * R + 2 + 15) // 16 * 16  # row table at a 64-byte aligned offset
-        self.meta_all = torch.zeros(T + R * C, **i32)
+        step = torch.zeros(T + R * C + 1, **i32)
+        self.meta_all, self._cursor = step[:-1], step[-1:]  # (the cursor: the device's place in the ring of pinned rows)
         self.meta = self.meta_all[: 7 * R + 2]
         self.tokens = self.meta[0:R]
         self.positions = self.meta[R : 2 * R]
@@ -107,7 +109,8 @@ class StepBuffers:
         self.slots = self.meta[4 * R : 6 * R].view(torch.int64)
         self.sel = self.meta[6 * R : 7 * R]
         self.shared = self.meta[7 * R : 7 * R + 2]
-        self.inert()
+        self.ctx_lens.fill_(1)  # (inert rows)
+        self.slots.fill_(-1)
         self.block_table = torch.zeros(max_seqs, max_blocks_per_seq, **i32)
         if hasattr(model, "step_buffers"):  # models with activations of their own
             for name, t in model.step_buffers(max_rows, max_ctx).items():
@@ -143,15 +146,22 @@ class StepBuffers:
         # the block table as the host has it (np_table; sequences come, grow and go at any time)
         self.np_table = np.zeros((max_seqs, max_blocks_per_seq), dtype=np.int32)
         self.table_dirty = True
-        self.staging = StagingRing(lambda n: StepStaging.sets(n, R, T, C, cuda), cuda)
-        self._ring = self.staging.sets[0].ring
-        self._cursor = torch.zeros(1, dtype=torch.int32, device=device)  # the device's place in the ring
+
+        def sets(n: int):
+            self._ring = torch.zeros(n, T + min(R, TABLE_ROWS) * C, dtype=torch.int32, pin_memory=cuda)
+            head = torch.zeros(n, R, dtype=torch.int64, pin_memory=cuda)
+            rows = self._ring.numpy()
+            rows[:, 3 * R : 4 * R] = 1  # inert rows, as the device's before the first step
+            rows[:, 4 * R : 6 * R] = -1
+            return lambda i: StepStaging(rows[i], head[i], R, T, C)
+
+        self.staging = StagingRing(sets, cuda)
 
     def stage(self, n_rows: int) -> None:
         """The ring's next set -- the step's metadata, and the rows' block tables where the chained launch reads them -- to the
         device's rows.  On the GPU a kernel that finds the set by a cursor of its own, so that a captured step holds it; whoever
         launches it (or replays it) calls staged()."""
-        n = self.row_at + n_rows * self.row_table.shape[1] if self.rt_cols and n_rows <= 4 else -(-self.meta.numel() // 2) * 2
+        n = self.row_at + n_rows * self.row_table.shape[1] if self.rt_cols and n_rows <= TABLE_ROWS else -(-self.meta.numel() // 2) * 2
         if self.meta_all.is_cuda:
             ops.ext().stage_rows(self._ring, self._cursor, self.meta_all, n)
         else:
@@ -176,17 +186,7 @@ class StepStaging:
     and numpy views of them -- the per-step row metadata is written with a handful of slice assignments instead of ~5 torch
     element writes per row."""
 
-    @classmethod
-    def sets(cls, n: int, R: int, T: int, C: int, pin: bool) -> List["StepStaging"]:
-        ring = torch.zeros(n, T + R * C, dtype=torch.int32, pin_memory=pin)
-        head = torch.zeros(n, R, dtype=torch.int64, pin_memory=pin)
-        rows = ring.numpy()
-        rows[:, 3 * R : 4 * R] = 1  # inert rows, as the device's before the first step
-        rows[:, 4 * R : 6 * R] = -1
-        return [cls(ring, r, h, R, T, C) for r, h in zip(rows, head.unbind())]
-
-    def __init__(self, ring: torch.Tensor, rows: np.ndarray, head_idx: torch.Tensor, R: int, T: int, C: int):
-        self.ring = ring  # (every set's)
+    def __init__(self, rows: np.ndarray, head_idx: torch.Tensor, R: int, T: int, C: int):
         self.np_i32 = rows[: 4 * R].reshape(4, R)
         self.np_slots = rows[4 * R : 6 * R].view(np.int64)
         self.np_sel = rows[6 * R : 7 * R]
@@ -432,7 +432,7 @@ class LLMEngine:
             if L < M:  # (L == M: no saving -- compute every row and index on the host side)
                 st.np_sel[:nl] = logits_for
                 st.np_sel[nl:L] = logits_for[-1]
-        rtab = st.np_row_table if b.rt_cols and M <= 4 else None
+        rtab = st.np_row_table if b.rt_cols and M <= TABLE_ROWS else None
         if rtab is not None:  # after the loop: a later row of a sequence may have added its last block
             for i, (seq, _) in enumerate(rows):
                 rtab[i, : len(seq.blocks)] = seq.blocks

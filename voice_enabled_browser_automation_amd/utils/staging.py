@@ -1,7 +1,7 @@
 """Pinned host rows for steps that are queued without a wait for the one before."""
 from __future__ import annotations
 
-from typing import Callable, Generic, List, TypeVar
+from typing import Callable, Generic, List, Optional, TypeVar
 
 import torch
 
@@ -9,13 +9,16 @@ T = TypeVar("T")
 
 
 class StagingRing(Generic[T]):
-    """``n`` sets of rows (``make(n)``: together, since an allocation of pinned memory costs a few us) in turn, one a step: a queued
-    step reads its own set, and a set is written again only when the step that had it is through, which an event behind every half
-    of the ring tells.  (An event a step costs the stream a few us.)  One stream at a time, as the device buffers that the rows go
-    to.  Without a GPU one set is enough."""
+    """``n`` sets of rows in turn, one a step: a queued step reads its own set, and a set is written again only when the step that
+    had it is through, which an event behind every half of the ring tells.  (An event a step costs the stream a few us.)  One
+    stream at a time, as the device buffers that the rows go to.  Without a GPU one set is enough.
 
-    def __init__(self, make: Callable[[int], List[T]], cuda: bool, n: int = 16):
-        self.sets: List[T] = make(n if cuda else 1)
+    ``make(n)`` allocates all of them (pinned memory costs a few us a piece) -> the function that gives set i when it is first
+    used: views of sixteen sets at once were 30 us of an engine's construction."""
+
+    def __init__(self, make: Callable[[int], Callable[[int], T]], cuda: bool, n: int = 16):
+        self.sets: List[Optional[T]] = [None] * (n if cuda else 1)
+        self._make = make(len(self.sets))
         self._done = [torch.cuda.Event(), torch.cuda.Event()] if cuda else []  # behind the last use of either half
         self._at, self._used = 0, False  # the next step's set
 
@@ -31,7 +34,10 @@ class StagingRing(Generic[T]):
                 if self._used:
                     self._done[half].synchronize()
                 self._used = self._used or half == 1
-        return self.sets[self._at]
+        st = self.sets[self._at]
+        if st is None:
+            st = self.sets[self._at] = self._make(self._at)
+        return st
 
     def take(self) -> None:
         """What reads that set is queued."""
