@@ -60,6 +60,18 @@ def engine(model, **kw):
     return LLMEngine(model, **dict(dict(max_seqs=3, max_model_len=256, kv_blocks=40), **kw))
 
 
+@pytest.mark.parametrize("rows", [1, 7, 16, 17, 777])
+def test_branch_rows_of_prompts(rows):
+    """A row of the branch buffer for each of a token's experts, and four for each of few tokens (a 32-bit product's quarters): not four
+    for every token of a prompt."""
+    top = 2
+    cfg = O.model_config(76, 101, [O.rglru_layer(60, 3, 4, O.dense(56)), O.rglru_layer(40, 1, 1, O.moe(4, top, 40))])
+    w = O.random_weights(cfg, 5)
+    for dtype, few in ((torch.float32, 4 * min(rows, 16)), (torch.bfloat16, 0)):
+        m = RipupelModel(RipupelConfig.from_json(cfg), weights=w, dtype=dtype)
+        assert m.row_buffers(rows, 256)["branch"].shape[0] == max(top * rows, few)
+
+
 def test_config_and_registry(folder):
     cfg = config_from_dir(folder)
     assert isinstance(cfg, RipupelConfig) and get_config(folder) == cfg and model_class(cfg) is RipupelModel

@@ -287,14 +287,15 @@ class RipupelModel:
         # once, never written (so each distinct layout has rows of its own)
         cols = {D.cols for D in self.dims}
         moes = [(L.mlp.experts, L.mlp.top, F) for L, F in zip(self.cfg.layers, self.ffs) if isinstance(L.mlp, MoEConfig)]
-        parts = max([4 if dt == torch.float32 else 1] + [t for _, t, _ in moes])  # (32-bit products leave quarters, ops.linear_rows)
+        parts = max([1] + [t for _, t, _ in moes])
+        quarters = 4 * min(rows, ops.QUARTER_ROWS) if dt == torch.float32 else 0  # (rows of few tokens' products, ops.linear_rows)
         lat = [D.H * D.dk for D in self.dims if isinstance(D, LatentDims)]
         dense = [F for L, F in zip(self.cfg.layers, self.ffs) if isinstance(L.mlp, DenseFFConfig)]
         return dict(hidden=e(rows, self.d_pad, t=torch.float32), normed=e(rows, self.d_pad),
                     mix=e(rows * max(D.n_in for D in self.dims)), q=e(rows * max(lat)) if lat else None,
                     cat={c: e(rows, c) if c % 128 == 0 else torch.zeros(rows, _up(c, 128), dtype=dt, device=dev) for c in cols},
                     # (rows of pairs no token chose -- padded rows of a step graph -- are never written)
-                    branch=torch.zeros(rows * parts, self.n_out, dtype=dt, device=dev),
+                    branch=torch.zeros(max(rows * parts, quarters), self.n_out, dtype=dt, device=dev),
                     act=e(rows * max(dense)) if dense else None,
                     moe=ops.moe_buffers(rows, moes, dt, dev) if moes else None)
 

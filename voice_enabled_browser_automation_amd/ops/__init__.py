@@ -1229,5 +1229,5 @@ def env_int(name: str) -> int:
 
 from .mixers import (LatentScratch, LatentWeights, MoeWeights, RgLruWeights, fragments, gate_fragments,  # noqa: E402,F401
                      latent_attention, latent_qkv, moe, moe_buffers, rglru, tile_weights)
-from .stack import (TalkScratch, add_norm, embedding_f32, layernorm_f32, linear_parts, linear_rows, linear_split, mingru, plan_runs,  # noqa: E402,F401
+from .stack import (QUARTER_ROWS, TalkScratch, add_norm, embedding_f32, layernorm_f32, linear_parts, linear_rows, linear_split, mingru, plan_runs,  # noqa: E402,F401
                     qkv_cache_mingru, qkv_cache_write, talk_attention, talk_fragment, talk_mingru_step)

@@ -137,6 +137,9 @@ def linear_parts(x: torch.Tensor, w) -> Optional[torch.Tensor]:
     return _ext().linear_parts(x, w.t, GEMM_WS_FLOATS)
 
 
+QUARTER_ROWS = 16  # rows up to which a 32-bit product has quarters: one row tile (vwa_gemm_f32_quarters)
+
+
 def linear_rows(x: torch.Tensor, w, rows: torch.Tensor) -> int:
     """x @ w^T to the first rows of ``rows`` for add_norm, as many for a row of x as this returns: one, or (few rows of 32-bit
     weights) the four quarters of its sums, which add_norm adds in the order of a whole product's."""
