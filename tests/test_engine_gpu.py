@@ -376,6 +376,42 @@ def test_failed_chained_step_is_rerun_on_per_kernel_path(monkeypatch):
         assert err < 0.02 * (1 + want.abs().max().item()), err
 
 
+@pytest.mark.parametrize("fails", [True, False])
+def test_a_ranks_head_waits_for_its_layers_check(monkeypatch, fails):
+    """A verified step of a tensor-parallel rank: where its chained launch timed out on a peer it raises, without the head's gather
+    having been started; else the gathered logits are returned."""
+    from types import SimpleNamespace
+
+    from voice_enabled_browser_automation_amd.runtime.engine import TPGroupFailure
+
+    ops.ext()
+    model = LlamaModel(CFG, device="cuda", seed=4)
+    e = LLMEngine(model, max_seqs=1, max_model_len=128, kv_blocks=10, block_size=16)
+    s = e.new_sequence(list(range(10)), use_prefix_cache=False)
+    e.prefill(s)
+    e.run_rows([(s, 11)])
+    queued, gathered = e._chain_word, []
+    group = SimpleNamespace(size=2, all_gather_vocab=lambda t, n: gathered.append(n) or t)
+
+    def after_the_layers():
+        model.tp = group
+        if fails:
+            model.chain_error_word().fill_(1)  # what a timed-out barrier spin writes
+        return queued()
+
+    monkeypatch.setattr(e, "_chain_word", after_the_layers)
+    alone = model.tp
+    try:
+        if fails:
+            with pytest.raises(TPGroupFailure):
+                e.run_rows([(s, 12)])
+            assert not gathered
+        else:
+            assert e.run_rows([(s, 12)]) is not None and gathered == [CFG.vocab_size]
+    finally:
+        model.tp = alone
+
+
 def test_asr_device_decode_loop_matches_host_loop():
     """The device-resident greedy loop (sampled token fed back on the GPU, decode_advance kernel,
     step graphs replayed back to back) produces the same tokens as the host-driven loop, in the

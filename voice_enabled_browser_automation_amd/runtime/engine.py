@@ -482,11 +482,14 @@ class LLMEngine:
             self._head_rows = hs[:nl]
         check = check and chained and self.device.type == "cuda"
         done = self._chain_word() if check else None
-        logits = None if defer_head else self.head_logits()  # (queued while the host waits for the layers: a failed step's are dropped)
+        # the head is queued while the host waits for the layers (a failed step's logits are dropped), but for a rank's: its gather
+        # is not to wait for peers that the failure is about
+        late = check and getattr(getattr(self.model, "tp", None), "size", 1) > 1
+        logits = None if defer_head or late else self.head_logits()
         if check and self._chain_failed(done):
             self._head_rows = None
             return self.recover_step()
-        return logits
+        return self.head_logits() if late and not defer_head else logits
 
     def _chain_word(self) -> Optional["torch.cuda.Event"]:
         """Queues the copy of the chained launch's error word to the host behind the step's layers -> the event behind it."""
