@@ -217,9 +217,9 @@ VWA_DEVICE float silu(float x) { return x / (1.f + __expf(-x)); }
 // branch: some 25 vector instructions of which 2 are transcendental, where erff has two branches of some 20 each, gone through element
 // by element while an epilogue's waves do nothing else.  us of a product with it, 0.5 x (1 + erff(x / sqrt 2)) -> here (without: in
 // brackets): 12000 x 5120 x 1280 201 -> 180 (147), 1500 x 5120 x 1280 33.2 -> 29.4 (25.6), 8 x 5120 x 1280 8.7 -> 8.2 (8.1).
-// Error against 64 bits, at most (mean), erff -> here: [-4, -2) 6.0e-8 (2.3e-8) -> 2.5e-8 (2.3e-9), [-1, 0) 4.1e-8
-// (6.2e-9) -> 3.9e-8 (5.2e-9), [0, 1) 9.1e-8 (1.2e-8) -> 6.1e-8 (8.8e-9), [2, 6) 4.5e-7 (9.9e-8) -> 2.4e-7 (8.1e-8); nor is any other
-// part of [-14, 14) less exact.  The tail alone, at all |x|, would be: 166 us, but 4.8e-8 in [-1, -1/2).
+// Error against 64 bits, at most (mean), erff -> here, 840 thousand values of each of 32 parts of [-14.5, 14.5): [-3, -2.5) 4.9e-8
+// (2.1e-8) -> 1.3e-8 (2.5e-9), [-1.25, -1) 6.6e-8 (1.5e-8) -> 5.7e-8 (1.2e-8), [-1, -3/4) 4.3e-8 (1.0e-8) -> 3.9e-8 (9.9e-9), [3/4, 1)
+// 9.4e-8 (2.3e-8) -> 6.2e-8 (1.7e-8), [4, 6) 4.5e-7 (1.2e-7) -> 2.4e-7 (1.0e-7); no part is less exact.  The tail alone, at all |x|, would be: 166 us, but 4.8e-8 in [-1, -1/2).
 // NaN and -infinity give NaN, infinity itself, either way.
 VWA_DEVICE float gelu_erf(float x) {
   const float t = fminf(fabsf(x), 14.5f), s = t * t, h = 0.5f * x, m = t * __builtin_amdgcn_rcpf(t + 4.5f);

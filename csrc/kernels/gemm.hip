@@ -1415,13 +1415,18 @@ extern "C" void vwa_gemm_set_split_fill(int pct) { g_split_fill_pct = pct < 0 ? 
 
 extern "C" void vwa_gemm_set_p8(int mode) { g_p8_mode = mode; }
 
-extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int parts, int* columns, int* splits) {
+extern "C" void vwa_gemm_plan(int epi, const GemmParams* pp, int parts, int* columns, int* splits, int* groups) {
   GemmParams p = *pp;
   p.keep_order = keeps_order(epi, p);
   const Plan pl = choose(p, epi, parts);
   const int per = cdiv(p.K / BKG, pl.splits);
   p.splits = *splits = cdiv(p.K / BKG, per);
-  *columns = pl.p8 ? CfgP8::BN : !p.keep_order && !p.sw && takes_narrow(epi) && narrow(p) ? CfgN::BN : small_tile(p, epi) == CfgKw::BN ? CfgKw::BN : CfgS::BN;
+  *columns = pl.p8 ? CfgP8::BN : !p.keep_order && !p.sw && takes_narrow(epi) && narrow(p) ? CfgN::BN : CfgS::BN;
+  *groups = 1;
+  if (!pl.p8 && small_tile(p, epi) != CfgS::BN) {
+    *columns = small_tile(p, epi) == CfgKw::BN ? CfgKw::BN : CfgK::BN;
+    *groups = CfgK::GROUPS;
+  }
 }
 
 namespace {

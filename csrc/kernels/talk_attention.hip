@@ -209,8 +209,9 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
 // heads and 1024 channels 10.9 -> 8.6.  The row's query and own key are turned once a workgroup, through LDS: every wave for itself
 // took 6.6 and 10.7 (94 registers, and the table's row four times).  Bound by its round trips: ids and positions, table, keys.
 constexpr int kStepParts = 2;                        // workgroups of a row's keys and values
-// Scoring workgroups of a launch at most: as many as are resident at once beside the others.  Each row's walk its chunks; one a
-// chunk of the longest context would be mostly workgroups without keys (48 rows of 2048: 3840, 11.1 -> 10.7 us).
+// Scoring workgroups that a launch aims at: as many as are resident at once beside the others, in whole ones to a row, kv head and 16 of
+// its query heads, and at least one (64 rows of 16 kv heads: 1024; none waits for another).  They walk the row's chunks; one a chunk of
+// the longest context would be mostly workgroups without keys (48 rows of 2048: 3840, 11.1 -> 10.7 us).
 constexpr int kStepWgs = 768;
 
 template <class T>

@@ -279,11 +279,12 @@ int vwa_gemm_grouped(int epi, const GemmParams* p, hipStream_t st);
 int vwa_gemm_splits(int M, int N, int K, int cus, int64_t ws_floats, int f8);
 void vwa_gemm_set_split_fill(int pct);  // split-K while tiles x splits < pct % of the CUs (0: bf16 75, fp8 100)
 void vwa_gemm_set_p8(int mode);  // 0: 128^2 kernel only, 1: 256^2 from 256 rows (bf16: of pre-tiled whole column tiles), 2: by an estimate
-// the columns of a tile (256: the 256^2 one) and the slices that vwa_gemm (parts: vwa_gemm_parts) would take
+// the columns of the tile (64, 128, 192; 256: the 256^2 one), the slices and the groups of waves (2: they take the stages of K in turn;
+// of 128 or 192 columns) that vwa_gemm (parts: vwa_gemm_parts) would take
+void vwa_gemm_plan(int epi, const GemmParams* p, int parts, int* columns, int* splits, int* groups);
 // Columns of a product's first launch where two share them (0: one launch), and the parameters of either
 int vwa_gemm_cut(int epi, const GemmParams* p);
 void vwa_gemm_part(int epi, const GemmParams* p, int n, int second, GemmParams* part);
-void vwa_gemm_plan(int epi, const GemmParams* p, int parts, int* columns, int* splits);
 int vwa_row_rstd(const uint16_t* x, int ldx, int M, int K, float eps, float* rstd, hipStream_t st);
 int vwa_rmsnorm(const uint16_t* x, const uint16_t* residual, uint16_t* residual_out, const uint16_t* w,
                 uint16_t* y, int rows, int D, int ldx, float eps, hipStream_t st);

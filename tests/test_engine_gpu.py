@@ -1051,7 +1051,6 @@ def test_a_sequence_freed_behind_its_last_step_keeps_its_pages_there(rows):
         for at in range(0, 144, 48):
             eng.step_batch([(seq, toks[at : at + 48])])
         torch.cuda.synchronize()
-        eng.host_synced()
         if delay:
             torch.cuda._sleep(100_000_000)  # (some 50 ms: the copies and the step queue behind it)
         out = eng.step_batch([(seq, toks[144:])], range(rows))  # (position 144: a block of its own)

@@ -91,8 +91,8 @@ def test_columns_of_two_launches_are_whole_rounds(E):
                 if cut:
                     seen += 1
                     rows = -(-M // 256)
-                    tiles = rows * cut // 256
-                    assert tiles // 256 * 256 <= tiles and -(-tiles // 256) * 256 - tiles < rows  # (no column tile more fits its rounds)
+                    rounds, tiles = rows * -(-N // 256) // 256, rows * cut // 256
+                    assert tiles <= 256 * rounds < tiles + rows  # (all of the whole rounds: no column tile more fits them)
                 assert E.gemm_cut(0, M, N, K, keep_order=True) == 0 and E.gemm_cut(5, M, N, K) == 0
     assert seen > 5 and E.gemm_cut(0, 64, 32896, 4096) == 0 and E.gemm_cut(6, 2048, 32896, 4096) == 32768
     E.gemm_set_p8(0)

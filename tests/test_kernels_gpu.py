@@ -223,6 +223,31 @@ def test_gelu_of_every_value():
     assert y[xd == math.inf].eq(math.inf).all() and y[xd == -math.inf].isnan().all() and y[xd.isnan()].isnan().all()
 
 
+@pytest.mark.parametrize("a,b", [(-14, -8), (-8, -6), (-6, -4), (-4, -2), (-2, -1), (-1, -0.5), (-0.5, 0), (0, 0.5), (0.5, 1), (1, 2), (2, 4),
+                                 (4, 6), (6, 14)])
+def test_gelu_in_32_bits_is_as_exact_as_erf(a, b):
+    """x Phi(x) of 32-bit values, as a product with 32-bit results stores it, against 64 bits: nowhere further off than x (1 + erf) / 2
+    computed in 32 bits on the same device, at most and on average.  (A value is three bf16 pieces times ones: the sums are exact.)"""
+    n, cols = 6000, 42
+    gen = torch.Generator().manual_seed(int(16 * (a + 20)))
+    v = (torch.rand(n, cols, generator=gen, dtype=torch.float64) * (b - a) + a).float()
+    hi = v.to(BF)
+    mid = (v - hi.float()).to(BF)
+    lo = (v - hi.float() - mid.float()).to(BF)
+    x, w = torch.zeros(n, 128, dtype=BF), torch.zeros(48, 128, dtype=BF)
+    for k, piece in enumerate((hi, mid, lo)):
+        x[:, k : 3 * cols : 3] = piece
+        w[torch.arange(cols), 3 * torch.arange(cols) + k] = 1
+    x, w, y, v = x.to(DEV), w.to(DEV), torch.empty(n, 48, device=DEV), v.to(DEV)
+    ops.gemm(x, w, y)
+    assert torch.equal(y[:, :cols], v)
+    ops.gemm(x, w, y, epi="gelu")
+    d = v.double()
+    want = d / 2 * torch.erfc(-d / 2 ** 0.5)
+    here, erf = ((t.double() - want).abs() for t in (y[:, :cols], 0.5 * v * (1 + torch.erf(v * 0.5 ** 0.5))))
+    assert here.max() <= erf.max() and here.mean() <= erf.mean()
+
+
 def test_bias_act_embedding():
     x, b, r = rnd(5, 64), rnd(64), rnd(5, 64)
     y = torch.empty_like(x)
@@ -748,28 +773,40 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
-@pytest.mark.parametrize("M,N,K,columns", [(128, 28672, 4096, 128), (1011, 4096, 640, 128), (1010, 1040, 2048, 128), (700, 2048, 4096, 128),
-                                           (130, 24496, 2048, 192), (1011, 6144, 4096, 192), (513, 4096, 4096, 192), (300, 12208, 4224, 192)])
-def test_gemm_of_two_wave_groups(M, N, K, columns):
-    """Two groups of waves that take the stages of K in turn, over the epilogues: odd numbers of k-groups, slices, rows
-    and columns past the last whole tile.  f32 results: K additions, each rounded by 2^-24 of a partial sum, signs at random, and in
-    bf16 half a unit in the last place, of the result and (residuals) of nothing else."""
+@pytest.mark.parametrize("M,N,K,columns,slices", [(128, 528, 640, 128, 1), (128, 28672, 4096, 128, 1), (1011, 4096, 640, 128, 1),
+                                                  (385, 4112, 2048, 128, 1), (1011, 3088, 1408, 128, 1), (1010, 1040, 2176, 128, 3),
+                                                  (1011, 1040, 4224, 128, 3), (130, 24496, 2048, 192, 1), (1011, 6144, 4096, 192, 1),
+                                                  (300, 12208, 4224, 192, 1), (513, 4096, 4096, 192, 2), (700, 1296, 8192, 192, 6)])
+def test_gemm_of_two_wave_groups(M, N, K, columns, slices):
+    """Two groups of waves that take the stages of K in turn, over the epilogues: odd and even numbers of k-groups, slices (of equal
+    and unequal lengths), rows and columns past the last whole tile.  Every product here is asked whether it takes them: the tile of
+    192 columns has no residuals.  f32 results: K additions, each rounded by 2^-24 of a partial sum, signs at random, and in bf16 half a
+    unit in the last place, of the result and (residuals) of nothing else.  Sums of squares (64 bits of 2^-24): those of the stored
+    row, each chunk's to 2^-25 and 32 bits."""
     E = ops.ext()
-    assert E.gemm_tile(0, M, N, K)[0] == columns
+    takes = lambda epi: E.gemm_choice(epi, M, N, K)  # noqa: E731
     x, w = torch.randn(M, K, device=DEV).to(BF), (torch.randn(N, K, device=DEV) * K ** -0.5).to(BF)
     wt, b, res = ops.TiledWeight(w), rnd(N), rnd(M, N)
     exp = x.double() @ w.double().T
     out = torch.empty(M, N, device=DEV)
+    assert takes(0) == (columns, slices, 2)
     for _ in range(3):
         ops.gemm(x, wt, out.fill_(7.0))
         assert float((out.double() - exp).norm() / exp.norm()) < 2.0 ** -24 * K ** 0.5
     near = lambda got, y: float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
     y = exp + b.double()
     assert near(ops.linear(x, wt, b), y)
+    assert takes(3)[::2] == (columns, 2)
     assert near(ops.linear(x, wt, b, act="gelu"), y / 2 * torch.erfc(-y / 2 ** 0.5))
-    assert near(ops.linear(x, wt, b, residual=res), y + res.double())
-    g, u = exp.view(M, N // 32, 2, 16).unbind(2) if N % 32 == 0 else (None, None)
-    if g is not None:
+    assert takes(1)[::2] == (128, 2) if columns == 128 else takes(1)[0] != 192
+    got, ss = torch.empty(M, N, dtype=BF, device=DEV), torch.zeros(M, dtype=torch.int64, device=DEV)
+    ops.gemm(x, wt, got, epi="resid", bias=b, residual=res, ss_out=ss)
+    assert near(got, y + res.double())
+    squares = got.double().square().sum(1)
+    assert bool(((ss.double() * 2.0 ** -24 - squares).abs() <= N / 8 * 2.0 ** -25 + squares * 2.0 ** -20).all())
+    if N % 32 == 0:
+        assert takes(2)[::2] == (columns, 2)
+        g, u = exp.view(M, N // 32, 2, 16).unbind(2)
         assert near(ops.linear_swiglu(x, wt), (g * torch.sigmoid(g) * u).reshape(M, N // 2))
 
 
@@ -1196,13 +1233,14 @@ def test_gemm_qkv_epilogue_fused(M, kind, monkeypatch):
             close(a, b, 3e-2, 3e-2)
 
 
-@pytest.mark.parametrize("hd,nq,nkv", [(128, 32, 8), (64, 64, 16)])
-def test_qkv_epilogue_of_two_wave_groups(hd, nq, nkv, monkeypatch):
-    """Heads rotated and written in the epilogue of the 192-column tile, heads across its edges, against product and rotation apart:
+@pytest.mark.parametrize("hd,nq,nkv,M,K,columns", [(128, 32, 8, 1011, 4096, 192), (64, 64, 16, 1011, 4096, 192), (128, 32, 8, 257, 2048, 128),
+                                                   (64, 64, 16, 300, 1408, 128)])
+def test_qkv_epilogue_of_two_wave_groups(hd, nq, nkv, M, K, columns, monkeypatch):
+    """Heads rotated and written in the epilogue of the tiles of 192 (heads across its edges) and 128 columns, against product and rotation apart:
     values of a normed row are of order one, 6 at most, rounded once (2^-9 of them) here and twice there, the first time both of a
     rotated pair: 2^-9 6 (2 + sqrt 2) = 4e-2."""
-    M, K, n = 1011, 4096, (nq + 2 * nkv) * hd
-    assert ops.ext().gemm_tile(5, M, n, K)[0] == 192
+    n = (nq + 2 * nkv) * hd
+    assert ops.ext().gemm_choice(5, M, n, K) == (columns, 1, 2)
     w = ops.TiledWeight(ops.permute_qkv_rows(rnd(n, K, scale=K ** -0.5), nq + 2 * nkv, hd))
     x, rope = rnd(M, K), ops.rope_table(2048, hd, 5e5, device=DEV)
     pos = torch.arange(100, 100 + M, dtype=torch.int32, device=DEV)

@@ -87,7 +87,6 @@ def main():
             hs.append((time.perf_counter() - h0) * 1e6)
             ev[1].record()
             torch.cuda.synchronize()
-            e.host_synced()
             ts.append(ev[0].elapsed_time(ev[1]))
         fwd = sorted(ts)[len(ts) // 2]
         host_us = sorted(hs)[len(hs) // 2]  # CPU time of building + launching the step
@@ -97,7 +96,6 @@ def main():
             e.run_rows(rows(), check=False)
             ev[1].record()
             torch.cuda.synchronize()
-            e.host_synced()
             ts.append(ev[0].elapsed_time(ev[1]))
         full = sorted(ts)[len(ts) // 2]
         emit({"what": "decode_step", "model": a.model, "dtype": a.dtype, "rows": M, "chained": m._chain_ok(M),

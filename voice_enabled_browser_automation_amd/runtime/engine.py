@@ -508,10 +508,6 @@ class LLMEngine:
         done.synchronize()
         return bool(self._step_err[0].item() != 0)
 
-    def host_synced(self) -> None:
-        """The caller has observed the stream past the last step (e.g. read its sampled tokens).  (Steps need no such word any more:
-        each has staging rows of its own.)"""
-
     def head_logits(self, col_mask: Optional[torch.Tensor] = None, mask_rows: int = 1,
                     gather: bool = True) -> torch.Tensor:
         """LM head of the last ``run_rows`` step's selected rows -> f32 logits [rows, V].

@@ -104,7 +104,6 @@ class TokenScheduler:
         self.engine.sample(logits, mask=None, temperature=None if self.d_temp is None else self.d_temp[:k],
                            seed=self.d_seed, step=self.d_step, out_tokens=self.d_tok[:k])
         toks = self.d_tok[:k].tolist()
-        self.engine.host_synced()
         self.stats["sampled"] += k
         finished = []
         for r, t in zip(sampled, toks):
