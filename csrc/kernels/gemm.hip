@@ -1145,9 +1145,13 @@ bool takes_groups(const GemmParams& p, int epi, int n) {
 // slices in powers of two until 75 % of the CUs have a tile) were 12 %: 12000 x 1280 x 5120 (235 large tiles) 165 -> 115 us,
 // 768 x 4096 x 14336 155 -> 86, 512 x 28672 x 4096 132 -> 93, 1863 x 6144 x 4096 115 -> 83.
 //   a round of the CUs costs so much per k-group and so much to start and store; a part of a last round 70 % and its share;
-//   128^2 tiles run two to a CU, one alone is faster, two groups on one (CfgK, CfgKw: fitted to 16 shapes against it) faster still
-//   wherever every tile has a CU; beyond that tiles by twos are (1024 x 8192 x 2048, 512 tiles: 41 us, 48 of two groups);
+//   128^2 tiles run two to a CU, one alone is faster, two groups on one (CfgK, CfgKw) faster still wherever every tile has a CU;
+//   beyond that tiles by twos are (1024 x 8192 x 2048, 512 tiles: 41 us, 48 of two groups);
 //   the slices' f32 partials are written and read.
+//   Two groups have fewer k-groups each to pay for their start and the meeting of their sums: from 8 of a slice on (over 131 products of
+//   5 .. 7 they were 1.4 % slower, 1.14 times at worst), from 11 where one row block has the weight to itself (128 rows: 8 and 10 up to
+//   1.08 times).  192 columns in slices must be 5 % ahead by the estimate: taken at any lead, 29 of 70 such products were slower.  Of 728
+//   products with other tiles than without groups: 8.0 % less time on average, 12 are 2 - 4.5 % slower (profiles/gemm_tiles_ab.csv).
 // W8A8 (k-groups of half the stages): fitted to 690 timings of 60 shapes (80 .. 6000 rows, 1024 .. 28672 columns, K 1280 ..
 // 14336), 11 % off; it picks the tile alone: slices in another order move a few bf16 activations by a bit, and every moved one
 // can flip its fp8 code further on, so they stay those of vwa_gemm_splits.  2720 x 4096 x 14336 224 -> 125 us, 2720 x 28672 x
@@ -1170,8 +1174,8 @@ float estimate(const GemmParams& p, bool p8, int s, int epi, int* tile = nullptr
   if (!p8) {
     if (tile) *tile = CfgS::BN;
     for (const int n : {CfgK::BN, CfgKw::BN}) {
-      if (!takes_groups(p, epi, n) || (int64_t)cdiv(p.M, CfgK::BM) * cdiv(p.N, n) * s > p.cus) continue;
-      const float g = n == CfgK::BN ? kg * 0.99f + 3.6f : kg * 1.18f + 5.f;
+      if (!takes_groups(p, epi, n) || kg < (p.M <= CfgK::BM ? 11 : 8) || (int64_t)cdiv(p.M, CfgK::BM) * cdiv(p.N, n) * s > p.cus) continue;
+      const float g = n == CfgK::BN ? kg * 0.99f + 3.6f : s == 1 ? kg * 1.18f + 5.f : 1.05f * (kg * 1.18f + 5.f) + 0.05f * sum;
       if (g < us) {
         us = g;
         if (tile) *tile = n == CfgK::BN ? -CfgK::BN : CfgKw::BN;
@@ -1212,7 +1216,8 @@ bool reachable(const GemmParams& p) {
 // Columns of a product that fill whole rounds of the CUs with large tiles, where it is cheaper by the estimate to give the rest a
 // launch of its own, with tiles and slices of its own (0: not).  The tiles past the last whole round cost nearly a round of their
 // own, however few: 2048 x 32896 x 4096 is four rounds and eight tiles, 482 -> 438 us in two launches (398 of them the whole rounds').
-// 1024 x 17664 x 2048 86 -> 76 us, 1300 x 22528 x 4096 238 -> 206, 1900 x 26624 x 4096 341 -> 333.
+// 1024 x 17664 x 2048 86 -> 76 us, 1300 x 22528 x 4096 238 -> 206, 1900 x 26624 x 4096 341 -> 333.  182 products that are cut: 10 % less
+// time on average, one (850 x 17664 x 2048, whose one-group tiles fill two rounds) 4 - 7 % more (profiles/gemm_tiles_ab.csv).
 int whole_rounds(const GemmParams& p, int epi) {
   if (!reachable(p)) return 0;  // (one launch, which refuses it whole)
   if (p.M < 128 || p.keep_order || p.sw || p.nbatch > 1 || p.cus <= 0 || g_p8_mode != 2 || g_split_fill_pct != 0) return 0;

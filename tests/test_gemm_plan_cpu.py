@@ -106,3 +106,25 @@ def test_a_product_past_the_offsets_has_one_launch(E):
     assert 32768 * 32640 * 2 < 32896 * 32640 * 2 < reach <= 32912 * 32640 * 2
     assert E.gemm_cut(0, 2048, 32896, 32640) == 32768
     assert E.gemm_cut(0, 2048, 32912, 32640) == 0
+
+
+def test_two_wave_groups_have_stages_to_share(E):
+    """Two groups of waves from 8 k-groups of a slice on, from 11 where one row block takes the weight alone, with every tile and slice
+    on a CU of its own; other tiles, kept orders, row-major and fp8 weights have one group."""
+    seen = set()
+    for M in (65, 127, 128, 129, 300, 513, 1011, 2048, 4096):
+        for N in (400, 1024, 2560, 6144, 12288, 28672):
+            for K in (128, 640, 1024, 1280, 1408, 4096, 14336):
+                for epi in (0, 1, 3, 5):
+                    columns, slices, groups = E.gemm_choice(epi, M, N, K)
+                    assert groups == 1 or columns in (128, 192)
+                    assert columns != 192 or (groups == 2 and epi != 1)
+                    if groups == 2:
+                        seen.add((columns, slices > 1))
+                        assert M >= 128 and -(-K // 128 // slices) >= (11 if M <= 128 else 8)
+                        assert -(-M // 128) * -(-N // columns) * slices <= 256
+                for kw in (dict(keep_order=True), dict(w_tiled=False), dict(f8=1), dict(f8=2)):
+                    assert E.gemm_choice(0, M, N, K, **kw)[2] == 1
+    assert seen == {(c, s) for c in (128, 192) for s in (False, True)}
+    assert E.gemm_choice(0, 2048, 2048, 640)[2] == 1 and E.gemm_choice(0, 2048, 2048, 1024)[2] == 2
+    assert E.gemm_choice(0, 128, 28672, 1280)[2] == 1 and E.gemm_choice(0, 129, 12288, 1280)[2] == 2

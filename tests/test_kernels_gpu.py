@@ -773,10 +773,10 @@ def test_gemm_planned_tiles_and_slices(M, N, K, tiled):
     assert float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
 
 
-@pytest.mark.parametrize("M,N,K,columns,slices", [(128, 528, 640, 128, 1), (128, 28672, 4096, 128, 1), (1011, 4096, 640, 128, 1),
-                                                  (385, 4112, 2048, 128, 1), (1011, 3088, 1408, 128, 1), (1010, 1040, 2176, 128, 3),
-                                                  (1011, 1040, 4224, 128, 3), (130, 24496, 2048, 192, 1), (1011, 6144, 4096, 192, 1),
-                                                  (300, 12208, 4224, 192, 1), (513, 4096, 4096, 192, 2), (700, 1296, 8192, 192, 6)])
+@pytest.mark.parametrize("M,N,K,columns,slices", [(1011, 4096, 1024, 128, 1), (128, 28672, 4096, 128, 1), (385, 4112, 2048, 128, 1),
+                                                  (1011, 3088, 1408, 128, 1), (1010, 1040, 3072, 128, 3), (1011, 1040, 4224, 128, 3),
+                                                  (1011, 784, 4224, 128, 4), (130, 24496, 2048, 192, 1), (1011, 6144, 4096, 192, 1),
+                                                  (300, 12208, 4224, 192, 1), (385, 1296, 14336, 192, 8), (700, 1296, 8192, 192, 6)])
 def test_gemm_of_two_wave_groups(M, N, K, columns, slices):
     """Two groups of waves that take the stages of K in turn, over the epilogues: odd and even numbers of k-groups, slices (of equal
     and unequal lengths), rows and columns past the last whole tile.  Every product here is asked whether it takes them: the tile of
