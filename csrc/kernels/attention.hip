@@ -663,4 +663,19 @@ extern "C" int vwa_flash_attention(const FlashAttnParams* p, hipStream_t st) {
 
 // chunk granularity of the decode grid (grid.y = ceil(max_ctx / this)); the split kernel's
 // 256-key chunks use every other grid row
+// Prefix chunks of a step over P shared keys whose groups' own keys (`own` of a row at most) are a chunk with a wave to each run; 0: a
+// chunk to each run
+extern "C" int vwa_decode_wave_runs(int D, int G, int nkv, int rows, int P, int own, int n_splits) {
+  const int RG = kMqCols / G, gr = (rows + RG - 1) / RG * nkv;
+  if (RG > kWaves || n_splits <= RG || P < 1 || rows < 1) return 0;
+  float best = 0.f;
+  int at = 0;
+  for (int c = 1; c < n_splits; ++c) {
+    const float cost = mq_cascade_keys(P, gr, c, 1, mq_run_keys(own, kWaves), kMqChunk, D);
+    if (!at || cost < best) best = cost, at = c;
+  }
+  const float apart = mq_cascade_keys(P, gr, mq_prefix_chunks(n_splits, RG, gr), RG, (own + kMqChunk - 1) / kMqChunk * kMqChunk, kMqChunk, D);
+  return best < kMqRunsAhead * apart ? at : 0;
+}
+
 extern "C" int vwa_attention_split_tokens() { return kMqChunk; }

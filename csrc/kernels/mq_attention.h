@@ -128,6 +128,33 @@ struct NoStamp {
   VWA_DEVICE void operator()(int) const {}
 };
 
+// What a cascade over P shared keys costs, in keys of the busiest CU: `pre` prefix chunks at most and n_own chunks of own_len keys for
+// each of `groups` (row group, kv head).  Chunks without keys end at once and are not counted.  (Counted, they made a few sessions'
+// own keys look dear -- 12 prefix chunks of 64 shared keys, one of which has any -- and a wave to each of them cheaper than it is: 2
+// sessions of 110 own keys 9.2 -> 11.4 us, 8 of them behind 1008 keys 11.7 -> 14.4.)
+inline __host__ __device__ float mq_cascade_keys(int P, int groups, int pre, int n_own, int own_len, int chunk, int D) {
+  auto over = [](int a, int b) {  // (a whole number that is met may come out a little above)
+#ifdef __HIP_DEVICE_COMPILE__
+    return (int)ceilf((float)a * __builtin_amdgcn_rcpf((float)b) - 1e-4f);
+#else
+    return (int)ceilf((float)a / (float)b - 1e-4f);
+#endif
+  };
+  const int len = over(P, pre * chunk) * chunk, n = over(P, len);
+  const int per_cu = (groups * (n + n_own) + kMqCus - 1) / kMqCus;
+  return (float)(per_cu * (len > own_len ? len : own_len) + (n + n_own) * 30 + (per_cu - 1) * (D == 64 ? 100 : 350));
+}
+// Prefix chunks where every run of a group has an own chunk (gh: row groups x kv heads)
+inline __host__ __device__ int mq_prefix_chunks(int n_splits, int RG, int gh) {
+  const int wide = kMqCus / gh - RG, half = kMqCus / 2 / gh, n = wide > half ? wide : half, most = n_splits - RG;
+  return n < 1 || most < 1 ? 1 : n < most ? n : most;
+}
+// Own keys of a run behind one wave of NW, as a chunk's
+inline __host__ __device__ int mq_run_keys(int own, int NW) { return (own + kMqStep - 1) / kMqStep * kMqStep * NW; }
+// The form with a wave to a run has to be ahead by this: its groups wait for their longest run (64 sessions of 450 .. 900 own keys at a
+// tie: 43.7 -> 48.4 us)
+constexpr float kMqRunsAhead = 0.95f;
+
 // Returns true when this workgroup had no item (after calling on_idle(), before any barrier).
 // FINE (the chained launch's attention phase): chunks are multiples of ONE 32-key step, the
 // steps of a chunk go to the waves round-robin, and the last arriver merges the chunks with two
@@ -263,25 +290,21 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     // one item per CU over prefix and own chunks, and prefix chunks for half of the CUs where the own
     // chunks alone take them all (they are short): 32 sessions x 8 kv heads of D = 128 behind 1008
     // shared keys (gh = 64) measured 24.4 / 18.7 / 21.1 us at 1 / 2 / 4 prefix chunks
-    n_pc = max(1, min(p.n_splits - RG, max(kMqCus / gh - RG, kMqCus / 2 / gh)));
+    n_pc = mq_prefix_chunks(p.n_splits, RG, gh);
     n_eff = n_pc + RG;
     if constexpr (RG <= NW) {
       // ... or the own keys of all of a group's runs in one chunk, a wave to a run: many sessions' own chunks do not fit the CUs
-      // once, but a run's keys lie behind one wave then.  The cheaper form by the other branch's count over the groups of real
-      // rows (the padded ones' items are short); lane c - 1: c prefix chunks.
+      // once, but a run's keys lie behind one wave then.  The cheaper form by mq_cascade_keys over the groups of real rows (the
+      // padded ones' items are short); lane c - 1: c prefix chunks.
       // Measured (us; 8 kv heads of D = 128, 992 shared keys): 32 sessions of ~110 own keys 18.2 -> 15.0 (384 items were two rounds of
       // the CUs, 256 are one, and the merge reads four partials instead of six), 48 of ~110 25.1 -> 20.0, 64 of ~100 27.1 -> 20.6,
       // 24 of ~150 19.7 -> 16.1; 32 of ~400 (kept as they were) 28.2 / 27.4.
       const int gr = (n_real + RG - 1) / RG * nkv;
       const int own = (int)wave_max(lane < n_real ? (float)max(cl - P, 0) : 0.f);
-      auto keys = [&](int pre, int n_own, int own_len) {
-        const int len = (int)ceilf((float)P * __builtin_amdgcn_rcpf((float)pre * kChunk)) * kChunk;
-        const int per_cu = (gr * (pre + n_own) + kMqCus - 1) / kMqCus;
-        return (float)(per_cu * max(len, own_len) + (pre + n_own) * 30 + (per_cu - 1) * (D == 64 ? 100 : 350));
-      };
-      const float cost = keys(min(lane + 1, p.n_splits - 1), 1, (own + kMqStep - 1) / kMqStep * kMqStep * NW);
+      auto keys = [&](int pre, int n_own, int own_len) { return mq_cascade_keys(P, gr, pre, n_own, own_len, kChunk, D); };
+      const float cost = keys(min(lane + 1, p.n_splits - 1), 1, mq_run_keys(own, NW));
       const float best = -wave_max(-cost);
-      wave_runs = best < keys(n_pc, RG, (own + kChunk - 1) / kChunk * kChunk);
+      wave_runs = best < kMqRunsAhead * keys(n_pc, RG, (own + kChunk - 1) / kChunk * kChunk);
       if (wave_runs) {
         n_pc = min(__builtin_ctzll(__ballot(cost == best)) + 1, p.n_splits - 1);
         n_eff = n_pc + 1;

@@ -321,6 +321,7 @@ int vwa_pcm16_to_f32(const int16_t* pcm, float* out, int n_in, int n_out, float 
 int vwa_log_mel(const float* audio, int n_samples, int n_frames, const float* window, const float* basis,
                 const float* fb_frag, int n_mels, float* mel_out, float* max_buf, uint16_t* out_bf16, int ld_out,
                 hipStream_t st);
+int vwa_decode_wave_runs(int D, int G, int nkv, int rows, int P, int own, int n_splits);
 int vwa_attention_split_tokens();
 int vwa_decode_advance(int* tokens, int* positions, int* ctx_lens, int64_t* slots, const int* sampled,
                        int* out, int* counter, int max_out, int base_block, int block_size, hipStream_t st);

@@ -1,0 +1,33 @@
+"""Which form a decoded step's launches take: rules on sizes alone, no launch."""
+import os
+
+import pytest
+
+from voice_enabled_browser_automation_amd.ops import build
+
+pytestmark = pytest.mark.skipif(not os.path.exists(build.KERNEL_SO), reason="the kernel library is not built")
+
+
+@pytest.fixture(scope="module")
+def E():
+    import torch  # noqa: F401  (the HIP runtime comes with it)
+
+    from voice_enabled_browser_automation_amd.ops import _vwa_kernels as E
+
+    return E
+
+
+@pytest.mark.parametrize("D,G,nkv", [(128, 4, 8), (128, 8, 2), (64, 4, 8)])
+@pytest.mark.parametrize("P", [16, 64, 256, 1008])
+def test_sessions_behind_a_prompt_share_a_chunk_where_it_is_ahead(E, D, G, nkv, P):
+    """A wave to a session's own keys: always for so few of them that one wave step holds them, never where every session's chunk has a
+    CU and more than a wave's steps of keys, nor for very long ones; its prefix chunks are some that the partials have room for."""
+    for rows in (1, 2, 4, 8, 12, 16, 24, 32, 48, 64):
+        forms = [E.decode_wave_runs(D, G, nkv, rows, P, own, 16) for own in (1, 32, 110, 300, 900)]
+        assert forms[0] and forms[1] and all(0 <= f < 16 for f in forms) and not forms[4]
+        groups = -(-rows // (16 // G)) * nkv
+        if groups * (-(-P // 128) + 16 // G) <= 256:
+            assert forms[2:] == [0, 0, 0]
+        assert E.decode_wave_runs(D, G, nkv, rows, P, 32, 16 // G) == 0  # (no room for another chunk)
+    assert E.decode_wave_runs(128, 4, 8, 32, P, 110, 16) and E.decode_wave_runs(128, 4, 8, 64, P, 300, 16)
+    assert E.decode_wave_runs(128, 1, 8, 32, P, 1, 16) == 0          # (more runs to a group than waves)
