@@ -404,6 +404,7 @@ void bind_mixers(py::module_& m) {
   m.def("rglru", &rglru, py::arg("yx"), py::arg("yb"), py::arg("xb"), py::arg("cw"), py::arg("cb"), py::arg("gw"), py::arg("rb"),
         py::arg("ib"), py::arg("decay"), py::arg("nb"), py::arg("seq_ids"), py::arg("positions"), py::arg("slots"), py::arg("state"),
         py::arg("out"), py::arg("chunks") = py::none(), py::arg("scratch") = py::none(), py::arg("u") = py::none(), py::arg("tickets") = py::none());
+  m.def("rglru_parts", [](int64_t bs, bool f32) { return vwa_rglru_parts((int)bs, f32); });
   m.def("head_linear", &head_linear, py::arg("x"), py::arg("xs"), py::arg("w"), py::arg("nb"), py::arg("N"), py::arg("K"), py::arg("y"),
         py::arg("ys"), py::arg("row_list") = py::none());
   m.def("latent_rows", &latent_rows);

@@ -131,6 +131,7 @@ struct MoeGemmParams {
 #ifdef __cplusplus
 extern "C" {
 #endif
+int vwa_rglru_parts(int bs, int f32);
 int vwa_rglru_rows(const RgLruParams* p, hipStream_t st);
 int vwa_rglru_scan(const RgLruParams* p, hipStream_t st);
 int vwa_head_linear(const HeadLinearParams* p, hipStream_t st);

@@ -219,12 +219,18 @@ VWA_DEVICE void save_inputs4(const RgLruParams& p, int r, int n, bool fresh, flo
 
 // ------------------------------------------------------------------------------------------ rows form
 // Workgroup (block, tile, part): the runs whose first row lies in rows 16 tile .. 16 tile + 15, 16 rows at a time to
-// their ends (other runs' rows count as inert); kRowTiles of the block's 16-channel tiles.  Every part forms the whole block's u,
+// their ends (other runs' rows count as inert); row_parts of the block's 16-channel tiles.  Every part forms the whole block's u,
 // so the inputs it is formed from are replaced by the last part that has read them (RgLruParams::tickets).
 // What bounds it is one CU drawing a block's gates (256 and 512 KB of 256 channels) behind a chain of round trips, on 4 - 16 CUs.
 // us with parts of all 16, 8, 4, 2 tiles, gates in L2: 32 bits, 4 rows x 4 blocks 16.1, 12.0, 10.6, 10.6; bf16, 16 rows x 8 11.2, 10.6,
 // 10.7, 11.0.  (The save by the waves without a tile, beside the products: 0.3 - 1 slower.)
-constexpr int kRowTiles = 4;
+// A part is worth its own forming of u and its ticket from 128 KB of gates on, and a wave to each of four tiles: of fewer, blocks of 80
+// and 128 channels were 9 - 18 % slower in 16 bits (4 rows of 128: 6.8 -> 7.7) and up to 4 % in 32, 10 blocks of 256 in 16 bits at 48 rows 10 %.
+constexpr int kPartBytes = 128 * 1024;
+int row_parts(int bs, int bytes) {
+  const int tiles = bs / 16, draw = 32 * bs * bytes, per = (kPartBytes + draw - 1) / draw;
+  return (tiles + (per > 4 ? per : 4) - 1) / (per > 4 ? per : 4);
+}
 
 template <class T>
 __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
@@ -489,8 +495,8 @@ size_t u_bytes(int rows, int bs) { return (size_t)rows * (bs * sizeof(T) + kPad)
 template <class T>
 int launch_rows(const RgLruParams& p, hipStream_t st) {
   if (u_bytes<T>(16, p.bs) > kMaxLds) return -10;
-  const int tiles = p.bs / 16, per = p.tickets ? kRowTiles : tiles;
-  const dim3 grid(p.nb, (p.rows + 15) / 16, (tiles + per - 1) / per), block(64 * (tiles < 16 ? tiles : 16));
+  const int tiles = p.bs / 16;
+  const dim3 grid(p.nb, (p.rows + 15) / 16, p.tickets ? row_parts(p.bs, sizeof(T)) : 1), block(64 * (tiles < 16 ? tiles : 16));
   hipLaunchKernelGGL((rglru_rows_kernel<T>), grid, block, u_bytes<T>(16, p.bs), st, p);
   return (int)hipGetLastError();
 }
@@ -514,6 +520,9 @@ int launch_scan(const RgLruParams& p, hipStream_t st) {
 }
 
 }  // namespace
+
+// Workgroups that a block's channels take in the rows form
+extern "C" int vwa_rglru_parts(int bs, int f32) { return bs < 16 || bs % 16 ? 0 : row_parts(bs, f32 ? 4 : 2); }
 
 extern "C" int vwa_rglru_rows(const RgLruParams* p, hipStream_t st) {
   const int rc = check(*p);

@@ -31,3 +31,16 @@ def test_sessions_behind_a_prompt_share_a_chunk_where_it_is_ahead(E, D, G, nkv, 
         assert E.decode_wave_runs(D, G, nkv, rows, P, 32, 16 // G) == 0  # (no room for another chunk)
     assert E.decode_wave_runs(128, 4, 8, 32, P, 110, 16) and E.decode_wave_runs(128, 4, 8, 64, P, 300, 16)
     assert E.decode_wave_runs(128, 1, 8, 32, P, 1, 16) == 0          # (more runs to a group than waves)
+
+
+def test_a_blocks_channels_are_split_by_the_bytes_of_their_gates(E):
+    """RG-LRU of decoded rows: parts of at least 128 KB of gates and four tiles; every part has some of the block's tiles."""
+    for f32, size in ((False, 2), (True, 4)):
+        for bs in range(16, 1025, 16):
+            tiles, n = bs // 16, E.rglru_parts(bs, f32)
+            per = -(-tiles // n)
+            assert n >= 1 and (n - 1) * per < tiles and (n == 1 or per >= 4)
+            assert n == 1 or -(-tiles // (n - 1)) * 32 * bs * size >= 128 * 1024
+    assert [E.rglru_parts(bs, False) for bs in (64, 80, 128, 256)] == [1, 1, 1, 2]
+    assert [E.rglru_parts(bs, True) for bs in (64, 80, 128, 256)] == [1, 1, 1, 4]
+    assert E.rglru_parts(768, True) == 12 and E.rglru_parts(8, True) == 0
