@@ -405,6 +405,7 @@ void bind_mixers(py::module_& m) {
         py::arg("ib"), py::arg("decay"), py::arg("nb"), py::arg("seq_ids"), py::arg("positions"), py::arg("slots"), py::arg("state"),
         py::arg("out"), py::arg("chunks") = py::none(), py::arg("scratch") = py::none(), py::arg("u") = py::none(), py::arg("tickets") = py::none());
   m.def("rglru_parts", [](int64_t bs, bool f32) { return vwa_rglru_parts((int)bs, f32); });
+  m.def("moe_ranks", [](int64_t E, int64_t top) { return vwa_moe_ranks((int)E, (int)top) != 0; });
   m.def("head_linear", &head_linear, py::arg("x"), py::arg("xs"), py::arg("w"), py::arg("nb"), py::arg("N"), py::arg("K"), py::arg("y"),
         py::arg("ys"), py::arg("row_list") = py::none());
   m.def("latent_rows", &latent_rows);

@@ -143,6 +143,7 @@ int vwa_latent_out(const LatentOutParams* p, hipStream_t st);
 int vwa_latent_prefill_fits(int dim_p, int rot_p, int vdk);
 int vwa_latent_gather(const LatentPrefillParams* p, hipStream_t st);
 int vwa_latent_prefill(const LatentPrefillParams* p, hipStream_t st);
+int vwa_moe_ranks(int E, int top);
 int vwa_moe_route(const MoeRouteParams* p, hipStream_t st);
 int vwa_moe_gemm(const MoeGemmParams* p, hipStream_t st);
 // x (f32 rows) += norm(sum of the row's n_parts branch rows) * w1; h (T) = norm(x) * w2 (w2 null: no h)

@@ -21,11 +21,14 @@ constexpr int kRouteWaves = 8, kRouteThreads = kRouteWaves * 64, kMaxExperts = 2
 // Experts whose places among a row's choices are counted: a lane each of the 32 that a row has.  The launch is bound by its serial
 // chain (loads, sums, choices, groups), and the choices one after another are top x 5 dependent exchanges of it.  us, chosen in turn ->
 // counted, top 4: bf16, K 2048, 16 rows of 16 experts 8.1 -> 6.5; K 1024, 48 rows 9.2 -> 7.5; 24 experts 10.5 -> 9.2; f32, K 1024,
-// 4 rows 7.5 -> 6.0.  Of more experts than lanes a lane would count several, and a maximum after another stays.
+// 4 rows 7.5 -> 6.0.  Of more experts than lanes a lane would count several, and a maximum after another stays; so it does where few are
+// chosen of many, since the count goes over all of them: one of 32 6.5 -> 7.0 (K 256, 1 row) and 24.7 -> 25.3, one of 16 the same.
 constexpr int kRankExperts = 32;
+bool ranks(int E, int top) { return E <= kRankExperts && E <= 16 * top; }
 // A score as it is ranked: one that is not a number is ahead of every other (they are <= 1) and its weight shows it, as torch.topk has it
 constexpr float kNoNumber = 2.f;
 VWA_DEVICE float rank_of(float score) { return score == score ? score : kNoNumber; }
+VWA_DEVICE float weight_of(float rank) { return rank == kNoNumber ? __builtin_nanf("") : rank; }
 
 // pairs -> tiles of one expert each (the whole workgroup); id_of(pair): its expert
 // (One wave that counts expert after expert from ballots, without LDS and barriers: 0.25 us an expert.)
@@ -80,7 +83,7 @@ VWA_DEVICE void group_pairs(const MoeRouteParams& p, F&& id_of) {
   for_pairs([&](int i, int e) { p.order[atomicAdd(&cnt[e], 1)] = i; });
 }
 
-template <class T>
+template <class T, bool COUNT>
 __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams p) {
   using M = MM<T>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -114,24 +117,24 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     float z = 0.f;
 #pragma unroll
     for (int k = 0; k < kRouteWaves; ++k) z += red[k * Ep * 16 + i];
-    sc[(i & 15) * (Ep + 1) + (i >> 4)] = (i >> 4) < p.E ? 1.f / (1.f + expf(-z)) : -2.f;
+    sc[(i & 15) * (Ep + 1) + (i >> 4)] = (i >> 4) < p.E ? rank_of(1.f / (1.f + expf(-z))) : -2.f;
   }
   int* lds_ids = reinterpret_cast<int*>(red);        // (a launch of one workgroup groups from here)
   __syncthreads();
   const int r = tid >> 5, q = tid & 31, row = r0 + r;  // 32 lanes per row: the choices stay inside a wave
-  if (p.E <= kRankExperts) {
+  if constexpr (COUNT) {
     // an expert's place is the number of experts ahead of it (a larger score; of equal ones the lower number): all choices at once
     // where one maximum after another is a chain of lane exchanges.
     const float* s = sc + r * (Ep + 1);
-    const float mine = s[min(q, p.E - 1)], v = rank_of(mine);
+    const float v = s[min(q, p.E - 1)];
     int place = q < p.E ? 0 : p.E;
 #pragma unroll 4
     for (int o = 0; o < p.E; ++o) {
-      const float u = rank_of(s[o]);
+      const float u = s[o];
       place += u > v || (u == v && o < q) ? 1 : 0;
     }
     if (place < p.top && r < nr) {
-      p.wts[row * p.top + place] = live ? mine : 0.f;
+      p.wts[row * p.top + place] = live ? weight_of(v) : 0.f;
       lds_ids[r * p.top + place] = live ? q : -1;
       __hip_atomic_store(p.ids + row * p.top + place, live ? q : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     float best = -3.f;
     int at = 0;
     for (int e = q; e < p.E; e += 32) {
-      const float v = rank_of(sc[r * (Ep + 1) + e]);
+      const float v = sc[r * (Ep + 1) + e];
       if (v > best) {
         best = v;
         at = e;
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     }
     if (q == 0 && r < nr) {
       sc[r * (Ep + 1) + at] = -1.f;                  // (taken; scores are positive)
-      p.wts[row * p.top + k] = live ? (best == kNoNumber ? __builtin_nanf("") : best) : 0.f;
+      p.wts[row * p.top + k] = live ? weight_of(best) : 0.f;
       lds_ids[r * p.top + k] = live ? at : -1;
       __hip_atomic_store(p.ids + row * p.top + k, live ? at : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -327,6 +330,9 @@ void launch_small(const MoeGemmParams& p, hipStream_t st) {
 
 }  // namespace
 
+// Whether a row's choices are counted into their places (else: one maximum after another)
+extern "C" int vwa_moe_ranks(int E, int top) { return ranks(E, top); }
+
 extern "C" int vwa_moe_route(const MoeRouteParams* p, hipStream_t st) {
   if (p->rows < 1 || p->E < 1 || p->E > kMaxExperts || p->top < 1 || p->top > p->E || p->K % 32 || p->ldh % 8 || p->tile < 1 ||
       !p->wts || !p->ids || !p->tiles || !p->order || !p->ticket)
@@ -338,8 +344,13 @@ extern "C" int vwa_moe_route(const MoeRouteParams* p, hipStream_t st) {
   const size_t lds = (size_t)kRouteWaves * Ep * 16 * 4 + 16 * (Ep + 1) * 4;
   if (lds > kMaxLds) return -10;
   const dim3 grid((p->rows + 15) / 16), block(kRouteThreads);
-  if (p->f32) hipLaunchKernelGGL((moe_route_kernel<float>), grid, block, lds, st, *p);
-  else hipLaunchKernelGGL((moe_route_kernel<u16>), grid, block, lds, st, *p);
+  if (ranks(p->E, p->top)) {
+    if (p->f32) hipLaunchKernelGGL((moe_route_kernel<float, true>), grid, block, lds, st, *p);
+    else hipLaunchKernelGGL((moe_route_kernel<u16, true>), grid, block, lds, st, *p);
+  } else {
+    if (p->f32) hipLaunchKernelGGL((moe_route_kernel<float, false>), grid, block, lds, st, *p);
+    else hipLaunchKernelGGL((moe_route_kernel<u16, false>), grid, block, lds, st, *p);
+  }
   return (int)hipGetLastError();
 }
 

@@ -44,3 +44,10 @@ def test_a_blocks_channels_are_split_by_the_bytes_of_their_gates(E):
     assert [E.rglru_parts(bs, False) for bs in (64, 80, 128, 256)] == [1, 1, 1, 2]
     assert [E.rglru_parts(bs, True) for bs in (64, 80, 128, 256)] == [1, 1, 1, 4]
     assert E.rglru_parts(768, True) == 12 and E.rglru_parts(8, True) == 0
+
+
+def test_places_are_counted_where_many_of_few_experts_are_chosen(E):
+    """Router: up to 32 experts, and 16 for every one chosen."""
+    for n in range(1, 257):
+        for top in range(1, min(n, 8) + 1):
+            assert E.moe_ranks(n, top) == (n <= 32 and n <= 16 * top)
