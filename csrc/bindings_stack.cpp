@@ -431,6 +431,7 @@ void bind_stack(py::module_& m) {
   m.def("qkv_cache", &qkv_cache);
   m.def("qkv_mingru", &qkv_mingru);
   m.def("talk_step", &talk_step);
+  m.def("talk_step_wgs", [](int64_t n, int64_t chunks) { return vwa_talk_step_wgs((int)n, (int)chunks); });
   m.def("talk_prefill_part", [](int64_t H, int64_t G, int64_t dk, int64_t dv) {
     return vwa_talk_prefill_part((int)H, (int)G, (int)dk, (int)dv);
   });

@@ -112,6 +112,7 @@ int vwa_talk_attention(const TalkAttnParams* p, hipStream_t st);
 // a decode step's qkv_mingru and rows-form attention (p->q unused) in the attention's two launches; <= 64 rows, those of a
 // sequence side by side at consecutive positions; rot_dims a multiple of 16 (not 0)
 int vwa_talk_step(const TalkAttnParams* p, const QkvCacheParams* qc, const MinGruParams* g, hipStream_t st);
+int vwa_talk_step_wgs(int n, int chunks);
 int vwa_talk_prefill(const TalkPrefillParams* p, hipStream_t st);
 // partial floats per (tile, split) of vwa_talk_prefill, < 0 if it does not take these sizes
 int64_t vwa_talk_prefill_part(int H, int G, int dk, int dv);

@@ -210,9 +210,16 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
 // took 6.6 and 10.7 (94 registers, and the table's row four times).  Bound by its round trips: ids and positions, table, keys.
 constexpr int kStepParts = 2;                        // workgroups of a row's keys and values
 // Scoring workgroups that a launch aims at: as many as are resident at once beside the others, in whole ones to a row, kv head and 16 of
-// its query heads, and at least one (64 rows of 16 kv heads: 1024; none waits for another).  They walk the row's chunks; one a chunk of
-// the longest context would be mostly workgroups without keys (48 rows of 2048: 3840, 11.1 -> 10.7 us).
-constexpr int kStepWgs = 768;
+// its query heads, but three of them at least, which share the row's chunks (64 rows of 16 kv heads: 3072; none waits for another).
+// One a chunk of the longest context would be mostly workgroups without keys: 48 rows of 2048 tokens' room and 90 .. 250 keys, 3840
+// workgroups 11.1 us, 768 10.7; 240 steps (1 .. 64 rows, 20 .. 2000 keys, six head shapes) against three launches: 0.93 of the time, and
+// 0.914 so.  With one a row and kv head where they are many, a row's chunks were one after another: 64 rows x 8 kv heads of 2000 keys 111 ->
+// 141 us, now 116 (16 bits: 64 rows and 1000 keys and more stay 2 - 8 % slower than three launches, and 3 - 14 % faster up to 225).
+constexpr int kStepWgs = 768, kStepLeast = 3;
+int step_wgs(int n, int chunks) {
+  const int per = kStepWgs / n > kStepLeast ? kStepWgs / n : kStepLeast;
+  return chunks < per ? chunks : per;
+}
 
 template <class T>
 __global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, QkvCacheParams qc, MinGruParams g, int per_row) {
@@ -1001,7 +1008,7 @@ int launch_rows(const TalkAttnParams& p, hipStream_t st, const QkvCacheParams* q
   if (lds > kMaxLds - 64) return -5;
   const int nz = (p.H / p.G + 15) / 16;
   if (qc) {
-    const int n = p.rows * p.G * nz, per_row = p.nst < kStepWgs / n ? p.nst : kStepWgs / n > 1 ? kStepWgs / n : 1;
+    const int n = p.rows * p.G * nz, per_row = step_wgs(n, p.nst);
     hipLaunchKernelGGL((talk_step_kernel<T>), dim3(p.rows * (kStepParts + (g->width + 255) / 256) + n * per_row), dim3(256), 0, st, p, *qc, *g, per_row);
   } else
     hipLaunchKernelGGL((talk_scores_kernel<T, GRP>), dim3(p.rows * p.G, p.nst, nz), dim3(256), 0, st, p);
@@ -1024,6 +1031,9 @@ extern "C" int vwa_talk_attention(const TalkAttnParams* p, hipStream_t st) {
   if (talk_chunk_tiles(p->H, 0) == 16) return p->f32 ? launch_rows<float, 16, false>(*p, st) : launch_rows<u16, 16, false>(*p, st);
   return p->f32 ? launch_rows<float, 8, false>(*p, st) : launch_rows<u16, 8, false>(*p, st);
 }
+
+// Scoring workgroups of a row, kv head and 16 query heads in vwa_talk_step, of n such and so many chunks of tiles
+extern "C" int vwa_talk_step_wgs(int n, int chunks) { return n < 1 || chunks < 1 ? 0 : step_wgs(n, chunks); }
 
 extern "C" int vwa_talk_step(const TalkAttnParams* p, const QkvCacheParams* qc, const MinGruParams* g, hipStream_t st) {
   const int rc = check_attn(*p);

@@ -51,3 +51,11 @@ def test_places_are_counted_where_many_of_few_experts_are_chosen(E):
     for n in range(1, 257):
         for top in range(1, min(n, 8) + 1):
             assert E.moe_ranks(n, top) == (n <= 32 and n <= 16 * top)
+
+
+def test_rows_of_talking_heads_share_their_chunks(E):
+    """Scores of a decoded step: a workgroup a chunk of few rows, some 768 of them of more, and three at least to a row's long context."""
+    for n in (1, 4, 48, 192, 256, 384, 512, 1024):
+        for chunks in (1, 2, 4, 17, 128):
+            per = E.talk_step_wgs(n, chunks)
+            assert min(chunks, 3) <= per <= chunks and (per <= 3 or n * per <= 768) and (per == chunks or n * (per + 1) > 768)
