@@ -293,7 +293,8 @@ using CfgP8 = Cfg<256, 256, 2, 4>;
 // slices before) 20.6 -> 15.2; 192 columns: 1011 x 6144 x 4096 62.8 -> 54.0, 130 x 12288 x 2048 29.4 -> 24.0.
 // Residuals and heads are stored by both groups, in turn, with a row's position and slot requested in front of the LDS round trip and
 // its rotation behind the sums: a product into rotated heads and cache, 1011 x 6144 x 4096, 69.5 -> 63.7 us, 600 rows 50.2 -> 47.0.
-// (Plain results: no difference.)
+// (Plain results: no difference.)  What leaves straight from the registers -- 32-bit results, slices -- is half of either group: by one
+// group, with 32-bit residuals, 2048 x 1024 x 2048 34.4 -> 28.2, 600 x 2048 x 1536 24.3 -> 20.6, and 1011 x 4096 x 6144 72.2 -> 65.3.
 // half-tile `which` (0 A-lo, 1 A-hi, 2 B-lo, 3 B-hi) into the stage image `st`: 16 wave-instructions of 1 KB, 2 per
 // wave, from the byte offsets voff (past the resource: zeros) + soff
 VWA_DEVICE void p8_issue(__amdgpu_buffer_rsrc_t r, const unsigned (&voff)[8], unsigned soff, int which, char* st) {
@@ -775,21 +776,35 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
     if (grp == 0) asm volatile("s_barrier" ::: "memory");  // (group 1 started one barrier later)
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
     f32x4* ex = reinterpret_cast<f32x4*>(lds) + w * FM * FN * 64 + l;
-    if (grp == 1) {
+    if (p.splits > 1 || p.y_f32) {  // stored from the registers: half of the rows by either group
 #pragma unroll
       for (int i = 0; i < FM; ++i)
+        if (i / (FM / 2) != grp)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) ex[(i * FN + j) * 64] = acc[i][j];
-    }
-    __syncthreads();
-    if (grp == 0) {
+          for (int j = 0; j < FN; ++j) ex[(i * FN + j) * 64] = acc[i][j];
+      __syncthreads();
 #pragma unroll
       for (int i = 0; i < FM; ++i)
+        if (i / (FM / 2) == grp)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] += ex[(i * FN + j) * 64];
+          for (int j = 0; j < FN; ++j) acc[i][j] += ex[(i * FN + j) * 64];
+    } else {
+      if (grp == 1) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) ex[(i * FN + j) * 64] = acc[i][j];
+      }
+      __syncthreads();
+      if (grp == 0) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] += ex[(i * FN + j) * 64];
+      }
+      __syncthreads();  // (the epilogue writes LDS again)
+      if (grp == 1 && !(kResid<EPI> || EPI == EPI_QKV)) return;  // (these store by both groups)
     }
-    __syncthreads();  // (the epilogue writes LDS again)
-    if (grp == 1 && (!(kResid<EPI> || EPI == EPI_QKV) || p.splits > 1 || p.y_f32)) return;  // (these store by both groups)
   } else {
   if (nh > 0) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0, lds, rows);
   if (nh > 1) issue_stage<C, WT, F8, W8, GRP, LINES>(p, rx, rw, bm, bn, h0 + 1, lds + STG, rows);
@@ -822,7 +837,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = row0 + i * 16 + r;
-        if (m >= p.M) continue;
+        if (m >= p.M || (C::GROUPS > 1 && i / (FM / 2) != grp)) continue;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           const int n = col0 + j * 16;
@@ -870,7 +885,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = row0 + i * 16 + r;
-        if (m >= p.M) continue;
+        if (m >= p.M || (C::GROUPS > 1 && i / (FM / 2) != grp)) continue;
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           const int n = col0 + j * 16;
@@ -1152,6 +1167,9 @@ bool takes_groups(const GemmParams& p, int epi, int n) {
 //   5 .. 7 they were 1.4 % slower, 1.14 times at worst), from 11 where one row block has the weight to itself (128 rows: 8 and 10 up to
 //   1.08 times).  192 columns in slices must be 5 % ahead by the estimate: taken at any lead, 29 of 70 such products were slower.  Of 728
 //   products with other tiles than without groups: 8.0 % less time on average, 12 are 2 - 4.5 % slower (profiles/gemm_tiles_ab.csv).
+//   A residual in 32 bits is added element by element behind whole tiles, 8 us on two groups and 14 on one, which the sum of slices does
+//   not pay: its product has the slices that it would have on one-group tiles (2048 x 1024 x 2048 whole 28.2 us, two slices 25.6 on one
+//   group).
 // W8A8 (k-groups of half the stages): fitted to 690 timings of 60 shapes (80 .. 6000 rows, 1024 .. 28672 columns, K 1280 ..
 // 14336), 11 % off; it picks the tile alone: slices in another order move a few bf16 activations by a bit, and every moved one
 // can flip its fp8 code further on, so they stay those of vwa_gemm_splits.  2720 x 4096 x 14336 224 -> 125 us, 2720 x 28672 x
@@ -1173,14 +1191,16 @@ float estimate(const GemmParams& p, bool p8, int s, int epi, int* tile = nullptr
   float us = rounds * (kg * per + (p8 ? 5.6f : 2.3f));
   if (!p8) {
     if (tile) *tile = CfgS::BN;
+    float least = us;
     for (const int n : {CfgK::BN, CfgKw::BN}) {
       if (!takes_groups(p, epi, n) || kg < (p.M <= CfgK::BM ? 11 : 8) || (int64_t)cdiv(p.M, CfgK::BM) * cdiv(p.N, n) * s > p.cus) continue;
       const float g = n == CfgK::BN ? kg * 0.99f + 3.6f : s == 1 ? kg * 1.18f + 5.f : 1.05f * (kg * 1.18f + 5.f) + 0.05f * sum;
-      if (g < us) {
-        us = g;
+      if (g < least) {
+        least = g;
         if (tile) *tile = n == CfgK::BN ? -CfgK::BN : CfgKw::BN;
       }
     }
+    if (p.y_f32 != 2 || s > 1) us = least;
   }
   return us + sum;
 }

@@ -128,3 +128,18 @@ def test_two_wave_groups_have_stages_to_share(E):
     assert seen == {(c, s) for c in (128, 192) for s in (False, True)}
     assert E.gemm_choice(0, 2048, 2048, 640)[2] == 1 and E.gemm_choice(0, 2048, 2048, 1024)[2] == 2
     assert E.gemm_choice(0, 128, 28672, 1280)[2] == 1 and E.gemm_choice(0, 129, 12288, 1280)[2] == 2
+
+
+def test_a_residual_in_32_bits_keeps_its_slices(E):
+    """Such a product has as many slices as on one-group tiles (which switching the groups' weights off shows), and two groups where
+    these take them; other 32-bit results are planned as 16-bit ones."""
+    grouped = 0
+    for M in (128, 600, 1011, 2048, 4096):
+        for N in (1024, 1280, 2048, 4096, 6144):
+            for K in (1024, 1536, 2048, 3840, 6144):
+                got, one = E.gemm_choice(1, M, N, K, y_f32=2), E.gemm_choice(1, M, N, K, w_tiled=False)
+                assert E.gemm_choice(0, M, N, K, y_f32=1) == E.gemm_choice(0, M, N, K)
+                whole = E.gemm_choice(1, M, N, K)
+                assert got[1] > 1 or one[1] == 1, (M, N, K, got, one)
+                grouped += got[2] == 2 and got != whole
+    assert grouped and E.gemm_choice(1, 2048, 1024, 2048)[1] == 1 and E.gemm_choice(1, 2048, 1024, 2048, y_f32=2)[1] == 2

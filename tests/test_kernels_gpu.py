@@ -796,6 +796,8 @@ def test_gemm_of_two_wave_groups(M, N, K, columns, slices):
     near = lambda got, y: float(((got.double() - y).abs() - 2.0 ** -8 * y.abs()).max()) < 1e-5
     y = exp + b.double()
     assert near(ops.linear(x, wt, b), y)
+    r32 = torch.randn(M, N, device=DEV)  # (a residual stream in 32 bits, in place)
+    assert float((ops.linear(x, wt, out=r32.clone(), residual=r32).double() - (exp + r32)).norm() / (exp + r32).norm()) < 2.0 ** -24 * K ** 0.5
     assert takes(3)[::2] == (columns, 2)
     assert near(ops.linear(x, wt, b, act="gelu"), y / 2 * torch.erfc(-y / 2 ** 0.5))
     assert takes(1)[::2] == (128, 2) if columns == 128 else takes(1)[0] != 192
