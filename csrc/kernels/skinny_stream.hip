@@ -20,18 +20,16 @@
 // XG variant (X does not fit in LDS: e.g. the down projection, K = 14336, with more than 5 rows):
 // the activation fragments are streamed from global memory alongside the weights (X is a few
 // hundred KB and stays L2-resident, so the extra loads hit L2, not HBM), with the same
-// two-register-set pipeline; only the reduction scratch lives in LDS.
+// two-register-set pipeline; LDS holds an item of each wave and the reduction scratch.
 #include "skinny_epilogue.h"
 
 namespace {
 
-// MT: 16-row MFMA row fragments per weight fragment (only MT = 1 is instantiated since round 5: the
-// 17..64-row form measured slower than the tiled GEMM and was removed).
-template <int EPI, int NT, int KS, bool XG, int MT = 1>
-__global__ __launch_bounds__(KS * 64) void skinny_stream_kernel(SkinnyParams p, int nb, int xstride, int xskew) {
-  // k-groups (128 wide) per item; MT > 1: one (the X fragments of MT row tiles share the
-  // register budget of the item's weights)
-  constexpr int U = MT > 1 ? 1 : XG ? 2 : 4 / NT;
+// U: k-groups (128 wide) of an item, and ONE: every workgroup has one item, whose loads are all it asks for (launch()).
+// Four waves: the registers that let as many workgroups share a CU as grid_of counts on.
+template <int EPI, int NT, int KS, bool XG, int U, bool ONE>
+__global__ __launch_bounds__(KS * 64, KS == 4 && EPI != EPI_QKV && !XG ? 3 : 1) void skinny_stream_kernel(
+    SkinnyParams p, int nb, int tiles, int more, int xstride, int xskew) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int M = p.M, K = p.K, N = p.N;
   u16* xs = reinterpret_cast<u16*>(smem);
@@ -39,13 +37,13 @@ __global__ __launch_bounds__(KS * 64) void skinny_stream_kernel(SkinnyParams p, 
   // one 16-B bank slot after row m; the extra 64-B skew every 4 rows (xskew 32) makes each
   // ds_read_b128 lane group ({0-3,12-15,20-27}, ...: rows nl, k-quarters g) hit 16 distinct slots
   // -- without it lanes (nl, g) and (nl + 4, g - 1)... share slots, a 2-way conflict on every read.
-  const int xbytes = XG ? 0 : ((M * xstride * 2) + 4 * xskew * 2 + 15) & ~15;
-  float* red = reinterpret_cast<float*>(smem + xbytes);  // [KS][NT][MT][4][64]
+  const int xbytes = XG ? KS * U * 4096 : ((M * xstride * 2) + 4 * xskew * 2 + 15) & ~15;
+  float* red = reinterpret_cast<float*>(smem + xbytes);  // [KS][NT][4][64]
   auto xrow = [&](int m) { return m * xstride + (m >> 2) * xskew; };
-  float* rs = red + KS * NT * MT * 4 * 64;                // [16 MT] row scales (1/rms, LayerNorm rstd)
-  float* mu = rs + 16 * MT;                               // [16 MT] row means (folded LayerNorm)
+  float* rs = red + KS * NT * 4 * 64;                     // [16] row scales (1/rms, LayerNorm rstd)
+  float* mu = rs + 16;                                    // [16] row means (folded LayerNorm)
   const float* mus = (p.fuse_rms == 2) ? mu : nullptr;
-  const int lane = VWA_TX & 63, w = VWA_TX >> 6;
+  const int lane = VWA_TX & 63, w = __builtin_amdgcn_readfirstlane(VWA_TX >> 6);
   const int nl = lane & 15, g = lane >> 4;
 
   EpiPre pre;
@@ -54,16 +52,14 @@ __global__ __launch_bounds__(KS * 64) void skinny_stream_kernel(SkinnyParams p, 
   const int gb = (G * w) / KS, ge = (G * (w + 1)) / KS;
   const __amdgpu_buffer_rsrc_t rw =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(p.W), (short)0, (int)((size_t)N * K * 2), 0x00020000);
-  // X fragments (XG): lane (row nl, k-quarter g); rows >= M read the zero OOB answer
   const __amdgpu_buffer_rsrc_t rx =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<u16*>(p.X), (short)0, (int)((size_t)M * p.ldx * 2), 0x00020000);
-  const int ntiles = N / (16 * NT);
-  const int my_tiles = (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int my_tiles = ONE ? 1 : tiles + ((int)blockIdx.x < more);  // (of `tiles`, and the first `more` workgroups one more)
   // grammar-masked LM head (p.col_mask; the launcher keeps it only for NT 1, EPI store, LDS-staged
   // X and <= 64 tiles per workgroup): this workgroup's tiles that hold an admissible token of some
   // row, compacted into lanes (lane k: the k-th live tile).  Measured on the intent grammar: 42 %
   // of the LM head's tiles live per decode step on average, 10 % at the median.
-  const bool masked = NT == 1 && !XG && p.col_mask != nullptr;
+  const bool masked = !ONE && NT == 1 && !XG && p.col_mask != nullptr;
   int n_live = my_tiles, live_tile = 0;
   if (masked) {
     const int tl = (int)blockIdx.x + lane * (int)gridDim.x;
@@ -76,144 +72,227 @@ __global__ __launch_bounds__(KS * 64) void skinny_stream_kernel(SkinnyParams p, 
     const int rank = __popcll(live & ((1ull << lane) - 1ull));
     const int dst = ((live >> lane) & 1ull) ? rank : n_live + (lane - rank);  // a permutation of the lanes
     live_tile = __builtin_amdgcn_ds_permute(dst * 4, tl);
+    if (n_live == 0) return;
   }
-  const int n_items = n_live * nb;
-  auto tile_of = [&](int it) { return masked ? __shfl(live_tile, it / nb, 64) : (int)blockIdx.x + (it / nb) * (int)gridDim.x; };
+  // items: (tile t of this workgroup, k-batch b), one after another
+  struct Item {
+    int t, b;
+  };
+  auto next = [&](Item i) { return ++i.b == nb ? Item{i.t + 1, 0} : i; };
+  auto tile_of = [&](Item i) { return masked ? __builtin_amdgcn_readlane(live_tile, i.t) : (int)blockIdx.x + i.t * (int)gridDim.x; };
 
-  auto load_x = [&](uint4 (&xr)[MT][U][4], int it) {
-    const int b = it % nb;
+  // Offsets: what the lanes differ in, and scalars (past the end: kOOB2, above every resource whatever is added).  One form for both
+  // weight layouts, without branches: behind a join the compiler waits for as many loads as the shorter way in has.
+  // XG: an item's X, 16 rows of U k-groups, is asked for 1 KB of rows at a time and turned to the fragments (lane (row nl, group g),
+  // substep s: k 32 g + 8 s of the k-group) through the wave's own piece of LDS.  Asked for as fragments, a load touched 64 pieces of
+  // 16 bytes 64 apart, four times the cycles of the address unit: 16 x 2048 x 8192 16.9 -> 11.9 us.  Chunk c of row r sits at slot
+  // c ^ ((r + 4) & 15) of its 16: rows and chunks of a ds_read_b128's lane groups ({0-3,12-15,20-27}, ..) meet in no slot.
+  constexpr int XC = 16 * U;  // 16-byte chunks of a row
+  char* const xw = smem + w * (XG ? 16 * XC * 16 : 0);
+  auto load_x = [&](uint4 (&xr)[U][4], Item i) {
+    const int kg = gb + i.b * U;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int j = 0; j < 4 * U; ++j) {
+      const int row = (j * 64 + lane) / XC, c = (j * 64 + lane) % XC;
+      const bool ok = i.t < n_live && row < M && kg + c / 16 < ge;
+      xr[j / 4][j % 4] = bload_w_so<0>(rx, ok ? (unsigned)row * (unsigned)p.ldx * 2u + 16u * c : kOOB2, i.t < n_live ? kg * 256 : 0);
+    }
+  };
+  auto turn_x = [&](const uint4 (&xr)[U][4]) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int kg = gb + b * U + u, row = 16 * mt + nl;
-        const bool ok = (it < n_items) && (kg < ge) && (row < M);
-        const unsigned base = ((unsigned)row * (unsigned)p.ldx + (unsigned)(kg * 128 + 32 * g)) * 2u;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) xr[mt][u][s] = bload(rx, ok ? base + 16u * s : kOOB);
-      }
+    for (int j = 0; j < 4 * U; ++j) {
+      const int row = (j * 64 + lane) / XC, c = (j * 64 + lane) % XC;
+      *reinterpret_cast<uint4*>(xw + (row * XC + (c ^ ((row + 4) & 15))) * 16) = xr[j / 4][j % 4];
+    }
+    asm volatile("" ::: "memory");  // (a wave's LDS operations keep their order)
   };
 
-  auto load_item = [&](uint4 (&wr)[NT][U][4], int it) {
-    const int tile = tile_of(it);
-    const int b = it % nb;
+  // pre-tiled: 1 KB contiguous per load instruction; row-major: 16 bytes of 64 pieces
+  const unsigned w_lane = p.w_tiled ? lane * 16u : ((unsigned)nl * (unsigned)K + 32u * g) * 2u;
+  const int w_kg = p.w_tiled ? 4096 : 256, w_s = p.w_tiled ? 1024 : 16;
+  auto load_item = [&](uint4 (&wr)[NT][U][4], Item i) {
+    const int tile = tile_of(i);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int kg = gb + b * U + u;
-      const bool ok = (it < n_items) && (kg < ge);
+      const int kg = gb + i.b * U + u;
+      const bool ok = i.t < n_live && kg < ge;
+      const unsigned voff = ok ? w_lane : kOOB2;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        if (p.w_tiled) {  // pre-tiled: 1 KB contiguous per load instruction
-          const unsigned T = (unsigned)(tile * NT + nt);
-          const unsigned base = ((T * (unsigned)G + (unsigned)kg) * 4u) * 1024u + (unsigned)lane * 16u;
+        const int at = ok ? (tile * NT + nt) * (32 * K) + kg * w_kg : 0;
 #pragma unroll
-          for (int s = 0; s < 4; ++s) wr[nt][u][s] = bload(rw, ok ? base + 1024u * s : kOOB);
-        } else {
-          const unsigned row = (unsigned)(tile * 16 * NT + nt * 16 + nl);
-          const unsigned base = (row * (unsigned)K + (unsigned)(kg * 128 + 32 * g)) * 2u;
-#pragma unroll
-          for (int s = 0; s < 4; ++s) wr[nt][u][s] = bload(rw, ok ? base + 16u * s : kOOB);
-        }
+        for (int s = 0; s < 4; ++s) wr[nt][u][s] = bload_w_so<0>(rw, voff, at + s * w_s);
       }
     }
   };
 
-  f32x4 acc[NT * MT];
+  f32x4 acc[NT];
 #pragma unroll
-  for (int k = 0; k < NT * MT; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < NT; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  auto compute_item = [&](const uint4 (&wr)[NT][U][4], const uint4 (&xr)[MT][U][4], int it) {
-    const int b = it % nb;
+  const int xrl = xrow(min(nl, M - 1));  // (rows past the last: any values, no row of the results depends on another)
+  auto compute_item = [&](const uint4 (&wr)[NT][U][4], const uint4 (&xr)[U][4], Item i) {
+    if constexpr (XG) turn_x(xr);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int kg = gb + b * U + u;
+      const int kg = gb + i.b * U + u;
       if (kg >= ge) break;  // wave-uniform
+      if constexpr (!ONE) __builtin_amdgcn_sched_barrier(0);  // (a k-group's fragments at a time: two items have the registers)
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
+        uint4 a;
+        if constexpr (XG) a = *reinterpret_cast<const uint4*>(xw + (nl * XC + 16 * u + ((4 * g + s) ^ ((nl + 4) & 15))) * 16);
+        else a = *reinterpret_cast<const uint4*>(xs + xrl + kg * 128 + 32 * g + 8 * s);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          uint4 a = make_uint4(0, 0, 0, 0);
-          if constexpr (XG) a = xr[mt][u][s];
-          else if (16 * mt + nl < M)
-            a = *reinterpret_cast<const uint4*>(xs + xrow(16 * mt + nl) + kg * 128 + 32 * g + 8 * s);
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt)
-            acc[nt * MT + mt] = mfma16(as_bf16x8(a), as_bf16x8(wr[nt][u][s]), acc[nt * MT + mt]);
-        }
+        for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma16(as_bf16x8(a), as_bf16x8(wr[nt][u][s]), acc[nt]);
       }
     }
+    if constexpr (XG) asm volatile("" ::: "memory");  // (the next item's rows take the place of these)
   };
 
-  auto finish_tile = [&](int it) {
-    tile_epilogue<EPI, NT, KS, false, MT>(p, red, rs, mus, tile_of(it), acc, w, lane, pre, !masked && it < nb);
+  auto finish = [&](Item i) {  // behind a tile's last batch
+    if (i.b == nb - 1)
+      tile_epilogue<EPI, NT, KS, false>(p, red, rs, mus, tile_of(i), acc, w, lane, pre, !masked && i.t == 0);
   };
 
   uint4 A[NT][U][4], B[NT][U][4];
-  uint4 XA[MT][U][4], XB[MT][U][4];  // XG only (dead otherwise)
-  // w_first: issue the first weight item before staging X (its round trip then overlaps the X
-  // staging + fused-RMSNorm statistics); otherwise stage X first (the X round trip is short).
-  if (p.w_first) {
-    load_item(A, 0);
-    if constexpr (XG) load_x(XA, 0);
-  }
-  // ---- stage X rows into LDS
-  const int k8 = K / 8;
-  if constexpr (!XG) {
-    for (int c = VWA_TX; c < M * k8; c += KS * 64) {
-      const int m = c / k8, kk = c % k8;
-      *reinterpret_cast<uint4*>(xs + xrow(m) + kk * 8) =
-          *reinterpret_cast<const uint4*>(p.X + (size_t)m * p.ldx + kk * 8);
-    }
-  }
-  lds_sync();
-  for (int m = w; m < 16 * MT; m += KS) {
-    float sc = 1.f, mean = 0.f;
-    if (p.fuse_rms && m < M) {
-      float s = 0.f, s1 = 0.f;
-      for (int kk = lane; kk < k8; kk += 64) {
-        float f[8];
-        unpack8(XG ? *reinterpret_cast<const uint4*>(p.X + (size_t)m * p.ldx + kk * 8)
-                   : *reinterpret_cast<const uint4*>(xs + xrow(m) + kk * 8), f);
+  uint4 XA[U][4], XB[U][4];  // XG only (dead otherwise)
+  // ---- X rows into LDS, in batches of PB 16-byte pieces a thread whose loads are all on the way, the first batch in front of the
+  // first weight item and the others behind it.  (Piece by piece each store waited for its own load and, vmcnt being in order, the
+  // first one for the weights too: a chain of M K / 8 / threads round trips in front of any product.)
+  constexpr int T = KS * 64, PB = KS == 4 ? 4 : 8;  // (four waves: three workgroups share a CU's registers)
+  const int k8 = K / 8, pieces = M * k8;
+  // (quotients below 2^14 by a float reciprocal: half a k8-th away from the next integer, 4e-6 off)
+  const float rk8 = __builtin_amdgcn_rcpf((float)k8);
+  const int dm = (int)((T + 0.5f) * rk8), dk = T - dm * k8;
+  int xm = (int)(((float)VWA_TX + 0.5f) * rk8), xk = VWA_TX - xm * k8;  // this thread's next piece
+  u32x4 px[PB];
+  auto walk = [&](int c0, auto&& f) {
+    int m = xm, kk = xk;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          s += f[j] * f[j];
-          s1 += f[j];
-        }
-      }
-      s = wave_sum(s);
-      if (p.fuse_rms == 2) {  // LayerNorm: rstd from E[x^2] - mean^2
-        mean = wave_sum(s1) / (float)K;
-        sc = rsqrtf(fmaxf(s / (float)K - mean * mean, 0.f) + p.eps);
-      } else {
-        sc = rsqrtf(s / (float)K + p.eps);
+    for (int i = 0; i < PB; ++i) {
+      if (c0 + i * T < pieces) f(i, m, kk);
+      m += dm;
+      kk += dk;
+      if (kk >= k8) {
+        kk -= k8;
+        ++m;
       }
     }
-    if (lane == 0) {
-      rs[m] = sc;
-      mu[m] = mean;
+    return make_int2(m, kk);
+  };
+  auto load_pieces = [&](int c0) {
+    walk(c0, [&](int i, int m, int kk) {
+      px[i] = gld(reinterpret_cast<const u32x4*>(p.X + (size_t)min(m, M - 1) * p.ldx + kk * 8));
+    });
+  };
+  auto store_pieces = [&](int c0) {
+    const int2 at = walk(c0, [&](int i, int m, int kk) {
+      if (m < M) *reinterpret_cast<u32x4*>(xs + xrow(m) + kk * 8) = px[i];
+    });
+    xm = at.x;
+    xk = at.y;
+  };
+  Item load{0, 0};
+  if constexpr (!XG) load_pieces(0);
+  load_item(A, load);
+  if constexpr (XG) load_x(XA, load);
+  if constexpr (!XG) {
+    store_pieces(0);
+    for (int c0 = PB * T; c0 < pieces; c0 += PB * T) {
+      load_pieces(c0);
+      store_pieces(c0);
     }
-  }
-  lds_sync();
-
-  if (!p.w_first) {
-    load_item(A, 0);
-    if constexpr (XG) load_x(XA, 0);
   }
   // the next item into a register set is issued right after that set's compute, BEFORE the tile
   // epilogue, so two items stay in flight through every epilogue
-  load_item(B, 1);
-  if constexpr (XG) load_x(XB, 1);
-  for (int it = 0; it < n_items; it += 2) {
-    compute_item(A, XA, it);
-    load_item(A, it + 2);
-    if constexpr (XG) load_x(XA, it + 2);
-    if (it % nb == nb - 1) finish_tile(it);
-    if (it + 1 >= n_items) break;
-    compute_item(B, XB, it + 1);
-    load_item(B, it + 3);
-    if constexpr (XG) load_x(XB, it + 3);
-    if ((it + 1) % nb == nb - 1) finish_tile(it + 1);
+  auto load_next = [&](uint4 (&wr)[NT][U][4], uint4 (&xr)[U][4]) {
+    load = next(load);
+    load_item(wr, load);
+    if constexpr (XG) load_x(xr, load);
+  };
+  if constexpr (!ONE) load_next(B, XB);
+  if constexpr (!XG) lds_sync();
+  // row scales (read behind the barrier of the first tile's reduction): rows w, w + KS, .. (two at a time where registers are free)
+  constexpr int R = ONE ? 2 : 1;
+  if (!p.fuse_rms) {
+    if (VWA_TX < 16) rs[VWA_TX] = 1.f;
+  } else {
+    for (int m0 = w; m0 < M; m0 += R * KS) {
+      float s[R] = {}, s1[R] = {};
+      for (int k0 = lane; k0 < k8; k0 += 4 * 64) {
+        uint4 v[R][4];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int kk = k0 + 64 * u, m = min(m0 + r * KS, M - 1);
+            v[r][u] = make_uint4(0, 0, 0, 0);
+            if (kk < k8)
+              v[r][u] = XG ? *reinterpret_cast<const uint4*>(p.X + (size_t)m * p.ldx + kk * 8)
+                           : *reinterpret_cast<const uint4*>(xs + xrow(m) + kk * 8);
+          }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)  // (pieces past the row's end add zeros)
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            float f[8];
+            unpack8(v[r][u], f);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              s[r] += f[j] * f[j];
+              s1[r] += f[j];
+            }
+          }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        s[r] = wave_sum(s[r]);
+        float sc, mean = 0.f;
+        if (p.fuse_rms == 2) {  // LayerNorm: rstd from E[x^2] - mean^2
+          mean = wave_sum(s1[r]) / (float)K;
+          sc = rsqrtf(fmaxf(s[r] / (float)K - mean * mean, 0.f) + p.eps);
+        } else {
+          sc = rsqrtf(s[r] / (float)K + p.eps);
+        }
+        if (lane == 0 && m0 + r * KS < M) {
+          rs[m0 + r * KS] = sc;
+          mu[m0 + r * KS] = mean;
+        }
+      }
+    }
   }
+
+  if constexpr (ONE) {
+    compute_item(A, XA, Item{0, 0});
+    finish(Item{0, 0});
+    return;
+  }
+  // The last items ask for nothing further: loads past the end bring no data, but their addresses take the unit as long as any
+  const int n_items = n_live * nb;
+  Item at{0, 0};
+  int left = n_items;
+  for (; left > 3; left -= 2) {
+    compute_item(A, XA, at);
+    load_next(A, XA);
+    finish(at);
+    at = next(at);
+    compute_item(B, XB, at);
+    load_next(B, XB);
+    finish(at);
+    at = next(at);
+  }
+  compute_item(A, XA, at);
+  if (left == 3) load_next(A, XA);
+  finish(at);
+  if (left == 1) return;
+  at = next(at);
+  compute_item(B, XB, at);
+  finish(at);
+  if (left == 2) return;
+  at = next(at);
+  compute_item(A, XA, at);
+  finish(at);
 }
 
 int g_x_skew = 32;  // LDS X row skew (elements per 4 rows; 0: none -- A/B knob, vwa_skinny_set_x_skew)
@@ -230,15 +309,11 @@ int grid_of(int ntiles, int grid_cap, size_t lds) {
   return ntiles < grid_cap * per ? ntiles : grid_cap * per;
 }
 
-template <int EPI, int NT, int KS, bool XG, int MT = 1>
-int launch_v(const SkinnyParams& p, hipStream_t st, int grid_cap, size_t lds, int xstride) {
-  constexpr int U = MT > 1 ? 1 : XG ? 2 : 4 / NT;
-  const int G = p.K / 128;
-  const int per_wave = (G + KS - 1) / KS;
-  const int nb = (per_wave + U - 1) / U;
-  const int grid = grid_of<EPI, KS>(p.N / (16 * NT), grid_cap, lds);
-  hipLaunchKernelGGL((skinny_stream_kernel<EPI, NT, KS, XG, MT>), dim3(grid), dim3(KS * 64), lds, st, p, nb, xstride,
-                     XG ? 0 : g_x_skew);
+template <int EPI, int NT, int KS, bool XG, int U, bool ONE>
+int launch_v(const SkinnyParams& p, hipStream_t st, int grid, size_t lds, int xstride, int nb) {
+  const int ntiles = p.N / (16 * NT);
+  hipLaunchKernelGGL((skinny_stream_kernel<EPI, NT, KS, XG, U, ONE>), dim3(grid), dim3(KS * 64), lds, st, p, nb, ntiles / grid,
+                     ntiles % grid, xstride, XG ? 0 : g_x_skew);
   return 0;
 }
 
@@ -260,9 +335,28 @@ int launch(const SkinnyParams& p0, hipStream_t st, int grid_cap) {
     if (EPI != EPI_STORE || NT != 1 || !lds_x || (ntiles + grid - 1) / grid > 64 || p.col_mask_rows < 1)
       p.col_mask = nullptr;
   }
-  if (lds_x) return launch_v<EPI, NT, KS, false>(p, st, grid_cap, xbytes + red, xstride);
-  if ((size_t)p.M * p.ldx * 2 >= 0x7FFFFFF0ull) return -10;
-  return launch_v<EPI, NT, KS, true>(p, st, grid_cap, red, xstride);
+  constexpr int UX = 2 / NT;  // (XG)
+  const size_t lds = lds_x ? xbytes + red : KS * UX * 4096 + red;
+  const int ntiles = p.N / (16 * NT), grid = grid_of<EPI, KS>(ntiles, grid_cap, lds);
+  const int per_wave = (p.K / 128 + KS - 1) / KS;  // k-groups of a tile's K that a wave has at most
+  if (!lds_x) {
+    if ((size_t)p.M * p.ldx * 2 >= 0x7FFFFFF0ull) return -10;
+    return launch_v<EPI, NT, KS, true, UX, false>(p, st, grid, lds, xstride, (per_wave + UX - 1) / UX);
+  }
+  // One tile a workgroup whose k-groups a wave holds at once: the form without a second register set, of as many k-groups as there
+  // are.  (The general one asked for two further items past the end and for the k-groups up to four that a wave does not have, each
+  // as long in the address unit as a load that brings data.)  us in decoding, X staged piece by piece -> in batches -> with this form:
+  // 16 x 2048 x 2048 9.2 -> 7.8 -> 4.9, 8 x 1280 x 1280 7.6 -> 6.5 -> 4.8, 8 x 5120 x 1280 with folded LayerNorm 10.1 -> 9.8 -> 7.2; general
+  // form, its last items asking for none behind them: 16 x 16384 x 2048 (SwiGLU) 18.2 -> 15.7 -> 13.9.
+  constexpr int U = 4 / NT;
+  if (grid == ntiles && per_wave <= U && !p.col_mask) {
+    if (per_wave <= 2) return launch_v<EPI, NT, KS, false, 2, true>(p, st, grid, lds, xstride, 1);
+    if constexpr (U > 2) {
+      if (per_wave == 3) return launch_v<EPI, NT, KS, false, 3, true>(p, st, grid, lds, xstride, 1);
+      return launch_v<EPI, NT, KS, false, 4, true>(p, st, grid, lds, xstride, 1);
+    }
+  }
+  return launch_v<EPI, NT, KS, false, U, false>(p, st, grid, lds, xstride, (per_wave + U - 1) / U);
 }
 
 
@@ -273,7 +367,7 @@ int launch(const SkinnyParams& p0, hipStream_t st, int grid_cap) {
 // and both scales are applied in the epilogue.  Weight bytes per decode step are halved.
 // ------------------------------------------------------------------------------------------
 template <int EPI, int NT, int KS>
-__global__ __launch_bounds__(KS * 64) void skinny_fp8_kernel(SkinnyParams p, int nb, int xstride) {
+__global__ __launch_bounds__(KS * 64, KS == 4 && EPI != EPI_QKV ? 3 : 1) void skinny_fp8_kernel(SkinnyParams p, int nb, int xstride) {
   constexpr int U = 8 / NT;  // k-groups (128 wide) per item: 2 x b128 weight loads per k-group
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int M = p.M, K = p.K, N = p.N;
@@ -281,52 +375,12 @@ __global__ __launch_bounds__(KS * 64) void skinny_fp8_kernel(SkinnyParams p, int
   const int xbytes = ((M * xstride) + 15) & ~15;
   float* red = reinterpret_cast<float*>(smem + xbytes);  // [KS][NT][4][64]
   float* rs = red + KS * NT * 4 * 64;                     // [16] row scale (rms * x-quant scale)
-  float* inv = rs + 16;                                    // [16] 1 / x-quant scale
-  const int lane = VWA_TX & 63, w = VWA_TX >> 6;
+  const int lane = VWA_TX & 63, w = __builtin_amdgcn_readfirstlane(VWA_TX >> 6);
   const int nl = lane & 15, g = lane >> 4;
   const int k8 = K / 8;
 
   EpiPre pre;
   epi_values<EPI, NT>(p, blockIdx.x, VWA_TX, pre);  // first tile's epilogue operands, early
-  // ---- per-row statistics (sum of squares for the fused RMSNorm, amax for the fp8 scale)
-  for (int m = w; m < 16; m += KS) {
-    float sc = 1.f, iv = 1.f;
-    if (m < M) {
-      float ss = 0.f, am = 0.f;
-      for (int kk = lane; kk < k8; kk += 64) {
-        float f[8];
-        unpack8(*reinterpret_cast<const uint4*>(p.X + (size_t)m * p.ldx + kk * 8), f);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          ss += f[j] * f[j];
-          am = fmaxf(am, fabsf(f[j]));
-        }
-      }
-      ss = wave_sum(ss);
-      am = wave_max(am);
-      const float sx = am > 0.f ? am * (1.f / 448.f) : 1.f;
-      iv = 1.f / sx;
-      sc = (p.fuse_rms ? rsqrtf(ss / (float)K + p.eps) : 1.f) * sx;
-    }
-    if (lane == 0) {
-      rs[m] = sc;
-      inv[m] = iv;
-    }
-  }
-  lds_sync();
-  // ---- quantise X rows into LDS (e4m3, 8 values -> 8 bytes)
-  for (int c = VWA_TX; c < M * k8; c += KS * 64) {
-    const int m = c / k8, kk = c % k8;
-    float f[8];
-    unpack8(*reinterpret_cast<const uint4*>(p.X + (size_t)m * p.ldx + kk * 8), f);
-    const float iv = inv[m];
-    uint2 q;
-    q.x = cvt_pk_fp8(f[0] * iv, f[1] * iv) | (cvt_pk_fp8(f[2] * iv, f[3] * iv) << 16);
-    q.y = cvt_pk_fp8(f[4] * iv, f[5] * iv) | (cvt_pk_fp8(f[6] * iv, f[7] * iv) << 16);
-    *reinterpret_cast<uint2*>(xs + m * xstride + kk * 8) = q;
-  }
-  lds_sync();
-
   const int G = K / 128;
   const int gb = (G * w) / KS, ge = (G * (w + 1)) / KS;
   const __amdgpu_buffer_rsrc_t rw =
@@ -335,6 +389,10 @@ __global__ __launch_bounds__(KS * 64) void skinny_fp8_kernel(SkinnyParams p, int
   const int my_tiles = (ntiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x;
   const int n_items = my_tiles * nb;
 
+  // (offsets as in skinny_stream_kernel.  fp8 tiled layout (ops.tile_weight_fp8): the (16-row tile, k-group) block is 2 KB
+  // [s][lane][16 B], lane (nl, g) gets W[row][128 kg + 32 g + 16 s .. + 16), the same bytes as of row-major weights)
+  const unsigned w_lane = p.w_tiled ? lane * 16u : (unsigned)nl * (unsigned)K + 32u * g;
+  const int w_kg = p.w_tiled ? 2048 : 128, w_s = p.w_tiled ? 1024 : 16;
   auto load_item = [&](uint4 (&wr)[NT][U][2], int it) {
     const int tile = blockIdx.x + (it / nb) * gridDim.x;
     const int b = it % nb;
@@ -342,22 +400,12 @@ __global__ __launch_bounds__(KS * 64) void skinny_fp8_kernel(SkinnyParams p, int
     for (int u = 0; u < U; ++u) {
       const int kg = gb + b * U + u;
       const bool ok = (it < n_items) && (kg < ge);
+      const unsigned voff = ok ? w_lane : kOOB2;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        if (p.w_tiled) {
-          // fp8 tiled layout (ops.tile_weight_fp8): the (16-row tile, k-group) block is 2 KB
-          // [s][lane][16 B] -- each load instruction reads 1 KB contiguous, lane (nl, g) gets
-          // W[row][128 kg + 32 g + 16 s .. + 16), the same bytes as the row-major addressing below
-          const unsigned T = (unsigned)(tile * NT + nt);
-          const unsigned base = (T * (unsigned)G + (unsigned)kg) * 2048u + (unsigned)lane * 16u;
+        const int at = ok ? (tile * NT + nt) * (16 * K) + kg * w_kg : 0;
 #pragma unroll
-          for (int s = 0; s < 2; ++s) wr[nt][u][s] = bload(rw, ok ? base + 1024u * s : kOOB);
-        } else {
-          const unsigned row = (unsigned)(tile * 16 * NT + nt * 16 + nl);
-          const unsigned base = row * (unsigned)K + (unsigned)(kg * 128 + 32 * g);
-#pragma unroll
-          for (int s = 0; s < 2; ++s) wr[nt][u][s] = bload(rw, ok ? base + 16u * s : kOOB);
-        }
+        for (int s = 0; s < 2; ++s) wr[nt][u][s] = bload_w_so<0>(rw, voff, at + s * w_s);
       }
     }
   };
@@ -389,7 +437,62 @@ __global__ __launch_bounds__(KS * 64) void skinny_fp8_kernel(SkinnyParams p, int
   };
 
   uint4 A[NT][U][2], B[NT][U][2];
+  // ---- rows w, w + KS, .. of X are this wave's: statistics (sum of squares for the fused RMSNorm, amax for the fp8 scale), then
+  // e4m3 codes into LDS.  A row's first PB pieces a lane stay in registers in between, and the next row's are requested in front
+  // of them, the first weight item behind the first row's.
+  constexpr int PB = KS == 4 ? 4 : 8;  // (four waves: rows of less than 2048)
+  u32x4 row[PB], ahead[PB];
+  auto load_row = [&](u32x4 (&v)[PB], int m, int k0) {  // pieces past the row's end: zeros
+#pragma unroll
+    for (int u = 0; u < PB; ++u) {
+      const int kk = k0 + 64 * u + lane;
+      v[u] = u32x4{0, 0, 0, 0};
+      if (m < M && kk < k8) v[u] = gld(reinterpret_cast<const u32x4*>(p.X + (size_t)m * p.ldx + kk * 8));
+    }
+  };
+  load_row(ahead, w, 0);
   load_item(A, 0);
+  for (int m = w; m < 16; m += KS) {
+    float sc = 1.f;
+    if (m < M) {
+#pragma unroll
+      for (int u = 0; u < PB; ++u) row[u] = ahead[u];
+      load_row(ahead, m + KS, 0);
+      float ss = 0.f, am = 0.f;
+      for (int k0 = 0; k0 < k8; k0 += 64 * PB) {
+        if (k0) load_row(row, m, k0);
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+          float f[8];
+          unpack8(__builtin_bit_cast(uint4, row[u]), f);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            ss += f[j] * f[j];
+            am = fmaxf(am, fabsf(f[j]));
+          }
+        }
+      }
+      ss = wave_sum(ss);
+      am = wave_max(am);
+      const float sx = am > 0.f ? am * (1.f / 448.f) : 1.f, iv = 1.f / sx;
+      sc = (p.fuse_rms ? rsqrtf(ss / (float)K + p.eps) : 1.f) * sx;
+      for (int k0 = 0; k0 < k8; k0 += 64 * PB) {
+        if (k8 > 64 * PB) load_row(row, m, k0);
+#pragma unroll
+        for (int u = 0; u < PB; ++u) {
+          const int kk = k0 + 64 * u + lane;
+          float f[8];
+          unpack8(__builtin_bit_cast(uint4, row[u]), f);
+          uint2 q;
+          q.x = cvt_pk_fp8(f[0] * iv, f[1] * iv) | (cvt_pk_fp8(f[2] * iv, f[3] * iv) << 16);
+          q.y = cvt_pk_fp8(f[4] * iv, f[5] * iv) | (cvt_pk_fp8(f[6] * iv, f[7] * iv) << 16);
+          if (kk < k8) *reinterpret_cast<uint2*>(xs + m * xstride + kk * 8) = q;
+        }
+      }
+    }
+    if (lane == 0) rs[m] = sc;
+  }
+  lds_sync();
   for (int it = 0; it < n_items; it += 2) {
     load_item(B, it + 1);
     compute_item(A, it);

@@ -24,7 +24,6 @@ struct SkinnyParams {
   int block_size;
   int64_t cache_stride_block, cache_stride_head, cache_stride_tok;
   const float* w_scale;  // non-null: W is OCP fp8 e4m3 [N, K] bytes with per-row scales (W8A8 path)
-  int w_first;           // stream kernel: issue the first weight loads before staging X
   // fuse_rms == 2: LayerNorm folded into the GEMM (stream kernel, bf16 weights): W holds
   // W*gamma, bias holds b + W.beta, ln_c[n] = sum_k (W*gamma)[n][k]; the kernel computes each
   // row's mean/rstd from the staged X and applies y = rstd * (acc - mean * ln_c[n]) + bias

@@ -457,6 +457,29 @@ def test_skinny_stream_many_tiles_and_k_tail(skinny_mode):
         close(out, exp, 1e-2)
 
 
+@pytest.mark.parametrize("ks,groups", [(8, 8), (8, 16), (8, 17), (8, 32), (8, 33), (8, 64), (4, 3), (4, 10), (4, 12), (4, 15)])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 5, 8, 9])
+def test_skinny_stream_items(ks, groups, tiles):
+    """One item a workgroup (of two, three or four k-groups a wave), one to five of them on two workgroups, with and without a remainder of
+    k-groups, X in LDS (8192 values of 16 rows: beside the weights): rows and columns against 64 bits."""
+    N, K = 16 * tiles, 128 * groups
+    ops.ext().set_skinny_mode(1, 2, ks, 2)
+    ops.ext().set_small_gemm_bytes(0)
+    try:
+        for M in (1, 7, 16):
+            x, w, r = rnd(M, K), rnd(N, K, scale=K**-0.5), rnd(M, N)
+            exact = x.double() @ w.double().T + r.double()
+            # half a bf16 ulp of the result, and as many f32 roundings as a wave's sums and the waves' have behind one another
+            tol = 2.0**-8 * exact.abs() + (K // ks + ks) * 2.0**-24 * (x.double().abs() @ w.double().abs().T + r.double().abs())
+            for weight in (w, ops.TiledWeight(w)):
+                out = torch.empty(M, N, dtype=BF, device=DEV)
+                ops.linear(x, weight, out=out, residual=r)
+                assert ((out.double() - exact).abs() <= tol).all(), (M, type(weight))
+    finally:
+        ops.ext().set_skinny_mode(1, 256, 0, 2)
+        ops.ext().set_small_gemm_bytes(4 << 20)
+
+
 def test_sample_greedy_masked_and_gumbel():
     rows, V = 3, 128256
     logits = torch.randn(rows, V, device=DEV)
