@@ -172,6 +172,12 @@ VWA_DEVICE float wave_max(float v) {
 
 VWA_DEVICE int lane_id() { return threadIdx.x & 63; }
 
+// x / k of uniform 0 <= x < 2^21, 1 <= k: by a float reciprocal (x + 1/2 lies half a k-th from the next quotient, the product is off by
+// 2.7e-7 of itself).  The compiler's division is a chain of 25 operations, and a kernel of a few us starts with several.
+VWA_DEVICE int small_div(int x, int k) {
+  return __builtin_amdgcn_readfirstlane((int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)k)));
+}
+
 // The workitem id through an empty volatile asm: every use is a fresh value, so address math
 // derived from it cannot be hoisted out of an enclosing loop.  The chained decode kernels read
 // their thread ids through this (VWA_TX): in the multi-layer launch (chain_kernel MULTI) LICM

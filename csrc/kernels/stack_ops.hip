@@ -310,7 +310,8 @@ int check_qkv(const QkvCacheParams* p) {
          p->max_pos < 1 || p->block_size < 1;
 }
 bool qkv_vec(const QkvCacheParams* p) {
-  return (p->rot_dims / 2) % 8 == 0 && p->dk % 8 == 0 && p->ldq % 8 == 0 && p->ldx % 8 == 0;
+  return (p->rot_dims / 2) % 8 == 0 && p->dk % 8 == 0 && p->ldq % 8 == 0 && p->ldx % 8 == 0 &&
+         ((reinterpret_cast<uintptr_t>(p->x) | reinterpret_cast<uintptr_t>(p->rope)) & 15) == 0;  // (16-byte loads)
 }
 }  // namespace
 

@@ -25,6 +25,8 @@
 #include "stack_kernels.h"
 #include "stack_types.h"
 
+#include <type_traits>
+
 using namespace vwa;
 
 namespace {
@@ -61,9 +63,12 @@ VWA_DEVICE f32x4 ld_sc1_x4(__amdgpu_buffer_rsrc_t r, int off) {
 // once for all of them.  777 rows of a 32-bit prompt, 8 / 4 heads of 128: both launches 332 -> 86 us per layer.
 //
 // Few rows are bound by the dependent round trips through memory (about 0.8 us each), not by bytes: everything whose address
-// is known is requested first; scores are spread by a tile per wave (kTalkStat tiles a workgroup); and a mixing chunk holds CT
+// known is requested first; scores are spread by a tile per wave (kTalkStat tiles a workgroup); and a mixing chunk holds CT
 // = 16 tiles, so that contexts of up to 256 keys take no partial sums, tickets and merging.  1 row of 225 keys, 16 / 4 heads
 // of 128: scores 5.4 -> 4.8, mixing 9.9 -> 8.4 us; 48 rows of 90 .. 250 keys, 8 / 4 heads: 7.4 -> 6.7, 10.5 -> 8.2.
+// What is requested first has to be read off the assembly: a gate's sigmoid behind its load, a load in a branch, a scalar load behind
+// an early return each waited for everything in front of them, and a cache place a value tile made the values wait for one another.  With
+// those out, the heads' weights mixed in batches and divisions by reciprocals: mixing 8.3 -> 6.2 us (1 row), 8.05 -> 6.75 (48 rows).
 constexpr int kWaves = 8;                      // of the mixing
 // (CT, most tiles of a chunk: talk_chunk_tiles)
 
@@ -73,8 +78,8 @@ struct Chunks {
 // the visible tiles are dealt evenly to the fewest chunks; chunk c holds tiles c * per ..
 template <int CT>
 VWA_DEVICE Chunks chunks_of(int tiles) {
-  const int k = (tiles + CT - 1) / CT, per = (tiles + k - 1) / k;
-  return Chunks{per, (tiles + per - 1) / per};
+  const int k = (tiles + CT - 1) / CT, per = small_div(tiles + k - 1, k);
+  return Chunks{per, small_div(tiles + per - 1, per)};
 }
 
 struct Unit {
@@ -88,10 +93,15 @@ VWA_DEVICE Unit unit_of(const TalkAttnParams& p, int ri) {
   Unit u;
   u.row = GRP ? p.groups[2 * ri] : p.row_list ? p.row_list[ri] : ri;
   u.cnt = GRP ? p.groups[2 * ri + 1] : 1;
-  const int64_t slot = p.slots[u.row];  // (requested together)
-  u.pos = p.positions[u.row];
-  u.seq = p.seq_ids[u.row];
-  u.live = GRP || slot >= 0;
+  // (requested together, as vector loads: of scalar ones the compiler puts the last two behind the caller's return for inert rows)
+  int row = u.row;
+  asm volatile("" : "+v"(row));
+  const int64_t slot = p.slots[row];
+  const int pos = p.positions[row], seq = p.seq_ids[row];
+  asm volatile("" ::: "memory");
+  u.pos = __builtin_amdgcn_readfirstlane(pos);
+  u.seq = __builtin_amdgcn_readfirstlane(seq);
+  u.live = GRP || __builtin_amdgcn_readfirstlane((int)(slot >> 32)) >= 0;
   u.v = vis_tiles(u.pos, u.pos + u.cnt - 1, p.window, p.keep);
   u.v.n = min(u.v.n, p.nst * kTalkStat);  // (a position past the context that the scratch is sized for stays inside of it)
   return u;
@@ -207,7 +217,9 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
 // other key comes from the cache.  The first workgroups write the cache and run the recurrence.
 // us, both launches -> this one: 1 row of 225 keys, 16 / 4 heads of 128 and 2048 channels 9.4 -> 5.9; 48 rows of 90 .. 250 keys, 8 / 4
 // heads and 1024 channels 10.9 -> 8.6.  The row's query and own key are turned once a workgroup, through LDS: every wave for itself
-// took 6.6 and 10.7 (94 registers, and the table's row four times).  Bound by its round trips: ids and positions, table, keys.
+// took 6.6 and 10.7 (94 registers, and the table's row four times).  Bound by its round trips: ids with the row's own projections, the
+// tile's place with the table's row, keys.  (The keys used to be requested behind the turned query: 5.9 -> 4.8 and 8.6 -> 7.5 us, with
+// the cache's and the recurrence's workgroups down to three trips.)
 constexpr int kStepParts = 2;                        // workgroups of a row's keys and values
 // Scoring workgroups that a launch aims at: as many as are resident at once beside the others, in whole ones to a row, kv head and 16 of
 // its query heads, but three of them at least, which share the row's chunks (64 rows of 16 kv heads: 3072; none waits for another).
@@ -222,7 +234,7 @@ int step_wgs(int n, int chunks) {
 }
 
 template <class T>
-__global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, QkvCacheParams qc, MinGruParams g, int per_row) {
+__global__ __launch_bounds__(256, sizeof(T) == 2 ? 4 : 3) void talk_step_kernel(TalkAttnParams p, QkvCacheParams qc, MinGruParams g, int per_row) {
   using M = MM<T>;
   static_assert(kTalkStat == 4, "a tile per wave");
   constexpr int NB = kScoreStep<T>;
@@ -230,19 +242,38 @@ __global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, Qkv
   __shared__ uint4 qs[NB][64], ks[NB][4];            // the query's fragments; those of the row's own key
   const int parts = kStepParts + (g.width + 255) / 256, n_parts = parts * p.rows;
   if ((int)blockIdx.x < n_parts) {
-    const int row = blockIdx.x / parts, part = blockIdx.x % parts;
+    const int row = small_div(blockIdx.x, parts), part = blockIdx.x - row * parts;
     if (part < kStepParts) qkv_cache_row<T, 8>(qc, row, part, kStepParts, p.H);
     else mingru_row<T>(g, row, (part - kStepParts) * 256 + threadIdx.x);
     return;
   }
-  const int R = p.H / p.G, nz = (R + 15) / 16, bid = blockIdx.x - n_parts;
-  const int rg = bid % (p.rows * p.G), cz = bid / (p.rows * p.G);
-  const int ri = rg / p.G, c = rg % p.G, r0 = cz % nz * 16;
+  const int R = small_div(p.H, p.G), nz = (R + 15) / 16, bid = blockIdx.x - n_parts;
+  const int cz = small_div(bid, p.rows * p.G), rg = bid - cz * (p.rows * p.G);
+  const int ri = small_div(rg, p.G), c = rg - ri * p.G, chunk0 = small_div(cz, nz), r0 = (cz - chunk0 * nz) * 16;
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, b = lane >> 4;
   // the step's rows, one a lane: this row's place, and the first row of its run (rows of one sequence, at consecutive positions)
   const int lr = min(lane, p.rows - 1);
   const int64_t slot_l = p.slots[lr];
   const int pos_l = p.positions[lr], seq_l = p.seq_ids[lr];
+  // requested with them: this wave's fragments of the query and of the row's own key, with their partners
+  constexpr int SN = (NB + 3) / 4;
+  const int Rb = min(16, R - r0), e0 = b * M::EPL;
+  const T* x = reinterpret_cast<const T*>(qc.x);
+  const T* xq = x + (size_t)ri * qc.ldx + (size_t)(c * R + r0 + min(rl, Rb - 1)) * p.dk;
+  const T* xk = x + (size_t)ri * qc.ldx + (size_t)(p.H + c) * p.dk;
+  uint4 fq[SN][2], fk[SN][2];
+  auto load_own = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < SN; ++i) {
+      const int e = min(k0 + (w + 4 * i) * M::KS, p.dk - M::KS) + e0, pe = turn_of(e, qc.rot_dims).pe;
+      fq[i][0] = *reinterpret_cast<const uint4*>(xq + e);
+      fq[i][1] = *reinterpret_cast<const uint4*>(xq + pe);
+      fk[i][0] = *reinterpret_cast<const uint4*>(xk + e);
+      fk[i][1] = *reinterpret_cast<const uint4*>(xk + pe);
+    }
+  };
+  load_own(0);
+  asm volatile("" ::: "memory");  // (not behind the wait for the ids)
   const int before = __shfl_up(seq_l, 1, 64), inert = __shfl_up((int)(slot_l < 0), 1, 64);
   const unsigned long long heads = __ballot(lane == 0 || before != seq_l || inert);
   if (!((__ballot(slot_l >= 0) >> ri) & 1)) return;
@@ -257,34 +288,38 @@ __global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, Qkv
   un.v.n = min(un.v.n, p.nst * kTalkStat);
   const Vis v = un.v;
   const int fresh = __builtin_amdgcn_readlane(pos_l, head);  // keys fresh .. un.pos are rows head .. ri
-  const int Rb = min(16, R - r0);
-  const T* x = reinterpret_cast<const T*>(qc.x);
-  const T* xq = x + (size_t)ri * qc.ldx + (size_t)(c * R + r0 + min(rl, Rb - 1)) * p.dk;
-  const T* xk = x + (size_t)ri * qc.ldx + (size_t)(p.H + c) * p.dk;
   auto table_row = [&](int pos) { return qc.rope + (size_t)min(max(pos, 0), qc.max_pos - 1) * qc.rot_dims; };
   const float* cq = table_row(un.pos);
   const int lb = __builtin_ctz(p.block_size);
-  const int e0 = b * M::EPL;
-  bool have_q = false;
-  for (int chunk = cz / nz; chunk * kTalkStat < v.n; chunk += per_row) {
+  // the scores of one chunk; First: this workgroup's first, for which the fragments asked for above are turned
+  auto chunk_scores = [&](auto First, int chunk) {
+    constexpr bool first = decltype(First)::value;
     const int t = chunk * kTalkStat + w;
     const bool ok[1] = {t < v.n};
     const int key0[1] = {tile_of(v, ok[0] ? t : v.n - 1) * kTile}, key = key0[0] + rl;
-    const int64_t blk = p.block_table[(int64_t)un.seq * p.table_stride + (key0[0] >> lb)];
+    const int blk = p.block_table[(int64_t)un.seq * p.table_stride + (key0[0] >> lb)];
     f32x4 acc[1] = {};
-    for (int k0 = 0; k0 < p.dk; k0 += NB * M::KS) {
-      const bool new_q = !have_q || p.dk > NB * M::KS;
-      if (have_q && new_q) lds_sync();                   // (the fragments before are read)
-      if (new_q) {
-#pragma unroll 1
-        for (int s = w; s < NB && k0 + s * M::KS < p.dk; s += 4) {
-          const uint4 fq = turned_frag(xq, k0 + s * M::KS + e0, qc.rot_dims, cq);
-          const uint4 fk = turned_frag(xk, k0 + s * M::KS + e0, qc.rot_dims, cq);
-          qs[s][lane] = fq;
-          ks[s][b] = fk;                                 // (the same of 16 lanes)
-        }
+    auto part = [&](auto Own, int k0) {                  // Own: with the query and the own key in LDS (dimensions k0 ..)
+      Turns<T> turns[SN];
+      if constexpr (decltype(Own)::value) {
+#pragma unroll
+        for (int i = 0; i < SN; ++i) load_turns<T>(turns[i], turn_of(min(k0 + (w + 4 * i) * M::KS, p.dk - M::KS) + e0, qc.rot_dims), cq);
+        asm volatile("" ::: "memory");                   // (not behind the wait for the tile's place)
       }
-      const T* kp = reinterpret_cast<const T*>(p.k) + blk * p.k_sb + (int64_t)c * p.k_sh +
+      auto turn_own = [&]() {
+        if constexpr (decltype(Own)::value) {
+#pragma unroll
+          for (int i = 0; i < SN; ++i) {
+            const int s = w + 4 * i;
+            if (s >= NB || k0 + s * M::KS >= p.dk) break;
+            const Turn u = turn_of(k0 + s * M::KS + e0, qc.rot_dims);
+            qs[s][lane] = turn_frag<T>(u, fq[i][0], fq[i][1], turns[i]);
+            ks[s][b] = turn_frag<T>(u, fk[i][0], fk[i][1], turns[i]);  // (the same of 16 lanes)
+          }
+          lds_sync();
+        }
+      };
+      const T* kp = reinterpret_cast<const T*>(p.k) + (int64_t)blk * p.k_sb + (int64_t)c * p.k_sh +
                     (int64_t)((key0[0] & (p.block_size - 1)) + rl) * p.dk + e0;
       auto product = [&](const uint4& cached, int s) {
         const uint4 own = ks[s][b];
@@ -294,7 +329,7 @@ __global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, Qkv
         uint4 kf[NB];
 #pragma unroll
         for (int s = 0; s < NB; ++s) kf[s] = *reinterpret_cast<const uint4*>(kp + min(k0 + s * M::KS, p.dk - M::KS));
-        if (new_q) lds_sync();
+        turn_own();
 #pragma unroll
         for (int s = 0; s < NB; ++s)
           if (k0 + s * M::KS < p.dk) product(kf[s], s);
@@ -302,25 +337,38 @@ __global__ __launch_bounds__(256, 5) void talk_step_kernel(TalkAttnParams p, Qkv
         const bool mine = key >= fresh && key < un.pos;  // (keys past the row's are masked)
         const T* xr = x + (size_t)(mine ? head + key - fresh : ri) * qc.ldx + (size_t)(p.H + c) * p.dk;
         const float* ck = table_row(mine ? key : un.pos);
-        if (new_q) lds_sync();
+        turn_own();
 #pragma unroll 1
         for (int s = 0; s < NB && k0 + s * M::KS < p.dk; ++s) {
           const uint4 old = *reinterpret_cast<const uint4*>(kp + k0 + s * M::KS), now = turned_frag(xr, k0 + s * M::KS + e0, qc.rot_dims, ck);
           product(mine ? now : old, s);
         }
       }
-      have_q = true;
+    };
+    if constexpr (first) part(std::true_type{}, 0);
+    for (int k0 = first ? NB * M::KS : 0; k0 < p.dk; k0 += NB * M::KS) {
+      if (p.dk <= NB * M::KS) {                          // (as the first chunk left them)
+        part(std::false_type{}, k0);
+      } else {
+        lds_sync();                                      // (the fragments before are read)
+        load_own(k0);
+        part(std::true_type{}, k0);
+      }
     }
     store_scores<false, 1>(p, un, ri, 0, c * R + r0 + rl, rl < Rb, chunk, key0, ok, acc, sm);
-    if ((chunk + per_row) * kTalkStat < v.n) lds_sync();  // (the statistics' LDS is written again)
+  };
+  int chunk = chunk0;
+  if (chunk * kTalkStat >= v.n) return;
+  chunk_scores(std::true_type{}, chunk);
+  for (chunk += per_row; chunk * kTalkStat < v.n; chunk += per_row) {
+    lds_sync();                                          // (the statistics' LDS is written again)
+    chunk_scores(std::false_type{}, chunk);
   }
 }
 
+VWA_DEVICE float gate_of(const TalkAttnParams& p, float g) { return p.gate ? p.out_scale / (1.f + __expf(-g)) : p.out_scale; }
 template <class T>
-VWA_DEVICE float head_gate(const TalkAttnParams& p, int row, int h) {
-  if (!p.gate) return p.out_scale;
-  return p.out_scale / (1.f + __expf(-ldv(reinterpret_cast<const T*>(p.gate) + (size_t)row * p.ldg + h)));
-}
+VWA_DEVICE const T* gate_at(const TalkAttnParams& p, int row, int h) { return reinterpret_cast<const T*>(p.gate) + (size_t)row * p.ldg + h; }
 
 // LDS: mixed weights [keys / KS][64][16 B], weights [rows of the unit x heads][keys] f32, statistics [rows x heads][2]
 template <class T, int CT>
@@ -337,9 +385,12 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
   static_assert(CH % 64 == 0 && HP >= 1);
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int s_last;
-  const int ri = blockIdx.x / p.G, c = blockIdx.x % p.G, chunk = blockIdx.y, r0 = blockIdx.z * 16;
+  const int ri = blockIdx.x / (unsigned)p.G, c = blockIdx.x - ri * p.G, chunk = blockIdx.y, r0 = blockIdx.z * 16;
+  // (all of the parameters in one round trip)
+  asm volatile("" ::"s"(p.window), "s"(p.keep), "s"(p.nst), "s"(p.nch), "s"(p.talk), "s"(p.gate), "s"(p.q), "s"(p.v), "s"(p.v_sb), "s"(p.v_sh),
+               "s"(p.block_table), "s"(p.table_stride), "s"(p.block_size), "s"(p.s), "s"(p.stat), "s"(p.dv), "s"(p.out), "s"(p.ldo), "s"(p.nq));
   const Unit un = unit_of<GRP>(p, ri);
-  const int R = p.H / p.G, Rb = min(16, R - r0), h0 = c * R + r0;
+  const int R = small_div(p.H, p.G), Rb = min(16, R - r0), h0 = c * R + r0;
   T* out = reinterpret_cast<T*>(p.out) + (size_t)un.row * p.ldo;
   if (!un.live) {
     if (chunk == 0)
@@ -358,18 +409,22 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
   float* hm = wt + nw * CH;                                             // [row][head] max
   float* hl = hm + nw;                                                  // [row][head] 1 / sum
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rl = lane & 15, b = lane >> 4;
-  // ---- everything that is read is requested first: the scores of this thread's (key; row, head)s, the first value tiles
-  // of this wave (16-column tiles w, w + 8, ...), the mixing rows of this wave's columns, the gates, the chunk statistics
+  // ---- everything that is read is requested first, and nothing of it is waited for until all of it is on its way: the cache places
+  // of the chunk's tiles (a lane each), the scores of this thread's (key; row, head)s, the mixing rows of this wave's columns, the gates,
+  // the chunk statistics, and behind the places the first value tiles of this wave (16-column tiles w, w + 8, ...)
+  const int lb = __builtin_ctz(p.block_size);
+  const int my_key = tile_of(v, t0 + min(lane & (CT - 1), nt - 1)) * kTile;
+  const int my_blk = p.block_table[(int64_t)un.seq * p.table_stride + (my_key >> lb)];
   constexpr int kPre = GRP ? 16 : 8;
   const int j = threadIdx.x & (CH - 1), hp = w / (CH / 64);             // key, first (row, head)
   const size_t srow = (size_t)ri * p.nq;
   const int64_t sld = (int64_t)p.nst * (kTalkStat * kTile);
-  const float* sbase = p.s + (srow * p.H + g0) * sld + t0 * kTile + j;
+  const float* sbase = p.s + (srow * p.H + g0) * sld + t0 * kTile + j;  // (keys past the chunk's: inside of the scratch, never used)
   auto head_of = [&](int i) { return GRP ? (i / hn) * p.H + i % hn : i; };  // (row, needed head) i from the unit's first
   auto score = [&](int i) -> const float* { return sbase + (int64_t)head_of(i) * sld; };
   float sv[kPre];
 #pragma unroll
-  for (int k = 0; k < kPre; ++k) sv[k] = j < nkey ? *score(min(hp + HP * k, nw - 1)) : 0.f;
+  for (int k = 0; k < kPre; ++k) sv[k] = *score(min(hp + HP * k, nw - 1));
   constexpr int kCols = 16 / HP;                                        // columns of a wave
   const bool in_lanes = p.talk && p.H <= 64;                            // lane g holds the weight of head g
   float tk[kCols];
@@ -382,83 +437,136 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
   const bool col = qi < un.cnt && r < Rb;
   // (an inert row of a group is zero whatever its query and its key hold)
   const bool on = !GRP || (col && p.slots[un.row + qi] >= 0);
-  float gate = 0.f;
-  if (nact == 1 && col && on) gate = head_gate<T>(p, un.row + qi, h0 + r);
+  const T gate_raw = *(p.gate ? gate_at<T>(p, un.row + min(qi, un.cnt - 1), h0 + min(r, Rb - 1)) : reinterpret_cast<const T*>(p.q));
+  auto stat = [&](int i, int k) { return *reinterpret_cast<const float2*>(p.stat + ((srow * p.H + g0 + head_of(i)) * p.nst + k) * 2); };
+  const int si = threadIdx.x >> 4, sk = threadIdx.x & 15;               // this thread's first statistics
+  const float2 stat0 = stat(min(si, nw - 1), min(sk, nstat - 1));
   constexpr int TPS = M::KS / kTile;                 // tiles per step (bf16 2, f32 1)
   constexpr int NST = CT / TPS;
-  const int lb = __builtin_ctz(p.block_size);
+  // place of the lane's tile (lanes past the chunk's tiles: of its last)
+  const int64_t my_place = (int64_t)my_blk * p.v_sb + (int64_t)c * p.v_sh + (my_key & (p.block_size - 1));
+  // (what has been asked for so far arrives with the places: behind the value loads, whose number depends on the chunk, the compiler
+  // would wait for all of them)
+  asm volatile("" ::"v"(stat0.x), "v"(stat0.y));
   const T* vb[NST];
-  bool vok[NST];
 #pragma unroll
   for (int s = 0; s < NST; ++s) {
-    const int lt = s * TPS + (TPS == 2 ? b >> 1 : 0);
-    vok[s] = lt < nt;
-    const int key = tile_of(v, vok[s] ? t0 + lt : v.n - 1) * kTile;
-    const int64_t blk = p.block_table[(int64_t)un.seq * p.table_stride + (key >> lb)];
-    vb[s] = reinterpret_cast<const T*>(p.v) + blk * p.v_sb + (int64_t)c * p.v_sh + (int64_t)rl * p.block_size +
-            (key & (p.block_size - 1)) + (TPS == 2 ? (b & 1) : b) * M::EPL;
+    auto part = [&](int v) {
+      const unsigned lo = __builtin_amdgcn_readlane(v, s * TPS), hi = __builtin_amdgcn_readlane(v, s * TPS + TPS - 1);
+      return TPS == 2 && b >> 1 ? hi : lo;
+    };
+    const unsigned lo = part((int)my_place), hi = part((int)(my_place >> 32));
+    vb[s] = reinterpret_cast<const T*>(p.v) + (int64_t)((uint64_t)hi << 32 | lo) + (int64_t)rl * p.block_size +
+            (TPS == 2 ? (b & 1) : b) * M::EPL;
   }
   uint4 va[NST];
   auto load_v = [&](int d) {
 #pragma unroll
     for (int s = 0; s < NST; ++s)
-      va[s] = vok[s] ? *reinterpret_cast<const uint4*>(vb[s] + (int64_t)min(d, p.dv - 16) * p.block_size) : make_uint4(0, 0, 0, 0);
+      if (s * TPS < nt) va[s] = *reinterpret_cast<const uint4*>(vb[s] + (int64_t)min(d, p.dv - 16) * p.block_size);
   };
   load_v(w * 16);
   // ---- statistics of every needed (row, head): 16 lanes each
-  for (int i = threadIdx.x >> 4; i < nw; i += NT / 16) {
-    const float* st = p.stat + (srow * p.H + g0 + head_of(i)) * p.nst * 2;
-    float m = -INFINITY, s = 0.f;
-    for (int k = threadIdx.x & 15; k < nstat; k += 16) {
-      const float2 ms = *reinterpret_cast<const float2*>(st + 2 * k);
-      const float mn = fmaxf(m, ms.x);
-      if (ms.y > 0.f) s = (s > 0.f ? s * __expf(m - mn) : 0.f) + ms.y * __expf(ms.x - mn);
-      m = mn;
-    }
-    auto merge = [&](float mo, float so) {
-      const float mn = fmaxf(m, mo);
-      s = (s > 0.f ? s * __expf(m - mn) : 0.f) + (so > 0.f ? so * __expf(mo - mn) : 0.f);
-      m = mn;
+  {
+    struct Stat {
+      float m, s;
     };
-    merge(row_ror<8>(m), row_ror<8>(s));
-    merge(row_ror<4>(m), row_ror<4>(s));
-    merge(row_ror<2>(m), row_ror<2>(s));
-    merge(row_ror<1>(m), row_ror<1>(s));
-    if ((threadIdx.x & 15) == 0) {
-      hm[i] = m;
-      hl[i] = 1.f / s;
+    auto add = [](Stat& a, float m, float s) {
+      const float mn = fmaxf(a.m, m);
+      if (s > 0.f) a.s = (a.s > 0.f ? a.s * __expf(a.m - mn) : 0.f) + s * __expf(m - mn);
+      a.m = mn;
+    };
+    auto merge = [](Stat& a, float mo, float so) {
+      const float mn = fmaxf(a.m, mo);
+      a.s = (a.s > 0.f ? a.s * __expf(a.m - mn) : 0.f) + (so > 0.f ? so * __expf(mo - mn) : 0.f);
+      a.m = mn;
+    };
+    auto finish = [&](Stat& a, int i) {
+      merge(a, row_ror<8>(a.m), row_ror<8>(a.s));
+      merge(a, row_ror<4>(a.m), row_ror<4>(a.s));
+      merge(a, row_ror<2>(a.m), row_ror<2>(a.s));
+      merge(a, row_ror<1>(a.m), row_ror<1>(a.s));
+      if (sk == 0) {
+        hm[i] = a.m;
+        hl[i] = 1.f / a.s;
+      }
+    };
+    Stat a{-INFINITY, 0.f};
+    if (sk < nstat) add(a, stat0.x, stat0.y);
+    for (int k = sk + 16; k < nstat; k += 16) {
+      const float2 ms = stat(min(si, nw - 1), k);
+      add(a, ms.x, ms.y);
+    }
+    if (si < nw) finish(a, si);
+    for (int i = si + NT / 16; i < nw; i += NT / 16) {
+      a = Stat{-INFINITY, 0.f};
+      for (int k = sk; k < nstat; k += 16) {
+        const float2 ms = stat(i, k);
+        add(a, ms.x, ms.y);
+      }
+      finish(a, i);
     }
   }
   lds_sync();
   // ---- normalised weights of the chunk's keys (0 past the last tile)
-  auto weight = [&](int i, float s) { wt[i * CH + j] = j < nkey && s != -INFINITY ? __expf(s - hm[i]) * hl[i] : 0.f; };
+  auto weight = [&](float s, float m, float l) {
+    const float e = __expf(s - m) * l;
+    return j < nkey && s != -INFINITY ? e : 0.f;
+  };
+  {
+    float mk[kPre], lk[kPre];
 #pragma unroll
-  for (int k = 0; k < kPre; ++k)
-    if (hp + HP * k < nw) weight(hp + HP * k, sv[k]);
+    for (int k = 0; k < kPre; ++k) {
+      mk[k] = hm[min(hp + HP * k, nw - 1)];
+      lk[k] = hl[min(hp + HP * k, nw - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < kPre; ++k)
+      if (hp + HP * k < nw) wt[(hp + HP * k) * CH + j] = weight(sv[k], mk[k], lk[k]);
+  }
 #pragma unroll 4
-  for (int i = hp + HP * kPre; i < nw; i += HP) weight(i, *score(i));
+  for (int i = hp + HP * kPre; i < nw; i += HP) wt[i * CH + j] = weight(*score(i), hm[i], hl[i]);
   lds_sync();
   // ---- mixed weights of this kv head's columns (row, query head)
   {
     const int idx = ((j / M::KS) * 64 + 16 * ((j % M::KS) / M::EPL)) * M::EPL + j % M::EPL;
+    // (the weights of eight heads are requested together, of one row for all of the wave's columns; a loop over the heads with the lane
+    // read in it is not unrolled: an LDS round trip a head, 1.3 us of 16 heads in two columns -> 0.9)
+    constexpr int GB = 8;
+    float x[kCols] = {};
+    if (in_lanes) {
+#pragma unroll
+      for (int i = 0; i < kCols; ++i) tk[i] = lane < p.H ? tk[i] : 0.f;
+      for (int gb = 0; gb < p.H; gb += GB) {         // (heads past the last: a weight of 0)
+        float wv[GB];
+        auto read = [&](int row) {
+#pragma unroll
+          for (int u = 0; u < GB; ++u) wv[u] = wt[(row * hn + min(gb + u, p.H - 1)) * CH + j];
+        };
+        if constexpr (!GRP) read(0);
+#pragma unroll
+        for (int i = 0; i < kCols; ++i) {
+          if (hp + HP * i >= ncol) break;              // (uniform per wave)
+          if constexpr (GRP) read((hp + HP * i) / Rb);
+#pragma unroll
+          for (int u = 0; u < GB; ++u)
+            x[i] += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tk[i]), gb + u)) * wv[u];
+        }
+      }
+    }
 #pragma unroll
     for (int i = 0; i < kCols; ++i) {
       const int cc = hp + HP * i, cr = GRP ? cc % Rb : cc;
       if (cc >= ncol) break;                         // (uniform per wave)
       const float* wr = wt + (GRP ? cc / Rb : 0) * hn * CH + j;
-      float x = 0.f;
-      if (in_lanes) {
-#pragma unroll 8
-        for (int g = 0; g < p.H; ++g)
-          x += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, tk[i]), g)) * wr[g * CH];
-      } else if (p.talk) {
+      if (!p.talk) {
+        x[i] = wr[cr * CH];
+      } else if (!in_lanes) {
         const float* t = p.talk + (size_t)(h0 + cr) * p.H;
 #pragma unroll 8
-        for (int g = 0; g < p.H; ++g) x += t[g] * wr[g * CH];
-      } else {
-        x = wr[cr * CH];
+        for (int g = 0; g < p.H; ++g) x[i] += t[g] * wr[g * CH];
       }
-      stv(pf + idx + cc * M::EPL, x);
+      stv(pf + idx + cc * M::EPL, x[i]);
     }
   }
   lds_sync();
@@ -466,11 +574,12 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
   const int nz = gridDim.z;
   float* prow = p.part + srow * p.nch * p.H * p.dv;
   const __amdgpu_buffer_rsrc_t rp = rsrc_f32(prow, (int64_t)p.nq * p.nch * p.H * p.dv);
+  const float gate = on ? gate_of(p, ldv(&gate_raw)) : 0.f;
   for (int d = w * 16; d < p.dv; d += 16 * kWaves) {
     f32x4 acc = {};
 #pragma unroll
     for (int s = 0; s < NST; ++s)
-      acc = M::mma(va[s], *reinterpret_cast<const uint4*>(pf + ((size_t)s * 64 + lane) * M::EPL), acc);
+      if (s * TPS < nt) acc = M::mma(va[s], *reinterpret_cast<const uint4*>(pf + ((size_t)s * 64 + lane) * M::EPL), acc);
     if (d + 16 * kWaves < p.dv) load_v(d + 16 * kWaves);
     if (!col) continue;
     const int h = h0 + r;
@@ -511,7 +620,7 @@ __global__ __launch_bounds__(64 * kWaves) void talk_mix_kernel(TalkAttnParams p)
       stv(out + (size_t)k0 * p.ldo + o + 1, 0.f);
       continue;
     }
-    const float g = head_gate<T>(p, row, h0 + e / p.dv);
+    const float g = gate_of(p, p.gate ? ldv(gate_at<T>(p, row, h0 + e / p.dv)) : 0.f);
     stv(out + (size_t)k0 * p.ldo + o, a0 * g);
     stv(out + (size_t)k0 * p.ldo + o + 1, a1 * g);
   }
@@ -704,7 +813,7 @@ __global__ __launch_bounds__(kPW * 64) void talk_prefill_kernel(TalkPrefillParam
     const int h = u >> 4, q = u & 15;
     const int at = ((h / R) * RP + h % R) * 16 + q;
     lse[at] = pp.lse[(size_t)(row0 + min(q, nq - 1)) * p.H + h];
-    gate[at] = head_gate<u16>(p, row0 + min(q, nq - 1), h);
+    gate[at] = gate_of(p, p.gate ? ldv(gate_at<u16>(p, row0 + min(q, nq - 1), h)) : 0.f);
   }
   // (operand slots no head writes -- padding heads, blocks past 2 HT -- stay zero)
   for (int u = threadIdx.x; u < C::X_BYTES / 16; u += kPW * 64) reinterpret_cast<uint4*>(xm)[u] = make_uint4(0, 0, 0, 0);
