@@ -39,7 +39,7 @@ VWA_DEVICE void head_linear_wg(const HeadLinearParams& p, int b, int cg, int r0)
   for (int j = 0; j < kHlTiles; ++j)
     wp[j] = reinterpret_cast<const uint4*>(p.w) + ((size_t)b * nt + min(t0 + j, nt - 1)) * steps * 64 + lane;
   f32x4 acc[NT][kHlTiles] = {};
-  constexpr int U = NT == 1 ? 4 : 2;                 // steps whose loads are in flight together
+  constexpr int U = NT == 1 ? 128 / M::KS : 2;       // steps whose loads are in flight together (few rows: a head's 128 dimensions)
   for (int s0 = 0; s0 < steps; s0 += U) {
     uint4 a[U][NT], f[U][kHlTiles];
 #pragma unroll
@@ -50,6 +50,7 @@ VWA_DEVICE void head_linear_wg(const HeadLinearParams& p, int b, int cg, int r0)
 #pragma unroll
       for (int t = 0; t < NT; ++t) a[u][t] = *reinterpret_cast<const uint4*>(xp[t] + s * M::KS);
     }
+    asm volatile("" ::: "memory");                   // (the compiler would put each step's loads behind its condition, a round trip a step)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (s0 + u >= steps) break;
@@ -133,8 +134,8 @@ template <class T, int NT>
 __global__ __launch_bounds__(256) void latent_qkv_kernel(LatentRowsParams p, HeadLinearParams q, int n_lin) {
   if ((int)blockIdx.x < n_lin) {
     const int cgs = (q.N + kHlCols - 1) / kHlCols, per = q.nb * cgs;
-    const int u = blockIdx.x % per;
-    head_linear_wg<T, NT>(q, u / cgs, u % cgs, (blockIdx.x / per) * 16 * NT);
+    const int rg = n_lin == per ? 0 : blockIdx.x / (unsigned)per, u = blockIdx.x - rg * per, b = small_div(u, cgs);
+    head_linear_wg<T, NT>(q, b, u - b * cgs, rg * 16 * NT);
   } else {
     latent_row<T>(p, blockIdx.x - n_lin);
   }
@@ -153,13 +154,18 @@ struct Item {                                        // one workgroup's work
 // false: no key in the chunk (its statistics say so)
 VWA_DEVICE bool attn_item(const LatentAttnParams& p, Item& x) {
   const int hgs = (p.H + 15) / 16, chunk = blockIdx.y;
-  x.ri = blockIdx.x / hgs;
-  x.h0 = (blockIdx.x % hgs) * 16;
+  x.ri = hgs == 1 ? blockIdx.x : blockIdx.x / (unsigned)hgs;
+  x.h0 = (blockIdx.x - x.ri * hgs) * 16;
   x.row = p.row_list ? p.row_list[x.ri] : x.ri;
   x.Hb = min(16, p.H - x.h0);
-  x.pos = p.slots[x.row] >= 0 ? p.positions[x.row] : -1;
-  x.table = p.block_table + (int64_t)p.seq_ids[x.row] * p.table_stride;
-  const int nt = x.pos >= 0 ? x.pos / kKeys + 1 : 0, per = (nt + p.nch - 1) / p.nch;
+  int row = x.row;                                   // (the ids as vector loads, all three in one round trip)
+  asm volatile("" : "+v"(row));
+  const int64_t slot = p.slots[row];
+  const int pos = p.positions[row], seq = p.seq_ids[row];
+  asm volatile("" ::: "memory");
+  x.pos = __builtin_amdgcn_readfirstlane(slot >= 0 ? pos : -1);
+  x.table = p.block_table + (int64_t)__builtin_amdgcn_readfirstlane(seq) * p.table_stride;
+  const int nt = x.pos >= 0 ? x.pos / kKeys + 1 : 0, per = nt <= p.nch ? min(nt, 1) : (nt + p.nch - 1) / p.nch;
   x.t_beg = chunk * per;
   x.t_end = min(nt, x.t_beg + per);
   x.stat = p.stat + (((size_t)x.ri * p.nch + chunk) * p.H + x.h0) * 2;
@@ -327,14 +333,16 @@ __global__ __launch_bounds__(256, 2) void latent_attn_kernel(LatentAttnParams p)
 // in flight over the softmax.  4 rows x 8 heads x 140 keys, rank 512: 25.3 -> 13.9 us (144 + 128
 // MFMAs of a wave: 3.6); 64 rows x 1000 keys 161 -> 55.
 constexpr int kKeyPre = 12;
-template <int NT, bool EXACT>  // EXACT: rank_p = 64 NT, the columns at constant offsets of a key's first
+// EXACT: rank_p = 64 NT and rot_p 64: the columns at constant offsets of a key's first, and as many steps as there are known to the
+// compiler (a load behind a condition is waited for with everything behind it)
+template <int NT, bool EXACT>
 __global__ __launch_bounds__(256, EXACT && NT <= 8 ? 2 : 1) void latent_attn_f32_kernel(LatentAttnParams p) {
   using M = MM<float>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float s_max[2][4][16];
   Item x;
   if (!attn_item(p, x)) return;
-  const int dk = p.rank_p + p.rot_p, steps = dk / M::KS, tid = threadIdx.x;
+  const int dk = EXACT ? 64 * NT + 64 : p.rank_p + p.rot_p, steps = dk / M::KS, tid = threadIdx.x;
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6), rl = lane & 15, g = lane >> 4;
   char* pf = smem;                                   // [4][64][16 B]
   char* qf = smem + 4096;                            // [steps][64][16 B]
@@ -356,10 +364,16 @@ __global__ __launch_bounds__(256, EXACT && NT <= 8 ? 2 : 1) void latent_attn_f32
       for (int j = 0; j < 4; ++j) va[st][j] = key_row(key0 + 16 * st + 4 * g + j) + 16 * min(w, p.rank_p / 16 - 1) + rl;
   };
   rows_of(x.t_beg * kKeys);
-  for (int i = tid; i < steps * 64; i += 256) {
-    const int s = i >> 6, ln = i & 63;
-    const float* q = reinterpret_cast<const float*>(p.q) + (size_t)x.row * p.ldq + (size_t)(x.h0 + min(ln & 15, x.Hb - 1)) * dk;
-    *reinterpret_cast<uint4*>(qf + i * 16) = *reinterpret_cast<const uint4*>(q + s * M::KS + (ln >> 4) * M::EPL);
+  // (the wave's steps of the query, all of a batch's loads in flight: one after another, nine round trips of 576 columns)
+  constexpr int kQPre = 9;
+  const float* qr = reinterpret_cast<const float*>(p.q) + (size_t)x.row * p.ldq + (size_t)(x.h0 + min(rl, x.Hb - 1)) * dk + g * M::EPL;
+  for (int s0 = w; s0 < steps; s0 += 4 * kQPre) {
+    u32x4 v[kQPre];
+#pragma unroll
+    for (int i = 0; i < kQPre; ++i) v[i] = *reinterpret_cast<const u32x4*>(qr + min(s0 + 4 * i, steps - 1) * M::KS);
+#pragma unroll
+    for (int i = 0; i < kQPre; ++i)
+      if (s0 + 4 * i < steps) *reinterpret_cast<u32x4*>(qf + ((s0 + 4 * i) * 64 + lane) * 16) = v[i];
   }
   const float sl2 = p.scale * kLog2e;
   float m = -1e30f, l = 0.f;
@@ -393,11 +407,17 @@ __global__ __launch_bounds__(256, EXACT && NT <= 8 ? 2 : 1) void latent_attn_f32
         if (s1 + i < steps) s0 = M::mma(__builtin_bit_cast(uint4, kf[q][i]), *reinterpret_cast<const uint4*>(qf + ((s1 + i) * 64 + lane) * 16), s0);
       __builtin_amdgcn_sched_barrier(0);
     };
-    for (int s = 0; s < steps; s += 2 * kKeyPre) {
+    auto two = [&](int s) {
       if (s + kKeyPre < steps) load_k(1, s + kKeyPre);
       products(0, s);
       if (s + 2 * kKeyPre < steps) load_k(0, s + 2 * kKeyPre);
       if (s + kKeyPre < steps) products(1, s + kKeyPre);
+    };
+    if constexpr (EXACT) {
+#pragma unroll
+      for (int s = 0; s < steps; s += 2 * kKeyPre) two(s);
+    } else {
+      for (int s = 0; s < steps; s += 2 * kKeyPre) two(s);
     }
     load_v(0, 0);
     attn_weights<float, NT>(s0, sl2, key0, x.pos, s_max[t & 1], pf, m, l, acc);
@@ -428,12 +448,19 @@ template <class T>
 __global__ __launch_bounds__(kOutThreads) void latent_out_kernel(LatentOutParams p, int rb) {
   using M = MM<T>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  __shared__ int s_used[16];                         // chunks of a row up to its last key
   const int h = blockIdx.x, r0 = blockIdx.y * rb, tid = threadIdx.x, nr = min(rb, p.rows - r0);
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6), rl = lane & 15, g = lane >> 4;
   const int stride = p.rank_p * (int)sizeof(T) + 16;
   float4* red = reinterpret_cast<float4*>(smem + 16 * stride);               // [512]
   float* fac = reinterpret_cast<float*>(smem + 16 * stride + kOutThreads * 16);  // [16][nch]: weight of every chunk's sums
   const size_t cs = (size_t)p.H * p.rank_p;
+  // ---- the first chunk's statistics of this thread (32 lanes per row), in front of the weights: what is asked for later arrives later
+  const int fr = min(tid >> 5, nr - 1);
+  const float2* const st = reinterpret_cast<const float2*>(p.stat) + (size_t)(r0 + fr) * p.nch * p.H + h;
+  const float2 first = st[(size_t)min(tid & 31, p.nch - 1) * p.H];
+  const float sink = p.sink[h] * kLog2e;
+  asm volatile("" ::: "memory");
   // ---- this wave's weights: column tile t, steps s0 .. s1
   const int steps = p.rank_p / M::KS, nt = p.vd >> 4, t = blockIdx.z * 4 + (w & 3), hs = (steps + 1) / 2;
   const int s0 = (w >> 2) * hs, s1 = min(steps, s0 + hs);
@@ -441,21 +468,24 @@ __global__ __launch_bounds__(kOutThreads) void latent_out_kernel(LatentOutParams
   uint4 wf[kOutPre];
 #pragma unroll
   for (int i = 0; i < kOutPre; ++i) wf[i] = wp[min(s0 + i, steps - 1) * 64];
-  // ---- chunk factors: 32 lanes per row
+  // ---- chunk factors
   {
     const int r = tid >> 5, k0 = tid & 31;
     if (r < nr) {
-      const float2* st = reinterpret_cast<const float2*>(p.stat) + (size_t)(r0 + r) * p.nch * p.H + h;
-      const float sink = p.sink[h] * kLog2e;
-      float mx = sink;
+      float mx = sink, used = 0.f;
       for (int k = k0; k < p.nch; k += 32) {
-        const float2 v = st[(size_t)k * p.H];
-        if (v.y > 0.f) mx = fmaxf(mx, v.x);
+        const float2 v = k == k0 ? first : st[(size_t)k * p.H];
+        if (v.y > 0.f) {
+          mx = fmaxf(mx, v.x);
+          used = (float)(k + 1);
+        }
       }
       mx = half_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
+      used = half_reduce(used, [](float a, float b) { return fmaxf(a, b); });
+      if (k0 == 0) s_used[r] = (int)used;
       float sum = 0.f;
       for (int k = k0; k < p.nch; k += 32) {
-        const float2 v = st[(size_t)k * p.H];
+        const float2 v = k == k0 ? first : st[(size_t)k * p.H];
         const float e = v.y > 0.f ? __builtin_amdgcn_exp2f(v.x - mx) : 0.f;
         fac[r * p.nch + k] = e;
         sum += v.y * e;
@@ -472,13 +502,15 @@ __global__ __launch_bounds__(kOutThreads) void latent_out_kernel(LatentOutParams
     const int q = i % items, part = i / items, r = q / quads, d = (q % quads) * 4;
     const float* pt = p.part + ((size_t)(r0 + r) * p.nch * p.H + h) * p.rank_p + d;
     float v[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int k = part; k < p.nch; k += 8 * P) {
+    // (a row's chunks up to the last that holds a key, not the launch's: 16 rows of 320 keys use 5 of 32; the merge 3.7 -> 1.7 us, all of it 9.2 -> 6.0)
+    const int used = s_used[r];
+    for (int k = part; k < used; k += 8 * P) {
       float u[8][4], f[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int kk = min(k + e * P, p.nch - 1);
+        const int kk = min(k + e * P, used - 1);
         ld4(pt + (size_t)kk * cs, u[e]);
-        f[e] = k + e * P < p.nch ? fac[r * p.nch + kk] : 0.f;
+        f[e] = k + e * P < used ? fac[r * p.nch + kk] : 0.f;
       }
 #pragma unroll
       for (int e = 0; e < 8; ++e)
@@ -584,7 +616,7 @@ int launch_attn_f32(const LatentAttnParams& p, hipStream_t st) {
   const size_t lds = 4096 + (size_t)(p.rank_p + p.rot_p) * 64;
   if (lds > kMaxLds) return -10;
   const dim3 grid(p.rows * ((p.H + 15) / 16), p.nch), block(256);
-  if (p.rank_p == 64 * NT) hipLaunchKernelGGL((latent_attn_f32_kernel<NT, true>), grid, block, lds, st, p);
+  if (p.rank_p == 64 * NT && p.rot_p == 64) hipLaunchKernelGGL((latent_attn_f32_kernel<NT, true>), grid, block, lds, st, p);
   else hipLaunchKernelGGL((latent_attn_f32_kernel<NT, false>), grid, block, lds, st, p);
   return (int)hipGetLastError();
 }

@@ -63,7 +63,7 @@ VWA_DEVICE f32x4 ld_sc1_x4(__amdgpu_buffer_rsrc_t r, int off) {
 // once for all of them.  777 rows of a 32-bit prompt, 8 / 4 heads of 128: both launches 332 -> 86 us per layer.
 //
 // Few rows are bound by the dependent round trips through memory (about 0.8 us each), not by bytes: everything whose address
-// known is requested first; scores are spread by a tile per wave (kTalkStat tiles a workgroup); and a mixing chunk holds CT
+// is known is requested first; scores are spread by a tile per wave (kTalkStat tiles a workgroup); and a mixing chunk holds CT
 // = 16 tiles, so that contexts of up to 256 keys take no partial sums, tickets and merging.  1 row of 225 keys, 16 / 4 heads
 // of 128: scores 5.4 -> 4.8, mixing 9.9 -> 8.4 us; 48 rows of 90 .. 250 keys, 8 / 4 heads: 7.4 -> 6.7, 10.5 -> 8.2.
 // What is requested first has to be read off the assembly: a gate's sigmoid behind its load, a load in a branch, a scalar load behind
