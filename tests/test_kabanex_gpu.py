@@ -717,6 +717,26 @@ def test_norm_adds_a_projections_slices(M, N, K, D):
     assert (ops.linear_parts(a[:1], ops.TiledWeight(w)) is None) == (N >= 4096)
 
 
+@pytest.mark.parametrize("n", [1, 2, 4, 5, 8, 9, 15, 16, 17, 24])
+@pytest.mark.parametrize("N,D", [(1024, 1022), (2048, 2048), (4096, 4090)])
+def test_norm_adds_any_number_of_slices(n, N, D):
+    """Batches of slices (up to 15, 7, 3 in flight by the row's width), each added once and in their order."""
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    x, parts, w = rnd(3, N), rnd(n, 3, N), rnd(D)
+    x[:, D:] = 0
+    parts[:, :, D:] = 0
+    s = parts[0].clone()
+    for k in range(1, n):
+        s += parts[k]
+    want = x + s
+    out = torch.empty(3, N, device="cuda")
+    ops.layernorm_f32(x, w, None, eps=1e-5, out=out, parts=parts)
+    assert torch.equal(x, want)
+    # (f32: a mean and a variance of D terms, some sqrt(D) roundings of 2^-24)
+    assert rel(out[:, :D], torch.nn.functional.layer_norm(want[:, :D].double(), (D,), w.double(), None, 1e-5).cpu()) < 4e-6
+
+
 def test_a_projections_slices_are_the_callers():
     """What linear_parts returned stands, whatever is launched before the norm that reads it: another projection's slices, a sum
     of slices, both captured behind it."""
