@@ -13,6 +13,8 @@
 //    and writes the outputs; the run's last chunk writes the state.
 //
 // A run that starts at position 0 starts from zeros whatever its slot holds.
+#include <type_traits>
+
 #include "mixer_kernels.h"
 #include "stack_types.h"
 
@@ -57,12 +59,11 @@ template <class T> VWA_DEVICE int u_stride(int bs) { return bs * (int)sizeof(T) 
 template <int PRE>
 struct GateFrags {
   uint4 r[PRE], i[PRE];
-  template <class T> VWA_DEVICE void load(const T* gw, int steps, int s0, int beg = 0, int end = PRE) {
+  template <class T> VWA_DEVICE void load(const T* gw, int steps, int s0) {
     const uint4* wr = reinterpret_cast<const uint4*>(gw);
     const unsigned l = lane_id();                    // (uniform bases: one offset register)
 #pragma unroll
     for (int s = 0; s < PRE; ++s) {
-      if (s < beg || s >= end) continue;
       const uint4* ws = wr + min(s0 + s, steps - 1) * 64;
       r[s] = ws[l];
       i[s] = (ws + steps * 64)[l];
@@ -221,33 +222,146 @@ VWA_DEVICE void save_inputs4(const RgLruParams& p, int r, int n, bool fresh, flo
 // Workgroup (block, tile, part): the runs whose first row lies in rows 16 tile .. 16 tile + 15, 16 rows at a time to
 // their ends (other runs' rows count as inert); row_parts of the block's 16-channel tiles.  Every part forms the whole block's u,
 // so the inputs it is formed from are replaced by the last part that has read them (RgLruParams::tickets).
-// What bounds it is one CU drawing a block's gates (256 and 512 KB of 256 channels) behind a chain of round trips, on 4 - 16 CUs.
-// us with parts of all 16, 8, 4, 2 tiles, gates in L2: 32 bits, 4 rows x 4 blocks 16.1, 12.0, 10.6, 10.6; bf16, 16 rows x 8 11.2, 10.6,
-// 10.7, 11.0.  (The save by the waves without a tile, beside the products: 0.3 - 1 slower.)
-// A part is worth its own forming of u and its ticket from 128 KB of gates on, and a wave to each of four tiles: of fewer, blocks of 80
-// and 128 channels were 9 - 18 % slower in 16 bits (4 rows of 128: 6.8 -> 7.7) and up to 4 % in 32, 10 blocks of 256 in 16 bits at 48 rows 10 %.
 constexpr int kPartBytes = 128 * 1024;
 int row_parts(int bs, int bytes) {
   const int tiles = bs / 16, draw = 32 * bs * bytes, per = (kPartBytes + draw - 1) / draw;
   return (tiles + (per > 4 ? per : 4) - 1) / (per > 4 ? per : 4);
 }
 
-template <class T>
+// four consecutive values as they were read
+template <class T> struct Raw4;
+template <> struct Raw4<u16> { typedef u32x2 V; };
+template <> struct Raw4<float> { typedef f32x4 V; };
+VWA_DEVICE void from_raw(const u32x2& u, float (&v)[4]) {
+  v[0] = __uint_as_float(u.x << 16), v[1] = __uint_as_float(u.x & 0xffff0000u);
+  v[2] = __uint_as_float(u.y << 16), v[3] = __uint_as_float(u.y & 0xffff0000u);
+}
+VWA_DEVICE void from_raw(const f32x4& u, float (&v)[4]) { v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w; }
+
+struct ConvRow {
+  int r, j;                                          // row; rows of its run in front of it
+  const float* st;
+  bool fresh, live;
+};
+// four channels of u of N rows of at most kTaps taps, and the inputs it was formed from (old[n][k]: k tokens back; the furthest is not
+// kept, the next token needs it no more).  What the rows share is loaded once; all loads are in flight together (those of a row that
+// is not live bring nothing that counts).
+constexpr int kTaps = 4;
+template <class T, int N>
+VWA_DEVICE void conv_rows(const RgLruParams& p, const ConvRow (&q)[N], int ch, float (&u)[N][4], f32x4 (&old)[N][kTaps - 1]) {
+  typedef typename Raw4<T>::V Raw;
+  const int W = p.nb * p.bs;
+  f32x4 w[kTaps], s[N][kTaps - 1];                   // (the row's own input is never the state's)
+  Raw x[N][kTaps];
+  const f32x4 cb = *reinterpret_cast<const f32x4*>(p.cb + ch), xb = *reinterpret_cast<const f32x4*>(p.xb + ch);
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+#pragma unroll
+    for (int e = 0; e < kTaps; ++e) {
+      const int k = min(e, p.taps - 1);
+      x[n][e] = *reinterpret_cast<const Raw*>(input_at<T>(p, q[n].r - min(k, q[n].j), ch));
+      if (e) s[n][e - 1] = *reinterpret_cast<const f32x4*>(q[n].st + (size_t)min(p.taps - (k - q[n].j), p.taps - 1) * W + ch);
+    }
+#pragma unroll
+  for (int e = 0; e < kTaps; ++e) w[e] = *reinterpret_cast<const f32x4*>(p.cw + (size_t)max(p.taps - 1 - e, 0) * W + ch);
+  asm volatile("" ::: "memory");
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) u[n][c] = cb[c];
+#pragma unroll
+    for (int e = 0; e < kTaps; ++e) {
+      float v[4];
+      from_raw(x[n][e], v);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        v[c] = e <= q[n].j ? v[c] + xb[c] : q[n].fresh ? 0.f : s[n][e ? e - 1 : 0][c];
+        if (e < p.taps) u[n][c] += w[e][c] * v[c];
+        if (e < kTaps - 1) old[n][e][c] = v[c];
+      }
+    }
+  }
+}
+
+// fragments of 16 channels' gates: both, or the one a wave has
+template <int G, int PRE>
+struct RowGates {
+  uint4 v[G][PRE];
+  VWA_DEVICE void load(const uint4* w, int steps, int s0) {
+    const unsigned l = lane_id();                    // (uniform bases: one offset register)
+#pragma unroll
+    for (int s = 0; s < PRE; ++s)
+#pragma unroll
+      for (int k = 0; k < G; ++k) v[k][s] = (w + (k * steps + min(s0 + s, steps - 1)) * 64)[l];
+  }
+  template <class T>
+  VWA_DEVICE void products(const char* ua, const uint4* w, int steps, f32x4 (&acc)[G]) {
+#pragma unroll
+    for (int k = 0; k < G; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto u_at = [&](int s) { return *reinterpret_cast<const u32x4*>(ua + s * 64); };
+#pragma unroll 1
+    for (int s0 = 0; s0 < steps; s0 += PRE) {
+      if (steps - s0 >= PRE) {                       // (no branches: u is read a batch ahead of its products)
+        constexpr int B = 2;
+        u32x4 a[2][B];
+#pragma unroll
+        for (int e = 0; e < B; ++e) a[0][e] = u_at(s0 + e);
+#pragma unroll
+        for (int b = 0; b < PRE / B; ++b) {
+          if (b + 1 < PRE / B)
+#pragma unroll
+            for (int e = 0; e < B; ++e) a[(b + 1) & 1][e] = u_at(s0 + (b + 1) * B + e);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int e = 0; e < B; ++e)
+#pragma unroll
+            for (int k = 0; k < G; ++k) acc[k] = MM<T>::mma(__builtin_bit_cast(uint4, a[b & 1][e]), v[k][b * B + e], acc[k]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < PRE; ++s) {
+          if (s0 + s >= steps) break;
+          const u32x4 a = u_at(s0 + s);
+#pragma unroll
+          for (int k = 0; k < G; ++k) acc[k] = MM<T>::mma(__builtin_bit_cast(uint4, a), v[k][s], acc[k]);
+        }
+      }
+      if (s0 + PRE < steps) load(w, steps, s0 + PRE);
+    }
+  }
+};
+
+// A wave has one of two tasks, so that neither waits for the other's loads (they come back in order).  The first draw a 16-channel
+// tile's gates, requested before anything is known of the rows, multiply and scan; the others form u and write back the inputs it was
+// formed from, out of registers where the run's last row is in their hands.  Every wave finds the runs by itself.
+// What bounds it is one CU drawing 128 KB of gates (2 to 3 us, cold) and the convolution's 50 - 110 KB behind them: u is there 5.3 us
+// after the first wave's start (4 rows in 32 bits) or 6.4 (16 in 16 bits), products, step and results take 2 - 3 more.  us of a launch in
+// a model's step, one task a wave, which waits for half of the gates, then the convolution, then the other half, and reads the inputs
+// again to write them back -> here: 4 rows of 4 blocks of 256 in 32 bits 12.5 -> 9.4, 16 rows of 8 in 16 bits 13.5 -> 9.7.
+// SPLIT: at most four tiles, a wave for each of a tile's gates: eight waves request them, and 16 steps of 256 channels stay in registers.
+template <class T, bool SPLIT>
 __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
-  constexpr int PRE = 8;
+  constexpr int NR = 2, G = SPLIT ? 1 : 2, PRE = SPLIT ? 16 : 8;  // rows a thread takes at most with their inputs kept
   extern __shared__ __attribute__((aligned(16))) char us[];
   // of a row: its sequence; its run's first row (-1: inert); its run's rows (at the run's last row, else 0); whether
   // tokens precede it / its run
   __shared__ int s_seq[64], s_first[64], s_len[64], s_old[64], s_run_old[64];
   __shared__ int s_last;
+  __shared__ f32x4 s_gate[SPLIT ? 4 : 1][64];
   const int blk = blockIdx.x, lo = blockIdx.y * 16, bs = p.bs, c0 = blk * bs;
-  const int tid0 = threadIdx.x, nthr = blockDim.x, w = __builtin_amdgcn_readfirstlane(tid0 >> 6);
-  const int stride = u_stride<T>(bs), steps = bs / MM<T>::KS, tiles = bs / 16, waves = nthr >> 6;
-  const int tper = (tiles + gridDim.z - 1) / gridDim.z, ct0 = blockIdx.z * tper, ct1 = min(tiles, ct0 + tper);  // this workgroup's
+  const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int stride = u_stride<T>(bs), steps = bs / MM<T>::KS, tiles = bs / 16;
+  const int tper = small_div(tiles + gridDim.z - 1, gridDim.z), ct0 = blockIdx.z * tper, ct1 = min(tiles, ct0 + tper);  // this workgroup's
+  const int side = min(tper, SPLIT ? 4 : 8), gw = SPLIT ? 2 * side : side;  // tiles side by side, the waves they take
+  const int ctid = tid - gw * 64, cthr = blockDim.x - gw * 64;
+  const bool meet = SPLIT || gridDim.z > 1;          // the two kinds of waves meet behind the products
   T* out = reinterpret_cast<T*>(p.out);
-  const T* gw0 = reinterpret_cast<const T*>(p.gw) + (size_t)blk * tiles * 32 * bs;
-  if (tid0 < 64) {                                   // (one wave: runs from the rows' ids)
-    const int r = tid0, rc = min(r, p.rows - 1), id = p.seq_ids[rc], old = p.positions[rc] > 0;
+  const int hi = min(lo + 16, p.rows);
+  auto owned = [&](int r) { return s_first[r] >= lo && s_first[r] < hi; };
+  auto state_of = [&](int r) { return p.state + (size_t)s_seq[r] * p.state_ld; };
+  auto find_runs = [&] {                             // (all waves leave the same)
+    const int r = lane, rc = min(r, p.rows - 1), id = p.seq_ids[rc], old = p.positions[rc] > 0;
     const bool live = p.slots[rc] >= 0 && r < p.rows;
     const int seq = live ? id : -1 - r;
     const int before = __shfl_up(seq, 1, 64), after = __shfl_down(seq, 1, 64);
@@ -259,83 +373,159 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(RgLruParams p) {
     s_len[r] = live && (r == 63 || after != seq) ? r + 1 - first : 0;
     s_old[r] = old;
     s_run_old[r] = __shfl(old, max(first, 0), 64);
-  }
-  __syncthreads();
-  const int quads = bs / 4, hi = min(lo + 16, p.rows);
-  auto owned = [&](int r) { return s_first[r] >= lo && s_first[r] < hi; };
-  auto state_of = [&](int r) { return p.state + (size_t)s_seq[r] * p.state_ld; };
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+
+  if (w < gw) {
+    const int wt = SPLIT ? w >> 1 : w, gate = SPLIT ? w & 1 : 0;  // this wave's tile of those side by side
+    const uint4* gw0 = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(p.gw) + (size_t)blk * tiles * 32 * bs) + gate * steps * 64;
+    RowGates<G, PRE> f;
+    f.load(gw0 + (size_t)min(ct0 + wt, ct1 - 1) * steps * 128, steps, 0);
+    asm volatile("" ::: "memory");
+    find_runs();
 #pragma unroll 1
-  for (int r0 = lo; r0 < p.rows; r0 += 16) {
-    if (r0 > lo && !owned(r0)) break;                // (a run that goes past the tile owns the next row)
-    const int n = min(16, p.rows - r0);
-    const bool ends = r0 + 16 >= p.rows || !owned(r0 + 16);
+    for (int r0 = lo; r0 < p.rows; r0 += 16) {
+      if (r0 > lo && !owned(r0)) break;              // (a run that goes past the tile owns the next row)
+      const int n = min(16, p.rows - r0);
+      const bool ends = r0 + 16 >= p.rows || !owned(r0 + 16);
 #pragma unroll 1
-    for (int t0 = ct0; t0 < ct1; t0 += waves) {
-      // (mostly the only pass: addresses are formed where they are used, not kept across passes)
-      const int tid = opaque(tid0), lane = tid & 63, rl = lane & 15, g = lane >> 4;
-      const int ct = min(t0 + w, ct1 - 1), ch = c0 + ct * 16 + rl;
-      // ---- requested ahead of the convolution
-      const T* gw = gw0 + (size_t)ct * 32 * bs;
-      GateFrags<PRE> f;
-      f.load(gw, steps, 0, 0, PRE / 2);
-      const float rb = p.rb[ch], ib = p.ib[ch], dec = p.decay[ch], yb = p.yb[ch];
-      T yv[4];
-      float s_in[4];
+      for (int t0 = ct0; t0 < ct1; t0 += side) {
+        // (mostly the only pass: addresses are formed where they are used, not kept across passes)
+        const int l = opaque(lane), rl = l & 15, g = l >> 4, ct = min(t0 + wt, ct1 - 1), ch = c0 + ct * 16 + rl;
+        const uint4* gwt = gw0 + (size_t)ct * steps * 128;
+        if (r0 > lo || t0 > ct0) f.load(gwt, steps, 0);
+        // what the step needs beside u: asked for behind the gates, made ready before u is
+        const float rb = p.rb[ch], ib = p.ib[ch], dec = p.decay[ch], yb = p.yb[ch];
+        T yv[4];
+        float s_in[4], y[4];
+        bool mine[4], head[4], goes_on[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = r0 + min(4 * g + i, n - 1);
-        yv[i] = reinterpret_cast<const T*>(p.yx)[(size_t)r * p.ld + ch];
-        s_in[i] = state_of(r)[ch];
-      }
-      if (t0 == ct0) {
-#pragma unroll 1
-        for (int x = tid; x < 16 * quads; x += nthr) {
-          const int i = x / quads, c = (x % quads) * 4, r = r0 + i;
-          float u[4] = {0.f, 0.f, 0.f, 0.f};
-          if (i < n && owned(r)) conv4<T, 4>(p, r, r - s_first[r], state_of(r), !s_run_old[r], c0 + c, u);
-          st4(reinterpret_cast<T*>(us + i * stride) + c, u);
+        for (int i = 0; i < 4; ++i) {
+          const int li = 4 * g + i, r = r0 + min(li, n - 1);
+          yv[i] = reinterpret_cast<const T*>(p.yx)[(size_t)r * p.ld + ch];
+          s_in[i] = state_of(r)[ch];
+          mine[i] = li < n && owned(r);
+          head[i] = s_first[r] == r || li == 0;
+          goes_on[i] = head[i] && s_old[r];          // (also a run that goes on from the rows before: its state was saved)
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = gelu_tanh(ldv(&yv[i]) + yb);
+        if (t0 == ct0) lds_sync();                   // u is formed
+        if (t0 + wt >= ct1 && !SPLIT) continue;
+        f32x4 acc[G];
+        f.template products<T>(us + rl * stride + g * 16, gwt, steps, acc);
+        if constexpr (SPLIT) {
+          if (gate) s_gate[wt][l] = acc[0];
+          lds_sync();                                // (the other waves' ticket as well)
+          if (gate || t0 + wt >= ct1) continue;
+        }
+        const f32x4 ar = acc[0], ai = SPLIT ? s_gate[SPLIT ? wt : 0][l] : acc[G - 1];
+        float a[4], b[4], s[4], A, B;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float u = ldv(reinterpret_cast<const T*>(us + (4 * g + i) * stride) + ct * 16 + rl);
+          const Step st = lru_step(ar[i] + rb, ai[i] + ib, dec, u);
+          b[i] = !mine[i] ? 0.f : goes_on[i] ? st.b + st.a * s_in[i] : st.b;
+          a[i] = mine[i] && !head[i] ? st.a : 0.f;
+        }
+        scan_tile(a, b, 0.f, s, A, B);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int li = 4 * g + i, r = r0 + li;
+          if (li >= n) continue;
+          if (mine[i]) {
+            stv(out + (size_t)r * p.ldo + ch, s[i] * y[i]);
+            if (s_len[r] > 0 || li == n - 1) state_of(r)[ch] = s[i];
+          } else if (s_first[r] < 0 && r0 == lo) {
+            stv(out + (size_t)r * p.ldo + ch, 0.f);  // inert row of a padded step
+          }
         }
       }
-      __builtin_amdgcn_sched_barrier(0);             // (the convolution's registers are free from here)
-      f.load(gw, steps, 0, PRE / 2, PRE);
-      __syncthreads();                               // (every read of the old inputs is done as well)
-      if (gridDim.z > 1 && ends && t0 == ct0 && tid0 == 0) {
+      if (ends) {
+        if (meet && !SPLIT) lds_sync();
+        return;
+      }
+      __syncthreads();                               // u is overwritten; saved states are read by the next rows
+    }
+    return;
+  }
+
+  find_runs();
+  const int quads = bs / 4, cols = min(quads, cthr), per = small_div(cthr, cols);  // rows side by side
+  const int i0 = ctid / cols, ch = (ctid - i0 * cols) * 4;
+  const bool spread = cols == quads;                 // (else: more columns than threads)
+#pragma unroll 1
+  for (int r0 = lo; r0 < p.rows; r0 += 16) {
+    if (r0 > lo && !owned(r0)) break;
+    const int n = min(16, p.rows - r0);
+    const bool ends = r0 + 16 >= p.rows || !owned(r0 + 16);
+    // every part's waves have read the old inputs: the last one's replace them (behind the barrier the gates' waves come to as well)
+    auto last_part = [&] {
+      if (gridDim.z > 1 && ctid == 0) {
         int* at = p.tickets + blockIdx.y * gridDim.x + blk;
         s_last = __hip_atomic_fetch_add(at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.z - 1;
         if (s_last) __hip_atomic_store(at, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-      if (t0 + w >= ct1) continue;
-      f32x4 ar[1], ai[1];
-      gate_products<T, 1, PRE>(us, stride, gw, steps, f, ar, ai);
-      float a[4], b[4], s[4], A, B;
+      if (meet) lds_sync();
+      return gridDim.z == 1 || s_last;
+    };
+    auto in_registers = [&](auto rows) {             // the one pass, each of its rows in one thread's hands
+      constexpr int N = decltype(rows)::value;
+      ConvRow q[N];
+      float u[N][4];
+      f32x4 old[N][kTaps - 1];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int li = 4 * g + i, r = r0 + min(li, n - 1);
-        const bool mine = li < n && owned(r), head = s_first[r] == r || li == 0;
-        const float u = ldv(reinterpret_cast<const T*>(us + li * stride) + ct * 16 + rl);
-        const Step st = lru_step(ar[0][i] + rb, ai[0][i] + ib, dec, u);
-        // (a run that goes on from the rows before: its state was saved)
-        b[i] = !mine ? 0.f : head && s_old[r] ? st.b + st.a * s_in[i] : st.b;
-        a[i] = mine && !head ? st.a : 0.f;
+      for (int k = 0; k < N; ++k) {
+        const int i = i0 + k * per, r = r0 + min(i, n - 1), first = s_first[r];
+        const bool live = i < n && first >= lo && first < hi;
+        q[k] = ConvRow{r, live ? r - first : 0, state_of(r), !s_run_old[r], live};
       }
-      scan_tile(a, b, 0.f, s, A, B);
+      conv_rows<T, N>(p, q, c0 + ch, u, old);
+      if (i0 < per) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int li = 4 * g + i, r = r0 + li;
-        if (li >= n) continue;
-        if (owned(r)) {
-          stv(out + (size_t)r * p.ldo + ch, s[i] * gelu_tanh(ldv(&yv[i]) + yb));
-          if (s_len[r] > 0 || li == n - 1) state_of(r)[ch] = s[i];
-        } else if (s_first[r] < 0 && r0 == lo) {
-          stv(out + (size_t)r * p.ldo + ch, 0.f);    // inert row of a padded step
+        for (int k = 0; k < N; ++k) {
+          const int i = i0 + k * per;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) u[k][c] = q[k].live ? u[k][c] : 0.f;
+          if (i < 16) st4(reinterpret_cast<T*>(us + i * stride) + ch, u[k]);
         }
+        const float zero[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int i = i0 + N * per; i < 16; i += per) st4(reinterpret_cast<T*>(us + i * stride) + ch, zero);
       }
+      lds_sync();                                    // (the values were used: every read of the old inputs is done)
+      if (!last_part() || i0 >= per) return;
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        if (!q[k].live || s_len[q[k].r] == 0) continue;
+#pragma unroll
+        for (int e = 0; e < kTaps - 1; ++e)
+          if (e < p.taps - 1)
+            *reinterpret_cast<f32x4*>(const_cast<float*>(q[k].st) + (size_t)(p.taps - 1 - e) * (p.nb * bs) + c0 + ch) = old[k][e];
+      }
+    };
+    if (r0 == lo && ends && spread && p.taps <= kTaps && n <= NR * per) {
+      if (n <= per) in_registers(std::integral_constant<int, 1>{});
+      else in_registers(std::integral_constant<int, NR>{});
+      return;
     }
-    __syncthreads();                                 // u is overwritten; saved states are read by the next rows
-    if (!ends) continue;
-    if (gridDim.z > 1 && !s_last) return;            // (the last one of the block's workgroups to read the old inputs replaces them)
 #pragma unroll 1
-    for (int x = opaque(tid0); x < (r0 + n - lo) * quads; x += nthr) {
+    for (int x = opaque(ctid); x < 16 * quads; x += cthr) {
+      const int i = x / quads, cx = (x % quads) * 4, r = r0 + i;
+      float u[4] = {0.f, 0.f, 0.f, 0.f};
+      if (i < n && owned(r)) conv4<T, 4>(p, r, r - s_first[r], state_of(r), !s_run_old[r], c0 + cx, u);
+      st4(reinterpret_cast<T*>(us + i * stride) + cx, u);
+    }
+    lds_sync();
+    if (!ends) {
+      if (SPLIT) lds_sync();
+      __syncthreads();                               // u is overwritten
+      continue;
+    }
+    if (!last_part()) return;
+#pragma unroll 1
+    for (int x = opaque(ctid); x < (r0 + n - lo) * quads; x += cthr) {
       const int r = lo + x / quads, len = s_len[r];
       if (len > 0 && owned(r)) save_inputs4<T>(p, r, len, !s_run_old[r], state_of(r), c0 + (x % quads) * 4);
     }
@@ -495,9 +685,11 @@ size_t u_bytes(int rows, int bs) { return (size_t)rows * (bs * sizeof(T) + kPad)
 template <class T>
 int launch_rows(const RgLruParams& p, hipStream_t st) {
   if (u_bytes<T>(16, p.bs) > kMaxLds) return -10;
-  const int tiles = p.bs / 16;
-  const dim3 grid(p.nb, (p.rows + 15) / 16, p.tickets ? row_parts(p.bs, sizeof(T)) : 1), block(64 * (tiles < 16 ? tiles : 16));
-  hipLaunchKernelGGL((rglru_rows_kernel<T>), grid, block, u_bytes<T>(16, p.bs), st, p);
+  const int tiles = p.bs / 16, parts = p.tickets ? row_parts(p.bs, sizeof(T)) : 1, tper = (tiles + parts - 1) / parts;
+  const int form = (16 * (p.bs / 4) + 63) / 64, gates = tper <= 4 ? 2 * tper : tper < 8 ? tper : 8;
+  const dim3 grid(p.nb, (p.rows + 15) / 16, parts), block(64 * (gates + (form < 8 ? form : 8)));
+  if (tper <= 4) hipLaunchKernelGGL((rglru_rows_kernel<T, true>), grid, block, u_bytes<T>(16, p.bs), st, p);
+  else hipLaunchKernelGGL((rglru_rows_kernel<T, false>), grid, block, u_bytes<T>(16, p.bs), st, p);
   return (int)hipGetLastError();
 }
 

@@ -153,6 +153,29 @@ def test_rglru(dtype, W, nb, taps, lens):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("W,nb,taps", [(512, 2, 4), (256, 4, 3), (320, 1, 4), (512, 1, 5)])
+def test_rglru_decoded_rows(dtype, W, nb, taps):
+    """One row of every sequence, as many as a thread takes one or two of (8, 16 of 256 channels), into the next tile; a block's parts and one
+    workgroup: the same bits as every row alone, whose results test_rglru has, and an inert row among them."""
+    _, p, _ = rglru_case(W, nb, taps, dtype)
+    for rows in (1, 4, 5, 8, 9, 16, 17):
+        yx = rnd(rows, 2 * W, seed=rows, dtype=dtype).to(DEV)
+        ids = torch.randperm(20, generator=torch.Generator().manual_seed(rows))[:rows].int().to(DEV)
+        pos = (torch.arange(rows, dtype=torch.int32) % 6).to(DEV)  # (fresh ones, some with fewer tokens behind them than taps)
+        slots = pos.long().clone()
+        if rows > 2:
+            slots[1] = -1
+        st0 = rnd(20, taps * W, seed=3).to(DEV)
+        want, end = torch.zeros(rows, W, dtype=dtype, device=DEV), st0.clone()
+        for r in range(rows):
+            ops.rglru(yx[r : r + 1], p, seq_ids=ids[r : r + 1], positions=pos[r : r + 1], slots=slots[r : r + 1], state=end, out=want[r : r + 1])
+        for t in (None, torch.zeros(p.nb * 2, dtype=torch.int32, device=DEV)):
+            st, out = st0.clone(), torch.full((rows, W), float("nan"), dtype=dtype, device=DEV)
+            ops.rglru(yx, p, seq_ids=ids, positions=pos, slots=slots, state=st, out=out, tickets=t)
+            assert torch.equal(out, want) and torch.equal(st, end) and (t is None or not t.any())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_rglru_inert_rows(dtype):
     w, p, chan = rglru_case(256, 2, 3, dtype)
     yx = rnd(6, 512, seed=1, dtype=dtype).to(DEV)
