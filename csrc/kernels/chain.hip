@@ -842,10 +842,11 @@ __global__ __launch_bounds__(KS * 64) void chain_kernel(const ChainParams* __res
   pf_prev = pf_next;
   pf_next = false;
   const ChainParams& cp = cpp[li];  // device-resident descriptor
-  // Warm the scalar cache with the whole descriptor (25 x 64-byte lines) in ONE round trip: the
+  // Warm the scalar cache with the whole descriptor (24 x 64-byte lines) in ONE round trip: the
   // fields are otherwise fetched behind branches and earlier fields' values, a chain of dependent
   // scalar misses (the attention prologue measured ~6 of them before its first vector load)
-  static_assert(sizeof(ChainParams) <= 25 * 64, "descriptor warm-up covers 25 lines");
+  // (exactly: a line past the last descriptor may be of no allocation, and reading it faults)
+  static_assert(sizeof(ChainParams) == 24 * 64, "the warm-up reads the descriptor's 24 lines and no other");
   {
     // (non-volatile, no memory clobber: a volatile block counts as a memory write and turns every
     // later descriptor read into a vector load; the never-true test keeps it alive)
@@ -855,7 +856,7 @@ __global__ __launch_bounds__(KS * 64) void chain_kernel(const ChainParams* __res
         "s_load_dword %0, %1, 0x200\n\t""s_load_dword %0, %1, 0x240\n\t""s_load_dword %0, %1, 0x280\n\t""s_load_dword %0, %1, 0x2c0\n\t"
         "s_load_dword %0, %1, 0x300\n\t""s_load_dword %0, %1, 0x340\n\t""s_load_dword %0, %1, 0x380\n\t""s_load_dword %0, %1, 0x3c0\n\t"
         "s_load_dword %0, %1, 0x400\n\t""s_load_dword %0, %1, 0x440\n\t""s_load_dword %0, %1, 0x480\n\t""s_load_dword %0, %1, 0x4c0\n\t""s_load_dword %0, %1, 0x500\n\t"
-        "s_load_dword %0, %1, 0x540\n\t""s_load_dword %0, %1, 0x580\n\t""s_load_dword %0, %1, 0x5c0\n\t""s_load_dword %0, %1, 0x600\n\t"
+        "s_load_dword %0, %1, 0x540\n\t""s_load_dword %0, %1, 0x580\n\t""s_load_dword %0, %1, 0x5c0\n\t"
         "s_waitcnt lgkmcnt(0)"
         : "=&s"(junk)
         : "s"(cpp + li));

@@ -100,7 +100,7 @@ struct ChainTP {
 };
 
 // (64-byte aligned: a multi-layer launch indexes an array of them, and each one's scalar-cache
-// warm-up, chain_kernel, covers exactly its 25 lines)
+// warm-up, chain_kernel, covers exactly its 24 lines)
 struct alignas(64) ChainParams {
   ChainPhase ph[kChainMaxPhases];
   int n;
