@@ -341,10 +341,13 @@ VWA_DEVICE unsigned long long ss_fix(float sq) {
   return (unsigned long long)fminf(sq * (float)kSsScale + 0.5f, 9.2e18f);  // (>= 0)
 }
 
+VWA_DEVICE float ss_scale(const GemmParams& p, unsigned long long ss) {
+  return rsqrtf((float)((double)ss * (1.0 / kSsScale)) / (float)p.K + p.ss_eps);
+}
 // per-row RMSNorm scale: rstd[m], or from the handed-off sum of squares (ss_in), or 1
 VWA_DEVICE float row_scale(const GemmParams& p, int m) {
   if (p.rstd) return p.rstd[m];
-  if (p.ss_in) return rsqrtf((float)((double)p.ss_in[m] * (1.0 / kSsScale)) / (float)p.K + p.ss_eps);
+  if (p.ss_in) return ss_scale(p, p.ss_in[m]);
   return 1.f;
 }
 
@@ -407,11 +410,11 @@ VWA_DEVICE void qkv_store(const GemmParams& p, int m, int n, const float (&o)[8]
 // f32 partial slab loads of the split-K reduce (AUX: buffer cache bits; the reduce runs after the
 // GEMM launch's end made the slabs visible, so plain loads)
 template <int AUX>
-VWA_DEVICE float4 ld_f4(__amdgpu_buffer_rsrc_t r, size_t idx) {
-  return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(idx * 4), 0, AUX));
+VWA_DEVICE f32x4 ld_f4(__amdgpu_buffer_rsrc_t r, size_t idx) {
+  return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(idx * 4), 0, AUX));
 }
 
-VWA_DEVICE void add8(float (&v)[8], const float4& a, const float4& b) {
+VWA_DEVICE void add8(float (&v)[8], const f32x4& a, const f32x4& b) {
   v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w; v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
 }
 
@@ -427,79 +430,106 @@ VWA_DEVICE int item_src1(int c) { return EPI == EPI_SWIGLU ? item_src0<EPI>(c) +
 template <int EPI>
 constexpr bool kTwoSrc = EPI == EPI_SWIGLU || EPI == EPI_QKV;
 
-// sums a (src0) / b (src1) of NI items (row m, first columns c[i]); the slices in batches of ZB,
-// all of a batch's loads (every item) in flight before any is used; slices past the last read
-// past the slab range (the buffer returns zeros)
-template <int EPI, int AUX, int NI, int ZB>
-VWA_DEVICE void sum_items(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, int m, const int (&c)[NI],
-                          const bool (&ok)[NI], float (&a)[NI][8], float (&b)[NI][8]) {
-  const size_t slab = (size_t)p.M * p.N;
+// one item's slices z0 .. z0 + ZB - 1; those past the last read past the slab range (the buffer returns zeros)
+template <int EPI, int AUX, int ZB>
+struct ItemSlabs {
+  f32x4 x[ZB][2], y[kTwoSrc<EPI> ? ZB : 1][2];
+  VWA_DEVICE void load(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, int m, int c, int z0) {
+    const size_t slab = (size_t)p.M * p.N;
+    const int n0 = item_src0<EPI>(c), n1 = item_src1<EPI>(c);
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) a[i][e] = b[i][e] = 0.f;
-  for (int z0 = 0; z0 < p.splits; z0 += ZB) {
-    float4 x[NI][ZB][2], y[NI][ZB][2];
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int u = 0; u < ZB; ++u) {
-        const size_t base = (size_t)(z0 + u) * slab + (size_t)m * p.N;
-        const int n0 = item_src0<EPI>(c[i]), n1 = item_src1<EPI>(c[i]);
-        // (an item past the row end reads offset 0 of slice z: in range, discarded)
-        x[i][u][0] = ld_f4<AUX>(rws, ok[i] ? base + n0 : 0);
-        x[i][u][1] = ld_f4<AUX>(rws, ok[i] ? base + n0 + 4 : 0);
-        if constexpr (kTwoSrc<EPI>) {
-          y[i][u][0] = ld_f4<AUX>(rws, ok[i] ? base + n1 : 0);
-          y[i][u][1] = ld_f4<AUX>(rws, ok[i] ? base + n1 + 4 : 0);
-        }
+    for (int u = 0; u < ZB; ++u) {
+      const size_t base = (size_t)(z0 + u) * slab + (size_t)m * p.N;
+      x[u][0] = ld_f4<AUX>(rws, base + n0);
+      x[u][1] = ld_f4<AUX>(rws, base + n0 + 4);
+      if constexpr (kTwoSrc<EPI>) {
+        y[u][0] = ld_f4<AUX>(rws, base + n1);
+        y[u][1] = ld_f4<AUX>(rws, base + n1 + 4);
       }
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-#pragma unroll
-      for (int u = 0; u < ZB; ++u) {
-        add8(a[i], x[i][u][0], x[i][u][1]);
-        if constexpr (kTwoSrc<EPI>) add8(b[i], y[i][u][0], y[i][u][1]);
-      }
+    }
   }
-}
+  VWA_DEVICE void add(float (&a)[8], float (&b)[8]) const {
+#pragma unroll
+    for (int u = 0; u < ZB; ++u) {
+      add8(a, x[u][0], x[u][1]);
+      if constexpr (kTwoSrc<EPI>) add8(b, y[u][0], y[u][1]);
+    }
+  }
+};
 
-// what the epilogue of an item reads besides the slabs, requested in front of them: behind the sums each was one more
-// dependent round trip (two with the rotary row), and a reduction of few rows is nothing else (32 rows x 8 slices: 4096
-// columns 5.8 -> 5.1 us, 6144 with the rotation 7.3 -> 5.5)
+// what the epilogue of an item reads besides the slabs, as it was read: nothing here waits for a load (behind the sums each was one more
+// dependent round trip, and a reduction of few rows is nothing else)
+template <int EPI> struct ItemRaw {
+  static constexpr bool kBias = EPI != EPI_SWIGLU;
+  int pos;
+  int64_t slot;
+  float sx;
+  unsigned scale[2];  // rstd's value or the two halves of the sum of squares
+  f32x4 swa[2], swb[2];
+  u32x4 ba, bb;    // 8 bf16
+  u32x4 r0, r1;    // residual: 8 bf16 (r0) or f32 (vectors: as structs they went through 272 bytes of scratch a lane)
+};
+// (parts of a caller's tensors: aligned as their elements)
+typedef u32x4 u32x4_bf __attribute__((aligned(2)));
+typedef f32x4 f32x4_f __attribute__((aligned(4)));
+VWA_DEVICE u32x4 ld_bf8(const u16* q) { return *reinterpret_cast<const u32x4_bf*>(q); }
+VWA_DEVICE void ld_f8(const float* q, f32x4 (&v)[2]) {
+  v[0] = *reinterpret_cast<const f32x4_f*>(q);
+  v[1] = *reinterpret_cast<const f32x4_f*>(q + 4);
+}
+template <int EPI>
+VWA_DEVICE ItemRaw<EPI> item_raw(const GemmParams& p, int m, int c) {
+  ItemRaw<EPI> q;
+  const int n0 = item_src0<EPI>(c), n1 = item_src1<EPI>(c);
+  q.pos = EPI == EPI_QKV && p.use_rope ? p.positions[m] : 0;
+  q.slot = EPI == EPI_QKV ? p.slots[m] : 0;
+  q.sx = p.sx ? p.sx[m] : 1.f;
+  q.scale[0] = q.scale[1] = 0;
+  if (p.rstd || p.ss_in) {
+    const unsigned* s = p.rstd ? reinterpret_cast<const unsigned*>(p.rstd + m) : reinterpret_cast<const unsigned*>(p.ss_in + m);
+    q.scale[0] = s[0];
+    q.scale[1] = s[p.rstd ? 0 : 1];
+  }
+  q.swa[0] = q.swa[1] = q.swb[0] = q.swb[1] = f32x4{1.f, 1.f, 1.f, 1.f};
+  q.ba = q.bb = q.r0 = q.r1 = u32x4{0, 0, 0, 0};
+  if (p.sw) {
+    ld_f8(p.sw + n0, q.swa);
+    if constexpr (kTwoSrc<EPI>) ld_f8(p.sw + n1, q.swb);
+  }
+  if (ItemRaw<EPI>::kBias && p.bias) {
+    q.ba = ld_bf8(p.bias + n0);
+    if constexpr (EPI == EPI_QKV) q.bb = ld_bf8(p.bias + n1);
+  }
+  const bool wide = p.y_f32 == 2;                    // f32 residual stream: 16-byte accesses (rows are 32-byte aligned)
+  if (wide || (kResid<EPI> && !p.y_f32)) {
+    const char* r = reinterpret_cast<const char*>(p.R) + ((size_t)m * p.ldr + c) * (wide ? 4 : 2);
+    q.r0 = *reinterpret_cast<const u32x4*>(r);
+    q.r1 = *reinterpret_cast<const u32x4*>(r + (wide ? 16 : 0));
+  }
+  return q;
+}
+// ... made ready, under the slabs' loads or behind them
 template <int EPI> struct ItemPre {
   float scale, swa[8], swb[8], ba[8], bb[8];
-  u32x4 r0, r1;    // residual: 8 bf16 (r0) or f32 (vectors: as structs they went through 272 bytes of scratch a lane)
-  float4 rope[4];
+  u32x4 r0, r1;
+  f32x4 rope[4];
   int64_t slot;
 };
 template <int EPI>
-VWA_DEVICE ItemPre<EPI> item_pre(const GemmParams& p, int m, int c) {
+VWA_DEVICE ItemPre<EPI> item_ready(const GemmParams& p, const ItemRaw<EPI>& r, const f32x4 (&rope)[4]) {
   ItemPre<EPI> q;
-  const int n0 = item_src0<EPI>(c), n1 = item_src1<EPI>(c);
-  const int pos = EPI == EPI_QKV && p.use_rope ? p.positions[m] : 0;
-  q.slot = EPI == EPI_QKV ? p.slots[m] : 0;
-  const float sx = p.sx ? p.sx[m] : 1.f;
-  q.scale = row_scale(p, m) * sx;
+  unsigned lo = r.scale[0], hi = r.scale[1];
+  asm volatile("" : "+v"(lo), "+v"(hi));             // (else the conversion, and a wait, follow the loads into their branch)
+  q.scale = (p.rstd ? __uint_as_float(lo) : p.ss_in ? ss_scale(p, (unsigned long long)hi << 32 | lo) : 1.f) * r.sx;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    q.swa[e] = p.sw ? p.sw[n0 + e] : 1.f;
-    q.ba[e] = EPI == EPI_SWIGLU ? 0.f : bias_at(p, n0 + e);
-    if constexpr (kTwoSrc<EPI>) q.swb[e] = p.sw ? p.sw[n1 + e] : 1.f;
-    if constexpr (EPI == EPI_QKV) q.bb[e] = bias_at(p, n1 + e);
-  }
-  q.r0 = q.r1 = u32x4{0, 0, 0, 0};
-  if (p.y_f32 == 2) {  // f32 residual stream: 16-byte accesses (rows are 32-byte aligned)
-    const u32x4* r = reinterpret_cast<const u32x4*>(reinterpret_cast<const float*>(p.R) + (size_t)m * p.ldr + c);
-    q.r0 = r[0];
-    q.r1 = r[1];
-  } else if (kResid<EPI> && !p.y_f32) {
-    q.r0 = *reinterpret_cast<const u32x4*>(p.R + (size_t)m * p.ldr + c);
-  }
-  if (EPI == EPI_QKV && p.use_rope) {
+  for (int e = 0; e < 8; ++e) q.swa[e] = r.swa[e >> 2][e & 3], q.swb[e] = r.swb[e >> 2][e & 3];
+  unpack8(__builtin_bit_cast(uint4, r.ba), q.ba);
+  unpack8(__builtin_bit_cast(uint4, r.bb), q.bb);
+  q.r0 = r.r0;
+  q.r1 = r.r1;
+  q.slot = r.slot;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) q.rope[e] = rope_at(p, pos, c)[e];
-  }
+  for (int e = 0; e < 4; ++e) q.rope[e] = rope[e];
   return q;
 }
 
@@ -523,7 +553,10 @@ VWA_DEVICE float finish_item(const GemmParams& p, const ItemPre<EPI>& q, int m, 
     if constexpr (EPI == EPI_QKV) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) b[e] = b[e] * rs * q.swb[e] + q.bb[e];
-      qkv_store(p, m, c, v, b, q.rope, q.slot);
+      float4 rope[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) rope[e] = __builtin_bit_cast(float4, q.rope[e]);
+      qkv_store(p, m, c, v, b, rope, q.slot);
       return 0.f;
     }
   }
@@ -577,14 +610,30 @@ VWA_DEVICE void ss_add(unsigned long long* ss_out, int m, float sq) {
   }
 }
 
+// Few rows: everything the item reads is in flight together, the rotary row behind its position.  (With the scale, the bias and the
+// rotary row each waited for ahead of the slabs, us of the launch: 8 rows of 1280 columns with bias and residual 5.0 -> 4.0, 32 rows of
+// 4096, 8 slices, 5.0 -> 4.7, of 6144 with the rotation 5.0 -> 4.8.)
 template <int EPI, int AUX, int ZB>
 VWA_DEVICE float reduce_item(const GemmParams& p, __amdgpu_buffer_rsrc_t rws, int m, int c) {
-  const int cc[1] = {c};
-  const bool ok[1] = {true};
-  float a[1][8], b[1][8];
-  const ItemPre<EPI> q = item_pre<EPI>(p, m, c);
-  sum_items<EPI, AUX, 1, ZB>(p, rws, m, cc, ok, a, b);
-  return finish_item<EPI>(p, q, m, c, a[0], b[0]);
+  float a[8] = {}, b[8] = {};
+  const ItemRaw<EPI> q = item_raw<EPI>(p, m, c);
+  ItemSlabs<EPI, AUX, ZB> s;
+  s.load(p, rws, m, c, 0);
+  asm volatile("" ::: "memory");
+  f32x4 rope[4] = {};
+  if (EPI == EPI_QKV && p.use_rope) {
+    const f32x4* at = reinterpret_cast<const f32x4*>(rope_at(p, q.pos, c));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rope[e] = at[e];
+    asm volatile("" ::: "memory");
+  }
+  const ItemPre<EPI> pre = item_ready<EPI>(p, q, rope);
+  s.add(a, b);
+  for (int z0 = ZB; z0 < p.splits; z0 += ZB) {
+    s.load(p, rws, m, c, z0);
+    s.add(a, b);
+  }
+  return finish_item<EPI>(p, pre, m, c, a, b);
 }
 
 // (a 4-stage variant for one-row-block GEMMs measured slower in whole decode steps -- 128 KB
@@ -1101,8 +1150,9 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmParams p) {
   const bool ok = id < (int64_t)p.M * cpr;
   const __amdgpu_buffer_rsrc_t rws = rsrc(p.ws, (size_t)p.splits * p.M * p.N * 4);
   float sq = 0.f;
-  if (ok) sq = reduce_item<EPI, 0, ZB>(p, rws, (int)(id / cpr), (int)(id % cpr) * 8);
-  if (kResid<EPI> && p.ss_out) ss_add(p.ss_out, ok ? (int)(id / cpr) : -1, sq);
+  const int m = (int)((unsigned)id / (unsigned)cpr);  // (M N fits 32-bit slab offsets)
+  if (ok) sq = reduce_item<EPI, 0, ZB>(p, rws, m, (int)((unsigned)id - (unsigned)m * cpr) * 8);
+  if (kResid<EPI> && p.ss_out) ss_add(p.ss_out, ok ? m : -1, sq);
 }
 
 // per-row 1/rms of X (the RMSNorm of a projection whose gamma is folded into W)
