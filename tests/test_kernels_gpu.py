@@ -207,6 +207,33 @@ def test_norms():
         close(y, y2, 3e-2)
 
 
+@pytest.mark.parametrize("D", [8, 504, 520, 1024, 1280, 2048, 2056, 4096, 4104, 8192])
+@pytest.mark.parametrize("rows", [1, 5])
+def test_layernorm_of_any_width(rows, D):
+    """Every number of 512-column steps a row is held in, whole and not, with a residual (also in place) and without."""
+    x, r, w, b = rnd(rows, D), rnd(rows, D), rnd(D), rnd(D)
+    y = torch.empty_like(x)
+    ops.ext().layernorm(x, None, None, w, b, y, 1e-5)
+    ln = lambda v: torch.nn.functional.layer_norm(v, (D,), w.double(), b.double(), 1e-5)  # noqa: E731
+    want = ln(x.double())
+    assert ((y.double() - want).abs() <= 2.0**-8 * want.abs() + 1e-5 * want.abs().max()).all()  # (half a bf16 ulp, f32 sums)
+    s, out = x.double() + r.double(), r.clone()
+    ops.ext().layernorm(x, out, out, w, b, y, 1e-5)
+    want = ln(s)
+    assert torch.equal(out, (x.float() + r.float()).bfloat16())
+    assert ((y.double() - want).abs() <= 2.0**-8 * want.abs() + 1e-5 * want.abs().max()).all()  # (of the sum before it is rounded)
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 1280, 5120), (40, 2048, 4096)])
+def test_a_sum_of_slices_reads_its_bias_where_it_lies(M, N, K):
+    """The bias as a part of another tensor, aligned as its elements only: the bits of an aligned copy."""
+    x, w, r, b = rnd(M, K), ops.TiledWeight(rnd(N, K, scale=K**-0.5)), rnd(M, N), rnd(N + 8)
+    assert ops.ext().gemm_plan(0, M, N, K)[1] > 1
+    for at in (1, 2, 5):
+        got = [ops.linear(x, w, bias=v, residual=r, out=torch.empty(M, N, dtype=BF, device=DEV)) for v in (b[at : at + N], b[at : at + N].clone())]
+        assert torch.equal(*got)
+
+
 def test_gelu_of_every_value():
     """x Phi(x) of every 16-bit value against 64 bits: half a unit in the last place of the result (8 bits: 2^-8 of it at most),
     beside it 32-bit arithmetic -- the tail's exponent, 130 in powers of two at most, rounded twice: 130 ln 2 2^-23 = 1.1e-5 -- and
