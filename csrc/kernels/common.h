@@ -177,6 +177,8 @@ VWA_DEVICE int lane_id() { return threadIdx.x & 63; }
 VWA_DEVICE int small_div(int x, int k) {
   return __builtin_amdgcn_readfirstlane((int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)k)));
 }
+// ... of each lane's
+VWA_DEVICE int lane_div(int x, int k) { return (int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)k)); }
 
 // The workitem id through an empty volatile asm: every use is a fresh value, so address math
 // derived from it cannot be hoisted out of an enclosing loop.  The chained decode kernels read

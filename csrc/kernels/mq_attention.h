@@ -146,7 +146,11 @@ inline __host__ __device__ float mq_cascade_keys(int P, int groups, int pre, int
 }
 // Prefix chunks where every run of a group has an own chunk (gh: row groups x kv heads)
 inline __host__ __device__ int mq_prefix_chunks(int n_splits, int RG, int gh) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const int wide = small_div(kMqCus, gh) - RG, half = small_div(kMqCus / 2, gh), n = wide > half ? wide : half, most = n_splits - RG;
+#else
   const int wide = kMqCus / gh - RG, half = kMqCus / 2 / gh, n = wide > half ? wide : half, most = n_splits - RG;
+#endif
   return n < 1 || most < 1 ? 1 : n < most ? n : most;
 }
 // Own keys of a run behind one wave of NW, as a chunk's
@@ -230,7 +234,16 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       plan = __builtin_amdgcn_readlane(ev, 2) != 3 && __builtin_amdgcn_readlane(ev, 10) == p.rows;
     }
   }
-  if (w == 0 && !plan) {
+  int sl = -1, cl = 0;  // lane: row's sequence and context
+  if constexpr (!FINE) {  // (every wave for itself: no LDS and barrier behind the round trip)
+    const __amdgpu_buffer_rsrc_t r_sid =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(p.seq_ids), (short)0, p.rows * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r_ctx =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(p.ctx_lens), (short)0, p.rows * 4, 0x00020000);
+    const int sv = (int)__builtin_amdgcn_raw_buffer_load_b32(r_sid, lane * 4, 0, 0);
+    cl = (int)__builtin_amdgcn_raw_buffer_load_b32(r_ctx, lane * 4, 0, 0);
+    sl = lane < p.rows ? sv : -1;
+  } else if (w == 0 && !plan) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       *reinterpret_cast<int2*>(s_meta + r * 128 + 2 * lane) = __builtin_bit_cast(
@@ -242,29 +255,31 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
         __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(p.ctx_lens), (short)0, p.rows * 4, 0x00020000);
     s_meta[512 + lane] = (int)__builtin_amdgcn_raw_buffer_load_b32(r_sid, lane * 4, 0, 0);
     s_meta[576 + lane] = (int)__builtin_amdgcn_raw_buffer_load_b32(r_ctx, lane * 4, 0, 0);
-    if constexpr (!FINE) {
-      const __amdgpu_buffer_rsrc_t r_sh =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(p.shared), (short)0, p.shared ? 8 : 0, 0x00020000);
-      if (lane < 2) s_meta[640 + lane] = (int)__builtin_amdgcn_raw_buffer_load_b32(r_sh, lane * 4, 0, 0);
-    }
   }
-  if (!plan) {
+  if (FINE && !plan) {
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; ++r) rt[r] = *reinterpret_cast<const int2*>(s_meta + r * 128 + 2 * lane);
   }
   stamp(12);  // (diagnostic: step metadata in LDS / the plan entry in registers)
-  const int sl = plan ? -1 : lane < p.rows ? s_meta[512 + lane] : -1;
-  const int cl = plan ? 0 : lane < p.rows ? s_meta[576 + lane] : 0;
+  if constexpr (FINE) {
+    sl = plan ? -1 : lane < p.rows ? s_meta[512 + lane] : -1;
+    cl = plan ? 0 : lane < p.rows ? s_meta[576 + lane] : 0;
+  }
   stamp(16);
-  const int sp = __shfl(sl, lane > 0 ? lane - 1 : 0, 64);
+  const int sp = FINE ? __shfl(sl, lane > 0 ? lane - 1 : 0, 64)
+                      : __builtin_amdgcn_update_dpp(-2, sl, 0x138, 0xF, 0xF, false);  // (wave_shr: from the lane below)
   const unsigned long long seq_starts = __ballot(lane < p.rows && (lane == 0 || sl != sp));
   // shared cached prefix (p.shared): rows 0 .. n_real-1 are grouped RG at a time regardless of
   // sequence (their first P keys are the same blocks), the padded rows behind them by sequence
   int P = 0, n_real = p.rows;
   if constexpr (!FINE) {
-    P = s_meta[640];
-    n_real = min(p.rows, s_meta[641]);
+    if (p.shared) {
+      P = __builtin_amdgcn_readfirstlane(p.shared[0]);
+      n_real = min(p.rows, __builtin_amdgcn_readfirstlane(p.shared[1]));
+    } else {
+      n_real = 0;
+    }
   }
   const bool cascade = !FINE && P > 0 && n_real > 0 && p.n_splits > RG;
   unsigned long long run_starts = seq_starts;
@@ -300,10 +315,10 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       // the CUs, 256 are one, and the merge reads four partials instead of six), 48 of ~110 25.1 -> 20.0, 64 of ~100 27.1 -> 20.6,
       // 24 of ~150 19.7 -> 16.1; 32 of ~400 (kept as they were) 28.2 / 27.4.
       const int gr = (n_real + RG - 1) / RG * nkv;
-      const int own = (int)wave_max(lane < n_real ? (float)max(cl - P, 0) : 0.f);
+      const int own = __builtin_amdgcn_readfirstlane((int)wave_max(lane < n_real ? (float)max(cl - P, 0) : 0.f));
       auto keys = [&](int pre, int n_own, int own_len) { return mq_cascade_keys(P, gr, pre, n_own, own_len, kChunk, D); };
       const float cost = keys(min(lane + 1, p.n_splits - 1), 1, mq_run_keys(own, NW));
-      const float best = -wave_max(-cost);
+      const float best = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(-wave_max(-cost))));
       wave_runs = best < kMqRunsAhead * keys(n_pc, RG, (own + kChunk - 1) / kChunk * kChunk);
       if (wave_runs) {
         n_pc = min(__builtin_ctzll(__ballot(cost == best)) + 1, p.n_splits - 1);
@@ -317,13 +332,13 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     // 20 heads of D = 64 x 1500 keys, 1 row 16.1 / 12.6 / 11.3 / 9.9 / 10.4 and 8 rows 21.3 / 22.5 /
     // 19.7; 8 kv heads of D = 128 x 1110 keys, 4 rows 19.0 / 15.5 / 12.9 / 12.9 / 11.8 and 16 rows
     // 23.2 / 21.0 / 27.1
-    const int ctx_all = (int)wave_max((float)cl);
+    const int ctx_all = __builtin_amdgcn_readfirstlane((int)wave_max((float)cl));
     const int c = min(lane + 1, p.n_splits);
-    const int len = ((ctx_all + c - 1) / c + kChunk - 1) / kChunk * kChunk;
-    const int cnt = len > 0 ? (ctx_all + len - 1) / len : 1;
+    const int len = (lane_div(ctx_all + c - 1, c) + kChunk - 1) / kChunk * kChunk;
+    const int cnt = len > 0 ? lane_div(ctx_all + len - 1, len) : 1;
     const int per_cu = (gh * cnt + kMqCus - 1) / kMqCus;
     const int cost = per_cu * len + (cnt > 1 ? cnt * (D == 64 ? 70 : 30) : 0) + (per_cu - 1) * (D == 64 ? 100 : 350);
-    const float best = wave_max(-(float)cost);
+    const float best = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(-(float)cost))));
     n_eff = __builtin_ctzll(__ballot((float)cost == -best)) + 1;
   }
   const int n_items = plan ? __builtin_amdgcn_readlane(ev, 0) : n_groups * nkv * n_eff;
@@ -355,8 +370,17 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     __syncthreads();
     if (VWA_TX == 0) __hip_atomic_fetch_add(gp(done), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
+  const int lane_of = lane;
   for (int item = bid; item < n_items; item += grid) {
   if (item == bid) stamp(18);
+  // (standalone: mostly the only item.  What is formed from the lane's number was formed in front of the loop, 390 instructions of one
+  // wave, 0.8 us ahead of the first load; so it is where it is used, under the loads.  With the step's rows read by every wave, without
+  // LDS and a barrier, and divisions by reciprocals the first keys are asked for 3.4 us after the start instead of 4.5.  us of a launch in
+  // a model's step: 8 rows x 20 heads of 64, 1500 keys 16.5 -> 15.8, their own keys 5.6 -> 4.8; 32 sessions x 8 kv heads of 128 behind
+  // 1008 shared keys 17.1 -> 16.8)
+  int lane = lane_of;
+  if constexpr (!FINE) asm volatile("" : "+v"(lane));
+  const int n = lane & 15, g = lane >> 4;
   int kvh, r0, nr, CL, kbeg, kend, nact, slot, kv_seq, ctx_n;
   bool own_run = false;  // [kbeg, kend) are this wave's alone
   const int rho = n / G;  // group row of this lane's query column
@@ -375,25 +399,37 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     ctx_n = rho < nr ? c_rho : 0;
   } else {
   // item -> (kv head, group, chunk); kv head fastest so a head's workgroups share one XCD (b % 8)
-  kvh = item % nkv;
-  const int gi = (item / nkv) % n_groups, chunk = item / (nkv * n_groups);
+  int gi, chunk;
+  if constexpr (FINE) {
+    kvh = item % nkv;
+    gi = (item / nkv) % n_groups, chunk = item / (nkv * n_groups);
+  } else {
+    const int ig = small_div(item, nkv);
+    kvh = item - ig * nkv;
+    chunk = small_div(ig, n_groups);
+    gi = ig - chunk * n_groups;
+  }
   const unsigned long long pick = __ballot(((leaders >> lane) & 1ull) && my_rank == gi);
   r0 = __builtin_ctzll(pick);
   const unsigned long long later = run_starts & ~((2ull << r0) - 1ull);
   const int run_end = later ? __builtin_ctzll(later) : p.rows;
   nr = min(RG, run_end - r0);  // rows in this group
-  const int seq = __shfl(sl, r0, 64);
+  const int seq = FINE ? __shfl(sl, r0, 64) : __builtin_amdgcn_readlane(sl, r0);
   if (item == bid) stamp(11);  // (diagnostic: before the item's barrier)
-  __syncthreads();  // the previous item's LDS readers are done
+  if (FINE || item != bid) __syncthreads();  // the previous item's LDS readers are done
   if (item == bid) stamp(9);  // step rows / contexts known
-  const int c_src = __shfl(cl, min(r0 + lane, 63), 64);
-  const int c_own = lane < nr ? c_src : 0;
+  int c_own = 0;
+  if constexpr (FINE) {
+    const int c_src = __shfl(cl, min(r0 + lane, 63), 64);
+    c_own = lane < nr ? c_src : 0;
+  }
   int ctxmax = 0;  // (scalars: lane shuffles here and below were 0.3 us of every workgroup's start)
 #pragma unroll
   for (int r = 0; r < RG; ++r) ctxmax = r < nr ? max(ctxmax, __builtin_amdgcn_readlane(cl, min(r0 + r, 63))) : ctxmax;
   if (item == bid) stamp(19);
-  ctx_n = __shfl(c_own, rho, 64);  // its context (0 for padded columns)
+  ctx_n = FINE ? __shfl(c_own, rho, 64) : __shfl(cl, min(r0 + min(rho, nr - 1), 63), 64);  // its context (0 for padded columns)
 
+  if (!FINE && rho >= nr) ctx_n = 0;
   // ---- this item's chunk of the group's keys (NW waves x CL/NW keys): [kbeg, kend), partial slot
   slot = chunk;
   kv_seq = seq;
@@ -413,8 +449,8 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       if (c > P) own_mask |= 1 << run;
       if (run == j) my_max = max(my_max, c);
     }
-    CL = ((P + n_pc - 1) / n_pc + kChunk - 1) / kChunk * kChunk;
-    const int npa = (P + CL - 1) / CL;
+    CL = (small_div(P + n_pc - 1, n_pc) + kChunk - 1) / kChunk * kChunk;
+    const int npa = small_div(P + CL - 1, CL);
     nact = npa + (wave_runs ? own_mask != 0 : __builtin_popcount(own_mask));
     if (chunk < n_pc) {
       kbeg = chunk * CL;
@@ -438,11 +474,11 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       CL = (kend - kbeg + kChunk - 1) / kChunk * kChunk;
       own_run = wave_runs;
       slot = npa + (wave_runs ? 0 : __builtin_popcount(own_mask & ((1 << j) - 1)));
-      kv_seq = __shfl(sl, a, 64);
+      kv_seq = __builtin_amdgcn_readlane(sl, a);
       if (rho < a - r0 || rho >= b - r0) ctx_n = 0;  // other runs' columns: no keys in this chunk
     }
   } else {
-    CL = ((ctxmax + n_eff - 1) / n_eff + kChunk - 1) / kChunk * kChunk;
+    CL = ((FINE ? (ctxmax + n_eff - 1) / n_eff : small_div(ctxmax + n_eff - 1, n_eff)) + kChunk - 1) / kChunk * kChunk;
     if (cascade) CL = (ctxmax + kChunk - 1) / kChunk * kChunk;  // padded rows: one chunk
     kbeg = chunk * CL;
     if (kbeg >= ctxmax) {
@@ -450,7 +486,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       continue;
     }
     kend = min(ctxmax, kbeg + CL);
-    nact = (ctxmax + CL - 1) / CL;
+    nact = FINE ? (ctxmax + CL - 1) / CL : small_div(ctxmax + CL - 1, CL);
   }
   if (item == bid) write_plan(cascade ? 3 : 1, kvh, r0, nr, kbeg, kend, nact, slot, c_own);
   }  // (metadata path)
@@ -474,7 +510,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   int64_t tabA = 0, tabB = 0;
   auto load_tab = [&](int s0) {
     const int ka = min(wb + (s0 + lane) * kMqStep, kmax), kb = min(ka + 16, kmax);
-    const int ia = ka / bs, ib = kb / bs;
+    const int ia = lane_div(ka, bs), ib = lane_div(kb, bs);
     gint* tab = (gint*)(p.kv.block_table + (int64_t)kv_seq * p.kv.table_stride);
     const int ba = tab[ia], bb = tab[ib];
     tabA = ba * p.kv.stride_block + (ka - ia * bs) * p.kv.stride_tok;
