@@ -398,6 +398,24 @@ def test_mingru(dtype, W):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [32, 33, 512, 513, 545, 1056, 1300])
+def test_mingru_folds_the_chunks_in_front(dtype, n):
+    """Runs of one to forty-one chunks, sixteen of which are folded together, behind another run's; slow channels, whose state spans them."""
+    W, first = 40, 70
+    z, x, g = rnd(first + n, W, seed=1, std=2, dtype=dtype), rnd(first + n, W, seed=2, dtype=dtype), rnd(first + n, W, seed=3, dtype=dtype)
+    zb, xb, st0 = rnd(W, seed=4) - 6.0, rnd(W, seed=5), rnd(2, W, seed=6, std=5.0)
+    S = O.min_gru(z[first:].double() + zb.double(), x[first:].double() + xb.double(), st0[1].double())
+    want = S * O.silu(g[first:].double())
+    ids = torch.cat([torch.zeros(first), torch.ones(n)]).int().to(DEV)
+    pos = torch.cat([torch.arange(first), torch.arange(9, 9 + n)]).int().to(DEV)
+    st, out = st0.clone().to(DEV), torch.zeros(first + n, W, dtype=dtype, device=DEV)
+    y = torch.cat([z, x, g], 1).to(DEV)
+    ops.mingru(y[:, :W], y[:, W : 2 * W], y[:, 2 * W :], zb.to(DEV), xb.to(DEV), seq_ids=ids, positions=pos, slots=pos.long(), state=st,
+               out_scale=1.0, out=out, plan=ops.plan_runs([(0, first), (first, n)], DEV, 2000))
+    assert rel(out[first:], want) < (1e-5 if dtype == F32 else 8e-3) and rel(st[1], S[-1]) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,G,dk,dv,rot,window,keep,bs", [
     (8, 4, 128, 128, 64, 1024, 4, 16),
     (6, 2, 32, 48, 16, 33, 3, 16),        # half of a fragment step rotates
