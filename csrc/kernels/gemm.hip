@@ -646,9 +646,12 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   static_assert(!GRP || (WT && !F8 && !W8 && (EPI == EPI_SWIGLU || EPI == EPI_STORE)), "grouped: tiled bf16");
   const int mb = GRP ? p.g_tiles[0] : (p.M + C::BM - 1) / C::BM, nb = (p.N + C::BN - 1) / C::BN;
   const int tiles = mb * nb;
-  const int split = blockIdx.x / tiles % p.splits;  // split-K slice (blocks of one slice are contiguous)
-  if (p.nbatch > 1) {  // batch z = blockIdx.x / (tiles * splits), splits == 1 (vwa_gemm)
-    const int z = blockIdx.x / tiles;
+  // (few rows' launches are over in 8 us, and the compiler's divisions are a chain of 25 operations each in front of the first load)
+  const bool small = gridDim.x < (1u << 21);
+  const int part = gridDim.x == (unsigned)tiles ? 0 : small ? small_div(blockIdx.x, tiles) : blockIdx.x / tiles;
+  const int split = p.nbatch > 1 ? 0 : part;  // split-K slice (blocks of one slice are contiguous)
+  if (p.nbatch > 1) {  // batch z = blockIdx.x / tiles, splits == 1 (vwa_gemm)
+    const int z = part;
     p.X += (size_t)z * p.bsx;
     p.Y = reinterpret_cast<char*>(p.Y) + (size_t)z * p.bsy * (p.y_f32 ? 4 : 2);
     if (p.R) p.R += (size_t)z * p.bsr;
@@ -658,15 +661,16 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   if (p.ss_zero && blockIdx.x == 0)
     for (int i = threadIdx.x; i < p.ss_zero_n; i += C::THREADS) p.ss_zero[i] = 0ull;
   if (GRP && (int)blockIdx.x >= tiles) return;       // (the grid is sized for the most row blocks there can be)
-  const int lt = xcd_remap((int)(blockIdx.x % tiles), tiles);
+  const int lt = xcd_remap((int)blockIdx.x - part * tiles, tiles);
   // (grouped: column blocks of kGroup row blocks -- mostly one expert's -- after one another)
   const int band = GRP ? lt / (kGroup * nb) * kGroup : 0, bh = GRP ? min(kGroup, mb - band) : mb, bt = lt - band * nb;
-  const int bn = (bt / bh) * C::BN;
-  int bm = (bt % bh) * C::BM, place = 0;
+  const int col = bh == 1 ? bt : small ? small_div(bt, bh) : bt / bh, row = bt - col * bh;
+  const int bn = col * C::BN;
+  int bm = row * C::BM, place = 0;
   int rows[C::BM / 8 / C::NW];
   size_t x_rows = 0;
   if constexpr (GRP) {
-    const int gt = band + bt % bh;
+    const int gt = band + row;
     p.W += (size_t)p.g_tiles[1 + 3 * gt] * p.g_wstride;
     place = p.g_tiles[2 + 3 * gt];
     x_rows = (size_t)p.M;                            // (X rows the buffer holds)
