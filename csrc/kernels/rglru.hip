@@ -686,9 +686,12 @@ template <class T>
 int launch_rows(const RgLruParams& p, hipStream_t st) {
   if (u_bytes<T>(16, p.bs) > kMaxLds) return -10;
   const int tiles = p.bs / 16, parts = p.tickets ? row_parts(p.bs, sizeof(T)) : 1, tper = (tiles + parts - 1) / parts;
-  const int form = (16 * (p.bs / 4) + 63) / 64, gates = tper <= 4 ? 2 * tper : tper < 8 ? tper : 8;
+  const int form = (16 * (p.bs / 4) + 63) / 64;
+  // (the gates' meeting place takes 4 KB: blocks whose u fills LDS without it keep both gates in a wave)
+  const bool split = tper <= 4 && u_bytes<T>(16, p.bs) + 6144 <= 160 * 1024;
+  const int gates = split ? 2 * tper : tper < 8 ? tper : 8;
   const dim3 grid(p.nb, (p.rows + 15) / 16, parts), block(64 * (gates + (form < 8 ? form : 8)));
-  if (tper <= 4) hipLaunchKernelGGL((rglru_rows_kernel<T, true>), grid, block, u_bytes<T>(16, p.bs), st, p);
+  if (split) hipLaunchKernelGGL((rglru_rows_kernel<T, true>), grid, block, u_bytes<T>(16, p.bs), st, p);
   else hipLaunchKernelGGL((rglru_rows_kernel<T, false>), grid, block, u_bytes<T>(16, p.bs), st, p);
   return (int)hipGetLastError();
 }

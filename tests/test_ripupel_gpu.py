@@ -153,10 +153,10 @@ def test_rglru(dtype, W, nb, taps, lens):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("W,nb,taps", [(512, 2, 4), (256, 4, 3), (320, 1, 4), (512, 1, 5)])
+@pytest.mark.parametrize("W,nb,taps", [(512, 2, 4), (256, 4, 3), (320, 1, 4), (512, 1, 5), (2496, 1, 2)])
 def test_rglru_decoded_rows(dtype, W, nb, taps):
     """One row of every sequence, as many as a thread takes one or two of (8, 16 of 256 channels), into the next tile; a block's parts and one
-    workgroup: the same bits as every row alone, whose results test_rglru has, and an inert row among them."""
+    workgroup: the same bits as every row alone, whose results test_rglru has, and an inert row among them.  2496 channels fill LDS in 32 bits."""
     _, p, _ = rglru_case(W, nb, taps, dtype)
     for rows in (1, 4, 5, 8, 9, 16, 17):
         yx = rnd(rows, 2 * W, seed=rows, dtype=dtype).to(DEV)
