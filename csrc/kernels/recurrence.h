@@ -14,6 +14,9 @@ struct Gate {
 VWA_DEVICE Gate min_gru_gate(float zp, float u) {
   return Gate{sigm(zp), u >= 0.f ? u + 0.5f : sigm(u)};
 }
+// (1 - z) S + z c with one product rounded before the sum.  Written out: which one it is was the compiler's choice, and code around it
+// changed the choice and with it the bits of whole answers.
+VWA_DEVICE float min_gru_step(const Gate& g, float S) { return fmaf(1.f - g.z, S, g.z * g.c); }
 
 // Rows form of one (row, channel): the head row of a run of its sequence walks the run.  A decoded row is three round trips long:
 // the ids of the row and its neighbours with its projections, the state, the results.
@@ -41,7 +44,7 @@ VWA_DEVICE void mingru_row(const MinGruParams& p, int r0, int ch) {
   float S = pos > 0 ? *st : 0.f;
   for (int r = r0;;) {
     const Gate gt = min_gru_gate(ldv(&zv) + zb, ldv(&xv) + xb);
-    S = (1.f - gt.z) * S + gt.z * gt.c;
+    S = min_gru_step(gt, S);
     stv(out + (size_t)r * p.ldo + ch, S * silu(ldv(&gv)) * p.out_scale);
     if (++r == p.rows || seq_next != seq || slot_next < 0) break;
     const size_t o = (size_t)r * p.ld;

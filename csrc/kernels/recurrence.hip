@@ -29,10 +29,12 @@ constexpr int kFold = 16;      // chunks in front that are folded together
 
 // PASS 1: per (chunk, channel) A = prod (1 - z), B = the chunk's end state from a zero start
 // PASS 2: outputs (and the state of a run's last chunk)
+// PAIRS (even widths whose columns pair up to a load): z c is added unrounded, else (1 - z) S (min_gru_step); the two were different kernels
+// once, and their results stay what they were.
 // A thread a channel.  Bound by a chunk's chain of rows and, with many chunks, by the exact exponentials and divisions of the gates: what
 // counts is threads.  us of both passes, two channels a thread (and the chunks in front by sixteens, the rest of them one by one) ->
 // here: 777 rows x 1024 in 32 bits 33.3 -> 16.5, 200 x 2048 in 16 bits 26.9 -> 17.4, 2048 x 4096 57 -> 42.5, 7200 x 1024 (pass 2) 24.8 -> 16.8.
-template <class T, int PASS>
+template <class T, int PASS, bool PAIRS>
 __global__ __launch_bounds__(256) void mingru_scan_kernel(MinGruParams p) {
   const int ck = blockIdx.y, ch = blockIdx.x * 256 + threadIdx.x;
   if (ch >= p.width) return;
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(256) void mingru_scan_kernel(MinGruParams p) {
       if (t0 + t >= n) break;
       const Gate gt = min_gru_gate(bz[q][t] + zb, bx[q][t] + xb);
       A *= 1.f - gt.z;
-      S = (1.f - gt.z) * S + gt.z * gt.c;
+      S = PAIRS ? fmaf(gt.z, gt.c, (1.f - gt.z) * S) : min_gru_step(gt, S);
       if (PASS == 2) stv(out + (size_t)(t0 + t) * p.ldo, S * silu(bg[q][t]) * p.out_scale);
     }
   };
@@ -98,11 +100,11 @@ __global__ __launch_bounds__(256) void mingru_scan_kernel(MinGruParams p) {
   }
 }
 
-template <class T>
+template <class T, bool PAIRS>
 void launch_scan(const MinGruParams& p, hipStream_t st) {
   const dim3 grid((p.width + 255) / 256, p.n_chunks), block(256);
-  hipLaunchKernelGGL((mingru_scan_kernel<T, 1>), grid, block, 0, st, p);
-  hipLaunchKernelGGL((mingru_scan_kernel<T, 2>), grid, block, 0, st, p);
+  hipLaunchKernelGGL((mingru_scan_kernel<T, 1, PAIRS>), grid, block, 0, st, p);
+  hipLaunchKernelGGL((mingru_scan_kernel<T, 2, PAIRS>), grid, block, 0, st, p);
 }
 
 }  // namespace
@@ -117,6 +119,10 @@ extern "C" int vwa_mingru_rows(const MinGruParams* p, hipStream_t st) {
 
 extern "C" int vwa_mingru_scan(const MinGruParams* p, hipStream_t st) {
   if (p->rows < 1 || p->width < 1 || p->n_chunks < 1 || !p->chunks || !p->cA || !p->cB || !p->cS) return -1;
-  p->f32 ? launch_scan<float>(*p, st) : launch_scan<u16>(*p, st);
+  const uintptr_t al = p->f32 ? 7 : 3;
+  const bool pairs = p->width % 2 == 0 && p->ld % 2 == 0 && !((reinterpret_cast<uintptr_t>(p->z) | reinterpret_cast<uintptr_t>(p->x) |
+                                                               reinterpret_cast<uintptr_t>(p->g)) & al);
+  if (p->f32) pairs ? launch_scan<float, true>(*p, st) : launch_scan<float, false>(*p, st);
+  else pairs ? launch_scan<u16, true>(*p, st) : launch_scan<u16, false>(*p, st);
   return (int)hipGetLastError();
 }

@@ -416,6 +416,34 @@ def test_mingru_folds_the_chunks_in_front(dtype, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("W,first,pairs", [(256, 0, True), (255, 0, False), (256, 1, False)])
+def test_mingru_rounds_one_product(dtype, W, first, pairs):
+    """(1 - z) S + z c, bit for bit: of the scan over columns that pair up z c is added unrounded, else and of decoded rows (1 - z) S.
+    The gates themselves come from rows that start at c = 1: S = z."""
+    n = 20
+    y = rnd(n, 3 * W + first, seed=1, dtype=dtype)
+    y[:, first + W : first + 2 * W] = y[:, first + W : first + 2 * W].abs()  # (u >= 0: c = u + 1/2)
+    one = y.clone()
+    one[:, first + W : first + 2 * W] = 0.5
+    cols = lambda t: [t.to(DEV)[:, first + i * W : first + (i + 1) * W] for i in range(3)]  # noqa: E731
+    none = torch.zeros(W, device=DEV)
+    row = torch.arange(n, dtype=torch.int32, device=DEV)
+    out = torch.empty(n, W, dtype=dtype, device=DEV)
+    z = torch.zeros(n, W, device=DEV)
+    ops.mingru(*cols(one), none, none, seq_ids=row, positions=torch.zeros_like(row), slots=row.long(), state=z, out_scale=1.0, out=out)
+    z, c, st0 = z.cpu().numpy(), y[:, first + W : first + 2 * W].float().numpy() + np.float32(0.5), rnd(1, W, seed=2)
+    for plan in (None, ops.plan_runs([(0, n)], DEV, 100)):
+        st = st0.clone().to(DEV)
+        ops.mingru(*cols(y), none, none, seq_ids=torch.zeros_like(row), positions=row + 5, slots=row.long(), state=st, out_scale=1.0, out=out, plan=plan)
+        S = st0[0].numpy()
+        for t in range(n):  # (64 bits of significand hold either sum)
+            a, b = (np.float32(1) - z[t], S), (z[t], c[t])
+            exact, rounded = (b, a) if plan is not None and pairs else (a, b)
+            S = (np.multiply(*exact, dtype=np.longdouble) + (rounded[0] * rounded[1]).astype(np.longdouble)).astype(np.float32)
+        assert np.array_equal(st[0].cpu().numpy(), S)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,G,dk,dv,rot,window,keep,bs", [
     (8, 4, 128, 128, 64, 1024, 4, 16),
     (6, 2, 32, 48, 16, 33, 3, 16),        # half of a fragment step rotates
