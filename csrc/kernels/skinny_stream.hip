@@ -561,6 +561,7 @@ extern "C" void vwa_skinny_set_x_skew(int skew) { g_x_skew = skew == 0 ? 0 : 32;
 extern "C" int vwa_skinny_stream(int epi, const SkinnyParams* p, int grid_cap, int ks, hipStream_t st) {
   if (p->M < 1 || p->M > 16 || p->K % 128 != 0) return -10;
   if ((size_t)p->N * p->K * (p->w_scale ? 1 : 2) >= 0x7FFFFFF0ull) return -10;
+  if (p->N < (epi == EPI_SWIGLU ? 32 : 16) || grid_cap < 1) return -2;  // (no tile: launch_v deals the tiles over the grid)
 #ifdef VWA_ONLY_MULTI
   const int r = -10;
 #else

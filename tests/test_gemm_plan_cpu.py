@@ -1,4 +1,5 @@
 """Which tile and how many K slices the GEMM takes (gemm.hip): a rule on sizes, types and the diagnostic switches, no launch."""
+import ctypes
 import os
 
 import pytest
@@ -143,3 +144,15 @@ def test_a_residual_in_32_bits_keeps_its_slices(E):
                 assert got[1] > 1 or one[1] == 1, (M, N, K, got, one)
                 grouped += got[2] == 2 and got != whole
     assert grouped and E.gemm_choice(1, 2048, 1024, 2048)[1] == 1 and E.gemm_choice(1, 2048, 1024, 2048, y_f32=2)[1] == 2
+
+
+@pytest.mark.parametrize("epi,N,cap", [(0, 8, 256), (1, 15, 256), (2, 16, 256), (2, 31, 256), (0, 64, 0)])
+def test_streaming_of_less_than_a_tile_is_an_error(E, epi, N, cap):
+    """A weight of fewer rows than a tile, or a grid of none, is refused with a code ahead of the launch, which divides by the grid."""
+
+    class Params(ctypes.Structure):  # (the first fields of SkinnyParams; the others are zero)
+        _fields_ = [("X", ctypes.c_void_p), ("ldx", ctypes.c_int), ("W", ctypes.c_void_p), ("M", ctypes.c_int), ("N", ctypes.c_int),
+                    ("K", ctypes.c_int), ("rest", ctypes.c_char * 448)]
+
+    lib, p = ctypes.CDLL(build.KERNEL_SO), Params(X=1 << 20, ldx=1024, W=1 << 20, M=1, N=N, K=1024)
+    assert [lib.vwa_skinny_stream(epi, ctypes.byref(p), cap, ks, None) for ks in (4, 8)] == [-2, -2]
