@@ -333,16 +333,16 @@ __global__ __launch_bounds__(256, 2) void latent_attn_kernel(LatentAttnParams p)
 // in flight over the softmax.  4 rows x 8 heads x 140 keys, rank 512: 25.3 -> 13.9 us (144 + 128
 // MFMAs of a wave: 3.6); 64 rows x 1000 keys 161 -> 55.
 constexpr int kKeyPre = 12;
-// EXACT: rank_p = 64 NT and rot_p 64: the columns at constant offsets of a key's first, and as many steps as there are known to the
-// compiler (a load behind a condition is waited for with everything behind it)
-template <int NT, bool EXACT>
+// EXACT: rank_p = 64 NT, the value columns at constant offsets of a key's first.  ROT64: rot_p 64 as well, as many steps as there are known
+// to the compiler (a load behind a condition is waited for with everything behind it)
+template <int NT, bool EXACT, bool ROT64>
 __global__ __launch_bounds__(256, EXACT && NT <= 8 ? 2 : 1) void latent_attn_f32_kernel(LatentAttnParams p) {
   using M = MM<float>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float s_max[2][4][16];
   Item x;
   if (!attn_item(p, x)) return;
-  const int dk = EXACT ? 64 * NT + 64 : p.rank_p + p.rot_p, steps = dk / M::KS, tid = threadIdx.x;
+  const int dk = ROT64 ? 64 * NT + 64 : p.rank_p + p.rot_p, steps = dk / M::KS, tid = threadIdx.x;
   const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(tid >> 6), rl = lane & 15, g = lane >> 4;
   char* pf = smem;                                   // [4][64][16 B]
   char* qf = smem + 4096;                            // [steps][64][16 B]
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(256, EXACT && NT <= 8 ? 2 : 1) void latent_attn_f32
       if (s + 2 * kKeyPre < steps) load_k(0, s + 2 * kKeyPre);
       if (s + kKeyPre < steps) products(1, s + kKeyPre);
     };
-    if constexpr (EXACT) {
+    if constexpr (ROT64) {
 #pragma unroll
       for (int s = 0; s < steps; s += 2 * kKeyPre) two(s);
     } else {
@@ -616,8 +616,9 @@ int launch_attn_f32(const LatentAttnParams& p, hipStream_t st) {
   const size_t lds = 4096 + (size_t)(p.rank_p + p.rot_p) * 64;
   if (lds > kMaxLds) return -10;
   const dim3 grid(p.rows * ((p.H + 15) / 16), p.nch), block(256);
-  if (p.rank_p == 64 * NT && p.rot_p == 64) hipLaunchKernelGGL((latent_attn_f32_kernel<NT, true>), grid, block, lds, st, p);
-  else hipLaunchKernelGGL((latent_attn_f32_kernel<NT, false>), grid, block, lds, st, p);
+  if (p.rank_p != 64 * NT) hipLaunchKernelGGL((latent_attn_f32_kernel<NT, false, false>), grid, block, lds, st, p);
+  else if (p.rot_p == 64) hipLaunchKernelGGL((latent_attn_f32_kernel<NT, true, true>), grid, block, lds, st, p);
+  else hipLaunchKernelGGL((latent_attn_f32_kernel<NT, true, false>), grid, block, lds, st, p);
   return (int)hipGetLastError();
 }
 

@@ -67,3 +67,9 @@ def test_attention_and_gemm_kernels_do_not_spill():
         assert ks, pat
         bad = {k: v for k, v in ks.items() if v[0] > 0}
         assert not bad, f"{pat} instantiations use scratch: {bad}"
+
+
+def test_latent_attention_of_whole_ranks_keeps_two_waves():
+    """32 bits, rank 512: 256 registers at most whatever the rotary width (one form knows it, one takes any)."""
+    ks = {k: v for k, v in _kernels("latent.hip.o").items() if "latent_attn_f32_kernelILi8ELb1E" in k}
+    assert len(ks) == 2 and all(scratch == 0 and vgpr <= 256 for scratch, vgpr in ks.values()), ks

@@ -383,6 +383,13 @@ def test_latent_attention_32_bit_tiles(case):
     test_latent_attention(F32, case)
 
 
+@pytest.mark.parametrize("case", [(3, 24, 64, 32, 128, 16, 90), (5, 32, 32, 32, 512, 32, 700), (4, 24, 96, 32, 512, 16, 150), (2, 24, 64, 32, 1024, 16, 90)],
+                         ids=str)
+def test_latent_attention_32_bit_rotary_widths(case):
+    """Ranks of whole waves, each with the rotary width whose steps the compiler knows (64) and with another."""
+    test_latent_attention(F32, case)
+
+
 @pytest.mark.parametrize("case", LATENT, ids=str)
 @pytest.mark.parametrize("cuts", [[(0, 1000)], [(7, 2), (30, 60), (3, 1), (-1, 1), (16, 49)], [(0, 33), (64, 64), (33, 31)], [(1, 40)]], ids=str)
 def test_latent_prefill(case, cuts, monkeypatch):
