@@ -259,27 +259,38 @@ int dispatch_g(const DecodeAttnParams& p, hipStream_t st) {
 
 constexpr int kMqChunk = kWaves * kMqStep;  // chunk granularity of the standalone kernel (keys)
 
-template <int D, int G>
+template <int D, int G, bool FAR>
 __global__ __launch_bounds__(kWaves * 64) void decode_mq_kernel(DecodeAttnParams p) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[MqLds<D, kWaves>::bytes];
-  mq_body<D, G, kWaves, false>(p, lds, (int)gridDim.x, (int)blockIdx.x);
+  mq_body<D, G, kWaves, false, true, false, FAR>(p, lds, (int)gridDim.x, (int)blockIdx.x);
 }
 
 constexpr int kMqMaxGrid = 512;  // two workgroups per CU (D = 64: both resident)
 
-template <int D>
-int dispatch_mq(const DecodeAttnParams& p, hipStream_t st) {
+template <int D, bool FAR>
+int launch_mq(const DecodeAttnParams& p, hipStream_t st) {
   const int items = p.rows * p.n_kv_heads * p.n_splits;  // upper bound (every row its own group)
   const dim3 grid(items < kMqMaxGrid ? items : kMqMaxGrid), block(kWaves * 64);
   switch (p.n_q_heads / p.n_kv_heads) {
-    case 1: hipLaunchKernelGGL((decode_mq_kernel<D, 1>), grid, block, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((decode_mq_kernel<D, 2>), grid, block, 0, st, p); break;
-    case 4: hipLaunchKernelGGL((decode_mq_kernel<D, 4>), grid, block, 0, st, p); break;
-    case 8: hipLaunchKernelGGL((decode_mq_kernel<D, 8>), grid, block, 0, st, p); break;
-    case 16: hipLaunchKernelGGL((decode_mq_kernel<D, 16>), grid, block, 0, st, p); break;
+    case 1: hipLaunchKernelGGL((decode_mq_kernel<D, 1, FAR>), grid, block, 0, st, p); break;
+    case 2: hipLaunchKernelGGL((decode_mq_kernel<D, 2, FAR>), grid, block, 0, st, p); break;
+    case 4: hipLaunchKernelGGL((decode_mq_kernel<D, 4, FAR>), grid, block, 0, st, p); break;
+    case 8: hipLaunchKernelGGL((decode_mq_kernel<D, 8, FAR>), grid, block, 0, st, p); break;
+    case 16: hipLaunchKernelGGL((decode_mq_kernel<D, 16, FAR>), grid, block, 0, st, p); break;
     default: return -2;
   }
   return 0;
+}
+
+// Whether a launch may meet numbers that small_div does not hold for.  The block table bounds the contexts; the largest dividend of them is
+// a context and a chunk of it less one.
+bool mq_far(const DecodeAttnParams& p) {
+  return (int64_t)p.kv.table_stride * p.kv.block_size + kMqChunk > kSmallDiv / 2 || (int64_t)p.rows * p.n_kv_heads * p.n_splits > kSmallDiv;
+}
+
+template <int D>
+int dispatch_mq(const DecodeAttnParams& p, hipStream_t st) {
+  return mq_far(p) ? launch_mq<D, true>(p, st) : launch_mq<D, false>(p, st);
 }
 
 int g_attn_impl = 1;  // 1: multi-query MFMA kernel (default), 0: split VALU kernel

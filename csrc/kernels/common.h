@@ -172,8 +172,11 @@ VWA_DEVICE float wave_max(float v) {
 
 VWA_DEVICE int lane_id() { return threadIdx.x & 63; }
 
-// x / k of uniform 0 <= x < 2^21, 1 <= k: by a float reciprocal (x + 1/2 lies half a k-th from the next quotient, the product is off by
-// 2.7e-7 of itself).  The compiler's division is a chain of 25 operations, and a kernel of a few us starts with several.
+// x / k of uniform 0 <= x < kSmallDiv, 1 <= k: by a float reciprocal.  x + 1/2 lies half a k-th from the next quotient; the product is off
+// by a unit of the reciprocal's last place and half a one of its own, 1.8e-7 of itself, which is 0.38 k-ths at most.  (With every k to 4096
+// and the reciprocal a unit off either way, the first wrong quotient is 2100734 / 4095.)  The compiler's division is a chain of 25
+// operations, and a kernel of a few us starts with several.
+constexpr int kSmallDiv = 1 << 21;
 VWA_DEVICE int small_div(int x, int k) {
   return __builtin_amdgcn_readfirstlane((int)(((float)x + 0.5f) * __builtin_amdgcn_rcpf((float)k)));
 }

@@ -647,7 +647,7 @@ __global__ __launch_bounds__(C::THREADS, C::NW == 4 ? 2 : 1) void gemm_kernel(Ge
   const int mb = GRP ? p.g_tiles[0] : (p.M + C::BM - 1) / C::BM, nb = (p.N + C::BN - 1) / C::BN;
   const int tiles = mb * nb;
   // (few rows' launches are over in 8 us, and the compiler's divisions are a chain of 25 operations each in front of the first load)
-  const bool small = gridDim.x < (1u << 21);
+  const bool small = gridDim.x < (unsigned)kSmallDiv;
   const int part = gridDim.x == (unsigned)tiles ? 0 : small ? small_div(blockIdx.x, tiles) : blockIdx.x / tiles;
   const int split = p.nbatch > 1 ? 0 : part;  // split-K slice (blocks of one slice are contiguous)
   if (p.nbatch > 1) {  // batch z = blockIdx.x / tiles, splits == 1 (vwa_gemm)

@@ -176,7 +176,8 @@ constexpr float kMqRunsAhead = 0.95f;
 // after the wave's key steps (at once for a wave without one) and before the merge -- the chained
 // launch issues a weight item of a later phase there, so the attention workgroups' memory pipe is
 // not idle through the attention's merge (and, for the waves without a key step, all of it).
-template <int D, int G, int NW, bool SC1OUT, bool DB = true, bool FINE = false, class OnIdle = NoIdle,
+// FAR: numbers of keys or items past what the divisions by reciprocals hold for (kSmallDiv): divided exactly
+template <int D, int G, int NW, bool SC1OUT, bool DB = true, bool FINE = false, bool FAR = false, class OnIdle = NoIdle,
           class Stamp = NoStamp, class OnKv = NoIdle>
 VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid, int bid, OnIdle on_idle = {},
                         int* n_items_out = nullptr, Stamp stamp = {}, unsigned long long* done = nullptr,
@@ -193,6 +194,9 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   float* ow = reinterpret_cast<float*>(lds + L::ow);    // [NW][kMqCols][OWP]
   float* mlw = reinterpret_cast<float*>(lds + L::mlw);  // [NW][kMqCols][2]
   int& s_last = *reinterpret_cast<int*>(lds + L::last);
+
+  auto quot = [](int x, int k) { return FAR ? __builtin_amdgcn_readfirstlane(x / k) : small_div(x, k); };  // (uniform)
+  auto lane_quot = [](int x, int k) { return FAR ? x / k : lane_div(x, k); };
 
   const int nkv = p.n_kv_heads, nq = p.n_q_heads;
   const int lane = VWA_TX & 63, w = FINE ? VWA_TX >> 6 : __builtin_amdgcn_readfirstlane(VWA_TX >> 6);
@@ -334,8 +338,8 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     // 23.2 / 21.0 / 27.1
     const int ctx_all = __builtin_amdgcn_readfirstlane((int)wave_max((float)cl));
     const int c = min(lane + 1, p.n_splits);
-    const int len = (lane_div(ctx_all + c - 1, c) + kChunk - 1) / kChunk * kChunk;
-    const int cnt = len > 0 ? lane_div(ctx_all + len - 1, len) : 1;
+    const int len = (lane_quot(ctx_all + c - 1, c) + kChunk - 1) / kChunk * kChunk;
+    const int cnt = len > 0 ? lane_quot(ctx_all + len - 1, len) : 1;
     const int per_cu = (gh * cnt + kMqCus - 1) / kMqCus;
     const int cost = per_cu * len + (cnt > 1 ? cnt * (D == 64 ? 70 : 30) : 0) + (per_cu - 1) * (D == 64 ? 100 : 350);
     const float best = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(wave_max(-(float)cost))));
@@ -404,9 +408,9 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
     kvh = item % nkv;
     gi = (item / nkv) % n_groups, chunk = item / (nkv * n_groups);
   } else {
-    const int ig = small_div(item, nkv);
+    const int ig = quot(item, nkv);
     kvh = item - ig * nkv;
-    chunk = small_div(ig, n_groups);
+    chunk = quot(ig, n_groups);
     gi = ig - chunk * n_groups;
   }
   const unsigned long long pick = __ballot(((leaders >> lane) & 1ull) && my_rank == gi);
@@ -449,8 +453,8 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       if (c > P) own_mask |= 1 << run;
       if (run == j) my_max = max(my_max, c);
     }
-    CL = (small_div(P + n_pc - 1, n_pc) + kChunk - 1) / kChunk * kChunk;
-    const int npa = small_div(P + CL - 1, CL);
+    CL = (quot(P + n_pc - 1, n_pc) + kChunk - 1) / kChunk * kChunk;
+    const int npa = quot(P + CL - 1, CL);
     nact = npa + (wave_runs ? own_mask != 0 : __builtin_popcount(own_mask));
     if (chunk < n_pc) {
       kbeg = chunk * CL;
@@ -478,7 +482,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       if (rho < a - r0 || rho >= b - r0) ctx_n = 0;  // other runs' columns: no keys in this chunk
     }
   } else {
-    CL = ((FINE ? (ctxmax + n_eff - 1) / n_eff : small_div(ctxmax + n_eff - 1, n_eff)) + kChunk - 1) / kChunk * kChunk;
+    CL = ((FINE ? (ctxmax + n_eff - 1) / n_eff : quot(ctxmax + n_eff - 1, n_eff)) + kChunk - 1) / kChunk * kChunk;
     if (cascade) CL = (ctxmax + kChunk - 1) / kChunk * kChunk;  // padded rows: one chunk
     kbeg = chunk * CL;
     if (kbeg >= ctxmax) {
@@ -486,7 +490,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
       continue;
     }
     kend = min(ctxmax, kbeg + CL);
-    nact = FINE ? (ctxmax + CL - 1) / CL : small_div(ctxmax + CL - 1, CL);
+    nact = FINE ? (ctxmax + CL - 1) / CL : quot(ctxmax + CL - 1, CL);
   }
   if (item == bid) write_plan(cascade ? 3 : 1, kvh, r0, nr, kbeg, kend, nact, slot, c_own);
   }  // (metadata path)
@@ -510,7 +514,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   int64_t tabA = 0, tabB = 0;
   auto load_tab = [&](int s0) {
     const int ka = min(wb + (s0 + lane) * kMqStep, kmax), kb = min(ka + 16, kmax);
-    const int ia = lane_div(ka, bs), ib = lane_div(kb, bs);
+    const int ia = lane_quot(ka, bs), ib = lane_quot(kb, bs);
     gint* tab = (gint*)(p.kv.block_table + (int64_t)kv_seq * p.kv.table_stride);
     const int ba = tab[ia], bb = tab[ib];
     tabA = ba * p.kv.stride_block + (ka - ia * bs) * p.kv.stride_tok;

@@ -401,6 +401,46 @@ def test_decode_attention_block_sizes(hd, nq, nkv, bs, ctx, splits):
     close(out, exp, 2e-2)  # q, the weights and the output are rounded to bf16 (2^-9 each; scores are ~N(0, 1))
 
 
+@pytest.mark.parametrize("hd,nq,nkv", [(128, 32, 8), (128, 8, 1), (64, 6, 6), (64, 32, 2)])
+@pytest.mark.parametrize("bs", [16, 48, 24])
+def test_decode_attention_of_a_wide_table(hd, nq, nkv, bs):
+    """A block table of a million keys and more takes the form that divides exactly: the same bits, with rows that share a prefix, runs of
+    one sequence and contexts of one key and several chunks."""
+    seqs, ctx = [0, 0, 0, 1, 2, 2, 3], [300, 301, 302, 97, 640, 641, 1]
+    per, P = -(-641 // bs), 96
+    kc, vc, q = rnd(4 * per, nkv, bs, hd), rnd(4 * per, nkv, bs, hd), rnd(7, nq * hd)
+    table = torch.randperm(4 * per, device=DEV).view(4, per).to(torch.int32)
+    table[:, : P // bs] = table[0, : P // bs]
+    wide = torch.zeros(4, -(-(1 << 20) // bs), dtype=torch.int32, device=DEV)
+    wide[:, :per] = table
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    for shared, n in ((None, 7), (i32([P // bs * bs, 6]), 7)):
+        got = []
+        for t in (table, wide):
+            out = torch.empty(n, nq * hd, dtype=BF, device=DEV)
+            ops.decode_attention(q, ops.KVLayout.paged(kc, vc, t), i32(ctx), i32(seqs), n_q_heads=nq, n_kv_heads=nkv, head_dim=hd,
+                                 scale=hd ** -0.5, max_ctx=per * bs, out=out, shared=shared)
+            got.append(out)
+        assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("bs,ctx", [(16, (1 << 23) + 16), (48, 4_000_032)])
+def test_decode_attention_of_millions_of_keys(bs, ctx):
+    """Places of keys past what a 32-bit reciprocal divides: eight keys of score 40 among zeros of score 0, whose 2^23 weights are 4e-11
+    of theirs, so the output is the mean of their values, rounded once."""
+    n, at = ctx // bs, torch.tensor([0, 17, (1 << 21) - 1, 1 << 21, ctx // 2 + 5, ctx - 1000, ctx - 17, ctx - 1], device=DEV)
+    kc, vc = torch.zeros(n, 1, bs, 64, dtype=BF, device=DEV), torch.zeros(n, 1, bs, 64, dtype=BF, device=DEV)
+    table = torch.arange(n - 1, -1, -1, dtype=torch.int32, device=DEV)[None].contiguous()
+    v = rnd(8, 64)
+    kc[n - 1 - at // bs, 0, at % bs], vc[n - 1 - at // bs, 0, at % bs] = 0.625, v
+    q, out = torch.ones(1, 64, dtype=BF, device=DEV), torch.empty(1, 64, dtype=BF, device=DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    ops.decode_attention(q, ops.KVLayout.paged(kc, vc, table), i32([ctx]), i32([0]), n_q_heads=1, n_kv_heads=1, head_dim=64, scale=1.0,
+                         max_ctx=ctx, out=out, n_splits=64)
+    want = v.double().mean(0)
+    assert ((out[0].double() - want).abs() <= 2.0**-8 * want.abs() + 1e-6).all()
+
+
 def test_flash_attention_causal_paged_prefix():
     hd, nq, nkv, bs = 128, 8, 2, 16
     blocks = 40
