@@ -33,13 +33,13 @@ def close(a, b, atol, rtol=2e-2):
     assert err <= tol, f"max err {err} > tol {tol}"
 
 
-@pytest.fixture(params=[(0, 256, 8), (1, 256, 8, 0), (1, 768, 4), (1, 256, 8, 2)],
-                ids=["tile", "stream8_xfirst", "stream4", "stream8"])
+@pytest.fixture(params=[(0, 256, 8), (1, 3, 8), (1, 768, 4), (1, 256, 8)],  # (three workgroups: every epilogue behind several items)
+                ids=["tile", "stream8_few", "stream4", "stream8"])
 def skinny_mode(request):
     ops.ext().set_skinny_mode(*request.param)
     ops.ext().set_small_gemm_bytes(0)  # every shape on the selected kernel (no small-weight routing)
     yield request.param
-    ops.ext().set_skinny_mode(1, 256, 0, 2)
+    ops.ext().set_skinny_mode(1, 256, 0)
     ops.ext().set_small_gemm_bytes(4 << 20)
 
 
@@ -530,7 +530,7 @@ def test_skinny_stream_items(ks, groups, tiles):
     """One item a workgroup (of two, three or four k-groups a wave), one to five of them on two workgroups, with and without a remainder of
     k-groups, X in LDS (8192 values of 16 rows: beside the weights): rows and columns against 64 bits."""
     N, K = 16 * tiles, 128 * groups
-    ops.ext().set_skinny_mode(1, 2, ks, 2)
+    ops.ext().set_skinny_mode(1, 2, ks)
     ops.ext().set_small_gemm_bytes(0)
     try:
         for M in (1, 7, 16):
@@ -543,7 +543,7 @@ def test_skinny_stream_items(ks, groups, tiles):
                 ops.linear(x, weight, out=out, residual=r)
                 assert ((out.double() - exact).abs() <= tol).all(), (M, type(weight))
     finally:
-        ops.ext().set_skinny_mode(1, 256, 0, 2)
+        ops.ext().set_skinny_mode(1, 256, 0)
         ops.ext().set_small_gemm_bytes(4 << 20)
 
 

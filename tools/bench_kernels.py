@@ -41,7 +41,7 @@ def timeit(fn, iters=40, reps=5):
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--json", default=None)
-    ap.add_argument("--only", default="gemm,attn,flash", help="comma list of floor,gemm,gemm8,wfirst,attn,flash,mall")
+    ap.add_argument("--only", default="gemm,attn,flash", help="comma list of floor,gemm,gemm8,attn,flash,mall")
     args = ap.parse_args()
     only = set(args.only.split(","))
     dev = "cuda"
@@ -110,27 +110,6 @@ def main():
                  torch_fill_us=round(timeit(lambda: o1.fill_(1.0)), 2))
         print(json.dumps(r), flush=True)
         res.append(r)
-    # prologue order A/B: first weight item before / after the X staging (+ fused RMSNorm)
-    for M in ((1, 4) if "wfirst" in only else ()):
-        for name, N, K in shapes[:4]:
-            x = torch.randn(M, K, device=dev).to(torch.bfloat16)
-            ncopy = max(1, int(1.0e9 // (N * K * 2)) + 1)
-            ws = [(torch.randn(N, K, device=dev) * 0.02).to(torch.bfloat16) for _ in range(ncopy)]
-            y = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
-            it = [0]
-            out = {}
-            for rms in (False, True):
-                for wf in (0, 2):
-                    def f():
-                        it[0] = (it[0] + 1) % ncopy
-                        ops.ext().skinny_gemm(x, ws[it[0]], None, y, 0, rms, 1e-5, None)
-                    ops.ext().set_skinny_mode(1, 256, 8, wf)
-                    out[f"rms{int(rms)}_wf{wf}"] = round(timeit(f), 2)
-            ops.ext().set_skinny_mode(1, 256, 0, 2)
-            del ws
-            r = dict(kernel="prologue_order", shape=name, M=M, **out)
-            print(json.dumps(r), flush=True)
-            res.append(r)
     # fp8 (W8A8) streaming GEMM on the same shapes, vs torch._scaled_mm (hipBLASLt fp8) where available
     for M in ((1, 4, 16) if "gemm8" in only else ()):
         for name, N, K in shapes:

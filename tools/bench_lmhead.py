@@ -31,9 +31,9 @@ def main():
         r = {"shape": name, "MB": round(N * K * 2 / 1e6, 1)}
         for cap in (256, 512, 1024):
             for ks in (4, 8):
-                E.set_skinny_mode(1, cap, ks, 2)
+                E.set_skinny_mode(1, cap, ks)
                 r[f"g{cap}_k{ks}_us"] = round(timeit(f), 2)
-        E.set_skinny_mode(1, 256, 0, 2)
+        E.set_skinny_mode(1, 256, 0)
         best = min(v for k, v in r.items() if k.endswith("_us"))
         r["best_tbps"] = round(N * K * 2 / best / 1e6, 2)
         print(json.dumps(r), flush=True)

@@ -36,14 +36,14 @@ def main():
 
         r = {"shape": name, "N": N, "K": K, "MB": round(N * K * 2 / 1e6, 2)}
         E.set_small_gemm_bytes(64 << 20)
-        E.set_skinny_mode(0, 256, 8, 2)
+        E.set_skinny_mode(0, 256, 8)
         r["rowmajor_onetile_us"] = round(timeit(run(False, ws)), 2)
         E.set_small_gemm_bytes(0)
         for cap, ks in ((256, 8), (128, 8), (256, 4)):
-            E.set_skinny_mode(1, cap, ks, 2)
+            E.set_skinny_mode(1, cap, ks)
             r[f"rowmajor_stream_g{cap}_k{ks}_us"] = round(timeit(run(False, ws)), 2)
             r[f"tiled_stream_g{cap}_k{ks}_us"] = round(timeit(run(True, wt)), 2)
-        E.set_skinny_mode(1, 256, 0, 2)
+        E.set_skinny_mode(1, 256, 0)
         E.set_small_gemm_bytes(4 << 20)
         best = min(v for k, v in r.items() if k.endswith("_us"))
         r["best_tbps"] = round(N * K * 2 / (best * 1e-6) / 1e12, 3)

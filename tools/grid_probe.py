@@ -23,7 +23,7 @@ def main():
         x = torch.randn(M, K, device=dev).to(bf)
         out = torch.empty(M, N, dtype=torch.float32 if name == "lm_head" else bf, device=dev)
         for cap in (256, 512, 256, 512):
-            E.set_skinny_mode(1, cap, 8, 2)
+            E.set_skinny_mode(1, cap, 8)
             for i in range(3):
                 ops.linear(x, ws[i % copies], out=out)
             torch.cuda.synchronize()
@@ -38,7 +38,7 @@ def main():
             res.setdefault(name, {}).setdefault(str(cap), []).append(round(us, 2))
         del ws
         torch.cuda.empty_cache()
-    E.set_skinny_mode(1, 256, 0, 2)
+    E.set_skinny_mode(1, 256, 0)
     print(json.dumps({"kernel": "grid_probe", "us": res}))
 
 

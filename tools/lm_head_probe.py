@@ -38,7 +38,7 @@ def main():
     ref = None
     res = {}
     for cap in [int(v) for v in a.caps.split(",")]:
-        E.set_skinny_mode(1, cap, 0, 2)
+        E.set_skinny_mode(1, cap, 0)
         ts = []
         for i in range(a.iters + 3):
             flush_b.copy_(flush_a)
@@ -56,7 +56,7 @@ def main():
         print(json.dumps(dict(tool="lm_head_probe", asr=a.asr, grid_cap=cap, us=res[cap]["us"],
                               tb_s=round(w.numel() * 2 / (statistics.median(ts) * 1e-6) / 1e12, 2),
                               same_bits=same)), flush=True)
-    E.set_skinny_mode(1, 256, 0, 2)
+    E.set_skinny_mode(1, 256, 0)
 
 
 if __name__ == "__main__":
