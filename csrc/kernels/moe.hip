@@ -131,7 +131,6 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     for (int k = 0; k < kRouteWaves; ++k) z += red[k * Ep * 16 + i];
     sc[(i & 15) * (Ep + 1) + (i >> 4)] = (i >> 4) < p.E ? rank_of(1.f / (1.f + expf(-z))) : -2.f;
   }
-  int* lds_ids = reinterpret_cast<int*>(red);        // (a launch of one workgroup groups from here)
   lds_sync();
   const int r = tid >> 5, q = tid & 31, row = r0 + r;  // 32 lanes per row: the choices stay inside a wave
   if constexpr (COUNT) {
@@ -172,42 +171,43 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(MoeRouteParams
     }
     if (chosen) {
       p.wts[row * p.top + place] = live ? weight_of(v) : 0.f;
-      lds_ids[r * p.top + place] = live ? q : -1;
       __hip_atomic_store(p.ids + row * p.top + place, live ? q : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-  } else
-  for (int k = 0; k < p.top; ++k) {
-    float best = -3.f;
-    int at = 0;
-    for (int e = q; e < p.E; e += 32) {
-      const float v = sc[r * (Ep + 1) + e];
-      if (v > best) {
-        best = v;
-        at = e;
+  } else {
+    int* lds_ids = reinterpret_cast<int*>(red);      // (a launch of one workgroup groups from here)
+    for (int k = 0; k < p.top; ++k) {
+      float best = -3.f;
+      int at = 0;
+      for (int e = q; e < p.E; e += 32) {
+        const float v = sc[r * (Ep + 1) + e];
+        if (v > best) {
+          best = v;
+          at = e;
+        }
       }
-    }
 #pragma unroll
-    for (int o = 16; o > 0; o >>= 1) {
-      const float bo = __shfl_xor(best, o, 32);
-      const int ao = __shfl_xor(at, o, 32);
-      if (bo > best || (bo == best && ao < at)) {
-        best = bo;
-        at = ao;
+      for (int o = 16; o > 0; o >>= 1) {
+        const float bo = __shfl_xor(best, o, 32);
+        const int ao = __shfl_xor(at, o, 32);
+        if (bo > best || (bo == best && ao < at)) {
+          best = bo;
+          at = ao;
+        }
       }
+      if (q == 0 && r < nr) {
+        sc[r * (Ep + 1) + at] = -1.f;                // (taken; scores are positive)
+        p.wts[row * p.top + k] = live ? weight_of(best) : 0.f;
+        lds_ids[r * p.top + k] = live ? at : -1;
+        __hip_atomic_store(p.ids + row * p.top + k, live ? at : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
-    if (q == 0 && r < nr) {
-      sc[r * (Ep + 1) + at] = -1.f;                  // (taken; scores are positive)
-      p.wts[row * p.top + k] = live ? weight_of(best) : 0.f;
-      lds_ids[r * p.top + k] = live ? at : -1;
-      __hip_atomic_store(p.ids + row * p.top + k, live ? at : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    lds_sync();
+    if (gridDim.x == 1) {
+      group_pairs(p, [&](int i) { return lds_ids[i]; });
+      return;
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-  lds_sync();
-  if (gridDim.x == 1) {
-    group_pairs(p, [&](int i) { return lds_ids[i]; });
-    return;
   }
   // ---- the last workgroup groups the pairs
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -10,12 +10,6 @@ namespace {
 
 enum Epi { EPI_STORE = 0, EPI_RESID = 1, EPI_SWIGLU = 2, EPI_GELU = 3, EPI_QKV = 4, EPI_SPLIT = 5 };
 
-constexpr unsigned kOOB = 0xFFFFFFF0u;
-
-VWA_DEVICE uint4 bload(__amdgpu_buffer_rsrc_t r, unsigned off) {
-  u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
 // weight-stream load with cache policy AUX (gfx950 buffer aux bits: 1 sc0, 2 nt, 16 sc1): decode
 // weights are read once per step by one CU, so nt (2) keeps them from displacing L2 lines
 template <int AUX>
@@ -94,28 +88,25 @@ VWA_DEVICE void epi_values(const SkinnyParams& p, int tile, int o, EpiPre& e) {
 // Cross-wave reduction of one column tile + fused epilogue.  rs[m]: per-row scale (fused RMSNorm
 // / LayerNorm rstd and, on the fp8 path, the activation quantisation scale); mus[m] (folded
 // LayerNorm only, else null): row mean, removed as mean * ln_c[n]; column scales (fp8) come
-// with the epilogue operands (`pre` when this is the workgroup's first tile).
-// MT: 16-row MFMA row fragments per tile (M <= 16 MT; MT > 1 only in the streaming kernel's
-// many-row form, skinny_stream_kernel); red = [KS][NT][MT][4][64] partial sums.
-template <int EPI, int NT, int KS, bool SC1 = false, int MT = 1>
+// with the epilogue operands (`pre` when this is the workgroup's first tile); red = [KS][NT][4][64]
+// partial sums.
+template <int EPI, int NT, int KS, bool SC1 = false>
 VWA_DEVICE void tile_epilogue(const SkinnyParams& p, float* red, const float* rs, const float* mus, int tile,
-                              f32x4 (&acc)[NT * MT], int w, int lane, const EpiPre& pre, bool first,
+                              f32x4 (&acc)[NT], int w, int lane, const EpiPre& pre, bool first,
                               const float* partner = nullptr) {
   const int M = p.M;
   const int n0 = tile * 16 * NT;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) red[(((w * NT + nt) * MT + mt) * 4 + i) * 64 + lane] = acc[nt * MT + mt][i];
+    for (int i = 0; i < 4; ++i) red[((w * NT + nt) * 4 + i) * 64 + lane] = acc[nt][i];
   lds_sync();
   auto red_at = [&](int m, int nn) -> float {
-    const int nt = nn >> 4, q = nn & 15, mt = MT > 1 ? m >> 4 : 0, mm = m & 15;
+    const int nt = nn >> 4, q = nn & 15, mm = m & 15;
     const int ln = q + 16 * (mm >> 2), i = mm & 3;
     float s = 0.f;
 #pragma unroll
-    for (int ww = 0; ww < KS; ++ww) s += red[(((ww * NT + nt) * MT + mt) * 4 + i) * 64 + ln];
+    for (int ww = 0; ww < KS; ++ww) s += red[((ww * NT + nt) * 4 + i) * 64 + ln];
     // split tile (chain kernel): the other workgroup's partial sums, published with sc1 stores
     if (partner) s += __hip_atomic_load(gp(partner + m * 16 * NT + nn), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return s;
@@ -197,7 +188,7 @@ VWA_DEVICE void tile_epilogue(const SkinnyParams& p, float* red, const float* rs
   }
   lds_sync();
 #pragma unroll
-  for (int k = 0; k < NT * MT; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int k = 0; k < NT; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
 }  // namespace
