@@ -381,7 +381,7 @@ VWA_DEVICE bool mq_body(const DecodeAttnParams& p, unsigned char* lds, int grid,
   // wave, 0.8 us ahead of the first load; so it is where it is used, under the loads.  With the step's rows read by every wave, without
   // LDS and a barrier, and divisions by reciprocals the first keys are asked for 3.4 us after the start instead of 4.5.  us of a launch in
   // a model's step: 8 rows x 20 heads of 64, 1500 keys 16.5 -> 15.8, their own keys 5.6 -> 4.8; 32 sessions x 8 kv heads of 128 behind
-  // 1008 shared keys 17.1 -> 16.8)
+  // 1008 shared keys 17.1 -> 16.6)
   int lane = lane_of;
   if constexpr (!FINE) asm volatile("" : "+v"(lane));
   const int n = lane & 15, g = lane >> 4;

@@ -222,6 +222,11 @@ VWA_DEVICE void save_inputs4(const RgLruParams& p, int r, int n, bool fresh, flo
 // Workgroup (block, tile, part): the runs whose first row lies in rows 16 tile .. 16 tile + 15, 16 rows at a time to
 // their ends (other runs' rows count as inert); row_parts of the block's 16-channel tiles.  Every part forms the whole block's u,
 // so the inputs it is formed from are replaced by the last part that has read them (RgLruParams::tickets).
+// A part is worth its own forming of u and its ticket from 128 KB of gates and four tiles on.  Measured while every wave had one tile and
+// both tasks: us with parts of all 16, 8, 4, 2 tiles, gates in L2, 32 bits, 4 rows x 4 blocks of 256 16.1, 12.0, 10.6, 10.6; bf16, 16 rows
+// x 8 11.2, 10.6, 10.7, 11.0; parts of fewer tiles made blocks of 80 and 128 channels 9 - 18 % slower in 16 bits (4 rows of 128: 6.8 -> 7.7)
+// and up to 4 % in 32, 10 blocks of 256 in 16 bits at 48 rows 10 %.  The line was not drawn again for waves of one task: a part of four tiles
+// has eight that draw its gates now, and 72 sizes as a whole take 1 - 37 % less with it where it was.
 constexpr int kPartBytes = 128 * 1024;
 int row_parts(int bs, int bytes) {
   const int tiles = bs / 16, draw = 32 * bs * bytes, per = (kPartBytes + draw - 1) / draw;

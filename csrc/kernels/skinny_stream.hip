@@ -12,9 +12,10 @@
 //    waves split K, and every wave walks a flat list of (tile, k-batch) items;
 //  * weight loads are raw buffer loads (SRD with num_records = N*K*2): the next item's 16 x
 //    dwordx4 per lane are issued BEFORE the current item's MFMAs (two named register sets,
-//    static indices -> counted vmcnt), and past-the-end items/groups use an out-of-range offset
-//    that the hardware answers with zeros and no memory traffic, so the pipeline has no
-//    data-dependent load predicates;
+//    static indices -> counted vmcnt); k-groups that a wave does not have use an out-of-range offset
+//    that the hardware answers with zeros and no memory traffic, but their addresses occupy its unit
+//    as long as any load's: items past the last are not asked for, and a workgroup with one item takes
+//    a form of as many k-groups as there are;
 //  * the cross-wave reduction + fused epilogue of tile t runs while tile t+1's loads are in flight.
 //
 // XG variant (X does not fit in LDS: e.g. the down projection, K = 14336, with more than 5 rows):
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(KS * 64, KS == 4 && EPI != EPI_QKV && !XG ? 3 : 1) 
   // first one for the weights too: a chain of M K / 8 / threads round trips in front of any product.)
   constexpr int T = KS * 64, PB = KS == 4 ? 4 : 8;  // (four waves: three workgroups share a CU's registers)
   const int k8 = K / 8, pieces = M * k8;
-  // (quotients below 2^14 by a float reciprocal: half a k8-th away from the next integer, 4e-6 off)
+  // (numbers of threads by a float reciprocal: small_div's bound)
   const float rk8 = __builtin_amdgcn_rcpf((float)k8);
   const int dm = (int)((T + 0.5f) * rk8), dk = T - dm * k8;
   int xm = (int)(((float)VWA_TX + 0.5f) * rk8), xk = VWA_TX - xm * k8;  // this thread's next piece
@@ -297,11 +298,12 @@ __global__ __launch_bounds__(KS * 64, KS == 4 && EPI != EPI_QKV && !XG ? 3 : 1) 
 
 int g_x_skew = 32;  // LDS X row skew (elements per 4 rows; 0: none -- A/B knob, vwa_skinny_set_x_skew)
 
-// Persistent workgroups of a launch: grid_cap (one a CU) times what a CU holds.  Of four waves (K < 2048; 148 - 189 registers) that
+// Persistent workgroups of a launch: grid_cap (one a CU) times what a CU holds.  Of four waves (K < 2048; up to 188 registers) that
 // is three, two of the QKV epilogue, where the X rows leave LDS for them: more weight bytes are on the way, and tiles past one a CU
 // are not drawn one after the other.  us at one / two / three a CU, 8 rows: 5120 x 1280 10.7 / 9.9 / 9.9, 51872 x 1280 43.0 / 36.0 /
 // 33.0, 32768 x 1024 27.5 / 21.9 / 21.0, 6144 x 1536 11.7 / 10.7 / 10.7; fp8 weights 32768 x 1024 17.5 / 15.8 / 14.8, 8192 x 1024 7.9 / 7.7
-// / 7.6; up to 256 tiles the same launch.
+// / 7.6; up to 256 tiles the same launch.  (Measured before X was staged in batches and an fp8 row was quantised by one wave, which took
+// 160 - 196 registers to 82 - 188: a CU holds as many workgroups as then.)
 template <int EPI, int KS>
 int grid_of(int ntiles, int grid_cap, size_t lds) {
   int per = KS == 4 ? EPI == EPI_QKV ? 2 : 3 : 1;
@@ -439,7 +441,9 @@ __global__ __launch_bounds__(KS * 64, KS == 4 && EPI != EPI_QKV ? 3 : 1) void sk
   uint4 A[NT][U][2], B[NT][U][2];
   // ---- rows w, w + KS, .. of X are this wave's: statistics (sum of squares for the fused RMSNorm, amax for the fp8 scale), then
   // e4m3 codes into LDS.  A row's first PB pieces a lane stay in registers in between, and the next row's are requested in front
-  // of them, the first weight item behind the first row's.
+  // of them, the first weight item behind the first row's.  (A row used to be read twice, one piece a lane waited for at a time, by its
+  // own wave for the statistics and by all for the codes, and the weights were asked for behind both.  Not timed against that form; the
+  // results are the same bits.)
   constexpr int PB = KS == 4 ? 4 : 8;  // (four waves: rows of less than 2048)
   u32x4 row[PB], ahead[PB];
   auto load_row = [&](u32x4 (&v)[PB], int m, int k0) {  // pieces past the row's end: zeros

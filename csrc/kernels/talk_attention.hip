@@ -221,8 +221,10 @@ __global__ __launch_bounds__(256) void talk_scores_kernel(TalkAttnParams p) {
 // tile's place with the table's row, keys.  (The keys used to be requested behind the turned query: 5.9 -> 4.8 and 8.6 -> 7.5 us, with
 // the cache's and the recurrence's workgroups down to three trips.)
 constexpr int kStepParts = 2;                        // workgroups of a row's keys and values
-// Scoring workgroups that a launch aims at: as many as are resident at once beside the others, in whole ones to a row, kv head and 16 of
-// its query heads, but three of them at least, which share the row's chunks (64 rows of 16 kv heads: 3072; none waits for another).
+// Scoring workgroups that a launch aims at, in whole ones to a row, kv head and 16 of its query heads, but three of them at least, which
+// share the row's chunks (64 rows of 16 kv heads: 3072; none waits for another).  768 is what was resident at once beside the others while
+// five workgroups fitted a CU.  The requests ahead of the first wait take registers: four fit in 16 bits (127), 1024 with the others, three
+// in 32 bits (137), 768 with them.  The figures below are of five a CU; the number was not measured again.
 // One a chunk of the longest context would be mostly workgroups without keys: 48 rows of 2048 tokens' room and 90 .. 250 keys, 3840
 // workgroups 11.1 us, 768 10.7; 240 steps (1 .. 64 rows, 20 .. 2000 keys, six head shapes) against three launches: 0.93 of the time, and
 // 0.914 so.  With one a row and kv head where they are many, a row's chunks were one after another: 64 rows x 8 kv heads of 2000 keys 111 ->

@@ -449,6 +449,8 @@ def test_mingru_rounds_one_product(dtype, W, first, pairs):
     (6, 2, 32, 48, 16, 33, 3, 16),        # half of a fragment step rotates
     (20, 1, 64, 16, 64, 0, 0, 32),        # two column groups; every dimension rotates
     (4, 4, 96, 32, 32, 1, 17, 16),        # a window of one behind kept keys
+    (4, 2, 160, 64, 160, 0, 0, 16),       # a head in two pieces, the second in part; pairs across the two
+    (8, 2, 256, 32, 64, 48, 2, 16),       # two whole pieces
 ])
 def test_talk_mingru_step(dtype, H, G, dk, dv, rot, window, keep, bs):
     """A decode step's two launches against the ops they stand for, over one set of caches: single rows, runs that start at 0, end
